@@ -1,0 +1,131 @@
+"""The compiled host path (csrc/xq_torch.cpp) against the Python path over the same library calls: the same bits, forward and
+backward, for every module kind; calls it leaves to the Python path still work."""
+
+import pytest
+import torch
+
+from tests.test_gpu_moe import _make_experts, _zipf_routing
+from tests.util_cases import gen, make_dense_module
+
+pytestmark = pytest.mark.gpu
+
+
+class _Declines:
+    """Stands in for the extension and leaves every call to the Python path."""
+
+    def __getattr__(self, name):
+        return lambda *a: None
+
+
+@pytest.fixture
+def both_paths(monkeypatch):
+    import xorl_amd.moe_functional as MF
+    import xorl_amd.qlora.linear as LIN
+    import xorl_amd.qlora.moe_experts as EXP
+
+    def run(fn):
+        got = fn()
+        with monkeypatch.context() as mp:
+            for mod in (MF, LIN, EXP):
+                mp.setattr(mod, "native", lambda: _Declines())
+            want = fn()
+        assert len(got) == len(want)
+        for a, b in zip(got, want):
+            assert a.dtype == b.dtype and torch.equal(a, b)
+        return got
+
+    return run
+
+
+@pytest.mark.parametrize("fmt,bias", [("block_fp8", False), ("nvfp4", True), ("int4", False), ("nf4", True)])
+@pytest.mark.parametrize("shape", [(1, 512), (2, 9, 512), (65, 512)])
+def test_linear(hip_device, both_paths, fmt, bias, shape):
+    m, _ = make_dense_module(fmt, 256, 512, 16, 32, 3, hip_device, bias=bias)
+    x = gen(shape, 1.0, 4, torch.bfloat16).to(hip_device)
+    dy = gen((*shape[:-1], 256), 1.0, 5, torch.bfloat16).to(hip_device)
+
+    def infer():
+        with torch.no_grad():
+            return [m(x), m(x.transpose(0, -1).contiguous().transpose(0, -1))]      # a layout that needs a packed copy
+
+    def train():
+        xr = x.clone().requires_grad_(True)
+        y = m(xr)
+        return [y.detach(), *torch.autograd.grad(y, [xr, m.lora_A, m.lora_B], dy)]
+
+    both_paths(infer)
+    both_paths(train)
+
+
+@pytest.mark.parametrize("fmt", ["block_fp8", "nvfp4"])
+@pytest.mark.parametrize("M", [1, 33, 200])
+def test_mlp_and_joint_linears(hip_device, both_paths, fmt, M):
+    from xorl_amd.qlora import qlora_linears_forward, qlora_mlp_forward
+
+    H, I = 512, 768
+    mods = [make_dense_module(fmt, n, k, 8, 16, 11 + i, hip_device)[0] for i, (n, k) in enumerate(((I, H), (I, H), (H, I)))]
+    x = gen((M, H), 1.0, 4, torch.bfloat16).to(hip_device)
+    dy = gen((M, H), 1.0, 5, torch.bfloat16).to(hip_device)
+
+    def infer():
+        with torch.no_grad():
+            return [qlora_mlp_forward(*mods, x), *qlora_linears_forward(mods[:2], x)]
+
+    def train():
+        xr = x.clone().requires_grad_(True)
+        y = qlora_mlp_forward(*mods, xr)
+        return [y.detach(), *torch.autograd.grad(y, [xr] + [p for m in mods for p in m.get_lora_parameters()], dy)]
+
+    both_paths(infer)
+    both_paths(train)
+
+
+@pytest.mark.parametrize("fmt,hybrid,rw_dtype", [("block_fp8", False, torch.bfloat16), ("nvfp4", True, torch.float32), ("nf4", False, torch.float64)])
+@pytest.mark.parametrize("T", [3, 300])
+def test_experts(hip_device, both_paths, fmt, hybrid, rw_dtype, T):
+    E, H, I, topk = 6, 256, 256, 2
+    m, _ = _make_experts(fmt, E, H, I, 8, hybrid, 7, hip_device)
+    rw, sel = _zipf_routing(T, E, topk, seed=2)
+    rw, sel = rw.to(rw_dtype).to(hip_device), sel.long().to(hip_device)
+    x = gen((T, H), 1.0, 4, torch.bfloat16).to(hip_device)
+    dy = gen((T, H), 1.0, 5, torch.bfloat16).to(hip_device)
+
+    def infer():
+        with torch.no_grad():
+            return [m(x, rw, sel)]
+
+    def train():
+        xr, rr = x.clone().requires_grad_(True), rw.clone().requires_grad_(True)
+        y = m(xr, rr, sel)
+        return [y.detach(), *torch.autograd.grad(y, [xr, rr, *m.get_lora_parameters()], dy)]
+
+    both_paths(train)
+    if T == 3:      # (the Python path reaches _moe_infer with its banks)
+        import xorl_amd.moe_functional as MF
+
+        got = infer()[0]
+        with torch.no_grad():
+            gA, gB = m._active_lora_views("gate_proj")
+            uA, uB = m._active_lora_views("up_proj")
+            dA, dB = m._active_lora_views("down_proj")
+            want = MF.moe_experts_qlora_forward(E, rw, sel, x, m._bank("gate"), m._bank("up"), m._bank("down"), gA, gB, uA, uB, dA, dB,
+                                                m._active_scaling())
+        assert torch.equal(got, want)
+    else:
+        both_paths(infer)
+
+
+def test_calls_left_to_the_python_path(hip_device):
+    from xorl_amd import _C
+
+    m, _ = make_dense_module("int4", 128, 256, 16, 32, 3, hip_device)
+    x = gen((4, 256), 1.0, 4, torch.bfloat16).to(hip_device)
+    with torch.no_grad():
+        full = m(x)
+        m.set_runtime_lora_config(8, 16)                       # an active rank below the stored one
+        part = m(x)
+    assert full.shape == part.shape and not torch.equal(full, part)
+    with pytest.raises(_C.XqError):
+        m(x.float())
+    with pytest.raises(_C.XqError):
+        m(x[:, :128].contiguous())

@@ -1,4 +1,5 @@
-"""Compile the HIP sources in this directory into xorl_amd/lib/libxq_hip.so (gfx950)."""
+"""Compile the HIP sources in this directory into xorl_amd/lib/libxq_hip.so (gfx950), and the host path of the modules
+(xq_torch.cpp, host code against torch's C++ API) into xorl_amd/lib/xq_torch.so."""
 
 from __future__ import annotations
 
@@ -6,12 +7,14 @@ import glob
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_DIR = os.path.join(os.path.dirname(HERE), "lib")
 OBJ_DIR = os.path.join(HERE, "_obj")
 SO_PATH = os.path.join(LIB_DIR, "libxq_hip.so")
+TORCH_SO_PATH = os.path.join(LIB_DIR, "xq_torch.so")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
@@ -39,6 +42,29 @@ def _compile(src: str, force: bool) -> str:
     return obj
 
 
+def _build_torch(force: bool) -> None:
+    """xq_torch.so: a CPython extension linked to torch and, beside it, to libxq_hip.so."""
+    src, hdr = os.path.join(HERE, "xq_torch.cpp"), os.path.join(HERE, "..", "..", "include", "xq.h")
+    if not force and os.path.exists(TORCH_SO_PATH) and all(os.path.getmtime(TORCH_SO_PATH) >= os.path.getmtime(d) for d in (src, hdr)):
+        return
+    import torch
+
+    t = os.path.dirname(torch.__file__)
+    rocm = os.path.dirname(os.path.dirname(HIPCC))
+    includes = [os.path.join(t, "include"), os.path.join(t, "include", "torch", "csrc", "api", "include"),
+                os.path.join(rocm, "include"), sysconfig.get_paths()["include"]]
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-Wno-unused-parameter", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *[f for i in includes for f in ("-isystem", i)], src, "-o", TORCH_SO_PATH, f"-L{os.path.join(t, 'lib')}",
+           "-ltorch_python", "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip", f"-L{LIB_DIR}", "-lxq_hip",
+           "-Wl,-rpath,$ORIGIN"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"g++ failed for {src}:\n{r.stderr}")
+    if r.stderr.strip():
+        sys.stderr.write(r.stderr)
+
+
 def build(force: bool = False, jobs: int = 8) -> str:
     os.makedirs(LIB_DIR, exist_ok=True)
     os.makedirs(OBJ_DIR, exist_ok=True)
@@ -50,6 +76,7 @@ def build(force: bool = False, jobs: int = 8) -> str:
                            capture_output=True, text=True)
         if r.returncode != 0:
             raise RuntimeError(f"link failed:\n{r.stderr}")
+    _build_torch(force)
     return SO_PATH
 
 

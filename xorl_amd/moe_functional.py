@@ -19,6 +19,7 @@ import torch
 from torch import Tensor
 
 from . import _C
+from ._native import native
 from .functional import _CODE_TO_DT, _DT_TO_CODE, QuantWeight, _as_2d, _r_pad
 
 
@@ -353,10 +354,13 @@ class MoeExpertsQLoRAFunction(torch.autograd.Function):
 DECODE_PATH = True
 
 
-def _moe_infer(hidden: Tensor, routing_weights: Tensor, selected_experts: Tensor, factors, banks, num_experts: int,
-               scaling: float, swiglu_limit: float) -> Optional[Tensor]:
-    """xq_grouped_fwd_infer: the forward for a handful of tokens when nothing is differentiated (block-fp8 banks; the
-    touched experts' bytes streamed once).  None where the call does not fit it."""
+def _moe_infer(hidden: Tensor, routing_weights: Tensor, selected_experts: Tensor, factors=None, banks=None, num_experts: int = 0,
+               scaling: float = 0.0, swiglu_limit: float = 0.0, module=None) -> Optional[Tensor]:
+    """xq_grouped_fwd_infer: the forward for a handful of tokens when nothing is differentiated (the touched experts'
+    bytes streamed once).  None where the call does not fit it.  With `module` (an expert module) its banks and factors
+    are read by the compiled host path."""
+    if module is not None:
+        return native().moe(module, hidden, routing_weights, selected_experts, True)
     qg, qu, qd = banks
     H = qg.rows
     if (hidden.dtype != torch.bfloat16 or not hidden.is_cuda or hidden.numel() == 0 or hidden.shape[-1] != H

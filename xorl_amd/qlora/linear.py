@@ -31,6 +31,7 @@ from torch import Tensor
 
 from .. import _C
 from .. import quantize as Q
+from .._native import native
 from ..functional import MAX_FUSED_RANK, QuantWeight, qlora_linear
 
 
@@ -407,6 +408,10 @@ class QLoRALinear(LoraModule, nn.Module):
 
     # ------------------------------------------------------------------ forward
     def forward(self, x: Tensor) -> Tensor:
+        if not torch.compiler.is_compiling():
+            y = native().linear(self, x)
+            if y is not None:
+                return y
         if self.enable_aqn and self.training:
             return self._forward_with_noise(x)
         return qlora_linear(x, self._forward_quant_weight(), self.lora_A, self.lora_B, self.active_r,
@@ -798,6 +803,10 @@ def qlora_mlp_forward(gate_proj: "QLoRALinear", up_proj: "QLoRALinear", down_pro
     one; both ways give the same rounding points."""
     from ..functional import qlora_mlp, qlora_mlp_infer, silu_and_mul
 
+    if not torch.compiler.is_compiling():
+        y = native().mlp(gate_proj, up_proj, down_proj, x)
+        if y is not None:
+            return y
     mods = (gate_proj, up_proj, down_proj)
     if not all(isinstance(m, QLoRALinear) for m in mods):
         return down_proj(silu_and_mul(gate_proj(x), up_proj(x)))
@@ -855,6 +864,10 @@ def qlora_linears_forward(modules, x: Tensor) -> list:
     from .._C import XQ_LINEAR_MULTI_MAX
 
     mods = list(modules)
+    if not torch.compiler.is_compiling():
+        ys = native().linears(mods, x)
+        if ys is not None:
+            return ys
     needs_grad = torch.is_grad_enabled() and (x.requires_grad or any(
         p.requires_grad for m in mods for p in (m.lora_A, m.lora_B, m.bias) if p is not None))
     one_call = (1 < len(mods) <= XQ_LINEAR_MULTI_MAX and not needs_grad and not torch.compiler.is_compiling()

@@ -18,7 +18,9 @@ import torch.nn as nn
 from torch import Tensor
 
 from .. import _C
+from .. import moe_functional as MF
 from .. import quantize as Q
+from .._native import native
 from ..functional import QuantWeight
 from ..moe_functional import moe_experts_qlora_ep_compute, moe_experts_qlora_forward
 from .linear import LoraModule
@@ -317,6 +319,12 @@ class QLoRAMoeExperts(LoraModule, nn.Module):
         """Routed call (hidden [T, H], routing_weights / selected_experts [T, top-k]) or, with `expert_idx`, the
         MLP of one expert on the rows passed (moe_experts.py:576-620, :738-786): `expert_idx` is a global index,
         an expert that lives on another rank returns zeros."""
+        if expert_idx is None and MF.DECODE_PATH and MF.READ_ROUTED_ROWS_IN_PLACE and not torch.compiler.is_compiling():
+            out = MF._moe_infer(hidden_states, routing_weights, selected_experts, module=self)
+            if out is None:
+                out = native().moe(self, hidden_states, routing_weights, selected_experts, False)
+            if out is not None:
+                return out
         if self.moe_implementation == "eager" and expert_idx is None:
             raise ValueError("moe_implementation='eager' calls the experts one at a time: pass expert_idx")
         if expert_idx is not None:

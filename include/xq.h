@@ -526,6 +526,25 @@ int xq_grouped_fwd_infer(const xq_weight* gate, const xq_weight* up, const xq_we
                          const int32_t* selected, int32_t topk, void* out, int64_t ld_out, void* workspace,
                          int64_t workspace_bytes, void* stream);
 
+/* ---- encoding a weight ----------------------------------------------------------
+ * x [rows, cols] (bf16 or fp32, contiguous, 16-byte aligned) -> codes and scales of `format`, byte for byte what the
+ * reference quantizers emit (ops/quantize/int4_quantize.py:12-41, nvfp4_quantize.py:25-60,102-154, nf4_quantize.py:20-56,
+ * block_fp8_gkn_quantize.py:40-121 and the _gkn forms), in one pass over x (nvfp4 without a known tensor amax: one pass and
+ * a small launch over the blocks' maxima).
+ *   FLAT: groups along the contiguous elements (4-bit: a power of two, 16 .. 1024, dividing rows * cols); codes rows*cols/2
+ *         bytes, scales one per group in element order;
+ *   GKN:  groups down the rows (16, 32 or 64, dividing rows), byte (k, n) holds rows 2k and 2k + 1 of column n; cols % 8 == 0;
+ *   block-fp8 ignores the layout: 128 x 128 blocks, partial at the edges, cols % 8 == 0, fp32 scales;
+ *         amax_scale multiplies the block maximum (1 otherwise).
+ * scale_dtype: nvfp4 E4M3, nf4 and block-fp8 F32; int4 F32 for the reference's rule or BF16 for the symmetric one
+ * (scale = bf16(absmax / 7), codes rne(x / scale) + 8).  nvfp4: global_amax (one device float, may be NULL: the amax of x),
+ * global_scale (one device float, written).  workspace: xq_quantize_workspace_bytes() bytes, 256-byte aligned (nvfp4 with
+ * global_amax == NULL only). */
+int64_t xq_quantize_workspace_bytes(int format, int64_t rows, int64_t cols);
+int xq_quantize(int format, int layout, const void* x, int x_dtype, int64_t rows, int64_t cols, int32_t group, float amax_scale,
+                const float* global_amax, void* codes, void* scales, int scale_dtype, float* global_scale, void* workspace,
+                int64_t workspace_bytes, void* stream);
+
 /* ---- the dense SwiGLU MLP in two calls ---------------------------------------
  * y = down(silu(gate(x)) * up(x)) over three QLoRA linears: the reference's Qwen3MLP.forward
  * (models/transformers/qwen3/modeling_qwen3.py:60-81) on QLoRALinear modules (qlora/modules/linear.py:369-385) with

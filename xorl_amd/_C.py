@@ -93,6 +93,9 @@ _SIGNATURES = {
     "xq_profile_enable": (_INT, [_INT]),
     "xq_profile_collect": (_INT, [_P, _P, _P]),
     "xq_decode": (_INT, [_W, _P, _INT, _P]),
+    "xq_quantize_workspace_bytes": (_I64, [_INT, _I64, _I64]),
+    # format, layout, x, x_dtype, rows, cols, group, amax_scale, global_amax, codes, scales, scale_dtype, global_scale, ws, ws_bytes, stream
+    "xq_quantize": (_INT, [_INT, _INT, _P, _INT, _I64, _I64, _I32, _F, _P, _P, _P, _INT, _P, _P, _I64, _P]),
     "xq_linear_workspace_bytes": (_I64, [_I64, _I64, _I64, _INT]),
     # w, x, ldx, M, A, B, lora_dtype, r, scaling, bias, y, ldy, su_out, ws, ws_bytes, stream
     "xq_linear_fwd": (_INT, [_W, _P, _I64, _I64, _P, _P, _INT, _INT, _F, _P, _P, _I64, _P, _P, _I64, _P]),

@@ -467,7 +467,7 @@ class BlockFP8QLoRALinear(QLoRALinear):
         self.reset_lora_parameters()
 
     def _quantize_and_store(self, w: Tensor, global_amax: Optional[Tensor] = None) -> None:
-        fp8_w, scales = Q.block_fp8_quantize_gkn(w.float().contiguous(), self.quant_group_size)
+        fp8_w, scales = Q.block_fp8_quantize_gkn(w.contiguous(), self.quant_group_size)
         self._write_packed_weight(self._to_uint8(fp8_w))
         self._scale_dtypes = {"weight_block_scales": scales.dtype}
         self.weight_block_scales = self._to_uint8(scales)
@@ -667,7 +667,7 @@ class Int4QLoRALinear(QLoRALinear):
 
     def _quantize_and_store(self, w: Tensor, global_amax: Optional[Tensor] = None) -> None:
         fn = Q.int4_quantize_sym if self.symmetric else Q.int4_quantize
-        packed, scales = fn(w.float(), self.quant_group_size)
+        packed, scales = fn(w, self.quant_group_size)
         self._write_packed_weight(self._to_uint8(packed))
         self._scale_dtypes = {"weight_scales": scales.dtype}
         self.weight_scales = self._to_uint8(scales)

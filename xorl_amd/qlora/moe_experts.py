@@ -407,7 +407,7 @@ class BlockFP8QLoRAMoeExperts(QLoRAMoeExperts):
         self.reset_lora_parameters()
 
     def _quantize_2d(self, w: Tensor, global_amax=None):
-        fp8, scales = Q.block_fp8_quantize_gkn(w.float().contiguous(), 128)
+        fp8, scales = Q.block_fp8_quantize_gkn(w.contiguous(), 128)
         return self._to_uint8(fp8), {"weight_block_scales": (self._to_uint8(scales), scales.dtype)}
 
     def _dequantize_2d(self, packed: Tensor, scales_dict: dict, K: int, N: int) -> Tensor:

@@ -1,9 +1,10 @@
 """Codec functions with the names and signatures of ``xorl.ops.quantize``.
 
 Dequantizers launch the HIP decode kernels (``xq_decode``); they are bit-exact
-with the reference's Triton decoders.  Quantizers run once at load / merge
-time, are plain torch ops (IEEE fp32) on whatever device the tensor lives on,
-and restate the reference quantizers' arithmetic:
+with the reference's Triton decoders.  Quantizers of a GPU tensor in one of the
+formats' own group sizes run as one pass of ``xq_quantize``; on the CPU, and for
+other group sizes and element types, they are plain torch ops (IEEE fp32).  Both
+restate the reference quantizers' arithmetic and emit the same bytes:
 
   int4_quantize[_gkn]        ops/quantize/int4_quantize.py:97-110, int4_gkn_quantize.py:137-173
   int4_quantize_sym          the symmetric absmax/7 bf16-scale rule (not in the reference)
@@ -101,8 +102,36 @@ def block_fp8_dequantize_gkn(x: Tensor, s: Tensor, block_size: int = 128,
 
 
 # ---------------------------------------------------------------------------
-# quantizers (torch, load-time)
+# quantizers
 # ---------------------------------------------------------------------------
+def _on_hip(x: Tensor, group: int, gkn: bool) -> bool:
+    """Whether xq_quantize takes this tensor (4-bit formats)."""
+    if not x.is_cuda or torch.compiler.is_compiling() or x.dtype not in (torch.bfloat16, torch.float32) or x.numel() == 0:
+        return False
+    if not x.is_contiguous() or x.data_ptr() % 16 or group < 16 or group & (group - 1) or group > (64 if gkn else 1024):
+        return False
+    return (x.shape[0] % group == 0 and x.shape[1] % 8 == 0) if gkn else x.numel() % group == 0
+
+
+def _quantize_hip(fmt: str, gkn: bool, x: Tensor, group: int, scale_shape, scale_dtype: torch.dtype, amax_scale: float = 1.0,
+                  global_amax: Optional[Tensor] = None):
+    """xq_quantize -> (flat code bytes, scales, global scale [1] or None)."""
+    L, dev, f = _C.lib(), x.device, _C.FORMATS[fmt]
+    rows, cols = x.shape
+    codes = torch.empty(rows * cols if fmt == "block_fp8" else rows * cols // 2, dtype=torch.uint8, device=dev)
+    scales = torch.empty(scale_shape, dtype=scale_dtype, device=dev)
+    gs = torch.empty(1, dtype=torch.float32, device=dev) if fmt == "nvfp4" else None
+    if global_amax is not None:
+        global_amax = global_amax.to(device=dev, dtype=torch.float32).reshape(1)
+    ws_bytes = L.xq_quantize_workspace_bytes(f, rows, cols) if global_amax is None else 0
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
+    _C.check(L.xq_quantize(f, _C.XQ_LAYOUT_GKN if gkn else _C.XQ_LAYOUT_FLAT, x.data_ptr(),
+                           _C.XQ_DT_F32 if x.dtype == torch.float32 else _C.XQ_DT_BF16, rows, cols, group, amax_scale, _C.ptr(global_amax),
+                           codes.data_ptr(), scales.data_ptr(), _C._SCALE_DT[scale_dtype], _C.ptr(gs), _C.ptr(ws), ws_bytes,
+                           _C.stream_ptr(dev)))
+    return codes, scales, gs
+
+
 def _pack_nibbles_last(q: Tensor) -> Tensor:
     """[..., 2n] codes -> [..., n] bytes, even element in the low nibble."""
     q = q.to(torch.uint8)
@@ -146,6 +175,8 @@ def nf4_quantize(x: Tensor, group_size: int = 64) -> Tuple[Tensor, Tensor]:
     assert x.dim() == 2
     n = x.numel()
     assert n % group_size == 0 and group_size % 2 == 0
+    if _on_hip(x, group_size, False):
+        return _quantize_hip("nf4", False, x, group_size, (n // group_size,), torch.float32)[:2]
     xf = x.float().reshape(n // group_size, group_size)
     scale = xf.abs().amax(-1).clamp_min(1e-12)
     norm = (xf * (_const(scale, 1.0) / scale).unsqueeze(-1)).clamp_(-1.0, 1.0)
@@ -159,6 +190,9 @@ def nf4_quantize_gkn(x: Tensor, group_size: int = 64) -> Tuple[Tensor, Tensor]:
     assert x.dim() == 2
     K, N = x.shape
     assert K % group_size == 0 and group_size % 2 == 0
+    if _on_hip(x, group_size, True):
+        codes, scale, _ = _quantize_hip("nf4", True, x, group_size, (K // group_size, N), torch.float32)
+        return codes.reshape(K // 2, N), scale
     xf = x.float().reshape(K // group_size, group_size, N)
     scale = xf.abs().amax(1).clamp_min(1e-12)
     norm = (xf * (_const(scale, 1.0) / scale).unsqueeze(1)).clamp_(-1.0, 1.0)
@@ -171,6 +205,9 @@ def int4_quantize(x: Tensor, group_size: int = -1) -> Tuple[Tensor, Tensor]:
     M, K = x.shape
     gs = K if group_size == -1 else group_size
     assert K % gs == 0 and gs % 2 == 0
+    if _on_hip(x, gs, False):
+        codes, scale, _ = _quantize_hip("int4", False, x, gs, (M, K // gs), torch.float32)
+        return codes.reshape(M, K // 2), scale
     xf = x.float().reshape(M, K // gs, gs)
     scale = xf.abs().amax(-1).clamp_min(1e-12) * torch.tensor(2.0 / 15.0, dtype=torch.float32, device=x.device)
     inv = _const(scale, 1.0) / scale
@@ -183,6 +220,9 @@ def int4_quantize_gkn(x: Tensor, group_size: int = -1) -> Tuple[Tensor, Tensor]:
     K, N = x.shape
     gs = K if group_size == -1 else group_size
     assert K % gs == 0 and gs % 2 == 0
+    if _on_hip(x, gs, True):
+        codes, scale, _ = _quantize_hip("int4", True, x, gs, (K // gs, N), torch.float32)
+        return codes.reshape(K // 2, N), scale
     xf = x.float().reshape(K // gs, gs, N)
     scale = xf.abs().amax(1).clamp_min(1e-12) * torch.tensor(2.0 / 15.0, dtype=torch.float32, device=x.device)
     inv = _const(scale, 1.0) / scale
@@ -194,6 +234,9 @@ def int4_quantize_sym(x: Tensor, group_size: int = 128) -> Tuple[Tensor, Tensor]
     """Symmetric int4: scale = bf16(absmax/7), q = clamp(rne(w/scale), -7, 7) + 8."""
     M, K = x.shape
     assert K % group_size == 0
+    if _on_hip(x, group_size, False):
+        codes, scale, _ = _quantize_hip("int4", False, x, group_size, (M, K // group_size), torch.bfloat16)
+        return codes.reshape(M, K // 2), scale
     xf = x.float().reshape(M, K // group_size, group_size)
     scale = (xf.abs().amax(-1) / _const(xf, 7.0)).to(torch.bfloat16)
     sf = scale.float().unsqueeze(-1)
@@ -227,6 +270,8 @@ def nvfp4_quantize(x: Tensor, block_size: int = 16, global_amax: Optional[Tensor
     assert x.dim() == 2
     n = x.numel()
     assert n % block_size == 0 and block_size % 2 == 0
+    if block_size == 16 and _on_hip(x, 16, False):
+        return _quantize_hip("nvfp4", False, x, 16, (n // 16,), torch.float8_e4m3fn, global_amax=global_amax)
     xf = x.float().reshape(-1, block_size)
     amax = xf.abs().amax(-1).clamp_min(1e-12)
     scaled = (xf * (_const(amax, 6.0) / amax).unsqueeze(-1)).clamp_(-6.0, 6.0)
@@ -240,6 +285,9 @@ def nvfp4_quantize_gkn(x: Tensor, block_size: int = 16, global_amax: Optional[Te
     assert x.dim() == 2
     K, N = x.shape
     assert K % block_size == 0 and block_size % 2 == 0
+    if block_size == 16 and _on_hip(x, 16, True):
+        codes, bs, g = _quantize_hip("nvfp4", True, x, 16, (K // 16, N), torch.float8_e4m3fn, global_amax=global_amax)
+        return codes.reshape(K // 2, N), bs, g
     xf = x.float().reshape(K // block_size, block_size, N)
     amax = xf.abs().amax(1).clamp_min(1e-12)
     scaled = (xf * (_const(amax, 6.0) / amax).unsqueeze(1)).clamp_(-6.0, 6.0)
@@ -255,6 +303,10 @@ def block_fp8_quantize_gkn(x: Tensor, block_size: int = 128, amax_scale: float =
         raise ValueError(f"amax_scale must be positive, got {amax_scale}")
     R, Cc = x.shape
     bs = block_size
+    if (bs == 128 and x.is_cuda and x.dtype in (torch.bfloat16, torch.float32) and x.numel() and Cc % 8 == 0 and R < 128 * 65536
+            and x.data_ptr() % 16 == 0 and not torch.compiler.is_compiling()):
+        codes, s, _ = _quantize_hip("block_fp8", False, x, 128, (-(-R // 128), -(-Cc // 128)), torch.float32, amax_scale=amax_scale)
+        return codes.view(torch.float8_e4m3fn).reshape(R, Cc), s
     pr, pc = (-R) % bs, (-Cc) % bs
     xf = x.float()
     if pr or pc:

@@ -1,0 +1,51 @@
+"""GPU parity of the streaming skinny forward (M <= 64, two launches): joint forwards give the bits of the separate ones,
+and the gate + up launch whose epilogue writes h = SwiGLU gives the MLP of the oracle."""
+
+import pytest
+import torch
+
+from oracle import recipe as R
+from tests.util_cases import close, gen, make_dense_module
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture
+def stream_only(hip_device):
+    """the two-launch organisation at every M"""
+    from xorl_amd._C import lib
+    lib().xq_set_skinny_one_launch(0)
+    yield
+    lib().xq_set_skinny_one_launch(1)
+
+
+@pytest.mark.parametrize("M", [1, 3, 16, 17, 33, 64])
+@pytest.mark.parametrize("fmt,H,I,r", [
+    ("int4", 1152, 1152, 16),      # 9 steps of 128: uneven splits
+    ("nvfp4", 2944, 1088, 40),     # 68 row tiles: an uneven row block, a cut column block; ranks in three units of 16, the last one cut
+    ("block_fp8", 1024, 1280, 64), # the widest low-rank term
+    ("nf4", 1024, 1536, 1),
+])
+def test_joint_launches(stream_only, hip_device, fmt, H, I, r, M):
+    from xorl_amd.functional import silu_and_mul
+    from xorl_amd.qlora import qlora_linears_forward, qlora_mlp_forward
+
+    bias = fmt in ("int4", "nf4")
+    mods, w_ref = {}, {}
+    for i, (k, (N, K)) in enumerate({"gate": (I, H), "up": (I, H), "down": (H, I)}.items()):
+        mods[k], w_ref[k] = make_dense_module(fmt, N, K, r, 2 * r, seed=M + 10 * i, device=hip_device, bias=bias)
+    g, u, d = mods["gate"], mods["up"], mods["down"]
+    x = gen((M, H), 1.0, 71, torch.bfloat16)
+    xd = x.to(hip_device)
+    with torch.no_grad():
+        yg, yu = g(xd), u(xd)
+        for a, b in zip(qlora_linears_forward([g, u], xd), (yg, yu)):
+            assert torch.equal(a, b)
+        y = qlora_mlp_forward(g, u, d, xd)
+        assert torch.equal(qlora_mlp_forward(g, u, d, xd), y)
+        ref = d(silu_and_mul(yg, yu))
+    close(y.cpu(), ref.cpu().double(), 1e-2)
+    if not bias:
+        loras = {k: (m.lora_A.detach().cpu(), m.lora_B.detach().cpu()) for k, m in mods.items()}
+        ex = R.mlp_fwd_bwd_exact(x, w_ref["gate"], w_ref["up"], w_ref["down"], loras, g.scaling, torch.zeros(M, H, dtype=torch.bfloat16))
+        close(y.cpu(), ex["y"], 1e-2)

@@ -612,14 +612,15 @@ extern "C" int xq_linear_fwd_swiglu(const xq_weight* w, const void* x, int64_t l
 }
 
 extern "C" int64_t xq_linear_fwd_multi_workspace_bytes(const xq_linear_job* jobs, int n_jobs, int64_t M) {
-    int64_t need = 256 * 8;
+    int64_t need = 256 * 8, joint = 0;
     if (!jobs) return need;
     for (int i = 0; i < n_jobs; ++i) {
         if (!jobs[i].w) continue;
         const int64_t b = xq_linear_workspace_bytes(M, jobs[i].w->rows, jobs[i].w->cols, jobs[i].r);
         if (b > need) need = b;
+        if (M <= 64) joint += skinny_workspace_bytes(M, jobs[i].w->rows, jobs[i].w->cols, r_pad_of(jobs[i].r));   // side by side in a joint launch
     }
-    return need;
+    return need > joint ? need : joint;
 }
 
 extern "C" int xq_linear_fwd_multi(const xq_linear_job* jobs, int n_jobs, const void* x, int64_t ldx, int64_t M, int lora_dtype,
@@ -665,6 +666,28 @@ extern "C" int xq_linear_fwd_multi(const xq_linear_job* jobs, int n_jobs, const 
                 XQ_CHECK_LAUNCH("skinny forwards");
                 return XQ_OK;
             }
+        }
+    }
+    // decode shapes outside the whole-row kernel: every forward in one streaming launch and one epilogue
+    if (g_skinny_enabled && n_jobs > 1 && M <= 16 && ldx % 8 == 0 && xq_aligned(x, 16)) {
+        SkinnyRowsJob sj[XQ_LINEAR_MULTI_MAX];
+        double bytes = 2.0 * M * jobs[0].w->cols;
+        bool ok = true;
+        for (int i = 0; i < n_jobs; ++i) {
+            const xq_weight* w = jobs[i].w;
+            sj[i] = SkinnyRowsJob{w, jobs[i].lora_A, jobs[i].lora_B, jobs[i].r, jobs[i].scaling, (const bf16_t*)jobs[i].bias_bf16,
+                                  (bf16_t*)jobs[i].y, jobs[i].ldy};
+            ok = ok && skinny_takes_stream(w, M, jobs[i].lora_A, jobs[i].lora_B, lora_dtype, jobs[i].r);
+            bytes += (double)xq_packed_bytes_per_expert(w) + (double)xq_scale_bytes_per_expert(w) + 2.0 * M * w->rows +
+                     4.0 * jobs[i].r * (w->cols + w->rows);
+        }
+        if (ok && skinny_stream_multi_supported(sj, n_jobs, M)) {
+            const bool timed = xq_profile_mark_begin(stream, bytes);
+            const int rc = launch_skinny_stream(sj, n_jobs, false, (const bf16_t*)x, ldx, M, lora_dtype, workspace, stream);
+            if (timed) xq_profile_mark_end(stream);
+            if (rc) return rc;
+            XQ_CHECK_LAUNCH("skinny forwards");
+            return XQ_OK;
         }
     }
     // otherwise one after the other (the workspace is reused: the launches are ordered by the stream)

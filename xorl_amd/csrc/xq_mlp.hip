@@ -9,6 +9,7 @@
 //             and the two A gradients come from one pass over x.
 // Other formats (and shapes the fused forms do not take) run the same program launch by launch.
 #include "xq_lora.h"
+#include "xq_skinny.h"
 #include <atomic>
 #include <stdlib.h>
 
@@ -211,7 +212,12 @@ extern "C" int xq_mlp_fwd(const xq_weight* gate, const xq_weight* up, const xq_w
 // ---- forward only: nothing is kept for a backward, so each projection is free to take the kernel that suits the row
 // count -- at decode sizes the weight-streaming kernels (gate and up as one launch), not the tile kernels above
 static int64_t infer_linear_ws(int64_t M, int64_t H, int64_t I, int r) {
-    const int64_t a = xq_linear_workspace_bytes(M, I, H, r), b = xq_linear_workspace_bytes(M, H, I, r);
+    const int64_t b = xq_linear_workspace_bytes(M, H, I, r);
+    int64_t a = xq_linear_workspace_bytes(M, I, H, r);
+    if (M <= 64) {                                // gate and up side by side in a joint launch
+        const int64_t joint = 2 * skinny_workspace_bytes(M, I, H, r_pad_of(r));
+        a = a > joint ? a : joint;
+    }
     return al256((a > b ? a : b) > 2048 ? (a > b ? a : b) : 2048);
 }
 
@@ -243,6 +249,18 @@ extern "C" int xq_mlp_fwd_infer(const xq_weight* gate, const xq_weight* up, cons
         {gate, lora->A[0], lora->B[0], d.r, lora->scaling, lora->bias[0], gu, 2 * d.I},
         {up, lora->A[1], lora->B[1], d.r, lora->scaling, lora->bias[1], gu + d.I, 2 * d.I},
     };
+    // up to 64 rows outside the one-launch kernel: gate and up in one streaming launch whose epilogue writes h
+    const SkinnyRowsJob gu_jobs[2] = {
+        {gate, lora->A[0], lora->B[0], d.r, lora->scaling, (const bf16_t*)lora->bias[0], h, d.I},
+        {up, lora->A[1], lora->B[1], d.r, lora->scaling, (const bf16_t*)lora->bias[1], h, d.I},
+    };
+    if (skinny_takes_stream(gate, M, lora->A[0], lora->B[0], lora->dtype, d.r) && skinny_takes_stream(up, M, lora->A[1], lora->B[1], lora->dtype, d.r) &&
+        ldx % 8 == 0 && xq_aligned(x, 16) && skinny_stream_multi_supported(gu_jobs, 2, M)) {
+        if ((rc = launch_skinny_stream(gu_jobs, 2, true, (const bf16_t*)x, ldx, M, lora->dtype, ws, (hipStream_t)stream))) return rc;
+        XQ_CHECK_LAUNCH(who);
+        return xq_linear_fwd(down, h, d.I, M, lora->A[2], lora->B[2], lora->dtype, d.r, lora->scaling, lora->bias[2], y, ldy, nullptr, ws,
+                             ws_bytes, stream);
+    }
     if ((rc = xq_linear_fwd_multi(jobs, 2, x, ldx, M, lora->dtype, ws, ws_bytes, stream))) return rc;
     if ((rc = xq_silu_mul_fwd(gu, gu + d.I, 2 * d.I, nullptr, h, d.I, M, d.I, stream))) return rc;
     return xq_linear_fwd(down, h, d.I, M, lora->A[2], lora->B[2], lora->dtype, d.r, lora->scaling, lora->bias[2], y, ldy, nullptr, ws,

@@ -2,28 +2,33 @@
 //
 //   y[M, N] = x[M, K] . deq(W)^T + bias + s * (x . A^T) . B^T          (W FLAT [N, K])
 //
-// Every byte of the packed weight is read from HBM exactly once, decoded in registers to the exact bf16
-// value of the reference decoder and fed to v_mfma_f32_32x32x16_bf16 against x fragments.  Two launches per
-// forward, no atomics, no zeroed buffers, fixed summation orders (deterministic):
+// Every byte of the packed weight is read from HBM exactly once, decoded in registers to the exact bf16 value of the
+// reference decoder and fed to v_mfma_f32_16x16x32_bf16 against x fragments.  Two launches for up to four forwards on one x
+// (q + k + v, gate + up), no atomics, no zeroed buffers, fixed summation orders (deterministic):
 //
-//  1. skinny_split_kernel: a grid of (128-row block) x (K split) tiles.  A block's four waves own 32 weight
-//     rows each and the same K range of at most four 128-element chunks.  Every load is unconditional and
-//     issued ahead of its use with exactly counted waits: the x slice first, then the weight chunks as a
-//     stream with two chunks in flight (a chunk's registers are requested again once it has been multiplied),
-//     and the number of K splits is chosen so that the whole grid is resident at once (four blocks per CU at
-//     M <= 16, three above).  Weight loads are coalesced (a load instruction covers whole rows of a chunk) and
-//     reach the MFMA layout through a wave-private XOR-swizzled LDS slab; x goes through LDS once per block
-//     and is shared by the four waves: the whole [rows, K range] slice up to 32 rows, chunk by chunk (all 64
-//     rows of 128 elements, two buffers) above, so that a weight chunk is decoded once whatever M is.  Each
-//     block stores its fp32 partial tile to part[split][M][N]; the first row of blocks carries no weight rows
-//     and computes the low-rank intermediate su = x . A^T for one K split each.
-//  2. skinny_epilogue_kernel: sums the splits in order, adds bias and s * su . B^T in fp32 and rounds once
-//     to bf16.
+//  1. stream_split_kernel: a grid of (row block) x (K split) tiles, one block of 8 waves per compute unit (two at M <= 32).
+//     A wave owns 16 RT weight rows and streams them straight from memory into registers in the MFMA operand layout (a load
+//     instruction takes 64 contiguous bytes of each of 16 rows), D steps of 128 elements in flight; rows are not shared
+//     between waves, so the weight never passes through LDS.  x does: the block's whole slice [16 MT rows][K range] comes by
+//     direct-to-LDS loads at the start (one barrier) and every wave reads its fragments from there -- the slice costs
+//     1 / (8 RT) of what it would if each 16 weight rows fetched it, and nothing in the stream waits for a barrier.
+//     The tile's sides balance what a block moves beside its weights, x (2 M K_b bytes) and fp32 partial sums
+//     (8 M R_b bytes, written and read back): few, tall blocks for wide weights.  The blocks of `splits` leading tiles
+//     compute the low-rank parts x . A^T of one split each.
+//  2. stream_epilogue_kernel: sums the splits in order, adds bias and s * su . B^T in fp32 and rounds once to bf16; for gate
+//     and up of an MLP it writes h = SwiGLU(gate, up) of the two rounded outputs instead.
 //
-// Measured per forward on an MI355X, launches back to back (block_fp8, r = 16): 4096->12288 (48 MiB) 15.6 us
-// at M = 1, 21 us at M = 32, 31 us at M = 64; 4096->1024 (4 MiB) 8 us at M = 1.  A kernel that only reads
-// the 48 MiB takes 8-9 us.  (M <= 16 normally takes the one-launch kernel of xq_skinny_rows.hip instead.)
+// The split of K depends on a forward's own shape only: a joint launch gives the bits of the separate ones.
+//
+// What bounds it: at 64 rows the vector units (the 25 instructions that decode and feed one fragment of 8 weights a lane) and the
+// matrix units, not memory: gate | up of 4096 -> 2 x 12288 in int4 takes 26 us (30 MB fetched) and its epilogue 13 us, half of
+// which is the trip of the partial sums; at few rows the fixed costs of two dependent launches.  Forward of a SwiGLU MLP, us,
+// against one that fetched x per 16 weight rows and ran gate, up, SwiGLU and down as separate launches:
+//     int4  4096/12288, r 16: M = 24 62 -> 49, M = 64 90 -> 65      int4  2944/7808, r 32: M = 1 64 -> 34, M = 64 70 -> 49
+//     fp8   4096/12288, r 16: M = 64 92 -> 76                       nvfp4 2944/7808, r 32: M = 1 71 -> 36
 #include <stdlib.h>
+
+#include <atomic>
 
 #include "xq_common.h"
 #include "xq_lora.h"
@@ -31,623 +36,578 @@
 
 namespace xq {
 
-struct SkinnyArgs {
-    const bf16_t* x;
-    int64_t ldx;
-    int32_t M, N, K;
+constexpr int kStreamJobs = 4;
+constexpr int kStreamWaves = 8;          // of a block
+
+struct StreamJob {
     const uint8_t* packed;
     const uint8_t* scales;
     const float* global_scale;
-    int32_t group, scale_dtype;
-    int32_t splits;            // K splits
-    int32_t su_blocks;         // leading grid rows (0 or 1) whose blocks compute the su part of their split
-    int32_t chunk_q, chunk_rem; // 128-element chunks per split: chunk_q, one more in the first chunk_rem splits
-    int32_t xp;                // LDS row pitch of the x slice in bf16 elements (longest split + 8)
-    float* partial;            // [splits][M][N]
-    float* su_part;            // [splits * 4][M][r_pad]
     const void* lora_A;        // [r, K] fp32 or bf16
+    float* partial;            // [splits][M][N]
+    float* su_part;            // [K / 128][M][r_pad]
+    int32_t N, group, scale_dtype;
+    int32_t splits;            // K splits
+    int32_t chunk_q, chunk_rem; // 128-element steps per split: chunk_q, one more in the first chunk_rem splits
+    int32_t row_blocks;
     int32_t lora_f32, r, r_pad;
 };
-
-struct SkinnyEpiArgs {
-    const float* partial;
-    const float* su_part;
-    int32_t splits, su_parts, M, N;
-    const void* lora_B;        // [N, r] fp32 or bf16
-    int32_t lora_f32, r, r_pad;
-    float su_scale;
-    const bf16_t* bias;
-    bf16_t* y;
-    int64_t ldy;
+struct StreamBatch {
+    StreamJob job[kStreamJobs];
 };
 
-// One block = 128 weight rows x one K split (or, for the leading su blocks, the x . A^T part of one split).
-// MR = 16, 32 or 64 bounds M.  Up to 32 rows the split's whole x slice is staged in LDS once; at MR = 64 weight
-// blocks take x one 128-element chunk at a time (all 64 rows, two LDS buffers), so that a weight chunk is decoded
-// once and multiplied into both halves of the rows, and three blocks still fit a CU.  (The su blocks at MR = 64
-// stage their x rows 32 at a time.)
-// The arguments that the first loads need are the leading scalars: the hardware hands a kernel's first 14 argument dwords
-// to each wave in registers (where the platform supports it; otherwise they are fetched like the rest), so those loads do
-// not wait for a round trip to the argument block.  fmt_bits = group | scale_dtype << 24, split_bits = splits |
-// su_blocks << 16, chunk_bits = chunk_q | chunk_rem << 16; `rest` carries the other fields (its copies of these are unused).
-template <int FMT, int MR, int NCH>
-__global__ void __launch_bounds__(256, MR == 16 ? 4 : 3)
-skinny_split_kernel(const bf16_t* x_, int32_t ldx_, int32_t M_, int32_t N_, int32_t K_, const uint8_t* packed_, const uint8_t* scales_,
-                    int32_t fmt_bits, int32_t split_bits, int32_t chunk_bits, int32_t xp_, SkinnyArgs rest) {
-    constexpr int TR = MR < 32 ? MR : 32;              // x rows staged at a time
-    constexpr int NPASS = MR / TR;
-    SkinnyArgs g = rest;
-    g.x = x_; g.ldx = ldx_; g.M = M_; g.N = N_; g.K = K_; g.packed = packed_; g.scales = scales_;
-    g.group = fmt_bits & 0xFFFFFF; g.scale_dtype = fmt_bits >> 24;
-    g.splits = split_bits & 0xFFFF; g.su_blocks = split_bits >> 16;
-    g.chunk_q = chunk_bits & 0xFFFF; g.chunk_rem = chunk_bits >> 16;
-    g.xp = xp_;
-    // The other arguments are pinned in scalar registers in one go once the first loads are out (left to the compiler,
-    // argument loads are placed lazily, each batch with its own wait).
-    auto pin_rest = [&]() {
-        asm volatile("" ::"s"(g.global_scale), "s"(g.partial), "s"(g.su_part), "s"(g.lora_A), "s"(g.lora_f32), "s"(g.r), "s"(g.r_pad));
-    };
+// how a lane gets the scales of its codes: with the step's weights (one or two words), four steps' bf16 scales of int4
+// groups of 128 in one load, four steps' 8 scale bytes dealt over the row's four lanes, per fragment at use, or (block-fp8)
+// one value per row tile and step from registers
+enum { kScFp8 = 0, kScInt4Window = 1, kScDealt = 2, kScStep = 3, kScUse = 4 };
+
+// element offset of fragment (j, q) within a 128-element step: what lane q of a row holds after its loads (block-fp8: two
+// loads of 16 bytes, 64 apart; 4-bit: one load of 16 bytes), so that a load instruction covers 64 contiguous bytes of a row
+template <int FMT>
+__device__ __forceinline__ int frag_k(int j, int q) {
+    return FMT == XQ_FMT_FP8 ? (j >> 1) * 64 + q * 16 + (j & 1) * 8 : q * 32 + j * 8;
+}
+
+template <int FMT, int SC, int MT, int RT>
+__global__ void __launch_bounds__(64 * kStreamWaves, MT == 4 || RT == 3 ? 2 : 4)
+stream_split_kernel(const bf16_t* x, int32_t ldx, int32_t M, int32_t K, int32_t first1, int32_t first2, int32_t first3, StreamBatch b) {
+    constexpr int EB = FMT == XQ_FMT_FP8 ? 1 : 2;                 // elements per byte
+    constexpr int NL = FMT == XQ_FMT_FP8 ? 2 : 1;                 // 16-byte loads per lane, row tile and step
+    constexpr int D = FMT == XQ_FMT_FP8 && RT > 1 ? 2 : 4;        // steps in flight
+    constexpr int NS = SC != kScStep ? 0 : FMT == XQ_FMT_NVFP4 ? 2 : 1;   // scale words per row tile that travel with a step
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    bf16_t* xs = (bf16_t*)smem;                                  // [min(M, 32) rows][xp]; fragment rows past M read row 0:
-    const int XP = g.xp;                                         // they feed only output columns >= M, which are never stored
-    const int xrows = g.M < 32 ? g.M : 32;
-    const int tid = threadIdx.x, lane = tid & 63;
+    const int tid = threadIdx.x, lane = tid & 63, q = lane >> 4, lr = lane & 15;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int fr = lane & 31, fh = lane >> 5;
-    constexpr int EB = FMT == XQ_FMT_FP8 ? 1 : 2;      // elements per byte
-    constexpr int NLOAD = FMT == XQ_FMT_FP8 ? 4 : 2;   // 16-byte loads per lane per 128-k chunk
-    constexpr int NSC = FMT == XQ_FMT_NVFP4 ? 4 : FMT == XQ_FMT_NF4 ? 2 : 1;   // scale registers per chunk
-
-    // grid: x = K split, y = 128-row block, preceded by one row of su blocks when there is a low-rank term
-    const int split = blockIdx.x;
-    const bool su_block = (int)blockIdx.y < g.su_blocks;
-    const int rb = su_block ? 0 : (int)blockIdx.y - g.su_blocks;
-    // the first `chunk_rem` splits hold chunk_q + 1 chunks of 128 elements, the others chunk_q (no divisions here:
-    // nothing is in flight until the loads below are issued)
+    const int bx = blockIdx.x;
+    const int ji = (bx >= first1 ? 1 : 0) + (bx >= first2 ? 1 : 0) + (bx >= first3 ? 1 : 0);
+    const StreamJob& g = b.job[ji];
+    const int at = bx - (ji == 0 ? 0 : ji == 1 ? first1 : ji == 2 ? first2 : first3);
+    const int split = at % g.splits, rb = at / g.splits;
     const int c_begin = split * g.chunk_q + (split < g.chunk_rem ? split : g.chunk_rem);
-    const int nch = g.chunk_q + (split < g.chunk_rem ? 1 : 0);   // 1 .. NCH (the launcher guarantees it)
-    const int c_end = c_begin + nch;
+    const int n_steps = g.chunk_q + (split < g.chunk_rem ? 1 : 0);
     const int k_begin = c_begin << 7;
 
-    // ---- x slice [rows of pass h][nch*128]: coalesced 16-byte pieces, row-major over the block's threads.  Every
-    // load of this kernel is unconditional (rows and chunks past the end are clamped onto valid ones and their
-    // data ignored): with no branches between the loads and their uses the waits count exactly, so the x slice
-    // is staged and each weight chunk decoded while the chunks behind it are still in flight.
-    // Thread t owns column piece t % (NCH*16) of rows t / (NCH*16) + i * (16/NCH); pieces past the split's own
-    // nch*16 columns (a split shorter than NCH chunks) are loaded clamped and never stored.
-    constexpr int XL = TR * NCH / 16;                            // pieces per thread: TR rows x NCH*16 / 256
-    constexpr int CPR = NCH * 16, RSTEP = 16 / NCH;              // column pieces per row, rows per step
-    const int ppr = nch << 4;                                    // pieces of a row that belong to this split
-    u32x4 xr[XL];
-    auto load_x = [&](int h, int t) {
-        const int col = t % CPR < ppr ? t % CPR : ppr - 1;
-#pragma unroll
-        for (int i = 0; i < XL; ++i) {
-            const int row = h * 32 + t / CPR + i * RSTEP;
-            xr[i] = *(const u32x4*)(g.x + (int64_t)(row < g.M ? row : g.M - 1) * g.ldx + k_begin + col * 8);
+    // ---- x slice -> LDS: [step][16 MT rows][16 pieces of 8 elements].  Piece (j, q) of row m lies at (4 j + q) ^ (m & 15): the
+    // 16 lanes that one LDS pass of a fragment read serves fall on 16 different pieces.  Lane l of a load instruction lands at
+    // piece l % 16 of row l / 16 of its four rows, so the swizzle is applied to the address it fetches.  (rows past M repeat the
+    // last one: their products are never stored)
+    {
+        const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem;
+        const int total = n_steps * MT * 4;
+        for (int i = wave; i < total; i += kStreamWaves) {
+            const int step = i / (MT * 4), m = (i % (MT * 4)) * 4 + (lane >> 4);
+            const int col = (lane & 15) ^ (m & 15);
+            const bf16_t* src = x + (int64_t)(m < M ? m : M - 1) * ldx + k_begin + step * 128 + frag_k<FMT>(col >> 2, col & 3);
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+                         :: "s"(__builtin_amdgcn_readfirstlane(lds0 + i * 1024)), "v"(src) : "memory");
         }
-    };
-    // block barrier on LDS traffic only: __syncthreads() would also wait for every weight load in flight
-    auto lds_barrier = [&]() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
-    auto stage_x = [&](int h, int t) {
-        const int col = t % CPR;
-#pragma unroll
-        for (int i = 0; i < XL; ++i) {
-            const int row = t / CPR + i * RSTEP;
-            if (col < ppr && h * 32 + row < g.M) *(u32x4*)(xs + row * XP + col * 8) = xr[i];
-        }
-        lds_barrier();
-    };
-    // a value the optimiser cannot see through: index arithmetic derived from it inside a loop is redone per
-    // iteration instead of being hoisted into (and spilling) registers held across the whole loop
-    auto opaque = [](int v) { asm volatile("" : "+v"(v)); return v; };
-    if (MR < 64 || su_block) load_x(0, tid);      // (weight blocks at MR = 64 take x chunk by chunk, see below)
-
-    if (su_block) {
-        pin_rest();
-        // su part of this split, D[rank][m] (ranks >= r are zero): wave w takes the k16 steps t = w, w+4, ...; the
-        // four sums meet in LDS (behind the x slice) in wave order.  The factor rows are fetched with unconditional
-        // 16-byte loads (rows and steps past the end clamped, their values masked), the first rank tile's together
-        // with the x slice.
-        const int steps = nch << 3;
-        float* out = g.su_part + (int64_t)split * g.M * g.r_pad;
-        float* red = (float*)(smem + (size_t)xrows * XP * 2);      // [4 waves][16 regs][64 lanes]
-        u32x4 ar[2 * NCH][2];
-        auto load_a = [&](int jt) {
-            const int rrow = jt * 32 + fr;
-            const int64_t base = (int64_t)(rrow < g.r ? rrow : 0) * g.K + k_begin + fh * 8;
-#pragma unroll
-            for (int u = 0; u < 2 * NCH; ++u) {
-                const int t = wave + 4 * u < steps ? wave + 4 * u : steps - 1;
-                if (g.lora_f32) {
-                    ar[u][0] = *(const u32x4*)((const float*)g.lora_A + base + t * 16);
-                    ar[u][1] = *(const u32x4*)((const float*)g.lora_A + base + t * 16 + 4);
-                } else {
-                    ar[u][0] = *(const u32x4*)((const bf16_t*)g.lora_A + base + t * 16);
-                }
-            }
-        };
-        load_a(0);
-        for (int jt = 0; jt < ((g.r_pad + 31) >> 5); ++jt) {
-            if (jt > 0) load_a(jt);
-            const bool rvalid = jt * 32 + fr < g.r;
-            bf16x8 af[2 * NCH];
-#pragma unroll
-            for (int u = 0; u < 2 * NCH; ++u) {
-                u32x4 v = ar[u][0];
-                if (g.lora_f32) {
-                    v = u32x4{pack_bf16x2(__uint_as_float(ar[u][0][0]), __uint_as_float(ar[u][0][1])),
-                              pack_bf16x2(__uint_as_float(ar[u][0][2]), __uint_as_float(ar[u][0][3])),
-                              pack_bf16x2(__uint_as_float(ar[u][1][0]), __uint_as_float(ar[u][1][1])),
-                              pack_bf16x2(__uint_as_float(ar[u][1][2]), __uint_as_float(ar[u][1][3]))};
-                }
-                if (!rvalid || wave + 4 * u >= steps) v = u32x4{0, 0, 0, 0};
-                af[u] = __builtin_bit_cast(bf16x8, v);
-            }
-#pragma unroll 1
-            for (int h = 0; h < NPASS; ++h) {
-                if (h * 32 < g.M) {
-                    // the x tile in LDS is current only for a single pass and the first rank tile
-                    if (NPASS > 1 || jt == 0) {
-                        if (h > 0 || jt > 0) load_x(h, tid);       // earlier reads of the tile are behind two barriers
-                        stage_x(h, tid);
-                    }
-                    const int xrow = h * 32 + fr < g.M ? fr : 0;
-                    f32x16 sacc;
-#pragma unroll
-                    for (int q = 0; q < 16; ++q) sacc[q] = 0.0f;
-#pragma unroll
-                    for (int u = 0; u < 2 * NCH; ++u) {
-                        const int t = wave + 4 * u;
-                        if (t < steps) {
-                            const bf16x8 xf = *(const bf16x8*)(xs + xrow * XP + t * 16 + fh * 8);
-                            sacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[u], xf, sacc, 0, 0, 0);
-                        }
-                    }
-                    __syncthreads();   // the previous sums have been read
-#pragma unroll
-                    for (int q = 0; q < 16; ++q) red[(wave * 16 + q) * 64 + lane] = sacc[q];
-                    __syncthreads();
-                    // wave w sums register quad w of every lane: ranks jt*32 + 8w + 4*fh .. +3 of row m = 32h + fr
-                    f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-                    for (int ww = 0; ww < 4; ++ww)
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) v[e] += red[(ww * 16 + wave * 4 + e) * 64 + lane];
-                    const int j0 = jt * 32 + 8 * wave + 4 * fh, m = h * 32 + fr;
-                    if (m < g.M && j0 < g.r_pad) *(f32x4*)(out + (int64_t)m * g.r_pad + j0) = v;
-                }
-            }
-        }
-        return;
     }
+    // fragment (m tile, j) of step s: row lr of the tile
+    int xo[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) xo[j] = lr * 256 + (((4 * j + q) ^ lr) << 4);
+    const auto x_frag = [&](int s, int mt, int j) {
+        return *(const bf16x8*)(smem + (s * MT + mt) * 4096 + xo[j]);
+    };
 
-    // ---- the block's whole weight tile -> registers, fetched coalesced: a load instruction covers whole
-    // rows of the chunk (lane l: row l / PPR of the instruction's rows, 16-byte piece l % PPR)
-    constexpr int PPR = FMT == XQ_FMT_FP8 ? 8 : 4;     // 16-byte pieces per row per 128-k chunk
-    constexpr int RPI = 64 / PPR;                      // rows per load instruction
-    const int lrow = lane / PPR, lpiece = lane % PPR;
-    const int nbase = rb * 128 + wave * 32;
-    int n = nbase + fr;                                 // the row this lane feeds to the MFMA
-    n = n < g.N ? n : g.N - 1;
-    // A single pass over the weights (M <= 32) takes them as a short stream: two chunks in flight, a chunk's registers
-    // refilled with the chunk two further on once it has been multiplied.  A CU accepts loads only as fast as memory
-    // returns them, and with every chunk of its 12 to 16 waves requested at once the waves placed last start late and
-    // have all their decode work left when the stream ends.  (M > 32 takes the same stream with x chunk by chunk, below.)
-    constexpr int DC = NCH > 2 ? 2 : NCH;
-    u32x4 w[DC][NLOAD];
-    uint32_t sc[DC][NSC];
-    const bool int4_small_group = FMT == XQ_FMT_INT4 && (g.group & 127) != 0;   // looked up per 8 elements at use
-    const uint8_t* wp[NLOAD];
+    // ---- the low-rank parts: units of (step, 16 ranks) dealt over the waves of the split's blocks, the first of them over the
+    // blocks.  A wave's first unit is requested here, behind the x slice and ahead of the weights, and multiplied before the
+    // stream starts; D[rank][m] of one step goes out as it is (ranks >= r: whatever row 0 gives, never read).
+    const int rank_tiles = g.r_pad >> 4, units = n_steps * rank_tiles, unit0 = rb + g.row_blocks * wave;
+    const auto unit_base = [&](int u, int us) {
+        const int row = (u - us * rank_tiles) * 16 + lr;
+        return (int64_t)(row < g.r ? row : 0) * K + k_begin + us * 128;
+    };
+    const auto multiply_unit = [&](int u, int us, const u32x4 (&a)[4]) {
+        const int jt = u - us * rank_tiles;
+        f32x4 sacc[MT];
 #pragma unroll
-    for (int i = 0; i < NLOAD; ++i) {
-        int nl = nbase + RPI * i + lrow;
-        nl = nl < g.N ? nl : g.N - 1;
-        wp[i] = g.packed + ((int64_t)nl * g.K) / EB + lpiece * 16;
+        for (int mt = 0; mt < MT; ++mt) sacc[mt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+                sacc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a[j]), x_frag(us, mt, j), sacc[mt], 0, 0, 0);
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+            const int m = mt * 16 + lr;
+            if (m < M) *(f32x4*)(g.su_part + ((int64_t)(c_begin + us) * M + m) * g.r_pad + jt * 16 + q * 4) = sacc[mt];
+        }
+    };
+    f32x4 araw[8];                                                 // fp32 factors (bf16 ones are not requested ahead)
+    const auto load_unit = [&](int u) {
+        const float* p = (const float*)g.lora_A + unit_base(u, u / rank_tiles);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            araw[2 * j] = *(const f32x4*)(p + frag_k<FMT>(j, q));
+            araw[2 * j + 1] = *(const f32x4*)(p + frag_k<FMT>(j, q) + 4);
+        }
+    };
+    if (g.lora_f32 && unit0 < units) load_unit(unit0);
+
+    // ---- this wave's rows: tiles of 16 (N % 16 == 0: a tile is all in or all out; one past the end repeats the last)
+    const int row0 = (rb * kStreamWaves + wave) * (16 * RT);
+    const uint8_t* wp[RT];
+    int64_t srow[RT];                                              // SC-dependent: the row's scales
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+        const int n = (row0 + rt * 16 < g.N ? row0 + rt * 16 : g.N - 16) + lr;
+        wp[rt] = g.packed + ((int64_t)n * K + k_begin) / EB + q * 16;
+        srow[rt] = (int64_t)n * K + k_begin;
     }
-    auto load_chunk = [&](int c_) {
-        {
-            const int c = c_ % DC;
-            const int cc = c_begin + c_ < c_end ? c_begin + c_ : c_end - 1;
+    u32x4 w[D][RT][NL];
+    uint32_t sw[D][RT][NS > 0 ? NS : 1];
+    const auto load_step = [&](int slot, int s_) {
+        const int s = s_ < n_steps ? s_ : n_steps - 1;
 #pragma unroll
-            for (int i = 0; i < NLOAD; ++i) w[c][i] = *(const u32x4*)(wp[i] + (int64_t)cc * (128 / EB));
-            if (FMT == XQ_FMT_FP8) sc[c][0] = ((const uint32_t*)g.scales)[(n >> 7) * ((g.K + 127) >> 7) + cc];
-            else if (FMT == XQ_FMT_INT4) {
-                const int64_t si = int4_small_group ? 0 : ((int64_t)n * g.K + cc * 128) / g.group;
-                sc[c][0] = g.scale_dtype == XQ_SCALE_F32 ? ((const uint32_t*)g.scales)[si] : ((const uint16_t*)g.scales)[si];
-            } else if (FMT == XQ_FMT_NF4) {
-                const u32x2 t = *(const u32x2*)((const uint32_t*)g.scales + (((int64_t)n * g.K + cc * 128) >> 6));   // fp32, group 64
-                sc[c][0] = t[0];
-                sc[c][1] = t[1];
-            } else {
-                const int64_t si = ((int64_t)n * g.K + cc * 128) >> 4;   // the 8 block scales of this row's chunk
-                if (g.scale_dtype == XQ_SCALE_E4M3) {
-                    const u32x2 t = *(const u32x2*)(g.scales + si);
-                    sc[c][0] = t[0];
-                    sc[c][1] = t[1];
-                } else {
+        for (int rt = 0; rt < RT; ++rt) {
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) sc[c][j] = ((const uint32_t*)g.scales)[si + 2 * j + fh];   // this lane's four
-                }
+            for (int i = 0; i < NL; ++i) w[slot][rt][i] = *(const u32x4*)(wp[rt] + (int64_t)s * (128 / EB) + i * 64);
+            if constexpr (SC == kScStep && FMT == XQ_FMT_NVFP4) {
+                const u32x2 v = *(const u32x2*)((const uint32_t*)g.scales + ((srow[rt] + s * 128 + q * 32) >> 4));
+                sw[slot][rt][0] = v[0];
+                sw[slot][rt][1] = v[1];
+            } else if constexpr (SC == kScStep) {
+                const int64_t si = (srow[rt] + s * 128 + q * 32) / g.group;
+                sw[slot][rt][0] = g.scale_dtype == XQ_SCALE_F32 ? ((const uint32_t*)g.scales)[si] : (uint32_t)((const uint16_t*)g.scales)[si] << 16;
             }
         }
     };
-    // M > 32: all 64 x rows of one 128-element chunk at a time, requested just ahead of the chunk's weights (thread t: piece
-    // t % 16 of rows t / 16 + 16 i), so that a chunk is decoded once and multiplied into both halves of the rows
-    u32x4 xcr[4];                                           // one chunk's pieces: requested again as soon as they are in LDS
-    auto load_xc = [&](int c_) {
-        const int cc = c_begin + c_ < c_end ? c_begin + c_ : c_end - 1;
+    // windows of four steps (a window that would pass the row's end starts earlier; kScDealt clamps step by step)
+    typedef u32x2 u32x2_a2 __attribute__((aligned(2)));
+    u32x2 win[RT], win_next[RT];
+    const int row_steps = K >> 7;
+    const auto load_window = [&](u32x2* dst, int s0) {
+        if constexpr (SC == kScInt4Window) {
+            const int c = c_begin + s0 < row_steps - 4 ? c_begin + s0 : row_steps - 4;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int row = (tid >> 4) + 16 * i;
-            xcr[i] = *(const u32x4*)(g.x + (int64_t)(row < g.M ? row : g.M - 1) * g.ldx + cc * 128 + (tid & 15) * 8);
+            for (int rt = 0; rt < RT; ++rt)
+                dst[rt] = *(const u32x2_a2*)((const uint16_t*)g.scales + ((srow[rt] - k_begin) >> 7) + c);
+        } else if constexpr (SC == kScDealt) {
+            const int c = c_begin + s0 + q < row_steps - 1 ? c_begin + s0 + q : row_steps - 1;
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) dst[rt] = *(const u32x2*)(g.scales + ((srow[rt] - k_begin) >> 7) * 8 + (int64_t)c * 8);
         }
     };
+    float ts[RT];                                                  // block-fp8: lane l holds the scale of step l
+    if constexpr (SC == kScFp8) {
 #pragma unroll
-    for (int c = 0; c < DC; ++c) {
-        if (MR == 64 && c == 0) load_xc(0);
-        load_chunk(c);
+        for (int rt = 0; rt < RT; ++rt) {
+            const int n = row0 + rt * 16 < g.N ? row0 + rt * 16 : g.N - 16;
+            ts[rt] = ((const float*)g.scales)[(int64_t)(n >> 7) * ((K + 127) >> 7) + c_begin + (lane < n_steps ? lane : n_steps - 1)];
+        }
     }
-    pin_rest();
-
-    // ---- decode + multiply: D[n][m] += deq(W)[n][k] x[m][k].  Each chunk's slab goes through a wave-private LDS
-    // staging area (XOR-swizzled 16-byte pieces: writes and fragment reads are conflict free) to reach the
-    // MFMA layout: lane (row fr, half fh) reads piece 2u+fh of its row for the k16 steps 2u and 2u+1, i.e. step
-    // t = 2u+v covers k = 32u + 16*fh + 8v .. +7 of the chunk; the x fragments use the same map.  LDS operations
-    // of one wave execute in order, so the slab is reused chunk after chunk without barriers.
+    load_window(win, 0);
+#pragma unroll
+    for (int d = 0; d < D; ++d) load_step(d, d);
     const float gsc = FMT == XQ_FMT_NVFP4 ? g.global_scale[0] : 1.0f;
-    unsigned char* wst = smem + (size_t)xrows * XP * 2 + wave * (PPR * 32 * 16);
-    float* nf4_lds = (float*)(smem + (size_t)xrows * XP * 2 + 4 * 4096);    // 16 levels behind the slabs
-    if (FMT == XQ_FMT_NF4 && tid < 16) nf4_lds[tid] = kNf4Level[tid];        // ordered before its use by stage_x's barrier
-    if constexpr (MR == 64) {
-        constexpr int CXP = 128 + 8;                            // row pitch of an x chunk in LDS, bf16 elements
-        bf16_t* xc = (bf16_t*)smem;                             // [2 buffers][64 rows][CXP]
-        unsigned char* wst2 = smem + 2 * 64 * CXP * 2 + wave * (PPR * 32 * 16);
-        float* nf4_2 = (float*)(smem + 2 * 64 * CXP * 2 + 4 * 4096);
-        if (FMT == XQ_FMT_NF4 && tid < 16) nf4_2[tid] = kNf4Level[tid];     // ordered before its use by the first chunk's barrier
-        const int xrow0 = fr < g.M ? fr : 0, xrow1 = 32 + fr < g.M ? 32 + fr : 0;
-        f32x16 acc0, acc1;
+    float* nf4_lds = (float*)(smem + n_steps * MT * 4096);
+    if (FMT == XQ_FMT_NF4 && tid < 16) nf4_lds[tid] = kNf4Level[tid];
+
+    // the x slice is older than every load above: it has landed when no more than those are outstanding
+    constexpr int kAhead = D * RT * (NL + (NS ? 1 : 0));
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kAhead < 63 ? kAhead : 63) : "memory");
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (g.lora_f32) {
+#pragma unroll 1
+        for (int u = unit0; u < units; u += g.row_blocks * kStreamWaves) {      // (more than one only for narrow weights of high rank)
+            if (u != unit0) load_unit(u);
+            u32x4 a[4];
 #pragma unroll
-        for (int q = 0; q < 16; ++q) acc0[q] = acc1[q] = 0.0f;
-#pragma unroll
-        for (int c = 0; c < NCH; ++c) {
-            if (c < nch) {      // block-uniform
-                // x chunk -> buffer c & 1.  Behind this barrier every wave is also done with chunk c - 1, whose buffer
-                // the chunk after this one will overwrite.
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int row = (tid >> 4) + 16 * i;
-                    if (row < g.M) *(u32x4*)(xc + ((c & 1) * 64 + row) * CXP + (tid & 15) * 8) = xcr[i];
-                }
-                if (c + 1 < NCH) load_xc(c + 1);
-                lds_barrier();
-#pragma unroll
-                for (int i = 0; i < NLOAD; ++i) {
-                    const int rl = RPI * i + lrow;
-                    const int sw = FMT == XQ_FMT_FP8 ? (rl >> 1) & 7 : (rl >> 2) & 3;
-                    *(u32x4*)(wst2 + (rl * PPR + (lpiece ^ sw)) * 16) = w[c % DC][i];
-                }
-                __builtin_amdgcn_wave_barrier();
-                const int kc = (c_begin + c) * 128;
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    uint32_t f[4];
-                    if (FMT == XQ_FMT_FP8) {
-                        const u32x4 t = *(const u32x4*)(wst2 + (fr * 8 + ((2 * u + fh) ^ ((fr >> 1) & 7))) * 16);
-                        f[0] = t[0]; f[1] = t[1]; f[2] = t[2]; f[3] = t[3];
-                    } else {
-                        const u32x2 t = *(const u32x2*)(wst2 + (fr * 4 + (u ^ ((fr >> 2) & 3))) * 16 + fh * 8);
-                        f[0] = t[0]; f[1] = t[1];
-                    }
-#pragma unroll
-                    for (int v = 0; v < 2; ++v) {
-                        bf16x8 wf;
-                        if (FMT == XQ_FMT_FP8) {
-                            wf = decode8<FMT>(f[2 * v], f[2 * v + 1], __uint_as_float(sc[c % DC][0]), 0.0f);
-                        } else if (FMT == XQ_FMT_NF4) {
-                            wf = decode8<FMT>(f[v], 0u, __uint_as_float(sc[c % DC][u >> 1]), 0.0f, nf4_2);
-                        } else if (FMT == XQ_FMT_INT4) {
-                            float sv;
-                            if (int4_small_group) sv = load_scale(g.scales, ((int64_t)n * g.K + kc + 32 * u + 16 * fh + 8 * v) / g.group, g.scale_dtype);
-                            else sv = g.scale_dtype == XQ_SCALE_F32 ? __uint_as_float(sc[c % DC][0]) : __uint_as_float(sc[c % DC][0] << 16);
-                            wf = decode8<FMT>(f[v], 0u, sv, -8.0f * sv);
-                        } else {
-                            float sv;
-                            if (g.scale_dtype == XQ_SCALE_E4M3) sv = e4m3_to_f32((uint8_t)(sc[c % DC][u >> 1] >> (8 * (2 * (u & 1) + fh))));
-                            else sv = __uint_as_float(sc[c % DC][u]);
-                            wf = decode8<FMT>(f[v], 0u, sv * gsc, 0.0f);
-                        }
-                        const bf16_t* xb = xc + (c & 1) * 64 * CXP + 32 * u + 16 * fh + 8 * v;
-                        acc0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf, *(const bf16x8*)(xb + xrow0 * CXP), acc0, 0, 0, 0);
-                        acc1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf, *(const bf16x8*)(xb + xrow1 * CXP), acc1, 0, 0, 0);
-                    }
-                }
-                __builtin_amdgcn_wave_barrier();
-            }
-            if (c + DC < NCH) load_chunk(c + DC);
+            for (int j = 0; j < 4; ++j)
+                a[j] = u32x4{pack_bf16x2(araw[2 * j][0], araw[2 * j][1]), pack_bf16x2(araw[2 * j][2], araw[2 * j][3]),
+                             pack_bf16x2(araw[2 * j + 1][0], araw[2 * j + 1][1]), pack_bf16x2(araw[2 * j + 1][2], araw[2 * j + 1][3])};
+            multiply_unit(u, u / rank_tiles, a);
         }
-        float* out = g.partial + (int64_t)split * g.M * g.N;
+    } else {
+#pragma unroll 1
+        for (int u = unit0; u < units; u += g.row_blocks * kStreamWaves) {
+            const bf16_t* p = (const bf16_t*)g.lora_A + unit_base(u, u / rank_tiles);
+            u32x4 a[4];
 #pragma unroll
-        for (int hh = 0; hh < 2; ++hh) {
-            const int m = hh * 32 + fr;
-#pragma unroll
-            for (int q4 = 0; q4 < 4; ++q4) {
-                const int nn = nbase + 8 * q4 + 4 * fh;
-                if (m < g.M && nn < g.N) {
-                    const f32x16& a = hh ? acc1 : acc0;
-                    *(f32x4*)(out + (int64_t)m * g.N + nn) = f32x4{a[q4 * 4], a[q4 * 4 + 1], a[q4 * 4 + 2], a[q4 * 4 + 3]};
-                }
-            }
+            for (int j = 0; j < 4; ++j) a[j] = *(const u32x4*)(p + frag_k<FMT>(j, q));
+            multiply_unit(u, u / rank_tiles, a);
         }
-        return;
     }
+
+    f32x4 acc[RT][MT];
 #pragma unroll
-    for (int h = 0; h < NPASS; ++h) {
-        if (h * 32 < g.M) {
-            const int tv = h > 0 ? opaque(tid) : tid;
-            if (h > 0) {
-                lds_barrier();                         // every wave has read its fragments of the previous pass
-                load_x(h, tv);
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) acc[rt][mt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    uint32_t sx[SC == kScDealt ? RT : 1][4];
+    // register k of lane row r <- what lane row k fetched for lane row r
+    const auto deal = [&]() {
+        if constexpr (SC == kScDealt) {
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) {
+                const u32x2 d = win[rt];
+                const uint32_t x0 = d[0], x1 = FMT == XQ_FMT_NF4 ? d[0] : d[0] >> 16, x2 = d[1], x3 = FMT == XQ_FMT_NF4 ? d[1] : d[1] >> 16;
+                const auto p02 = __builtin_amdgcn_permlane32_swap(x0, x2, false, false);
+                const auto p13 = __builtin_amdgcn_permlane32_swap(x1, x3, false, false);
+                const auto q01 = __builtin_amdgcn_permlane16_swap(p02[0], p13[0], false, false);
+                const auto q23 = __builtin_amdgcn_permlane16_swap(p02[1], p13[1], false, false);
+                sx[rt][0] = q01[0]; sx[rt][1] = q01[1]; sx[rt][2] = q23[0]; sx[rt][3] = q23[1];
             }
-            stage_x(h, tv);
-            const int lv = tv & 63, fr = lv & 31, fh = lv >> 5, lrow = lv / PPR, lpiece = lv % PPR;
-            const int xrow = h * 32 + fr < g.M ? fr : 0;
-            f32x16 acc;
+        }
+    };
+    const auto multiply = [&](int slot, int s, int ph) {              // ph: the step's place in its window
+        float s0[RT], s1[RT];
 #pragma unroll
-            for (int q = 0; q < 16; ++q) acc[q] = 0.0f;
+        for (int rt = 0; rt < RT; ++rt) {
+            s1[rt] = 0.0f;
+            if constexpr (SC == kScFp8) {
+                s0[rt] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ts[rt]), s));
+            } else if constexpr (SC == kScInt4Window) {
+                const int c = c_begin + s - ph;
+                const int i = ph + (c < row_steps - 4 ? 0 : c - (row_steps - 4));          // uniform, 0 .. 3
+                const uint64_t v = (uint64_t)win[rt][1] << 32 | win[rt][0];
+                s0[rt] = __uint_as_float((uint32_t)(v >> (16 * i)) << 16);
+                s1[rt] = -8.0f * s0[rt];
+            } else if constexpr (SC == kScDealt && FMT == XQ_FMT_NF4) {
+                s0[rt] = __uint_as_float(sx[rt][ph]);
+            } else if constexpr (SC == kScDealt) {
+                s0[rt] = e4m3_to_f32((uint8_t)sx[rt][ph]) * gsc;
+                s1[rt] = e4m3_to_f32((uint8_t)(sx[rt][ph] >> 8)) * gsc;
+            } else if constexpr (SC == kScStep && FMT == XQ_FMT_NVFP4) {
+                s0[rt] = __uint_as_float(sw[slot][rt][0]) * gsc;
+                s1[rt] = __uint_as_float(sw[slot][rt][NS > 1 ? 1 : 0]) * gsc;
+            } else if constexpr (SC == kScStep) {
+                s0[rt] = __uint_as_float(sw[slot][rt][0]);
+                s1[rt] = -8.0f * s0[rt];
+            }
+        }
+        bf16x8 xf[2][MT];                                          // fragments are read one j ahead
 #pragma unroll
-            for (int c = 0; c < NCH; ++c) {
-                if (c < nch) {
+        for (int mt = 0; mt < MT; ++mt) xf[0][mt] = x_frag(s, mt, 0);
 #pragma unroll
-                    for (int i = 0; i < NLOAD; ++i) {
-                        const int rl = RPI * i + lrow;
-                        const int sw = FMT == XQ_FMT_FP8 ? (rl >> 1) & 7 : (rl >> 2) & 3;
-                        *(u32x4*)(wst + (rl * PPR + (lpiece ^ sw)) * 16) = w[c % DC][i];
-                    }
-                    __builtin_amdgcn_wave_barrier();
-                    const int kc = (c_begin + c) * 128;
+        for (int j = 0; j < 4; ++j) {
+            if (j < 3) {
 #pragma unroll
-                    for (int u = 0; u < 4; ++u) {
-                        uint32_t f[4];
-                        if (FMT == XQ_FMT_FP8) {
-                            const u32x4 t = *(const u32x4*)(wst + (fr * 8 + ((2 * u + fh) ^ ((fr >> 1) & 7))) * 16);
-                            f[0] = t[0]; f[1] = t[1]; f[2] = t[2]; f[3] = t[3];
-                        } else {
-                            const u32x2 t = *(const u32x2*)(wst + (fr * 4 + (u ^ ((fr >> 2) & 3))) * 16 + fh * 8);
-                            f[0] = t[0]; f[1] = t[1];
-                        }
+                for (int mt = 0; mt < MT; ++mt) xf[(j + 1) & 1][mt] = x_frag(s, mt, j + 1);
+            }
 #pragma unroll
-                        for (int v = 0; v < 2; ++v) {
-                            bf16x8 wf;
-                            if (FMT == XQ_FMT_FP8) {
-                                wf = decode8<FMT>(f[2 * v], f[2 * v + 1], __uint_as_float(sc[c % DC][0]), 0.0f);
-                            } else if (FMT == XQ_FMT_NF4) {
-                                wf = decode8<FMT>(f[v], 0u, __uint_as_float(sc[c % DC][u >> 1]), 0.0f, nf4_lds);   // group 64: k = 32u + ..
-                            } else if (FMT == XQ_FMT_INT4) {
-                                float sv;
-                                if (int4_small_group) sv = load_scale(g.scales, ((int64_t)n * g.K + kc + 32 * u + 16 * fh + 8 * v) / g.group, g.scale_dtype);
-                                else sv = g.scale_dtype == XQ_SCALE_F32 ? __uint_as_float(sc[c % DC][0]) : __uint_as_float(sc[c % DC][0] << 16);
-                                wf = decode8<FMT>(f[v], 0u, sv, -8.0f * sv);
-                            } else {
-                                float sv;   // block scale 2u + fh of the chunk
-                                if (g.scale_dtype == XQ_SCALE_E4M3) sv = e4m3_to_f32((uint8_t)(sc[c % DC][u >> 1] >> (8 * (2 * (u & 1) + fh))));
-                                else sv = __uint_as_float(sc[c % DC][u]);
-                                wf = decode8<FMT>(f[v], 0u, sv * gsc, 0.0f);
-                            }
-                            const bf16x8 xf = *(const bf16x8*)(xs + xrow * XP + c * 128 + 32 * u + 16 * fh + 8 * v);
-                            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf, xf, acc, 0, 0, 0);
-                        }
-                    }
-                    __builtin_amdgcn_wave_barrier();
+            for (int rt = 0; rt < RT; ++rt) {
+                bf16x8 wf;
+                if constexpr (FMT == XQ_FMT_FP8) {
+                    const u32x4 v = w[slot][rt][j >> 1];
+                    wf = decode8<FMT>(v[2 * (j & 1)], v[2 * (j & 1) + 1], s0[rt], 0.0f);
+                } else if constexpr (FMT == XQ_FMT_NVFP4) {
+                    wf = decode8<FMT>(w[slot][rt][0][j], 0u, j < 2 ? s0[rt] : s1[rt], 0.0f);
+                } else if constexpr (SC == kScUse) {
+                    const float sv = load_scale(g.scales, (srow[rt] + s * 128 + q * 32 + j * 8) / g.group, g.scale_dtype);
+                    wf = decode8<FMT>(w[slot][rt][0][j], 0u, sv, -8.0f * sv);
+                } else {
+                    wf = decode8<FMT>(w[slot][rt][0][j], 0u, s0[rt], s1[rt], nf4_lds);
                 }
-                if (c + DC < NCH) load_chunk(c + DC);      // this chunk's registers are free (single pass only: DC == NCH otherwise)
-            }
-            // fp32 partial tile: lane (m = 32h + fr) holds 4 consecutive weight rows per register quad
-            float* out = g.partial + (int64_t)split * g.M * g.N;
-            const int m = h * 32 + fr;
 #pragma unroll
-            for (int q4 = 0; q4 < 4; ++q4) {
-                const int nn = nbase + 8 * q4 + 4 * fh;
-                if (m < g.M && nn < g.N)   // N % 16 == 0: groups of 4 columns are all in or all out
-                    *(f32x4*)(out + (int64_t)m * g.N + nn) = f32x4{acc[q4 * 4], acc[q4 * 4 + 1], acc[q4 * 4 + 2], acc[q4 * 4 + 3]};
+                for (int mt = 0; mt < MT; ++mt) acc[rt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf, xf[j & 1][mt], acc[rt][mt], 0, 0, 0);
+            }
+        }
+    };
+
+    // ---- the stream: whole groups of four steps, each step's registers requested again once it has been multiplied, then the
+    // remaining steps from what is in flight.  No branch lies between a load and its use, so every wait counts exactly.
+    int s = 0;
+#pragma unroll 1
+    for (; s + 4 <= n_steps; s += 4) {
+        deal();
+        load_window(win_next, s + 4);
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+            multiply(d % D, s + d, d);
+            // (left alone the compiler decodes ahead, collects the products at the end and requests late)
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt) asm volatile("" : "+v"(acc[rt][mt]));
+            load_step(d % D, s + d + D);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr (SC == kScInt4Window || SC == kScDealt) {
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) win[rt] = win_next[rt];
+        }
+    }
+    if (s < n_steps) {
+        deal();
+        multiply(0, s, 0);
+        if constexpr (D == 2) load_step(0, s + 2);
+        if (s + 1 < n_steps) multiply(1, s + 1, 1);
+        if (s + 2 < n_steps) multiply(2 % D, s + 2, 2);
+    }
+
+    // ---- fp32 partial tile: lane (m = lr, quarter q) holds 4 consecutive weight rows of each row tile
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+        const int n = row0 + rt * 16;
+        if (n < g.N) {
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) {
+                const int m = mt * 16 + lr;
+                if (m < M) *(f32x4*)(g.partial + ((int64_t)split * M + m) * g.N + n + q * 4) = acc[rt][mt];
             }
         }
     }
 }
 
-// y[m][n..n+3] = sum_s part[s][m][n..] + bias + su_scale * sum_j su[m][j] * B[n][j], su = sum of the su parts.
-// One wave per output row m (up to four rows per block), a lane per 4 consecutive columns.  The block's 256 B rows
-// (64 B per output column and 16 ranks: twice the bytes of a row's partial tiles of eight splits) are fetched once,
-// coalesced, and shared by its waves through LDS.  Loads are unconditional (indices past the end are clamped, their
-// values masked to zero or never stored) and the first batch of each kind is issued before anything is waited for,
-// so that the B rows, partial tiles and su parts are all in flight together.  Every sum runs in a fixed order:
-// parts p = g, g+4, ... per lane group g, then the four groups; splits ascending.
-// RT = 16-rank tiles of the low-rank term (0 = none); VEC = B is fp32 with r % 4 == 0 (16-byte row pieces).
-// (leading scalars: see skinny_split_kernel; count_bits = splits | su_parts << 16, rank_bits = lora_f32 | r << 8 | r_pad << 16)
-template <int RT, bool VEC>
-__global__ void __launch_bounds__(256)
-skinny_epilogue_kernel(const float* partial_, const float* su_part_, const void* lora_B_, bf16_t* y_, int32_t ldy_, int32_t M_, int32_t N_,
-                       int32_t count_bits, int32_t rank_bits, SkinnyEpiArgs rest) {
-    SkinnyEpiArgs g = rest;
-    g.partial = partial_; g.su_part = su_part_; g.lora_B = lora_B_; g.y = y_; g.ldy = ldy_; g.M = M_; g.N = N_;
-    g.splits = count_bits & 0xFFFF; g.su_parts = count_bits >> 16;
-    g.lora_f32 = rank_bits & 255; g.r = (rank_bits >> 8) & 255; g.r_pad = rank_bits >> 16;
-    // B tile of rank tile jt: [64 lanes][16 pieces of 4 ranks] fp32 (piece 4 e + q = ranks 4q .. 4q+3 of the lane's column
-    // e), the pieces of a lane XOR-swizzled with the lane number: conflict-free 16-byte writes and reads
-    __shared__ __attribute__((aligned(16))) float bt[RT > 0 ? RT : 1][64 * 64];
-    const int tid = threadIdx.x, lane = tid & 63, nthreads = blockDim.x;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int mraw = blockIdx.y * 4 + wave;
-    const int m = mraw < g.M ? mraw : g.M - 1;                   // a wave past M repeats the last row and stores nothing
-    const int n0 = blockIdx.x * 256;
-    int n = n0 + lane * 4;
-    const bool nvalid = n < g.N;                                 // N % 4 == 0: a lane's 4 columns are all in or all out
-    n = nvalid ? n : 0;
-    const int j = lane & 15, pg = lane >> 4;
+struct EpiJob {
+    const float* partial;
+    const float* su_part;
+    const void* lora_B;        // [N, r] fp32 or bf16
+    const bf16_t* bias;
+    bf16_t* y;                 // GU: h, of the first job
+    int64_t ldy;
+    int32_t N, splits, parts, r, r_pad, lora_f32;
+    float su_scale;
+};
+struct EpiBatch {
+    EpiJob job[kStreamJobs];
+};
 
-    // ---- issue: B pieces (piece q = 4 ranks of column n0 + q / 4), then the first 16 splits, then the first 32 su parts
-    constexpr int NQ = RT > 0 ? RT * 4 : 1;                       // pieces per thread with 256 threads
-    f32x4 bq[NQ];
-    if (RT > 0) {
+// y[m][n..n+1] = sum_s part[s][m][n..] + bias + su_scale * sum_j su[m][j] * B[n][j], su = sum of the parts.  A wave takes 128
+// columns (a lane 2) of RW rows, the block's waves the rows next to each other.  The kernel is a few dependent memory round
+// trips long: everything the first sums need -- B values of the first 16 ranks, partial tiles, low-rank parts (dealt over all
+// threads, met in LDS) -- is requested before anything is waited for.  Every sum runs in a fixed order.
+// VEC: B is fp32 with r % 4 == 0 (16-byte pieces).  GU: jobs 0 and 1 are gate and up, h is written.
+template <int RW, bool VEC, bool GU>
+__global__ void __launch_bounds__(256)
+stream_epilogue_kernel(int32_t M, int32_t first1, int32_t first2, int32_t first3, EpiBatch b) {
+    constexpr int NP = GU ? 2 : 1;
+    __shared__ __attribute__((aligned(16))) float su[NP][4 * RW][64];
+    __shared__ f32x4 red[NP][256];
+    __shared__ f32x4 bt[NP][512];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int bx = blockIdx.x;
+    const int ji = GU ? 0 : (bx >= first1 ? 1 : 0) + (bx >= first2 ? 1 : 0) + (bx >= first3 ? 1 : 0);
+    const int at = bx - (ji == 0 ? 0 : ji == 1 ? first1 : ji == 2 ? first2 : first3);
+    const int m0 = blockIdx.y * (4 * RW);
+    const int nthreads = blockDim.x;
+    const EpiJob& g0 = b.job[ji];
+    const int n = at * 128 + lane * 2;
+    const int nn = n < g0.N ? n : 0;                               // N % 2 == 0
+    const int mw = m0 + wave * RW;
+
+    // B values of 16 ranks of the block's columns: fetched in 16-byte pieces of 4 ranks, neighbouring threads on neighbouring
+    // pieces, and shared through LDS; piece P = column * 4 + ranks / 4 lies at P ^ (column / 4 & 7), which lets the 16 lanes of a
+    // read pass (two columns a lane) fall on 16 different pieces
+    constexpr int kPieces = RW == 1 ? 8 : 2;                       // of a thread (RW > 1: always four waves)
+    f32x4 bq[NP][kPieces];
+    const auto load_b = [&](int p, int rc) {
+        const EpiJob& g = b.job[ji + p];
 #pragma unroll
-        for (int jt = 0; jt < RT; ++jt)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int q = tid + i * nthreads;                 // blocks of fewer than 4 waves go round again below
-                const int col = n0 + (q >> 2) < g.N ? n0 + (q >> 2) : 0, jr = jt * 16 + 4 * (q & 3);
-                f32x4 t = {0.0f, 0.0f, 0.0f, 0.0f};
-                if (VEC) {
-                    t = *(const f32x4*)((const float*)g.lora_B + (int64_t)col * g.r + (jr < g.r ? jr : 0));
+        for (int i = 0; i < kPieces; ++i) {
+            if (i * nthreads < 512) {
+                const int P = (tid + i * nthreads) & 511, col = at * 128 + (P >> 2), j = rc + 4 * (P & 3);
+                const int64_t row = (int64_t)(col < g.N ? col : 0) * g.r;
+                if constexpr (VEC) {
+                    bq[p][i] = *(const f32x4*)((const float*)g.lora_B + row + (j < g.r ? j : 0));
                 } else {
-                    // (the storage type is tested around the four loads, not around each: a branch per load would make
-                    // every load wait for the one before)
-                    if (g.lora_f32) {
 #pragma unroll
-                        for (int c = 0; c < 4; ++c) t[c] = ((const float*)g.lora_B)[(int64_t)col * g.r + (jr + c < g.r ? jr + c : 0)];
-                    } else {
-                        bf16_t raw[4];
-#pragma unroll
-                        for (int c = 0; c < 4; ++c) raw[c] = ((const bf16_t*)g.lora_B)[(int64_t)col * g.r + (jr + c < g.r ? jr + c : 0)];
-#pragma unroll
-                        for (int c = 0; c < 4; ++c) t[c] = bf16_to_f32(raw[c]);
+                    for (int f = 0; f < 4; ++f) {
+                        const int64_t bi = row + (j + f < g.r ? j + f : 0);
+                        bq[p][i][f] = g.lora_f32 ? ((const float*)g.lora_B)[bi] : bf16_to_f32(((const bf16_t*)g.lora_B)[bi]);
                     }
                 }
-                bq[jt * 4 + i] = t;
             }
-    }
-    const float* pp = g.partial + (int64_t)m * g.N + n;
-    const int64_t sstride = (int64_t)g.M * g.N;
-    f32x4 pt[16];
-#pragma unroll
-    for (int u = 0; u < 16; ++u) pt[u] = *(const f32x4*)(pp + (int64_t)(u < g.splits ? u : g.splits - 1) * sstride);
-    const int64_t pstride = (int64_t)g.M * g.r_pad;
-    float st[RT > 0 ? RT : 1][8];
-#pragma unroll
-    for (int jt = 0; jt < RT; ++jt)
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const int pi = pg + 4 * u;
-            st[jt][u] = g.su_part[(int64_t)(pi < g.su_parts ? pi : g.su_parts - 1) * pstride + (int64_t)m * g.r_pad + jt * 16 + j];
         }
-
-    asm volatile("" ::"s"(g.su_scale), "s"(g.bias));        // the arguments that did not come with the wave, in one go
-    // ---- B pieces -> LDS
-    if (RT > 0) {
+    };
+    const auto store_b = [&](int p) {
 #pragma unroll
-        for (int jt = 0; jt < RT; ++jt)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int q = tid + i * nthreads;
-                if (q < 1024) *(f32x4*)(&bt[jt][(q >> 4) * 64 + ((q ^ (q >> 4)) & 15) * 4]) = bq[jt * 4 + i];
+        for (int i = 0; i < kPieces; ++i)
+            if (i * nthreads < 512) {
+                const int P = (tid + i * nthreads) & 511;
+                bt[p][P ^ ((P >> 4) & 7)] = bq[p][i];
             }
-        // blocks of one or two waves (M < 4): the pieces the first four rounds did not reach
-        for (int q = tid + 4 * nthreads; q < 1024; q += nthreads) {
-            const int col = n0 + (q >> 2) < g.N ? n0 + (q >> 2) : 0;
+    };
+    constexpr int SB = 4;                                          // splits requested at a time
+    f32x2 t[NP][SB][RW];
+    const auto load_part = [&](int p, int s0) {
+        const EpiJob& g = b.job[ji + p];
+        const int64_t ss = (int64_t)M * g.N;
 #pragma unroll
-            for (int jt = 0; jt < RT; ++jt) {
-                const int jr = jt * 16 + 4 * (q & 3);
-                f32x4 t;
-                if (g.lora_f32) {
+        for (int v = 0; v < SB; ++v)
 #pragma unroll
-                    for (int c = 0; c < 4; ++c) t[c] = ((const float*)g.lora_B)[(int64_t)col * g.r + (jr + c < g.r ? jr + c : 0)];
-                } else {
-                    bf16_t raw[4];
+            for (int u = 0; u < RW; ++u)
+                t[p][v][u] = *(const f32x2*)(g.partial + (int64_t)(s0 + v < g.splits ? s0 + v : g.splits - 1) * ss + (int64_t)(mw + u < M ? mw + u : M - 1) * g.N + nn);
+    };
 #pragma unroll
-                    for (int c = 0; c < 4; ++c) raw[c] = ((const bf16_t*)g.lora_B)[(int64_t)col * g.r + (jr + c < g.r ? jr + c : 0)];
+    for (int p = 0; p < NP; ++p)
+        if (b.job[ji + p].r > 0) load_b(p, 0);
 #pragma unroll
-                    for (int c = 0; c < 4; ++c) t[c] = bf16_to_f32(raw[c]);
+    for (int p = 0; p < NP; ++p) load_part(p, 0);
+
+    // ---- su of the block's rows -> LDS: thread (quad of ranks of a row, group of parts)
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+        const EpiJob& g = b.job[ji + p];
+        if (g.r > 0) {
+            const int qr = g.r_pad >> 2, quads = 4 * RW * qr, groups = nthreads / quads;
+            const int qd = tid % quads, gi = tid / quads, m = qd / qr;
+            const float* sp = g.su_part + (int64_t)(m0 + m < M ? m0 + m : M - 1) * g.r_pad + (qd - m * qr) * 4;
+            f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
+            for (int p0 = gi; p0 < g.parts; p0 += 8 * groups) {
+                f32x4 a[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    const int pi = p0 + u * groups;
+                    a[u] = *(const f32x4*)(sp + (int64_t)(pi < g.parts ? pi : g.parts - 1) * M * g.r_pad);
                 }
-                *(f32x4*)(&bt[jt][(q >> 4) * 64 + ((q ^ (q >> 4)) & 15) * 4]) = t;
+#pragma unroll
+                for (int u = 0; u < 8; ++u)
+                    if (p0 + u * groups < g.parts) v += a[u];
             }
-        }
-        __syncthreads();
-    }
-
-    // ---- su parts: lane (j, pg) sums parts pg, pg+4, ... of rank j of each tile
-    float sv[RT > 0 ? RT : 1];
-#pragma unroll
-    for (int jt = 0; jt < RT; ++jt) {
-        sv[jt] = 0.0f;
-#pragma unroll
-        for (int u = 0; u < 8; ++u) sv[jt] += pg + 4 * u < g.su_parts ? st[jt][u] : 0.0f;
-    }
-    for (int p0 = 32; p0 < g.su_parts; p0 += 32) {
-#pragma unroll
-        for (int jt = 0; jt < RT; ++jt)
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const int pi = p0 + pg + 4 * u;
-                st[jt][u] = g.su_part[(int64_t)(pi < g.su_parts ? pi : g.su_parts - 1) * pstride + (int64_t)m * g.r_pad + jt * 16 + j];
-            }
-#pragma unroll
-        for (int jt = 0; jt < RT; ++jt)
-#pragma unroll
-            for (int u = 0; u < 8; ++u) sv[jt] += p0 + pg + 4 * u < g.su_parts ? st[jt][u] : 0.0f;
-    }
-    // ---- partial tiles
-    f32x4 o = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int u = 0; u < 16; ++u) {
-        if (u < g.splits) o += pt[u];                             // wave-uniform
-    }
-    for (int s0 = 16; s0 < g.splits; s0 += 16) {
-#pragma unroll
-        for (int u = 0; u < 16; ++u) pt[u] = *(const f32x4*)(pp + (int64_t)(s0 + u < g.splits ? s0 + u : g.splits - 1) * sstride);
-#pragma unroll
-        for (int u = 0; u < 16; ++u) {
-            if (s0 + u < g.splits) o += pt[u];
+            red[p][tid] = v;
+            store_b(p);
         }
     }
-    // ---- low-rank term, 16 ranks at a time; ranks >= r hold zeros in su (and finite values in the B tile)
+    __syncthreads();
 #pragma unroll
-    for (int jt = 0; jt < RT; ++jt) {
-        float tot = __shfl(sv[jt], j, 64);
-        tot += __shfl(sv[jt], 16 + j, 64);
-        tot += __shfl(sv[jt], 32 + j, 64);
-        tot += __shfl(sv[jt], 48 + j, 64);
-        tot *= g.su_scale;                                        // lane l holds su[m][jt*16 + (l & 15)], zero for ranks >= r
-        if (jt * 16 + j >= g.r) tot = 0.0f;
+    for (int p = 0; p < NP; ++p) {
+        const EpiJob& g = b.job[ji + p];
+        if (g.r > 0) {
+            const int qr = g.r_pad >> 2, quads = 4 * RW * qr, groups = nthreads / quads;
+            if (tid < quads) {
+                f32x4 v = red[p][tid];
+                for (int gi = 1; gi < groups; ++gi) v += red[p][gi * quads + tid];
+                const int m = tid / qr, j = (tid - m * qr) * 4;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            f32x4 bv[4];
+                for (int e = 0; e < 4; ++e) su[p][m][j + e] = j + e < g.r ? v[e] * g.su_scale : 0.0f;
+            }
+        }
+    }
+    f32x2 o[NP][RW];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) bv[e] = *(const f32x4*)(&bt[jt][lane * 64 + (((e * 4 + q) ^ lane) & 15) * 4]);
+    for (int p = 0; p < NP; ++p) {
+        const EpiJob& g = b.job[ji + p];
+#pragma unroll
+        for (int u = 0; u < RW; ++u) o[p][u] = f32x2{0.0f, 0.0f};
+        for (int s0 = 0;;) {
+#pragma unroll
+            for (int v = 0; v < SB; ++v)
+                if (s0 + v < g.splits) {
+#pragma unroll
+                    for (int u = 0; u < RW; ++u) {
+                        o[p][u][0] += t[p][v][u][0];
+                        o[p][u][1] += t[p][v][u][1];
+                    }
+                }
+            s0 += SB;
+            if (s0 >= g.splits) break;
+            load_part(p, s0);
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+        const EpiJob& g = b.job[ji + p];
+        for (int rc = 0; rc < g.r; rc += 16) {
+            if (rc + 16 < g.r) load_b(p, rc + 16);
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
-                const float sj = __shfl(tot, 4 * q + c, 64);
+                f32x4 bv[2];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) o[e] = __builtin_fmaf(sj, bv[e][c], o[e]);
+                for (int e = 0; e < 2; ++e) bv[e] = bt[p][((lane * 2 + e) * 4 + c) ^ ((lane >> 1) & 7)];
+#pragma unroll
+                for (int u = 0; u < RW; ++u) {
+                    const f32x4 sv = *(const f32x4*)&su[p][wave * RW + u][rc + 4 * c];
+#pragma unroll
+                    for (int f = 0; f < 4; ++f)
+#pragma unroll
+                        for (int e = 0; e < 2; ++e) o[p][u][e] = __builtin_fmaf(sv[f], bv[e][f], o[p][u][e]);
+                }
+            }
+            if (rc + 16 < g.r) {
+                __syncthreads();
+                store_b(p);
+                __syncthreads();
+            }
+        }
+        if (g.bias) {
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                const float bb = bf16_to_f32(g.bias[nn + e]);
+#pragma unroll
+                for (int u = 0; u < RW; ++u) o[p][u][e] += bb;
             }
         }
     }
-    if (!nvalid || mraw >= g.M) return;
-    if (g.bias) {
+    if (n >= g0.N) return;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) o[e] += bf16_to_f32(g.bias[n + e]);
+    for (int u = 0; u < RW; ++u) {
+        if (mw + u < M) {
+            f32x2 r = o[0][u];
+            if constexpr (GU) {
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    const float gate = round_bf16(r[e]);
+                    r[e] = round_bf16(gate * sigmoid_f32(gate)) * round_bf16(o[NP - 1][u][e]);
+                }
+            }
+            *(uint32_t*)(g0.y + (int64_t)(mw + u) * g0.ldy + n) = pack_bf16x2(r[0], r[1]);
+        }
     }
-    *(u32x2*)(g.y + (int64_t)m * g.ldy + n) = u32x2{pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3])};
 }
 
 static inline int64_t al256(int64_t b) { return (b + 255) & ~(int64_t)255; }
 
-// K splits for the split organisation: at most four chunks per split; more splits until the grid holds
-// about two blocks per CU, never more than the 1024 blocks that are resident at once (four per CU).
-struct SkinnyPlan { int splits, nch, row_blocks; };
-static SkinnyPlan skinny_plan(int64_t N, int64_t K) {
-    const int ct = (int)(K >> 7), rb = (int)xq_cdiv(N, 128);
-    int splits = (int)xq_cdiv(ct, 4);
-    while (splits < ct && (int64_t)(rb + 1) * splits < 512 && (int64_t)(rb + 1) * (splits + 1) <= 1024) ++splits;
-    SkinnyPlan p;
-    p.splits = splits;
-    p.nch = (int)xq_cdiv(ct, splits);   // the longest split
-    p.row_blocks = rb;
-    return p;
+// What a launch of `blocks` blocks of 8 waves with RT row tiles and `steps` steps takes, in us, from a sweep of M 1..64 and widths
+// 1024..16384: a start of ~4 us (launch, the x slice, the first weights), then the decode and the products of a SIMD's
+// (row tile, step) units, which two waves to a SIMD overlap worse than four.  Two blocks are resident per CU at M <= 32, where
+// their x slices fit.
+static double stream_run_us(int64_t blocks, int rt, int steps, int mt) {
+    const int per_cu = mt == 4 || rt == 3 || steps * mt * 4096 > 78 * 1024 ? 1 : 2;
+    const int64_t cus = num_cus();
+    const double rounds = (double)xq_cdiv(blocks, cus * per_cu);
+    const double on_cu = (double)xq_cdiv(blocks, cus) < rounds * per_cu ? (double)xq_cdiv(blocks, cus) : rounds * per_cu;
+    const double unit = on_cu > 1 && per_cu == 2 ? 0.12 + 0.04 * mt : 0.2 + 0.07 * mt;
+    return 4.0 * rounds + on_cu * 2 * rt * steps * unit;
+}
+// row tiles of a wave by that estimate (they change nothing in the results); `tiles`, `splits` of each forward of the launch
+static int stream_row_tiles(const int* tiles, const int* splits, int n, int steps, int mt, int rt_max, double* us) {
+    int best = 1;
+    double cost = 0;
+    for (int rt = 1; rt <= rt_max; ++rt) {
+        int64_t blocks = 0;
+        for (int i = 0; i < n; ++i) blocks += xq_cdiv(tiles[i], (int64_t)kStreamWaves * rt) * splits[i];
+        const double c = stream_run_us(blocks, rt, steps, mt);
+        if (cost == 0 || c < cost) { cost = c; best = rt; }
+    }
+    if (us) *us = cost;
+    return best;
+}
+// steps of a split at most (128 KB of x slice)
+static int stream_steps_max(int64_t M) { return M <= 16 ? 32 : M <= 32 ? 16 : 8; }
+// K splits of a forward, by its own shape: the cheapest sum of that and of the partial sums' trip (written and read back, ~6
+// TB/s)
+static int stream_splits(int64_t M, int64_t N, int64_t K) {
+    const int ct = (int)(K >> 7), tiles = (int)(N / 16);
+    const int mt = M <= 16 ? 1 : M <= 32 ? 2 : 4;
+    int best = 0, last_steps = 0;
+    double best_cost = 0;
+    for (int s = (int)xq_cdiv(ct, stream_steps_max(M)); s <= ct && s <= 64; ++s) {
+        const int steps = (int)xq_cdiv(ct, s);
+        if (steps == last_steps) continue;                         // more splits, none of them shorter
+        last_steps = steps;
+        double c;
+        stream_row_tiles(&tiles, &s, 1, steps, mt, 3, &c);
+        c += (double)s * M * N * 8.0 / 6.0e6;
+        if (best == 0 || c < best_cost) { best = s; best_cost = c; }
+    }
+    return best;
+}
+
+// whether a forward of this shape runs on the two launches of this file (and not in one, xq_skinny_rows.hip)
+bool skinny_takes_stream(const xq_weight* w, int64_t M, const void* lora_A, const void* lora_B, int lora_dtype, int r) {
+    return skinny_supported(w, M) && !(skinny_rows_enabled() && skinny_rows_supported(w, M, lora_A, lora_B, lora_dtype, r));
 }
 
 int64_t skinny_workspace_bytes(int64_t M, int64_t N, int64_t K, int r_pad) {
+    if (K < 128 || N < 16) return 256;
     const int rp = r_pad ? r_pad : 16;
-    const SkinnyPlan p = skinny_plan(N, K);
-    return al256((int64_t)p.splits * M * N * 4) + al256((int64_t)p.splits * M * rp * 4) + 256;
+    const int s = stream_splits(M, N, K);
+    return al256((int64_t)s * M * N * 4) + al256((K >> 7) * M * rp * 4) + 256;
 }
 
 bool skinny_supported(const xq_weight* w, int64_t M) {
@@ -659,82 +619,148 @@ bool skinny_supported(const xq_weight* w, int64_t M) {
     return true;
 }
 
-template <int FMT, int NCH>
-static int launch_split_one(const SkinnyArgs& g, dim3 grid, size_t lds, hipStream_t s) {
-    // at most 32 rows of 1040 B + the slabs = 49 KB: below the default dynamic LDS limit
-    XQ_REQUIRE(g.ldx < (1ll << 31) && g.group < (1 << 24) && g.splits < (1 << 16) && g.chunk_q < (1 << 16),
-               "xq_linear_fwd: internal error: skinny launch arguments out of range");
-    const int32_t fmt_bits = g.group | g.scale_dtype << 24, split_bits = g.splits | g.su_blocks << 16, chunk_bits = g.chunk_q | g.chunk_rem << 16;
-#define XQ_SPLIT_ARGS g.x, (int32_t)g.ldx, g.M, g.N, g.K, g.packed, g.scales, fmt_bits, split_bits, chunk_bits, g.xp, g
-    if (g.M <= 16) skinny_split_kernel<FMT, 16, NCH><<<grid, 256, lds, s>>>(XQ_SPLIT_ARGS);
-    else if (g.M <= 32) skinny_split_kernel<FMT, 32, NCH><<<grid, 256, lds, s>>>(XQ_SPLIT_ARGS);
-    else skinny_split_kernel<FMT, 64, NCH><<<grid, 256, lds, s>>>(XQ_SPLIT_ARGS);
-#undef XQ_SPLIT_ARGS
-    return XQ_OK;
+static int scale_mode(const xq_weight* w) {
+    if (w->format == XQ_FMT_FP8) return kScFp8;
+    if (w->format == XQ_FMT_NF4) return xq_aligned(w->scales, 8) ? kScDealt : -1;
+    if (w->format == XQ_FMT_NVFP4) return w->scale_dtype == XQ_SCALE_E4M3 ? (xq_aligned(w->scales, 8) ? kScDealt : -1)
+                                        : (w->scale_dtype == XQ_SCALE_F32 && xq_aligned(w->scales, 8) ? kScStep : -1);
+    if (w->group == 128 && w->scale_dtype == XQ_SCALE_BF16) return kScInt4Window;
+    return w->group % 32 == 0 && w->cols % w->group == 0 ? kScStep : kScUse;
 }
 
-template <int FMT>
-static int launch_split_cfg(const SkinnyArgs& g, int nch, dim3 grid, size_t lds, hipStream_t s) {
-    if (nch <= 1) return launch_split_one<FMT, 1>(g, grid, lds, s);
-    if (nch <= 2) return launch_split_one<FMT, 2>(g, grid, lds, s);
-    return launch_split_one<FMT, 4>(g, grid, lds, s);
-}
+// (the uncommon scale storages keep more registers per row tile)
+template <int SC>
+constexpr int kRowTilesMax = SC == kScUse ? 1 : SC == kScStep ? 2 : 3;
 
-static int launch_skinny_split(const xq_weight* w, const bf16_t* x, int64_t ldx, int64_t M, const void* lora_A, const void* lora_B,
-                               int lora_dtype, int r, int rp, float scaling, const bf16_t* bias, bf16_t* y, int64_t ldy,
-                               void* workspace, hipStream_t stream) {
-    const int64_t N = w->rows, K = w->cols;
-    const SkinnyPlan p = skinny_plan(N, K);
-    XQ_REQUIRE(p.nch <= 4, "xq_linear_fwd: internal error: K split too long (%d chunks)", p.nch);
-    XQ_REQUIRE(rp == 0 || xq_aligned(lora_A, 16), "xq_linear_fwd: lora_A must be 16-byte aligned");
-    SkinnyArgs g;
-    g.x = x; g.ldx = ldx; g.M = (int)M; g.N = (int)N; g.K = (int)K;
-    g.packed = (const uint8_t*)w->packed; g.scales = (const uint8_t*)w->scales; g.global_scale = w->global_scale;
-    g.group = w->group; g.scale_dtype = w->scale_dtype;
-    g.splits = p.splits; g.su_blocks = rp ? 1 : 0; g.xp = p.nch * 128 + 8;
-    g.chunk_q = (int)(K >> 7) / p.splits; g.chunk_rem = (int)(K >> 7) % p.splits;
-    g.partial = (float*)workspace;
-    g.su_part = (float*)((char*)workspace + al256((int64_t)p.splits * M * N * 4));
-    g.lora_A = rp ? lora_A : nullptr; g.lora_f32 = lora_dtype == XQ_DT_F32; g.r = r; g.r_pad = rp;
-    const dim3 grid((unsigned)p.splits, (unsigned)(p.row_blocks + g.su_blocks));
-    size_t lds = (size_t)(M < 32 ? M : 32) * g.xp * 2 + 4 * 4096 + 64;   // x slice + the four weight slabs (or the su reduction buffer) + nf4 levels
-    if (M > 32 && lds < 2 * 64 * 136 * 2 + 4 * 4096 + 64) lds = 2 * 64 * 136 * 2 + 4 * 4096 + 64;   // two x chunk buffers of 64 rows
-
-    SkinnyEpiArgs e;
-    e.partial = g.partial; e.su_part = g.su_part; e.splits = p.splits; e.su_parts = rp ? p.splits : 0;
-    e.M = (int)M; e.N = (int)N; e.lora_B = rp ? lora_B : nullptr; e.lora_f32 = g.lora_f32; e.r = r; e.r_pad = rp;
-    e.su_scale = scaling; e.bias = bias; e.y = y; e.ldy = ldy;
-
-    int rc;
-    if (w->format == XQ_FMT_FP8) rc = launch_split_cfg<XQ_FMT_FP8>(g, p.nch, grid, lds, stream);
-    else if (w->format == XQ_FMT_INT4) rc = launch_split_cfg<XQ_FMT_INT4>(g, p.nch, grid, lds, stream);
-    else if (w->format == XQ_FMT_NF4) rc = launch_split_cfg<XQ_FMT_NF4>(g, p.nch, grid, lds, stream);
-    else rc = launch_split_cfg<XQ_FMT_NVFP4>(g, p.nch, grid, lds, stream);
-    if (rc) return rc;
-    const int waves = M < 4 ? (int)M : 4;
-    const dim3 egrid((unsigned)xq_cdiv(N, 256), (unsigned)xq_cdiv(M, 4));
-    const bool vec = g.lora_f32 && r % 4 == 0 && xq_aligned(lora_B, 16);
-    XQ_REQUIRE(ldy < (1ll << 31) && p.splits < (1 << 16), "xq_linear_fwd: internal error: skinny epilogue arguments out of range");
-    const int32_t count_bits = e.splits | e.su_parts << 16, rank_bits = e.lora_f32 | e.r << 8 | e.r_pad << 16;
-#define XQ_EPI_ARGS e.partial, e.su_part, e.lora_B, e.y, (int32_t)e.ldy, e.M, e.N, count_bits, rank_bits, e
-#define XQ_EPI(RT)                                                                                      \
-    do {                                                                                                \
-        if (vec) skinny_epilogue_kernel<RT, true><<<egrid, waves * 64, 0, stream>>>(XQ_EPI_ARGS);       \
-        else skinny_epilogue_kernel<RT, false><<<egrid, waves * 64, 0, stream>>>(XQ_EPI_ARGS);          \
-    } while (0)
-    switch (rp >> 4) {
-        case 0: skinny_epilogue_kernel<0, false><<<egrid, waves * 64, 0, stream>>>(XQ_EPI_ARGS); break;
-        case 1: XQ_EPI(1); break;
-        case 2: XQ_EPI(2); break;
-        case 3: XQ_EPI(3); break;
-        default: XQ_EPI(4); break;
+template <int FMT, int SC, int MT, int RT>
+static int launch_stream_one(const StreamBatch& b, const int* first, const bf16_t* x, int64_t ldx, int64_t M, int64_t K, size_t lds, hipStream_t s) {
+    static std::atomic<bool> attr_set{false};
+    if (!attr_set) {
+        const hipError_t e = hipFuncSetAttribute((const void*)stream_split_kernel<FMT, SC, MT, RT>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        if (e != hipSuccess) {
+            xq_set_error("xq_linear_fwd: cannot raise the dynamic LDS limit: %s", hipGetErrorString(e));
+            return XQ_ERR_LAUNCH;
+        }
+        attr_set = true;
     }
+    stream_split_kernel<FMT, SC, MT, RT><<<(unsigned)first[4], 64 * kStreamWaves, lds, s>>>(x, (int32_t)ldx, (int32_t)M, (int32_t)K, first[1], first[2], first[3], b);
+    return XQ_OK;
+}
+template <int FMT, int SC, int MT>
+static int launch_stream_mt(const StreamBatch& b, const int* first, const bf16_t* x, int64_t ldx, int64_t M, int64_t K, int rt, size_t lds, hipStream_t s) {
+    constexpr int most = kRowTilesMax<SC>;
+    if constexpr (most > 2)
+        if (rt == 3) return launch_stream_one<FMT, SC, MT, 3>(b, first, x, ldx, M, K, lds, s);
+    if constexpr (most > 1)
+        if (rt == 2) return launch_stream_one<FMT, SC, MT, 2>(b, first, x, ldx, M, K, lds, s);
+    return launch_stream_one<FMT, SC, MT, 1>(b, first, x, ldx, M, K, lds, s);
+}
+template <int FMT, int SC>
+static int launch_stream_sc(const StreamBatch& b, const int* first, const bf16_t* x, int64_t ldx, int64_t M, int64_t K, int rt, size_t lds, hipStream_t s) {
+    if (M <= 16) return launch_stream_mt<FMT, SC, 1>(b, first, x, ldx, M, K, rt, lds, s);
+    if (M <= 32) return launch_stream_mt<FMT, SC, 2>(b, first, x, ldx, M, K, rt, lds, s);
+    return launch_stream_mt<FMT, SC, 4>(b, first, x, ldx, M, K, rt, lds, s);
+}
+
+bool skinny_stream_multi_supported(const SkinnyRowsJob* jobs, int n_jobs, int64_t M) {
+    if (n_jobs < 1 || n_jobs > kStreamJobs) return false;
+    for (int i = 0; i < n_jobs; ++i) {
+        const xq_weight* w = jobs[i].w;
+        if (!skinny_supported(w, M) || scale_mode(w) < 0 || w->format != jobs[0].w->format || w->cols != jobs[0].w->cols ||
+            scale_mode(w) != scale_mode(jobs[0].w) || !xq_aligned(w->packed, 16) || jobs[i].ldy % 4 != 0 || !xq_aligned(jobs[i].y, 8))
+            return false;
+        if (jobs[i].r > 0 && (!xq_aligned(jobs[i].lora_A, 16) || !xq_aligned(jobs[i].lora_B, 4))) return false;
+    }
+    return true;
+}
+
+int64_t skinny_stream_multi_workspace_bytes(const SkinnyRowsJob* jobs, int n_jobs, int64_t M) {
+    int64_t b = 0;
+    for (int i = 0; i < n_jobs; ++i) b += skinny_workspace_bytes(M, jobs[i].w->rows, jobs[i].w->cols, jobs[i].r > 0 ? (jobs[i].r + 15) / 16 * 16 : 0);
+    return b;
+}
+
+int launch_skinny_stream(const SkinnyRowsJob* jobs, int n_jobs, bool swiglu, const bf16_t* x, int64_t ldx, int64_t M, int lora_dtype,
+                         void* workspace, hipStream_t stream) {
+    const xq_weight* w0 = jobs[0].w;
+    const int64_t K = w0->cols;
+    const int sc = scale_mode(w0), mt = M <= 16 ? 1 : M <= 32 ? 2 : 4;
+    XQ_REQUIRE(sc >= 0 && ldx < (1ll << 31), "xq_linear_fwd: internal error: shape not supported by the streaming kernel");
+    StreamBatch b{};
+    EpiBatch e{};
+    uint8_t* ws = (uint8_t*)workspace;
+    bool vec = true;
+    int steps = 0;
+    for (int i = 0; i < n_jobs; ++i) {
+        const SkinnyRowsJob& j = jobs[i];
+        const int rp = j.r > 0 ? (j.r + 15) / 16 * 16 : 0;
+        const int64_t N = j.w->rows;
+        StreamJob& g = b.job[i];
+        g.splits = stream_splits(M, N, K);
+        g.packed = (const uint8_t*)j.w->packed; g.scales = (const uint8_t*)j.w->scales; g.global_scale = j.w->global_scale;
+        g.N = (int)N; g.group = j.w->group; g.scale_dtype = j.w->scale_dtype;
+        g.chunk_q = (int)(K >> 7) / g.splits; g.chunk_rem = (int)(K >> 7) % g.splits;
+        const int longest = g.chunk_q + (g.chunk_rem ? 1 : 0);
+        steps = longest > steps ? longest : steps;
+        g.partial = (float*)ws;
+        ws += al256((int64_t)g.splits * M * N * 4);
+        g.su_part = (float*)ws;
+        ws += al256((K >> 7) * M * (rp ? rp : 16) * 4) + 256;
+        g.lora_A = rp ? j.lora_A : nullptr; g.lora_f32 = lora_dtype == XQ_DT_F32; g.r = j.r; g.r_pad = rp;
+        EpiJob& ej = e.job[i];
+        ej.partial = g.partial; ej.su_part = g.su_part; ej.lora_B = rp ? j.lora_B : nullptr; ej.bias = j.bias; ej.y = j.y; ej.ldy = j.ldy;
+        ej.N = (int)N; ej.splits = g.splits; ej.parts = (int)(K >> 7); ej.r = j.r; ej.r_pad = rp; ej.lora_f32 = g.lora_f32; ej.su_scale = j.scaling;
+        vec = vec && (j.r == 0 || (g.lora_f32 && j.r % 4 == 0 && xq_aligned(j.lora_B, 16)));
+    }
+    int tiles[kStreamJobs], splits[kStreamJobs];
+    for (int i = 0; i < n_jobs; ++i) { tiles[i] = b.job[i].N / 16; splits[i] = b.job[i].splits; }
+    const int rt = stream_row_tiles(tiles, splits, n_jobs, steps, mt, sc == kScUse ? kRowTilesMax<kScUse> : sc == kScStep ? kRowTilesMax<kScStep> : 3, nullptr);
+    int first[5] = {0, 0, 0, 0, 0}, efirst[5] = {0, 0, 0, 0, 0};
+    for (int i = 0; i < kStreamJobs; ++i) {
+        first[i + 1] = first[i];
+        efirst[i + 1] = efirst[i];
+        if (i < n_jobs) {
+            b.job[i].row_blocks = (int)xq_cdiv(tiles[i], (int64_t)kStreamWaves * rt);
+            first[i + 1] += b.job[i].row_blocks * b.job[i].splits;
+            efirst[i + 1] += (int)xq_cdiv(b.job[i].N, 128);
+        } else {
+            b.job[i] = b.job[0];
+            e.job[i] = e.job[0];
+        }
+    }
+    const size_t lds = (size_t)steps * mt * 4096 + 64;             // the x slice of the longest split, the nf4 levels
+    int rc = XQ_ERR_UNSUPPORTED;
+#define XQ_STREAM_CASE(F, S) \
+    if (w0->format == F && sc == S) rc = launch_stream_sc<F, S>(b, first, x, ldx, M, K, rt, lds, stream)
+    XQ_STREAM_CASE(XQ_FMT_FP8, kScFp8);
+    XQ_STREAM_CASE(XQ_FMT_INT4, kScInt4Window);
+    XQ_STREAM_CASE(XQ_FMT_INT4, kScStep);
+    XQ_STREAM_CASE(XQ_FMT_INT4, kScUse);
+    XQ_STREAM_CASE(XQ_FMT_NVFP4, kScDealt);
+    XQ_STREAM_CASE(XQ_FMT_NVFP4, kScStep);
+    XQ_STREAM_CASE(XQ_FMT_NF4, kScDealt);
+#undef XQ_STREAM_CASE
+    if (rc) return rc;
+    const int rw = M <= 16 ? 1 : 4;
+    const unsigned cols = (unsigned)(swiglu ? efirst[1] : efirst[4]), threads = M < 4 && rw == 1 ? (unsigned)M * 64 : 256;
+    const dim3 grid(cols, (unsigned)xq_cdiv(M, 4 * rw));
+#define XQ_EPI(RW)                                                                                                                             \
+    do {                                                                                                                                       \
+        if (swiglu) {                                                                                                                          \
+            if (vec) stream_epilogue_kernel<RW, true, true><<<grid, threads, 0, stream>>>((int)M, efirst[1], efirst[2], efirst[3], e);         \
+            else stream_epilogue_kernel<RW, false, true><<<grid, threads, 0, stream>>>((int)M, efirst[1], efirst[2], efirst[3], e);            \
+        } else {                                                                                                                               \
+            if (vec) stream_epilogue_kernel<RW, true, false><<<grid, threads, 0, stream>>>((int)M, efirst[1], efirst[2], efirst[3], e);        \
+            else stream_epilogue_kernel<RW, false, false><<<grid, threads, 0, stream>>>((int)M, efirst[1], efirst[2], efirst[3], e);           \
+        }                                                                                                                                      \
+    } while (0)
+    if (rw == 1) XQ_EPI(1);
+    else XQ_EPI(4);
 #undef XQ_EPI
-#undef XQ_EPI_ARGS
     return XQ_OK;
 }
 
-// XQ_SKINNY_ROWS=0 (or xq_set_skinny_rows(0)) keeps every skinny forward on the two-launch organisation: a process-wide
+// XQ_SKINNY_ROWS=0 (or xq_set_skinny_one_launch(0)) keeps every skinny forward on the two-launch organisation: a process-wide
 // test switch, to be set while no other thread is inside the library
 static int g_skinny_rows = [] { const char* e = getenv("XQ_SKINNY_ROWS"); return e ? atoi(e) : 1; }();
 void set_skinny_rows(int enabled) { g_skinny_rows = enabled; }
@@ -749,7 +775,8 @@ int launch_skinny(const xq_weight* w, const bf16_t* x, int64_t ldx, int64_t M, c
                "xq_linear_fwd: workspace missing, misaligned or too small for the skinny path");
     XQ_REQUIRE(ldx % 8 == 0 && xq_aligned(x, 16) && xq_aligned(w->packed, 16), "xq_linear_fwd: operands must be 16-byte aligned");
     XQ_REQUIRE(ldy % 4 == 0 && xq_aligned(y, 8), "xq_linear_fwd: output rows must be 8-byte aligned");
-    XQ_REQUIRE(rp == 0 || xq_aligned(lora_A, 4) && xq_aligned(lora_B, 4), "xq_linear_fwd: LoRA factors must be 4-byte aligned");
+    XQ_REQUIRE(rp == 0 || (xq_aligned(lora_A, 16) && xq_aligned(lora_B, 4)), "xq_linear_fwd: lora_A must be 16-byte and lora_B 4-byte aligned");
+    XQ_REQUIRE(scale_mode(w) >= 0, "xq_linear_fwd: scales must be 8-byte aligned");
     // algorithmic bytes: packed weight + scales + x + y (+ LoRA factors), for the roofline figure; the timed
     // region is the whole forward (both launches)
     const double wbytes = (double)xq_packed_bytes_per_expert(w) + (double)xq_scale_bytes_per_expert(w);
@@ -758,8 +785,10 @@ int launch_skinny(const xq_weight* w, const bf16_t* x, int64_t ldx, int64_t M, c
     int rc = XQ_ERR_UNSUPPORTED;
     if (g_skinny_rows && skinny_rows_supported(w, M, lora_A, lora_B, lora_dtype, r))
         rc = launch_skinny_rows(w, x, ldx, M, lora_A, lora_B, r, scaling, bias, y, ldy, workspace, stream);
-    if (rc == XQ_ERR_UNSUPPORTED)
-        rc = launch_skinny_split(w, x, ldx, M, lora_A, lora_B, lora_dtype, r, rp, scaling, bias, y, ldy, workspace, stream);
+    if (rc == XQ_ERR_UNSUPPORTED) {
+        const SkinnyRowsJob job{w, lora_A, lora_B, rp ? r : 0, scaling, bias, y, ldy};
+        rc = launch_skinny_stream(&job, 1, false, x, ldx, M, lora_dtype, workspace, stream);
+    }
     if (timed) xq_profile_mark_end(stream);
     if (rc) return rc;
     XQ_CHECK_LAUNCH("skinny forward");

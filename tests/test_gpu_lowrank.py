@@ -1,0 +1,88 @@
+"""GPU parity of the dense low-rank products (read from the factors as the caller holds them) and of the per-expert
+weight-gradient launch, at the sizes where their launches change form."""
+
+import pytest
+import torch
+
+from oracle import recipe as R
+from tests.util_cases import close, gen, make_dense_module
+
+pytestmark = pytest.mark.gpu
+TOL = 1e-2
+
+
+@pytest.mark.parametrize("bf16_factors", [False, True])
+@pytest.mark.parametrize("M,N,K,r", [
+    (65, 320, 64, 1),          # one unit of the contraction for sixteen waves
+    (100, 64, 1088, 17),       # rows and units that fill no block; ranks of two tiles, the second nearly empty
+    (1025, 256, 256, 40),      # wide factors: eight waves; two row splits of the weight gradients
+    (4096, 128, 192, 16),      # the last size of short blocks
+    (4097, 192, 128, 64),      # tall blocks and bf16 panels
+])
+def test_linear_training_at_the_edges(hip_device, M, N, K, r, bf16_factors):
+    m, w_ref = make_dense_module("block_fp8", N, K, r, 2 * r, seed=M, device=hip_device)
+    if bf16_factors:
+        m.lora_A.data = m.lora_A.data.to(torch.bfloat16)
+        m.lora_B.data = m.lora_B.data.to(torch.bfloat16)
+    else:                      # a factor that starts 4 bytes off a 16-byte boundary (a view into a flat parameter)
+        flat = torch.zeros(r * K + 1, device=hip_device)
+        flat[1:] = m.lora_A.data.reshape(-1)
+        m.lora_A.data = flat[1:].view(r, K)
+    x = gen((M, K), 1.0, 1, torch.bfloat16)
+    dy = gen((M, N), 1.0, 2, torch.bfloat16)
+    xd = x.to(hip_device).requires_grad_(True)
+    y = m(xd)
+    y.backward(dy.to(hip_device))
+    ex = R.linear_fwd_bwd_exact(x, w_ref, m.lora_A.detach().float().cpu(), m.lora_B.detach().float().cpu(), m.scaling, dy)
+    close(y.detach().cpu(), ex["y"], TOL)
+    close(xd.grad.cpu(), ex["dx"], TOL)
+    close(m.lora_A.grad.float().cpu(), ex["dA"], TOL)
+    close(m.lora_B.grad.float().cpu(), ex["dB"], TOL, rows="last" if r > 1 else "none")       # (rank 1: a row is one dot product)
+
+
+@pytest.mark.parametrize("M,H,I,r", [
+    (70, 128, 576, 16),        # nine units of columns for four waves, one column split
+    (300, 256, 1600, 12),      # 25 units over three column splits
+    (2047, 128, 512, 32),      # factors as they are, 2048: from panels
+    (2048, 128, 512, 32),
+])
+def test_mlp_training_at_the_edges(hip_device, M, H, I, r):
+    from xorl_amd.qlora import qlora_mlp_forward
+
+    mods, w_ref = {}, {}
+    for i, (k, (N, K)) in enumerate({"gate": (I, H), "up": (I, H), "down": (H, I)}.items()):
+        mods[k], w_ref[k] = make_dense_module("nvfp4", N, K, r, 2 * r, seed=M + 10 * i, device=hip_device)
+    x = gen((M, H), 1.0, 3, torch.bfloat16)
+    dy = gen((M, H), 1.0, 4, torch.bfloat16)
+    loras = {k: (m.lora_A.detach().cpu(), m.lora_B.detach().cpu()) for k, m in mods.items()}
+    ex = R.mlp_fwd_bwd_exact(x, w_ref["gate"], w_ref["up"], w_ref["down"], loras, mods["gate"].scaling, dy)
+    xd = x.to(hip_device).requires_grad_(True)
+    y = qlora_mlp_forward(mods["gate"], mods["up"], mods["down"], xd)
+    y.backward(dy.to(hip_device))
+    close(y.detach().cpu(), ex["y"], TOL)
+    close(xd.grad.cpu(), ex["dx"], TOL)
+    for k, m in mods.items():
+        close(m.lora_A.grad.cpu(), ex[f"dA_{k}"], TOL)
+        close(m.lora_B.grad.cpu(), ex[f"dB_{k}"], TOL)
+
+
+@pytest.mark.parametrize("over", [0, 1])      # 256 rows an expert on average: a block per expert; one more row: row chunks
+@pytest.mark.parametrize("r,rp,transpose", [(16, 16, False), (33, 48, True)])
+def test_expert_weight_gradients_either_side_of_the_rule(hip_device, r, rp, transpose, over):
+    from xorl_amd import moe_functional as MF
+
+    E, width = 4, 200
+    counts = torch.tensor([0, 1, 33, 256 * E - 34 + over])
+    ends = counts.cumsum(0)
+    offsets = torch.cat([torch.zeros(1, dtype=torch.int64), ends]).to(torch.int32).to(hip_device)
+    P = gen((int(ends[-1]), width), 1.0, 5, torch.bfloat16)
+    Q = gen((int(ends[-1]), rp), 1.0, 6, torch.bfloat16)
+    g = MF._wgrad(P.to(hip_device), Q.to(hip_device), r, offsets, E, transpose).cpu()
+    for e in range(E):
+        lo, hi = int(ends[e] - counts[e]), int(ends[e])
+        ref = P[lo:hi].double().t() @ Q[lo:hi, :r].double()
+        ref = ref.t() if transpose else ref
+        if hi == lo:
+            assert torch.count_nonzero(g[e]) == 0
+        else:
+            close(g[e], ref, 1e-2, rows="none")

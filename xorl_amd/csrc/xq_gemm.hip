@@ -197,7 +197,8 @@ static int launch_tile_gemm_t(const xq_weight* w, bool contract_cols, const bf16
                               const int32_t* offsets, const int32_t* tile_offsets, const bf16_t* su, const bf16_t* lora_right,
                               int r_pad, const bf16_t* bias, bf16_t* C, int64_t ldc, hipStream_t stream, const char* who,
                               int force_T, int force_split, float* partial, int64_t partial_bytes,
-                              const TwoBanks* two = nullptr, const int32_t* a_rows = nullptr, int64_t a_span_rows = 0) {
+                              const TwoBanks* two = nullptr, const LowRankRight* right = nullptr, const int32_t* a_rows = nullptr,
+                              int64_t a_span_rows = 0) {
     const int64_t a_rows_span = a_rows ? a_span_rows : n_rows;      // rows of A that the launch may touch (0: not known)
     TileArgs g;
     g.A = A; g.lda = lda; g.C = C; g.ldc = ldc;
@@ -228,13 +229,16 @@ static int launch_tile_gemm_t(const xq_weight* w, bool contract_cols, const bf16
         }
     }
     g.n_rows = n_rows; g.offsets = offsets; g.tile_offsets = tile_offsets; g.num_experts = w->num_experts;
-    g.su = su; g.lora_right = lora_right; g.r_pad = (su && lora_right) ? r_pad : 0;
+    XQ_REQUIRE(!offsets || !right, "%s: expert banks take their right-hand factors as panels", who);
+    XQ_REQUIRE(offsets || !lora_right, "%s: internal error: a dense launch takes the right-hand factor as it is", who);
+    g.su = su; g.lora_right = lora_right; g.right = right ? *right : LowRankRight{}; g.r_pad = (su && (lora_right || right)) ? r_pad : 0;
     g.bias = bias;
     XQ_REQUIRE(g.Kc % BK == 0, "%s: contraction length %d must be a multiple of %d", who, g.Kc, BK);
     XQ_REQUIRE(g.Nout % 16 == 0, "%s: output width %d must be a multiple of 16", who, g.Nout);
     XQ_REQUIRE(lda % 8 == 0 && xq_aligned(A, 16), "%s: activation rows must be 16-byte aligned", who);
     XQ_REQUIRE(xq_aligned(w->packed, 16) && g.packed_stride % 16 == 0, "%s: packed weight must be 16-byte aligned", who);
-    XQ_REQUIRE(g.r_pad == 0 || (g.r_pad % 16 == 0 && g.r_pad <= 64 && xq_aligned(su, 16) && xq_aligned(lora_right, 16)),
+    XQ_REQUIRE(g.r_pad == 0 || (g.r_pad % 16 == 0 && g.r_pad <= 64 && xq_aligned(su, 16) && xq_aligned(lora_right, 16) &&
+                                (!right || (right->r >= 1 && right->r <= right->rp && right->rp * (right->f[1] ? 2 : 1) == r_pad))),
                "%s: bad low-rank side term (r_pad %d)", who, g.r_pad);
     if (w->format != XQ_FMT_FP8 && w->layout == XQ_LAYOUT_GKN)
         XQ_REQUIRE(w->rows % 2 == 0, "%s: GKN 4-bit storage needs an even row count", who);
@@ -259,11 +263,11 @@ static int launch_tile_gemm_t(const xq_weight* w, bool contract_cols, const bf16
         if (planned && plan.head_rows < n_rows) {
             const int64_t head = plan.head_rows;
             const int rc = launch_tile_gemm_t(w, contract_cols, A, lda, head, nullptr, nullptr, su, lora_right, r_pad,
-                                              bias, C, ldc, stream, who, 256, 1, nullptr, 0);
+                                              bias, C, ldc, stream, who, 256, 1, nullptr, 0, nullptr, right);
             if (rc) return rc;
             return launch_tile_gemm_t(w, contract_cols, A + head * lda, lda, n_rows - head, nullptr, nullptr,
                                       su ? su + head * r_pad : nullptr, lora_right, r_pad, bias, C + head * ldc, ldc,
-                                      stream, who, plan.tail_T, plan.tail_split, partial, partial_bytes);
+                                      stream, who, plan.tail_T, plan.tail_split, partial, partial_bytes, nullptr, right);
         }
         const int64_t tiles_m = xq_cdiv(n_rows, T) + (grouped ? w->num_experts : 0);
         const int64_t tiles_n = xq_cdiv(g.Nout, T);
@@ -277,7 +281,7 @@ static int launch_tile_gemm_t(const xq_weight* w, bool contract_cols, const bf16
             f.offsets = offsets;
             f.tile_prefix = !grouped ? nullptr : (T == 256 ? tile_offsets + (w->num_experts + 1) : tile_offsets);
             f.num_experts = w->num_experts;
-            f.su = g.r_pad ? su : nullptr; f.lora_right = g.r_pad ? lora_right : nullptr; f.r_pad = g.r_pad;
+            f.su = g.r_pad ? su : nullptr; f.lora_right = g.r_pad ? lora_right : nullptr; f.right = g.right; f.r_pad = g.r_pad;
             f.bias = bias;
             f.tiles_m = (int32_t)tiles_m; f.tiles_n = (int32_t)tiles_n;
             int ksplit = grouped || two_dense ? 1 : force_T ? force_split : planned ? plan.split : ksplit_for(tiles_m * tiles_n, T, g.Kc / BK);
@@ -341,9 +345,8 @@ static int launch_tile_gemm_t(const xq_weight* w, bool contract_cols, const bf16
 // gate | up | SwiGLU of a dense block-fp8 MLP in one launch: gu[M, 2I] = (x . deq(Wg)^T + side term | x . deq(Wu)^T +
 // side term) and h[M, I] = bf16(silu(gate)) * up from the rounded projections.  Both weights [I, K] block-fp8.
 int launch_gate_up_swiglu(const xq_weight* wg, const xq_weight* wu, const bf16_t* x, int64_t ldx, int64_t M,
-                          const bf16_t* su_g, const bf16_t* su_u, int64_t ld_su, const bf16_t* lr_g, const bf16_t* lr_u,
-                          int r_pad, const bf16_t* bias_g, const bf16_t* bias_u, bf16_t* gu, int64_t ldgu, bf16_t* h,
-                          int64_t ldh, hipStream_t stream) {
+                          const bf16_t* su_g, const bf16_t* su_u, int64_t ld_su, const LowRankRight& right, int r_pad, const bf16_t* bias_g,
+                          const bf16_t* bias_u, bf16_t* gu, int64_t ldgu, bf16_t* h, int64_t ldh, hipStream_t stream) {
     static const char* who = "gate_up_swiglu";
     XQ_REQUIRE(wg->format == XQ_FMT_FP8 && wu->format == XQ_FMT_FP8 && wg->rows == wu->rows && wg->cols == wu->cols,
                "%s: two block-fp8 weights of one shape", who);
@@ -353,9 +356,9 @@ int launch_gate_up_swiglu(const xq_weight* wg, const xq_weight* wu, const bf16_t
                "%s: operands must be 16-byte aligned", who);
     XQ_REQUIRE(ldgu % 8 == 0 && ldh % 8 == 0 && xq_aligned(gu, 16) && xq_aligned(h, 16), "%s: output rows must be 16-byte aligned", who);
     XQ_REQUIRE(xq_aligned(bias_g, 8) && xq_aligned(bias_u, 8), "%s: bias vectors must be 8-byte aligned", who);
-    const bool side = su_g && su_u && lr_g && lr_u && r_pad > 0;
+    const bool side = su_g && su_u && right.f[0] && right.f[1] && r_pad > 0;
     XQ_REQUIRE(!side || (r_pad % 16 == 0 && r_pad <= 64 && ld_su >= r_pad && ld_su % 8 == 0 && xq_aligned(su_g, 16) &&
-                         xq_aligned(su_u, 16) && xq_aligned(lr_g, 16) && xq_aligned(lr_u, 16)),
+                         xq_aligned(su_u, 16)),
                "%s: bad low-rank side term", who);
     if (M == 0) return XQ_OK;
     G256Args f{};
@@ -366,7 +369,7 @@ int launch_gate_up_swiglu(const xq_weight* wg, const xq_weight* wu, const bf16_t
     f.Kc = (int32_t)K; f.Nout = (int32_t)I; f.M = M;
     f.num_experts = 1;
     f.su = side ? su_g : nullptr; f.su2 = side ? su_u : nullptr; f.ld_su = ld_su;
-    f.lora_right = side ? lr_g : nullptr; f.lora_right2 = side ? lr_u : nullptr; f.r_pad = side ? r_pad : 0;
+    f.right = right; f.r_pad = side ? r_pad : 0;
     f.bias = bias_g; f.bias2 = bias_u;
     f.tiles_m = (int32_t)xq_cdiv(M, 256); f.tiles_n = (int32_t)xq_cdiv(I, 128);
     f.ksplit = 1;
@@ -390,10 +393,11 @@ int launch_gate_up_swiglu(const xq_weight* wg, const xq_weight* wu, const bf16_t
 int launch_tile_gemm(const xq_weight* w, bool contract_cols, const bf16_t* A, int64_t lda, int64_t n_rows,
                      const int32_t* offsets, const int32_t* tile_offsets, const bf16_t* su, const bf16_t* lora_right,
                      int r_pad, const bf16_t* bias, bf16_t* C, int64_t ldc, hipStream_t stream, const char* who,
-                     float* partial, int64_t partial_bytes, const TwoBanks* two, const int32_t* a_rows, int64_t a_span_rows) {
+                     float* partial, int64_t partial_bytes, const TwoBanks* two, const LowRankRight* right, const int32_t* a_rows,
+                     int64_t a_span_rows) {
     XQ_REQUIRE(!a_rows || offsets, "%s: a row map goes with a grouped launch", who);
     return launch_tile_gemm_t(w, contract_cols, A, lda, n_rows, offsets, tile_offsets, su, lora_right, r_pad, bias, C, ldc,
-                              stream, who, 0, 1, partial, partial_bytes, two, a_rows, a_span_rows);
+                              stream, who, 0, 1, partial, partial_bytes, two, right, a_rows, a_span_rows);
 }
 
 // whether a grouped launch over this bank runs on the pipelined tile kernel, which can read its activation rows through
@@ -473,12 +477,10 @@ extern "C" int64_t xq_linear_workspace_bytes(int64_t M, int64_t N, int64_t K, in
     const int64_t pb = align256(tile_gemm_partial_bytes(M, K, N));
     int64_t need = (pf > pb ? pf : pb) + 256;
     if (rp) {
-        int64_t fwd = align256(rp * K * 2) + align256(N * rp * 2) + align256(M * rp * 2) + pf;
-        int64_t tnp = tn_partial_bytes(M, N, rp);
-        int64_t tnk = tn_partial_bytes(M, K, rp);
-        int64_t tn = align256(tnp > tnk ? tnp : tnk);     // the weight-gradient partials reuse the dgrad's region
-        int64_t bwd = align256(rp * N * 2) + align256(K * rp * 2) + align256(rp * K * 2) + 2 * align256(M * rp * 2) +
-                      (tn > pb ? tn : pb);
+        const int64_t panel = lowrank_panel_bytes(1, M, rp, K);
+        int64_t fwd = align256(M * rp * 2) + panel + pf;
+        int64_t tn = tn_partial_bytes(M, N, rp) + tn_partial_bytes(M, K, rp);     // the weight-gradient partials reuse the dgrad's region
+        int64_t bwd = 2 * align256(M * rp * 2) + panel + (tn > pb ? tn : pb);
         need = (fwd > bwd ? fwd : bwd) + 256;
     }
     return need > skinny ? need : skinny;
@@ -510,25 +512,22 @@ extern "C" int xq_linear_fwd(const xq_weight* w, const void* x, int64_t ldx, int
     if (!su_out && g_skinny_enabled && skinny_supported(w, M))
         return launch_skinny(w, (const bf16_t*)x, ldx, M, lora_A, lora_B, lora_dtype, r, scaling,
                              (const bf16_t*)bias_bf16, (bf16_t*)y, ldy, workspace, workspace_bytes, stream);
-    bf16_t *A_bf = nullptr, *Bl = nullptr, *su = nullptr;
+    bf16_t* su = nullptr;
+    const LowRankRight right{{lora_B, nullptr}, r, r, rp, lora_dtype == XQ_DT_F32, 0};
     Carver cv{(workspace && xq_aligned(workspace, 256)) ? (uint8_t*)workspace : nullptr, 0, workspace_bytes};
     if (rp) {
         XQ_REQUIRE(workspace && xq_aligned(workspace, 256) && workspace_bytes >= xq_linear_workspace_bytes(M, N, K, r),
                    "xq_linear_fwd: workspace missing, misaligned or smaller than xq_linear_workspace_bytes()");
-        A_bf = (bf16_t*)cv.take(rp * K * 2);
-        Bl = (bf16_t*)cv.take(N * rp * 2);
         su = su_out ? (bf16_t*)su_out : (bf16_t*)cv.take(M * rp * 2);
-        FactorPrepJobs jobs{};
-        jobs.in_f32 = lora_dtype == XQ_DT_F32;
-        jobs.add(lora_A, r, K, false, A_bf, rp, K);
-        jobs.add(lora_B, N, r, false, Bl, N, rp);
-        if ((rc = launch_factor_prep_multi(jobs, stream))) return rc;
-        if ((rc = launch_small_nt((const bf16_t*)x, ldx, M, K, A_bf, rp, scaling, su, nullptr, nullptr, 1, true, stream))) return rc;
+        bf16_t* panel = (bf16_t*)cv.take(lowrank_panel_bytes(1, M, rp, K));
+        const LowRankJob job{(const bf16_t*)x, ldx, K, {lora_A, nullptr}, 1, r, rp, scaling, su, rp, 0};
+        if ((rc = launch_lowrank(&job, 1, M, factor_mode(lora_dtype, false), panel, stream))) return rc;
     }
     // what is left of the workspace holds split-K partial sums (small row counts); without it the launch is unsplit
     float* partial = (float*)cv.take(0);
-    return launch_tile_gemm(w, true, (const bf16_t*)x, ldx, M, nullptr, nullptr, su, Bl, rp, (const bf16_t*)bias_bf16,
-                            (bf16_t*)y, ldy, stream, "xq_linear_fwd", partial, partial ? workspace_bytes - cv.used : 0);
+    return launch_tile_gemm(w, true, (const bf16_t*)x, ldx, M, nullptr, nullptr, su, nullptr, rp, (const bf16_t*)bias_bf16,
+                            (bf16_t*)y, ldy, stream, "xq_linear_fwd", partial, partial ? workspace_bytes - cv.used : 0, nullptr,
+                            rp ? &right : nullptr);
 }
 
 // ---- forward for callers that cannot allocate ------------------------------------------------------------------
@@ -740,29 +739,23 @@ extern "C" int xq_linear_bwd(const xq_weight* w, const void* x, int64_t ldx, con
         if (dB && (rc = launch_zero_fill(dB, N * r * 4, stream))) return rc;
         return XQ_OK;
     }
-    bf16_t *Bt = nullptr, *At = nullptr, *v = nullptr;
+    bf16_t* v = nullptr;
     const bf16_t* su = (const bf16_t*)su_in;
+    const LowRankRight right{{lora_A, nullptr}, K, r, rp, lora_dtype == XQ_DT_F32, 1};
     float* partial = nullptr;
     Carver cv{(workspace && xq_aligned(workspace, 256)) ? (uint8_t*)workspace : nullptr, 0, workspace_bytes};
     if (rp) {
         XQ_REQUIRE(workspace && xq_aligned(workspace, 256) && workspace_bytes >= xq_linear_workspace_bytes(M, N, K, r),
                    "xq_linear_bwd: workspace missing, misaligned or smaller than xq_linear_workspace_bytes()");
-        Bt = (bf16_t*)cv.take(rp * N * 2);
-        At = (bf16_t*)cv.take(K * rp * 2);
-        bf16_t* A_bf = (bf16_t*)cv.take(rp * K * 2);
         v = (bf16_t*)cv.take(M * rp * 2);
         bf16_t* su_ws = (bf16_t*)cv.take(M * rp * 2);
-        // every factor layout this call needs, in one launch
-        FactorPrepJobs jobs{};
-        jobs.in_f32 = lora_dtype == XQ_DT_F32;
-        jobs.add(lora_B, N, r, true, Bt, rp, N);
-        if (dx) jobs.add(lora_A, r, K, true, At, K, rp);
-        if (dB && !su) jobs.add(lora_A, r, K, false, A_bf, rp, K);
-        if ((rc = launch_factor_prep_multi(jobs, stream))) return rc;
+        bf16_t* panel = (bf16_t*)cv.take(lowrank_panel_bytes(1, M, rp, K));
         // v = bf16(s * dy . B)   [M, rp]
-        if ((rc = launch_small_nt((const bf16_t*)dy, lddy, M, N, Bt, rp, scaling, v, nullptr, nullptr, 1, true, stream))) return rc;
+        const LowRankJob jv{(const bf16_t*)dy, lddy, N, {lora_B, nullptr}, 1, r, rp, scaling, v, rp, 0};
+        if ((rc = launch_lowrank(&jv, 1, M, factor_mode(lora_dtype, true), nullptr, stream))) return rc;
         if (dB && !su) {
-            if ((rc = launch_small_nt((const bf16_t*)x, ldx, M, K, A_bf, rp, scaling, su_ws, nullptr, nullptr, 1, true, stream))) return rc;
+            const LowRankJob ju{(const bf16_t*)x, ldx, K, {lora_A, nullptr}, 1, r, rp, scaling, su_ws, rp, 0};
+            if ((rc = launch_lowrank(&ju, 1, M, factor_mode(lora_dtype, false), panel, stream))) return rc;
             su = su_ws;
         }
     }
@@ -771,14 +764,17 @@ extern "C" int xq_linear_bwd(const xq_weight* w, const void* x, int64_t ldx, con
     partial = (float*)cv.take(0);
     if (dx) {
         XQ_REQUIRE(lddx % 8 == 0 && xq_aligned(dx, 16), "xq_linear_bwd: dx rows must be 16-byte aligned");
-        if ((rc = launch_tile_gemm(w, false, (const bf16_t*)dy, lddy, M, nullptr, nullptr, v, At, rp, nullptr, (bf16_t*)dx,
-                                   lddx, stream, "xq_linear_bwd(dx)", partial, partial ? workspace_bytes - cv.used : 0)))
+        if ((rc = launch_tile_gemm(w, false, (const bf16_t*)dy, lddy, M, nullptr, nullptr, v, nullptr, rp, nullptr, (bf16_t*)dx,
+                                   lddx, stream, "xq_linear_bwd(dx)", partial, partial ? workspace_bytes - cv.used : 0, nullptr,
+                                   rp ? &right : nullptr)))
             return rc;
     }
     // dB[N, r] = dy^T . su ; dA[r, K] = (x^T . v)^T
-    if (dB && (rc = launch_tn((const bf16_t*)dy, lddy, N, su, rp, r, M, false, dB, partial, nullptr, 1, stream))) return rc;
-    if (dA && (rc = launch_tn((const bf16_t*)x, ldx, K, v, rp, r, M, true, dA, partial, nullptr, 1, stream))) return rc;
-    return XQ_OK;
+    TnJob jobs[2];
+    int n = 0;
+    if (dB) jobs[n++] = TnJob{(const bf16_t*)dy, lddy, N, su, rp, rp, r, false, dB};
+    if (dA) jobs[n++] = TnJob{(const bf16_t*)x, ldx, K, v, rp, rp, r, true, dA};
+    return n ? launch_tn_multi(jobs, n, M, partial, stream) : XQ_OK;
 }
 
 extern "C" int xq_grouped_gemm(const xq_weight* w, int transpose_w, const void* a, int64_t lda, int64_t n_rows,

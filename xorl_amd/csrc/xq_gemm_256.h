@@ -31,6 +31,7 @@
 #pragma once
 
 #include "xq_common.h"
+#include "xq_lora.h"
 
 namespace xq {
 
@@ -80,7 +81,8 @@ struct G256Args {
     const int32_t* tile_prefix;// grouped: [E+1] prefix of ceil(count / tile rows)
     int32_t num_experts;
     const bf16_t* su;          // [M, r_pad] or NULL
-    const bf16_t* lora_right;  // [E][Nout, r_pad] or NULL
+    const bf16_t* lora_right;  // [E][Nout, r_pad] panels (grouped), or NULL: `right` (dense)
+    LowRankRight right;
     int32_t r_pad;
     const bf16_t* bias;
     int32_t tiles_m, tiles_n;  // grouped: tiles_m is an upper bound
@@ -747,11 +749,12 @@ __global__ void __launch_bounds__(2 * T, 2) gemm_256_kernel(G256Args g) {
                     *(u32x4*)(As + F8_A_STAGE + swz(r, c)) = *(const u32x4*)(g.su2 + row * g.ld_su + c * 8);
                     int n = cur.n0 + (r & 127);
                     n = n < g.Nout ? n : g.Nout - 1;
-                    *(u32x4*)(Bs + swz(r, c)) = *(const u32x4*)((r < 128 ? g.lora_right : g.lora_right2) + (int64_t)n * rp + c * 8);
+                    *(u32x4*)(Bs + swz(r, c)) = right_chunk(g.right, r < 128 ? 0 : 1, n, c);
                 } else {
                     int n = cur.n0w + r;
                     n = n < cur.bank_width ? n : cur.bank_width - 1;
-                    *(u32x4*)(Bs + swz(r, c)) = *(const u32x4*)(lr + (int64_t)n * rp + c * 8);
+                    if constexpr (GROUPED) *(u32x4*)(Bs + swz(r, c)) = *(const u32x4*)(lr + (int64_t)n * rp + c * 8);
+                    else *(u32x4*)(Bs + swz(r, c)) = right_chunk(g.right, -1, n, c);
                 }
             }
             __syncthreads();

@@ -419,7 +419,8 @@ __global__ void __launch_bounds__(NW * 64, NW == 8 ? 2 : 1) gemm_dtl16_kernel(G2
             n = n < bank_width ? n : bank_width - 1;
             const u32x4 z = {0, 0, 0, 0};
             *(u32x4*)(As + swz(r, c)) = c < have ? *(const u32x4*)(su_b + row * g.ld_su + c * 8) : z;
-            *(u32x4*)(Bs + swz(r, c)) = c < have ? *(const u32x4*)(lr + (int64_t)n * rp + c * 8) : z;
+            if constexpr (GROUPED) *(u32x4*)(Bs + swz(r, c)) = c < have ? *(const u32x4*)(lr + (int64_t)n * rp + c * 8) : z;
+            else *(u32x4*)(Bs + swz(r, c)) = c < have ? right_chunk(g.right, -1, n, c) : z;
         }
         __syncthreads();
         for (int ks = 0; ks < steps; ++ks) {

@@ -14,6 +14,7 @@
 #pragma once
 
 #include "xq_common.h"
+#include "xq_lora.h"
 
 namespace xq {
 
@@ -37,7 +38,8 @@ struct TileArgs {
     const int32_t* tile_offsets;          // grouped: [E+1] prefix of ceil(count/BM)
     int32_t num_experts;
     const bf16_t* su;                     // [rows, r_pad] or NULL
-    const bf16_t* lora_right;             // [E][Nout][r_pad] or NULL
+    const bf16_t* lora_right;             // [E][Nout][r_pad] panels, or NULL: `right` (dense)
+    LowRankRight right;
     int32_t r_pad;
     const bf16_t* bias;                   // [Nout] or NULL
 };
@@ -293,7 +295,8 @@ __global__ void __launch_bounds__(256) gemm_tile_kernel(TileArgs g) {
             *(u32x4*)(As + r * LDS_PITCH + c) = *(const u32x4*)(g.su + row * rp + c);
             int n = n0 + r;
             n = n < g.Nout ? n : g.Nout - 1;
-            *(u32x4*)(Bs + r * LDS_PITCH + c) = *(const u32x4*)(g.lora_right + ((int64_t)e * g.Nout + n) * rp + c);
+            *(u32x4*)(Bs + r * LDS_PITCH + c) = g.lora_right ? *(const u32x4*)(g.lora_right + ((int64_t)e * g.Nout + n) * rp + c)
+                                                             : right_chunk(g.right, -1, n, c >> 3);
         }
         __syncthreads();
         mma_steps(rp / 16);

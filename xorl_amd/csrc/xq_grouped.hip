@@ -204,10 +204,10 @@ extern "C" int xq_grouped_fwd(const xq_weight* gate, const xq_weight* up, const 
     }
     if (fuse_gate_up(gate, up)) {       // both projections in one launch: column tiles past I take the up bank
         const TwoBanks two{up, su_u, Lr_uB};
-        if ((rc = launch_tile_gemm(gate, false, xr, ld_xr, R, off, toff, su_g, Lr_gB, rp, nullptr, gu, 2 * I, stream, who, nullptr, 0, &two, xr_rows, d.T))) return rc;
+        if ((rc = launch_tile_gemm(gate, false, xr, ld_xr, R, off, toff, su_g, Lr_gB, rp, nullptr, gu, 2 * I, stream, who, nullptr, 0, &two, nullptr, xr_rows, d.T))) return rc;
     } else {
-        if ((rc = launch_tile_gemm(gate, false, xr, ld_xr, R, off, toff, su_g, Lr_gB, rp, nullptr, gu, 2 * I, stream, who, nullptr, 0, nullptr, xr_rows, d.T))) return rc;
-        if ((rc = launch_tile_gemm(up, false, xr, ld_xr, R, off, toff, su_u, Lr_uB, rp, nullptr, gu + I, 2 * I, stream, who, nullptr, 0, nullptr, xr_rows, d.T))) return rc;
+        if ((rc = launch_tile_gemm(gate, false, xr, ld_xr, R, off, toff, su_g, Lr_gB, rp, nullptr, gu, 2 * I, stream, who, nullptr, 0, nullptr, nullptr, xr_rows, d.T))) return rc;
+        if ((rc = launch_tile_gemm(up, false, xr, ld_xr, R, off, toff, su_u, Lr_uB, rp, nullptr, gu + I, 2 * I, stream, who, nullptr, 0, nullptr, nullptr, xr_rows, d.T))) return rc;
     }
     if ((rc = xq_moe_scatter_scalar(routing_w, rw_dtype, saved->scatter_index, R, saved->w_row, stream))) return rc;
     // SwiGLU (times the row's routing weight) and s * h . A_d^T of the down projection: one pass where the rank allows
@@ -325,7 +325,7 @@ extern "C" int xq_grouped_bwd(const xq_weight* gate, const xq_weight* up, const 
     const bf16_t* gd = in_place ? (const bf16_t*)dy : g_down;      // the routed gradient rows: dy through the map, or the copy
     const int64_t ld_gd = in_place ? ld_dy : H;
     const int32_t* gd_rows = in_place ? token_of_row : nullptr;
-    if ((rc = launch_tile_gemm(down, true, gd, ld_gd, R, off, toff, v_d, Lr_dA, rp, nullptr, dh, I, stream, who, nullptr, 0, nullptr, gd_rows, d.T))) return rc;
+    if ((rc = launch_tile_gemm(down, true, gd, ld_gd, R, off, toff, v_d, Lr_dA, rp, nullptr, dh, I, stream, who, nullptr, 0, nullptr, nullptr, gd_rows, d.T))) return rc;
     if ((rc = launch_tn(gd, ld_gd, H, su_d, rp, r, R, true, grads->dB[2], wg, dBe == 1 ? nullptr : off, E, stream, n_valid, 0, gd_rows))) return rc;   // [E|1, r, H]
     if ((rc = launch_tn(h, I, I, v_d, rp, r, R, false, grads->dA[2], wg, dAe == 1 ? nullptr : off, E, stream, n_valid))) return rc;        // [E|1, I, r]
 
@@ -333,7 +333,7 @@ extern "C" int xq_grouped_bwd(const xq_weight* gate, const xq_weight* up, const 
     // one pass over (gate, up, dh) where the rank allows, so that the two products do not read dgate | dup back
     static const bool silu_nt = [] { const char* e = getenv("XQ_MLP_SILU_NT"); return e ? atoi(e) != 0 : true; }();
     if (silu_nt && silu_bwd_nt_supported(I, rp)) {
-        if ((rc = launch_silu_bwd_nt(gu, gu + I, 2 * I, dh, I, dgate, dup, 2 * I, R, I, F_gB, F_uB, rp, s, v_g, v_u, ld_v, stream, off, toff, E,
+        if ((rc = launch_silu_bwd_nt(gu, gu + I, 2 * I, dh, I, dgate, dup, 2 * I, R, I, F_gB, F_uB, kFacBf16, rp, rp, s, v_g, v_u, ld_v, nullptr, stream, off, toff, E,
                                      gBe == 1, uBe == 1, saved->w_row, d_w_row, limit)))
             return rc;
     } else {

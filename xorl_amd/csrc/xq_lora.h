@@ -7,21 +7,55 @@
 
 namespace xq {
 
-// out[i][j] (bf16, [R_out, C_out], zero padded) = in[i][j] or in[j][i];  `in` is
-// fp32 or bf16 with shape [R_in, C_in] per expert.
-// up to three single-matrix conversions (same source dtype) done by one launch
-struct FactorPrepJobs {
-    const void* in[3];
-    bf16_t* out[3];
-    int64_t R_in[3], C_in[3], R_out[3], C_out[3];
-    int transpose[3];
-    int in_f32, n;
-    void add(const void* src, int64_t r_in, int64_t c_in, bool tr, bf16_t* dst, int64_t r_out, int64_t c_out) {
-        in[n] = src; out[n] = dst; R_in[n] = r_in; C_in[n] = c_in; R_out[n] = r_out; C_out[n] = c_out; transpose[n] = tr ? 1 : 0;
-        ++n;
-    }
+// The right-hand factor of a low-rank side term as the caller holds it: element (n, j), j < r, is f[n * ld + j], or f[j * ld + n]
+// (transposed); columns from r to rp are zero.  With two factors (f[1] != NULL) the columns rp .. 2 rp are the second one's.
+// The GEMM kernels round it to bf16 while they stage it: a dense call has no pass that prepares panels.
+struct LowRankRight {
+    const void* f[2];
+    int64_t ld;
+    int32_t r, rp;
+    int32_t f32, transposed;
 };
-int launch_factor_prep_multi(const FactorPrepJobs& jobs, hipStream_t stream);
+// 8 consecutive columns (chunk c) of row n, packed bf16; `which` >= 0 names the factor, < 0: by column
+__device__ __forceinline__ u32x4 right_chunk(const LowRankRight& q, int which, int n, int c) {
+    int j0 = c * 8, k = which;
+    if (k < 0) {
+        k = q.f[1] != nullptr && j0 >= q.rp ? 1 : 0;
+        j0 -= k * q.rp;
+    }
+    const void* f = k ? q.f[1] : q.f[0];
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const int j = j0 + e < q.r ? j0 + e : q.r - 1;
+        const int64_t i = q.transposed ? j * q.ld + n : n * q.ld + j;
+        v[e] = q.f32 ? ((const float*)f)[i] : bf16_to_f32(((const bf16_t*)f)[i]);
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = j0 + e < q.r ? v[e] : 0.0f;
+    return u32x4{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7])};
+}
+
+// the form a factor of a low-rank product comes in: [r, K] (rows along the contraction) or transposed, [K, r]
+enum FactorMode { kFacBf16 = 0, kFacF32 = 1, kFacF32T = 2, kFacBf16T = 3 };
+inline FactorMode factor_mode(int lora_dtype, bool transposed) {
+    return lora_dtype == XQ_DT_F32 ? (transposed ? kFacF32T : kFacF32) : (transposed ? kFacBf16T : kFacBf16);
+}
+
+// T[rows, rp] = bf16(scale * In[rows, Kc] . F^T), dense rows, up to kLowRankJobs products in one launch.  nf = 2: a second
+// factor of the same rank against the same rows, its result at T + t_step.  Ranks from r to rp come out zero.
+constexpr int kLowRankJobs = 4;
+struct LowRankJob {
+    const bf16_t* In;
+    int64_t ld_in, Kc;
+    const void* F[2];
+    int32_t nf, r, rp;
+    float scale;
+    bf16_t* T;
+    int64_t ld_t, t_step;
+};
+int64_t lowrank_panel_bytes(int n, int64_t n_rows, int cols, int64_t Kc);   // scratch a launch of n products (nf * rp = cols each) may want
+int launch_lowrank(const LowRankJob* jobs, int n, int64_t n_rows, FactorMode mode, bf16_t* panels, hipStream_t stream);
 
 // Every LoRA panel of a call in one launch: job k converts a [n_src, R_in, C_in] fp32 / bf16 factor (n_src = 1 or
 // the expert count) into bf16 [n_out, R_out, C_out], optionally transposed, zero padded; n_src == 1 < n_out repeats
@@ -51,9 +85,7 @@ int launch_panel_prep(const PanelJobs& jobs, hipStream_t stream);
 int launch_factor_prep(const void* in, int in_dtype, int64_t R_in, int64_t C_in, bool transpose,
                        bf16_t* out, int64_t R_out, int64_t C_out, int64_t num_experts, hipStream_t stream);
 
-// T[rows, r_pad] = bf16(scale * In[rows, Kc] . F[r_pad, Kc]^T).
-//   dense (offsets == NULL): rows = n_rows, one F;
-//   grouped: rows in expert order, F[e] = F + e*r_pad*Kc (or shared).
+// T[rows, r_pad] = bf16(scale * In[rows, Kc] . F[r_pad, Kc]^T), rows in expert order, F[e] = F + e*r_pad*Kc (or shared).
 int launch_small_nt(const bf16_t* In, int64_t ld_in, int64_t n_rows, int64_t Kc, const bf16_t* F,
                     int r_pad, float scale, bf16_t* T, const int32_t* offsets,
                     const int32_t* tile_offsets, int32_t num_experts, bool shared_f, hipStream_t stream,
@@ -64,23 +96,24 @@ int launch_small_nt(const bf16_t* In, int64_t ld_in, int64_t n_rows, int64_t Kc,
 
 // SwiGLU backward and the two low-rank products of its outputs in one pass (r_pad 16 or 32): dgate | dup as
 // xq_silu_mul_bwd writes them, Tg = scale * dgate . Fg^T, Tu = scale * dup . Fu^T as two
-// launch_small_nt calls on them would (same bits)
+// a low-rank launch on them would.  `partial`: silu_nt_partial_bytes() of scratch (dense; NULL keeps one block per 32 rows)
 bool silu_bwd_nt_supported(int64_t cols, int r_pad);
+int64_t silu_nt_partial_bytes(int64_t n_rows, int64_t cols, int r_pad);
 int launch_silu_bwd_nt(const bf16_t* gate, const bf16_t* up, int64_t ld_gu, const bf16_t* dh, int64_t ld_dh, bf16_t* dgate,
-                       bf16_t* dup, int64_t ld_out, int64_t n_rows, int64_t cols, const bf16_t* Fg, const bf16_t* Fu, int r_pad,
-                       float scale, bf16_t* Tg, bf16_t* Tu, int64_t ld_t, hipStream_t stream,
+                       bf16_t* dup, int64_t ld_out, int64_t n_rows, int64_t cols, const void* Fg, const void* Fu, FactorMode mode, int r, int r_pad,
+                       float scale, bf16_t* Tg, bf16_t* Tu, int64_t ld_t, float* partial, hipStream_t stream,
                        // routed rows in expert order (offsets != NULL): a factor pair per expert ([E][r_pad][cols]) unless
                        // shared, the rows' routing weights applied and (d_row_w != NULL) their gradients written
                        const int32_t* offsets = nullptr, const int32_t* tile_offsets = nullptr, int32_t num_experts = 1,
                        bool shared_fg = true, bool shared_fu = true, const float* row_w = nullptr, float* d_row_w = nullptr,
                        float swiglu_limit = 0.0f);     // > 0: the gate pre-activation is clamped to [-limit, limit], its gradient masked outside
 
-// the forward in the same organisation: h = SwiGLU(gate, up) as xq_silu_mul_fwd writes it (routed rows: times the row's
-// weight) and T = scale * h . F^T as launch_small_nt on h would (same bits)
+// the forward in the same organisation: h = SwiGLU(gate, up) (routed rows: times the row's weight), T = scale * h . F^T, F as
+// bf16 panels; dense rows in blocks of 32 over all columns, for launches that fill the chip so
 int launch_silu_fwd_nt(const bf16_t* gate, const bf16_t* up, int64_t ld_gu, bf16_t* h, int64_t ld_h, int64_t n_rows, int64_t cols,
-                       const bf16_t* F, int r_pad, float scale, bf16_t* T, int64_t ld_t, hipStream_t stream,
-                       const int32_t* offsets = nullptr, const int32_t* tile_offsets = nullptr, int32_t num_experts = 1,
-                       bool shared_f = true, const float* row_w = nullptr, float swiglu_limit = 0.0f);
+                       const bf16_t* F, int r_pad, float scale, bf16_t* T, int64_t ld_t, hipStream_t stream, const int32_t* offsets = nullptr,
+                       const int32_t* tile_offsets = nullptr, int32_t num_experts = 1, bool shared_f = true, const float* row_w = nullptr,
+                       float swiglu_limit = 0.0f);
 
 // xq_silu_mul_fwd / xq_silu_mul_bwd with a SwiGLU limit on the gate pre-activation (ops/moe/triton.py:127-141; <= 0: none)
 int silu_mul_fwd_limit(const void* gate, const void* up, int64_t ld_in, const float* row_w, void* h, int64_t ld_h, int64_t rows,
@@ -93,6 +126,22 @@ int silu_mul_bwd_limit(const void* gate, const void* up, int64_t ld_in, const vo
 //          ([splits][width][r_pad] fp32) reduced in fixed order (deterministic);
 //   grouped: out[e] over rows [offsets[e], offsets[e+1]); zero for empty experts.
 // r_out is the number of valid columns of Q (<= r_pad) written.
+// Dense products of the same rows can share a launch (launch_tn_multi): their partials lie one after the other,
+// tn_partial_bytes() each.  out2 (may be NULL): columns of Q from split_j on are a second result's columns.
+constexpr int kTnJobs = 6;
+struct TnJob {
+    const bf16_t* P;
+    int64_t ldp, width;
+    const bf16_t* Q;
+    int64_t ldq;
+    int32_t r_pad, r_out;
+    bool transpose_out;
+    float* out;
+    const int32_t* p_rows;
+    float* out2;
+    int32_t split_j;
+};
+int launch_tn_multi(const TnJob* jobs, int n, int64_t n_rows, float* partial, hipStream_t stream, const int32_t* row_limit = nullptr);
 int64_t tn_partial_bytes(int64_t n_rows, int64_t width, int r_pad);
 int launch_tn(const bf16_t* P, int64_t ldp, int64_t width, const bf16_t* Q, int r_pad, int r_out,
               int64_t n_rows, bool transpose_out, float* out, float* partial,
@@ -115,13 +164,14 @@ int64_t tile_gemm_partial_bytes(int64_t n_rows, int64_t Nout, int64_t Kc);   // 
 bool two_banks_supported(const xq_weight* w);
 bool two_dense_supported(const xq_weight* w);   // dense [N, K] pair: one dgrad launch, dX = [dY1 | dY2] . [W1 ; W2]
 int launch_gate_up_swiglu(const xq_weight* wg, const xq_weight* wu, const bf16_t* x, int64_t ldx, int64_t M,
-                          const bf16_t* su_g, const bf16_t* su_u, int64_t ld_su, const bf16_t* lr_g, const bf16_t* lr_u,
+                          const bf16_t* su_g, const bf16_t* su_u, int64_t ld_su, const LowRankRight& right,
                           int r_pad, const bf16_t* bias_g, const bf16_t* bias_u, bf16_t* gu, int64_t ldgu, bf16_t* h,
                           int64_t ldh, hipStream_t stream);
 int launch_tile_gemm(const xq_weight* w, bool contract_cols, const bf16_t* A, int64_t lda, int64_t n_rows,
                      const int32_t* offsets, const int32_t* tile_offsets, const bf16_t* su, const bf16_t* lora_right,
                      int r_pad, const bf16_t* bias, bf16_t* C, int64_t ldc, hipStream_t stream, const char* who,
                      float* partial, int64_t partial_bytes, const TwoBanks* two = nullptr,
+                     const LowRankRight* right = nullptr,   // dense: the side term's right-hand factor (then lora_right is NULL)
                      const int32_t* a_rows = nullptr,    // grouped, optional: row i of the problem is row a_rows[i] of A,
                      int64_t a_span_rows = 0);           // ... which has this many rows (0: not known)
 bool tile_gemm_takes_row_map(const xq_weight* w);        // ... which only the pipelined tile kernel does

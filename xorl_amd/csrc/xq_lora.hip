@@ -51,32 +51,6 @@ int launch_factor_prep(const void* in, int in_dtype, int64_t R_in, int64_t C_in,
     return XQ_OK;
 }
 
-// Two or three dense factor conversions in one launch (blockIdx.y = job): the linear entry points prepare both
-// factors of a call together, which matters where a step is a dozen short launches.
-__global__ void __launch_bounds__(256) factor_prep_multi_kernel(FactorPrepJobs j) {
-    const int k = blockIdx.y;
-    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    const int64_t R_out = j.R_out[k], C_out = j.C_out[k], R_in = j.R_in[k], C_in = j.C_in[k];
-    if (t >= R_out * C_out) return;
-    const int64_t i = t / C_out, c = t - i * C_out;
-    const int64_t si = j.transpose[k] ? c : i, sj = j.transpose[k] ? i : c;
-    float v = 0.0f;
-    if (si < R_in && sj < C_in) {
-        const int64_t idx = si * C_in + sj;
-        v = j.in_f32 ? ((const float*)j.in[k])[idx] : bf16_to_f32(((const bf16_t*)j.in[k])[idx]);
-    }
-    j.out[k][t] = to_bf16(v);
-}
-
-int launch_factor_prep_multi(const FactorPrepJobs& j, hipStream_t stream) {
-    int64_t most = 0;
-    for (int k = 0; k < j.n; ++k) most = j.R_out[k] * j.C_out[k] > most ? j.R_out[k] * j.C_out[k] : most;
-    if (j.n == 0 || most == 0) return XQ_OK;
-    factor_prep_multi_kernel<<<dim3((unsigned)xq_cdiv(most, 256), (unsigned)j.n), 256, 0, stream>>>(j);
-    XQ_CHECK_LAUNCH("factor_prep_multi");
-    return XQ_OK;
-}
-
 // A block converts one tile of a destination panel through LDS -- 16 x 256 (rows x columns) of a wide panel, 256 x 16
 // of a tall one -- so that both the source and the destination are touched in whole row pieces whichever way the job
 // transposes: e.g. a transposing job into a wide panel reads 256 source rows of 16 entries (one contiguous run when
@@ -173,8 +147,7 @@ struct SmallNtArgs {
     int64_t ld_copy;
 };
 
-// TR rows per block: 32 (dense; the 4 waves split K) or 128 (grouped; one wave per 32 rows).  FJ = rows of F in
-// use / 4 (4, 8, 12 or 16).
+// 128 rows of one expert per block, a wave per 32 rows.  FJ = rows of F in use / 4 (4, 8, 12 or 16).
 // Both operands are fetched with coalesced 16-byte loads (16 lanes per 256-byte row piece, 4 rows
 // per instruction) and reach the MFMA operand layout through wave-private LDS tiles of 128 k per
 // row (row pitch 272 B: the 16 lanes of a b128 read phase hit distinct banks); per-lane row-strided
@@ -184,19 +157,19 @@ struct SmallNtArgs {
 // valid ones and their values never used -- so the waits count exactly and the loads of chunk k+2 stay in
 // flight while chunk k is multiplied.
 constexpr int SN_P = 136;   // LDS row pitch in bf16 elements
-template <int TR, int FJ, bool GATHER = false>
+template <int FJ, bool GATHER = false>
 __global__ void __launch_bounds__(256) small_nt_kernel(SmallNtArgs g) {
     constexpr int NT = (FJ + 7) / 8;
-    constexpr int RG = TR / 32, KS = 4 / RG;
+    constexpr int TR = 128;
     constexpr int WTILE = (32 + NT * 32) * SN_P;   // bf16 elements per wave: In tile + F tile
     extern __shared__ __attribute__((aligned(16))) bf16_t sn_lds[];
     __shared__ int sh_info[3];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int rg = wave % RG, ks = wave / RG;
+    const int rg = wave;
 
     int e = 0;
     int64_t row0, row_end;
-    if (g.offsets) {
+    {
         // the expert whose tile range holds this block's tile: one look per thread, all loads in flight together
         // (a binary search by one thread is a chain of dependent memory round trips)
         if (tid == 0) sh_info[0] = -1;
@@ -216,10 +189,6 @@ __global__ void __launch_bounds__(256) small_nt_kernel(SmallNtArgs g) {
         if (e < 0) return;
         row0 = sh_info[1];
         row_end = sh_info[2];
-    } else {
-        row0 = (int64_t)blockIdx.x * TR;
-        row_end = g.n_rows;
-        if (row0 >= row_end) return;
     }
     const bf16_t* F = g.F + (int64_t)e * g.f_stride;
     bf16_t* xs = sn_lds + wave * WTILE;          // [32][SN_P]
@@ -235,8 +204,7 @@ __global__ void __launch_bounds__(256) small_nt_kernel(SmallNtArgs g) {
 #pragma unroll
         for (int q = 0; q < 16; ++q) acc[n][q] = 0.0f;
 
-    const int64_t kspan = g.Kc / KS;  // multiple of 16
-    const int64_t kbeg = ks * kspan, kend = kbeg + kspan;
+    const int64_t kbeg = 0, kend = g.Kc;
     const bf16_t* xp[8];
     int32_t orow[GATHER ? 8 : 1];                // GATHER: the rows of copy_out this lane's pieces belong to
 #pragma unroll
@@ -304,24 +272,6 @@ __global__ void __launch_bounds__(256) small_nt_kernel(SmallNtArgs g) {
         chunk(xr[1], k + 128);
     }
 
-    if (KS > 1) {
-        float* red = (float*)sn_lds;   // [(KS-1)][NT][16][64] floats, over the (now dead) tiles
-        __syncthreads();
-        if (ks > 0) {
-#pragma unroll
-            for (int n = 0; n < NT; ++n)
-#pragma unroll
-                for (int q = 0; q < 16; ++q) red[(((ks - 1) * NT + n) * 16 + q) * 64 + lane] = acc[n][q];
-        }
-        __syncthreads();
-        if (ks > 0) return;
-#pragma unroll
-        for (int s = 1; s < KS; ++s)
-#pragma unroll
-            for (int n = 0; n < NT; ++n)
-#pragma unroll
-                for (int q = 0; q < 16; ++q) acc[n][q] += red[(((s - 1) * NT + n) * 16 + q) * 64 + lane];
-    }
     const int rgrp = (lane >> 5) * 4;
 #pragma unroll
     for (int n = 0; n < NT; ++n) {
@@ -338,30 +288,30 @@ __global__ void __launch_bounds__(256) small_nt_kernel(SmallNtArgs g) {
     }
 }
 
-template <int TR, int FJ, bool GATHER = false>
+template <int FJ, bool GATHER = false>
 static int launch_small_nt_one(const SmallNtArgs& g, unsigned blocks, hipStream_t stream) {
     constexpr int NT = (FJ + 7) / 8;
     constexpr size_t lds = (size_t)4 * (32 + NT * 32) * SN_P * 2;
     static std::atomic<bool> attr_set{false};   // the attribute call is idempotent: a race only repeats it
     if (!attr_set) {
-        hipError_t e = hipFuncSetAttribute((const void*)small_nt_kernel<TR, FJ, GATHER>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        hipError_t e = hipFuncSetAttribute((const void*)small_nt_kernel<FJ, GATHER>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) {
             xq_set_error("small_nt: cannot raise the dynamic LDS limit: %s", hipGetErrorString(e));
             return XQ_ERR_LAUNCH;
         }
         attr_set = true;
     }
-    small_nt_kernel<TR, FJ, GATHER><<<dim3(blocks), 256, lds, stream>>>(g);
+    small_nt_kernel<FJ, GATHER><<<dim3(blocks), 256, lds, stream>>>(g);
     return XQ_OK;
 }
 
-template <int TR, bool GATHER = false>
+template <bool GATHER>
 static int launch_small_nt_rows(const SmallNtArgs& g, unsigned blocks, hipStream_t stream) {
     switch (g.r_pad) {
-        case 16: return launch_small_nt_one<TR, 4, GATHER>(g, blocks, stream);
-        case 32: return launch_small_nt_one<TR, 8, GATHER>(g, blocks, stream);
-        case 48: return launch_small_nt_one<TR, 12, GATHER>(g, blocks, stream);
-        default: return launch_small_nt_one<TR, 16, GATHER>(g, blocks, stream);
+        case 16: return launch_small_nt_one<4, GATHER>(g, blocks, stream);
+        case 32: return launch_small_nt_one<8, GATHER>(g, blocks, stream);
+        case 48: return launch_small_nt_one<12, GATHER>(g, blocks, stream);
+        default: return launch_small_nt_one<16, GATHER>(g, blocks, stream);
     }
 }
 
@@ -376,30 +326,351 @@ int launch_small_nt(const bf16_t* In, int64_t ld_in, int64_t n_rows, int64_t Kc,
     XQ_REQUIRE(Kc % 64 == 0, "small_nt: contraction length %lld must be a multiple of 64", (long long)Kc);
     XQ_REQUIRE(ld_in % 8 == 0 && xq_aligned(In, 16) && xq_aligned(F, 16), "small_nt: operands must be 16-byte aligned");
     if (n_rows == 0) return XQ_OK;
-    XQ_REQUIRE(!row_map || (offsets && (!copy_out || (ld_copy % 8 == 0 && ld_copy >= Kc && xq_aligned(copy_out, 16)))),
-               "small_nt: gathered rows need the grouped form, and a copy of them a 16-byte aligned copy_out");
+    XQ_REQUIRE(offsets && tile_offsets && num_experts >= 1, "small_nt: rows in expert order");
+    XQ_REQUIRE(!row_map || !copy_out || (ld_copy % 8 == 0 && ld_copy >= Kc && xq_aligned(copy_out, 16)),
+               "small_nt: a copy of gathered rows needs a 16-byte aligned copy_out");
     SmallNtArgs g{In, ld_in, n_rows, Kc, F, shared_f ? 0 : (int64_t)r_pad * Kc, r_pad, scale, T, ld_t, T2, split, offsets,
                   tile_offsets, num_experts, row_map, copy_out, ld_copy};
-    int rc;
-    if (offsets && row_map) {
-        rc = launch_small_nt_rows<128, true>(g, (unsigned)(xq_cdiv(n_rows, 128) + num_experts), stream);
-    } else if (offsets) {
-        rc = launch_small_nt_rows<128>(g, (unsigned)(xq_cdiv(n_rows, 128) + num_experts), stream);
-    } else {
-        g.f_stride = 0;
-        rc = launch_small_nt_rows<32>(g, (unsigned)xq_cdiv(n_rows, 32), stream);
-    }
+    const unsigned blocks = (unsigned)(xq_cdiv(n_rows, 128) + num_experts);
+    const int rc = row_map ? launch_small_nt_rows<true>(g, blocks, stream) : launch_small_nt_rows<false>(g, blocks, stream);
     if (rc) return rc;
     XQ_CHECK_LAUNCH("small_nt");
     return XQ_OK;
 }
 
+// ------------------------------------------------------------------ dense low-rank products from the factors as they are
+// 8 consecutive contraction elements of one rank of a factor, in the four forms a factor comes in; an fp32 factor is
+// rounded to bf16 on its way to the MFMA.  Loads are unconditional (the caller clamps rank and position).
+typedef u32x4 __attribute__((aligned(2))) u32x4_a2;
+typedef u32x4 __attribute__((aligned(4))) u32x4_a4;
+typedef f32x4 __attribute__((aligned(4))) f32x4_a4;
+template <int MODE>
+struct FactorPiece;
+template <>
+struct FactorPiece<kFacBf16> {
+    u32x4 v;
+    __device__ __forceinline__ void load(const void* F, int, int64_t Kc, int rank, int64_t k) {
+        v = *(const u32x4_a2*)((const bf16_t*)F + (int64_t)rank * Kc + k);
+    }
+    __device__ __forceinline__ u32x4 get() const { return v; }
+};
+template <>
+struct FactorPiece<kFacF32> {
+    f32x4 a, b;
+    __device__ __forceinline__ void load(const void* F, int, int64_t Kc, int rank, int64_t k) {
+        const float* p = (const float*)F + (int64_t)rank * Kc + k;
+        a = *(const f32x4_a4*)p;
+        b = *(const f32x4_a4*)(p + 4);
+    }
+    __device__ __forceinline__ u32x4 get() const {
+        return u32x4{pack_bf16x2(a[0], a[1]), pack_bf16x2(a[2], a[3]), pack_bf16x2(b[0], b[1]), pack_bf16x2(b[2], b[3])};
+    }
+};
+template <>
+struct FactorPiece<kFacF32T> {
+    float v[8];
+    __device__ __forceinline__ void load(const void* F, int r, int64_t, int rank, int64_t k) {
+        const float* p = (const float*)F + k * r + rank;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = p[(int64_t)e * r];
+    }
+    __device__ __forceinline__ u32x4 get() const {
+        return u32x4{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7])};
+    }
+};
+template <>
+struct FactorPiece<kFacBf16T> {
+    uint32_t v[8];
+    __device__ __forceinline__ void load(const void* F, int r, int64_t, int rank, int64_t k) {
+        const bf16_t* p = (const bf16_t*)F + k * r + rank;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = p[(int64_t)e * r];
+    }
+    __device__ __forceinline__ u32x4 get() const {
+        return u32x4{v[0] | (v[1] << 16), v[2] | (v[3] << 16), v[4] | (v[5] << 16), v[6] | (v[7] << 16)};
+    }
+};
+
+struct LowRankBatch {
+    LowRankJob job[kLowRankJobs];
+    int32_t first[kLowRankJobs];      // first block of a job
+    int32_t n;
+    int64_t n_rows;
+};
+
+// T[rows, nf * rp] = bf16(scale * In . F^T), up to kLowRankJobs products in one launch.  A block owns 16 RT rows; its NW waves
+// take 64 contraction elements each in turn and their sums meet in LDS in wave order.  Activations and [r, K] factors are
+// fetched in whole 128-byte lines and reach the MFMA operand layout through wave-private LDS rows: taken from memory in that
+// layout, 16 rows a power of two apart land in one set of the L1 and the two loads that share a line fetch it twice (512 rows,
+// K 4096, r 16: 16 us against 8).  A [K, r] factor is contiguous and is read element by element.  The next unit's loads are in
+// flight while one is multiplied.  Few rows leave most of the chip idle whatever a block does, so it is made short instead:
+// sixteen waves (eight for wide factors) pull a block's rows at the rate of one compute unit.  NT: column tiles of 16 ranks.
+constexpr int LR_P = 72;              // LDS row pitch in bf16 elements: the 16 rows of a 16-byte fragment read fall on 16 bank quads
+template <int MODE, int NT, int RT, int NW>
+struct LowRankLds {
+    static constexpr bool STAGE_F = MODE == kFacF32 || MODE == kFacBf16;
+    static constexpr int WAVE = (RT + (STAGE_F ? NT : 0)) * 16 * LR_P;                      // bf16 elements per wave
+    static constexpr size_t tiles = (size_t)NW * WAVE * 2, sums = (size_t)NW * RT * NT * 64 * 16;
+    static constexpr size_t bytes = tiles > sums ? tiles : sums;
+};
+template <int MODE, int NT, int RT, int NW>
+__global__ void __launch_bounds__(64 * NW, NW / 4) lowrank_kernel(LowRankBatch b) {
+    using L = LowRankLds<MODE, NT, RT, NW>;
+    extern __shared__ __attribute__((aligned(16))) unsigned char lr_lds[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l16 = lane & 15, lg = lane >> 4;
+    int ji = 0;
+#pragma unroll
+    for (int i = 1; i < kLowRankJobs; ++i)
+        if (i < b.n && (int)blockIdx.x >= b.first[i]) ji = i;
+    const LowRankJob& g = b.job[ji];
+    const int64_t row0 = (int64_t)((int)blockIdx.x - b.first[ji]) * (16 * RT);
+    const int rp = g.rp, cols = g.nf * rp;
+    bf16_t* xs = (bf16_t*)lr_lds + wave * L::WAVE;      // [16 RT][LR_P]
+    bf16_t* fs = xs + RT * 16 * LR_P;                   // [16 NT][LR_P]
+    // activations: 8 rows of 128 bytes per load instruction
+    const bf16_t* xp[2 * RT];
+#pragma unroll
+    for (int i = 0; i < 2 * RT; ++i) {
+        const int64_t r = row0 + i * 8 + (lane >> 3);
+        xp[i] = g.In + (r < b.n_rows ? r : b.n_rows - 1) * g.ld_in + (lane & 7) * 8;
+    }
+    // staged factor: fp32, 4 ranks of 256 bytes per instruction; bf16, 8 ranks of 128 bytes
+    constexpr int FI = MODE == kFacF32 ? 4 : 2;         // instructions per 16 ranks
+    struct Unit {
+        u32x4 x[2 * RT];
+        u32x4 fv[L::STAGE_F ? NT * FI : 1];
+        FactorPiece<L::STAGE_F ? kFacBf16 : MODE> fd[L::STAGE_F ? 1 : NT][2];
+    };
+    const void* fp[NT];
+    int j0[NT];                                         // first rank of the tile within its factor
+    bool in_job[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        const int f = t * 16 >= rp && g.nf > 1 ? 1 : 0;
+        fp[t] = f ? g.F[1] : g.F[0];
+        j0[t] = t * 16 - f * rp;
+        in_job[t] = t * 16 < cols;
+    }
+    const int r1 = g.r - 1;
+    // (a staged factor's lane offsets, in bytes from the factor: 32 bits, beside a base every lane shares)
+    uint32_t fo[L::STAGE_F ? NT * FI : 1];
+    if constexpr (L::STAGE_F) {
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int i = 0; i < FI; ++i) {
+                const int j = min(j0[t] + i * (16 / FI) + (MODE == kFacF32 ? lane >> 4 : lane >> 3), r1);
+                fo[t * FI + i] = MODE == kFacF32 ? ((uint32_t)j * (uint32_t)g.Kc + (lane & 15) * 4) * 4 : ((uint32_t)j * (uint32_t)g.Kc + (lane & 7) * 8) * 2;
+            }
+    }
+    f32x4 acc[RT][NT];
+#pragma unroll
+    for (int i = 0; i < RT; ++i)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[i][t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    auto load = [&](Unit& u, int unit) {
+        const int64_t k = (int64_t)unit * 64;
+#pragma unroll
+        for (int i = 0; i < 2 * RT; ++i) u.x[i] = *(const u32x4*)(xp[i] + k);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            if constexpr (L::STAGE_F) {
+#pragma unroll
+                for (int i = 0; i < FI; ++i) {
+                    const unsigned char* base = (const unsigned char*)fp[t] + k * (MODE == kFacF32 ? 4 : 2);
+                    if constexpr (MODE == kFacF32) u.fv[t * FI + i] = *(const u32x4_a4*)(base + fo[t * FI + i]);
+                    else u.fv[t * FI + i] = *(const u32x4_a2*)(base + fo[t * FI + i]);
+                }
+            } else {
+#pragma unroll
+                for (int h = 0; h < 2; ++h) u.fd[t][h].load(fp[t], g.r, g.Kc, min(j0[t] + l16, r1), k + h * 32 + lg * 8);
+            }
+        }
+    };
+    auto multiply = [&](const Unit& u) {
+        // (LDS operations of one wave execute in order: the previous unit's fragment reads are ahead of these writes)
+#pragma unroll
+        for (int i = 0; i < 2 * RT; ++i) *(u32x4*)(xs + (i * 8 + (lane >> 3)) * LR_P + (lane & 7) * 8) = u.x[i];
+        if constexpr (L::STAGE_F) {
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int i = 0; i < FI; ++i) {
+                    const int jr = i * (16 / FI) + (MODE == kFacF32 ? lane >> 4 : lane >> 3);
+                    const uint32_t keep = in_job[t] && j0[t] + jr < g.r ? 0xffffffffu : 0u;      // ranks beyond r are zero
+                    const u32x4 v = u.fv[t * FI + i];
+                    bf16_t* d = fs + (t * 16 + jr) * LR_P;
+                    if constexpr (MODE == kFacF32)
+                        *(u32x2*)(d + (lane & 15) * 4) = u32x2{pack_bf16x2(__uint_as_float(v[0]), __uint_as_float(v[1])) & keep,
+                                                               pack_bf16x2(__uint_as_float(v[2]), __uint_as_float(v[3])) & keep};
+                    else
+                        *(u32x4*)(d + (lane & 7) * 8) = u32x4{v[0] & keep, v[1] & keep, v[2] & keep, v[3] & keep};
+                }
+        }
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            bf16x8 x[RT];
+#pragma unroll
+            for (int i = 0; i < RT; ++i) x[i] = *(const bf16x8*)(xs + (i * 16 + l16) * LR_P + h * 32 + lg * 8);
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                bf16x8 w;
+                if constexpr (L::STAGE_F) {
+                    w = *(const bf16x8*)(fs + (t * 16 + l16) * LR_P + h * 32 + lg * 8);
+                } else {
+                    const uint32_t keep = in_job[t] && j0[t] + l16 < g.r ? 0xffffffffu : 0u;
+                    const u32x4 v = u.fd[t][h].get();
+                    w = __builtin_bit_cast(bf16x8, u32x4{v[0] & keep, v[1] & keep, v[2] & keep, v[3] & keep});
+                }
+#pragma unroll
+                for (int i = 0; i < RT; ++i) acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, x[i], acc[i][t], 0, 0, 0);
+            }
+        }
+    };
+    const int units = (int)(g.Kc >> 6), last = units - 1;
+    if (wave < units) {
+        Unit a, c;
+        load(a, wave);
+#pragma unroll 1
+        for (int u = wave;;) {
+            int nx = u + NW;
+            load(c, nx < last ? nx : last);            // (past the end: fetched again, never used)
+            multiply(a);
+            if (nx >= units) break;
+            u = nx;
+            nx = u + NW;
+            load(a, nx < last ? nx : last);
+            multiply(c);
+            if (nx >= units) break;
+            u = nx;
+        }
+    }
+    f32x4* red = (f32x4*)lr_lds;                        // [NW][RT * NT][64], over the (now dead) tiles
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < RT; ++i)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) red[(wave * (RT * NT) + i * NT + t) * 64 + lane] = acc[i][t];
+    __syncthreads();
+    for (int idx = tid; idx < RT * NT * 64; idx += 64 * NW) {
+        f32x4 v = red[idx];
+#pragma unroll
+        for (int w = 1; w < NW; ++w) v += red[w * (RT * NT * 64) + idx];
+        const int l = idx & 63, t = (idx >> 6) % NT, i = (idx >> 6) / NT;
+        const int64_t m = row0 + i * 16 + (l & 15);
+        if (t * 16 >= cols || m >= b.n_rows) continue;
+        const int f = t * 16 >= rp ? 1 : 0;
+        *(u32x2*)(g.T + f * g.t_step + m * g.ld_t + t * 16 - f * rp + 4 * (l >> 4)) =
+            u32x2{pack_bf16x2(v[0] * g.scale, v[1] * g.scale), pack_bf16x2(v[2] * g.scale, v[3] * g.scale)};
+    }
+}
+
+template <int MODE, int NT, int RT, int NW>
+static int launch_lowrank_one(const LowRankBatch& b, unsigned blocks, hipStream_t stream) {
+    constexpr size_t lds = LowRankLds<MODE, NT, RT, NW>::bytes;
+    static std::atomic<bool> attr_set{false};   // the attribute call is idempotent: a race only repeats it
+    if (!attr_set) {
+        hipError_t e = hipFuncSetAttribute((const void*)lowrank_kernel<MODE, NT, RT, NW>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) {
+            xq_set_error("lowrank: cannot raise the dynamic LDS limit: %s", hipGetErrorString(e));
+            return XQ_ERR_LAUNCH;
+        }
+        attr_set = true;
+    }
+    lowrank_kernel<MODE, NT, RT, NW><<<dim3(blocks), 64 * NW, lds, stream>>>(b);
+    return XQ_OK;
+}
+template <int MODE, int RT, int NW>
+static int launch_lowrank_nt(const LowRankBatch& b, int nt, unsigned blocks, hipStream_t stream) {
+    switch (nt) {
+        case 1: return launch_lowrank_one<MODE, 1, RT, NW>(b, blocks, stream);
+        case 2: return launch_lowrank_one<MODE, 2, RT, NW>(b, blocks, stream);
+        case 3: return launch_lowrank_one<MODE, 3, RT, 8>(b, blocks, stream);      // (two units of three factor tiles take more than 128 registers)
+        default: return launch_lowrank_one<MODE, 4, RT, 8>(b, blocks, stream);
+    }
+}
+
+// 16 rows and sixteen waves to a block until every compute unit has one, then 32 rows and eight waves
+static bool lowrank_tall(int n, int64_t n_rows) { return n_rows * n > 16ll * num_cus(); }
+
+int64_t lowrank_panel_bytes(int n, int64_t n_rows, int cols, int64_t Kc) {
+    return lowrank_tall(n, n_rows) ? (((int64_t)cols * Kc * 2 + 255) & ~(int64_t)255) * n : 0;
+}
+
+int launch_lowrank(const LowRankJob* jobs, int n, int64_t n_rows, FactorMode mode, bf16_t* panels, hipStream_t stream) {
+    XQ_REQUIRE(n >= 1 && n <= kLowRankJobs, "lowrank: %d products", n);
+    if (n_rows == 0) return XQ_OK;
+    LowRankBatch b{};
+    const bool tall = lowrank_tall(n, n_rows);
+    // every block reads the whole factor: where there are many, fp32 [r, K] factors are laid out as bf16 panels first (8192 rows,
+    // K 4096, two factors of rank 32: 70 us against 40 and 6)
+    LowRankJob own[kLowRankJobs];
+    if (tall && mode == kFacF32 && panels) {
+        PanelJobs pj{};
+        pj.in_f32 = 1;
+        for (int i = 0; i < n; ++i) {
+            own[i] = jobs[i];
+            for (int f = 0; f < jobs[i].nf; ++f)
+                own[i].F[f] = pj.add(jobs[i].F[f], 1, jobs[i].r, jobs[i].Kc, false, panels + (int64_t)f * jobs[i].rp * jobs[i].Kc, 1, jobs[i].rp, jobs[i].Kc);
+            own[i].r = jobs[i].rp;
+            panels += (((int64_t)jobs[i].nf * jobs[i].rp * jobs[i].Kc * 2 + 255) & ~(int64_t)255) / 2;
+        }
+        const int rc = launch_panel_prep(pj, stream);
+        if (rc) return rc;
+        jobs = own;
+        mode = kFacBf16;
+    }
+    const int64_t per = tall ? 32 : 16, blocks = xq_cdiv(n_rows, per);
+    int nt = 1;
+    for (int i = 0; i < n; ++i) {
+        const LowRankJob& j = jobs[i];
+        XQ_REQUIRE(j.rp > 0 && j.rp % 16 == 0 && j.r >= 1 && j.r <= j.rp && j.nf >= 1 && j.nf <= 2 && j.nf * j.rp <= 64, "lowrank: bad rank (r %d, r_pad %d)", j.r, j.rp);
+        XQ_REQUIRE(j.Kc < (1ll << 24), "lowrank: contraction length %lld", (long long)j.Kc);
+        XQ_REQUIRE(j.Kc % 64 == 0, "lowrank: contraction length %lld must be a multiple of 64", (long long)j.Kc);
+        XQ_REQUIRE(j.ld_in % 8 == 0 && xq_aligned(j.In, 16), "lowrank: activation rows must be 16-byte aligned");
+        XQ_REQUIRE(j.ld_t % 4 == 0 && j.t_step % 4 == 0 && xq_aligned(j.T, 8), "lowrank: result rows must be 8-byte aligned");
+        b.job[i] = j;
+        b.first[i] = (int32_t)(blocks * i);
+        nt = j.nf * j.rp / 16 > nt ? j.nf * j.rp / 16 : nt;
+    }
+    b.n = n; b.n_rows = n_rows;
+    const unsigned grid = (unsigned)(blocks * n);
+    int rc;
+#define XQ_LR(MODE) rc = tall ? launch_lowrank_nt<MODE, 2, 8>(b, nt, grid, stream) : launch_lowrank_nt<MODE, 1, 16>(b, nt, grid, stream)
+    switch (mode) {
+        case kFacBf16: XQ_LR(kFacBf16); break;
+        case kFacF32: XQ_LR(kFacF32); break;
+        case kFacF32T: XQ_LR(kFacF32T); break;
+        default: XQ_LR(kFacBf16T); break;
+    }
+#undef XQ_LR
+    if (rc) return rc;
+    XQ_CHECK_LAUNCH("lowrank");
+    return XQ_OK;
+}
+
+// T[m][j] = bf16(scale * (partial[0][m][j] + partial[1][m][j] + ...)), the splits in index order; columns from rp on are the
+// second product's
+__global__ void __launch_bounds__(256) lowrank_reduce_kernel(const float* partial, int splits, int64_t n_rows, int rp, int nprod, float scale,
+                                                             bf16_t* T, bf16_t* T2, int64_t ld_t) {
+    const int cols = nprod * rp;
+    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x, total = n_rows * cols;
+    if (t >= total) return;
+    float v = partial[t];
+    for (int s = 1; s < splits; ++s) v += partial[(int64_t)s * total + t];
+    const int64_t m = t / cols;
+    const int j = (int)(t - m * cols);
+    (j < rp ? T : T2)[m * ld_t + (j < rp ? j : j - rp)] = to_bf16(v * scale);
+}
+
 // ------------------------------------------------------------------ SwiGLU backward + its two low-rank products
 // One pass over (gate, up, dh): writes dgate | dup (the elementwise kernel's arithmetic, ops/moe/lora.py:855-917 with no
 // routing weight) and forms Tg = s * dgate . Fg^T and Tu = s * dup . Fu^T from the values on their way out -- the two
-// products no longer read dgate | dup back.  Dense rows; organisation and summation order of small_nt_kernel<32, FJ>
-// (32 rows per block, the four waves split the columns, 128 columns at a time through wave-private LDS tiles), so Tg
-// and Tu are the bits the two small_nt launches produce.
+// products do not read dgate | dup back.  Dense rows: 32 per block, the four waves (and blockIdx.y) split the columns, 64 at a
+// time through wave-private LDS tiles.  A block of 32 rows runs ~140 us at 12288 columns however many there are, so a launch
+// of fewer than a block per compute unit deals the columns over blockIdx.y too and leaves fp32 sums to
+// lowrank_reduce_kernel (200 rows of 12288 columns: 141 us in 7 blocks, 18 us in 168 and the reduction).
 struct SiluNtArgs {
     const bf16_t* gate;
     const bf16_t* up;
@@ -410,9 +681,9 @@ struct SiluNtArgs {
     bf16_t* dup;
     int64_t ld_out;
     int64_t n_rows, Kc;        // rows; columns of gate / up / dh (the contraction length of the two products)
-    const bf16_t* Fg;          // [r_pad][Kc]
-    const bf16_t* Fu;
-    int r_pad;
+    const void* Fg;            // factors in the kernel's MODE (routed rows: bf16 panels [r_pad][Kc] per expert)
+    const void* Fu;
+    int r, r_pad;
     float scale;
     bf16_t* Tg;                // [n_rows][ld_t]
     bf16_t* Tu;
@@ -426,6 +697,7 @@ struct SiluNtArgs {
     const float* row_w;
     float* d_row_w;
     float limit;               // SwiGLU limit on the gate pre-activation (<= 0: none)
+    float* partial;            // dense with gridDim.y > 1: fp32 sums [gridDim.y][n_rows][products * r_pad]
 };
 
 // GROUPED: routed rows in expert order, organisation of small_nt_kernel<128, FJ> (a block = a 128-row tile of one expert, a
@@ -434,7 +706,7 @@ struct SiluNtArgs {
 // FWD: the forward pass in the same organisation -- h = bf16(bf16(silu(gate)) * up) (routed: then rounded and times the row's
 // weight), the elementwise forward kernel's arithmetic, written through `dgate`, and Tg = scale * h . Fg^T from the values
 // on their way out (dh, dup, Fu, Tu, d_row_w unused).
-template <int FJ, bool GROUPED, bool FWD = false>
+template <int FJ, bool GROUPED, bool FWD, int MODE>
 __global__ void __launch_bounds__(256, 2) silu_bwd_nt_kernel(SiluNtArgs g) {
     static_assert(FJ <= 8, "one MFMA column tile per product");
     // 64 columns at a time (where small_nt_kernel takes 128: the same MFMA steps in the same order): three operands' pieces
@@ -474,15 +746,16 @@ __global__ void __launch_bounds__(256, 2) silu_bwd_nt_kernel(SiluNtArgs g) {
         row_end = g.n_rows;
         if (row0 >= row_end) return;
     }
-    const bf16_t* Fg = g.Fg + (int64_t)e * g.fg_stride;
-    const bf16_t* Fu = g.Fu + (int64_t)e * g.fu_stride;
+    const void* Fg = GROUPED ? (const void*)((const bf16_t*)g.Fg + (int64_t)e * g.fg_stride) : g.Fg;
+    const void* Fu = GROUPED ? (const void*)((const bf16_t*)g.Fu + (int64_t)e * g.fu_stride) : g.Fu;
     bf16_t* xs = sn_lds + wave * WTILE;          // [32][P]
     bf16_t* fs = xs + 32 * P;                    // [32][P]
     const int fr = lane & 31, fk = (lane >> 5) * 8;
     const int crow = lane / (CW / 8), cpiece = (lane % (CW / 8)) * 8;
     const int frows = g.r_pad;
-    const int64_t kspan = GROUPED ? g.Kc : g.Kc / 4;        // multiple of 16
-    const int64_t kbeg = GROUPED ? 0 : wave * kspan, kend = kbeg + kspan;
+    // (dense: the 64-column units dealt evenly over the waves of the block column)
+    const int64_t units = g.Kc / CW, parts = 4 * gridDim.y, part = 4 * blockIdx.y + wave;
+    const int64_t kbeg = GROUPED ? 0 : units * part / parts * CW, kend = GROUPED ? g.Kc : units * (part + 1) / parts * CW;
     const int64_t rbase = row0 + crow;           // this lane's rows: rbase + RPI j, clamped onto the last row
     auto row_of = [&](int j) { const int64_t r = rbase + j * RPI; return r < row_end ? r : row_end - 1; };
     float rw[GROUPED ? NL : 1], wsum[GROUPED ? NL : 1];
@@ -493,7 +766,8 @@ __global__ void __launch_bounds__(256, 2) silu_bwd_nt_kernel(SiluNtArgs g) {
             wsum[j] = 0.0f;
         }
     }
-    u32x4 gq[NL], uq[NL], dq[NL], fq[FL];
+    u32x4 gq[NL], uq[NL], dq[NL];
+    FactorPiece<MODE> fq[FL];
     // every load is unconditional: rows past the end and pieces past the wave's columns are clamped onto valid ones
     auto fetch = [&](int64_t k) {
         int64_t kc = k + cpiece;
@@ -506,16 +780,17 @@ __global__ void __launch_bounds__(256, 2) silu_bwd_nt_kernel(SiluNtArgs g) {
             if constexpr (!FWD) dq[j] = *(const u32x4*)(g.dh + r * g.ld_dh + kc);
         }
     };
-    auto fetch_f = [&](const bf16_t* F, int64_t k) {
+    auto fetch_f = [&](const void* F, int64_t k) {
         int64_t kc = k + cpiece;
         kc = kc < kend ? kc : kend - 8;
 #pragma unroll
-        for (int j = 0; j < FL; ++j) fq[j] = *(const u32x4*)(F + (int64_t)(j * RPI + crow < FJ * 4 ? j * RPI + crow : FJ * 4 - 1) * g.Kc + kc);
+        for (int j = 0; j < FL; ++j) fq[j].load(F, g.r, g.Kc, j * RPI + crow < g.r ? j * RPI + crow : g.r - 1, kc);
     };
-    auto stage_f = [&]() {
+    auto stage_f = [&]() {                       // ranks from r to the padded count are zero
+        const u32x4 z = {0, 0, 0, 0};
 #pragma unroll
         for (int j = 0; j < FL; ++j)
-            if (j * RPI + crow < 32) *(u32x4*)(fs + (j * RPI + crow) * P + cpiece) = fq[j];
+            if (j * RPI + crow < 32) *(u32x4*)(fs + (j * RPI + crow) * P + cpiece) = j * RPI + crow < g.r ? fq[j].get() : z;
     };
     f32x16 acc_g, acc_u;
 #pragma unroll
@@ -534,9 +809,11 @@ __global__ void __launch_bounds__(256, 2) silu_bwd_nt_kernel(SiluNtArgs g) {
     // The factor chunks (from L2) are requested ahead of the value chunks and go to the LDS tile as soon as the MFMAs that
     // read its previous contents are issued (LDS operations of one wave execute in order), so their registers are free
     // while a chunk's values are worked out.
-    fetch_f(Fg, kbeg);
-    fetch(kbeg);
-    stage_f();
+    if (kbeg < kend) {                           // (fewer units than waves: nothing to fetch)
+        fetch_f(Fg, kbeg);
+        fetch(kbeg);
+        stage_f();
+    }
     if constexpr (FWD) {
         for (int64_t k = kbeg; k < kend; k += CW) {
             const int64_t kc = k + cpiece;
@@ -655,6 +932,21 @@ __global__ void __launch_bounds__(256, 2) silu_bwd_nt_kernel(SiluNtArgs g) {
             acc_g[q] += red[(((s - 1) * 2 + 0) * 16 + q) * 64 + lane];
             acc_u[q] += red[(((s - 1) * 2 + 1) * 16 + q) * 64 + lane];
         }
+    if (gridDim.y > 1) {
+        constexpr int NP = 2;
+        float* part_out = g.partial + (int64_t)blockIdx.y * g.n_rows * (NP * g.r_pad);
+        if (fr < g.r_pad) {
+#pragma unroll
+            for (int q = 0; q < 16; ++q) {
+                const int64_t row = row0 + (q & 3) + rgrp + 8 * (q >> 2);
+                if (row < row_end) {
+                    part_out[row * (NP * g.r_pad) + fr] = acc_g[q];
+                    part_out[row * (NP * g.r_pad) + g.r_pad + fr] = acc_u[q];
+                }
+            }
+        }
+        return;
+    }
     if (fr < g.r_pad) {
 #pragma unroll
         for (int q = 0; q < 16; ++q) {
@@ -667,46 +959,72 @@ __global__ void __launch_bounds__(256, 2) silu_bwd_nt_kernel(SiluNtArgs g) {
     }
 }
 
-template <int FJ, bool GROUPED, bool FWD = false>
-static int launch_silu_bwd_nt_one(const SiluNtArgs& g, unsigned blocks, hipStream_t stream) {
+template <int FJ, bool GROUPED, bool FWD, int MODE>
+static int launch_silu_nt_one(const SiluNtArgs& g, dim3 blocks, hipStream_t stream) {
     constexpr size_t lds = (size_t)4 * (32 + 32) * (64 + 8) * 2;
     static std::atomic<bool> attr_set{false};   // the attribute call is idempotent: a race only repeats it
     if (!attr_set) {
-        hipError_t e = hipFuncSetAttribute((const void*)silu_bwd_nt_kernel<FJ, GROUPED, FWD>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        hipError_t e = hipFuncSetAttribute((const void*)silu_bwd_nt_kernel<FJ, GROUPED, FWD, MODE>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) {
             xq_set_error("silu_bwd_nt: cannot raise the dynamic LDS limit: %s", hipGetErrorString(e));
             return XQ_ERR_LAUNCH;
         }
         attr_set = true;
     }
-    silu_bwd_nt_kernel<FJ, GROUPED, FWD><<<dim3(blocks), 256, lds, stream>>>(g);
+    silu_bwd_nt_kernel<FJ, GROUPED, FWD, MODE><<<blocks, 256, lds, stream>>>(g);
     XQ_CHECK_LAUNCH("silu_bwd_nt");
     return XQ_OK;
 }
 
 bool silu_bwd_nt_supported(int64_t cols, int r_pad) { return (r_pad == 16 || r_pad == 32) && cols % 64 == 0 && cols >= 512; }
 
+// column splits of the dense form: none from a block per compute unit on, else about three blocks per unit, 512 columns at least
+static int silu_nt_splits(int64_t n_rows, int64_t cols) {
+    const int64_t blocks = xq_cdiv(n_rows, 32);
+    if (blocks >= num_cus()) return 1;
+    int64_t s = xq_cdiv(3ll * num_cus(), blocks);
+    if (s > cols / 512) s = cols / 512;
+    return s < 2 ? 1 : (int)s;
+}
+
+int64_t silu_nt_partial_bytes(int64_t n_rows, int64_t cols, int r_pad) {
+    const int s = n_rows > 0 ? silu_nt_splits(n_rows, cols) : 1;
+    return s > 1 ? (int64_t)s * n_rows * 2 * r_pad * 4 : 0;
+}
+
 int launch_silu_bwd_nt(const bf16_t* gate, const bf16_t* up, int64_t ld_gu, const bf16_t* dh, int64_t ld_dh, bf16_t* dgate,
-                       bf16_t* dup, int64_t ld_out, int64_t n_rows, int64_t cols, const bf16_t* Fg, const bf16_t* Fu, int r_pad,
-                       float scale, bf16_t* Tg, bf16_t* Tu, int64_t ld_t, hipStream_t stream, const int32_t* offsets,
+                       bf16_t* dup, int64_t ld_out, int64_t n_rows, int64_t cols, const void* Fg, const void* Fu, FactorMode mode, int r, int r_pad,
+                       float scale, bf16_t* Tg, bf16_t* Tu, int64_t ld_t, float* partial, hipStream_t stream, const int32_t* offsets,
                        const int32_t* tile_offsets, int32_t num_experts, bool shared_fg, bool shared_fu, const float* row_w,
                        float* d_row_w, float swiglu_limit) {
     XQ_REQUIRE(silu_bwd_nt_supported(cols, r_pad), "silu_bwd_nt: %lld columns with r_pad %d are not handled here", (long long)cols, r_pad);
     XQ_REQUIRE(ld_gu % 8 == 0 && ld_dh % 8 == 0 && ld_out % 8 == 0 && ld_t >= r_pad, "silu_bwd_nt: row pitches must be multiples of 8");
-    XQ_REQUIRE(xq_aligned(gate, 16) && xq_aligned(up, 16) && xq_aligned(dh, 16) && xq_aligned(dgate, 16) && xq_aligned(dup, 16) &&
-                   xq_aligned(Fg, 16) && xq_aligned(Fu, 16),
+    XQ_REQUIRE(xq_aligned(gate, 16) && xq_aligned(up, 16) && xq_aligned(dh, 16) && xq_aligned(dgate, 16) && xq_aligned(dup, 16),
                "silu_bwd_nt: operands must be 16-byte aligned");
     XQ_REQUIRE(!offsets || (tile_offsets && row_w && num_experts >= 1), "silu_bwd_nt: the routed form needs tile offsets and row weights");
     if (n_rows == 0) return XQ_OK;
-    SiluNtArgs g{gate, up, ld_gu, dh, ld_dh, dgate, dup, ld_out, n_rows, cols, Fg, Fu, r_pad, scale, Tg, Tu, ld_t,
+    SiluNtArgs g{gate, up, ld_gu, dh, ld_dh, dgate, dup, ld_out, n_rows, cols, Fg, Fu, r, r_pad, scale, Tg, Tu, ld_t,
                  offsets, tile_offsets, num_experts, offsets && !shared_fg ? (int64_t)r_pad * cols : 0,
-                 offsets && !shared_fu ? (int64_t)r_pad * cols : 0, row_w, d_row_w, swiglu_limit};
+                 offsets && !shared_fu ? (int64_t)r_pad * cols : 0, row_w, d_row_w, swiglu_limit, nullptr};
     if (offsets) {
-        const unsigned blocks = (unsigned)(xq_cdiv(n_rows, 128) + num_experts);
-        return r_pad == 16 ? launch_silu_bwd_nt_one<4, true>(g, blocks, stream) : launch_silu_bwd_nt_one<8, true>(g, blocks, stream);
+        XQ_REQUIRE(mode == kFacBf16, "silu_bwd_nt: the routed form takes bf16 panels");
+        const dim3 blocks((unsigned)(xq_cdiv(n_rows, 128) + num_experts));
+        return r_pad == 16 ? launch_silu_nt_one<4, true, false, kFacBf16>(g, blocks, stream) : launch_silu_nt_one<8, true, false, kFacBf16>(g, blocks, stream);
     }
-    const unsigned blocks = (unsigned)xq_cdiv(n_rows, 32);
-    return r_pad == 16 ? launch_silu_bwd_nt_one<4, false>(g, blocks, stream) : launch_silu_bwd_nt_one<8, false>(g, blocks, stream);
+    XQ_REQUIRE(mode != kFacF32, "silu_bwd_nt: factor form %d", (int)mode);
+    const int splits = partial ? silu_nt_splits(n_rows, cols) : 1;
+    g.partial = splits > 1 ? partial : nullptr;
+    const dim3 blocks((unsigned)xq_cdiv(n_rows, 32), (unsigned)splits);
+    int rc;
+#define XQ_SILU(MODE) rc = r_pad == 16 ? launch_silu_nt_one<4, false, false, MODE>(g, blocks, stream) : launch_silu_nt_one<8, false, false, MODE>(g, blocks, stream)
+    if (mode == kFacBf16) XQ_SILU(kFacBf16);
+    else if (mode == kFacF32T) XQ_SILU(kFacF32T);
+    else XQ_SILU(kFacBf16T);
+#undef XQ_SILU
+    if (rc || splits == 1) return rc;
+    lowrank_reduce_kernel<<<(unsigned)xq_cdiv(n_rows * 2 * r_pad, 256), 256, 0, stream>>>(partial, splits, n_rows, r_pad, 2, scale, Tg, Tu, ld_t);
+    XQ_CHECK_LAUNCH("silu_bwd_nt(reduce)");
+    return XQ_OK;
 }
 
 int launch_silu_fwd_nt(const bf16_t* gate, const bf16_t* up, int64_t ld_gu, bf16_t* h, int64_t ld_h, int64_t n_rows, int64_t cols,
@@ -717,14 +1035,14 @@ int launch_silu_fwd_nt(const bf16_t* gate, const bf16_t* up, int64_t ld_gu, bf16
     XQ_REQUIRE(xq_aligned(gate, 16) && xq_aligned(up, 16) && xq_aligned(h, 16) && xq_aligned(F, 16), "silu_fwd_nt: operands must be 16-byte aligned");
     XQ_REQUIRE(!offsets || (tile_offsets && row_w && num_experts >= 1), "silu_fwd_nt: the routed form needs tile offsets and row weights");
     if (n_rows == 0) return XQ_OK;
-    SiluNtArgs g{gate, up, ld_gu, nullptr, 0, h, nullptr, ld_h, n_rows, cols, F, F, r_pad, scale, T, nullptr, ld_t,
-                 offsets, tile_offsets, num_experts, offsets && !shared_f ? (int64_t)r_pad * cols : 0, 0, row_w, nullptr, swiglu_limit};
-    if (offsets) {
-        const unsigned blocks = (unsigned)(xq_cdiv(n_rows, 128) + num_experts);
-        return r_pad == 16 ? launch_silu_bwd_nt_one<4, true, true>(g, blocks, stream) : launch_silu_bwd_nt_one<8, true, true>(g, blocks, stream);
+    SiluNtArgs g{gate, up, ld_gu, nullptr, 0, h, nullptr, ld_h, n_rows, cols, F, F, r_pad, r_pad, scale, T, nullptr, ld_t,
+                 offsets, tile_offsets, num_experts, offsets && !shared_f ? (int64_t)r_pad * cols : 0, 0, row_w, nullptr, swiglu_limit, nullptr};
+    if (!offsets) {
+        const dim3 blocks((unsigned)xq_cdiv(n_rows, 32));
+        return r_pad == 16 ? launch_silu_nt_one<4, false, true, kFacBf16>(g, blocks, stream) : launch_silu_nt_one<8, false, true, kFacBf16>(g, blocks, stream);
     }
-    const unsigned blocks = (unsigned)xq_cdiv(n_rows, 32);
-    return r_pad == 16 ? launch_silu_bwd_nt_one<4, false, true>(g, blocks, stream) : launch_silu_bwd_nt_one<8, false, true>(g, blocks, stream);
+    const dim3 blocks((unsigned)(xq_cdiv(n_rows, 128) + num_experts));
+    return r_pad == 16 ? launch_silu_nt_one<4, true, true, kFacBf16>(g, blocks, stream) : launch_silu_nt_one<8, true, true, kFacBf16>(g, blocks, stream);
 }
 
 // ------------------------------------------------------------------ tn (weight-gradient shape)
@@ -742,6 +1060,8 @@ struct TnArgs {
     const int32_t* row_limit;  // dense, optional (device): only rows below *row_limit are contracted
     int64_t ldq;               // row pitch of Q in elements
     const int32_t* p_rows;     // optional: row m of the contraction is row p_rows[m] of P
+    float* out2;               // optional: columns of Q from split_j on belong to a second result, columns split_j .. + r_out
+    int32_t split_j;
 };
 
 constexpr int TN_PP = 128 + 16;  // Ps pitch (bf16 elements): 288 B rows
@@ -815,15 +1135,17 @@ __device__ __forceinline__ void tn_accumulate(const TnArgs& g, int64_t c0, int64
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");   // the buffers are free again when this returns
 }
 
-// out[c][j] (pitch = row length of the destination) or, transposed, out[j][c]; j < r_lim
+// out[c][j] (pitch = row length of the destination) or, transposed, out[j][c]; j < r_lim.  out2 (may be NULL): the columns from
+// split_j on are that matrix's columns 0 ..
 template <int NT>
 __device__ __forceinline__ void tn_write(const f32x16* acc, float* out, int64_t c0, int64_t width, int r_lim, int pitch,
-                                         bool transposed) {
+                                         bool transposed, float* out2 = nullptr, int split_j = 0) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int rgrp = (lane >> 5) * 4;
 #pragma unroll
     for (int n = 0; n < NT; ++n) {
-        const int j = n * 32 + (lane & 31);
+        int j = n * 32 + (lane & 31);
+        if (out2 != nullptr && j >= split_j) { out = out2; j -= split_j; }
         if (j >= r_lim) continue;
 #pragma unroll
         for (int q = 0; q < 16; ++q) {
@@ -835,13 +1157,27 @@ __device__ __forceinline__ void tn_write(const f32x16* acc, float* out, int64_t 
     }
 }
 
-// dense: block (col tile, row split) -> partial[split][width][r_pad]
+// dense, up to kTnJobs products in one launch: block (job, col tile, row split) -> partial[split][width][r_pad], or the result
+// itself where a job's rows are not split
+struct TnBatch {
+    TnArgs job[kTnJobs];
+    float* partial[kTnJobs];
+    int32_t first[kTnJobs + 1];       // first block of a job
+    int32_t splits[kTnJobs];
+    int32_t n;
+};
 template <int NT>
-__global__ void __launch_bounds__(256) tn_kernel(TnArgs g) {
+__global__ void __launch_bounds__(256) tn_kernel(TnBatch b) {
     __shared__ __attribute__((aligned(16))) bf16_t Ps[2 * 32 * TN_PP];
     __shared__ __attribute__((aligned(16))) bf16_t Qs[2 * 32 * TN_QP];
-    const int64_t c0 = (int64_t)blockIdx.x * 128;
-    const int64_t m_begin = (int64_t)blockIdx.y * g.rows_per_split;
+    int ji = 0;
+#pragma unroll
+    for (int i = 1; i < kTnJobs; ++i)
+        if (i < b.n && (int)blockIdx.x >= b.first[i]) ji = i;
+    const TnArgs& g = b.job[ji];
+    const int splits = b.splits[ji], at = (int)blockIdx.x - b.first[ji], ct = at / splits, split = at - ct * splits;
+    const int64_t c0 = (int64_t)ct * 128;
+    const int64_t m_begin = (int64_t)split * g.rows_per_split;
     int64_t m_end = m_begin + g.rows_per_split;
     m_end = m_end < g.n_rows ? m_end : g.n_rows;
     if (g.row_limit) {
@@ -854,7 +1190,25 @@ __global__ void __launch_bounds__(256) tn_kernel(TnArgs g) {
 #pragma unroll
         for (int q = 0; q < 16; ++q) acc[n][q] = 0.0f;
     if (m_begin < m_end) tn_accumulate<NT>(g, c0, m_begin, m_end, Ps, Qs, acc);     // uniform over the block
-    tn_write<NT>(acc, g.out + (int64_t)blockIdx.y * g.width * g.r_pad, c0, g.width, g.r_pad, g.r_pad, false);
+    if (splits == 1) tn_write<NT>(acc, g.out, c0, g.width, g.r_out, g.r_out, g.transpose_out != 0, g.out2, g.split_j);
+    else tn_write<NT>(acc, b.partial[ji] + (int64_t)split * g.width * g.r_pad, c0, g.width, g.r_pad, g.r_pad, false);
+}
+
+// grouped, experts of few rows: block (col tile, expert) -> out[expert], zero for an expert without rows
+template <int NT>
+__global__ void __launch_bounds__(256) tn_expert_kernel(TnArgs g) {
+    __shared__ __attribute__((aligned(16))) bf16_t Ps[2 * 32 * TN_PP];
+    __shared__ __attribute__((aligned(16))) bf16_t Qs[2 * 32 * TN_QP];
+    const int64_t c0 = (int64_t)blockIdx.x * 128;
+    const int e = blockIdx.y;
+    const int64_t m_begin = g.offsets[e], m_end = g.offsets[e + 1];
+    f32x16 acc[NT];
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+        for (int q = 0; q < 16; ++q) acc[n][q] = 0.0f;
+    if (m_begin < m_end) tn_accumulate<NT>(g, c0, m_begin, m_end, Ps, Qs, acc);     // uniform over the block
+    tn_write<NT>(acc, g.out + (int64_t)e * g.width * g.r_out, c0, g.width, g.r_out, g.r_out, g.transpose_out != 0);
 }
 
 // grouped: block (col tile, chunk of TN_CHUNK global rows).  The chunk is walked expert by expert;
@@ -925,69 +1279,135 @@ __global__ void __launch_bounds__(256) tn_grouped_reduce_kernel(const float* par
     else o[c * r_out + j] = s;
 }
 
-// sums the dense partials in split order: out[c][j] or out[j][c], j < r_out
-__global__ void __launch_bounds__(256) tn_reduce_kernel(const float* partial, int splits, int64_t width, int r_pad,
-                                                        int r_out, int transpose_out, float* out) {
-    int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+// sums the dense partials of up to kTnJobs products in split order: out[c][j] or out[j][c], j < r_out
+struct TnReduceBatch {
+    const float* partial[kTnJobs];
+    float* out[kTnJobs];
+    float* out2[kTnJobs];
+    int64_t width[kTnJobs];
+    int32_t splits[kTnJobs], r_pad[kTnJobs], r_out[kTnJobs], transpose_out[kTnJobs], split_j[kTnJobs];
+    int32_t first[kTnJobs];
+    int32_t n;
+};
+__global__ void __launch_bounds__(256) tn_reduce_kernel(TnReduceBatch b) {
+    int ji = 0;
+#pragma unroll
+    for (int i = 1; i < kTnJobs; ++i)
+        if (i < b.n && (int)blockIdx.x >= b.first[i]) ji = i;
+    const int64_t t = (int64_t)((int)blockIdx.x - b.first[ji]) * 256 + threadIdx.x, width = b.width[ji];
+    const int r_pad = b.r_pad[ji], r_out = b.r_out[ji];
     if (t >= width * r_pad) return;
-    int64_t c = t / r_pad;
-    int j = (int)(t - c * r_pad);
-    if (j >= r_out) return;
+    // (consecutive threads write along the destination's rows)
+    int64_t c, j;
+    if (b.transpose_out[ji]) { j = t / width; c = t - j * width; }
+    else { c = t / r_pad; j = t - c * r_pad; }
     float s = 0.0f;
-    for (int i = 0; i < splits; ++i) s += partial[(int64_t)i * width * r_pad + t];
-    if (transpose_out) out[(int64_t)j * width + c] = s;
+    const float* p = b.partial[ji] + c * r_pad + j;
+    for (int i = 0; i < b.splits[ji]; ++i) s += p[(int64_t)i * width * r_pad];
+    float* out = b.out[ji];
+    if (b.out2[ji] != nullptr && j >= b.split_j[ji]) { out = b.out2[ji]; j -= b.split_j[ji]; }
+    if (j >= r_out) return;
+    if (b.transpose_out[ji]) out[j * width + c] = s;
     else out[c * r_out + j] = s;
 }
 
-static int tn_splits(int64_t n_rows, int64_t width) {
-    int64_t col_tiles = xq_cdiv(width, 128);
+// Row splits of `col_tiles` column tiles: about three blocks per compute unit, 512 rows each at least (below 1024 rows the
+// second launch that sums the splits costs more than the split saves)
+static int tn_splits(int64_t n_rows, int64_t col_tiles) {
     int64_t s = xq_cdiv(768, col_tiles);
-    int64_t max_s = n_rows / 256 > 0 ? n_rows / 256 : 1;
+    const int64_t max_s = n_rows / 512 > 0 ? n_rows / 512 : 1;
     if (s > max_s) s = max_s;
     if (s > 32) s = 32;
     return (int)(s < 1 ? 1 : s);
 }
 
 int64_t tn_partial_bytes(int64_t n_rows, int64_t width, int r_pad) {
-    const int64_t dense = (int64_t)tn_splits(n_rows, width) * width * r_pad * 4;
+    const int64_t dense = (int64_t)tn_splits(n_rows, xq_cdiv(width, 128)) * width * r_pad * 4;      // (a joint launch splits less)
     const int64_t grouped = xq_cdiv(n_rows > 0 ? n_rows : 1, TN_CHUNK) * 2 * width * r_pad * 4;
-    return dense > grouped ? dense : grouped;
+    const int64_t b = dense > grouped ? dense : grouped;
+    return (b + 255) & ~(int64_t)255;
+}
+
+static int tn_check(const bf16_t* P, int64_t ldp, int64_t width, const bf16_t* Q, int64_t ldq, int r_pad, int r_out) {
+    XQ_REQUIRE(ldq >= r_pad && ldq % 8 == 0, "tn: Q pitch %lld must be a multiple of 8 and at least r_pad", (long long)ldq);
+    XQ_REQUIRE(r_pad > 0 && r_pad <= 64 && r_pad % 16 == 0 && r_out <= r_pad, "tn: bad rank (r_pad %d, r_out %d)", r_pad, r_out);
+    XQ_REQUIRE(width % 8 == 0 && ldp % 8 == 0 && xq_aligned(P, 16) && xq_aligned(Q, 16), "tn: operands must be 16-byte aligned, width %% 8 == 0");
+    return XQ_OK;
+}
+
+int launch_tn_multi(const TnJob* jobs, int n, int64_t n_rows, float* partial, hipStream_t stream, const int32_t* row_limit) {
+    XQ_REQUIRE(n >= 0 && n <= kTnJobs, "tn: %d products", n);
+    XQ_REQUIRE(partial != nullptr, "tn: partial workspace is NULL");
+    TnBatch b{};
+    TnReduceBatch rb{};
+    int64_t col_tiles = 0;
+    for (int i = 0; i < n; ++i) col_tiles += xq_cdiv(jobs[i].width, 128);
+    const int S = col_tiles > 0 ? tn_splits(n_rows, col_tiles) : 1;
+    const int64_t rps = xq_cdiv(xq_cdiv(n_rows, S), 32) * 32;
+    int nt = 1;
+    int64_t blocks = 0, rblocks = 0;
+    for (int i = 0; i < n; ++i) {
+        const TnJob& j = jobs[i];
+        const int64_t ldq = j.ldq > 0 ? j.ldq : j.r_pad;
+        const int rc = tn_check(j.P, j.ldp, j.width, j.Q, ldq, j.r_pad, j.r_out);
+        if (rc) return rc;
+        if (j.width == 0 || j.r_out == 0) continue;
+        const int k = b.n++;
+        b.job[k] = TnArgs{j.P, j.ldp, j.width, j.Q, j.r_pad, j.r_out, n_rows, rps, j.transpose_out ? 1 : 0, j.out, nullptr, row_limit, ldq, j.p_rows, j.out2, j.split_j};
+        b.partial[k] = partial;
+        b.splits[k] = S;
+        b.first[k] = (int32_t)blocks;
+        blocks += xq_cdiv(j.width, 128) * S;
+        if (j.r_pad > 32) nt = 2;
+        rb.partial[k] = partial; rb.out[k] = j.out; rb.out2[k] = j.out2; rb.width[k] = j.width; rb.splits[k] = S;
+        rb.r_pad[k] = j.r_pad; rb.r_out[k] = j.r_out; rb.transpose_out[k] = j.transpose_out ? 1 : 0; rb.split_j[k] = j.split_j;
+        rb.first[k] = (int32_t)rblocks;
+        rblocks += xq_cdiv(j.width * j.r_pad, 256);
+        partial += tn_partial_bytes(n_rows, j.width, j.r_pad) / 4;
+    }
+    if (b.n == 0) return XQ_OK;
+    if (nt == 1) tn_kernel<1><<<(unsigned)blocks, 256, 0, stream>>>(b);
+    else tn_kernel<2><<<(unsigned)blocks, 256, 0, stream>>>(b);
+    XQ_CHECK_LAUNCH("tn");
+    if (S > 1) {
+        rb.n = b.n;
+        tn_reduce_kernel<<<(unsigned)rblocks, 256, 0, stream>>>(rb);
+        XQ_CHECK_LAUNCH("tn_reduce");
+    }
+    return XQ_OK;
 }
 
 int launch_tn(const bf16_t* P, int64_t ldp, int64_t width, const bf16_t* Q, int r_pad, int r_out, int64_t n_rows,
               bool transpose_out, float* out, float* partial, const int32_t* offsets, int32_t num_experts,
               hipStream_t stream, const int32_t* row_limit, int64_t ldq, const int32_t* p_rows) {
     if (ldq <= 0) ldq = r_pad;
-    XQ_REQUIRE(ldq >= r_pad && ldq % 8 == 0, "tn: Q pitch %lld must be a multiple of 8 and at least r_pad", (long long)ldq);
-    XQ_REQUIRE(r_pad > 0 && r_pad <= 64 && r_pad % 16 == 0 && r_out <= r_pad, "tn: bad rank (r_pad %d, r_out %d)", r_pad, r_out);
-    XQ_REQUIRE(width % 8 == 0 && ldp % 8 == 0 && xq_aligned(P, 16) && xq_aligned(Q, 16), "tn: operands must be 16-byte aligned, width %% 8 == 0");
+    if (!offsets) {
+        const TnJob j{P, ldp, width, Q, ldq, r_pad, r_out, transpose_out, out, p_rows};
+        return launch_tn_multi(&j, 1, n_rows, partial, stream, row_limit);
+    }
+    const int rc = tn_check(P, ldp, width, Q, ldq, r_pad, r_out);
+    if (rc) return rc;
     if (width == 0 || r_out == 0) return XQ_OK;
-    TnArgs g{P, ldp, width, Q, r_pad, r_out, n_rows, 0, transpose_out ? 1 : 0, out, offsets, offsets ? nullptr : row_limit, ldq, p_rows};
-    unsigned col_tiles = (unsigned)xq_cdiv(width, 128);
+    TnArgs g{P, ldp, width, Q, r_pad, r_out, n_rows, 0, transpose_out ? 1 : 0, out, offsets, nullptr, ldq, p_rows, nullptr, 0};
+    const unsigned col_tiles = (unsigned)xq_cdiv(width, 128);
     XQ_REQUIRE(partial != nullptr, "tn: partial workspace is NULL");
-    if (offsets) {
-        if (n_rows > 0) {
-            dim3 grid(col_tiles, (unsigned)xq_cdiv(n_rows, TN_CHUNK));
-            if (r_pad <= 32) tn_grouped_kernel<1><<<grid, 256, 0, stream>>>(g, num_experts, partial);
-            else tn_grouped_kernel<2><<<grid, 256, 0, stream>>>(g, num_experts, partial);
-            XQ_CHECK_LAUNCH("tn(grouped)");
-        }
-        dim3 rgrid((unsigned)xq_cdiv(width * r_pad, 256), (unsigned)num_experts);
-        tn_grouped_reduce_kernel<<<rgrid, 256, 0, stream>>>(partial, offsets, width, r_pad, r_out, transpose_out ? 1 : 0, out);
-        XQ_CHECK_LAUNCH("tn(grouped reduce)");
+    // up to 256 rows an expert on average a block takes an expert's rows whole and writes its result: nothing is summed
+    // afterwards, and the experts of a column tile run side by side instead of one after the other (456 rows of 128 experts,
+    // 768 columns: 289 us in 6 blocks, 8 us in 768); beyond that, chunks of the row range keep uneven experts level
+    if (n_rows <= 256ll * num_experts) {
+        const dim3 grid(col_tiles, (unsigned)num_experts);
+        if (r_pad <= 32) tn_expert_kernel<1><<<grid, 256, 0, stream>>>(g);
+        else tn_expert_kernel<2><<<grid, 256, 0, stream>>>(g);
+        XQ_CHECK_LAUNCH("tn(expert)");
         return XQ_OK;
     }
-    int S = tn_splits(n_rows, width);
-    int64_t rps = xq_cdiv(xq_cdiv(n_rows, S), 32) * 32;
-    g.rows_per_split = rps;
-    g.out = partial;
-    dim3 grid(col_tiles, (unsigned)S);
-    if (r_pad <= 32) tn_kernel<1><<<grid, 256, 0, stream>>>(g);
-    else tn_kernel<2><<<grid, 256, 0, stream>>>(g);
-    XQ_CHECK_LAUNCH("tn");
-    tn_reduce_kernel<<<dim3((unsigned)xq_cdiv(width * r_pad, 256)), 256, 0, stream>>>(partial, S, width, r_pad, r_out,
-                                                                                      transpose_out ? 1 : 0, out);
-    XQ_CHECK_LAUNCH("tn_reduce");
+    dim3 grid(col_tiles, (unsigned)xq_cdiv(n_rows, TN_CHUNK));
+    if (r_pad <= 32) tn_grouped_kernel<1><<<grid, 256, 0, stream>>>(g, num_experts, partial);
+    else tn_grouped_kernel<2><<<grid, 256, 0, stream>>>(g, num_experts, partial);
+    XQ_CHECK_LAUNCH("tn(grouped)");
+    dim3 rgrid((unsigned)xq_cdiv(width * r_pad, 256), (unsigned)num_experts);
+    tn_grouped_reduce_kernel<<<rgrid, 256, 0, stream>>>(partial, offsets, width, r_pad, r_out, transpose_out ? 1 : 0, out);
+    XQ_CHECK_LAUNCH("tn(grouped reduce)");
     return XQ_OK;
 }
 

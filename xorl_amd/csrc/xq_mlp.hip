@@ -10,6 +10,7 @@
 // Other formats (and shapes the fused forms do not take) run the same program launch by launch.
 #include "xq_lora.h"
 #include "xq_skinny.h"
+#include <algorithm>
 #include <atomic>
 #include <stdlib.h>
 
@@ -34,12 +35,6 @@ struct Dims {
     int64_t M, H, I;
     int r, rp;
 };
-
-// dst[j][c] = src[j0 + j][c] for j < rows: the two factor gradients that one pass over x left in one matrix
-__global__ void __launch_bounds__(256) copy_rows_kernel(const float* src, int64_t width, int j0, int rows, float* dst) {
-    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (t < (int64_t)rows * width) dst[t] = src[(int64_t)j0 * width + t];
-}
 
 // a[m][c] = bf16(a[m][c] + b[m][c]): the two shares of dX when the dgrads of gate and up run as separate launches
 __global__ void __launch_bounds__(256) add_rows_kernel(bf16_t* a, int64_t lda, const bf16_t* b, int64_t ldb, int64_t rows, int64_t cols8) {
@@ -105,21 +100,33 @@ int check_call(const xq_weight* gate, const xq_weight* up, const xq_weight* down
     return XQ_OK;
 }
 
-int64_t fwd_workspace(const Dims& d) {
-    const int64_t rp = d.rp ? d.rp : 16;
+// one region of split-K partial sums and fp32 sums of the SwiGLU passes (stream order)
+int64_t gemm_part_bytes(const Dims& d) {
     const int64_t pa = tile_gemm_partial_bytes(d.M, d.I, d.H), pb = tile_gemm_partial_bytes(d.M, d.H, d.I);
-    return al256(2 * rp * d.H * 2) + 2 * al256(d.I * rp * 2) + al256(rp * d.I * 2) + al256(d.H * rp * 2) + al256(pa > pb ? pa : pb) + 512;
+    const int64_t ps = d.rp && silu_bwd_nt_supported(d.I, d.rp) ? silu_nt_partial_bytes(d.M, d.I, d.rp) : 0;
+    return std::max(std::max(pa, pb), ps);
 }
 
+// From a block of 32 rows per compute unit on, the forward lays the A factors out as bf16 panels once and forms s * h . A_d^T in
+// the pass that writes h (8192 rows, 12288 columns: 142 us against 120 for the elementwise pass and 41 for the product).
+// Below, the product is a launch of its own: blocks of 32 rows would leave compute units idle.
+bool many_rows(const Dims& d) { return d.rp > 0 && d.M >= 32ll * num_cus() && silu_bwd_nt_supported(d.I, d.rp); }
+int64_t fwd_panel_bytes(const Dims& d) {
+    if (!d.rp) return 0;
+    if (many_rows(d)) return al256(2 * d.rp * d.H * 2) + al256(d.rp * d.I * 2);
+    const int64_t gu = 2 * d.rp <= 64 ? lowrank_panel_bytes(1, d.M, 2 * d.rp, d.H) : lowrank_panel_bytes(2, d.M, d.rp, d.H);
+    return std::max(gu, lowrank_panel_bytes(1, d.M, d.rp, d.I));
+}
+
+int64_t fwd_workspace(const Dims& d) { return fwd_panel_bytes(d) + al256(gemm_part_bytes(d)) + 512; }
+
 int64_t bwd_workspace(const Dims& d) {
-    const int64_t rp = d.rp ? d.rp : 16, wide = d.H > d.I ? d.H : d.I;
-    const int64_t panels = al256(rp * d.H * 2) + al256(d.I * rp * 2) + 2 * al256(rp * d.I * 2) + al256(d.H * 2 * rp * 2);
-    int64_t tn = tn_partial_bytes(d.M, wide, 2 * rp <= 64 ? 2 * rp : rp);
-    const int64_t pa = tile_gemm_partial_bytes(d.M, d.I, d.H), pb = tile_gemm_partial_bytes(d.M, d.H, d.I);
-    tn = tn > pa ? tn : pa;
-    tn = tn > pb ? tn : pb;
-    return panels + al256(d.M * d.I * 2) + al256(d.M * 2 * d.I * 2) + al256(d.M * d.H * 2) + al256(d.M * rp * 2) +
-           al256(d.M * 2 * rp * 2) + al256(2 * rp * d.H * 4) + al256(tn) + 512;
+    const int64_t rp = d.rp ? d.rp : 16;
+    // the six factor gradients share a launch: partial sums of all of them (dA of gate and up of twice the rank, or apart)
+    const int64_t tn = 3 * tn_partial_bytes(d.M, d.I, rp) + tn_partial_bytes(d.M, d.H, rp) +
+                       std::max(2 * tn_partial_bytes(d.M, d.H, rp), 2 * rp <= 64 ? tn_partial_bytes(d.M, d.H, 2 * rp) : 0);
+    return al256(d.M * d.I * 2) + al256(d.M * 2 * d.I * 2) + al256(d.M * d.H * 2) + al256(d.M * rp * 2) +
+           al256(d.M * 2 * rp * 2) + 2 * al256(rp * d.I * 2) + al256(std::max(gemm_part_bytes(d), tn)) + 512;
 }
 
 }  // namespace
@@ -162,55 +169,62 @@ extern "C" int xq_mlp_fwd(const xq_weight* gate, const xq_weight* up, const xq_w
     bf16_t *gu = (bf16_t*)saved->gate_up, *h = (bf16_t*)saved->h;
     bf16_t *su_gu = (bf16_t*)saved->su_gate_up, *su_d = (bf16_t*)saved->su_down;
     Carve cv{(uint8_t*)workspace, 0};
-    bf16_t *A_gu = nullptr, *Bl_g = nullptr, *Bl_u = nullptr, *A_d = nullptr, *Bl_d = nullptr;
     const SuLayout sl = su_layout(fused, rp, M);
-    const bool one_pass = fused && rp > 0 && 2 * rp <= 64;      // both low-rank intermediates from one pass over x
+    const int f32 = lora->dtype == XQ_DT_F32;
+    auto right_of = [&](int p) { return LowRankRight{{lora->B[p], nullptr}, r, r, rp, f32, 0}; };
+    const LowRankRight right_g = right_of(0), right_u = right_of(1), right_d = right_of(2);
+    FactorMode fm = factor_mode(lora->dtype, false);
+    bf16_t* panels = cv.take<bf16_t>(fwd_panel_bytes(d));
+    const void *A_g = lora->A[0], *A_u = lora->A[1];
+    const bool many = many_rows(d) && !fused;
+    bf16_t* A_d = panels + 2 * (int64_t)rp * H;
+    int ra = r;                                   // ranks in the factors the products read
+    if (many) {
+        PanelJobs pj{};
+        pj.in_f32 = f32;
+        A_g = pj.add(lora->A[0], 1, r, H, false, panels, 1, rp, H);
+        A_u = pj.add(lora->A[1], 1, r, H, false, panels + (int64_t)rp * H, 1, rp, H);
+        pj.add(lora->A[2], 1, r, I, false, A_d, 1, rp, I);
+        if ((rc = launch_panel_prep(pj, stream))) return rc;
+        fm = kFacBf16;
+        ra = rp;
+    }
     if (rp) {
-        // panels: [A_g ; A_u] as [2 rp, H] (the rows of x . A^T), B as [out, rp] right-hand panels
-        PanelJobs jobs{};
-        jobs.in_f32 = lora->dtype == XQ_DT_F32;
-        A_gu = cv.take<bf16_t>(2 * rp * H * 2);
-        jobs.add(lora->A[0], 1, r, H, false, A_gu, 1, rp, H);
-        jobs.add(lora->A[1], 1, r, H, false, A_gu + (int64_t)rp * H, 1, rp, H);
-        Bl_g = jobs.add(lora->B[0], 1, I, r, false, cv.take<bf16_t>(I * rp * 2), 1, I, rp);
-        Bl_u = jobs.add(lora->B[1], 1, I, r, false, cv.take<bf16_t>(I * rp * 2), 1, I, rp);
-        A_d = jobs.add(lora->A[2], 1, r, I, false, cv.take<bf16_t>(rp * I * 2), 1, rp, I);
-        Bl_d = jobs.add(lora->B[2], 1, H, r, false, cv.take<bf16_t>(H * rp * 2), 1, H, rp);
-        if ((rc = launch_panel_prep(jobs, stream))) return rc;
-        // bf16(s * x . A^T) of gate and up
-        if (one_pass) {
-            if ((rc = launch_small_nt(x, ldx, M, H, A_gu, 2 * rp, s, su_gu, nullptr, nullptr, 1, true, stream))) return rc;
-        } else {
-            if ((rc = launch_small_nt(x, ldx, M, H, A_gu, rp, s, su_gu, nullptr, nullptr, 1, true, stream, sl.pitch))) return rc;
-            if ((rc = launch_small_nt(x, ldx, M, H, A_gu + (int64_t)rp * H, rp, s, su_gu + sl.up_offset, nullptr, nullptr, 1, true, stream, sl.pitch))) return rc;
-        }
+        // bf16(s * x . A^T) of gate and up: one pass over x where both factors fit one
+        const LowRankJob both{x, ldx, H, {A_g, A_u}, 2, ra, rp, s, su_gu, sl.pitch, sl.up_offset};
+        const LowRankJob apart[2] = {{x, ldx, H, {A_g, nullptr}, 1, ra, rp, s, su_gu, sl.pitch, 0},
+                                     {x, ldx, H, {A_u, nullptr}, 1, ra, rp, s, su_gu + sl.up_offset, sl.pitch, 0}};
+        rc = 2 * rp <= 64 ? launch_lowrank(&both, 1, M, fm, panels, stream) : launch_lowrank(apart, 2, M, fm, panels, stream);
+        if (rc) return rc;
     }
     float* part = cv.take<float>(0);
     const int64_t part_bytes = workspace_bytes - cv.used;
     const bf16_t *bias_g = (const bf16_t*)lora->bias[0], *bias_u = (const bf16_t*)lora->bias[1], *bias_d = (const bf16_t*)lora->bias[2];
-    bool h_product_done = false;
     if (fused) {
-        if ((rc = launch_gate_up_swiglu(gate, up, x, ldx, M, rp ? su_gu : nullptr, rp ? su_gu + sl.up_offset : nullptr, sl.pitch, Bl_g, Bl_u,
-                                        rp, bias_g, bias_u, gu, 2 * I, h, I, stream)))
+        if ((rc = launch_gate_up_swiglu(gate, up, x, ldx, M, rp ? su_gu : nullptr, rp ? su_gu + sl.up_offset : nullptr, sl.pitch,
+                                        LowRankRight{{lora->B[0], lora->B[1]}, r, r, rp, f32, 0}, rp, bias_g, bias_u, gu, 2 * I, h, I, stream)))
             return rc;
     } else {
-        if ((rc = launch_tile_gemm(gate, true, x, ldx, M, nullptr, nullptr, rp ? su_gu : nullptr, Bl_g, rp, bias_g, gu, 2 * I, stream, who, part, part_bytes))) return rc;
-        if ((rc = launch_tile_gemm(up, true, x, ldx, M, nullptr, nullptr, rp ? su_gu + sl.up_offset : nullptr, Bl_u, rp, bias_u, gu + I, 2 * I, stream, who, part, part_bytes))) return rc;
-        // SwiGLU, and s * h . A_d^T of the down projection from the values on their way out where the rank allows
-        if (rp && g_mlp_silu_nt && silu_bwd_nt_supported(I, rp)) {
+        if ((rc = launch_tile_gemm(gate, true, x, ldx, M, nullptr, nullptr, rp ? su_gu : nullptr, nullptr, rp, bias_g, gu, 2 * I, stream, who, part, part_bytes, nullptr, rp ? &right_g : nullptr))) return rc;
+        if ((rc = launch_tile_gemm(up, true, x, ldx, M, nullptr, nullptr, rp ? su_gu + sl.up_offset : nullptr, nullptr, rp, bias_u, gu + I, 2 * I, stream, who, part, part_bytes, nullptr,
+                                   rp ? &right_u : nullptr))) return rc;
+        if (many) {
             if ((rc = launch_silu_fwd_nt(gu, gu + I, 2 * I, h, I, M, I, A_d, rp, s, su_d, rp, stream))) return rc;
-            h_product_done = true;
         } else if ((rc = xq_silu_mul_fwd(gu, gu + I, 2 * I, nullptr, h, I, M, I, stream))) {
             return rc;
         }
     }
-    if (rp && !h_product_done && (rc = launch_small_nt(h, I, M, I, A_d, rp, s, su_d, nullptr, nullptr, 1, true, stream))) return rc;
-    return launch_tile_gemm(down, true, h, I, M, nullptr, nullptr, rp ? su_d : nullptr, Bl_d, rp, bias_d, (bf16_t*)y, ldy, stream,
-                            who, part, part_bytes);
+    if (rp && !many) {
+        const LowRankJob jd{h, I, I, {lora->A[2], nullptr}, 1, r, rp, s, su_d, rp, 0};
+        if ((rc = launch_lowrank(&jd, 1, M, fm, panels, stream))) return rc;
+    }
+    return launch_tile_gemm(down, true, h, I, M, nullptr, nullptr, rp ? su_d : nullptr, nullptr, rp, bias_d, (bf16_t*)y, ldy, stream,
+                            who, part, part_bytes, nullptr, rp ? &right_d : nullptr);
 }
 
-// ---- forward only: nothing is kept for a backward, so each projection is free to take the kernel that suits the row
-// count -- at decode sizes the weight-streaming kernels (gate and up as one launch), not the tile kernels above
+// ---- forward only: nothing is kept for a backward, so up to 64 rows each projection is free to take the kernel that suits the
+// row count (the weight-streaming kernels, gate and up as one launch); beyond, the program of xq_mlp_fwd is the fastest one
+// and runs with the buffers it would keep in the workspace
 static int64_t infer_linear_ws(int64_t M, int64_t H, int64_t I, int r) {
     const int64_t b = xq_linear_workspace_bytes(M, H, I, r);
     int64_t a = xq_linear_workspace_bytes(M, I, H, r);
@@ -223,7 +237,10 @@ static int64_t infer_linear_ws(int64_t M, int64_t H, int64_t I, int r) {
 
 extern "C" int64_t xq_mlp_infer_workspace_bytes(int64_t M, int64_t hidden, int64_t intermediate, int r) {
     if (M < 0 || r < 0) return 0;
-    return al256(M * 2 * intermediate * 2) + al256(M * intermediate * 2) + infer_linear_ws(M, hidden, intermediate, r) + 256;
+    const int64_t act = al256(M * 2 * intermediate * 2) + al256(M * intermediate * 2);
+    const int64_t program = al256(M * 2 * r_pad_of(r) * 2) + al256(M * r_pad_of(r) * 2) + fwd_workspace(Dims{M, hidden, intermediate, r, r_pad_of(r)});
+    const int64_t apart = M <= 64 ? infer_linear_ws(M, hidden, intermediate, r) : 0;
+    return act + (program > apart ? program : apart) + 256;
 }
 
 extern "C" int xq_mlp_fwd_infer(const xq_weight* gate, const xq_weight* up, const xq_weight* down, const xq_mlp_lora* lora,
@@ -243,6 +260,13 @@ extern "C" int xq_mlp_fwd_infer(const xq_weight* gate, const xq_weight* up, cons
                "%s: workspace smaller than xq_mlp_infer_workspace_bytes()", who);
     bf16_t* gu = cv.take<bf16_t>(M * 2 * d.I * 2);
     bf16_t* h = cv.take<bf16_t>(M * d.I * 2);
+    if (!(skinny_supported(gate, M) || skinny_supported(up, M) || skinny_supported(down, M))) {
+        bf16_t* su_gu = cv.take<bf16_t>(M * 2 * d.rp * 2);
+        bf16_t* su_d = cv.take<bf16_t>(M * d.rp * 2);
+        xq_mlp_saved own{gu, h, su_gu, su_d, -1, 0};
+        void* program_ws = cv.take<uint8_t>(0);
+        return xq_mlp_fwd(gate, up, down, lora, x, ldx, M, y, ldy, &own, program_ws, workspace_bytes - cv.used, stream);
+    }
     void* ws = cv.take<uint8_t>(0);
     const int64_t ws_bytes = workspace_bytes - cv.used;
     xq_linear_job jobs[2] = {
@@ -304,38 +328,30 @@ extern "C" int xq_mlp_bwd(const xq_weight* gate, const xq_weight* up, const xq_w
     const bool fused = two_dense_supported(gate) && two_dense_supported(up) && rp2 <= 64;
 
     Carve cv{(uint8_t*)workspace, 0};
-    bf16_t *Bt_d = nullptr, *At_d = nullptr, *Bt_g = nullptr, *Bt_u = nullptr, *At_gu = nullptr;
-    if (rp) {
-        PanelJobs jobs{};
-        jobs.in_f32 = lora->dtype == XQ_DT_F32;
-        Bt_d = jobs.add(lora->B[2], 1, H, r, true, cv.take<bf16_t>(rp * H * 2), 1, rp, H);          // [rp, H]: rows of dy . B
-        At_d = jobs.add(lora->A[2], 1, r, I, true, cv.take<bf16_t>(I * rp * 2), 1, I, rp);          // [I, rp]: right-hand panel of the dgrad
-        Bt_g = jobs.add(lora->B[0], 1, I, r, true, cv.take<bf16_t>(rp * I * 2), 1, rp, I);
-        Bt_u = jobs.add(lora->B[1], 1, I, r, true, cv.take<bf16_t>(rp * I * 2), 1, rp, I);
-        At_gu = cv.take<bf16_t>(H * rp2 * 2);            // fused: [H, 2 rp] = A_g^T | A_u^T; else A_g^T [H, rp] then A_u^T [H, rp]
-        jobs.add(lora->A[0], 1, r, H, true, At_gu, 1, H, rp, fused ? rp2 : rp);
-        jobs.add(lora->A[1], 1, r, H, true, fused ? At_gu + rp : At_gu + H * rp, 1, H, rp, fused ? rp2 : rp);
-        if ((rc = launch_panel_prep(jobs, stream))) return rc;
-    } else {
-        (void)cv.take<bf16_t>(0);
-    }
+    const int f32 = lora->dtype == XQ_DT_F32;
+    const FactorMode ft = factor_mode(lora->dtype, true);
+    // right-hand factors of the dgrads: A^T of down, and of gate and up (side by side in the launch over both)
+    const LowRankRight right_d{{lora->A[2], nullptr}, I, r, rp, f32, 1}, right_gu{{lora->A[0], lora->A[1]}, H, r, rp, f32, 1},
+        right_g{{lora->A[0], nullptr}, H, r, rp, f32, 1}, right_u{{lora->A[1], nullptr}, H, r, rp, f32, 1};
     bf16_t* dh = cv.take<bf16_t>(M * I * 2);
     bf16_t* dgu = cv.take<bf16_t>(M * 2 * I * 2);         // [M, 2I]: dgate | dup
     bf16_t* dx_u = cv.take<bf16_t>(M * H * 2);            // unfused dgrads: the up projection's share of dX
     bf16_t* v_d = cv.take<bf16_t>(M * (rp ? rp : 16) * 2);
     bf16_t* v_gu = cv.take<bf16_t>(M * (rp ? rp2 : 32) * 2);
-    float* pair = cv.take<float>((int64_t)(rp ? rp2 : 32) * H * 4);
+    bf16_t* Bt_g = cv.take<bf16_t>((int64_t)(rp ? rp : 16) * I * 2);    // panels of the gate and up factors (many rows)
+    bf16_t* Bt_u = cv.take<bf16_t>((int64_t)(rp ? rp : 16) * I * 2);
     float* part = cv.take<float>(0);
     const int64_t part_bytes = workspace_bytes - cv.used;
     bf16_t *dgate = dgu, *dup = dgu + I;
 
     // ---- down projection
-    if (rp && (rc = launch_small_nt(dy, lddy, M, H, Bt_d, rp, s, v_d, nullptr, nullptr, 1, true, stream))) return rc;
-    if ((rc = launch_tile_gemm(down, false, dy, lddy, M, nullptr, nullptr, rp ? v_d : nullptr, At_d, rp, nullptr, dh, I, stream, who, part, part_bytes))) return rc;
     if (rp) {
-        if ((rc = launch_tn(dy, lddy, H, su_d, rp, r, M, false, grads->dB[2], part, nullptr, 1, stream))) return rc;       // [H, r]
-        if ((rc = launch_tn(h, I, I, v_d, rp, r, M, true, grads->dA[2], part, nullptr, 1, stream))) return rc;             // [r, I]
+        const LowRankJob jd{dy, lddy, H, {lora->B[2], nullptr}, 1, r, rp, s, v_d, rp, 0};
+        if ((rc = launch_lowrank(&jd, 1, M, ft, nullptr, stream))) return rc;
     }
+    if ((rc = launch_tile_gemm(down, false, dy, lddy, M, nullptr, nullptr, rp ? v_d : nullptr, nullptr, rp, nullptr, dh, I, stream, who, part, part_bytes,
+                               nullptr, rp ? &right_d : nullptr)))
+        return rc;
     // ---- SwiGLU, and s * dgate . B_g^T, s * dup . B_u^T: one pass over (gate, up, dh) where the rank allows, so that the
     // two products do not read dgate | dup back
     const int64_t ld_v = fused ? rp2 : rp;
@@ -343,38 +359,53 @@ extern "C" int xq_mlp_bwd(const xq_weight* gate, const xq_weight* up, const xq_w
     bf16_t* v_u = fused ? v_gu + rp : v_gu + M * rp;
     const bool one_pass = rp && g_mlp_silu_nt && silu_bwd_nt_supported(I, rp);
     if (one_pass) {
-        if ((rc = launch_silu_bwd_nt(gu, gu + I, 2 * I, dh, I, dgate, dup, 2 * I, M, I, Bt_g, Bt_u, rp, s, v_g, v_u, ld_v, stream))) return rc;
+        // every 32 rows read both factors: from 2048 rows on a launch that lays them out as bf16 panels once is the shorter way
+        // (8192 rows, r 32: 288 us from the fp32 factors, 206 + 8 from panels; 1000 rows, r 16: 37 against 30 + 6)
+        const void *Fg = lora->B[0], *Fu = lora->B[1];
+        FactorMode fmode = ft;
+        if (M >= 2048) {
+            PanelJobs jobs{};
+            jobs.in_f32 = f32;
+            Fg = jobs.add(lora->B[0], 1, I, r, true, Bt_g, 1, rp, I);
+            Fu = jobs.add(lora->B[1], 1, I, r, true, Bt_u, 1, rp, I);
+            if ((rc = launch_panel_prep(jobs, stream))) return rc;
+            fmode = kFacBf16;
+        }
+        if ((rc = launch_silu_bwd_nt(gu, gu + I, 2 * I, dh, I, dgate, dup, 2 * I, M, I, Fg, Fu, fmode, fmode == kFacBf16 ? rp : r, rp, s, v_g, v_u, ld_v, part, stream))) return rc;
     } else if ((rc = xq_silu_mul_bwd(gu, gu + I, 2 * I, dh, I, nullptr, dgate, dup, 2 * I, nullptr, M, I, stream))) {
         return rc;
     }
     // ---- gate / up
     if (rp) {
         if (!one_pass) {
-            if ((rc = launch_small_nt(dgate, 2 * I, M, I, Bt_g, rp, s, v_g, nullptr, nullptr, 1, true, stream, ld_v))) return rc;
-            if ((rc = launch_small_nt(dup, 2 * I, M, I, Bt_u, rp, s, v_u, nullptr, nullptr, 1, true, stream, ld_v))) return rc;
+            const LowRankJob jv[2] = {{dgate, 2 * I, I, {lora->B[0], nullptr}, 1, r, rp, s, v_g, ld_v, 0}, {dup, 2 * I, I, {lora->B[1], nullptr}, 1, r, rp, s, v_u, ld_v, 0}};
+            if ((rc = launch_lowrank(jv, 2, M, ft, nullptr, stream))) return rc;
         }
+        // the six factor gradients, one launch: dB[H, r] = dy^T . su_d, dA[r, I] = (h^T . v_d)^T, dB[I, r] of gate and up, dA[r, H] of both
         const SuLayout sl = su_layout(saved->gate_up_fused == 1, rp, M);
-        if ((rc = launch_tn(dgate, 2 * I, I, su_gu, rp, r, M, false, grads->dB[0], part, nullptr, 1, stream, nullptr, sl.pitch))) return rc;        // [I, r]
-        if ((rc = launch_tn(dup, 2 * I, I, su_gu + sl.up_offset, rp, r, M, false, grads->dB[1], part, nullptr, 1, stream, nullptr, sl.pitch))) return rc;
-        if (fused) {       // [2 rp, H] = [v_g | v_u]^T . x, then its two bands
-            if ((rc = launch_tn(x, ldx, H, v_gu, rp2, rp2, M, true, pair, part, nullptr, 1, stream))) return rc;
-            const unsigned blocks = (unsigned)xq_cdiv((int64_t)r * H, 256);
-            copy_rows_kernel<<<dim3(blocks), 256, 0, stream>>>(pair, H, 0, r, grads->dA[0]);
-            copy_rows_kernel<<<dim3(blocks), 256, 0, stream>>>(pair, H, rp, r, grads->dA[1]);
-            XQ_CHECK_LAUNCH(who);
+        TnJob jobs[6] = {{dy, lddy, H, su_d, rp, rp, r, false, grads->dB[2]},
+                         {h, I, I, v_d, rp, rp, r, true, grads->dA[2]},
+                         {dgate, 2 * I, I, su_gu, sl.pitch, rp, r, false, grads->dB[0]},
+                         {dup, 2 * I, I, su_gu + sl.up_offset, sl.pitch, rp, r, false, grads->dB[1]}};
+        int n = 4;
+        if (fused) {       // [v_g | v_u]^T . x: one pass over x
+            jobs[n++] = TnJob{x, ldx, H, v_gu, rp2, rp2, r, true, grads->dA[0], nullptr, grads->dA[1], rp};
         } else {
-            if ((rc = launch_tn(x, ldx, H, v_g, rp, r, M, true, grads->dA[0], part, nullptr, 1, stream))) return rc;       // [r, H]
-            if ((rc = launch_tn(x, ldx, H, v_u, rp, r, M, true, grads->dA[1], part, nullptr, 1, stream))) return rc;
+            jobs[n++] = TnJob{x, ldx, H, v_g, rp, rp, r, true, grads->dA[0]};
+            jobs[n++] = TnJob{x, ldx, H, v_u, rp, rp, r, true, grads->dA[1]};
         }
+        if ((rc = launch_tn_multi(jobs, n, M, part, stream))) return rc;
     }
     if (!dx) return XQ_OK;
     if (fused) {
         const TwoBanks two{up, nullptr, nullptr};
-        return launch_tile_gemm(gate, false, dgu, 2 * I, M, nullptr, nullptr, rp ? v_gu : nullptr, At_gu, rp2, nullptr, (bf16_t*)dx, lddx,
-                                stream, who, nullptr, 0, &two);
+        return launch_tile_gemm(gate, false, dgu, 2 * I, M, nullptr, nullptr, rp ? v_gu : nullptr, nullptr, rp2, nullptr, (bf16_t*)dx, lddx,
+                                stream, who, nullptr, 0, &two, rp ? &right_gu : nullptr);
     }
-    if ((rc = launch_tile_gemm(gate, false, dgate, 2 * I, M, nullptr, nullptr, rp ? v_g : nullptr, At_gu, rp, nullptr, (bf16_t*)dx, lddx, stream, who, part, part_bytes))) return rc;
-    if ((rc = launch_tile_gemm(up, false, dup, 2 * I, M, nullptr, nullptr, rp ? v_u : nullptr, At_gu + H * rp, rp, nullptr, dx_u, H, stream, who, part, part_bytes))) return rc;
+    if ((rc = launch_tile_gemm(gate, false, dgate, 2 * I, M, nullptr, nullptr, rp ? v_g : nullptr, nullptr, rp, nullptr, (bf16_t*)dx, lddx, stream, who, part, part_bytes, nullptr,
+                               rp ? &right_g : nullptr))) return rc;
+    if ((rc = launch_tile_gemm(up, false, dup, 2 * I, M, nullptr, nullptr, rp ? v_u : nullptr, nullptr, rp, nullptr, dx_u, H, stream, who, part, part_bytes, nullptr,
+                               rp ? &right_u : nullptr))) return rc;
     add_rows_kernel<<<dim3((unsigned)xq_cdiv(M * (H / 8), 256)), 256, 0, stream>>>((bf16_t*)dx, lddx, dx_u, H, M, H / 8);
     XQ_CHECK_LAUNCH(who);
     return XQ_OK;

@@ -129,3 +129,35 @@ def test_calls_left_to_the_python_path(hip_device):
         m(x.float())
     with pytest.raises(_C.XqError):
         m(x[:, :128].contiguous())
+
+
+def test_backward_reads_the_weight_where_it_is_then(hip_device):
+    """Sharded training frees the packed bytes after a forward and gathers them again before its backward, elsewhere."""
+    m, _ = make_dense_module("int4", 128, 256, 16, 32, 3, hip_device)
+    x = gen((70, 256), 1.0, 4, torch.bfloat16).to(hip_device).requires_grad_(True)
+    dy = gen((70, 128), 1.0, 5, torch.bfloat16).to(hip_device)
+    want = torch.autograd.grad(m(x), [x, m.lora_A, m.lora_B], dy)
+    y, y2, packed = m(x), m(x), m.packed_weight_f32
+    copy, storage = packed.detach().clone(), packed.untyped_storage()
+    nbytes = storage.nbytes()
+    storage.resize_(0)
+    other = torch.zeros_like(copy)                 # takes the block that was given back
+    with pytest.raises(RuntimeError, match="freed or resized"):
+        torch.autograd.grad(y2, [x, m.lora_A, m.lora_B], dy)
+    storage.resize_(nbytes)
+    assert packed.data_ptr() != other.data_ptr()
+    with torch.no_grad():
+        packed.copy_(copy)
+    for a, b in zip(torch.autograd.grad(y, [x, m.lora_A, m.lora_B], dy), want):
+        assert torch.equal(a, b)
+
+
+def test_tangents_and_transforms_are_refused_as_before(hip_device):
+    import torch.autograd.forward_ad as fwAD
+
+    m, _ = make_dense_module("int4", 128, 256, 16, 32, 3, hip_device)
+    x = gen((4, 256), 1.0, 4, torch.bfloat16).to(hip_device)
+    with fwAD.dual_level(), pytest.raises((RuntimeError, NotImplementedError)):
+        m(fwAD.make_dual(x, torch.ones_like(x)))
+    with pytest.raises(RuntimeError):
+        torch.vmap(lambda s: m(x) * s)(torch.ones(2, device=hip_device))

@@ -6,12 +6,15 @@
 // directly, outputs and workspaces come from torch's caching allocator without the dispatcher, and the backward is a C++
 // autograd node that runs without the interpreter.
 //
-// Every entry point returns None where anything is out of the ordinary (tensor subclasses, sharded or CPU state, quantization
-// noise, an active rank below the stored one, unexpected dtypes or layouts): the caller then takes its Python path, which
-// also raises the argument errors.  Nothing is remembered from one call to the next.
+// Every entry point returns None where anything is out of the ordinary (tensor subclasses, sharded or CPU state, tangents of
+// forward-mode differentiation, function transforms, a trace being recorded, quantization noise, an active rank below the
+// stored one, unexpected dtypes or layouts): the caller then takes its Python path, which also raises the argument errors.
+// Nothing is remembered from one call to the next, and a backward takes the addresses of the packed weights anew from
+// their tensors: storage may have been freed and filled again between the two.
 #include <Python.h>
 
 #include <ATen/TensorSubclassLikeUtils.h>
+#include <ATen/TracerMode.h>
 #include <ATen/core/Tensor.h>
 #include <ATen/EmptyTensor.h>
 #include <ATen/hip/impl/HIPCachingAllocatorMasqueradingAsCUDA.h>
@@ -80,13 +83,26 @@ bool get_number(PyObject* dict, PyObject* name, double* out) {
     return true;
 }
 
-// a plain torch tensor (or Parameter) on the GPU; subclasses, fakes and functorch wrappers are left to the Python path
+// a plain torch tensor (or Parameter) on the GPU; subclasses, fakes, functorch wrappers and tensors that carry a tangent are
+// left to the Python path (whose autograd functions refuse what they do not define)
 const Tensor* plain(PyObject* o) {
     if (!o || !THPVariable_CheckExact(o)) return nullptr;
     const Tensor& t = THPVariable_Unpack(o);
-    if (!t.defined() || !t.is_cuda() || at::isTensorSubclassLike(t)) return nullptr;
+    if (!t.defined() || !t.is_cuda() || at::isTensorSubclassLike(t) || t._fw_grad(0).defined()) return nullptr;
     return &t;
 }
+
+// a recorded trace or a function transform sees the operators of the Python path only
+bool under_transform() {
+    return at::tracer::impl::is_dispatch_enabled() ||
+           c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode);
+}
+
+// library calls launch kernels and may wait for room in the queue: other Python threads go on meanwhile
+struct ReleaseGil {
+    PyThreadState* state = PyEval_SaveThread();
+    ~ReleaseGil() { PyEval_RestoreThread(state); }
+};
 
 int scale_code(PyObject* dtype, int* bytes) {
     if (!dtype || !THPDtype_Check(dtype)) return -1;
@@ -113,6 +129,7 @@ int64_t nbytes(const Tensor& t) { return t.numel() * (int64_t)t.element_size(); 
 struct Weight {
     xq_weight w{};
     Tensor packed, scales, global_scale;
+    int64_t packed_bytes = 0, scale_bytes = 0;
 
     bool fill(int fmt, int layout, int64_t rows, int64_t cols, int64_t group, int64_t experts, PyObject* packed_o, PyObject* scales_o,
               PyObject* scale_dtype, PyObject* global_o, PyObject* global_dtype) {
@@ -139,7 +156,23 @@ struct Weight {
         w.format = fmt; w.layout = layout; w.scale_dtype = sd; w.group = (int32_t)group;
         w.rows = rows; w.cols = cols; w.num_experts = (int32_t)experts;
         w.packed = p->data_ptr(); w.scales = s->data_ptr();
+        packed_bytes = nbytes(*p); scale_bytes = nbytes(*s);
         return true;
+    }
+
+    // the descriptor for a later call: addresses as they are now, and storage that still holds the bytes
+    const xq_weight* now() {
+        auto held = [](const Tensor& t, int64_t bytes) {
+            return nbytes(t) == bytes && t.is_contiguous() &&
+                   (int64_t)t.storage().nbytes() >= t.storage_offset() * (int64_t)t.element_size() + bytes;
+        };
+        TORCH_CHECK(held(packed, packed_bytes) && held(scales, scale_bytes) &&
+                        (!global_scale.defined() || held(global_scale, nbytes(global_scale))),
+                    "the packed weight of a QLoRA module was freed or resized between forward and backward");
+        w.packed = packed.data_ptr();
+        w.scales = scales.data_ptr();
+        if (global_scale.defined()) w.global_scale = (const float*)global_scale.data_ptr();
+        return &w;
     }
 };
 
@@ -296,7 +329,7 @@ struct QLoRALinearBackward : public Node {
     variable_list apply(variable_list&& grads) override {
         std::lock_guard<std::mutex> lock(mutex_);
         variable_list out(4);
-        if (!grads[0].defined()) return out;
+        if (!grads[0].defined()) grads[0] = input_metadata(0).zeros_like();
         const Tensor x = x_.unpack(), A = A_.unpack(), B = B_.unpack(), su = su_.unpack(shared_from_this());
         const int64_t Nf = q.w.rows, K = q.w.cols;
         Tensor dy = cast_to(grads[0], at::kBFloat16);
@@ -308,7 +341,7 @@ struct QLoRALinearBackward : public Node {
         if (need_dA) out[1] = empty_f32({r, K});
         if (need_dB) out[2] = empty_f32({Nf, r});
         Scratch ws(xq_linear_workspace_bytes(M, Nf, K, r));
-        check(xq_linear_bwd(&q.w, xr.ptr, xr.ld, dr.ptr, dr.ld, M, A.data_ptr(), B.data_ptr(),
+        check(xq_linear_bwd(q.now(), xr.ptr, xr.ld, dr.ptr, dr.ld, M, A.data_ptr(), B.data_ptr(),
                             A.scalar_type() == at::kFloat ? XQ_DT_F32 : XQ_DT_BF16, r, (float)scaling, M ? su.data_ptr() : nullptr,
                             need_dx ? out[0].data_ptr() : nullptr, K, need_dA ? (float*)out[1].data_ptr() : nullptr,
                             need_dB ? (float*)out[2].data_ptr() : nullptr, ws.get(), ws.bytes, stream_of(x)));
@@ -348,7 +381,7 @@ struct QLoRAMLPBackward : public Node {
     variable_list apply(variable_list&& grads) override {
         std::lock_guard<std::mutex> lock(mutex_);
         variable_list out(7);                      // x, gate A, gate B, up A, up B, down A, down B
-        if (!grads[0].defined()) return out;
+        if (!grads[0].defined()) grads[0] = input_metadata(0).zeros_like();
         const Tensor x = x_.unpack();
         Tensor kept[4], A[3], B[3];
         for (int i = 0; i < 4; ++i) kept[i] = kept_[i].unpack(shared_from_this());
@@ -370,7 +403,7 @@ struct QLoRAMLPBackward : public Node {
         mlp_lora(&L, A, B, r, scaling);
         xq_mlp_saved S{kept[0].data_ptr(), kept[1].data_ptr(), kept[2].data_ptr(), kept[3].data_ptr(), gate_up_fused, 0};
         Scratch ws(xq_mlp_workspace_bytes(dr.M, H, I, r, 1));
-        check(xq_mlp_bwd(&q[0].w, &q[1].w, &q[2].w, &L, xr.ptr, xr.ld, dr.ptr, dr.ld, dr.M, &S, need_dx ? out[0].data_ptr() : nullptr, H, &G,
+        check(xq_mlp_bwd(q[0].now(), q[1].now(), q[2].now(), &L, xr.ptr, xr.ld, dr.ptr, dr.ld, dr.M, &S, need_dx ? out[0].data_ptr() : nullptr, H, &G,
                          ws.get(), ws.bytes, stream_of(x)));
         for (int p = 0; p < 3; ++p) {
             out[1 + 2 * p] = cast_to(out[1 + 2 * p], A[p].scalar_type());
@@ -423,7 +456,7 @@ struct QLoRAMoeBackward : public Node {
     variable_list apply(variable_list&& grads) override {
         std::lock_guard<std::mutex> lock(mutex_);
         variable_list out(8);                      // x, routing weights, then the factors as above
-        if (!grads[0].defined()) return out;
+        if (!grads[0].defined()) grads[0] = input_metadata(0).zeros_like();
         const Tensor x = x_.unpack();
         Tensor kept[kGroupedKept], A[3], B[3];
         for (int i = 0; i < kGroupedKept; ++i) kept[i] = kept_[i].unpack(shared_from_this());
@@ -448,7 +481,7 @@ struct QLoRAMoeBackward : public Node {
         xq_grouped_saved S;
         grouped_saved(&S, kept, &xr);
         Scratch ws(xq_grouped_workspace_bytes(T, (int32_t)topk, (int32_t)E, H, I, r, 1));
-        check(xq_grouped_bwd(&q[0].w, &q[1].w, &q[2].w, &L, dr.ptr, dr.ld, T, (int32_t)topk, &S, need_dx ? out[0].data_ptr() : nullptr, H,
+        check(xq_grouped_bwd(q[0].now(), q[1].now(), q[2].now(), &L, dr.ptr, dr.ld, T, (int32_t)topk, &S, need_dx ? out[0].data_ptr() : nullptr, H,
                              need_drw ? out[1].data_ptr() : nullptr, kernel_dt == at::kBFloat16 ? XQ_DT_BF16 : XQ_DT_F32, &G, ws.get(),
                              ws.bytes, stream_of(x)));
         if (need_drw) out[1] = cast_to(out[1], rw_dt);
@@ -488,7 +521,7 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
         if (n != 2) { PyErr_SetString(PyExc_TypeError, "linear(module, x)"); return nullptr; }
         const Tensor* x = plain(args[1]);
         Linear m;
-        if (!x || !m.read(args[0]) || !usable_input(x, m)) XQ_NONE;
+        if (under_transform() || !x || !m.read(args[0]) || !usable_input(x, m)) XQ_NONE;
         const int64_t Nf = m.q.w.rows, K = m.q.w.cols;
         const bool train = at::GradMode::is_enabled() && (x->requires_grad() || m.wants_grad());
         if (train && Nf % 64 != 0) XQ_NONE;
@@ -497,8 +530,11 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
         Tensor y = empty_bf(with_last(*x, Nf)), su;
         if (train) su = empty_bf({xr.M, r_pad_of(m.r)});
         Scratch ws(xq_linear_workspace_bytes(xr.M, Nf, K, m.r));
-        check(xq_linear_fwd(&m.q.w, xr.ptr, xr.ld, xr.M, m.A.data_ptr(), m.B.data_ptr(), m.lora_dtype(), m.r, (float)m.scaling, m.bias_ptr(),
-                            y.data_ptr(), Nf, train ? su.data_ptr() : nullptr, ws.get(), ws.bytes, stream_of(*x)));
+        {
+            ReleaseGil nogil;
+            check(xq_linear_fwd(&m.q.w, xr.ptr, xr.ld, xr.M, m.A.data_ptr(), m.B.data_ptr(), m.lora_dtype(), m.r, (float)m.scaling, m.bias_ptr(),
+                  y.data_ptr(), Nf, train ? su.data_ptr() : nullptr, ws.get(), ws.bytes, stream_of(*x)));
+        }
         if (!train) {
             if (!note_decode_forward(*x, xr.M)) return nullptr;
             return THPVariable_Wrap(std::move(y));
@@ -525,7 +561,7 @@ PyObject* linears(PyObject*, PyObject* const* args, Py_ssize_t n) {
         if (n != 2 || !PyList_Check(args[0])) { PyErr_SetString(PyExc_TypeError, "linears([modules], x)"); return nullptr; }
         const Py_ssize_t cnt = PyList_GET_SIZE(args[0]);
         const Tensor* x = plain(args[1]);
-        if (!x || cnt < 2 || cnt > XQ_LINEAR_MULTI_MAX) XQ_NONE;
+        if (under_transform() || !x || cnt < 2 || cnt > XQ_LINEAR_MULTI_MAX) XQ_NONE;
         const bool grad = at::GradMode::is_enabled();
         if (grad && x->requires_grad()) XQ_NONE;
         Linear m[XQ_LINEAR_MULTI_MAX];
@@ -543,7 +579,10 @@ PyObject* linears(PyObject*, PyObject* const* args, Py_ssize_t n) {
                                     y[i].data_ptr(), m[i].q.w.rows};
         }
         Scratch ws(xq_linear_fwd_multi_workspace_bytes(jobs, (int)cnt, xr.M));
-        check(xq_linear_fwd_multi(jobs, (int)cnt, xr.ptr, xr.ld, xr.M, m[0].lora_dtype(), ws.get(), ws.bytes, stream_of(*x)));
+        {
+            ReleaseGil nogil;
+            check(xq_linear_fwd_multi(jobs, (int)cnt, xr.ptr, xr.ld, xr.M, m[0].lora_dtype(), ws.get(), ws.bytes, stream_of(*x)));
+        }
         if (!note_decode_forward(*x, xr.M)) return nullptr;
         PyObject* out = PyList_New(cnt);
         if (!out) return nullptr;
@@ -557,7 +596,7 @@ PyObject* mlp(PyObject*, PyObject* const* args, Py_ssize_t n) {
     return guarded([&]() -> PyObject* {
         if (n != 4) { PyErr_SetString(PyExc_TypeError, "mlp(gate, up, down, x)"); return nullptr; }
         const Tensor* x = plain(args[3]);
-        if (!x) XQ_NONE;
+        if (under_transform() || !x) XQ_NONE;
         Linear m[3];
         for (int p = 0; p < 3; ++p)
             if (!m[p].read(args[p])) XQ_NONE;
@@ -580,7 +619,10 @@ PyObject* mlp(PyObject*, PyObject* const* args, Py_ssize_t n) {
         Tensor y = empty_bf(x->sizes());
         if (!train) {
             Scratch ws(xq_mlp_infer_workspace_bytes(M, H, I, r));
-            check(xq_mlp_fwd_infer(&m[0].q.w, &m[1].q.w, &m[2].q.w, &L, xr.ptr, xr.ld, M, y.data_ptr(), H, ws.get(), ws.bytes, stream_of(*x)));
+            {
+                ReleaseGil nogil;
+                check(xq_mlp_fwd_infer(&m[0].q.w, &m[1].q.w, &m[2].q.w, &L, xr.ptr, xr.ld, M, y.data_ptr(), H, ws.get(), ws.bytes, stream_of(*x)));
+            }
             if (!note_decode_forward(*x, M)) return nullptr;
             return THPVariable_Wrap(std::move(y));
         }
@@ -589,7 +631,10 @@ PyObject* mlp(PyObject*, PyObject* const* args, Py_ssize_t n) {
         const int gu = xq_get_mlp_gate_up_fused() && m[0].q.w.format == XQ_FMT_FP8 && m[1].q.w.format == XQ_FMT_FP8;
         xq_mlp_saved S{kept[0].data_ptr(), kept[1].data_ptr(), kept[2].data_ptr(), kept[3].data_ptr(), gu, 0};
         Scratch ws(xq_mlp_workspace_bytes(M, H, I, r, 0));
-        check(xq_mlp_fwd(&m[0].q.w, &m[1].q.w, &m[2].q.w, &L, xr.ptr, xr.ld, M, y.data_ptr(), H, &S, ws.get(), ws.bytes, stream_of(*x)));
+        {
+            ReleaseGil nogil;
+            check(xq_mlp_fwd(&m[0].q.w, &m[1].q.w, &m[2].q.w, &L, xr.ptr, xr.ld, M, y.data_ptr(), H, &S, ws.get(), ws.bytes, stream_of(*x)));
+        }
         TORCH_CHECK(S.gate_up_fused == gu, "xq_mlp_fwd ran gate and up in form ", S.gate_up_fused, ", asked for ", gu);
         auto node = std::shared_ptr<QLoRAMLPBackward>(new QLoRAMLPBackward(), torch::autograd::deleteNode);
         node->set_next_edges(torch::autograd::collect_next_edges(*x, A[0], B[0], A[1], B[1], A[2], B[2]));
@@ -615,7 +660,7 @@ PyObject* moe(PyObject*, PyObject* const* args, Py_ssize_t n) {
         if (n != 5) { PyErr_SetString(PyExc_TypeError, "moe(module, x, routing_weights, selected_experts, streaming)"); return nullptr; }
         const bool streaming = args[4] == Py_True;
         const Tensor *x = plain(args[1]), *rw = plain(args[2]), *sel = plain(args[3]);
-        if (!x || !rw || !sel || !PyObject_TypeCheck(args[0], g_experts_type)) XQ_NONE;
+        if (under_transform() || !x || !rw || !sel || !PyObject_TypeCheck(args[0], g_experts_type)) XQ_NONE;
         PyObject* d = dict_of(args[0]);
         PyObject *params = get(d, N.s__parameters), *bufs = get(d, N.s__buffers), *sdt = get(d, N.s__scale_dtypes);
         PyObject* impl = get(d, N.s_moe_implementation);
@@ -687,8 +732,11 @@ PyObject* moe(PyObject*, PyObject* const* args, Py_ssize_t n) {
         void* stream = stream_of(*x);
         if (streaming) {
             Scratch ws(xq_grouped_infer_workspace_bytes(T, (int32_t)topk, (int32_t)E, H, I, r));
-            check(xq_grouped_fwd_infer(&q[0].w, &q[1].w, &q[2].w, &L, xr.ptr, xr.ld, T, w.data_ptr(), rw_code, (const int32_t*)ids.data_ptr(),
-                                       (int32_t)topk, out.data_ptr(), H, ws.get(), ws.bytes, stream));
+            {
+                ReleaseGil nogil;
+                check(xq_grouped_fwd_infer(&q[0].w, &q[1].w, &q[2].w, &L, xr.ptr, xr.ld, T, w.data_ptr(), rw_code, (const int32_t*)ids.data_ptr(),
+                      (int32_t)topk, out.data_ptr(), H, ws.get(), ws.bytes, stream));
+            }
             return THPVariable_Wrap(std::move(out));
         }
         const int64_t R = T * topk;
@@ -700,8 +748,11 @@ PyObject* moe(PyObject*, PyObject* const* args, Py_ssize_t n) {
         xq_grouped_saved S;
         grouped_saved(&S, kept, nullptr);
         Scratch ws(xq_grouped_workspace_bytes(T, (int32_t)topk, (int32_t)E, H, I, r, 0));
-        check(xq_grouped_fwd(&q[0].w, &q[1].w, &q[2].w, &L, xr.ptr, xr.ld, T, w.data_ptr(), rw_code, (const int32_t*)ids.data_ptr(),
-                             (int32_t)topk, out.data_ptr(), H, &S, ws.get(), ws.bytes, stream));
+        {
+            ReleaseGil nogil;
+            check(xq_grouped_fwd(&q[0].w, &q[1].w, &q[2].w, &L, xr.ptr, xr.ld, T, w.data_ptr(), rw_code, (const int32_t*)ids.data_ptr(),
+                  (int32_t)topk, out.data_ptr(), H, &S, ws.get(), ws.bytes, stream));
+        }
         if (!train) return THPVariable_Wrap(std::move(out));
         auto node = std::shared_ptr<QLoRAMoeBackward>(new QLoRAMoeBackward(), torch::autograd::deleteNode);
         node->set_next_edges(torch::autograd::collect_next_edges(*x, *rw, A[0], B[0], A[1], B[1], A[2], B[2]));

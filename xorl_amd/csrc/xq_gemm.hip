@@ -3,7 +3,7 @@
 #include <algorithm>
 #include <atomic>
 #include "xq_gemm_256.h"
-#include "xq_gemm_dtl.h"
+#include "xq_gemm_dec.h"
 #include <stdlib.h>
 #include <mutex>
 #include "xq_lora.h"
@@ -162,8 +162,59 @@ static DensePlan plan_dense(int64_t n_rows, int64_t Nout, int64_t nk) {
     return p;
 }
 
+// ---- dense weights decoded once per launch (xq_gemm_dec.h).  The image costs a pass over the weight (50 M weights: 26-33 us)
+// and gives back what the tile kernels lose to their decode: a quarter to a third of a 4-bit launch's time, a tenth of a
+// block-fp8 one's (whose kernel keeps the bytes in LDS and decodes beside its MFMAs).  Forward, us, image against tile kernel:
+//   int4 [12288, 4096]: 512 rows 92 / 101, 700 115 / 128, 1357 153 / 171, 4096 323 / 403, 8192 636 / 820; [4096, 12288]: 512 114 / 94,
+//   700 114 / 143, 8192 627 / 786; [4096, 4096]: 512 55 / 45, 1024 69 / 70, 1357 80 / 96; [1024, 4096]: 2048 50 / 45, 4096 72 / 68,
+//   8192 101 / 113; block-fp8 [12288, 4096]: 1357 155 / 145, 4096 335 / 327, 8192 626 / 661; [8192, 5120]: 4096 271 / 267, 8192 518 / 545.
+// So 4-bit from 640 rows on, block-fp8 from 6144 on, and products too small to fill the chip stay with the tile kernels.
+constexpr int64_t kDecMinRows = 640, kDecMinRowsFp8 = 6144;
+constexpr double kDecMinWork = 2.0e10;               // rows x columns x contraction
+struct DecPlan {
+    int split;                // K splits of the leading rows
+    int64_t head_rows;        // leading rows; the others are a second launch in tail_split K splits
+    int tail_split;
+    int64_t partial;          // bytes of fp32 sums the splits take
+};
+static DecPlan plan_decoded(int64_t n_rows, int64_t Nout, int64_t Kc) {
+    // microseconds: a round of the chip takes 0.8 per K-step (0.78-0.84 measured) and 5 around them; the fp32 sums of splits are
+    // written and read at about 5 TB/s
+    const int64_t tc = xq_cdiv(Nout, GeoDec::T), steps = Kc / GeoDec::BK, cus = num_cus();
+    auto cost = [&](int64_t rows, int s) {
+        const double rounds = (double)xq_cdiv(xq_cdiv(rows, GeoDec::T) * tc * s, cus);
+        const double sums = s > 1 ? 3.0 + (8.0 * s + 2.0) * (double)rows * (double)Nout / 5.0e6 : 0.0;
+        return rounds * ((double)xq_cdiv(steps, s) * 0.8 + 5.0) + sums;
+    };
+    auto best = [&](int64_t rows, double* c) {
+        int b = 1;
+        *c = cost(rows, 1);
+        for (int s = 2; s <= 8 && steps / s >= 16; ++s)
+            if (cost(rows, s) < *c) { b = s; *c = cost(rows, s); }
+        return b;
+    };
+    double whole;
+    DecPlan p{best(n_rows, &whole), n_rows, 1, 0};
+    const int64_t tr = xq_cdiv(n_rows, GeoDec::T), keep = tr * tc / cus * cus / tc;      // tile rows of whole rounds
+    if (keep > 0 && keep < tr) {
+        double tail;
+        const int ts = best(n_rows - keep * GeoDec::T, &tail);
+        if (cost(keep * GeoDec::T, 1) + tail < whole) p = DecPlan{1, keep * GeoDec::T, ts, 0};
+    }
+    const int64_t tail_rows = n_rows - p.head_rows;
+    p.partial = std::max(p.split > 1 ? p.split * p.head_rows : 0, tail_rows && p.tail_split > 1 ? p.tail_split * tail_rows : 0) * Nout * 4;
+    return p;
+}
+static bool decode_first(int fmt, int64_t n_rows, int64_t Nout, int64_t Kc) {
+    return n_rows >= (fmt == XQ_FMT_FP8 ? kDecMinRowsFp8 : kDecMinRows) && (double)n_rows * (double)Nout * (double)Kc >= kDecMinWork &&
+           Kc % 64 == 0 && Kc >= 128 && Nout % 16 == 0;
+}
+static int64_t decoded_scratch_bytes(int64_t n_rows, int64_t Nout, int64_t Kc) {      // (whatever the format: its callers know only sizes)
+    return decode_first(XQ_FMT_INT4, n_rows, Nout, Kc) ? dec_image_bytes(Nout, Kc) + plan_decoded(n_rows, Nout, Kc).partial : 0;
+}
+
 // fp32 partial-sum bytes the split-K forms of a dense [n_rows, Nout] product over Kc may want, under any tile policy
-int64_t tile_gemm_partial_bytes(int64_t n_rows, int64_t Nout, int64_t Kc) {
+int64_t tile_gemm_split_bytes(int64_t n_rows, int64_t Nout, int64_t Kc) {
     if (n_rows <= 0 || Kc % BK) return 0;
     const int64_t nk = Kc / BK;
     int64_t elems = 0;
@@ -177,6 +228,13 @@ int64_t tile_gemm_partial_bytes(int64_t n_rows, int64_t Nout, int64_t Kc) {
     return elems * Nout * 4;
 }
 
+// scratch a dense launch may want: the above, or the decoded image of a 4-bit weight with the sums of its splits (without
+// room for those the launch decodes in the tile kernel)
+int64_t tile_gemm_partial_bytes(int64_t n_rows, int64_t Nout, int64_t Kc) {
+    if (n_rows <= 0 || Kc % BK) return 0;
+    return std::max(tile_gemm_split_bytes(n_rows, Nout, Kc), decoded_scratch_bytes(n_rows, Nout, Kc));
+}
+
 // Whether a grouped launch on this bank may take a second bank of the same shape (see G256Args::W2): block-fp8 on the
 // pipelined kernel, whole 256-column tiles per bank (which also keeps the K-step where the dgrad changes banks on a
 // scale-block boundary and away from the pipeline's prologue).
@@ -188,6 +246,64 @@ bool two_banks_supported(const xq_weight* w) {
 // the pipelined kernel, the change of matrix on a scale-block boundary and past the pipeline's prologue.
 bool two_dense_supported(const xq_weight* w) {
     return w->format == XQ_FMT_FP8 && g_tile_policy != 1 && w->num_experts == 1 && w->rows % 128 == 0 && w->rows >= 512;
+}
+
+// The launches of a dense weight decoded once: `f` is filled for the whole problem (f.W2: a second matrix that continues the
+// contraction), weights FLAT; `scratch` holds decoded_scratch_bytes().
+static int launch_decoded(G256Args f, bool cc, int fmt, uint8_t* scratch, hipStream_t stream, const char* who) {
+    static std::atomic<bool> attr_set{false};
+    if (!attr_set) {
+        int rc = raise_lds_limit(gemm_dec_kernel<false>, GeoDec::lds_bytes(), who);
+        if (!rc) rc = raise_lds_limit(gemm_dec_kernel<true>, GeoDec::lds_bytes(), who);
+        if (rc) return rc;
+        attr_set = true;
+    }
+    const DecPlan plan = plan_decoded(f.M, f.Nout, f.Kc);
+    bf16_t* image = (bf16_t*)scratch;
+    f.partial = (float*)(scratch + dec_image_bytes(f.Nout, f.Kc));
+    const int mats = f.W2 ? 2 : 1;
+    DecImageArgs im{f.W, f.scales, f.global_scale, f.wrows, f.wcols, f.gshift, f.scale_dtype, f.Kc / mats, f.Nout, image, f.Kc / GeoDec::BK, 0};
+    const unsigned tiles_n = (unsigned)xq_cdiv(f.Nout, GeoDec::T);
+    const bool timed = xq_profile_mark_begin(stream, 2.0 * (double)f.M * f.Nout * ((double)f.Kc + f.r_pad));
+    auto decode = [&](auto FMT_) {
+        constexpr int FMT = decltype(FMT_)::value;
+        if (cc) dec_image_kernel<FMT><<<dim3((unsigned)xq_cdiv(im.Kc, 256), tiles_n * 8), 256, 0, stream>>>(im);
+        else dec_image_t_kernel<FMT><<<dim3((unsigned)(im.Kc / 64), tiles_n), 256, 0, stream>>>(im);
+    };
+    for (int m = 0; m < mats; ++m) {
+        if (m) { im.packed = f.W2; im.scales = f.scales2; im.kt0 = im.Kc / GeoDec::BK; }
+        if (fmt == XQ_FMT_FP8) decode(std::integral_constant<int, XQ_FMT_FP8>{});
+        else if (fmt == XQ_FMT_INT4) decode(std::integral_constant<int, XQ_FMT_INT4>{});
+        else if (fmt == XQ_FMT_NF4) decode(std::integral_constant<int, XQ_FMT_NF4>{});
+        else decode(std::integral_constant<int, XQ_FMT_NVFP4>{});
+        XQ_CHECK_LAUNCH(who);
+    }
+    f.W = (const uint8_t*)image;
+    f.tiles_n = (int32_t)tiles_n;
+    const bf16_t *A = f.A, *su = f.su;
+    bf16_t* C = f.C;
+    const int64_t rows = f.M;
+    for (int64_t r0 = 0; r0 < rows; r0 += plan.head_rows) {
+        const bool head = r0 == 0;
+        f.M = head ? plan.head_rows : rows - r0;
+        f.A = A + r0 * f.lda;
+        f.su = su ? su + r0 * f.ld_su : nullptr;
+        f.C = C + r0 * f.ldc;
+        f.tiles_m = (int32_t)xq_cdiv(f.M, GeoDec::T);
+        f.ksplit = head ? plan.split : plan.tail_split;
+        const dim3 grid((unsigned)(f.tiles_m * f.tiles_n), (unsigned)f.ksplit);
+        if (f.ksplit > 1) {
+            gemm_dec_kernel<true><<<grid, GeoDec::NT, GeoDec::lds_bytes(), stream>>>(f);
+            XQ_CHECK_LAUNCH(who);
+            splitk_reduce_kernel<<<(unsigned)xq_cdiv(f.M * (f.Nout >> 2), 256), 256, 0, stream>>>(f.partial, f.ksplit, f.M, f.Nout, f.C, f.ldc);
+        } else {
+            gemm_dec_kernel<false><<<grid, GeoDec::NT, GeoDec::lds_bytes(), stream>>>(f);
+        }
+        XQ_CHECK_LAUNCH(who);
+        if (!head) break;
+    }
+    if (timed) xq_profile_mark_end(stream);
+    return XQ_OK;
 }
 
 // C[rows, Nout] = A . op(deq(W)) (+ su . Lr^T) (+ bias); see xq_gemm_tile.h.  force_T = 256 / 128 fixes the tile
@@ -260,6 +376,20 @@ static int launch_tile_gemm_t(const xq_weight* w, bool contract_cols, const bf16
         const DensePlan plan = plan_dense(n_rows, g.Nout, g.Kc / BK);
         const bool planned = !grouped && fmt_ok && g_tile_policy == 0 && force_T == 0 && !two_dense;   // two matrices: one unsplit launch
         const int T = force_T ? force_T : g_tile_policy == 2 ? 256 : g_tile_policy == 3 ? 128 : grouped ? (big ? 256 : 128) : plan.T;
+        if ((planned || (two_dense && g_tile_policy == 0)) && (w->format != XQ_FMT_FP8 || g_fp8_direct) &&
+            decode_first(w->format, n_rows, g.Nout, g.Kc) && partial && xq_aligned(partial, 16) &&
+            partial_bytes >= decoded_scratch_bytes(n_rows, g.Nout, g.Kc) && n_rows * lda * 2 < (1ll << 32) && xq_cdiv(n_rows, 256) * xq_cdiv(g.Nout, 256) < (1ll << 31) && g.Nout < 65536 * 16) {
+            G256Args f{};
+            f.A = A; f.lda = lda; f.C = C; f.ldc = ldc;
+            f.W = g.packed; f.scales = g.scales; f.global_scale = g.global_scale;
+            f.wrows = g.wrows; f.wcols = g.wcols; f.gshift = gshift; f.scale_dtype = g.scale_dtype;
+            f.Kc = g.Kc; f.Nout = g.Nout; f.M = n_rows; f.num_experts = 1;
+            if (two) { f.W2 = (const uint8_t*)two->w2->packed; f.scales2 = (const uint8_t*)two->w2->scales; }
+            f.su = g.r_pad ? su : nullptr; f.right = g.right; f.r_pad = g.r_pad; f.ld_su = g.r_pad;
+            f.bias = bias;
+            f.wide_rows = xq_aligned(C, 16) && ldc % 8 == 0 && xq_aligned(bias, 8);
+            return launch_decoded(f, contract_cols, w->format, (uint8_t*)partial, stream, who);
+        }
         if (planned && plan.head_rows < n_rows) {
             const int64_t head = plan.head_rows;
             const int rc = launch_tile_gemm_t(w, contract_cols, A, lda, head, nullptr, nullptr, su, lora_right, r_pad,
@@ -469,12 +599,14 @@ extern "C" int xq_set_persistent_tiles(int enabled) {
     return XQ_OK;
 }
 
-extern "C" int64_t xq_linear_workspace_bytes(int64_t M, int64_t N, int64_t K, int r) {
+// what a call must bring (`part` = tile_gemm_split_bytes) and what it is told to bring (tile_gemm_partial_bytes: with room for
+// the decoded image of a 4-bit weight under many rows)
+static int64_t linear_workspace(int64_t M, int64_t N, int64_t K, int r, int64_t (*part)(int64_t, int64_t, int64_t)) {
     int rp = r_pad_of(r);
     int64_t skinny = M <= 64 ? skinny_workspace_bytes(M, N, K, rp) : 0;
-    // split-K partial sums of the forward (output N, contraction K) and of the dgrad (output K, contraction N)
-    const int64_t pf = align256(tile_gemm_partial_bytes(M, N, K));
-    const int64_t pb = align256(tile_gemm_partial_bytes(M, K, N));
+    // scratch of the forward (output N, contraction K) and of the dgrad (output K, contraction N)
+    const int64_t pf = align256(part(M, N, K));
+    const int64_t pb = align256(part(M, K, N));
     int64_t need = (pf > pb ? pf : pb) + 256;
     if (rp) {
         const int64_t panel = lowrank_panel_bytes(1, M, rp, K);
@@ -485,6 +617,8 @@ extern "C" int64_t xq_linear_workspace_bytes(int64_t M, int64_t N, int64_t K, in
     }
     return need > skinny ? need : skinny;
 }
+static int64_t linear_workspace_needed(int64_t M, int64_t N, int64_t K, int r) { return linear_workspace(M, N, K, r, tile_gemm_split_bytes); }
+extern "C" int64_t xq_linear_workspace_bytes(int64_t M, int64_t N, int64_t K, int r) { return linear_workspace(M, N, K, r, tile_gemm_partial_bytes); }
 
 static int check_dense(const xq_weight* w, const char* who) {
     int rc = xq_validate_weight(w, who);
@@ -516,7 +650,7 @@ extern "C" int xq_linear_fwd(const xq_weight* w, const void* x, int64_t ldx, int
     const LowRankRight right{{lora_B, nullptr}, r, r, rp, lora_dtype == XQ_DT_F32, 0};
     Carver cv{(workspace && xq_aligned(workspace, 256)) ? (uint8_t*)workspace : nullptr, 0, workspace_bytes};
     if (rp) {
-        XQ_REQUIRE(workspace && xq_aligned(workspace, 256) && workspace_bytes >= xq_linear_workspace_bytes(M, N, K, r),
+        XQ_REQUIRE(workspace && xq_aligned(workspace, 256) && workspace_bytes >= linear_workspace_needed(M, N, K, r),
                    "xq_linear_fwd: workspace missing, misaligned or smaller than xq_linear_workspace_bytes()");
         su = su_out ? (bf16_t*)su_out : (bf16_t*)cv.take(M * rp * 2);
         bf16_t* panel = (bf16_t*)cv.take(lowrank_panel_bytes(1, M, rp, K));
@@ -705,7 +839,7 @@ extern "C" int xq_linear_fwd_static(const xq_weight* w, const void* x, int64_t l
     if (rc) return rc;
     XQ_REQUIRE(M >= 0, "xq_linear_fwd_static: negative row count");
     XQ_REQUIRE(r >= 0 && r <= 64, "xq_linear_fwd_static: LoRA rank %d out of range [0, 64]", r);
-    const int64_t need = xq_linear_workspace_bytes(M, w->rows, w->cols, r);
+    const int64_t need = linear_workspace_needed(M, w->rows, w->cols, r);
     XQ_REQUIRE(need <= XQ_STATIC_SCRATCH_BYTES,
                "xq_linear_fwd_static: M=%lld, N=%lld, K=%lld, r=%d needs %lld bytes of scratch, the built-in buffer "
                "holds %lld; use xq_linear_fwd with a caller workspace",
@@ -745,7 +879,7 @@ extern "C" int xq_linear_bwd(const xq_weight* w, const void* x, int64_t ldx, con
     float* partial = nullptr;
     Carver cv{(workspace && xq_aligned(workspace, 256)) ? (uint8_t*)workspace : nullptr, 0, workspace_bytes};
     if (rp) {
-        XQ_REQUIRE(workspace && xq_aligned(workspace, 256) && workspace_bytes >= xq_linear_workspace_bytes(M, N, K, r),
+        XQ_REQUIRE(workspace && xq_aligned(workspace, 256) && workspace_bytes >= linear_workspace_needed(M, N, K, r),
                    "xq_linear_bwd: workspace missing, misaligned or smaller than xq_linear_workspace_bytes()");
         v = (bf16_t*)cv.take(M * rp * 2);
         bf16_t* su_ws = (bf16_t*)cv.take(M * rp * 2);

@@ -64,6 +64,104 @@ __device__ __forceinline__ u32x2 dtl_decode4(uint32_t w, float sc) {
     return u32x2{pack_bf16x2(x0[0] * sc, x0[1] * sc), pack_bf16x2(x1[0] * sc, x1[1] * sc)};
 }
 
+// The end of a 256 x 256 tile of the kernels whose waves hold TM x TN tiles of 16 x 16 sums (gemm_dtl16_kernel,
+// gemm_dec_kernel).  `dsm` is the block's LDS, read by nobody else behind the barrier here; `second` bytes into it lies room
+// for a second 32 KB tile.  First the low-rank side term:
+template <int TM, int TN, int NW, bool GROUPED>
+__device__ __forceinline__ void dtl16_side_term(const G256Args& g, unsigned char* dsm, int second, f32x4 (&acc)[TM][TN], int64_t row0,
+                                                int64_t row_end, int n0w, int bank_width, const bf16_t* su_b, const bf16_t* lr_b, int e) {
+    constexpr int T = 256, NT = NW * 64, RW = TM * 16;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = NW == 8 ? wave >> 2 : 0, wn = wave & 3;
+    const int l16 = lane & 15, lg = lane >> 4;
+    // ---- low-rank side term: su[rows, rp] x lora_right[n, rp] as bf16 [row][64 k] tiles in the first two stages, k beyond
+    // rp zero up to the next multiple of 32
+    bf16_t* As = (bf16_t*)dsm;
+    bf16_t* Bs = (bf16_t*)(dsm + second);
+    __syncthreads();
+    if (g.r_pad > 0) {
+        const int rp = g.r_pad, steps = (rp + 31) >> 5, cpr = steps << 2, have = rp >> 3;
+        const bf16_t* lr = lr_b + (int64_t)e * bank_width * rp;
+        for (int idx = tid; idx < T * cpr; idx += NT) {
+            const int r = idx / cpr, c = idx - r * cpr;
+            int64_t row = row0 + r;
+            row = row < row_end ? row : row_end - 1;
+            int n = n0w + r;
+            n = n < bank_width ? n : bank_width - 1;
+            const u32x4 z = {0, 0, 0, 0};
+            *(u32x4*)(As + swz(r, c)) = c < have ? *(const u32x4*)(su_b + row * g.ld_su + c * 8) : z;
+            if constexpr (GROUPED) *(u32x4*)(Bs + swz(r, c)) = c < have ? *(const u32x4*)(lr + (int64_t)n * rp + c * 8) : z;
+            else *(u32x4*)(Bs + swz(r, c)) = c < have ? right_chunk(g.right, -1, n, c) : z;
+        }
+        __syncthreads();
+        for (int ks = 0; ks < steps; ++ks) {
+            bf16x8 bw[TN];
+#pragma unroll
+            for (int j = 0; j < TN; ++j) bw[j] = *(const bf16x8*)(Bs + swz(wn * 64 + j * 16 + l16, ks * 4 + lg));
+#pragma unroll
+            for (int i = 0; i < TM; ++i) {
+                const bf16x8 ax = *(const bf16x8*)(As + swz(wm * RW + i * 16 + l16, ks * 4 + lg));
+#pragma unroll
+                for (int j = 0; j < TN; ++j) {
+                    if constexpr (NW == 4) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(bw[j]), "v"(ax));
+                    else acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bw[j], ax, acc[i][j], 0, 0, 0);
+                }
+            }
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    }
+}
+
+// ... and the whole end: side term, bias, the way out as bf16
+template <int TM, int TN, int NW, bool GROUPED>
+__device__ __forceinline__ void dtl16_finish(const G256Args& g, unsigned char* dsm, int second, f32x4 (&acc)[TM][TN], int64_t row0,
+                                             int64_t row_end, int n0, int n0w, int bank_width, const bf16_t* su_b, const bf16_t* lr_b, int e) {
+    constexpr int RW = TM * 16;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wm = NW == 8 ? wave >> 2 : 0, wn = wave & 3;
+    dtl16_side_term<TM, TN, NW, GROUPED>(g, dsm, second, acc, row0, row_end, n0w, bank_width, su_b, lr_b, e);
+
+    // ---- the finished tile.  Lane l holds, per (i, j) tile, row 16 i + l % 16 and the 4 columns 16 j + 4 (l / 16) ..: 8 bytes
+    // of bf16.  Each wave passes its RW x 64 sub-tile through a private LDS area ([row][64] bf16, chunk swizzle) and writes
+    // whole 128-byte row pieces, 8 rows per instruction.
+    if constexpr (NW == 4) asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");     // the last MFMA results, written outside the compiler's hazard tracking
+    bf16_t* stg = (bf16_t*)dsm + wave * (RW * 64);
+    int lv = lane;
+    asm volatile("" : "+v"(lv));
+    const int s16 = lv & 15, sg = lv >> 4;
+    const bool wide = g.wide_rows != 0;
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+        float b4[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (g.bias) {
+            const u32x2 b = *(const u32x2*)(g.bias + min(n0 + wn * 64 + j * 16 + 4 * sg, g.Nout - 4));
+            b4[0] = __uint_as_float(b[0] << 16); b4[1] = __uint_as_float(b[0] & 0xffff0000u);
+            b4[2] = __uint_as_float(b[1] << 16); b4[3] = __uint_as_float(b[1] & 0xffff0000u);
+        }
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+            const u32x2 v = {pack_bf16x2(acc[i][j][0] + b4[0], acc[i][j][1] + b4[1]), pack_bf16x2(acc[i][j][2] + b4[2], acc[i][j][3] + b4[3])};
+            if (wide) {
+                *(u32x2*)(stg + swz(i * 16 + s16, 2 * j + (sg >> 1)) + 4 * (sg & 1)) = v;
+            } else {
+                const int64_t row = row0 + wm * RW + i * 16 + s16;
+                const int n = n0 + wn * 64 + j * 16 + 4 * sg;
+                if (row < row_end && n < g.Nout) *(u32x2*)(g.C + row * g.ldc + n) = v;
+            }
+        }
+    }
+    if (wide) {
+#pragma unroll
+        for (int t = 0; t < RW / 8; ++t) {
+            const int rl = t * 8 + (lv >> 3), ch = lv & 7;
+            const u32x4 v = *(const u32x4*)(stg + swz(rl, ch));
+            const int64_t row = row0 + wm * RW + rl;
+            const int n = n0 + wn * 64 + ch * 8;
+            if (row < row_end && n < g.Nout) *(u32x4*)(g.C + row * g.ldc + n) = v;
+        }
+    }
+}
+
 // NW = 8: eight waves as 2 x 4, a wave 128 x 64 (two waves per SIMD).  NW = 4: four waves side by side, a wave 256 x 64
 // with its 256 accumulator registers (one wave per SIMD): every weight value is then decoded by exactly one wave -- half
 // the conversions per MFMA of the eight-wave form, whose column blocks are shared by two waves -- and an activation
@@ -403,82 +501,7 @@ __global__ void __launch_bounds__(NW * 64, NW == 8 ? 2 : 1) gemm_dtl16_kernel(G2
 #undef XQ_DTL_READ_A
 #undef XQ_DTL_READ_W
 
-    // ---- low-rank side term: su[rows, rp] x lora_right[n, rp] as bf16 [row][64 k] tiles in the first two stages, k beyond
-    // rp zero up to the next multiple of 32
-    bf16_t* As = (bf16_t*)dsm;
-    bf16_t* Bs = (bf16_t*)(dsm + D::STAGE_BYTES);
-    __syncthreads();
-    if (g.r_pad > 0) {
-        const int rp = g.r_pad, steps = (rp + 31) >> 5, cpr = steps << 2, have = rp >> 3;
-        const bf16_t* lr = lr_b + (int64_t)e * bank_width * rp;
-        for (int idx = tid; idx < T * cpr; idx += NT) {
-            const int r = idx / cpr, c = idx - r * cpr;
-            int64_t row = row0 + r;
-            row = row < row_end ? row : row_end - 1;
-            int n = n0w + r;
-            n = n < bank_width ? n : bank_width - 1;
-            const u32x4 z = {0, 0, 0, 0};
-            *(u32x4*)(As + swz(r, c)) = c < have ? *(const u32x4*)(su_b + row * g.ld_su + c * 8) : z;
-            if constexpr (GROUPED) *(u32x4*)(Bs + swz(r, c)) = c < have ? *(const u32x4*)(lr + (int64_t)n * rp + c * 8) : z;
-            else *(u32x4*)(Bs + swz(r, c)) = c < have ? right_chunk(g.right, -1, n, c) : z;
-        }
-        __syncthreads();
-        for (int ks = 0; ks < steps; ++ks) {
-            bf16x8 bw[TN];
-#pragma unroll
-            for (int j = 0; j < TN; ++j) bw[j] = *(const bf16x8*)(Bs + swz(wn * 64 + j * 16 + l16, ks * 4 + lg));
-#pragma unroll
-            for (int i = 0; i < TM; ++i) {
-                const bf16x8 ax = *(const bf16x8*)(As + swz(wm * RW + i * 16 + l16, ks * 4 + lg));
-#pragma unroll
-                for (int j = 0; j < TN; ++j) {
-                    if constexpr (NW == 4) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(bw[j]), "v"(ax));
-                    else acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bw[j], ax, acc[i][j], 0, 0, 0);
-                }
-            }
-        }
-        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    }
-
-    // ---- the finished tile.  Lane l holds, per (i, j) tile, row 16 i + l % 16 and the 4 columns 16 j + 4 (l / 16) ..: 8 bytes
-    // of bf16.  Each wave passes its RW x 64 sub-tile through a private LDS area ([row][64] bf16, chunk swizzle) and writes
-    // whole 128-byte row pieces, 8 rows per instruction.
-    if constexpr (NW == 4) asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");     // the last MFMA results, written outside the compiler's hazard tracking
-    bf16_t* stg = (bf16_t*)dsm + wave * (RW * 64);
-    int lv = lane;
-    asm volatile("" : "+v"(lv));
-    const int s16 = lv & 15, sg = lv >> 4;
-    const bool wide = g.wide_rows != 0;
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-        float b4[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-        if (g.bias) {
-            const u32x2 b = *(const u32x2*)(g.bias + min(n0 + wn * 64 + j * 16 + 4 * sg, g.Nout - 4));
-            b4[0] = __uint_as_float(b[0] << 16); b4[1] = __uint_as_float(b[0] & 0xffff0000u);
-            b4[2] = __uint_as_float(b[1] << 16); b4[3] = __uint_as_float(b[1] & 0xffff0000u);
-        }
-#pragma unroll
-        for (int i = 0; i < TM; ++i) {
-            const u32x2 v = {pack_bf16x2(acc[i][j][0] + b4[0], acc[i][j][1] + b4[1]), pack_bf16x2(acc[i][j][2] + b4[2], acc[i][j][3] + b4[3])};
-            if (wide) {
-                *(u32x2*)(stg + swz(i * 16 + s16, 2 * j + (sg >> 1)) + 4 * (sg & 1)) = v;
-            } else {
-                const int64_t row = row0 + wm * RW + i * 16 + s16;
-                const int n = n0 + wn * 64 + j * 16 + 4 * sg;
-                if (row < row_end && n < g.Nout) *(u32x2*)(g.C + row * g.ldc + n) = v;
-            }
-        }
-    }
-    if (wide) {
-#pragma unroll
-        for (int t = 0; t < RW / 8; ++t) {
-            const int rl = t * 8 + (lv >> 3), ch = lv & 7;
-            const u32x4 v = *(const u32x4*)(stg + swz(rl, ch));
-            const int64_t row = row0 + wm * RW + rl;
-            const int n = n0 + wn * 64 + ch * 8;
-            if (row < row_end && n < g.Nout) *(u32x4*)(g.C + row * g.ldc + n) = v;
-        }
-    }
+    dtl16_finish<TM, TN, NW, GROUPED>(g, dsm, D::STAGE_BYTES, acc, row0, row_end, n0, n0w, bank_width, su_b, lr_b, e);
 }
 
 }  // namespace xq

@@ -101,10 +101,14 @@ int check_call(const xq_weight* gate, const xq_weight* up, const xq_weight* down
 }
 
 // one region of split-K partial sums and fp32 sums of the SwiGLU passes (stream order)
-int64_t gemm_part_bytes(const Dims& d) {
-    const int64_t pa = tile_gemm_partial_bytes(d.M, d.I, d.H), pb = tile_gemm_partial_bytes(d.M, d.H, d.I);
+// (`needed`: what a call must bring; without it what it is told to bring, room for decoded 4-bit weights included)
+int64_t gemm_part_bytes(const Dims& d, bool needed) {
+    auto part = needed ? tile_gemm_split_bytes : tile_gemm_partial_bytes;
+    const int64_t pa = part(d.M, d.I, d.H), pb = part(d.M, d.H, d.I);
     const int64_t ps = d.rp && silu_bwd_nt_supported(d.I, d.rp) ? silu_nt_partial_bytes(d.M, d.I, d.rp) : 0;
-    return std::max(std::max(pa, pb), ps);
+    // (the dgrad of gate and up as one sum: the contraction is twice as long)
+    const int64_t p2 = needed ? 0 : tile_gemm_partial_bytes(d.M, d.H, 2 * d.I);
+    return std::max(std::max(pa, pb), std::max(ps, p2));
 }
 
 // From a block of 32 rows per compute unit on, the forward lays the A factors out as bf16 panels once and forms s * h . A_d^T in
@@ -118,15 +122,15 @@ int64_t fwd_panel_bytes(const Dims& d) {
     return std::max(gu, lowrank_panel_bytes(1, d.M, d.rp, d.I));
 }
 
-int64_t fwd_workspace(const Dims& d) { return fwd_panel_bytes(d) + al256(gemm_part_bytes(d)) + 512; }
+int64_t fwd_workspace(const Dims& d, bool needed) { return fwd_panel_bytes(d) + al256(gemm_part_bytes(d, needed)) + 512; }
 
-int64_t bwd_workspace(const Dims& d) {
+int64_t bwd_workspace(const Dims& d, bool needed) {
     const int64_t rp = d.rp ? d.rp : 16;
     // the six factor gradients share a launch: partial sums of all of them (dA of gate and up of twice the rank, or apart)
     const int64_t tn = 3 * tn_partial_bytes(d.M, d.I, rp) + tn_partial_bytes(d.M, d.H, rp) +
                        std::max(2 * tn_partial_bytes(d.M, d.H, rp), 2 * rp <= 64 ? tn_partial_bytes(d.M, d.H, 2 * rp) : 0);
     return al256(d.M * d.I * 2) + al256(d.M * 2 * d.I * 2) + al256(d.M * d.H * 2) + al256(d.M * rp * 2) +
-           al256(d.M * 2 * rp * 2) + 2 * al256(rp * d.I * 2) + al256(std::max(gemm_part_bytes(d), tn)) + 512;
+           al256(d.M * 2 * rp * 2) + 2 * al256(rp * d.I * 2) + al256(std::max(gemm_part_bytes(d, needed), tn)) + 512;
 }
 
 }  // namespace
@@ -144,7 +148,7 @@ extern "C" int xq_get_mlp_gate_up_fused(void) { return g_mlp_gu.load() != 0; }
 extern "C" int64_t xq_mlp_workspace_bytes(int64_t M, int64_t hidden, int64_t intermediate, int r, int backward) {
     if (M < 0 || r < 0) return 0;
     Dims d{M, hidden, intermediate, r, r_pad_of(r)};
-    return backward ? bwd_workspace(d) : fwd_workspace(d);
+    return backward ? bwd_workspace(d, false) : fwd_workspace(d, false);
 }
 
 extern "C" int xq_mlp_fwd(const xq_weight* gate, const xq_weight* up, const xq_weight* down, const xq_mlp_lora* lora,
@@ -158,7 +162,7 @@ extern "C" int xq_mlp_fwd(const xq_weight* gate, const xq_weight* up, const xq_w
     saved->gate_up_fused = fused ? 1 : 0;       // what the backward must be told
     if (M == 0) return XQ_OK;
     XQ_REQUIRE(x_ && y, "%s: NULL activation pointer", who);
-    XQ_REQUIRE(workspace && xq_aligned(workspace, 256) && workspace_bytes >= fwd_workspace(d),
+    XQ_REQUIRE(workspace && xq_aligned(workspace, 256) && workspace_bytes >= fwd_workspace(d, true),
                "%s: workspace missing, misaligned or smaller than xq_mlp_workspace_bytes()", who);
     XQ_REQUIRE(ldy % 8 == 0 && xq_aligned(y, 16), "%s: y rows must be 16-byte aligned", who);
     hipStream_t stream = (hipStream_t)stream_;
@@ -235,12 +239,15 @@ static int64_t infer_linear_ws(int64_t M, int64_t H, int64_t I, int r) {
     return al256((a > b ? a : b) > 2048 ? (a > b ? a : b) : 2048);
 }
 
-extern "C" int64_t xq_mlp_infer_workspace_bytes(int64_t M, int64_t hidden, int64_t intermediate, int r) {
+static int64_t infer_workspace(int64_t M, int64_t hidden, int64_t intermediate, int r, bool needed) {
     if (M < 0 || r < 0) return 0;
     const int64_t act = al256(M * 2 * intermediate * 2) + al256(M * intermediate * 2);
-    const int64_t program = al256(M * 2 * r_pad_of(r) * 2) + al256(M * r_pad_of(r) * 2) + fwd_workspace(Dims{M, hidden, intermediate, r, r_pad_of(r)});
+    const int64_t program = al256(M * 2 * r_pad_of(r) * 2) + al256(M * r_pad_of(r) * 2) + fwd_workspace(Dims{M, hidden, intermediate, r, r_pad_of(r)}, needed);
     const int64_t apart = M <= 64 ? infer_linear_ws(M, hidden, intermediate, r) : 0;
     return act + (program > apart ? program : apart) + 256;
+}
+extern "C" int64_t xq_mlp_infer_workspace_bytes(int64_t M, int64_t hidden, int64_t intermediate, int r) {
+    return infer_workspace(M, hidden, intermediate, r, false);
 }
 
 extern "C" int xq_mlp_fwd_infer(const xq_weight* gate, const xq_weight* up, const xq_weight* down, const xq_mlp_lora* lora,
@@ -256,7 +263,7 @@ extern "C" int xq_mlp_fwd_infer(const xq_weight* gate, const xq_weight* up, cons
     if (rc) return rc;
     if (M == 0) return XQ_OK;
     XQ_REQUIRE(x && y, "%s: NULL activation pointer", who);
-    XQ_REQUIRE(workspace_bytes >= xq_mlp_infer_workspace_bytes(M, d.H, d.I, d.r),
+    XQ_REQUIRE(workspace_bytes >= infer_workspace(M, d.H, d.I, d.r, true),
                "%s: workspace smaller than xq_mlp_infer_workspace_bytes()", who);
     bf16_t* gu = cv.take<bf16_t>(M * 2 * d.I * 2);
     bf16_t* h = cv.take<bf16_t>(M * d.I * 2);
@@ -316,7 +323,7 @@ extern "C" int xq_mlp_bwd(const xq_weight* gate, const xq_weight* up, const xq_w
         return XQ_OK;
     }
     XQ_REQUIRE(x_ && dy_, "%s: NULL activation pointer", who);
-    XQ_REQUIRE(workspace && xq_aligned(workspace, 256) && workspace_bytes >= bwd_workspace(d),
+    XQ_REQUIRE(workspace && xq_aligned(workspace, 256) && workspace_bytes >= bwd_workspace(d, true),
                "%s: workspace missing, misaligned or smaller than xq_mlp_workspace_bytes()", who);
     XQ_REQUIRE(!dx || (lddx % 8 == 0 && xq_aligned(dx, 16)), "%s: dx rows must be 16-byte aligned", who);
     const bf16_t *x = (const bf16_t*)x_, *dy = (const bf16_t*)dy_;
@@ -400,7 +407,7 @@ extern "C" int xq_mlp_bwd(const xq_weight* gate, const xq_weight* up, const xq_w
     if (fused) {
         const TwoBanks two{up, nullptr, nullptr};
         return launch_tile_gemm(gate, false, dgu, 2 * I, M, nullptr, nullptr, rp ? v_gu : nullptr, nullptr, rp2, nullptr, (bf16_t*)dx, lddx,
-                                stream, who, nullptr, 0, &two, rp ? &right_gu : nullptr);
+                                stream, who, part, part_bytes, &two, rp ? &right_gu : nullptr);
     }
     if ((rc = launch_tile_gemm(gate, false, dgate, 2 * I, M, nullptr, nullptr, rp ? v_g : nullptr, nullptr, rp, nullptr, (bf16_t*)dx, lddx, stream, who, part, part_bytes, nullptr,
                                rp ? &right_g : nullptr))) return rc;

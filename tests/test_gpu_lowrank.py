@@ -5,6 +5,7 @@ import pytest
 import torch
 
 from oracle import recipe as R
+from tests.test_gpu_moe import test_moe_fwd_bwd_vs_oracle as check_experts
 from tests.util_cases import close, gen, make_dense_module
 
 pytestmark = pytest.mark.gpu
@@ -86,3 +87,13 @@ def test_expert_weight_gradients_either_side_of_the_rule(hip_device, r, rp, tran
             assert torch.count_nonzero(g[e]) == 0
         else:
             close(g[e], ref, 1e-2, rows="none")
+
+
+@pytest.mark.parametrize("fmt,E,T,I,r,hybrid", [
+    ("block_fp8", 3, 1500, 256, 24, False),     # row chunks; dA of gate and up side by side, 64 ranks wide
+    ("block_fp8", 12, 200, 256, 16, True),      # a block per expert; the shared factors' gradients in a launch of their own
+    ("nvfp4", 3, 1500, 192, 40, True),          # row chunks, every product by itself
+    ("nf4", 12, 200, 192, 8, False),
+])
+def test_expert_factor_gradients_of_a_call(hip_device, fmt, E, T, I, r, hybrid):
+    check_experts(hip_device, 0, fmt, E, T, 256, I, r, 2, hybrid)

@@ -22,17 +22,6 @@ struct Carve {
     }
 };
 
-// dst0[m][i][j] = src[m][i][j], dst1[m][i][j] = src[m][i][half + j] for j < r: the two factor gradients that one
-// pass over the rows produced side by side
-__global__ void __launch_bounds__(256) split_pair_kernel(const float* src, int64_t rows, int half, int r, float* dst0, float* dst1) {
-    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (t >= rows * r) return;
-    const int64_t i = t / r;
-    const int j = (int)(t - i * r);
-    dst0[t] = src[i * 2 * half + j];
-    dst1[t] = src[i * 2 * half + half + j];
-}
-
 // token_of_row[scatter_index[i]] = i / topk: the token whose copy sits in row r of the expert order (routed copies
 // with an invalid expert id have no row)
 __global__ void __launch_bounds__(256) invert_scatter_kernel(const int32_t* scatter_index, int64_t n, int topk, int32_t* token_of_row) {
@@ -88,11 +77,12 @@ int64_t fwd_workspace(const Dims& d) {
 int64_t bwd_workspace(const Dims& d) {
     const int64_t EH = al256((int64_t)d.E * d.rp * d.H * 2), EI = al256((int64_t)d.E * d.rp * d.I * 2);
     const int64_t panels = 3 * EH + 3 * EI;     // F_dB, Lr_gA, Lr_uA over H; Lr_dA, F_gB, F_uB over I
-    const int64_t wide = d.H > d.I ? d.H : d.I;
-    const int64_t wg = al256(xq_lora_wgrad_workspace_bytes(d.R, wide, 2 * d.rp <= 64 ? 2 * d.rp : d.rp));
-    const int64_t pair = al256((int64_t)d.E * d.H * 2 * d.rp * 4);      // the two A gradients side by side
+    // partial sums of the factor gradients, which share a launch: three products over I, dB of down over H, dA of gate and up
+    // over H side by side or apart
+    const int64_t wg = 3 * tn_partial_bytes(d.R, d.I, d.rp) + tn_partial_bytes(d.R, d.H, d.rp) +
+                       std::max(2 * tn_partial_bytes(d.R, d.H, d.rp), 2 * d.rp <= 64 ? tn_partial_bytes(d.R, d.H, 2 * d.rp) : 0) + 256;
     return panels + 3 * al256(d.R * d.H * 2) + al256(d.R * d.I * 2) + al256(d.R * 2 * d.I * 2) + 2 * al256(d.R * 4) +
-           al256(d.R * d.rp * 2) + al256(d.R * 2 * d.rp * 2) + pair + wg + 256;
+           al256(d.R * d.rp * 2) + al256(d.R * 2 * d.rp * 2) + wg + 256;
 }
 
 // one launch for gate and up (forward) / one sum for their two dgrads: block-fp8 banks on the pipelined kernel
@@ -290,7 +280,6 @@ extern "C" int xq_grouped_bwd(const xq_weight* gate, const xq_weight* up, const 
     float* d_w_row = cv.take<float>(R * 4);
     bf16_t* v_d = cv.take<bf16_t>(R * rp * 2);
     bf16_t* v_gu = cv.take<bf16_t>(R * rp2 * 2);          // fused: [R, 2 rp] = v_g | v_u; else v_g [R, rp] then v_u [R, rp]
-    float* pair = cv.take<float>((int64_t)E * H * rp2 * 4);
     int32_t* token_of_row = cv.take<int32_t>(R * 4);
     float* wg = cv.take<float>(0);
     bf16_t *dgate = dgu, *dup = dgu + I;
@@ -326,8 +315,6 @@ extern "C" int xq_grouped_bwd(const xq_weight* gate, const xq_weight* up, const 
     const int64_t ld_gd = in_place ? ld_dy : H;
     const int32_t* gd_rows = in_place ? token_of_row : nullptr;
     if ((rc = launch_tile_gemm(down, true, gd, ld_gd, R, off, toff, v_d, Lr_dA, rp, nullptr, dh, I, stream, who, nullptr, 0, nullptr, nullptr, gd_rows, d.T))) return rc;
-    if ((rc = launch_tn(gd, ld_gd, H, su_d, rp, r, R, true, grads->dB[2], wg, dBe == 1 ? nullptr : off, E, stream, n_valid, 0, gd_rows))) return rc;   // [E|1, r, H]
-    if ((rc = launch_tn(h, I, I, v_d, rp, r, R, false, grads->dA[2], wg, dAe == 1 ? nullptr : off, E, stream, n_valid))) return rc;        // [E|1, I, r]
 
     // ---- SwiGLU + routing weight, and s * dgate . B_g^T, s * dup . B_u^T of the up / gate projections (y = x.W + s*(x.A).B):
     // one pass over (gate, up, dh) where the rank allows, so that the two products do not read dgate | dup back
@@ -349,19 +336,27 @@ extern "C" int xq_grouped_bwd(const xq_weight* gate, const xq_weight* up, const 
         if ((rc = launch_tile_gemm(up, true, dup, 2 * I, R, off, toff, v_u, Lr_uA, rp, nullptr, dx_u, H, stream, who, nullptr, 0))) return rc;
         if ((rc = launch_tile_gemm(gate, true, dgate, 2 * I, R, off, toff, v_g, Lr_guA, rp, nullptr, dx_g, H, stream, who, nullptr, 0))) return rc;
     }
-    if ((rc = launch_tn(dup, 2 * I, I, su_u, rp, r, R, true, grads->dB[1], wg, uBe == 1 ? nullptr : off, E, stream, n_valid))) return rc;      // [E|1, r, I]
-    if ((rc = launch_tn(dgate, 2 * I, I, su_g, rp, r, R, true, grads->dB[0], wg, gBe == 1 ? nullptr : off, E, stream, n_valid))) return rc;
-    // gradients of the two A factors, [E|1, H, r] = x^T . v: both contract the same rows of x, so with v_g | v_u side
-    // by side they share one pass over them
+    // ---- the factor gradients, [E|1, r, out] = Q^T . P and [E|1, in, r] = P^T . Q: those held per expert share a launch, those
+    // shared by all experts another one over all rows
+    TnJob per_expert[kTnJobs], shared[kTnJobs];
+    int ne = 0, ns = 0;
+    auto add = [&](int matrices, const TnJob& j) {
+        if (matrices == 1) shared[ns++] = j;
+        else per_expert[ne++] = j;
+    };
+    add(dBe, TnJob{gd, ld_gd, H, su_d, rp, rp, r, true, grads->dB[2], gd_rows});
+    add(dAe, TnJob{h, I, I, v_d, rp, rp, r, false, grads->dA[2]});
+    add(uBe, TnJob{dup, 2 * I, I, su_u, rp, rp, r, true, grads->dB[1]});
+    add(gBe, TnJob{dgate, 2 * I, I, su_g, rp, rp, r, true, grads->dB[0]});
+    // (both A factors contract the same rows of x: with v_g | v_u side by side they share one pass over them)
     if (fused) {
-        if ((rc = launch_tn(xr, ld_xr, H, v_gu, rp2, rp2, R, false, pair, wg, gAe == 1 ? nullptr : off, E, stream, n_valid, 0, xr_rows))) return rc;
-        const int64_t rows = (int64_t)gAe * H;
-        split_pair_kernel<<<dim3((unsigned)xq_cdiv(rows * r, 256)), 256, 0, stream>>>(pair, rows, rp, r, grads->dA[0], grads->dA[1]);
-        XQ_CHECK_LAUNCH(who);
+        add(gAe, TnJob{xr, ld_xr, H, v_gu, rp2, rp2, r, false, grads->dA[0], xr_rows, grads->dA[1], rp});
     } else {
-        if ((rc = launch_tn(xr, ld_xr, H, v_g, rp, r, R, false, grads->dA[0], wg, gAe == 1 ? nullptr : off, E, stream, n_valid, 0, xr_rows))) return rc;
-        if ((rc = launch_tn(xr, ld_xr, H, v_u, rp, r, R, false, grads->dA[1], wg, uAe == 1 ? nullptr : off, E, stream, n_valid, 0, xr_rows))) return rc;
+        add(gAe, TnJob{xr, ld_xr, H, v_g, rp, rp, r, false, grads->dA[0], xr_rows});
+        add(uAe, TnJob{xr, ld_xr, H, v_u, rp, rp, r, false, grads->dA[1], xr_rows});
     }
+    if (ne && (rc = launch_tn_grouped_multi(per_expert, ne, R, wg, off, E, stream))) return rc;
+    if (ns && (rc = launch_tn_multi(shared, ns, R, wg, stream, n_valid))) return rc;
     if (!dx) return XQ_OK;
     return xq_moe_gather(dx_g, fused ? nullptr : dx_u, H, sidx, d.T, topk, H, dx, ld_dx, stream);
 }

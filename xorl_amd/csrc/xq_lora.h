@@ -142,6 +142,9 @@ struct TnJob {
     int32_t split_j;
 };
 int launch_tn_multi(const TnJob* jobs, int n, int64_t n_rows, float* partial, hipStream_t stream, const int32_t* row_limit = nullptr);
+// ... and so can grouped ones (one set of offsets)
+int launch_tn_grouped_multi(const TnJob* jobs, int n, int64_t n_rows, float* partial, const int32_t* offsets, int32_t num_experts,
+                            hipStream_t stream);
 int64_t tn_partial_bytes(int64_t n_rows, int64_t width, int r_pad);
 int launch_tn(const bf16_t* P, int64_t ldp, int64_t width, const bf16_t* Q, int r_pad, int r_out,
               int64_t n_rows, bool transpose_out, float* out, float* partial,

@@ -1194,13 +1194,38 @@ __global__ void __launch_bounds__(256) tn_kernel(TnBatch b) {
     else tn_write<NT>(acc, b.partial[ji] + (int64_t)split * g.width * g.r_pad, c0, g.width, g.r_pad, g.r_pad, false);
 }
 
-// grouped, experts of few rows: block (col tile, expert) -> out[expert], zero for an expert without rows
+// grouped, up to kTnJobs products of the same rows in one launch: block (job, row part, col tile)
+struct TnGroupedBatch {
+    TnArgs job[kTnJobs];
+    float* partial[kTnJobs];
+    int32_t first[kTnJobs];           // first block of a job
+    int32_t col_tiles[kTnJobs];
+    int32_t n;
+};
+__device__ __forceinline__ int tn_grouped_job(const TnGroupedBatch& b, int* part, int64_t* c0) {
+    int ji = 0;
+#pragma unroll
+    for (int i = 1; i < kTnJobs; ++i)
+        if (i < b.n && (int)blockIdx.x >= b.first[i]) ji = i;
+    const int at = (int)blockIdx.x - b.first[ji];
+    *part = at / b.col_tiles[ji];
+    *c0 = (int64_t)(at - *part * b.col_tiles[ji]) * 128;
+    return ji;
+}
 template <int NT>
-__global__ void __launch_bounds__(256) tn_expert_kernel(TnArgs g) {
+__device__ __forceinline__ void tn_write_expert(const TnArgs& g, const f32x16* acc, int64_t c0, int e) {
+    const int64_t at = (int64_t)e * g.width * g.r_out;
+    tn_write<NT>(acc, g.out + at, c0, g.width, g.r_out, g.r_out, g.transpose_out != 0, g.out2 ? g.out2 + at : nullptr, g.split_j);
+}
+
+// experts of few rows: row part = expert -> out[expert], zero for an expert without rows
+template <int NT>
+__global__ void __launch_bounds__(256) tn_expert_kernel(TnGroupedBatch b) {
     __shared__ __attribute__((aligned(16))) bf16_t Ps[2 * 32 * TN_PP];
     __shared__ __attribute__((aligned(16))) bf16_t Qs[2 * 32 * TN_QP];
-    const int64_t c0 = (int64_t)blockIdx.x * 128;
-    const int e = blockIdx.y;
+    int e;
+    int64_t c0;
+    const TnArgs& g = b.job[tn_grouped_job(b, &e, &c0)];
     const int64_t m_begin = g.offsets[e], m_end = g.offsets[e + 1];
     f32x16 acc[NT];
 #pragma unroll
@@ -1208,20 +1233,26 @@ __global__ void __launch_bounds__(256) tn_expert_kernel(TnArgs g) {
 #pragma unroll
         for (int q = 0; q < 16; ++q) acc[n][q] = 0.0f;
     if (m_begin < m_end) tn_accumulate<NT>(g, c0, m_begin, m_end, Ps, Qs, acc);     // uniform over the block
-    tn_write<NT>(acc, g.out + (int64_t)e * g.width * g.r_out, c0, g.width, g.r_out, g.r_out, g.transpose_out != 0);
+    tn_write_expert<NT>(g, acc, c0, e);
 }
 
-// grouped: block (col tile, chunk of TN_CHUNK global rows).  The chunk is walked expert by expert;
+// row part = chunk of TN_CHUNK global rows.  The chunk is walked expert by expert;
 // an expert that lies wholly inside the chunk is written to out[e] directly, a piece of an expert
 // that continues from the previous chunk goes to partial[chunk][0], one that continues into the
 // next chunk to partial[chunk][1] (tn_grouped_reduce_kernel adds the pieces in chunk order).
+// What bounds it: the rows in flight (two tiles of 32 a block).  A product of 131072 rows and 768 columns is 768 blocks, three a
+// compute unit; the joint launch keeps the five that fit there to the end:
+// the five products of 131072 rows (2048 and 768 columns, rank 16, gate and up side by side) 356 us one by one, 322 together.
 template <int NT>
-__global__ void __launch_bounds__(256) tn_grouped_kernel(TnArgs g, int32_t num_experts, float* partial) {
+__global__ void __launch_bounds__(256) tn_grouped_kernel(TnGroupedBatch b, int32_t num_experts) {
     __shared__ __attribute__((aligned(16))) bf16_t Ps[2 * 32 * TN_PP];
     __shared__ __attribute__((aligned(16))) bf16_t Qs[2 * 32 * TN_QP];
     __shared__ int sh_e;
-    const int64_t c0 = (int64_t)blockIdx.x * 128;
-    const int64_t r_begin = (int64_t)blockIdx.y * TN_CHUNK;
+    int chunk;
+    int64_t c0;
+    const int ji = tn_grouped_job(b, &chunk, &c0);
+    const TnArgs& g = b.job[ji];
+    const int64_t r_begin = (int64_t)chunk * TN_CHUNK;
     int64_t r_end = r_begin + TN_CHUNK;
     r_end = r_end < g.n_rows ? r_end : g.n_rows;
     // the expert that owns row r_begin (offsets[e] <= r_begin < offsets[e + 1]; r_begin < n_rows = offsets[E], so
@@ -1246,9 +1277,9 @@ __global__ void __launch_bounds__(256) tn_grouped_kernel(TnArgs g, int32_t num_e
             for (int q = 0; q < 16; ++q) acc[n][q] = 0.0f;
         tn_accumulate<NT>(g, c0, m, seg_end, Ps, Qs, acc);
         if (eb >= r_begin && ee <= r_end)
-            tn_write<NT>(acc, g.out + (int64_t)e * g.width * g.r_out, c0, g.width, g.r_out, g.r_out, g.transpose_out != 0);
+            tn_write_expert<NT>(g, acc, c0, e);
         else
-            tn_write<NT>(acc, partial + ((int64_t)blockIdx.y * 2 + (eb < r_begin ? 0 : 1)) * g.width * g.r_pad, c0, g.width,
+            tn_write<NT>(acc, b.partial[ji] + ((int64_t)chunk * 2 + (eb < r_begin ? 0 : 1)) * g.width * g.r_pad, c0, g.width,
                          g.r_pad, g.r_pad, false);
         m = seg_end;
         ++e;
@@ -1256,27 +1287,39 @@ __global__ void __launch_bounds__(256) tn_grouped_kernel(TnArgs g, int32_t num_e
 }
 
 // out[e] for the experts the chunk walk did not finish: zero for an expert without rows, the sum of
-// its pieces in chunk order for one that spans several chunks.
-__global__ void __launch_bounds__(256) tn_grouped_reduce_kernel(const float* partial, const int32_t* offsets, int64_t width,
-                                                                int r_pad, int r_out, int transpose_out, float* out) {
+// its pieces in chunk order for one that spans several chunks.  Block x: 1024 elements of a job's [width, r_pad], y: expert
+// (most blocks find their expert finished: four elements a thread keep their number down: 28 us for those five products,
+// 55 with one element).
+__global__ void __launch_bounds__(256) tn_grouped_reduce_kernel(TnGroupedBatch b) {
     const int e = blockIdx.y;
-    const int64_t b = offsets[e], en = offsets[e + 1];
-    const int64_t ch0 = b / TN_CHUNK, ch1 = en > b ? (en - 1) / TN_CHUNK : ch0;
-    if (en > b && ch0 == ch1) return;   // written directly
-    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (t >= width * r_pad) return;
-    const int64_t c = t / r_pad;
-    const int j = (int)(t - c * r_pad);
-    if (j >= r_out) return;
-    float s = 0.0f;
-    if (en > b) {
-        const int64_t per = width * r_pad;
-        s = partial[(ch0 * 2 + 1) * per + t];
-        for (int64_t ch = ch0 + 1; ch <= ch1; ++ch) s += partial[(ch * 2) * per + t];
+    int ji = 0;
+#pragma unroll
+    for (int i = 1; i < kTnJobs; ++i)
+        if (i < b.n && (int)blockIdx.x >= b.first[i]) ji = i;
+    const TnArgs& g = b.job[ji];
+    const int64_t rb = g.offsets[e], en = g.offsets[e + 1];
+    const int64_t ch0 = rb / TN_CHUNK, ch1 = en > rb ? (en - 1) / TN_CHUNK : ch0;
+    if (en > rb && ch0 == ch1) return;   // written directly
+    const int64_t t = ((int64_t)((int)blockIdx.x - b.first[ji]) * 256 + threadIdx.x) * 4;
+    if (t >= g.width * g.r_pad) return;
+    const int64_t c = t / g.r_pad;
+    int j = (int)(t - c * g.r_pad);      // (r_pad and split_j are multiples of 16: the four lie in one row of one result)
+    f32x4 s = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (en > rb) {
+        const int64_t per = g.width * g.r_pad;
+        const float* partial = b.partial[ji];
+        s = *(const f32x4*)(partial + (ch0 * 2 + 1) * per + t);
+        for (int64_t ch = ch0 + 1; ch <= ch1; ++ch) s += *(const f32x4*)(partial + (ch * 2) * per + t);
     }
-    float* o = out + (int64_t)e * width * r_out;
-    if (transpose_out) o[(int64_t)j * width + c] = s;
-    else o[c * r_out + j] = s;
+    float* o = g.out;
+    if (g.out2 != nullptr && j >= g.split_j) { o = g.out2; j -= g.split_j; }
+    o += (int64_t)e * g.width * g.r_out;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        if (j + u >= g.r_out) break;
+        if (g.transpose_out) o[(int64_t)(j + u) * g.width + c] = s[u];
+        else o[c * g.r_out + j + u] = s[u];
+    }
 }
 
 // sums the dense partials of up to kTnJobs products in split order: out[c][j] or out[j][c], j < r_out
@@ -1377,38 +1420,59 @@ int launch_tn_multi(const TnJob* jobs, int n, int64_t n_rows, float* partial, hi
     return XQ_OK;
 }
 
-int launch_tn(const bf16_t* P, int64_t ldp, int64_t width, const bf16_t* Q, int r_pad, int r_out, int64_t n_rows,
-              bool transpose_out, float* out, float* partial, const int32_t* offsets, int32_t num_experts,
-              hipStream_t stream, const int32_t* row_limit, int64_t ldq, const int32_t* p_rows) {
-    if (ldq <= 0) ldq = r_pad;
-    if (!offsets) {
-        const TnJob j{P, ldp, width, Q, ldq, r_pad, r_out, transpose_out, out, p_rows};
-        return launch_tn_multi(&j, 1, n_rows, partial, stream, row_limit);
-    }
-    const int rc = tn_check(P, ldp, width, Q, ldq, r_pad, r_out);
-    if (rc) return rc;
-    if (width == 0 || r_out == 0) return XQ_OK;
-    TnArgs g{P, ldp, width, Q, r_pad, r_out, n_rows, 0, transpose_out ? 1 : 0, out, offsets, nullptr, ldq, p_rows, nullptr, 0};
-    const unsigned col_tiles = (unsigned)xq_cdiv(width, 128);
+int launch_tn_grouped_multi(const TnJob* jobs, int n, int64_t n_rows, float* partial, const int32_t* offsets, int32_t num_experts,
+                            hipStream_t stream) {
+    XQ_REQUIRE(n >= 0 && n <= kTnJobs, "tn: %d products", n);
     XQ_REQUIRE(partial != nullptr, "tn: partial workspace is NULL");
     // up to 256 rows an expert on average a block takes an expert's rows whole and writes its result: nothing is summed
     // afterwards, and the experts of a column tile run side by side instead of one after the other (456 rows of 128 experts,
     // 768 columns: 289 us in 6 blocks, 8 us in 768); beyond that, chunks of the row range keep uneven experts level
-    if (n_rows <= 256ll * num_experts) {
-        const dim3 grid(col_tiles, (unsigned)num_experts);
-        if (r_pad <= 32) tn_expert_kernel<1><<<grid, 256, 0, stream>>>(g);
-        else tn_expert_kernel<2><<<grid, 256, 0, stream>>>(g);
+    const bool by_expert = n_rows <= 256ll * num_experts;
+    const int64_t parts = by_expert ? num_experts : xq_cdiv(n_rows, TN_CHUNK);
+    TnGroupedBatch b{};
+    int32_t rfirst[kTnJobs];
+    int nt = 1;
+    int64_t blocks = 0, rblocks = 0;
+    for (int i = 0; i < n; ++i) {
+        const TnJob& j = jobs[i];
+        const int64_t ldq = j.ldq > 0 ? j.ldq : j.r_pad;
+        const int rc = tn_check(j.P, j.ldp, j.width, j.Q, ldq, j.r_pad, j.r_out);
+        if (rc) return rc;
+        if (j.width == 0 || j.r_out == 0) continue;
+        const int k = b.n++;
+        b.job[k] = TnArgs{j.P, j.ldp, j.width, j.Q, j.r_pad, j.r_out, n_rows, 0, j.transpose_out ? 1 : 0, j.out, offsets, nullptr, ldq, j.p_rows, j.out2, j.split_j};
+        b.partial[k] = partial;
+        b.col_tiles[k] = (int32_t)xq_cdiv(j.width, 128);
+        b.first[k] = (int32_t)blocks;
+        blocks += b.col_tiles[k] * parts;
+        rfirst[k] = (int32_t)rblocks;
+        rblocks += xq_cdiv(j.width * j.r_pad, 1024);
+        if (j.r_pad > 32) nt = 2;
+        partial += tn_partial_bytes(n_rows, j.width, j.r_pad) / 4;
+    }
+    if (b.n == 0) return XQ_OK;
+    XQ_REQUIRE(blocks < (1ll << 31), "tn: %lld blocks", (long long)blocks);
+    if (by_expert) {
+        if (nt == 1) tn_expert_kernel<1><<<(unsigned)blocks, 256, 0, stream>>>(b);
+        else tn_expert_kernel<2><<<(unsigned)blocks, 256, 0, stream>>>(b);
         XQ_CHECK_LAUNCH("tn(expert)");
         return XQ_OK;
     }
-    dim3 grid(col_tiles, (unsigned)xq_cdiv(n_rows, TN_CHUNK));
-    if (r_pad <= 32) tn_grouped_kernel<1><<<grid, 256, 0, stream>>>(g, num_experts, partial);
-    else tn_grouped_kernel<2><<<grid, 256, 0, stream>>>(g, num_experts, partial);
+    if (nt == 1) tn_grouped_kernel<1><<<(unsigned)blocks, 256, 0, stream>>>(b, num_experts);
+    else tn_grouped_kernel<2><<<(unsigned)blocks, 256, 0, stream>>>(b, num_experts);
     XQ_CHECK_LAUNCH("tn(grouped)");
-    dim3 rgrid((unsigned)xq_cdiv(width * r_pad, 256), (unsigned)num_experts);
-    tn_grouped_reduce_kernel<<<rgrid, 256, 0, stream>>>(partial, offsets, width, r_pad, r_out, transpose_out ? 1 : 0, out);
+    for (int k = 0; k < b.n; ++k) b.first[k] = rfirst[k];
+    tn_grouped_reduce_kernel<<<dim3((unsigned)rblocks, (unsigned)num_experts), 256, 0, stream>>>(b);
     XQ_CHECK_LAUNCH("tn(grouped reduce)");
     return XQ_OK;
+}
+
+int launch_tn(const bf16_t* P, int64_t ldp, int64_t width, const bf16_t* Q, int r_pad, int r_out, int64_t n_rows,
+              bool transpose_out, float* out, float* partial, const int32_t* offsets, int32_t num_experts,
+              hipStream_t stream, const int32_t* row_limit, int64_t ldq, const int32_t* p_rows) {
+    const TnJob j{P, ldp, width, Q, ldq > 0 ? ldq : r_pad, r_pad, r_out, transpose_out, out, p_rows, nullptr, 0};
+    if (!offsets) return launch_tn_multi(&j, 1, n_rows, partial, stream, row_limit);
+    return launch_tn_grouped_multi(&j, 1, n_rows, partial, offsets, num_experts, stream);
 }
 
 }  // namespace xq

@@ -191,8 +191,10 @@ int xq_decode(const xq_weight* w, void* out, int out_dtype, void* stream);
 /* Bytes of scratch the dense entry points need for (M, N, K, r): the prepared
  * LoRA panels and partial sums of the factor gradients (r > 0) and, for row
  * counts that leave most of the chip without a tile, the fp32 partial sums of
- * the split-K product.  With r == 0 the workspace is optional: a call without
- * it (or with fewer bytes) runs the product unsplit. */
+ * the split-K product; under many rows (640 and more) also room for the weight
+ * decoded once to bf16.  That room is optional: a call without it decodes in
+ * the tiles.  With r == 0 the whole workspace is optional: a call without it
+ * (or with fewer bytes) runs the product unsplit. */
 int64_t xq_linear_workspace_bytes(int64_t M, int64_t N, int64_t K, int r);
 
 /* y[M,N] = x[M,K] . deq(W)^T + bias + s * (x . A^T) . B^T      (bf16 out)
@@ -253,8 +255,8 @@ int xq_linear_fwd_multi(const xq_linear_job* jobs, int n_jobs, const void* x, in
  * the scratch is a buffer of XQ_STATIC_SCRATCH_BYTES built into the library's
  * code object, one copy per device, resolved once per device at the first call
  * made with that device current.  The call allocates and frees nothing.
- * Shapes whose xq_linear_workspace_bytes(M, N, K, r) exceeds the buffer are
- * rejected with XQ_ERR_ARG.  All calls on one device share that device's
+ * Shapes whose workspace, the room for a decoded weight left out, exceeds the
+ * buffer are rejected with XQ_ERR_ARG.  All calls on one device share that device's
  * buffer: calls that overlap in time on one device (two streams, two host
  * threads) race; calls on one stream, or ordered by events, do not.  Nothing in
  * the buffer has to start at zero, so nothing is cleared between calls. */

@@ -44,12 +44,9 @@ MEASURED_TRAFFIC = {
     # gemm_256_kernel<int4, T=128> in 4 K splits + splitk_reduce_kernel: mean of the forward and dgrad launches
     # (64 MiB of it are the fp32 partial sums written and read back)
     0: (109.6 * 2 ** 20, "profiles/gemm_128_int4_linear_m512.txt", 0.04315),
-    # gemm_dtl16_kernel (dense block-fp8, 256x256 tiles): mean over the 5 launches of a step (gate, up and down
-    # forward, d_h, dx as one sum over the gate and up weights)
-    1: (1070.4 * 2 ** 20, "profiles/gemm_dtl16_fp8_mlp_m8192.txt", 0.7509),
-    # gemm_256_kernel<nvfp4>, 256x256 tiles (whole rounds; trailing rows in K splits) and 128x128 tiles
-    # (+ splitk_reduce_kernel): mean over the 12 launches of a step, fp32 partial sums included
-    2: (185.7 * 2 ** 20, "profiles/gemm_256_nvfp4_attn_m4096.txt", 0.14304),
+    # gemm_dec_kernel and the dec_image passes before it (dense block-fp8, 256x256 tiles over decoded images): mean over the 5
+    # products of a step (gate, up and down forward, d_h, dx as one sum over the gate and up weights)
+    1: (1708.6 * 2 ** 20, "profiles/gemm_dec_fp8_mlp_m8192.txt", 0.7336),
     # gemm_dtl16_kernel<.., grouped>: mean over the 4 launches of a step (gate|up forward over two banks, down
     # forward, d_h, dx as one sum over both banks)
     3: (1402.4 * 2 ** 20, "profiles/gemm_dtl16_fp8_grouped_moe_e128.txt", 0.6325),
@@ -59,8 +56,6 @@ MEASURED_TRAFFIC = {
     4: (39.3 * 2 ** 20, "profiles/skinny_kernels_decode_shapes.txt", 0.01712),
     # merge_prep_kernel + merge_kernel<fp8>: mean per call (re-quantise 96 MiB, publish 144 MiB algorithmic)
     5: (134.4 * 2 ** 20, "profiles/merge_kernel_fp8_mlp_weights.txt", 0.04168),
-    # gemm_256_kernel<nf4>: mean of the forward and dgrad launches
-    6: (748.2 * 2 ** 20, "profiles/gemm_256_nf4_mlp_m8192.txt", 0.84180),
     # gemm_256_kernel<nvfp4 GKN, grouped>: mean over the 6 launches of a step
     7: (893.9 * 2 ** 20, "profiles/gemm_256_nvfp4_gkn_grouped_moe_e128.txt", 0.52825),
     # merge_prep_kernel + merge_kernel<nvfp4>: mean per call over amax / re-quantise / publish of the four weights
@@ -199,7 +194,7 @@ def other_config(cfg: int, dev):
                 m(xs[k]).backward(dys[k])
         return (step, sum(lin_flops(Mtok, K, N, 16) for (N, K) in shapes.values()), False,
                 "configs[2]: nvfp4 QLoRA Qwen3-32B attention projections q/k/v/o, hidden 5120, M=4096, r=16, fwd+bwd",
-                "gemm_256_kernel<nvfp4> with 256x256 tiles (whole rounds of the chip; trailing tile rows in K splits + splitk_reduce_kernel) and 128x128 tiles (k/v forward and dgrad): fused dequant-GEMM, forward and dgrad launches")
+                "gemm_dec_kernel with its dec_image passes (nvfp4 decoded once per launch, 256x256x32 tiles; leading rows in whole rounds, trailing rows in K splits + splitk_reduce_kernel): forward and dgrad launches")
     if cfg in (3, 7, 8):
         # 7 / 8 are not BASELINE configs: configs[3] with the banks held as nvfp4 / NF4 (4-bit GKN storage)
         from xorl_amd.qlora import BlockFP8QLoRAMoeExperts, NF4QLoRAMoeExperts, NvFP4QLoRAMoeExperts
@@ -465,10 +460,10 @@ def main():
                    "tokens": M, "hidden": H, "intermediate": I, "lora_r": R, "format": "block_fp8"},
         "roofline": {"bound": "mfma", "achieved": achieved, "peak": BF16_MFMA_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": achieved / BF16_MFMA_PEAK_TFLOPS, "traffic": traffic, "traffic_source": traffic_source,
-                     "kernel": "gemm_dtl16_kernel<contract_cols true|false, 8 waves> (dense fused block-fp8 dequant-GEMM, "
-                               "256x256x64 tiles: gate, up and down forward, down dgrad, gate+up dgrad as one sum)"
+                     "kernel": "gemm_dec_kernel with its dec_image passes (dense block-fp8 decoded once per launch, "
+                               "256x256x32 tiles: gate, up and down forward, down dgrad, gate+up dgrad as one sum)"
                                if not args.unfused else
-                               "gemm_dtl16_kernel<contract_cols true|false, 8 waves> (dense fused block-fp8 dequant-GEMM, "
+                               "gemm_dec_kernel with its dec_image passes (dense block-fp8 decoded once per launch, "
                                "forward and dgrad launches)",
                      "launches": n.value, "avg_launch_ms": avg_launch_ms},
         "cpu_baseline": cpu,

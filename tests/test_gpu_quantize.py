@@ -68,3 +68,31 @@ def test_edges_of_the_dispatch(hip_device):
     d = w.to(hip_device)
     for fn in (Q.nvfp4_quantize, Q.nf4_quantize):
         _same(fn(d), fn(w))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("values", [(float("nan"),), (float("inf"), float("-inf")), (float("-inf"), float("nan"))])
+def test_nan_and_infinity_stay_visible(hip_device, monkeypatch, dtype, values):
+    """A damaged weight: the scales and codes of the torch forms on the same device.  (An e4m3 NaN counts as one whatever its sign.)"""
+    w = _weight((192, 640), dtype, 6)
+    w[7, 130], w[100, 3] = values[0], values[-1]
+    d = w.to(hip_device)
+    amax = torch.tensor([0.2])
+    calls = [lambda: Q.nf4_quantize(d), lambda: Q.nvfp4_quantize(d), lambda: Q.nvfp4_quantize(d, global_amax=amax),
+             lambda: Q.nvfp4_quantize(d, global_amax=amax * float("nan")), lambda: Q.int4_quantize_sym(d, 128),
+             lambda: Q.int4_quantize(d, 128), lambda: Q.int4_quantize(d, 32), lambda: Q.block_fp8_quantize_gkn(d),
+             lambda: Q.nf4_quantize_gkn(d), lambda: Q.nvfp4_quantize_gkn(d), lambda: Q.nvfp4_quantize_gkn(d, global_amax=amax),
+             lambda: Q.int4_quantize_gkn(d, 64), lambda: Q.int4_quantize_gkn(d, 32)]
+    got = [fn() for fn in calls]
+    with monkeypatch.context() as mp:
+        mp.setattr(torch.compiler, "is_compiling", lambda: True)          # leaves every call to the torch forms
+        want = [fn() for fn in calls]
+    for i, (a, b) in enumerate(zip(got, want)):
+        assert any(not torch.isfinite(t.float()).all() for t in b) or i in (2, 10)      # a given amax: an infinite block saturates
+        for s, t in zip(a, b):
+            assert s.dtype == t.dtype and s.shape == t.shape, i
+            if s.dtype == torch.uint8:
+                assert torch.equal(s, t), i
+            else:
+                assert torch.equal(s.float().isnan(), t.float().isnan()), i
+                assert torch.equal(s.float().nan_to_num(0.0, None, None), t.float().nan_to_num(0.0, None, None)), i

@@ -8,10 +8,10 @@ namespace xq {
 // from trunc(2a + 0.5) with the sum rounded in fp32, then 4 from a >= 1.75 and one more from 2.5, 3.5 and 5.  All of them are
 // integer thresholds of w = fl(4a + 1) = 2 fl(2a + 0.5) -- 2, 4, 6, 8, 11, 15, 21, the sum being exact from a = 1 on --, so the
 // code is the number of them at or below trunc(w): a population count.  10 instructions against 15 for the comparisons one
-// by one (scaling by 4 is exact: the caller folds it into the scale).
+// by one (scaling by 4 is exact: the caller folds it into the scale).  A NaN has code 0 (v_med3 takes the least of the others).
 __device__ __forceinline__ uint32_t fp4_code4(float v4) {
     constexpr uint32_t kAt = (1u << 2 | 1u << 4 | 1u << 6 | 1u << 8 | 1u << 11 | 1u << 15 | 1u << 21) >> 1;   // (no threshold at 0)
-    const uint32_t u = (uint32_t)(fminf(fabsf(v4), 24.0f) + 1.0f);
+    const uint32_t u = (uint32_t)(__builtin_amdgcn_fmed3f(fabsf(v4), 0.0f, 24.0f) + 1.0f);
     return (uint32_t)__builtin_popcount(kAt & ((1u << u) - 1u)) + (v4 < 0.0f ? 8u : 0u);
 }
 

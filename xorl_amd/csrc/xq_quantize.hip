@@ -6,7 +6,8 @@
 //   fp8    s = max(amax / 448, 1e-12) per 128 x 128 tile, e4m3(x / s)           ops/quantize/block_fp8_gkn_quantize.py:40-121
 //
 // Bound by HBM: the weight is read once (16-byte loads, held in registers between the group's absmax and its codes) and the
-// codes are written once.  Written in torch operations the same arithmetic was 15-25 passes over fp32 copies of the weight:
+// codes are written once.  A NaN stays visible: it makes its group's scale NaN (and nvfp4's global scale), and an infinity gives
+// an infinite scale, as in the torch forms.  Written in torch operations the same arithmetic was 15-25 passes over fp32 copies of the weight:
 // [12288, 4096] bf16 -> nvfp4 took 2250 us where the bytes need 26 at a large copy's rate.
 #include "xq_common.h"
 #include "xq_codes.h"
@@ -29,6 +30,12 @@ struct QuantArgs {
     void* amax_out;             // nvfp4 without a known tensor amax: the blocks' amax, in x's type (it is one of x's values),
     float* partial;             // and each thread block's maximum over them, for nvfp4_scales_kernel
 };
+
+// the larger / the smaller of the two, NaN where either is (fmaxf and fminf return the other operand); one instruction
+__device__ __forceinline__ float max_nan(float a, float b) { return __builtin_elementwise_maximum(a, b); }
+__device__ __forceinline__ float min_nan(float a, float b) { return __builtin_elementwise_minimum(a, b); }
+// into [-top, top], NaN kept
+__device__ __forceinline__ float clamp_nan(float v, float top) { return max_nan(min_nan(v, top), -top); }
 
 __device__ __forceinline__ void unpack8(u32x4 w, float* v) {
 #pragma unroll
@@ -68,16 +75,16 @@ struct GroupRule {
     const Nf4Bucket* nf4;
     __device__ __forceinline__ GroupRule(float amax, bool sym_, const Nf4Bucket* t) : sym(sym_), nf4(t) {
         if constexpr (FMT == XQ_FMT_NVFP4) {
-            scale = fmaxf(amax, 1e-12f);
+            scale = max_nan(amax, 1e-12f);
             mul = 4.0f * (6.0f / scale);                 // fp4_code4 takes 4 x the scaled value
         } else if constexpr (FMT == XQ_FMT_NF4) {
-            scale = fmaxf(amax, 1e-12f);
+            scale = max_nan(amax, 1e-12f);
             mul = 1.0f / scale;
         } else if (sym) {
             scale = round_bf16(amax / 7.0f);
             mul = scale > 0.0f ? 1.0f / scale : 0.0f;
         } else {
-            scale = fmaxf(amax, 1e-12f) * (float)(2.0 / 15.0);
+            scale = max_nan(amax, 1e-12f) * (float)(2.0 / 15.0);
             mul = 1.0f / scale;
         }
     }
@@ -85,26 +92,25 @@ struct GroupRule {
         if constexpr (FMT == XQ_FMT_NVFP4) {
             return fp4_code4(x * mul);
         } else if constexpr (FMT == XQ_FMT_NF4) {
-            return nf4_code(__builtin_amdgcn_fmed3f(x * mul, -1.0f, 1.0f), nf4);
+            return nf4_code(__builtin_amdgcn_fmed3f(x * mul, -1.0f, 1.0f), nf4);      // (NaN: -1, code 0)
         } else {
             if (sym) {
                 // x / scale rounded to fp32, as one multiplication by the rounded reciprocal and one correction: the remainder is
                 // exact, and with a bf16 scale no quotient lies closer than 2^-9 ulp to a rounding boundary, far outside the
-                // correction's error.  (Tiny scales, whose remainders would be denormal, and zero take the division.)
+                // correction's error.  (Tiny scales, whose remainders would be denormal, take the division; zero, infinite and NaN scales code 8.)
                 // [12288, 4096]: 44 -> 30 us
                 float q = x * mul;
                 q = __builtin_fmaf(__builtin_fmaf(-q, scale, x), mul, q);
-                if (scale < 0x1p-60f) q = scale > 0.0f ? x / scale : 0.0f;
+                if (!(scale >= 0x1p-60f && scale < INFINITY)) q = scale > 0.0f && scale < INFINITY ? x / scale : 0.0f;
                 return (uint32_t)((int)__builtin_amdgcn_fmed3f(__builtin_rintf(q), -7.0f, 7.0f) + 8);
             }
-            const int q = (int)__fadd_rn(__fmul_rn(x, mul), 8.5f);
-            return (uint32_t)(q < 0 ? 0 : q > 15 ? 15 : q);
+            return (uint32_t)__builtin_amdgcn_fmed3f(__fadd_rn(__fmul_rn(x, mul), 8.5f), 0.0f, 15.0f);      // (NaN: 0)
         }
     }
 };
 
 __device__ __forceinline__ uint8_t nvfp4_block_scale(float amax, float gamax) {
-    const float bs = __builtin_amdgcn_fmed3f(amax / gamax * 448.0f, -448.0f, 448.0f);
+    const float bs = clamp_nan(amax / gamax * 448.0f, 448.0f);
     return (uint8_t)(__builtin_amdgcn_cvt_pk_fp8_f32(bs, 0.0f, 0u, false) & 0xffu);
 }
 
@@ -114,10 +120,10 @@ __device__ __forceinline__ float nvfp4_global_scale(float gamax) { return gamax 
 __device__ __forceinline__ void store_block_max(float m, float* partial) {
     __shared__ float wm[4];
 #pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) m = fmaxf(m, __shfl_xor(m, d, 64));
+    for (int d = 32; d >= 1; d >>= 1) m = max_nan(m, __shfl_xor(m, d, 64));
     if ((threadIdx.x & 63) == 0) wm[threadIdx.x >> 6] = m;
     __syncthreads();
-    if (threadIdx.x == 0) partial[blockIdx.x] = fmaxf(fmaxf(wm[0], wm[1]), fmaxf(wm[2], wm[3]));
+    if (threadIdx.x == 0) partial[blockIdx.x] = max_nan(max_nan(wm[0], wm[1]), max_nan(wm[2], wm[3]));
 }
 
 template <bool F32>
@@ -135,7 +141,7 @@ __global__ void __launch_bounds__(256) quant_flat_kernel(QuantArgs g, int64_t ru
         __syncthreads();
     }
     const int lanes = g.group >> 4;
-    const float gm = FMT == XQ_FMT_NVFP4 && g.gamax ? fmaxf(g.gamax[0], 1e-12f) : 1.0f;
+    const float gm = FMT == XQ_FMT_NVFP4 && g.gamax ? max_nan(g.gamax[0], 1e-12f) : 1.0f;
     float top = 0.0f;
     // (the lanes of a group are in range together: the element count is a multiple of the group)
     for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < runs; t += (int64_t)gridDim.x * 256) {
@@ -147,8 +153,8 @@ __global__ void __launch_bounds__(256) quant_flat_kernel(QuantArgs g, int64_t ru
         b.get(v + 8);
         float m = 0.0f;
 #pragma unroll
-        for (int i = 0; i < 16; ++i) m = fmaxf(m, fabsf(v[i]));
-        for (int d = 1; d < lanes; d <<= 1) m = fmaxf(m, __shfl_xor(m, d, 64));
+        for (int i = 0; i < 16; ++i) m = max_nan(m, fabsf(v[i]));
+        for (int d = 1; d < lanes; d <<= 1) m = max_nan(m, __shfl_xor(m, d, 64));
         const GroupRule<FMT> rule(m, g.sym, nf4);
         uint32_t w[2] = {0u, 0u};
 #pragma unroll
@@ -157,7 +163,7 @@ __global__ void __launch_bounds__(256) quant_flat_kernel(QuantArgs g, int64_t ru
         if constexpr (FMT == XQ_FMT_NVFP4) {
             if (g.gamax) ((uint8_t*)g.scales)[t] = nvfp4_block_scale(rule.scale, gm);
             else store_amax<F32>(g.amax_out, t, m);
-            top = fmaxf(top, m);
+            top = max_nan(top, m);
         } else if ((threadIdx.x & (lanes - 1)) == 0) {
             if (FMT == XQ_FMT_INT4 && g.sym) ((bf16_t*)g.scales)[t / lanes] = to_bf16(rule.scale);
             else ((float*)g.scales)[t / lanes] = rule.scale;
@@ -180,7 +186,7 @@ __global__ void __launch_bounds__(256) quant_gkn_kernel(QuantArgs g, int64_t col
         __syncthreads();
     }
     const int lane = threadIdx.x & 63, rq = lane >> 4, cq = lane & 15;
-    const float gm = FMT == XQ_FMT_NVFP4 && g.gamax ? fmaxf(g.gamax[0], 1e-12f) : 1.0f;
+    const float gm = FMT == XQ_FMT_NVFP4 && g.gamax ? max_nan(g.gamax[0], 1e-12f) : 1.0f;
     float top = 0.0f;
     for (int64_t wv = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); wv < waves; wv += (int64_t)gridDim.x * 4) {
         const int64_t rb = wv / col_blocks, cb = wv - rb * col_blocks;
@@ -196,12 +202,12 @@ __global__ void __launch_bounds__(256) quant_gkn_kernel(QuantArgs g, int64_t col
             float v[8];
             raw[i].get(v);
 #pragma unroll
-            for (int c = 0; c < 8; ++c) m[c] = fmaxf(m[c], fabsf(v[c]));
+            for (int c = 0; c < 8; ++c) m[c] = max_nan(m[c], fabsf(v[c]));
         }
 #pragma unroll
         for (int c = 0; c < 8; ++c) {
-            if (g.group >= 32) m[c] = fmaxf(m[c], __shfl_xor(m[c], 16, 64));
-            if (g.group >= 64) m[c] = fmaxf(m[c], __shfl_xor(m[c], 32, 64));
+            if (g.group >= 32) m[c] = max_nan(m[c], __shfl_xor(m[c], 16, 64));
+            if (g.group >= 64) m[c] = max_nan(m[c], __shfl_xor(m[c], 32, 64));
         }
         uint32_t w[8][2];
 #pragma unroll
@@ -226,7 +232,7 @@ __global__ void __launch_bounds__(256) quant_gkn_kernel(QuantArgs g, int64_t col
                     ((float*)g.scales)[si] = rule.scale;
                 }
             }
-            top = fmaxf(top, ok ? m[c] : 0.0f);
+            top = max_nan(top, ok ? m[c] : 0.0f);
         }
         if (ok) {
 #pragma unroll
@@ -245,12 +251,12 @@ template <bool F32>
 __global__ void __launch_bounds__(256) nvfp4_scales_kernel(const void* amax, int64_t n, const float* partial, int parts, uint8_t* scales, float* gscale) {
     __shared__ float wm[4];
     float m = 0.0f;
-    for (int i = threadIdx.x; i < parts; i += 256) m = fmaxf(m, partial[i]);
+    for (int i = threadIdx.x; i < parts; i += 256) m = max_nan(m, partial[i]);
 #pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) m = fmaxf(m, __shfl_xor(m, d, 64));
+    for (int d = 32; d >= 1; d >>= 1) m = max_nan(m, __shfl_xor(m, d, 64));
     if ((threadIdx.x & 63) == 0) wm[threadIdx.x >> 6] = m;
     __syncthreads();
-    const float gm = fmaxf(fmaxf(fmaxf(wm[0], wm[1]), fmaxf(wm[2], wm[3])), 1e-12f);
+    const float gm = max_nan(max_nan(max_nan(wm[0], wm[1]), max_nan(wm[2], wm[3])), 1e-12f);
     if (blockIdx.x == 0 && threadIdx.x == 0) gscale[0] = nvfp4_global_scale(gm);
     for (int64_t t = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4; t < n; t += (int64_t)gridDim.x * 1024) {
         float a[4];
@@ -265,11 +271,11 @@ __global__ void __launch_bounds__(256) nvfp4_scales_kernel(const void* amax, int
             }
             uint32_t w = 0;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) w |= (uint32_t)nvfp4_block_scale(fmaxf(a[i], 1e-12f), gm) << (8 * i);
+            for (int i = 0; i < 4; ++i) w |= (uint32_t)nvfp4_block_scale(max_nan(a[i], 1e-12f), gm) << (8 * i);
             *(uint32_t*)(scales + t) = w;
         } else {
             for (int64_t i = t; i < n; ++i)
-                scales[i] = nvfp4_block_scale(fmaxf(F32 ? ((const float*)amax)[i] : bf16_to_f32(((const bf16_t*)amax)[i]), 1e-12f), gm);
+                scales[i] = nvfp4_block_scale(max_nan(F32 ? ((const float*)amax)[i] : bf16_to_f32(((const bf16_t*)amax)[i]), 1e-12f), gm);
         }
     }
 }
@@ -293,14 +299,14 @@ __global__ void __launch_bounds__(256) quant_fp8_kernel(QuantArgs g) {
         float v[8];
         raw[i].get(v);
 #pragma unroll
-        for (int c = 0; c < 8; ++c) m = fmaxf(m, fabsf(v[c]));
+        for (int c = 0; c < 8; ++c) m = max_nan(m, fabsf(v[c]));
     }
 #pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) m = fmaxf(m, __shfl_xor(m, d, 64));
+    for (int d = 32; d >= 1; d >>= 1) m = max_nan(m, __shfl_xor(m, d, 64));
     if ((tid & 63) == 0) wm[tid >> 6] = m;
     __syncthreads();
-    m = fmaxf(fmaxf(wm[0], wm[1]), fmaxf(wm[2], wm[3]));
-    const float s = fmaxf(m * g.amax_scale / 448.0f, 1e-12f);
+    m = max_nan(max_nan(wm[0], wm[1]), max_nan(wm[2], wm[3]));
+    const float s = max_nan(m * g.amax_scale / 448.0f, 1e-12f);
     if (tid == 0) ((float*)g.scales)[(int64_t)blockIdx.y * gridDim.x + blockIdx.x] = s;
     if (col >= g.cols) return;
 #pragma unroll
@@ -310,7 +316,7 @@ __global__ void __launch_bounds__(256) quant_fp8_kernel(QuantArgs g) {
         float v[8];
         raw[i].get(v);
 #pragma unroll
-        for (int c = 0; c < 8; ++c) v[c] = __builtin_amdgcn_fmed3f(v[c] / s, -448.0f, 448.0f);
+        for (int c = 0; c < 8; ++c) v[c] = clamp_nan(v[c] / s, 448.0f);
         uint32_t w[2];
 #pragma unroll
         for (int h = 0; h < 2; ++h) {

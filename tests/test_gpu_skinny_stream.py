@@ -49,3 +49,13 @@ def test_joint_launches(stream_only, hip_device, fmt, H, I, r, M):
         loras = {k: (m.lora_A.detach().cpu(), m.lora_B.detach().cpu()) for k, m in mods.items()}
         ex = R.mlp_fwd_bwd_exact(x, w_ref["gate"], w_ref["up"], w_ref["down"], loras, g.scaling, torch.zeros(M, H, dtype=torch.bfloat16))
         close(y.cpu(), ex["y"], 1e-2)
+
+
+@pytest.mark.parametrize("fmt,M,K", [("int4", 33, 65664), ("nvfp4", 64, 66560), ("block_fp8", 17, 131200), ("nf4", 2, 262272)])
+def test_a_contraction_of_more_than_64_splits(hip_device, fmt, M, K):
+    m, w_ref = make_dense_module(fmt, 64, K, 16, 32, seed=M, device=hip_device)
+    x = gen((M, K), 1.0, 72, torch.bfloat16)
+    with torch.no_grad():
+        y = m(x.to(hip_device))
+    ex = R.linear_fwd_bwd_exact(x, w_ref, m.lora_A.detach().cpu(), m.lora_B.detach().cpu(), m.scaling, torch.zeros(M, 64, dtype=torch.bfloat16))
+    close(y.cpu(), ex["y"], 1e-2)

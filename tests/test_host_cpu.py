@@ -132,3 +132,17 @@ def test_moe_module_state_matches_reference_contract():
         BlockFP8QLoRAMoeExperts(4, 4, 128, 256, target_modules=["q_proj"])
     with pytest.raises(ValueError):
         BlockFP8QLoRAMoeExperts(2, 4, 128, 256)          # expert parallel shards are out of scope
+
+
+@pytest.mark.parametrize("M,steps", [(1, 32), (16, 32), (17, 16), (32, 16), (33, 8), (64, 8)])
+def test_skinny_plan_holds_any_contraction(M, steps):
+    """A K split of the streaming forward keeps at most `steps` 128-element steps of x in LDS, so a contraction of K needs at
+    least K / 128 / steps splits, each with an fp32 partial sum in the workspace -- also beyond 64 of them."""
+    from xorl_amd import _C
+
+    N = 1024
+    for splits in (1, 63, 64, 65, 100):
+        for K in (128 * steps * splits - 128, 128 * steps * splits, 128 * steps * splits + 128):
+            if K >= 1024:
+                need = -(-K // (128 * steps)) * M * N * 4 + K // 128 * M * 16 * 4
+                assert _C.lib().xq_linear_workspace_bytes(M, N, K, 16) >= need, (M, K)

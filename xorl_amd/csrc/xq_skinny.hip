@@ -586,7 +586,8 @@ static int stream_splits(int64_t M, int64_t N, int64_t K) {
     const int mt = M <= 16 ? 1 : M <= 32 ? 2 : 4;
     int best = 0, last_steps = 0;
     double best_cost = 0;
-    for (int s = (int)xq_cdiv(ct, stream_steps_max(M)); s <= ct && s <= 64; ++s) {
+    // (a contraction so long that its x slices need more than 64 splits takes the fewest that hold them)
+    for (int s = (int)xq_cdiv(ct, stream_steps_max(M)); s <= ct && (s <= 64 || best == 0); ++s) {
         const int steps = (int)xq_cdiv(ct, s);
         if (steps == last_steps) continue;                         // more splits, none of them shorter
         last_steps = steps;

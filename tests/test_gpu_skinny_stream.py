@@ -59,3 +59,36 @@ def test_a_contraction_of_more_than_64_splits(hip_device, fmt, M, K):
         y = m(x.to(hip_device))
     ex = R.linear_fwd_bwd_exact(x, w_ref, m.lora_A.detach().cpu(), m.lora_B.detach().cpu(), m.scaling, torch.zeros(M, 64, dtype=torch.bfloat16))
     close(y.cpu(), ex["y"], 1e-2)
+
+
+@pytest.mark.parametrize("fmt,name,off", [("nvfp4", "weight_block_scales", 1), ("nf4", "weight_scales", 4), ("int4", "weight_scales", 2),
+                                          ("block_fp8", "weight_block_scales", 4)])
+@pytest.mark.parametrize("M,K", [(1, 1152), (1, 2048), (4, 1152), (4, 2048), (20, 1152), (64, 1152)])     # 2048: the one-launch kernels
+def test_scales_at_their_elements_alignment(hip_device, fmt, name, off, M, K):
+    """Scales that start anywhere an element may (a view into a larger buffer) are read where they are."""
+    m, _ = make_dense_module(fmt, 512, K, 16, 32, seed=M, device=hip_device)
+    x = gen((M, K), 1.0, 73, torch.bfloat16).to(hip_device)
+    with torch.no_grad():
+        want = m(x)
+        s = getattr(m, name)
+        flat = torch.zeros(s.numel() + 16, dtype=torch.uint8, device=hip_device)
+        moved = flat[off:off + s.numel()].view(s.shape)
+        moved.copy_(s)
+        setattr(m, name, moved)
+        assert moved.data_ptr() % 8 == off and torch.equal(m(x), want)
+
+
+def test_fp32_nvfp4_scales_at_four_bytes(hip_device):
+    """(sources merged at load keep fp32 block scales)"""
+    m, _ = make_dense_module("nvfp4", 512, 1152, 16, 32, seed=3, device=hip_device)
+    s = m.weight_block_scales.view(torch.float8_e4m3fn).float().view(torch.uint8).reshape(512, -1)
+    m._scale_dtypes["weight_block_scales"] = torch.float32
+    flat = torch.zeros(s.numel() + 16, dtype=torch.uint8, device=hip_device)
+    for M in (4, 40):
+        x = gen((M, 1152), 1.0, 74, torch.bfloat16).to(hip_device)
+        with torch.no_grad():
+            m.weight_block_scales = s
+            want = m(x)
+            m.weight_block_scales = flat[4:4 + s.numel()].view(s.shape)
+            m.weight_block_scales.copy_(s)
+            assert torch.equal(m(x), want)

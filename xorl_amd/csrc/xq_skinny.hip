@@ -61,6 +61,9 @@ struct StreamBatch {
 // one value per row tile and step from registers
 enum { kScFp8 = 0, kScInt4Window = 1, kScDealt = 2, kScStep = 3, kScUse = 4 };
 
+// scales lie where their elements may: a pair of words from any byte (one global_load_dwordx2 like an aligned one)
+typedef u32x2 u32x2_a1 __attribute__((aligned(1)));
+
 // element offset of fragment (j, q) within a 128-element step: what lane q of a row holds after its loads (block-fp8: two
 // loads of 16 bytes, 64 apart; 4-bit: one load of 16 bytes), so that a load instruction covers 64 contiguous bytes of a row
 template <int FMT>
@@ -164,7 +167,7 @@ stream_split_kernel(const bf16_t* x, int32_t ldx, int32_t M, int32_t K, int32_t 
 #pragma unroll
             for (int i = 0; i < NL; ++i) w[slot][rt][i] = *(const u32x4*)(wp[rt] + (int64_t)s * (128 / EB) + i * 64);
             if constexpr (SC == kScStep && FMT == XQ_FMT_NVFP4) {
-                const u32x2 v = *(const u32x2*)((const uint32_t*)g.scales + ((srow[rt] + s * 128 + q * 32) >> 4));
+                const u32x2 v = *(const u32x2_a1*)((const uint32_t*)g.scales + ((srow[rt] + s * 128 + q * 32) >> 4));
                 sw[slot][rt][0] = v[0];
                 sw[slot][rt][1] = v[1];
             } else if constexpr (SC == kScStep) {
@@ -174,7 +177,6 @@ stream_split_kernel(const bf16_t* x, int32_t ldx, int32_t M, int32_t K, int32_t 
         }
     };
     // windows of four steps (a window that would pass the row's end starts earlier; kScDealt clamps step by step)
-    typedef u32x2 u32x2_a2 __attribute__((aligned(2)));
     u32x2 win[RT], win_next[RT];
     const int row_steps = K >> 7;
     const auto load_window = [&](u32x2* dst, int s0) {
@@ -182,11 +184,11 @@ stream_split_kernel(const bf16_t* x, int32_t ldx, int32_t M, int32_t K, int32_t 
             const int c = c_begin + s0 < row_steps - 4 ? c_begin + s0 : row_steps - 4;
 #pragma unroll
             for (int rt = 0; rt < RT; ++rt)
-                dst[rt] = *(const u32x2_a2*)((const uint16_t*)g.scales + ((srow[rt] - k_begin) >> 7) + c);
+                dst[rt] = *(const u32x2_a1*)((const uint16_t*)g.scales + ((srow[rt] - k_begin) >> 7) + c);
         } else if constexpr (SC == kScDealt) {
             const int c = c_begin + s0 + q < row_steps - 1 ? c_begin + s0 + q : row_steps - 1;
 #pragma unroll
-            for (int rt = 0; rt < RT; ++rt) dst[rt] = *(const u32x2*)(g.scales + ((srow[rt] - k_begin) >> 7) * 8 + (int64_t)c * 8);
+            for (int rt = 0; rt < RT; ++rt) dst[rt] = *(const u32x2_a1*)(g.scales + ((srow[rt] - k_begin) >> 7) * 8 + (int64_t)c * 8);
         }
     };
     float ts[RT];                                                  // block-fp8: lane l holds the scale of step l
@@ -620,11 +622,11 @@ bool skinny_supported(const xq_weight* w, int64_t M) {
     return true;
 }
 
+// (the storages that xq_validate_weight and skinny_supported leave: nf4 fp32, nvfp4 e4m3 or fp32, int4 fp32 or bf16)
 static int scale_mode(const xq_weight* w) {
     if (w->format == XQ_FMT_FP8) return kScFp8;
-    if (w->format == XQ_FMT_NF4) return xq_aligned(w->scales, 8) ? kScDealt : -1;
-    if (w->format == XQ_FMT_NVFP4) return w->scale_dtype == XQ_SCALE_E4M3 ? (xq_aligned(w->scales, 8) ? kScDealt : -1)
-                                        : (w->scale_dtype == XQ_SCALE_F32 && xq_aligned(w->scales, 8) ? kScStep : -1);
+    if (w->format == XQ_FMT_NF4) return kScDealt;
+    if (w->format == XQ_FMT_NVFP4) return w->scale_dtype == XQ_SCALE_E4M3 ? kScDealt : kScStep;
     if (w->group == 128 && w->scale_dtype == XQ_SCALE_BF16) return kScInt4Window;
     return w->group % 32 == 0 && w->cols % w->group == 0 ? kScStep : kScUse;
 }
@@ -667,7 +669,7 @@ bool skinny_stream_multi_supported(const SkinnyRowsJob* jobs, int n_jobs, int64_
     if (n_jobs < 1 || n_jobs > kStreamJobs) return false;
     for (int i = 0; i < n_jobs; ++i) {
         const xq_weight* w = jobs[i].w;
-        if (!skinny_supported(w, M) || scale_mode(w) < 0 || w->format != jobs[0].w->format || w->cols != jobs[0].w->cols ||
+        if (!skinny_supported(w, M) || w->format != jobs[0].w->format || w->cols != jobs[0].w->cols ||
             scale_mode(w) != scale_mode(jobs[0].w) || !xq_aligned(w->packed, 16) || jobs[i].ldy % 4 != 0 || !xq_aligned(jobs[i].y, 8))
             return false;
         if (jobs[i].r > 0 && (!xq_aligned(jobs[i].lora_A, 16) || !xq_aligned(jobs[i].lora_B, 4))) return false;
@@ -686,7 +688,7 @@ int launch_skinny_stream(const SkinnyRowsJob* jobs, int n_jobs, bool swiglu, con
     const xq_weight* w0 = jobs[0].w;
     const int64_t K = w0->cols;
     const int sc = scale_mode(w0), mt = M <= 16 ? 1 : M <= 32 ? 2 : 4;
-    XQ_REQUIRE(sc >= 0 && ldx < (1ll << 31), "xq_linear_fwd: internal error: shape not supported by the streaming kernel");
+    XQ_REQUIRE(ldx < (1ll << 31), "xq_linear_fwd: internal error: shape not supported by the streaming kernel");
     StreamBatch b{};
     EpiBatch e{};
     uint8_t* ws = (uint8_t*)workspace;
@@ -777,7 +779,6 @@ int launch_skinny(const xq_weight* w, const bf16_t* x, int64_t ldx, int64_t M, c
     XQ_REQUIRE(ldx % 8 == 0 && xq_aligned(x, 16) && xq_aligned(w->packed, 16), "xq_linear_fwd: operands must be 16-byte aligned");
     XQ_REQUIRE(ldy % 4 == 0 && xq_aligned(y, 8), "xq_linear_fwd: output rows must be 8-byte aligned");
     XQ_REQUIRE(rp == 0 || (xq_aligned(lora_A, 16) && xq_aligned(lora_B, 4)), "xq_linear_fwd: lora_A must be 16-byte and lora_B 4-byte aligned");
-    XQ_REQUIRE(scale_mode(w) >= 0, "xq_linear_fwd: scales must be 8-byte aligned");
     // algorithmic bytes: packed weight + scales + x + y (+ LoRA factors), for the roofline figure; the timed
     // region is the whole forward (both launches)
     const double wbytes = (double)xq_packed_bytes_per_expert(w) + (double)xq_scale_bytes_per_expert(w);

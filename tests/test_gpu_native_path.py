@@ -161,3 +161,44 @@ def test_tangents_and_transforms_are_refused_as_before(hip_device):
         m(fwAD.make_dual(x, torch.ones_like(x)))
     with pytest.raises(RuntimeError):
         torch.vmap(lambda s: m(x) * s)(torch.ones(2, device=hip_device))
+
+
+def test_strided_activations_are_read_in_place(hip_device, both_paths):
+    """A [B, S, K] slice of a wider last dimension: the bits of the packed copy, and not the memory of one, in either direction."""
+    B, S, K, N = 2, 320, 4096, 128
+    m, _ = make_dense_module("block_fp8", N, K, 16, 32, 3, hip_device)
+    wide = gen((B, S, 2 * K), 1.0, 4, torch.bfloat16).to(hip_device)
+    wide_dy = gen((B, S, 3 * N), 1.0, 5, torch.bfloat16).to(hip_device)
+    x, dy = wide[..., K:], wide_dy[..., N:2 * N]
+
+    def step(x, dy):
+        xr = x.detach().requires_grad_(True)
+        y = m(xr)
+        return [y.detach(), *torch.autograd.grad(y, [xr, m.lora_A, m.lora_B], dy)]
+
+    def infer(x):
+        with torch.no_grad():
+            return [m(x), m(x[:, :1]), m(x[:1, 3]), m(x[:, ::2])]
+
+    def peak(fn, *args):
+        fn(*args)
+        torch.cuda.synchronize()
+        before = torch.cuda.memory_allocated()
+        torch.cuda.reset_peak_memory_stats()
+        fn(*args)
+        torch.cuda.synchronize()
+        return torch.cuda.max_memory_allocated() - before
+
+    packed = x.contiguous(), dy.contiguous()
+    for a, b in zip(both_paths(lambda: step(x, dy)), step(*packed)):
+        assert torch.equal(a, b)
+    for a, b in zip(both_paths(lambda: infer(x)), infer(packed[0])):
+        assert torch.equal(a, b)
+    assert peak(step, x, dy) == peak(step, *packed)
+    assert peak(lambda t: m(t).detach(), x) == peak(lambda t: m(t).detach(), packed[0])
+    # layouts that do need one: rows a varying pitch apart, a pitch that is no multiple of 16 bytes, rows that start off one
+    odd = gen((B * S, K + 4), 1.0, 6, torch.bfloat16).to(hip_device)
+    with torch.no_grad():
+        for t in (x.transpose(0, 1), wide[:, ::3, :K], odd[:, :K], wide[..., 4:K + 4]):
+            for a, b in zip(both_paths(lambda: [m(t)]), [m(t.contiguous())]):
+                assert torch.equal(a, b)

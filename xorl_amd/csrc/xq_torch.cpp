@@ -230,22 +230,33 @@ struct Linear {
     }
 };
 
-// activations as rows of `width`: the pointer and pitch the library takes (a packed copy where the layout does not allow it)
+// activations as rows of `width`: the pointer and pitch the library takes.  Rows that lie a fixed pitch apart over all leading
+// dimensions are read where they are (a slice of a wider last dimension, any number of dimensions); other layouts, and pitches
+// or addresses that are no multiple of 16 bytes, take a packed copy.
 struct Rows {
     Tensor keep;
     const void* ptr = nullptr;
     int64_t ld = 0, M = 0;
 
+    static bool pitched(const Tensor& x, int64_t* pitch) {
+        if (x.stride(-1) != 1 || (uintptr_t)x.data_ptr() % 16 != 0) return false;
+        int64_t rows = 1;                                          // of the dimensions looked at, the innermost first
+        for (int64_t d = x.dim() - 2; d >= 0; --d) {
+            if (x.size(d) == 1) continue;
+            if (rows == 1) *pitch = x.stride(d);
+            else if (x.stride(d) != *pitch * rows) return false;
+            rows *= x.size(d);
+        }
+        return rows == 1 || *pitch % 8 == 0;
+    }
+
     Rows(const Tensor& x, int64_t width) {
         M = width ? x.numel() / width : 0;
         ld = width;
         keep = x;
-        if (!x.is_contiguous()) {
-            if (x.dim() == 2 && x.stride(1) == 1 && (x.size(0) == 1 || x.stride(0) % 8 == 0) && (uintptr_t)x.data_ptr() % 16 == 0) {
-                if (M > 1) ld = x.stride(0);
-            } else {
-                keep = x.contiguous();
-            }
+        if (!x.is_contiguous() && !pitched(x, &ld)) {
+            keep = x.contiguous();
+            ld = width;
         }
         ptr = keep.data_ptr();
     }

@@ -202,3 +202,74 @@ def test_strided_activations_are_read_in_place(hip_device, both_paths):
         for t in (x.transpose(0, 1), wide[:, ::3, :K], odd[:, :K], wide[..., 4:K + 4]):
             for a, b in zip(both_paths(lambda: [m(t)]), [m(t.contiguous())]):
                 assert torch.equal(a, b)
+
+
+def test_overridden_methods_are_called(hip_device, monkeypatch):
+    """What a subclass, an instance or a patched class puts in the place of the methods that the native path stands for runs, in the
+    module call, the joint call and the MLP; a subclass that replaces nothing stays native."""
+    from xorl_amd._native import native
+    from xorl_amd.qlora import Int4QLoRALinear, qlora_linears_forward, qlora_mlp_forward
+
+    def module(cls, seed, n=256, k=256):
+        m, _ = make_dense_module("int4", n, k, 16, 32, seed, hip_device)
+        m.__class__ = cls
+        return m
+
+    class Same(Int4QLoRALinear):
+        def extra_repr(self):
+            return "same"
+
+    class NoUpdate(Int4QLoRALinear):
+        def _active_scaling(self):
+            return 0.0
+
+    class Other(Int4QLoRALinear):
+        def _forward_quant_weight(self):
+            return self.other._quant_weight()
+
+    class Held(Int4QLoRALinear):
+        @property
+        def lora_B(self):
+            return self._parameters["lora_B"] * 0.0
+
+    x = gen((4, 256), 1.0, 4, torch.bfloat16).to(hip_device)
+    with torch.no_grad():
+        plain, other = module(Int4QLoRALinear, 3), module(Int4QLoRALinear, 5)
+        want, base = plain(x), module(Int4QLoRALinear, 3)
+        base.lora_B.zero_()
+        base = base(x)
+        assert not torch.equal(want, base)
+        assert native().linear(module(Same, 3), x) is not None
+        for cls in (NoUpdate, Held):
+            m = module(cls, 3)
+            assert torch.equal(m(x), base)
+            assert torch.equal(qlora_linears_forward([m, m], x)[1], base)
+            assert torch.equal(qlora_mlp_forward(plain, plain, m, x), qlora_mlp_forward(plain, plain, m.eval(), x))
+            assert native().mlp(plain, plain, m, x) is None
+        m = module(Other, 3)
+        object.__setattr__(m, "other", other)
+        copy = module(Int4QLoRALinear, 5)
+        copy.lora_A.copy_(m.lora_A)
+        copy.lora_B.copy_(m.lora_B)
+        assert torch.equal(m(x), copy(x))
+        m = module(Int4QLoRALinear, 3)
+        m._active_scaling = lambda: 0.0
+        assert torch.equal(m(x), base)
+        with monkeypatch.context() as mp:
+            mp.setattr(Int4QLoRALinear, "_active_scaling", lambda self: 0.0)
+            assert torch.equal(plain(x), base)
+        assert torch.equal(plain(x), want)
+
+    e, _ = _make_experts("block_fp8", 4, 256, 256, 8, False, 7, hip_device)
+    rw, sel = _zipf_routing(40, 4, 2, seed=2)
+    rw, sel = rw.to(hip_device), sel.long().to(hip_device)
+    x = gen((40, 256), 1.0, 4, torch.bfloat16).to(hip_device)
+    with torch.no_grad():
+        want = e(x, rw, sel)
+        e._active_scaling = lambda: 0.0
+        got = e(x, rw, sel)
+        assert native().moe(e, x, rw, sel, False) is None and not torch.equal(got, want)
+        del e._active_scaling
+        for p in e.get_lora_parameters():
+            p.zero_()
+        assert torch.equal(got, e(x, rw, sel))

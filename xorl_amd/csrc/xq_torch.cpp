@@ -8,7 +8,7 @@
 //
 // Every entry point returns None where anything is out of the ordinary (tensor subclasses, sharded or CPU state, tangents of
 // forward-mode differentiation, function transforms, a trace being recorded, quantization noise, an active rank below the
-// stored one, unexpected dtypes or layouts): the caller then takes its Python path, which also raises the argument errors.
+// stored one, unexpected dtypes or layouts, a module that defines for itself what is read or done here): the caller then takes its Python path, which also raises the argument errors.
 // Nothing is remembered from one call to the next, and a backward takes the addresses of the packed weights anew from
 // their tensors: storage may have been freed and filled again between the two.
 #include <Python.h>
@@ -45,8 +45,14 @@ using torch::autograd::variable_list;
 // ---- names and classes handed over by the Python side (init)
 PyObject* g_error = nullptr;            // xorl_amd._C.XqError
 PyObject* g_functional = nullptr;       // the dict of xorl_amd.functional: SKINNY_CHECK_EVERY, skinny_status
-PyTypeObject* g_linear_type = nullptr;  // QLoRALinear
-PyTypeObject* g_experts_type = nullptr; // QLoRAMoeExperts
+
+// a module class and the methods whose work is done here in their place, as the class defines them
+struct Program {
+    PyTypeObject* type = nullptr;
+    std::vector<PyObject*> name, method;
+};
+constexpr int kFormats = XQ_FMT_NF4 + 1;
+Program g_linear[kFormats], g_experts[kFormats];      // by format; no type: no such class
 
 #define XQ_NAMES(F)                                                                                                       \
     F(_parameters) F(_buffers) F(lora_A) F(lora_B) F(bias) F(packed_weight_f32) F(weight_scales) F(weight_block_scales)   \
@@ -55,7 +61,8 @@ PyTypeObject* g_experts_type = nullptr; // QLoRAMoeExperts
     F(intermediate_size) F(use_rslora) F(swiglu_limit) F(moe_implementation) F(gate) F(up) F(down) F(gate_packed)         \
     F(up_packed) F(down_packed) F(gate_block_scales) F(up_block_scales) F(down_block_scales) F(gate_scales) F(up_scales)  \
     F(down_scales) F(gate_global_scale) F(up_global_scale) F(down_global_scale) F(gate_proj_lora_A) F(gate_proj_lora_B)   \
-    F(up_proj_lora_A) F(up_proj_lora_B) F(down_proj_lora_A) F(down_proj_lora_B) F(SKINNY_CHECK_EVERY) F(skinny_status)
+    F(up_proj_lora_A) F(up_proj_lora_B) F(down_proj_lora_A) F(down_proj_lora_B) F(SKINNY_CHECK_EVERY) F(skinny_status)     \
+    F(__getattr__) F(__getattribute__)
 #define XQ_DECLARE(n) PyObject* s_##n;
 struct Names { XQ_NAMES(XQ_DECLARE) } N;
 #undef XQ_DECLARE
@@ -65,6 +72,21 @@ PyObject* get(PyObject* dict, PyObject* name) { return dict ? PyDict_GetItem(dic
 PyObject* dict_of(PyObject* module) {
     PyObject** p = _PyObject_GetDictPtr(module);
     return p ? *p : nullptr;
+}
+
+// whether the methods of `p` are the ones that run on `module` (no subclass, instance attribute or patch replaces one) and, in
+// a subclass, whether what is read from the module's dictionaries is what attribute access gives (no property, no __getattr__
+// of its own).  The library's own classes: 4-6 look-ups in the type's method cache and as many in the instance's dictionary.
+bool as_defined(PyObject* module, PyObject* dict, const Program& p) {
+    if (!p.type || !PyObject_TypeCheck(module, p.type)) return false;
+    PyTypeObject* type = Py_TYPE(module);
+    for (size_t i = 0; i < p.name.size(); ++i)
+        if (_PyType_Lookup(type, p.name[i]) != p.method[i] || get(dict, p.name[i])) return false;
+    if (type == p.type) return true;
+#define XQ_SAME(n) if (_PyType_Lookup(type, N.s_##n) != _PyType_Lookup(p.type, N.s_##n)) return false;
+    XQ_NAMES(XQ_SAME)
+#undef XQ_SAME
+    return true;
 }
 
 bool get_int(PyObject* dict, PyObject* name, int64_t* out) {
@@ -189,7 +211,6 @@ struct Linear {
     const void* bias_ptr() const { return bias.defined() ? bias.data_ptr() : nullptr; }
 
     bool read(PyObject* module) {
-        if (!PyObject_TypeCheck(module, g_linear_type)) return false;
         PyObject* d = dict_of(module);
         PyObject *params = get(d, N.s__parameters), *bufs = get(d, N.s__buffers), *sdt = get(d, N.s__scale_dtypes);
         if (!params || !bufs || !sdt || !PyDict_Check(sdt)) return false;
@@ -198,7 +219,7 @@ struct Linear {
         const int fmt = format_code(get(d, N.s_quant_format));
         int64_t rank, group, n, k;
         double alpha;
-        if (fmt < 0 || !get_int(d, N.s_active_r, &rank) || !get_number(d, N.s_active_lora_alpha, &alpha) ||
+        if (fmt < 0 || !as_defined(module, d, g_linear[fmt]) || !get_int(d, N.s_active_r, &rank) || !get_number(d, N.s_active_lora_alpha, &alpha) ||
             !get_int(d, N.s_quant_group_size, &group) || !get_int(d, N.s_out_features, &n) || !get_int(d, N.s_in_features, &k))
             return false;
         PyObject* packed_o = get(params, N.s_packed_weight_f32);
@@ -671,14 +692,14 @@ PyObject* moe(PyObject*, PyObject* const* args, Py_ssize_t n) {
         if (n != 5) { PyErr_SetString(PyExc_TypeError, "moe(module, x, routing_weights, selected_experts, streaming)"); return nullptr; }
         const bool streaming = args[4] == Py_True;
         const Tensor *x = plain(args[1]), *rw = plain(args[2]), *sel = plain(args[3]);
-        if (under_transform() || !x || !rw || !sel || !PyObject_TypeCheck(args[0], g_experts_type)) XQ_NONE;
+        if (under_transform() || !x || !rw || !sel) XQ_NONE;
         PyObject* d = dict_of(args[0]);
         PyObject *params = get(d, N.s__parameters), *bufs = get(d, N.s__buffers), *sdt = get(d, N.s__scale_dtypes);
         PyObject* impl = get(d, N.s_moe_implementation);
         const int fmt = format_code(get(d, N.s_quant_format));
         int64_t rank, group, E, local, H, I;
         double alpha, limit = 0;
-        if (!params || !bufs || !sdt || !PyDict_Check(sdt) || fmt < 0 || !impl || !PyUnicode_Check(impl) ||
+        if (!params || !bufs || !sdt || !PyDict_Check(sdt) || fmt < 0 || !as_defined(args[0], d, g_experts[fmt]) || !impl || !PyUnicode_Check(impl) ||
             PyUnicode_CompareWithASCIIString(impl, "eager") == 0 || !get_int(d, N.s_active_r, &rank) ||
             !get_number(d, N.s_active_lora_alpha, &alpha) || !get_int(d, N.s_quant_group_size, &group) || !get_int(d, N.s_num_experts, &E) ||
             !get_int(d, N.s_num_local_experts, &local) || local != E || !get_int(d, N.s_hidden_size, &H) ||
@@ -786,17 +807,40 @@ PyObject* moe(PyObject*, PyObject* const* args, Py_ssize_t n) {
     });
 }
 
-// init(XqError, dict of xorl_amd.functional, QLoRALinear, QLoRAMoeExperts)
+// {format: (class, ((method name, method), ...))} -> programs by format
+bool fill_programs(PyObject* table, Program* out) {
+    PyObject *key, *entry;
+    for (Py_ssize_t at = 0; PyDict_Next(table, &at, &key, &entry);) {
+        const int fmt = format_code(key);
+        PyObject *type, *methods;
+        if (fmt < 0 || !PyArg_ParseTuple(entry, "O!O!", &PyType_Type, &type, &PyTuple_Type, &methods)) return false;
+        Program p;
+        p.type = (PyTypeObject*)type;
+        for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(methods); ++i) {
+            PyObject *name, *method;
+            if (!PyArg_ParseTuple(PyTuple_GET_ITEM(methods, i), "UO", &name, &method)) return false;
+            Py_INCREF(name);
+            PyUnicode_InternInPlace(&name);
+            Py_INCREF(method);
+            p.name.push_back(name);
+            p.method.push_back(method);
+        }
+        Py_INCREF(type);
+        out[fmt] = p;
+    }
+    return true;
+}
+
+// init(XqError, dict of xorl_amd.functional, programs of the linear modules, programs of the expert modules)
 PyObject* init(PyObject*, PyObject* const* args, Py_ssize_t n) {
-    if (n != 4 || !PyDict_Check(args[1]) || !PyType_Check(args[2]) || !PyType_Check(args[3])) {
-        PyErr_SetString(PyExc_TypeError, "init(error class, dict, QLoRALinear, QLoRAMoeExperts)");
+    if (n != 4 || !PyDict_Check(args[1]) || !PyDict_Check(args[2]) || !PyDict_Check(args[3]) || !fill_programs(args[2], g_linear) ||
+        !fill_programs(args[3], g_experts)) {
+        PyErr_SetString(PyExc_TypeError, "init(error class, dict, linear programs, expert programs)");
         return nullptr;
     }
-    for (Py_ssize_t i = 0; i < n; ++i) Py_INCREF(args[i]);
+    for (Py_ssize_t i = 0; i < 2; ++i) Py_INCREF(args[i]);
     g_error = args[0];
     g_functional = args[1];
-    g_linear_type = (PyTypeObject*)args[2];
-    g_experts_type = (PyTypeObject*)args[3];
 #define XQ_INTERN(m) N.s_##m = PyUnicode_InternFromString(#m);
     XQ_NAMES(XQ_INTERN)
 #undef XQ_INTERN

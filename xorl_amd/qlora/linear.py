@@ -31,7 +31,7 @@ from torch import Tensor
 
 from .. import _C
 from .. import quantize as Q
-from .._native import native
+from .._native import native, program
 from ..functional import MAX_FUSED_RANK, QuantWeight, qlora_linear
 
 
@@ -792,6 +792,15 @@ class NF4QLoRALinear(QLoRALinear):
 
     def _load_prequantized(self, _load_tensor) -> None:
         raise NotImplementedError("NF4 has no pre-quantized checkpoint format; use from_module() on bf16 weights")
+
+
+_NATIVE_METHODS = ("_forward_quant_weight", "_quant_weight", "_read_packed_weight_uint8", "_active_scaling")
+NATIVE_PROGRAMS = {
+    "block_fp8": program(BlockFP8QLoRALinear, *_NATIVE_METHODS),
+    "nvfp4": program(NvFP4QLoRALinear, *_NATIVE_METHODS, "_scales", "_recover_tensor"),
+    "int4": program(Int4QLoRALinear, *_NATIVE_METHODS),
+    "nf4": program(NF4QLoRALinear, *_NATIVE_METHODS),
+}
 
 
 # =============================================================================

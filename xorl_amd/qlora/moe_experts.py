@@ -20,7 +20,7 @@ from torch import Tensor
 from .. import _C
 from .. import moe_functional as MF
 from .. import quantize as Q
-from .._native import native
+from .._native import native, program
 from ..functional import QuantWeight
 from ..moe_functional import moe_experts_qlora_ep_compute, moe_experts_qlora_forward
 from .linear import LoraModule
@@ -623,3 +623,8 @@ class NF4QLoRAMoeExperts(QLoRAMoeExperts):
         out = torch.empty(self.num_local_experts, K, N, dtype=torch.bfloat16, device=getattr(self, f"{proj_name}_packed").device)
         _C.check(_C.lib().xq_decode(ctypes.byref(w), out.data_ptr(), _C.XQ_DT_BF16, _C.stream_ptr(out.device)))
         return out
+
+
+NATIVE_PROGRAMS = {
+    fmt: program(cls, "_bank", "_proj_dims", "_recover_tensor", "_active_lora_views", "_active_scaling")
+    for fmt, cls in (("block_fp8", BlockFP8QLoRAMoeExperts), ("nvfp4", NvFP4QLoRAMoeExperts), ("nf4", NF4QLoRAMoeExperts))}

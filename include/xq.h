@@ -194,8 +194,11 @@ int xq_decode(const xq_weight* w, void* out, int out_dtype, void* stream);
  * the split-K product; under many rows (640 and more) also room for the weight
  * decoded once to bf16.  That room is optional: a call without it decodes in
  * the tiles.  With r == 0 the whole workspace is optional: a call without it
- * (or with fewer bytes) runs the product unsplit. */
+ * (or with fewer bytes) runs the product unsplit.  The _fmt form knows the
+ * format of the weight (XQ_FMT_*; < 0: any) and leaves out the room for an image
+ * that this format does not use at that size (block-fp8 below 6144 rows). */
 int64_t xq_linear_workspace_bytes(int64_t M, int64_t N, int64_t K, int r);
+int64_t xq_linear_workspace_bytes_fmt(int format, int64_t M, int64_t N, int64_t K, int r);
 
 /* y[M,N] = x[M,K] . deq(W)^T + bias + s * (x . A^T) . B^T      (bf16 out)
  *   lora_A [r,K], lora_B [N,r] in lora_dtype (fp32 or bf16), r in {0..64};
@@ -217,6 +220,7 @@ int xq_linear_fwd(const xq_weight* w, const void* x, int64_t ldx, int64_t M,
  * Otherwise the two calls run one after the other inside this one (gate | up goes through the workspace).
  * workspace: xq_linear_fwd_swiglu_workspace_bytes(M, 2 I, K, r) bytes, 256-byte aligned. */
 int64_t xq_linear_fwd_swiglu_workspace_bytes(int64_t M, int64_t N2, int64_t K, int r);
+int64_t xq_linear_fwd_swiglu_workspace_bytes_fmt(int format, int64_t M, int64_t N2, int64_t K, int r);
 int xq_linear_fwd_swiglu(const xq_weight* w, const void* x, int64_t ldx, int64_t M,
                          const void* lora_A, const void* lora_B, int lora_dtype, int r, float scaling,
                          const void* bias_bf16, void* h, int64_t ldh, void* workspace, int64_t workspace_bytes, void* stream);
@@ -590,7 +594,9 @@ typedef struct xq_mlp_grads {
     float* dB[3];
 } xq_mlp_grads;
 
+/* (the _fmt form: the format that gate, up and down share, < 0 otherwise; see xq_linear_workspace_bytes) */
 int64_t xq_mlp_workspace_bytes(int64_t M, int64_t hidden, int64_t intermediate, int r, int backward);
+int64_t xq_mlp_workspace_bytes_fmt(int format, int64_t M, int64_t hidden, int64_t intermediate, int r, int backward);
 int xq_mlp_fwd(const xq_weight* gate, const xq_weight* up, const xq_weight* down, const xq_mlp_lora* lora,
                const void* x, int64_t ldx, int64_t M, void* y, int64_t ldy, xq_mlp_saved* saved,
                void* workspace, int64_t workspace_bytes, void* stream);
@@ -605,6 +611,7 @@ int xq_mlp_bwd(const xq_weight* gate, const xq_weight* up, const xq_weight* down
  * points are those of the separate module calls.  The intermediate gate|up and h live in the workspace
  * (xq_mlp_infer_workspace_bytes(...) bytes, 256-byte aligned). */
 int64_t xq_mlp_infer_workspace_bytes(int64_t M, int64_t hidden, int64_t intermediate, int r);
+int64_t xq_mlp_infer_workspace_bytes_fmt(int format, int64_t M, int64_t hidden, int64_t intermediate, int r);
 int xq_mlp_fwd_infer(const xq_weight* gate, const xq_weight* up, const xq_weight* down, const xq_mlp_lora* lora,
                      const void* x, int64_t ldx, int64_t M, void* y, int64_t ldy, void* workspace,
                      int64_t workspace_bytes, void* stream);

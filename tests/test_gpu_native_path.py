@@ -273,3 +273,24 @@ def test_overridden_methods_are_called(hip_device, monkeypatch):
         for p in e.get_lora_parameters():
             p.zero_()
         assert torch.equal(got, e(x, rw, sel))
+
+
+def test_block_fp8_calls_take_no_memory_for_an_image(hip_device):
+    """Below 6144 rows a block-fp8 weight is not decoded first: a module call's scratch stays below the decoded weight's size."""
+    from xorl_amd.qlora import QLoRALinear
+
+    M, N, K = 2048, 12288, 4096
+    x = torch.randn(M, K, dtype=torch.bfloat16, device=hip_device)
+    lin = torch.nn.Linear(K, N, bias=False, dtype=torch.bfloat16, device=hip_device)
+    for fmt, image in (("block_fp8", False), ("int4", True)):
+        m = QLoRALinear.from_module(lin, r=16, lora_alpha=32, quant_format=fmt)
+        with torch.no_grad():
+            y = m(x)
+            torch.cuda.synchronize()
+            del y
+            before = torch.cuda.memory_allocated()
+            torch.cuda.reset_peak_memory_stats()
+            y = m(x)
+            torch.cuda.synchronize()
+        scratch = torch.cuda.max_memory_allocated() - before - y.numel() * 2
+        assert (scratch >= 2 * N * K) == image, (fmt, scratch)

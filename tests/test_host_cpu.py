@@ -146,3 +146,30 @@ def test_skinny_plan_holds_any_contraction(M, steps):
             if K >= 1024:
                 need = -(-K // (128 * steps)) * M * N * 4 + K // 128 * M * 16 * 4
                 assert _C.lib().xq_linear_workspace_bytes(M, N, K, 16) >= need, (M, K)
+
+
+def test_workspace_holds_an_image_only_where_the_format_uses_one():
+    """Several forwards in one call know their weights, the _fmt queries the format: room for a decoded weight (two bytes an element)
+    is asked for 4-bit weights from 640 rows on and for block-fp8 ones from 6144 on; without a format it is the largest of all."""
+    from xorl_amd import _C
+
+    L, N, K = _C.lib(), 12288, 4096
+    image = 2 * N * K
+    for M in (639, 640, 2048, 6143, 6144, 8192):
+        sizes = {}
+        for fmt, code in _C.FORMATS.items():
+            sizes[fmt] = s = [L.xq_linear_workspace_bytes_fmt(code, M, N, K, 16), L.xq_linear_fwd_swiglu_workspace_bytes_fmt(code, M, N, K, 16) - 2 * M * N,
+                              L.xq_mlp_workspace_bytes_fmt(code, M, K, N, 16, 0), L.xq_mlp_infer_workspace_bytes_fmt(code, M, K, N, 16) - 6 * M * N]
+            w = _C.XqWeight()
+            w.format, w.rows, w.cols, w.num_experts = code, N, K, 1
+            job = _C.XqLinearJob(ctypes.pointer(w), None, None, 16, 1.0, None, None, N)
+            s.append(L.xq_linear_fwd_multi_workspace_bytes(ctypes.byref(job), 1, M))
+            for b in s:
+                assert (b >= image) == (M >= (6144 if fmt == "block_fp8" else 640)), (fmt, M, s)
+            bwd = L.xq_mlp_workspace_bytes_fmt(code, M, K, N, 16, 1)
+            assert bwd <= L.xq_mlp_workspace_bytes(M, K, N, 16, 1)
+            sizes[fmt].append(bwd)
+        any_fmt = [L.xq_linear_workspace_bytes(M, N, K, 16), L.xq_linear_fwd_swiglu_workspace_bytes(M, N, K, 16) - 2 * M * N,
+                   L.xq_mlp_workspace_bytes(M, K, N, 16, 0), L.xq_mlp_infer_workspace_bytes(M, K, N, 16) - 6 * M * N]
+        assert any_fmt == [max(s[i] for s in sizes.values()) for i in range(4)]
+        assert L.xq_mlp_workspace_bytes(M, K, N, 16, 1) == max(s[5] for s in sizes.values())

@@ -97,9 +97,11 @@ _SIGNATURES = {
     # format, layout, x, x_dtype, rows, cols, group, amax_scale, global_amax, codes, scales, scale_dtype, global_scale, ws, ws_bytes, stream
     "xq_quantize": (_INT, [_INT, _INT, _P, _INT, _I64, _I64, _I32, _F, _P, _P, _P, _INT, _P, _P, _I64, _P]),
     "xq_linear_workspace_bytes": (_I64, [_I64, _I64, _I64, _INT]),
+    "xq_linear_workspace_bytes_fmt": (_I64, [_INT, _I64, _I64, _I64, _INT]),
     # w, x, ldx, M, A, B, lora_dtype, r, scaling, bias, y, ldy, su_out, ws, ws_bytes, stream
     "xq_linear_fwd": (_INT, [_W, _P, _I64, _I64, _P, _P, _INT, _INT, _F, _P, _P, _I64, _P, _P, _I64, _P]),
     "xq_linear_fwd_swiglu_workspace_bytes": (_I64, [_I64, _I64, _I64, _INT]),
+    "xq_linear_fwd_swiglu_workspace_bytes_fmt": (_I64, [_INT, _I64, _I64, _I64, _INT]),
     # w, x, ldx, M, A, B, lora_dtype, r, scaling, bias, h, ldh, ws, ws_bytes, stream
     "xq_linear_fwd_swiglu": (_INT, [_W, _P, _I64, _I64, _P, _P, _INT, _INT, _F, _P, _P, _I64, _P, _I64, _P]),
     # jobs, n_jobs, M
@@ -173,7 +175,9 @@ _SIGNATURES = {
     "xq_grouped_fwd_infer": (_INT, [_W, _W, _W, ctypes.POINTER(XqGroupedLora), _P, _I64, _I64, _P, _INT, _P, _I32, _P, _I64,
                                     _P, _I64, _P]),
     "xq_mlp_workspace_bytes": (_I64, [_I64, _I64, _I64, _INT, _INT]),
+    "xq_mlp_workspace_bytes_fmt": (_I64, [_INT, _I64, _I64, _I64, _INT, _INT]),
     "xq_mlp_infer_workspace_bytes": (_I64, [_I64, _I64, _I64, _INT]),
+    "xq_mlp_infer_workspace_bytes_fmt": (_I64, [_INT, _I64, _I64, _I64, _INT]),
     # gate, up, down, lora, x, ldx, M, y, ldy, ws, ws_bytes, stream
     "xq_mlp_fwd_infer": (_INT, [_W, _W, _W, ctypes.POINTER(XqMlpLora), _P, _I64, _I64, _P, _I64, _P, _I64, _P]),
     # gate, up, down, lora, x, ldx, M, y, ldy, saved, ws, ws_bytes, stream

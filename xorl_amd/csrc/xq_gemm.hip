@@ -209,8 +209,9 @@ static bool decode_first(int fmt, int64_t n_rows, int64_t Nout, int64_t Kc) {
     return n_rows >= (fmt == XQ_FMT_FP8 ? kDecMinRowsFp8 : kDecMinRows) && (double)n_rows * (double)Nout * (double)Kc >= kDecMinWork &&
            Kc % 64 == 0 && Kc >= 128 && Nout % 16 == 0;
 }
-static int64_t decoded_scratch_bytes(int64_t n_rows, int64_t Nout, int64_t Kc) {      // (whatever the format: its callers know only sizes)
-    return decode_first(XQ_FMT_INT4, n_rows, Nout, Kc) ? dec_image_bytes(Nout, Kc) + plan_decoded(n_rows, Nout, Kc).partial : 0;
+// (fmt < 0: whatever the format; the 4-bit rule covers all)
+static int64_t decoded_scratch_bytes(int fmt, int64_t n_rows, int64_t Nout, int64_t Kc) {
+    return decode_first(fmt < 0 ? XQ_FMT_INT4 : fmt, n_rows, Nout, Kc) ? dec_image_bytes(Nout, Kc) + plan_decoded(n_rows, Nout, Kc).partial : 0;
 }
 
 // fp32 partial-sum bytes the split-K forms of a dense [n_rows, Nout] product over Kc may want, under any tile policy
@@ -228,11 +229,11 @@ int64_t tile_gemm_split_bytes(int64_t n_rows, int64_t Nout, int64_t Kc) {
     return elems * Nout * 4;
 }
 
-// scratch a dense launch may want: the above, or the decoded image of a 4-bit weight with the sums of its splits (without
-// room for those the launch decodes in the tile kernel)
-int64_t tile_gemm_partial_bytes(int64_t n_rows, int64_t Nout, int64_t Kc) {
+// scratch a dense launch of this format (< 0: of any) may want: the above, or the decoded image of the weight with the sums of
+// its splits (without room for those the launch decodes in the tile kernel)
+int64_t tile_gemm_partial_bytes(int fmt, int64_t n_rows, int64_t Nout, int64_t Kc) {
     if (n_rows <= 0 || Kc % BK) return 0;
-    return std::max(tile_gemm_split_bytes(n_rows, Nout, Kc), decoded_scratch_bytes(n_rows, Nout, Kc));
+    return std::max(tile_gemm_split_bytes(n_rows, Nout, Kc), decoded_scratch_bytes(fmt, n_rows, Nout, Kc));
 }
 
 // Whether a grouped launch on this bank may take a second bank of the same shape (see G256Args::W2): block-fp8 on the
@@ -378,7 +379,7 @@ static int launch_tile_gemm_t(const xq_weight* w, bool contract_cols, const bf16
         const int T = force_T ? force_T : g_tile_policy == 2 ? 256 : g_tile_policy == 3 ? 128 : grouped ? (big ? 256 : 128) : plan.T;
         if ((planned || (two_dense && g_tile_policy == 0)) && (w->format != XQ_FMT_FP8 || g_fp8_direct) &&
             decode_first(w->format, n_rows, g.Nout, g.Kc) && partial && xq_aligned(partial, 16) &&
-            partial_bytes >= decoded_scratch_bytes(n_rows, g.Nout, g.Kc) && n_rows * lda * 2 < (1ll << 32) && xq_cdiv(n_rows, 256) * xq_cdiv(g.Nout, 256) < (1ll << 31) && g.Nout < 65536 * 16) {
+            partial_bytes >= decoded_scratch_bytes(w->format, n_rows, g.Nout, g.Kc) && n_rows * lda * 2 < (1ll << 32) && xq_cdiv(n_rows, 256) * xq_cdiv(g.Nout, 256) < (1ll << 31) && g.Nout < 65536 * 16) {
             G256Args f{};
             f.A = A; f.lda = lda; f.C = C; f.ldc = ldc;
             f.W = g.packed; f.scales = g.scales; f.global_scale = g.global_scale;
@@ -599,9 +600,12 @@ extern "C" int xq_set_persistent_tiles(int enabled) {
     return XQ_OK;
 }
 
-// what a call must bring (`part` = tile_gemm_split_bytes) and what it is told to bring (tile_gemm_partial_bytes: with room for
-// the decoded image of a 4-bit weight under many rows)
-static int64_t linear_workspace(int64_t M, int64_t N, int64_t K, int r, int64_t (*part)(int64_t, int64_t, int64_t)) {
+// what a call must bring (`needed`) and what it is told to bring (with room for the decoded image of a weight of that format, or
+// of any, under many rows)
+static int64_t linear_workspace(int fmt, int64_t M, int64_t N, int64_t K, int r, bool needed) {
+    auto part = [&](int64_t rows, int64_t out, int64_t kc) {
+        return needed ? tile_gemm_split_bytes(rows, out, kc) : tile_gemm_partial_bytes(fmt, rows, out, kc);
+    };
     int rp = r_pad_of(r);
     int64_t skinny = M <= 64 ? skinny_workspace_bytes(M, N, K, rp) : 0;
     // scratch of the forward (output N, contraction K) and of the dgrad (output K, contraction N)
@@ -617,8 +621,9 @@ static int64_t linear_workspace(int64_t M, int64_t N, int64_t K, int r, int64_t 
     }
     return need > skinny ? need : skinny;
 }
-static int64_t linear_workspace_needed(int64_t M, int64_t N, int64_t K, int r) { return linear_workspace(M, N, K, r, tile_gemm_split_bytes); }
-extern "C" int64_t xq_linear_workspace_bytes(int64_t M, int64_t N, int64_t K, int r) { return linear_workspace(M, N, K, r, tile_gemm_partial_bytes); }
+static int64_t linear_workspace_needed(int64_t M, int64_t N, int64_t K, int r) { return linear_workspace(-1, M, N, K, r, true); }
+extern "C" int64_t xq_linear_workspace_bytes(int64_t M, int64_t N, int64_t K, int r) { return linear_workspace(-1, M, N, K, r, false); }
+extern "C" int64_t xq_linear_workspace_bytes_fmt(int format, int64_t M, int64_t N, int64_t K, int r) { return linear_workspace(format, M, N, K, r, false); }
 
 static int check_dense(const xq_weight* w, const char* who) {
     int rc = xq_validate_weight(w, who);
@@ -701,9 +706,12 @@ static int static_scratch(void** out, const char* who) {
 
 extern "C" int64_t xq_static_scratch_bytes(void) { return XQ_STATIC_SCRATCH_BYTES; }
 
-extern "C" int64_t xq_linear_fwd_swiglu_workspace_bytes(int64_t M, int64_t N2, int64_t K, int r) {
+extern "C" int64_t xq_linear_fwd_swiglu_workspace_bytes_fmt(int format, int64_t M, int64_t N2, int64_t K, int r) {
     if (M < 0 || N2 < 0) return 0;
-    return align256(xq_linear_workspace_bytes(M, N2, K, r)) + align256(M * N2 * 2) + 256;
+    return align256(xq_linear_workspace_bytes_fmt(format, M, N2, K, r)) + align256(M * N2 * 2) + 256;
+}
+extern "C" int64_t xq_linear_fwd_swiglu_workspace_bytes(int64_t M, int64_t N2, int64_t K, int r) {
+    return xq_linear_fwd_swiglu_workspace_bytes_fmt(-1, M, N2, K, r);
 }
 
 extern "C" int xq_linear_fwd_swiglu(const xq_weight* w, const void* x, int64_t ldx, int64_t M, const void* lora_A, const void* lora_B,
@@ -719,7 +727,7 @@ extern "C" int xq_linear_fwd_swiglu(const xq_weight* w, const void* x, int64_t l
     XQ_REQUIRE(lora_dtype == XQ_DT_F32 || lora_dtype == XQ_DT_BF16, "xq_linear_fwd_swiglu: bad lora_dtype");
     if (M == 0) return XQ_OK;
     XQ_REQUIRE(ldh % 8 == 0 && xq_aligned(h, 16), "xq_linear_fwd_swiglu: h rows must be 16-byte aligned");
-    XQ_REQUIRE(workspace && xq_aligned(workspace, 256) && workspace_bytes >= xq_linear_fwd_swiglu_workspace_bytes(M, N2, K, r),
+    XQ_REQUIRE(workspace && xq_aligned(workspace, 256) && workspace_bytes >= xq_linear_fwd_swiglu_workspace_bytes_fmt(w->format, M, N2, K, r),
                "xq_linear_fwd_swiglu: workspace missing, misaligned or smaller than xq_linear_fwd_swiglu_workspace_bytes()");
     hipStream_t stream = (hipStream_t)stream_;
     // decode sizes: one launch that holds a column's gate and up rows in the same block
@@ -738,7 +746,7 @@ extern "C" int xq_linear_fwd_swiglu(const xq_weight* w, const void* x, int64_t l
         }
     }
     // otherwise the forward into the workspace, then the elementwise kernel
-    const int64_t lin = align256(xq_linear_workspace_bytes(M, N2, K, r));
+    const int64_t lin = align256(xq_linear_workspace_bytes_fmt(w->format, M, N2, K, r));
     bf16_t* gu = (bf16_t*)((uint8_t*)workspace + lin);
     if ((rc = xq_linear_fwd(w, x, ldx, M, lora_A, lora_B, lora_dtype, r, scaling, bias_bf16, gu, N2, nullptr, workspace, lin, stream_))) return rc;
     return xq_silu_mul_fwd(gu, gu + I, N2, nullptr, h, ldh, M, I, stream_);
@@ -749,7 +757,7 @@ extern "C" int64_t xq_linear_fwd_multi_workspace_bytes(const xq_linear_job* jobs
     if (!jobs) return need;
     for (int i = 0; i < n_jobs; ++i) {
         if (!jobs[i].w) continue;
-        const int64_t b = xq_linear_workspace_bytes(M, jobs[i].w->rows, jobs[i].w->cols, jobs[i].r);
+        const int64_t b = xq_linear_workspace_bytes_fmt(jobs[i].w->format, M, jobs[i].w->rows, jobs[i].w->cols, jobs[i].r);
         if (b > need) need = b;
         if (M <= 64) joint += skinny_workspace_bytes(M, jobs[i].w->rows, jobs[i].w->cols, r_pad_of(jobs[i].r));   // side by side in a joint launch
     }

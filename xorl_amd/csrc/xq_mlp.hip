@@ -101,13 +101,17 @@ int check_call(const xq_weight* gate, const xq_weight* up, const xq_weight* down
 }
 
 // one region of split-K partial sums and fp32 sums of the SwiGLU passes (stream order)
-// (`needed`: what a call must bring; without it what it is told to bring, room for decoded 4-bit weights included)
-int64_t gemm_part_bytes(const Dims& d, bool needed) {
-    auto part = needed ? tile_gemm_split_bytes : tile_gemm_partial_bytes;
+// (`needed`: what a call must bring; without it what it is told to bring, room for decoded weights of that format, or of any,
+// included)
+int64_t gemm_part_bytes(const Dims& d, int fmt, bool needed, bool backward) {
+    auto part = [&](int64_t rows, int64_t out, int64_t kc) {
+        return needed ? tile_gemm_split_bytes(rows, out, kc) : tile_gemm_partial_bytes(fmt, rows, out, kc);
+    };
     const int64_t pa = part(d.M, d.I, d.H), pb = part(d.M, d.H, d.I);
     const int64_t ps = d.rp && silu_bwd_nt_supported(d.I, d.rp) ? silu_nt_partial_bytes(d.M, d.I, d.rp) : 0;
-    // (the dgrad of gate and up as one sum: the contraction is twice as long)
-    const int64_t p2 = needed ? 0 : tile_gemm_partial_bytes(d.M, d.H, 2 * d.I);
+    // the dgrad of block-fp8 gate and up as one sum: the contraction is twice as long
+    const bool joint = backward && !needed && (fmt < 0 || fmt == XQ_FMT_FP8) && 2 * d.rp <= 64;
+    const int64_t p2 = joint ? tile_gemm_partial_bytes(XQ_FMT_FP8, d.M, d.H, 2 * d.I) : 0;
     return std::max(std::max(pa, pb), std::max(ps, p2));
 }
 
@@ -122,15 +126,15 @@ int64_t fwd_panel_bytes(const Dims& d) {
     return std::max(gu, lowrank_panel_bytes(1, d.M, d.rp, d.I));
 }
 
-int64_t fwd_workspace(const Dims& d, bool needed) { return fwd_panel_bytes(d) + al256(gemm_part_bytes(d, needed)) + 512; }
+int64_t fwd_workspace(const Dims& d, int fmt, bool needed) { return fwd_panel_bytes(d) + al256(gemm_part_bytes(d, fmt, needed, false)) + 512; }
 
-int64_t bwd_workspace(const Dims& d, bool needed) {
+int64_t bwd_workspace(const Dims& d, int fmt, bool needed) {
     const int64_t rp = d.rp ? d.rp : 16;
     // the six factor gradients share a launch: partial sums of all of them (dA of gate and up of twice the rank, or apart)
     const int64_t tn = 3 * tn_partial_bytes(d.M, d.I, rp) + tn_partial_bytes(d.M, d.H, rp) +
                        std::max(2 * tn_partial_bytes(d.M, d.H, rp), 2 * rp <= 64 ? tn_partial_bytes(d.M, d.H, 2 * rp) : 0);
     return al256(d.M * d.I * 2) + al256(d.M * 2 * d.I * 2) + al256(d.M * d.H * 2) + al256(d.M * rp * 2) +
-           al256(d.M * 2 * rp * 2) + 2 * al256(rp * d.I * 2) + al256(std::max(gemm_part_bytes(d, needed), tn)) + 512;
+           al256(d.M * 2 * rp * 2) + 2 * al256(rp * d.I * 2) + al256(std::max(gemm_part_bytes(d, fmt, needed, true), tn)) + 512;
 }
 
 }  // namespace
@@ -145,10 +149,13 @@ extern "C" int xq_set_mlp_gate_up_fused(int enabled) {
 
 extern "C" int xq_get_mlp_gate_up_fused(void) { return g_mlp_gu.load() != 0; }
 
-extern "C" int64_t xq_mlp_workspace_bytes(int64_t M, int64_t hidden, int64_t intermediate, int r, int backward) {
+extern "C" int64_t xq_mlp_workspace_bytes_fmt(int format, int64_t M, int64_t hidden, int64_t intermediate, int r, int backward) {
     if (M < 0 || r < 0) return 0;
     Dims d{M, hidden, intermediate, r, r_pad_of(r)};
-    return backward ? bwd_workspace(d, false) : fwd_workspace(d, false);
+    return backward ? bwd_workspace(d, format, false) : fwd_workspace(d, format, false);
+}
+extern "C" int64_t xq_mlp_workspace_bytes(int64_t M, int64_t hidden, int64_t intermediate, int r, int backward) {
+    return xq_mlp_workspace_bytes_fmt(-1, M, hidden, intermediate, r, backward);
 }
 
 extern "C" int xq_mlp_fwd(const xq_weight* gate, const xq_weight* up, const xq_weight* down, const xq_mlp_lora* lora,
@@ -162,7 +169,7 @@ extern "C" int xq_mlp_fwd(const xq_weight* gate, const xq_weight* up, const xq_w
     saved->gate_up_fused = fused ? 1 : 0;       // what the backward must be told
     if (M == 0) return XQ_OK;
     XQ_REQUIRE(x_ && y, "%s: NULL activation pointer", who);
-    XQ_REQUIRE(workspace && xq_aligned(workspace, 256) && workspace_bytes >= fwd_workspace(d, true),
+    XQ_REQUIRE(workspace && xq_aligned(workspace, 256) && workspace_bytes >= fwd_workspace(d, -1, true),
                "%s: workspace missing, misaligned or smaller than xq_mlp_workspace_bytes()", who);
     XQ_REQUIRE(ldy % 8 == 0 && xq_aligned(y, 16), "%s: y rows must be 16-byte aligned", who);
     hipStream_t stream = (hipStream_t)stream_;
@@ -239,15 +246,18 @@ static int64_t infer_linear_ws(int64_t M, int64_t H, int64_t I, int r) {
     return al256((a > b ? a : b) > 2048 ? (a > b ? a : b) : 2048);
 }
 
-static int64_t infer_workspace(int64_t M, int64_t hidden, int64_t intermediate, int r, bool needed) {
+static int64_t infer_workspace(int fmt, int64_t M, int64_t hidden, int64_t intermediate, int r, bool needed) {
     if (M < 0 || r < 0) return 0;
     const int64_t act = al256(M * 2 * intermediate * 2) + al256(M * intermediate * 2);
-    const int64_t program = al256(M * 2 * r_pad_of(r) * 2) + al256(M * r_pad_of(r) * 2) + fwd_workspace(Dims{M, hidden, intermediate, r, r_pad_of(r)}, needed);
+    const int64_t program = al256(M * 2 * r_pad_of(r) * 2) + al256(M * r_pad_of(r) * 2) + fwd_workspace(Dims{M, hidden, intermediate, r, r_pad_of(r)}, fmt, needed);
     const int64_t apart = M <= 64 ? infer_linear_ws(M, hidden, intermediate, r) : 0;
     return act + (program > apart ? program : apart) + 256;
 }
+extern "C" int64_t xq_mlp_infer_workspace_bytes_fmt(int format, int64_t M, int64_t hidden, int64_t intermediate, int r) {
+    return infer_workspace(format, M, hidden, intermediate, r, false);
+}
 extern "C" int64_t xq_mlp_infer_workspace_bytes(int64_t M, int64_t hidden, int64_t intermediate, int r) {
-    return infer_workspace(M, hidden, intermediate, r, false);
+    return infer_workspace(-1, M, hidden, intermediate, r, false);
 }
 
 extern "C" int xq_mlp_fwd_infer(const xq_weight* gate, const xq_weight* up, const xq_weight* down, const xq_mlp_lora* lora,
@@ -263,7 +273,7 @@ extern "C" int xq_mlp_fwd_infer(const xq_weight* gate, const xq_weight* up, cons
     if (rc) return rc;
     if (M == 0) return XQ_OK;
     XQ_REQUIRE(x && y, "%s: NULL activation pointer", who);
-    XQ_REQUIRE(workspace_bytes >= infer_workspace(M, d.H, d.I, d.r, true),
+    XQ_REQUIRE(workspace_bytes >= infer_workspace(-1, M, d.H, d.I, d.r, true),
                "%s: workspace smaller than xq_mlp_infer_workspace_bytes()", who);
     bf16_t* gu = cv.take<bf16_t>(M * 2 * d.I * 2);
     bf16_t* h = cv.take<bf16_t>(M * d.I * 2);
@@ -323,7 +333,7 @@ extern "C" int xq_mlp_bwd(const xq_weight* gate, const xq_weight* up, const xq_w
         return XQ_OK;
     }
     XQ_REQUIRE(x_ && dy_, "%s: NULL activation pointer", who);
-    XQ_REQUIRE(workspace && xq_aligned(workspace, 256) && workspace_bytes >= bwd_workspace(d, true),
+    XQ_REQUIRE(workspace && xq_aligned(workspace, 256) && workspace_bytes >= bwd_workspace(d, -1, true),
                "%s: workspace missing, misaligned or smaller than xq_mlp_workspace_bytes()", who);
     XQ_REQUIRE(!dx || (lddx % 8 == 0 && xq_aligned(dx, 16)), "%s: dx rows must be 16-byte aligned", who);
     const bf16_t *x = (const bf16_t*)x_, *dy = (const bf16_t*)dy_;

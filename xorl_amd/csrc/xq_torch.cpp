@@ -322,6 +322,8 @@ std::vector<int64_t> with_last(const Tensor& x, int64_t last) {
 
 int r_pad_of(int r) { return (r + 15) / 16 * 16; }
 
+int shared_format(const xq_weight& a, const xq_weight& b, const xq_weight& c) { return a.format == b.format && a.format == c.format ? a.format : -1; }
+
 // the report of the one-launch decode forwards is read after every functional.SKINNY_CHECK_EVERY forwards of up to 16 rows
 bool note_decode_forward(const Tensor& x, int64_t M) {
     static int64_t calls = 0;       // (under the GIL)
@@ -372,7 +374,7 @@ struct QLoRALinearBackward : public Node {
         if (need_dx) out[0] = empty_bf(x.sizes());
         if (need_dA) out[1] = empty_f32({r, K});
         if (need_dB) out[2] = empty_f32({Nf, r});
-        Scratch ws(xq_linear_workspace_bytes(M, Nf, K, r));
+        Scratch ws(xq_linear_workspace_bytes_fmt(q.w.format, M, Nf, K, r));
         check(xq_linear_bwd(q.now(), xr.ptr, xr.ld, dr.ptr, dr.ld, M, A.data_ptr(), B.data_ptr(),
                             A.scalar_type() == at::kFloat ? XQ_DT_F32 : XQ_DT_BF16, r, (float)scaling, M ? su.data_ptr() : nullptr,
                             need_dx ? out[0].data_ptr() : nullptr, K, need_dA ? (float*)out[1].data_ptr() : nullptr,
@@ -434,7 +436,7 @@ struct QLoRAMLPBackward : public Node {
         xq_mlp_lora L;
         mlp_lora(&L, A, B, r, scaling);
         xq_mlp_saved S{kept[0].data_ptr(), kept[1].data_ptr(), kept[2].data_ptr(), kept[3].data_ptr(), gate_up_fused, 0};
-        Scratch ws(xq_mlp_workspace_bytes(dr.M, H, I, r, 1));
+        Scratch ws(xq_mlp_workspace_bytes_fmt(shared_format(q[0].w, q[1].w, q[2].w), dr.M, H, I, r, 1));
         check(xq_mlp_bwd(q[0].now(), q[1].now(), q[2].now(), &L, xr.ptr, xr.ld, dr.ptr, dr.ld, dr.M, &S, need_dx ? out[0].data_ptr() : nullptr, H, &G,
                          ws.get(), ws.bytes, stream_of(x)));
         for (int p = 0; p < 3; ++p) {
@@ -561,7 +563,7 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
         const Rows xr(*x, K);
         Tensor y = empty_bf(with_last(*x, Nf)), su;
         if (train) su = empty_bf({xr.M, r_pad_of(m.r)});
-        Scratch ws(xq_linear_workspace_bytes(xr.M, Nf, K, m.r));
+        Scratch ws(xq_linear_workspace_bytes_fmt(m.q.w.format, xr.M, Nf, K, m.r));
         {
             ReleaseGil nogil;
             check(xq_linear_fwd(&m.q.w, xr.ptr, xr.ld, xr.M, m.A.data_ptr(), m.B.data_ptr(), m.lora_dtype(), m.r, (float)m.scaling, m.bias_ptr(),
@@ -640,7 +642,7 @@ PyObject* mlp(PyObject*, PyObject* const* args, Py_ssize_t n) {
                 m[p].q.packed.device() != x->device() || m[p].A.device() != x->device())
                 XQ_NONE;
         const bool train = at::GradMode::is_enabled() && (x->requires_grad() || m[0].wants_grad() || m[1].wants_grad() || m[2].wants_grad());
-        const int r = m[0].r, rp = r_pad_of(r);
+        const int r = m[0].r, rp = r_pad_of(r), fmt = shared_format(m[0].q.w, m[1].q.w, m[2].q.w);
         c10::DeviceGuard guard(x->device());
         const Rows xr(*x, H);
         const int64_t M = xr.M;
@@ -650,7 +652,7 @@ PyObject* mlp(PyObject*, PyObject* const* args, Py_ssize_t n) {
         for (int p = 0; p < 3; ++p) L.bias[p] = m[p].bias_ptr();
         Tensor y = empty_bf(x->sizes());
         if (!train) {
-            Scratch ws(xq_mlp_infer_workspace_bytes(M, H, I, r));
+            Scratch ws(xq_mlp_infer_workspace_bytes_fmt(fmt, M, H, I, r));
             {
                 ReleaseGil nogil;
                 check(xq_mlp_fwd_infer(&m[0].q.w, &m[1].q.w, &m[2].q.w, &L, xr.ptr, xr.ld, M, y.data_ptr(), H, ws.get(), ws.bytes, stream_of(*x)));
@@ -662,7 +664,7 @@ PyObject* mlp(PyObject*, PyObject* const* args, Py_ssize_t n) {
         // gate and up in one launch or two: settled once, for this forward and its backward
         const int gu = xq_get_mlp_gate_up_fused() && m[0].q.w.format == XQ_FMT_FP8 && m[1].q.w.format == XQ_FMT_FP8;
         xq_mlp_saved S{kept[0].data_ptr(), kept[1].data_ptr(), kept[2].data_ptr(), kept[3].data_ptr(), gu, 0};
-        Scratch ws(xq_mlp_workspace_bytes(M, H, I, r, 0));
+        Scratch ws(xq_mlp_workspace_bytes_fmt(fmt, M, H, I, r, 0));
         {
             ReleaseGil nogil;
             check(xq_mlp_fwd(&m[0].q.w, &m[1].q.w, &m[2].q.w, &L, xr.ptr, xr.ld, M, y.data_ptr(), H, &S, ws.get(), ws.bytes, stream_of(*x)));

@@ -83,11 +83,11 @@ _WS_BYTES: dict = {}
 _EMPTY: dict = {}
 
 
-def _workspace_bytes(M: int, N: int, K: int, r: int) -> int:
-    key = (M, N, K, r)
+def _workspace_bytes(M: int, N: int, K: int, r: int, fmt: Optional[str] = None) -> int:
+    key = (M, N, K, r, fmt)
     v = _WS_BYTES.get(key)
     if v is None:
-        v = _WS_BYTES[key] = _C.lib().xq_linear_workspace_bytes(M, N, K, r)
+        v = _WS_BYTES[key] = _C.lib().xq_linear_workspace_bytes_fmt(_C.FORMATS.get(fmt, -1), M, N, K, r)
     return v
 
 
@@ -146,7 +146,7 @@ def _linear_fwd_impl(x: Tensor, packed: Tensor, scales: Tensor, global_scale: Op
         su = _EMPTY.get(dev)
         if su is None:
             su = _EMPTY[dev] = torch.empty(0, dtype=torch.bfloat16, device=dev)
-    ws_bytes = _workspace_bytes(M, N, K, r)
+    ws_bytes = _workspace_bytes(M, N, K, r, fmt)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
     A = lora_A.contiguous() if lora_A is not None else None
     B = lora_B.contiguous() if lora_B is not None else None
@@ -188,7 +188,7 @@ def _linear_bwd_impl(dy: Tensor, x: Tensor, su: Tensor, packed: Tensor, scales: 
     dA = torch.empty(r, K, dtype=torch.float32, device=dev) if need_dA else torch.empty(0, device=dev)
     dB = torch.empty(N, r, dtype=torch.float32, device=dev) if need_dB else torch.empty(0, device=dev)
     L = _C.lib()
-    ws_bytes = _workspace_bytes(M, N, K, r)
+    ws_bytes = _workspace_bytes(M, N, K, r, fmt)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
     A = lora_A.contiguous() if lora_A is not None else None
     B = lora_B.contiguous() if lora_B is not None else None
@@ -325,7 +325,7 @@ def qlora_linear_swiglu(x: Tensor, qw: QuantWeight, lora_A: Optional[Tensor], lo
     B = lora_B.detach()[:, :r].contiguous() if (lora_B is not None and r) else None
     b = bias.detach().to(torch.bfloat16).contiguous() if bias is not None else None
     L = _C.lib()
-    ws_bytes = L.xq_linear_fwd_swiglu_workspace_bytes(M, qw.rows, K, r)
+    ws_bytes = L.xq_linear_fwd_swiglu_workspace_bytes_fmt(_C.FORMATS[qw.fmt], M, qw.rows, K, r)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
     h = torch.empty(M, I, dtype=torch.bfloat16, device=dev)
     cw = qw.c()
@@ -420,11 +420,16 @@ def _mlp_gate_up_default() -> int:
     return int(_C.lib().xq_get_mlp_gate_up_fused())
 
 
-def _mlp_workspace(dev, M: int, H: int, I: int, r: int, backward: bool) -> Tensor:
-    key = (M, H, I, r, backward)
+def _shared_format(banks) -> int:
+    """The format code that gate, up and down share, -1 where they differ."""
+    return _C.FORMATS[banks[0].fmt] if len({b.fmt for b in banks}) == 1 else -1
+
+
+def _mlp_workspace(dev, banks, M: int, H: int, I: int, r: int, backward: bool) -> Tensor:
+    key = (_shared_format(banks), M, H, I, r, backward)
     n = _MLP_WS.get(key)
     if n is None:
-        n = _MLP_WS[key] = _C.lib().xq_mlp_workspace_bytes(M, H, I, r, int(backward))
+        n = _MLP_WS[key] = _C.lib().xq_mlp_workspace_bytes_fmt(key[0], M, H, I, r, int(backward))
     return torch.empty(n, dtype=torch.uint8, device=dev)
 
 
@@ -437,7 +442,7 @@ def _mlp_fwd_impl(x2: Tensor, factors, biases, banks, r: int, scaling: float, gu
     bf = lambda *shape: torch.empty(*shape, dtype=torch.bfloat16, device=dev)
     saved = (bf(M, 2 * I), bf(M, I), bf(M, 2 * rp), bf(M, rp))
     y = bf(M, H)
-    ws = _mlp_workspace(dev, M, H, I, r, False)
+    ws = _mlp_workspace(dev, banks, M, H, I, r, False)
     lora, S = _mlp_lora_struct(factors, biases, r, scaling), _mlp_saved_struct(saved, gu)
     wg, wu, wd = qg.c(), qu.c(), qd.c()
     _C.check(_C.lib().xq_mlp_fwd(ctypes.byref(wg), ctypes.byref(wu), ctypes.byref(wd), ctypes.byref(lora), x2.data_ptr(),
@@ -458,7 +463,7 @@ def _mlp_bwd_impl(dy2: Tensor, x2: Tensor, saved, factors, banks, r: int, scalin
     G = _C.XqMlpGrads()
     for p in range(3):
         G.dA[p], G.dB[p] = (grads[2 * p].data_ptr(), grads[2 * p + 1].data_ptr()) if r else (None, None)
-    ws = _mlp_workspace(dev, M, H, I, r, True)
+    ws = _mlp_workspace(dev, banks, M, H, I, r, True)
     lora, S = _mlp_lora_struct(factors, (None, None, None), r, scaling), _mlp_saved_struct(saved, gu)
     wg, wu, wd = qg.c(), qu.c(), qd.c()
     _C.check(_C.lib().xq_mlp_bwd(ctypes.byref(wg), ctypes.byref(wu), ctypes.byref(wd), ctypes.byref(lora), x2.data_ptr(),
@@ -613,10 +618,10 @@ def qlora_mlp_infer(x: Tensor, qw_gate: QuantWeight, qw_up: QuantWeight, qw_down
         factors[i] = None if t is None or r == 0 else t.detach()[:, :r].contiguous()
     biases = [None if b is None else b.detach().to(torch.bfloat16).contiguous() for b in (bias_gate, bias_up, bias_down)]
     L = _mlp_lora_struct(factors, biases, r if factors[0] is not None else 0, float(scaling))
-    key = (M, H, I, r)
+    key = (_shared_format((qw_gate, qw_up, qw_down)), M, H, I, r)
     n = _MLP_INFER_WS.get(key)
     if n is None:
-        n = _MLP_INFER_WS[key] = _C.lib().xq_mlp_infer_workspace_bytes(M, H, I, r)
+        n = _MLP_INFER_WS[key] = _C.lib().xq_mlp_infer_workspace_bytes_fmt(*key)
     dev = x.device
     ws = torch.empty(n, dtype=torch.uint8, device=dev)
     y = torch.empty(M, H, dtype=torch.bfloat16, device=dev)

@@ -97,3 +97,34 @@ def test_expert_weight_gradients_either_side_of_the_rule(hip_device, r, rp, tran
 ])
 def test_expert_factor_gradients_of_a_call(hip_device, fmt, E, T, I, r, hybrid):
     check_experts(hip_device, 0, fmt, E, T, 256, I, r, 2, hybrid)
+
+
+@pytest.mark.parametrize("r,rp,transpose", [(16, 16, False), (33, 48, True)])
+@pytest.mark.parametrize("counts", [
+    [0, 1, 33, 2600, 0, 100, 0, 0, 0, 0, 0, 0],          # one expert over three and a bit of four chunks
+    [1024, 1024, 0, 500, 1, 0, 0, 0, 0, 0, 0, 0],        # experts that end on the chunks' boundaries
+    [1000, 24, 1030, 0, 0, 0, 0, 0, 0, 0, 0, 1000],      # a boundary crossed by six rows; the last expert crosses the last one
+    [0, 0, 0, 3000, 0, 0, 0, 0, 0, 0, 0, 0],             # all rows in one
+    [1025, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0],
+])
+def test_expert_weight_gradients_of_uneven_loads(hip_device, counts, r, rp, transpose):
+    """Up to 256 rows an expert on average: the bits of the row chunks, which the same rows take under fewer experts."""
+    from xorl_amd import moe_functional as MF
+
+    width, counts = 200, torch.tensor(counts)
+    offsets = lambda c: torch.cat([torch.zeros(1, dtype=torch.int64), c.cumsum(0)]).to(torch.int32).to(hip_device)
+    R = int(counts.sum()) + 5                            # rows behind the last expert's belong to nobody
+    P, Q = gen((R, width), 1.0, 5, torch.bfloat16), gen((R, rp), 1.0, 6, torch.bfloat16)
+    assert R <= 256 * len(counts)
+    got = MF._wgrad(P.to(hip_device), Q.to(hip_device), r, offsets(counts), len(counts), transpose)
+    used = counts.nonzero().reshape(-1)
+    lo = 0
+    for e in range(len(counts)):
+        ref = P[lo:lo + counts[e]].double().t() @ Q[lo:lo + counts[e], :r].double()
+        lo += int(counts[e])
+        if counts[e]:
+            close(got[e].cpu(), ref.t() if transpose else ref, 1e-2, rows="none")
+        else:
+            assert torch.count_nonzero(got[e]) == 0
+    if R > 256 * len(used):
+        assert torch.equal(got[used.to(hip_device)], MF._wgrad(P.to(hip_device), Q.to(hip_device), r, offsets(counts[used]), len(used), transpose))

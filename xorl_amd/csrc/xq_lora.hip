@@ -1218,22 +1218,44 @@ __device__ __forceinline__ void tn_write_expert(const TnArgs& g, const f32x16* a
     tn_write<NT>(acc, g.out + at, c0, g.width, g.r_out, g.r_out, g.transpose_out != 0, g.out2 ? g.out2 + at : nullptr, g.split_j);
 }
 
-// experts of few rows: row part = expert -> out[expert], zero for an expert without rows
+// the expert that holds row `row` and the one before it (offsets[e] < row < offsets[e + 1]), -1 if a new expert, or none, starts
+// there; one look per thread, the same answer in the whole block
+__device__ __forceinline__ int tn_owner_across(const int32_t* offsets, int num_experts, int64_t row) {
+    __shared__ int sh;
+    if (threadIdx.x == 0) sh = -1;
+    __syncthreads();
+    for (int x = threadIdx.x; x < num_experts; x += 256)
+        if (offsets[x] < row && row < offsets[x + 1]) sh = x;
+    __syncthreads();
+    return sh;
+}
+
+// experts of few rows on average: a block takes one expert's rows within one chunk of TN_CHUNK global rows.  Part e < E: expert
+// e's first piece (written as the result where it is the only one, zero for an expert without rows); part E + c - 1: the piece
+// with which the expert that crosses into chunk c goes on there.  Pieces, their places and the order of their sum are those of
+// tn_grouped_kernel below: the same bits.
 template <int NT>
-__global__ void __launch_bounds__(256) tn_expert_kernel(TnGroupedBatch b) {
+__global__ void __launch_bounds__(256) tn_piece_kernel(TnGroupedBatch b, int32_t num_experts) {
     __shared__ __attribute__((aligned(16))) bf16_t Ps[2 * 32 * TN_PP];
     __shared__ __attribute__((aligned(16))) bf16_t Qs[2 * 32 * TN_QP];
-    int e;
+    int part;
     int64_t c0;
-    const TnArgs& g = b.job[tn_grouped_job(b, &e, &c0)];
-    const int64_t m_begin = g.offsets[e], m_end = g.offsets[e + 1];
+    const int ji = tn_grouped_job(b, &part, &c0);
+    const TnArgs& g = b.job[ji];
+    const bool first = part < num_experts;
+    const int e = first ? part : tn_owner_across(g.offsets, num_experts, (int64_t)(part - num_experts + 1) * TN_CHUNK);
+    if (e < 0) return;
+    const int64_t m_begin = first ? (int64_t)g.offsets[e] : (int64_t)(part - num_experts + 1) * TN_CHUNK;
+    const int64_t ee = g.offsets[e + 1], chunk = m_begin / TN_CHUNK, chunk_end = (chunk + 1) * TN_CHUNK;
+    const int64_t m_end = ee < chunk_end ? ee : chunk_end;
     f32x16 acc[NT];
 #pragma unroll
     for (int n = 0; n < NT; ++n)
 #pragma unroll
         for (int q = 0; q < 16; ++q) acc[n][q] = 0.0f;
     if (m_begin < m_end) tn_accumulate<NT>(g, c0, m_begin, m_end, Ps, Qs, acc);     // uniform over the block
-    tn_write_expert<NT>(g, acc, c0, e);
+    if (first && ee <= chunk_end) tn_write_expert<NT>(g, acc, c0, e);
+    else tn_write<NT>(acc, b.partial[ji] + (chunk * 2 + (first ? 1 : 0)) * g.width * g.r_pad, c0, g.width, g.r_pad, g.r_pad, false);
 }
 
 // row part = chunk of TN_CHUNK global rows.  The chunk is walked expert by expert;
@@ -1286,28 +1308,13 @@ __global__ void __launch_bounds__(256) tn_grouped_kernel(TnGroupedBatch b, int32
     }
 }
 
-// out[e] for the experts the chunk walk did not finish: zero for an expert without rows, the sum of
-// its pieces in chunk order for one that spans several chunks.  Block x: 1024 elements of a job's [width, r_pad], y: expert
-// (most blocks find their expert finished: four elements a thread keep their number down: 28 us for those five products,
-// 55 with one element).
-__global__ void __launch_bounds__(256) tn_grouped_reduce_kernel(TnGroupedBatch b) {
-    const int e = blockIdx.y;
-    int ji = 0;
-#pragma unroll
-    for (int i = 1; i < kTnJobs; ++i)
-        if (i < b.n && (int)blockIdx.x >= b.first[i]) ji = i;
-    const TnArgs& g = b.job[ji];
-    const int64_t rb = g.offsets[e], en = g.offsets[e + 1];
-    const int64_t ch0 = rb / TN_CHUNK, ch1 = en > rb ? (en - 1) / TN_CHUNK : ch0;
-    if (en > rb && ch0 == ch1) return;   // written directly
-    const int64_t t = ((int64_t)((int)blockIdx.x - b.first[ji]) * 256 + threadIdx.x) * 4;
-    if (t >= g.width * g.r_pad) return;
+// Four elements from t on of expert e's result: the sum of its pieces in chunk order, zero without rows
+__device__ __forceinline__ void tn_reduce_expert(const TnArgs& g, const float* partial, int e, int64_t rb, int64_t en, int64_t t) {
     const int64_t c = t / g.r_pad;
     int j = (int)(t - c * g.r_pad);      // (r_pad and split_j are multiples of 16: the four lie in one row of one result)
     f32x4 s = {0.0f, 0.0f, 0.0f, 0.0f};
     if (en > rb) {
-        const int64_t per = g.width * g.r_pad;
-        const float* partial = b.partial[ji];
+        const int64_t ch0 = rb / TN_CHUNK, ch1 = (en - 1) / TN_CHUNK, per = g.width * g.r_pad;
         s = *(const f32x4*)(partial + (ch0 * 2 + 1) * per + t);
         for (int64_t ch = ch0 + 1; ch <= ch1; ++ch) s += *(const f32x4*)(partial + (ch * 2) * per + t);
     }
@@ -1320,6 +1327,31 @@ __global__ void __launch_bounds__(256) tn_grouped_reduce_kernel(TnGroupedBatch b
         if (g.transpose_out) o[(int64_t)(j + u) * g.width + c] = s[u];
         else o[c * g.r_out + j + u] = s[u];
     }
+}
+
+// out[e] for the experts the chunk walk did not finish: zero for an expert without rows, the sum of
+// its pieces in chunk order for one that spans several chunks.  Block x: 1024 elements of a job's [width, r_pad], y: expert
+// (most blocks find their expert finished: four elements a thread keep their number down: 28 us for those five products,
+// 55 with one element).  CROSS, behind tn_piece_kernel, which has finished every expert within one chunk and those without
+// rows: y: the boundary before chunk y + 1, for the expert that crosses it as its first.
+template <bool CROSS>
+__global__ void __launch_bounds__(256) tn_grouped_reduce_kernel(TnGroupedBatch b, int32_t num_experts) {
+    int ji = 0;
+#pragma unroll
+    for (int i = 1; i < kTnJobs; ++i)
+        if (i < b.n && (int)blockIdx.x >= b.first[i]) ji = i;
+    const TnArgs& g = b.job[ji];
+    const int64_t boundary = (int64_t)(blockIdx.y + 1) * TN_CHUNK;
+    const int e = CROSS ? tn_owner_across(g.offsets, num_experts, boundary) : (int)blockIdx.y;
+    if (e < 0) return;
+    const int64_t rb = g.offsets[e], en = g.offsets[e + 1];
+    if constexpr (CROSS) {
+        if (rb < boundary - TN_CHUNK) return;       // it has crossed one before
+    } else {
+        if (en > rb && rb / TN_CHUNK == (en - 1) / TN_CHUNK) return;   // written directly
+    }
+    const int64_t t = ((int64_t)((int)blockIdx.x - b.first[ji]) * 256 + threadIdx.x) * 4;
+    if (t < g.width * g.r_pad) tn_reduce_expert(g, b.partial[ji], e, rb, en, t);
 }
 
 // sums the dense partials of up to kTnJobs products in split order: out[c][j] or out[j][c], j < r_out
@@ -1424,11 +1456,14 @@ int launch_tn_grouped_multi(const TnJob* jobs, int n, int64_t n_rows, float* par
                             hipStream_t stream) {
     XQ_REQUIRE(n >= 0 && n <= kTnJobs, "tn: %d products", n);
     XQ_REQUIRE(partial != nullptr, "tn: partial workspace is NULL");
-    // up to 256 rows an expert on average a block takes an expert's rows whole and writes its result: nothing is summed
-    // afterwards, and the experts of a column tile run side by side instead of one after the other (456 rows of 128 experts,
-    // 768 columns: 289 us in 6 blocks, 8 us in 768); beyond that, chunks of the row range keep uneven experts level
-    const bool by_expert = n_rows <= 256ll * num_experts;
-    const int64_t parts = by_expert ? num_experts : xq_cdiv(n_rows, TN_CHUNK);
+    // up to 256 rows an expert on average the experts of a column tile run side by side, a block for each (and for each further
+    // chunk of one that spans several); beyond, a block walks a chunk of the row range expert by expert.
+    // Backward of 128 block-fp8 experts [2048, 768], rank 16, us, walked chunks / blocks of an expert and chunk / one block an expert
+    // whatever its rows: Zipf(1.1) loads of 4 rows an expert on average 603 / 345 / 345, of 64 505 / 455 / 448, of 256 (the largest
+    // 3700) 769 / 732 / 752, of 384 961 / 931 / 960; even loads of 256 735 / 705 / 687; all rows in one expert, 8192 452 / 466 / 583,
+    // 32768 685 / 694 / 1201.  (So the line could lie higher; it was drawn for the form of one block an expert.)
+    const bool pieces = n_rows <= 256ll * num_experts;
+    const int64_t chunks = xq_cdiv(n_rows, TN_CHUNK), parts = pieces ? num_experts + (chunks > 1 ? chunks - 1 : 0) : chunks;
     TnGroupedBatch b{};
     int32_t rfirst[kTnJobs];
     int nt = 1;
@@ -1452,17 +1487,18 @@ int launch_tn_grouped_multi(const TnJob* jobs, int n, int64_t n_rows, float* par
     }
     if (b.n == 0) return XQ_OK;
     XQ_REQUIRE(blocks < (1ll << 31), "tn: %lld blocks", (long long)blocks);
-    if (by_expert) {
-        if (nt == 1) tn_expert_kernel<1><<<(unsigned)blocks, 256, 0, stream>>>(b);
-        else tn_expert_kernel<2><<<(unsigned)blocks, 256, 0, stream>>>(b);
-        XQ_CHECK_LAUNCH("tn(expert)");
-        return XQ_OK;
+    if (pieces) {
+        if (nt == 1) tn_piece_kernel<1><<<(unsigned)blocks, 256, 0, stream>>>(b, num_experts);
+        else tn_piece_kernel<2><<<(unsigned)blocks, 256, 0, stream>>>(b, num_experts);
+    } else {
+        if (nt == 1) tn_grouped_kernel<1><<<(unsigned)blocks, 256, 0, stream>>>(b, num_experts);
+        else tn_grouped_kernel<2><<<(unsigned)blocks, 256, 0, stream>>>(b, num_experts);
     }
-    if (nt == 1) tn_grouped_kernel<1><<<(unsigned)blocks, 256, 0, stream>>>(b, num_experts);
-    else tn_grouped_kernel<2><<<(unsigned)blocks, 256, 0, stream>>>(b, num_experts);
     XQ_CHECK_LAUNCH("tn(grouped)");
+    if (pieces && chunks < 2) return XQ_OK;
     for (int k = 0; k < b.n; ++k) b.first[k] = rfirst[k];
-    tn_grouped_reduce_kernel<<<dim3((unsigned)rblocks, (unsigned)num_experts), 256, 0, stream>>>(b);
+    if (pieces) tn_grouped_reduce_kernel<true><<<dim3((unsigned)rblocks, (unsigned)(chunks - 1)), 256, 0, stream>>>(b, num_experts);
+    else tn_grouped_reduce_kernel<false><<<dim3((unsigned)rblocks, (unsigned)num_experts), 256, 0, stream>>>(b, num_experts);
     XQ_CHECK_LAUNCH("tn(grouped reduce)");
     return XQ_OK;
 }

@@ -1,4 +1,4 @@
-// Values -> 4-bit codes, shared by the quantizers and the re-quantising merge.
+// Values -> 4-bit codes, for the quantizers.  (The re-quantising merge has encoders of its own.)
 #pragma once
 #include "xq_common.h"
 

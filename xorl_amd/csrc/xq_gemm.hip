@@ -168,7 +168,20 @@ static DensePlan plan_dense(int64_t n_rows, int64_t Nout, int64_t nk) {
 //   int4 [12288, 4096]: 512 rows 92 / 101, 700 115 / 128, 1357 153 / 171, 4096 323 / 403, 8192 636 / 820; [4096, 12288]: 512 114 / 94,
 //   700 114 / 143, 8192 627 / 786; [4096, 4096]: 512 55 / 45, 1024 69 / 70, 1357 80 / 96; [1024, 4096]: 2048 50 / 45, 4096 72 / 68,
 //   8192 101 / 113; block-fp8 [12288, 4096]: 1357 155 / 145, 4096 335 / 327, 8192 626 / 661; [8192, 5120]: 4096 271 / 267, 8192 518 / 545.
-// So 4-bit from 640 rows on, block-fp8 from 6144 on, and products too small to fill the chip stay with the tile kernels.
+// Block-fp8, forward / dgrad, per cent by which the image is faster (negative: slower), nine weights:
+//   rows                        3072       4096       5120       6144       7168       8192       16384
+//   [12288, 4096]              1 / 0      2 / 0      4 / 3      5 / 5      6 / 1      6 / 3      5 / 4
+//   [4096, 12288]              2 / -2     2 / 0      5 / 2      7 / 4      3 / 4      4 / 4      4 / 4
+//   [8192, 5120]               2 / -1     2 / 1      3 / -2     4 / 3      6 / 4      6 / 3      7 / 5
+//   [4096, 4096]               1 / 0      2 / 1     10 / 1      5 / 5      6 / 5      5 / 5      7 / 6
+//   [2048, 2048]             -13 / -16   -5 / -10    4 / 4      2 / 0      3 / 2      2 / 2      6 / 5
+//   [1024, 5120]               1 / -9     0 / -6    17 / -1    12 / -1    10 / -7     8 / 3      6 / 6
+//   [1024, 4096]              -3 / -9    -4 / -7    10 / -13    6 / -2     4 / 1      3 / 1      5 / 6
+//   [4096, 1024]              -8 / -7    -6 / -9   -11 / 8      0 / 2      1 / 2      2 / 1      5 / 5
+//   [512, 4096]              -16 / -14  -13 / -10   -7 / -14   -1 / -12   -3 / -3    -2 / -5     4 / 3
+// So 4-bit from 640 rows on, block-fp8 from 6144 on (both directions gain but for a narrow dgrad whose tiles fill a round badly,
+// and below it the wide weights gain less than the narrow ones lose), and products too small to fill the chip (2e10: the last
+// line up to 8192 rows) stay with the tile kernels.
 constexpr int64_t kDecMinRows = 640, kDecMinRowsFp8 = 6144;
 constexpr double kDecMinWork = 2.0e10;               // rows x columns x contraction
 struct DecPlan {

@@ -700,7 +700,7 @@ struct SiluNtArgs {
     float* partial;            // dense with gridDim.y > 1: fp32 sums [gridDim.y][n_rows][products * r_pad]
 };
 
-// GROUPED: routed rows in expert order, organisation of small_nt_kernel<128, FJ> (a block = a 128-row tile of one expert, a
+// GROUPED: routed rows in expert order, organisation of small_nt_kernel<FJ> (a block = a 128-row tile of one expert, a
 // wave = 32 rows over all columns, the expert's own factor pair), the routing weight applied and its gradient formed as
 // the elementwise kernel does (the sum over a row runs in another order here: 16 lanes' partial sums, then a butterfly).
 // FWD: the forward pass in the same organisation -- h = bf16(bf16(silu(gate)) * up) (routed: then rounded and times the row's

@@ -86,7 +86,6 @@ struct SkinnyRowsJob {
 // job 0's y receives h = silu(gate) * up.  Each forward gives the bits of a launch of its own.
 bool skinny_takes_stream(const xq_weight* w, int64_t M, const void* lora_A, const void* lora_B, int lora_dtype, int r);
 bool skinny_stream_multi_supported(const SkinnyRowsJob* jobs, int n_jobs, int64_t M);
-int64_t skinny_stream_multi_workspace_bytes(const SkinnyRowsJob* jobs, int n_jobs, int64_t M);
 int launch_skinny_stream(const SkinnyRowsJob* jobs, int n_jobs, bool swiglu, const bf16_t* x, int64_t ldx, int64_t M, int lora_dtype,
                          void* workspace, hipStream_t stream);
 bool skinny_rows_multi_supported(const SkinnyRowsJob* jobs, int n_jobs, int64_t M, int lora_dtype);

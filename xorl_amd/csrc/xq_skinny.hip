@@ -677,12 +677,6 @@ bool skinny_stream_multi_supported(const SkinnyRowsJob* jobs, int n_jobs, int64_
     return true;
 }
 
-int64_t skinny_stream_multi_workspace_bytes(const SkinnyRowsJob* jobs, int n_jobs, int64_t M) {
-    int64_t b = 0;
-    for (int i = 0; i < n_jobs; ++i) b += skinny_workspace_bytes(M, jobs[i].w->rows, jobs[i].w->cols, jobs[i].r > 0 ? (jobs[i].r + 15) / 16 * 16 : 0);
-    return b;
-}
-
 int launch_skinny_stream(const SkinnyRowsJob* jobs, int n_jobs, bool swiglu, const bf16_t* x, int64_t ldx, int64_t M, int lora_dtype,
                          void* workspace, hipStream_t stream) {
     const xq_weight* w0 = jobs[0].w;

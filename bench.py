@@ -47,13 +47,16 @@ MEASURED_TRAFFIC = {
     # gemm_dec_kernel and the dec_image passes before it (dense block-fp8, 256x256 tiles over decoded images): mean over the 5
     # products of a step (gate, up and down forward, d_h, dx as one sum over the gate and up weights)
     1: (1708.6 * 2 ** 20, "profiles/gemm_dec_fp8_mlp_m8192.txt", 0.7336),
+    # gemm_dec_kernel, dec_image passes and reductions over nvfp4 / NF4 weights: mean over the products of a step (8 and 6)
+    2: (501.4 * 2 ** 20, "profiles/gemm_dec_4bit_m4096_m8192.txt", 0.1802),
+    6: (1423.9 * 2 ** 20, "profiles/gemm_dec_4bit_m4096_m8192.txt", 0.6174),
     # gemm_dtl16_kernel<.., grouped>: mean over the 4 launches of a step (gate|up forward over two banks, down
     # forward, d_h, dx as one sum over both banks)
     3: (1402.4 * 2 ** 20, "profiles/gemm_dtl16_fp8_grouped_moe_e128.txt", 0.6325),
-    # skinny_gemv_kernel (M = 1), skinny_rows_kernel (M <= 16) and skinny_split_kernel + skinny_epilogue_kernel
+    # skinny_gemv_kernel (M = 1), skinny_rows_kernel (M <= 16) and stream_split_kernel + stream_epilogue_kernel
     # (M = 32, 64): mean per forward over the 32 cases (includes the fp32 partial tiles of the two-launch cases
     # written and read back: 23.3 MiB of it are algorithmic)
-    4: (39.3 * 2 ** 20, "profiles/skinny_kernels_decode_shapes.txt", 0.01712),
+    4: (34.2 * 2 ** 20, "profiles/skinny_kernels_decode_shapes.txt", 0.01557),
     # merge_prep_kernel + merge_kernel<fp8>: mean per call (re-quantise 96 MiB, publish 144 MiB algorithmic)
     5: (134.4 * 2 ** 20, "profiles/merge_kernel_fp8_mlp_weights.txt", 0.04168),
     # gemm_256_kernel<nvfp4 GKN, grouped>: mean over the 6 launches of a step
@@ -250,7 +253,7 @@ def other_config(cfg: int, dev):
                 "configs[4]: skinny-M forward, M in {1,8,32,64} x {q 4096->4096, kv 4096->1024, gate/up 4096->12288, "
                 "down 12288->4096} x {int4, block_fp8}, r=16 (32 forwards per step)",
                 "skinny_gemv_kernel<int4|fp8> (M = 1, dot products), skinny_rows_kernel<int4|fp8> (M <= 16, one launch) "
-                "and skinny_split_kernel<int4|fp8> + skinny_epilogue_kernel (M = 32, 64) (weight-streaming fused "
+                "and stream_split_kernel<int4|fp8> + stream_epilogue_kernel (M = 32, 64) (weight-streaming fused "
                 "dequant-GEMV/GEMM; the timed region is the whole forward)")
     if cfg == 5:
         # not a BASELINE config: the merge / re-quantise pass over configs[1]'s three block_fp8 weights (r = 32)
@@ -314,7 +317,7 @@ def other_config(cfg: int, dev):
         return (step, sum(lin_flops(Mtok, K, N, 32) for (N, K) in shapes.values()), False,
                 "NF4 (not a BASELINE config): QLoRA Qwen3-8B MLP projections gate/up 4096->12288, down 12288->4096 "
                 "as NF4 group 64, M=8192, r=32, fwd+bwd of each linear",
-                "gemm_256_kernel<nf4> (fused dequant-GEMM, forward and dgrad launches)")
+                "gemm_dec_kernel with its dec_image passes (NF4 decoded once per launch, 256x256x32 tiles): forward and dgrad launches")
     raise SystemExit(f"bench.py: unknown --config {cfg}")
 
 

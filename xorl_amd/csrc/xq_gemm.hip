@@ -4,6 +4,7 @@
 #include <atomic>
 #include "xq_gemm_256.h"
 #include "xq_gemm_dec.h"
+#include "xq_gemm_mid.h"
 #include <stdlib.h>
 #include <mutex>
 #include "xq_lora.h"
@@ -189,6 +190,7 @@ struct DecPlan {
     int64_t head_rows;        // leading rows; the others are a second launch in tail_split K splits
     int tail_split;
     int64_t partial;          // bytes of fp32 sums the splits take
+    double us;                // the estimate it was chosen by
 };
 static DecPlan plan_decoded(int64_t n_rows, int64_t Nout, int64_t Kc) {
     // microseconds: a round of the chip takes 0.8 per K-step (0.78-0.84 measured) and 5 around them; the fp32 sums of splits are
@@ -207,12 +209,12 @@ static DecPlan plan_decoded(int64_t n_rows, int64_t Nout, int64_t Kc) {
         return b;
     };
     double whole;
-    DecPlan p{best(n_rows, &whole), n_rows, 1, 0};
+    DecPlan p{best(n_rows, &whole), n_rows, 1, 0, whole};
     const int64_t tr = xq_cdiv(n_rows, GeoDec::T), keep = tr * tc / cus * cus / tc;      // tile rows of whole rounds
     if (keep > 0 && keep < tr) {
         double tail;
         const int ts = best(n_rows - keep * GeoDec::T, &tail);
-        if (cost(keep * GeoDec::T, 1) + tail < whole) p = DecPlan{1, keep * GeoDec::T, ts, 0};
+        if (cost(keep * GeoDec::T, 1) + tail < whole) p = DecPlan{1, keep * GeoDec::T, ts, 0, cost(keep * GeoDec::T, 1) + tail};
     }
     const int64_t tail_rows = n_rows - p.head_rows;
     p.partial = std::max(p.split > 1 ? p.split * p.head_rows : 0, tail_rows && p.tail_split > 1 ? p.tail_split * tail_rows : 0) * Nout * 4;
@@ -225,6 +227,75 @@ static bool decode_first(int fmt, int64_t n_rows, int64_t Nout, int64_t Kc) {
 // (fmt < 0: whatever the format; the 4-bit rule covers all)
 static int64_t decoded_scratch_bytes(int fmt, int64_t n_rows, int64_t Nout, int64_t Kc) {
     return decode_first(fmt < 0 ? XQ_FMT_INT4 : fmt, n_rows, Nout, Kc) ? dec_image_bytes(Nout, Kc) + plan_decoded(n_rows, Nout, Kc).partial : 0;
+}
+
+// ---- products that gemm_mid_kernel (xq_gemm_mid.h) takes.  Estimates in microseconds, each within about 5 per cent of what was
+// measured (four formats, rows 80 .. 3000, weights [4096, 4096], [12288, 4096], [1024, 4096] and [2560, 8192], both directions); the
+// launch goes to the kernel with the shorter one.  70 random products of 65 .. 4096 rows over the formats, both directions: 1.16
+// times as fast in the mean, up to 1.8.  Forward / dgrad, this kernel against the tile kernels (from 640 rows on 4-bit:
+// over decoded images):
+//   [4096, 4096]    rows       100          256          512         1024         2048         3000
+//   int4             21.3 / 24.9  26.5 / 31.2  35.0 / 42.6  44.6 / 63.0  63.8 / 84.7  103.9 / 89.6 (forward)
+//                    21.7 / 24.2  26.0 / 30.1  34.3 / 39.3  45.8 / 60.4  67.6 / 81.0  106.0 / 90.8 (dgrad)
+//   block-fp8        20.1 / 21.2  24.0 / 28.2  33.0 / 37.8  42.5 / 56.2  63.5 / 79.9  101.4 / 90.9 (forward)
+//   nf4              27.2 / 26.7  33.5 / 33.3  43.9 / 47.4  64.3 / 72.1  87.2 / 81.8  153.4 / 91.5 (forward)
+//   [12288, 4096], 512 rows: int4 forward 56.8 / 93.8, dgrad 64.1 / 82.5; block-fp8 54.8 / 73.9, 61.3 / 71.2
+struct MidPlan {
+    int mw, split;
+    double us;
+};
+static MidPlan plan_mid(int fmt, bool cc, int64_t rows, int64_t Nout, int64_t Kc) {
+    // a step of 64 k and both phases takes c + d f, f the share of the compute units that are at work
+    static const double kStep[3][3][2] = {{{0.93, 0.24}, {1.05, 0.34}, {1.20, 0.45}},       // int4, nvfp4: MW = 2, 3, 4
+                                          {{0.75, 0.25}, {0.88, 0.36}, {1.05, 0.47}},       // block-fp8
+                                          {{1.95, 0.18}, {2.00, 0.36}, {2.20, 0.32}}};      // nf4 (its level look-ups)
+    const int ws = cc && fmt != XQ_FMT_FP8 ? 2 : 1, kind = fmt == XQ_FMT_FP8 ? 1 : fmt == XQ_FMT_NF4 ? 2 : 0;
+    const int64_t units = Kc / 64 / ws, cus = num_cus();
+    MidPlan best{0, 1, 0.0};
+    for (int mw = 2; mw <= 4; ++mw)
+        for (int s = 1; s <= 8 && (s == 1 || units * ws >= 4 * s); ++s) {
+            const int64_t blocks = xq_cdiv(rows, 32 * mw) * xq_cdiv(Nout, 256) * s, rounds = xq_cdiv(blocks, cus);
+            const double f = rounds > 1 ? 1.0 : (double)blocks / (double)cus, *c = kStep[kind][mw - 2];
+            const double sums = s > 1 ? 2.0 + 0.18e-6 * (8.0 * s + 2.0) * (double)rows * (double)Nout : 0.0;
+            const double us = (double)rounds * (5.5 + 1.15 * mw + (double)(xq_cdiv(units, 2 * s) * ws) * (c[0] + c[1] * f)) + sums;
+            if (best.mw == 0 || us < best.us) best = MidPlan{mw, s, us};
+        }
+    return best;
+}
+// the same product without it: over a decoded image, or on 256- or 128-row tiles
+static double tile_kernels_us(int fmt, int64_t rows, int64_t Nout, int64_t Kc) {
+    if (decode_first(fmt, rows, Nout, Kc)) return 2.6 + 0.45e-6 * (double)Nout * (double)Kc + 0.8 * plan_decoded(rows, Nout, Kc).us;
+    const double nk = (double)(Kc / 64);
+    if (dense_tile_size(rows, Nout) == 256) {
+        const int64_t tiles = xq_cdiv(rows, 256) * xq_cdiv(Nout, 256), cus = num_cus(), full = tiles / cus;
+        const double per = fmt == XQ_FMT_FP8 ? 1.0 : 1.25;
+        return full ? ((double)full + (tiles % cus ? 0.7 : 0.0)) * (8.0 + per * 1.55 * nk) : 8.0 + per * (0.9 + 0.65 * (double)tiles / (double)cus) * nk;
+    }
+    static const double k128[3][4] = {{25.3, 0.61, 0.66, 0.15}, {22.9, 0.29, 0.77, 0.136}, {24.5, 0.77, 0.78, 0.142}};
+    const double* c = k128[fmt == XQ_FMT_FP8 ? 1 : fmt == XQ_FMT_NF4 ? 2 : 0];
+    const int64_t tiles = xq_cdiv(rows, 128) * xq_cdiv(Nout, 128);
+    const int s = ksplit_for(tiles, 128, Kc / 64);
+    const double st = (double)xq_cdiv(Kc / 64, s);
+    return c[0] + st * (c[1] + c[2] * (double)(tiles * s) / (2.0 * num_cus())) + (s > 1 ? -13.0 + c[3] * 1e-6 * (8.0 * s + 2.0) * (double)rows * (double)Nout : 0.0);
+}
+static bool mid_shape(int fmt, bool cc, int64_t rows, int64_t Nout, int64_t Kc) {
+    // whole units of the contraction for both phases; 4-bit dgrads: whole 16-byte pieces of 32 columns, whole scale groups
+    const int64_t unit = cc && fmt != XQ_FMT_FP8 ? 128 : 64;
+    // (block-fp8 forwards below 1024 k: the tile kernels' order of the sums, which the one launch over gate and up shares bit for bit)
+    return rows > 64 && Kc % unit == 0 && Kc >= (cc && fmt == XQ_FMT_FP8 ? 1024 : 2 * unit) &&
+           (fmt != XQ_FMT_FP8 || Kc <= 64 * 2 * GeoMid<XQ_FMT_FP8, true, 4>::SCL_MAX) &&
+           (cc || fmt == XQ_FMT_FP8 || Nout % (fmt == XQ_FMT_INT4 ? 128 : 64) == 0) && Nout >= 64;
+}
+static bool takes_mid(int fmt, bool cc, int64_t rows, int64_t Nout, int64_t Kc, MidPlan* plan) {
+    if (!mid_shape(fmt, cc, rows, Nout, Kc)) return false;
+    *plan = plan_mid(fmt, cc, rows, Nout, Kc);
+    // (a lead the estimates can carry: over random shapes a smaller one was a loss as often as a gain, up to 8 per cent for nf4)
+    const double lead = fmt == XQ_FMT_NF4 ? 0.92 : decode_first(fmt, rows, Nout, Kc) || dense_tile_size(rows, Nout) == 256 ? 0.94 : 1.0;
+    return plan->us < lead * tile_kernels_us(fmt, rows, Nout, Kc);
+}
+static int64_t mid_partial_bytes(int fmt, bool cc, int64_t rows, int64_t Nout, int64_t Kc) {
+    MidPlan p;
+    return takes_mid(fmt, cc, rows, Nout, Kc, &p) && p.split > 1 ? p.split * rows * Nout * 4 : 0;
 }
 
 // fp32 partial-sum bytes the split-K forms of a dense [n_rows, Nout] product over Kc may want, under any tile policy
@@ -246,7 +317,11 @@ int64_t tile_gemm_split_bytes(int64_t n_rows, int64_t Nout, int64_t Kc) {
 // its splits (without room for those the launch decodes in the tile kernel)
 int64_t tile_gemm_partial_bytes(int fmt, int64_t n_rows, int64_t Nout, int64_t Kc) {
     if (n_rows <= 0 || Kc % BK) return 0;
-    return std::max(tile_gemm_split_bytes(n_rows, Nout, Kc), decoded_scratch_bytes(fmt, n_rows, Nout, Kc));
+    int64_t mid = 0;
+    for (int f : {XQ_FMT_INT4, XQ_FMT_NVFP4, XQ_FMT_FP8, XQ_FMT_NF4})
+        if (fmt < 0 || fmt == f)
+            for (bool cc : {true, false}) mid = std::max(mid, mid_partial_bytes(f, cc, n_rows, Nout, Kc));
+    return std::max(mid, std::max(tile_gemm_split_bytes(n_rows, Nout, Kc), decoded_scratch_bytes(fmt, n_rows, Nout, Kc)));
 }
 
 // Whether a grouped launch on this bank may take a second bank of the same shape (see G256Args::W2): block-fp8 on the
@@ -320,6 +395,41 @@ static int launch_decoded(G256Args f, bool cc, int fmt, uint8_t* scratch, hipStr
     return XQ_OK;
 }
 
+template <int FMT, bool CC>
+static int launch_mid_t(const G256Args& f, int mw, dim3 grid, hipStream_t s, const char* who) {
+    static std::atomic<bool> attr_set{false};
+    if (!attr_set) {
+        int rc = raise_lds_limit(gemm_mid_kernel<FMT, CC, 4>, GeoMid<FMT, CC, 4>::lds_bytes(), who);
+        if (!rc) rc = raise_lds_limit(gemm_mid_kernel<FMT, CC, 3>, GeoMid<FMT, CC, 3>::lds_bytes(), who);
+        if (!rc) rc = raise_lds_limit(gemm_mid_kernel<FMT, CC, 2>, GeoMid<FMT, CC, 2>::lds_bytes(), who);
+        if (rc) return rc;
+        attr_set = true;
+    }
+    if (mw == 4) gemm_mid_kernel<FMT, CC, 4><<<grid, 512, GeoMid<FMT, CC, 4>::lds_bytes(), s>>>(f);
+    else if (mw == 3) gemm_mid_kernel<FMT, CC, 3><<<grid, 512, GeoMid<FMT, CC, 3>::lds_bytes(), s>>>(f);
+    else gemm_mid_kernel<FMT, CC, 2><<<grid, 512, GeoMid<FMT, CC, 2>::lds_bytes(), s>>>(f);
+    return XQ_OK;
+}
+static int launch_mid(G256Args f, bool cc, int fmt, int mw, hipStream_t s, const char* who) {
+    f.tiles_m = (int32_t)xq_cdiv(f.M, 32 * mw);
+    f.tiles_n = (int32_t)xq_cdiv(f.Nout, 256);
+    const dim3 grid((unsigned)(f.tiles_m * f.tiles_n), (unsigned)f.ksplit);
+    const bool timed = xq_profile_mark_begin(s, 2.0 * (double)f.M * f.Nout * ((double)f.Kc + f.r_pad));
+    int rc;
+    if (fmt == XQ_FMT_FP8) rc = cc ? launch_mid_t<XQ_FMT_FP8, true>(f, mw, grid, s, who) : launch_mid_t<XQ_FMT_FP8, false>(f, mw, grid, s, who);
+    else if (fmt == XQ_FMT_INT4) rc = cc ? launch_mid_t<XQ_FMT_INT4, true>(f, mw, grid, s, who) : launch_mid_t<XQ_FMT_INT4, false>(f, mw, grid, s, who);
+    else if (fmt == XQ_FMT_NF4) rc = cc ? launch_mid_t<XQ_FMT_NF4, true>(f, mw, grid, s, who) : launch_mid_t<XQ_FMT_NF4, false>(f, mw, grid, s, who);
+    else rc = cc ? launch_mid_t<XQ_FMT_NVFP4, true>(f, mw, grid, s, who) : launch_mid_t<XQ_FMT_NVFP4, false>(f, mw, grid, s, who);
+    if (rc) return rc;
+    XQ_CHECK_LAUNCH(who);
+    if (f.ksplit > 1) {
+        splitk_reduce_kernel<<<(unsigned)xq_cdiv(f.M * (f.Nout >> 2), 256), 256, 0, s>>>(f.partial, f.ksplit, f.M, f.Nout, f.C, f.ldc);
+        XQ_CHECK_LAUNCH(who);
+    }
+    if (timed) xq_profile_mark_end(s);
+    return XQ_OK;
+}
+
 // C[rows, Nout] = A . op(deq(W)) (+ su . Lr^T) (+ bias); see xq_gemm_tile.h.  force_T = 256 / 128 fixes the tile
 // size of the pipelined kernel (and force_split its K splits), 0 leaves both to the selection policy.  `partial` (may be NULL) is scratch for
 // split-K sums; a launch that would split but finds less than tile_gemm_partial_bytes() there runs unsplit.
@@ -390,7 +500,29 @@ static int launch_tile_gemm_t(const xq_weight* w, bool contract_cols, const bf16
         const DensePlan plan = plan_dense(n_rows, g.Nout, g.Kc / BK);
         const bool planned = !grouped && fmt_ok && g_tile_policy == 0 && force_T == 0 && !two_dense;   // two matrices: one unsplit launch
         const int T = force_T ? force_T : g_tile_policy == 2 ? 256 : g_tile_policy == 3 ? 128 : grouped ? (big ? 256 : 128) : plan.T;
-        if ((planned || (two_dense && g_tile_policy == 0)) && (w->format != XQ_FMT_FP8 || g_fp8_direct) &&
+        MidPlan mid;
+        const bool by_size = planned || (two_dense && g_tile_policy == 0);
+        // (its storages: the formats' usual groups and scale types; 32-bit offsets from a base for the operands)
+        const bool mid_storage = w->format == XQ_FMT_FP8 || (w->format == XQ_FMT_INT4 && g.group == 128 && g.scale_dtype == XQ_SCALE_BF16) ||
+                                 (w->format == XQ_FMT_NVFP4 && g.group == 16 && g.scale_dtype == XQ_SCALE_E4M3) ||
+                                 (w->format == XQ_FMT_NF4 && g.group == 64 && g.scale_dtype == XQ_SCALE_F32);
+        if (by_size && fmt_ok && mid_storage && (w->format != XQ_FMT_FP8 || g_fp8_direct) && g.wcols % (w->format == XQ_FMT_FP8 ? 16 : g.group) == 0 &&
+            takes_mid(w->format, contract_cols, n_rows, g.Nout, g.Kc, &mid) && n_rows * lda * 2 < (1ll << 32) &&
+            (int64_t)g.wrows * g.wcols < (1ll << 32) &&
+            (mid.split == 1 || (partial && xq_aligned(partial, 16) && partial_bytes >= mid.split * n_rows * g.Nout * 4))) {
+            G256Args f{};
+            f.A = A; f.lda = lda; f.C = C; f.ldc = ldc;
+            f.W = g.packed; f.scales = g.scales; f.global_scale = g.global_scale;
+            f.wrows = g.wrows; f.wcols = g.wcols; f.gshift = gshift; f.scale_dtype = g.scale_dtype;
+            f.Kc = g.Kc; f.Nout = g.Nout; f.M = n_rows; f.num_experts = 1;
+            if (two) { f.W2 = (const uint8_t*)two->w2->packed; f.scales2 = (const uint8_t*)two->w2->scales; f.nk1 = g.wrows / BK; }
+            f.su = g.r_pad ? su : nullptr; f.right = g.right; f.r_pad = g.r_pad; f.ld_su = g.r_pad;
+            f.bias = bias;
+            f.ksplit = mid.split; f.partial = mid.split > 1 ? partial : nullptr;
+            f.wide_rows = xq_aligned(C, 16) && ldc % 8 == 0;
+            return launch_mid(f, contract_cols, w->format, mid.mw, stream, who);
+        }
+        if (by_size && (w->format != XQ_FMT_FP8 || g_fp8_direct) &&
             decode_first(w->format, n_rows, g.Nout, g.Kc) && partial && xq_aligned(partial, 16) &&
             partial_bytes >= decoded_scratch_bytes(w->format, n_rows, g.Nout, g.Kc) && n_rows * lda * 2 < (1ll << 32) && xq_cdiv(n_rows, 256) * xq_cdiv(g.Nout, 256) < (1ll << 31) && g.Nout < 65536 * 16) {
             G256Args f{};

@@ -239,3 +239,33 @@ def test_merge_requant_int4(hip_device, N, K, r, symmetric):
     assert m._scale_dtypes["weight_scales"] == scales.dtype
     w_new = m._dequantize_weight().cpu().float()
     assert (w_new - merged.float()).abs().mean() / merged.float().abs().mean() < 0.16   # 15 or 16 levels per group: mean error ~ absmax / 28
+
+
+@pytest.mark.parametrize("r", [0, 16])
+@pytest.mark.parametrize("fmt", ["int4", "int4_symmetric", "nf4"])
+def test_requant_over_the_range_of_scales(hip_device, fmt, r):
+    """Groups from 2^-130 to 2^120, a last block of rows that is not full: the encoders' scaled and residual steps against the
+    oracle's divisions, codes and scales byte for byte (a symmetric code is the rounded quotient; its ties are exact)."""
+    from xorl_amd import _C
+    from xorl_amd.functional import QuantWeight, merge_dense, merge_requant_int4, merge_requant_nf4
+
+    N, K, group = 331, 512, 64 if fmt == "nf4" else 128
+    g = np.random.default_rng(7 + r)
+    packed = torch.from_numpy(g.integers(0, 256, (N, K // 2), dtype=np.uint8)).to(hip_device)
+    # eight significant bits: products with the codes, and quotients of them, meet every rounding case
+    scales = (1 + g.integers(0, 128, (N, K // group)) / 128) * 2.0 ** g.integers(-130, 121, (N, K // group))
+    qw = QuantWeight("nf4" if fmt == "nf4" else "int4", _C.XQ_LAYOUT_FLAT, packed,
+                     torch.from_numpy(scales.astype(np.float32)).to(hip_device), torch.float32, N, K, group)
+    A = gen((16, K), 1.0, 5).to(hip_device)
+    B = (gen((N, 16), 1.0, 6) * 2.0 ** torch.from_numpy(g.integers(-120, 100, (N, 1))).float()).to(hip_device)
+    merged = merge_dense(qw, A, B, r, 0.5, torch.bfloat16).cpu().float()
+    assert bool(torch.isfinite(merged).all())
+    if fmt == "nf4":
+        codes, got = merge_requant_nf4(qw, A, B, r, 0.5)
+        want, want_scales = C.nf4_quantize_flat(merged.numpy(), group)
+    else:
+        sym = fmt == "int4_symmetric"
+        codes, got = merge_requant_int4(qw, A, B, r, 0.5, sym)
+        want, want_scales = (C.int4_quantize_sym_flat if sym else C.int4_quantize_flat)(merged.numpy(), group)
+    assert np.array_equal(got.cpu().contiguous().view(torch.uint8).numpy().reshape(-1), np.asarray(want_scales).reshape(-1).view(np.uint8))
+    assert np.array_equal(codes.cpu().numpy().reshape(-1), np.asarray(want).reshape(-1))

@@ -1,4 +1,4 @@
-// Values -> 4-bit codes, for the quantizers.  (The re-quantising merge has encoders of its own.)
+// Values -> 4-bit codes, for the quantizers and the re-quantising merge.
 #pragma once
 #include "xq_common.h"
 

@@ -22,6 +22,7 @@
 //      s = max(amax / 448, 1e-12) and writes e4m3(clamp(x / s)) bytes and the scale: decode -> add ->
 //      re-encode in one pass over 1 byte per weight each way.
 #include "xq_common.h"
+#include "xq_codes.h"
 #include <atomic>
 #include "xq_lora.h"
 
@@ -59,29 +60,6 @@ struct MergeArgs {
     float* gscale_out;   // mode 4: one float
 };
 
-// NF4 code of a value already normalised into [-1, 1]: the number of midpoints between neighbouring levels that lie
-// strictly below it (ops/quantize/nf4_codec.py:42-64)
-__device__ __forceinline__ uint32_t nf4_encode(float v) {
-    constexpr float kMid[15] = {(float)-0.8480964004993439, (float)-0.6106329262256622, (float)-0.4599952697753906,
-                                (float)-0.3396794348955154, (float)-0.2346074059605598, (float)-0.1379117332398891,
-                                (float)-0.0455250181257725, (float)0.0397901497781277,  (float)0.1202552504837513,
-                                (float)0.2035212516784668,  (float)0.2920137718319893,  (float)0.3893125355243683,
-                                (float)0.5016634166240692,  (float)0.6427869200706482,  (float)0.8614784181118012};
-    uint32_t c = 0;
-#pragma unroll
-    for (int i = 0; i < 15; ++i) c += v > kMid[i] ? 1u : 0u;
-    return c;
-}
-
-// e2m1 code of a value already scaled into [-6, 6] (ops/quantize/fp4_codec.py:12-19: ties go up in magnitude)
-__device__ __forceinline__ uint32_t fp4_encode(float v) {
-    const float a = fabsf(v);
-    int lo = (int)(a * 2.0f + 0.5f);
-    lo = lo > 3 ? 3 : lo;
-    const int hi = 4 + (a >= 2.5f) + (a >= 3.5f) + (a >= 5.0f);
-    return (uint32_t)(a >= 1.75f ? hi : lo) + (v < 0.0f ? 8u : 0u);
-}
-
 // hi/lo bf16 split of the factors, once per call instead of once per tile: Bh/Bl[n][j] from scaling * B[n][j],
 // Ah/Al[k][j] from A[j][k] (transposed so that a tile's MFMA operand rows are contiguous 16-byte pieces).
 // Rows beyond N / K (up to the next multiple of 128) and ranks beyond r are zero, so the tile kernel reads the
@@ -111,20 +89,72 @@ __global__ void __launch_bounds__(256) merge_prep_kernel(MergeArgs g, int npad, 
     }
 }
 
-// REQ: the block-fp8 re-quantise mode (results are held in registers until the tile's absmax is known) and, for an
-// int4 weight, the int4 one (held until the row's 128-element group, which is the tile's whole row, is known).
-// 512 threads per tile: 32 result registers per thread in that mode, so that two blocks (16 waves) fit a CU.
-template <int FMT, int RP, bool REQ>
+// N values are rounded to bf16 and come back as floats: pairs[i] the packed results
+template <int N>
+__device__ __forceinline__ void round_pairs(const float* v, uint32_t* pairs, float* out) {
+#pragma unroll
+    for (int i = 0; i < N / 2; ++i) {
+        pairs[i] = pack_bf16x2(v[2 * i], v[2 * i + 1]);
+        out[2 * i] = __uint_as_float(pairs[i] << 16);
+        out[2 * i + 1] = __uint_as_float(pairs[i] & 0xffff0000u);
+    }
+}
+
+// 16 consecutive 4-bit codes of one scale -> fp32 values, by pairs: the values of val4 (xq_common.h).  int4: a byte 0x0n read as
+// e4m3 is n * 2^-9, and n - 8 is exact.
+template <int FMT>
+__device__ __forceinline__ void values16(float (&v)[16], uint32_t w0, uint32_t w1, float s, const float* levels) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const uint32_t w = u ? w1 : w0;
+        float* o = v + 8 * u;
+        if constexpr (FMT == XQ_FMT_INT4) {
+            const uint32_t ev = w & 0x0f0f0f0fu, od = (w >> 4) & 0x0f0f0f0fu;
+            const f32x2 e01 = e4m3x2_to_f32(ev, false), e23 = e4m3x2_to_f32(ev, true);
+            const f32x2 o01 = e4m3x2_to_f32(od, false), o23 = e4m3x2_to_f32(od, true);
+            const float n[8] = {e01[0], o01[0], e01[1], o01[1], e23[0], o23[0], e23[1], o23[1]};
+#pragma unroll
+            for (int i = 0; i < 8; ++i) o[i] = __builtin_fmaf(n[i], 512.0f, -8.0f) * s;
+        } else if constexpr (FMT == XQ_FMT_NVFP4) {
+            const f32x2 x0 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 0), x1 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 1);
+            const f32x2 x2 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 2), x3 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 3);
+            o[0] = x0[0] * s; o[1] = x0[1] * s; o[2] = x1[0] * s; o[3] = x1[1] * s;
+            o[4] = x2[0] * s; o[5] = x2[1] * s; o[6] = x3[0] * s; o[7] = x3[1] * s;
+        } else {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) o[i] = levels[(w >> (4 * i)) & 0xfu] * s;
+        }
+    }
+}
+
+// MODE: MergeArgs::mode.  It is a template argument because the passes below are bound by their vector instructions: with the mode
+// (and the kind of scales) tested at run time, element by element, the compiler left 64 small blocks with a branch each in the
+// middle of the pass.  With that, pairwise conversions and the encoders of the quantizers, [12288, 4096], r 32, us with the
+// preparing launch: block-fp8 publish 41.7 -> 36.2, requantise 35.7 -> 32.6; int4 46.7 -> 41.2, 65.2 -> 50.1; nvfp4 56.7 -> 41.4,
+// 131.6 -> 102.4 (absmax and codes); nf4 56.6 -> 43.6, 92.0 -> 53.7.
+// REQ: the modes that hold a tile's results in registers until its absmax (block-fp8) or the row's 128-element group, the
+// tile's whole row (int4), is known.
+// 512 threads per tile: 32 result registers per thread in those, so that two blocks (16 waves) fit a CU.
+template <int FMT, int RP, int MODE>
 __global__ void __launch_bounds__(512, 4) merge_kernel(MergeArgs g) {
+    constexpr bool REQ = MODE == 2 || MODE >= 6;
+    constexpr bool ROUNDED = MODE == 0 || MODE >= 3 || FMT != XQ_FMT_FP8;       // sums of bf16 values (4-bit decoders return bf16)
     asm volatile("" ::"s"(g.packed), "s"(g.scales), "s"(g.global_scale), "s"(g.group), "s"(g.scale_dtype), "s"(g.N), "s"(g.K),
-                 "s"(g.Bh), "s"(g.Bl), "s"(g.Ah), "s"(g.Al), "s"(g.mode), "s"(g.out), "s"(g.packed_out), "s"(g.scales_out));
+                 "s"(g.Bh), "s"(g.Bl), "s"(g.Ah), "s"(g.Al), "s"(g.out), "s"(g.packed_out), "s"(g.scales_out));
     // (all arguments in scalar registers after one round trip)
     extern __shared__ __attribute__((aligned(16))) uint8_t mg_lds[];
     __shared__ float sh_amax[8];
+    __shared__ float sh_level[FMT == XQ_FMT_NF4 ? 16 : 1];
+    __shared__ Nf4Bucket sh_bucket[MODE == 5 ? 32 : 1];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int k0 = blockIdx.x * MG_T, n0 = blockIdx.y * MG_T;
     constexpr bool FP8 = FMT == XQ_FMT_FP8;
+    if constexpr (FMT == XQ_FMT_NF4)
+        if (tid < 16) sh_level[tid] = kNf4Level[tid];
+    if constexpr (MODE == 5)
+        if (tid >= 64 && tid < 96) sh_bucket[tid - 64] = nf4_bucket(tid - 64);
+    if constexpr (RP == 0 && FMT == XQ_FMT_NF4) __syncthreads();       // (otherwise a barrier of the update lies between)
     auto lds_barrier = [&]() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
 
     // ---- 0a. this tile's rows of the four factor panels -> registers (16-byte pieces, each tile one contiguous
@@ -219,7 +249,7 @@ __global__ void __launch_bounds__(512, 4) merge_kernel(MergeArgs g) {
         }
         const int k = k0 + h * 64 + rcol;
         const bool ok = n < g.N && k < g.K;               // K % 16 == 0: runs are all in or all out
-        float v[16];
+        float v[16], x[16];
         if (FP8) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
@@ -227,41 +257,48 @@ __global__ void __launch_bounds__(512, 4) merge_kernel(MergeArgs g) {
                 v[4 * i] = lo[0] * tile_scale; v[4 * i + 1] = lo[1] * tile_scale;
                 v[4 * i + 2] = hi[0] * tile_scale; v[4 * i + 3] = hi[1] * tile_scale;
             }
-        } else {
+        } else if (run_scale) {
             const uint32_t sr = sraw[h];
             const float srun = g.scale_dtype == XQ_SCALE_F32 ? __uint_as_float(sr)
                              : g.scale_dtype == XQ_SCALE_BF16 ? __uint_as_float(sr << 16) : e4m3_to_f32((uint8_t)sr);
-#pragma unroll
+            values16<FMT>(v, wr[h][0], wr[h][1], FMT == XQ_FMT_NVFP4 ? srun * gs : srun, sh_level);
+        } else {
+            // groups that are not multiples of 16 (never with the reference's formats): per-element lookup
             for (int i = 0; i < 16; ++i) {
-                const uint32_t nib = (wr[h][i >> 3] >> (4 * (i & 7))) & 0xfu;
-                // groups that are not multiples of 16 (never with the reference's formats): per-element lookup
-                const float sc = run_scale ? srun : load_scale(g.scales, (nrow * g.K + (k < g.K ? k : 0) + i) / g.group, g.scale_dtype);
-                v[i] = val4<FMT>(nib, FMT == XQ_FMT_NVFP4 ? sc * gs : sc);
+                const float sc = load_scale(g.scales, (nrow * g.K + (k < g.K ? k : 0) + i) / g.group, g.scale_dtype);
+                const float t = val4<FMT>((wr[h][i >> 3] >> (4 * (i & 7))) & 0xfu, FMT == XQ_FMT_NVFP4 ? sc * gs : sc);
+#pragma unroll
+                for (int e = 0; e < 16; ++e) v[e] = e == i ? t : v[e];
             }
         }
-        float x[16];
+        float d[16];
 #pragma unroll
         for (int i = 0; i < 16; i += 4) {
-            f32x4 d = {0.0f, 0.0f, 0.0f, 0.0f};
-            if (RP > 0) d = *(const f32x4*)(dt + rrow * MG_HP + rcol + i);
+            f32x4 t = {0.0f, 0.0f, 0.0f, 0.0f};
+            if (RP > 0) t = *(const f32x4*)(dt + rrow * MG_HP + rcol + i);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                float t;
-                if (g.mode == 0 || g.mode >= 3 || !FP8) t = bf16_to_f32(to_bf16(bf16_to_f32(to_bf16(v[i + e])) + bf16_to_f32(to_bf16(d[e]))));   // 4-bit decoders return bf16
-                else t = v[i + e] + d[e];
-                x[i + e] = ok ? t : 0.0f;
-            }
+            for (int e = 0; e < 4; ++e) d[i + e] = t[e];
         }
-        if (REQ) {
+        uint32_t px[8];                                   // the values as bf16 pairs (ROUNDED)
+        if constexpr (ROUNDED) {
+            round_pairs<16>(v, px, v);
+            round_pairs<16>(d, px, d);
+#pragma unroll
+            for (int i = 0; i < 16; ++i) x[i] = v[i] + d[i];
+            round_pairs<16>(x, px, x);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) x[i] = v[i] + d[i];
+        }
+        if constexpr (REQ || MODE == 3) {
+            float hm = 0.0f;
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
-                m[h * 16 + i] = x[i];
-                amax = fmaxf(amax, fabsf(x[i]));
+                if constexpr (REQ) m[h * 16 + i] = x[i];
+                hm = fmaxf(hm, fabsf(x[i]));
             }
-        } else if (g.mode == 3) {
-#pragma unroll
-            for (int i = 0; i < 16; ++i) amax = fmaxf(amax, fabsf(x[i]));
-        } else if (g.mode == 4) {
+            amax = fmaxf(amax, ok ? hm : 0.0f);
+        } else if constexpr (MODE == 4) {
             // one nvfp4 block per run (ops/quantize/nvfp4_quantize.py:25-60,102-111): codes against the raw block
             // amax, block scale = e4m3(amax / global amax * 448)
             if (ok) {
@@ -269,19 +306,19 @@ __global__ void __launch_bounds__(512, 4) merge_kernel(MergeArgs g) {
 #pragma unroll
                 for (int i = 0; i < 16; ++i) bmax = fmaxf(bmax, fabsf(x[i]));
                 bmax = fmaxf(bmax, 1e-12f);
-                const float q = 6.0f / bmax;
+                const float q4 = 6.0f / bmax * 4.0f;
                 uint32_t lo = 0, hi = 0;
 #pragma unroll
                 for (int i = 0; i < 8; ++i) {
-                    lo |= fp4_encode(__builtin_amdgcn_fmed3f(x[i] * q, -6.0f, 6.0f)) << (4 * i);
-                    hi |= fp4_encode(__builtin_amdgcn_fmed3f(x[8 + i] * q, -6.0f, 6.0f)) << (4 * i);
+                    lo |= fp4_code4(__builtin_amdgcn_fmed3f(x[i] * q4, -24.0f, 24.0f)) << (4 * i);
+                    hi |= fp4_code4(__builtin_amdgcn_fmed3f(x[8 + i] * q4, -24.0f, 24.0f)) << (4 * i);
                 }
                 *(u32x2*)(g.codes_out + ((n * g.K + k) >> 1)) = u32x2{lo, hi};
                 const float gm = fmaxf(g.gamax[0], 1e-12f);
                 const float bs = __builtin_amdgcn_fmed3f(bmax / gm * 448.0f, -448.0f, 448.0f);
                 g.bscale_out[(n * g.K + k) >> 4] = (uint8_t)(__builtin_amdgcn_cvt_pk_fp8_f32(bs, 0.0f, 0u, false) & 0xffu);
             }
-        } else if (g.mode == 5) {
+        } else if constexpr (MODE == 5) {
             // NF4 (ops/quantize/nf4_quantize.py:20-56): a 64-element group is the four runs of four neighbouring lanes;
             // scale = max(absmax, 1e-12), code = encode(clamp(x * (1 / scale), +-1))
             float bmax = 0.0f;
@@ -294,20 +331,17 @@ __global__ void __launch_bounds__(512, 4) merge_kernel(MergeArgs g) {
                 uint32_t lo = 0, hi = 0;
 #pragma unroll
                 for (int i = 0; i < 8; ++i) {
-                    lo |= nf4_encode(__builtin_amdgcn_fmed3f(x[i] * inv, -1.0f, 1.0f)) << (4 * i);
-                    hi |= nf4_encode(__builtin_amdgcn_fmed3f(x[8 + i] * inv, -1.0f, 1.0f)) << (4 * i);
+                    lo |= nf4_code(__builtin_amdgcn_fmed3f(x[i] * inv, -1.0f, 1.0f), sh_bucket) << (4 * i);
+                    hi |= nf4_code(__builtin_amdgcn_fmed3f(x[8 + i] * inv, -1.0f, 1.0f), sh_bucket) << (4 * i);
                 }
                 *(u32x2*)(g.codes_out + ((n * g.K + k) >> 1)) = u32x2{lo, hi};
                 if ((tid & 3) == 0) g.scales_out[(n * g.K + k) >> 6] = sc;
             }
         } else if (ok) {
-            if (g.mode == 0) {
+            if constexpr (MODE == 0) {
                 bf16_t* o = (bf16_t*)g.out + n * g.K + k;
-                uint32_t pk[8];
-#pragma unroll
-                for (int i = 0; i < 8; ++i) pk[i] = pack_bf16x2(x[2 * i], x[2 * i + 1]);
-                *(u32x4*)o = u32x4{pk[0], pk[1], pk[2], pk[3]};
-                *(u32x4*)(o + 8) = u32x4{pk[4], pk[5], pk[6], pk[7]};
+                *(u32x4*)o = u32x4{px[0], px[1], px[2], px[3]};
+                *(u32x4*)(o + 8) = u32x4{px[4], px[5], px[6], px[7]};
             } else {
                 float* o = (float*)g.out + n * g.K + k;
 #pragma unroll
@@ -323,15 +357,27 @@ __global__ void __launch_bounds__(512, 4) merge_kernel(MergeArgs g) {
         if (n >= g.N) return;
         const int64_t gi = (n * g.K + k0) >> 7;
         uint32_t pk[4] = {0u, 0u, 0u, 0u};
-        if (g.mode == 6) {
+        if constexpr (MODE == 6) {
             // scale = bf16(absmax / 7); code = clamp(rne(x / scale), -7, 7) + 8, all zero codes (8) for a zero group
             const bf16_t sb = to_bf16(ga / 7.0f);
             const float sc = bf16_to_f32(sb);
             if ((tid & 3) == 0) ((bf16_t*)g.scales_out)[gi] = sb;
+            if (sc > 1e-30f && sc <= 3.0e38f) {
+                // m and sc have 8 significant bits: a quotient that is no tie lies 2^-12 or more off one, far beyond the error of
+                // m * (1 / sc), and the residual step returns ties (half integers) exactly -- the rounded quotient's codes with
+                // 3 instructions for the division's 10 (an infinite scale leaves finite values at code 8: the division's case)
+                const float inv = 1.0f / sc;
 #pragma unroll
-            for (int i = 0; i < 32; ++i) {
-                const float q = sc > 0.0f ? __builtin_amdgcn_fmed3f(__builtin_rintf(m[i] / sc), -7.0f, 7.0f) : 0.0f;
-                pk[i >> 3] |= (uint32_t)((int)q + 8) << (4 * (i & 7));
+                for (int i = 0; i < 32; ++i) {
+                    const float y = m[i] * inv, t = __builtin_fmaf(__builtin_fmaf(-y, sc, m[i]), inv, y);
+                    pk[i >> 3] |= (uint32_t)((int)__builtin_amdgcn_fmed3f(__builtin_rintf(t), -7.0f, 7.0f) + 8) << (4 * (i & 7));
+                }
+            } else {
+#pragma unroll
+                for (int i = 0; i < 32; ++i) {
+                    const float q = sc > 0.0f ? __builtin_amdgcn_fmed3f(__builtin_rintf(m[i] / sc), -7.0f, 7.0f) : 0.0f;
+                    pk[i >> 3] |= (uint32_t)((int)q + 8) << (4 * (i & 7));
+                }
             }
         } else {
             // ops/quantize/int4_quantize.py:12-41: scale = max(absmax, 1e-12) * (2/15); code = clamp(trunc(x * (1 / scale)
@@ -351,8 +397,8 @@ __global__ void __launch_bounds__(512, 4) merge_kernel(MergeArgs g) {
         }
         return;
     }
-    if (!REQ) {
-        if (g.mode == 3) {       // tile absmax -> one atomic per block (values are non-negative: integer order = float order)
+    if constexpr (!REQ) {
+        if constexpr (MODE == 3) {       // tile absmax -> one atomic per block (values are non-negative: integer order = float order)
 #pragma unroll
             for (int off = 32; off >= 1; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 64));
             if (lane == 0) sh_amax[wave] = amax;
@@ -362,7 +408,7 @@ __global__ void __launch_bounds__(512, 4) merge_kernel(MergeArgs g) {
                 for (int i = 0; i < 8; ++i) t = fmaxf(t, sh_amax[i]);
                 atomicMax((unsigned int*)g.amax_out, __float_as_uint(t));
             }
-        } else if (g.mode == 4 && tid == 0 && blockIdx.x == 0 && blockIdx.y == 0) {
+        } else if (MODE == 4 && tid == 0 && blockIdx.x == 0 && blockIdx.y == 0) {
             // global scale = amax / 6 / 448 in the quantizer's operation order
             g.gscale_out[0] = fmaxf(g.gamax[0], 1e-12f) * (1.0f / 6.0f) / 448.0f;
         }
@@ -410,32 +456,32 @@ static double merge_bytes(const xq_weight* w, int mode) {
     return in + (mode == 0 ? 2.0 * n : mode == 1 ? 4.0 * n : mode == 3 ? 0.0 : in);
 }
 
-template <int FMT, int RP, bool REQ>
+template <int FMT, int RP, int MODE>
 static int launch_merge_one(const MergeArgs& g, dim3 grid, hipStream_t s, const char* who) {
     // LDS: the four factor tiles, then the delta half tile in their place
     constexpr size_t lds_f = (size_t)4 * MG_T * (RP + 8) * 2, lds_d = (size_t)MG_T * MG_HP * 4;
     constexpr size_t lds = RP == 0 ? 16 : (lds_f > lds_d ? lds_f : lds_d);
     static std::atomic<bool> attr_set{false};   // per instantiation; the attribute call is idempotent: a race only repeats it
     if (!attr_set && lds > 64 * 1024) {
-        hipError_t e = hipFuncSetAttribute((const void*)merge_kernel<FMT, RP, REQ>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        hipError_t e = hipFuncSetAttribute((const void*)merge_kernel<FMT, RP, MODE>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) {
             xq_set_error("%s: cannot raise the dynamic LDS limit: %s", who, hipGetErrorString(e));
             return XQ_ERR_LAUNCH;
         }
         attr_set = true;
     }
-    merge_kernel<FMT, RP, REQ><<<grid, 512, lds, s>>>(g);
+    merge_kernel<FMT, RP, MODE><<<grid, 512, lds, s>>>(g);
     return XQ_OK;
 }
 
-template <int FMT, bool REQ>
+template <int FMT, int MODE>
 static int launch_merge_fmt(const MergeArgs& g, dim3 grid, hipStream_t s, const char* who) {
     switch (g.r_pad) {
-        case 0: return launch_merge_one<FMT, 0, REQ>(g, grid, s, who);
-        case 16: return launch_merge_one<FMT, 16, REQ>(g, grid, s, who);
-        case 32: return launch_merge_one<FMT, 32, REQ>(g, grid, s, who);
-        case 48: return launch_merge_one<FMT, 48, REQ>(g, grid, s, who);
-        default: return launch_merge_one<FMT, 64, REQ>(g, grid, s, who);
+        case 0: return launch_merge_one<FMT, 0, MODE>(g, grid, s, who);
+        case 16: return launch_merge_one<FMT, 16, MODE>(g, grid, s, who);
+        case 32: return launch_merge_one<FMT, 32, MODE>(g, grid, s, who);
+        case 48: return launch_merge_one<FMT, 48, MODE>(g, grid, s, who);
+        default: return launch_merge_one<FMT, 64, MODE>(g, grid, s, who);
     }
 }
 
@@ -486,12 +532,13 @@ static int launch_merge(const xq_weight* w, const void* A, const void* B, int lo
     const bool timed = xq_profile_mark_begin(stream, merge_bytes(w, mode));
     if (g.r_pad > 0)
         merge_prep_kernel<<<dim3((unsigned)xq_cdiv((npad + kpad) * g.r_pad, 256)), 256, 0, stream>>>(g, (int)npad, (int)kpad);
-    if (w->format == XQ_FMT_FP8) rc = mode == 2 ? launch_merge_fmt<XQ_FMT_FP8, true>(g, grid, stream, who)
-                                                : launch_merge_fmt<XQ_FMT_FP8, false>(g, grid, stream, who);
-    else if (w->format == XQ_FMT_INT4) rc = mode >= 6 ? launch_merge_fmt<XQ_FMT_INT4, true>(g, grid, stream, who)
-                                                      : launch_merge_fmt<XQ_FMT_INT4, false>(g, grid, stream, who);
-    else if (w->format == XQ_FMT_NF4) rc = launch_merge_fmt<XQ_FMT_NF4, false>(g, grid, stream, who);
-    else rc = launch_merge_fmt<XQ_FMT_NVFP4, false>(g, grid, stream, who);
+    rc = XQ_ERR_UNSUPPORTED;
+#define XQ_MERGE(FMT, MODE) if (w->format == FMT && mode == MODE) rc = launch_merge_fmt<FMT, MODE>(g, grid, stream, who)
+    XQ_MERGE(XQ_FMT_FP8, 0); XQ_MERGE(XQ_FMT_FP8, 1); XQ_MERGE(XQ_FMT_FP8, 2); XQ_MERGE(XQ_FMT_FP8, 3);
+    XQ_MERGE(XQ_FMT_INT4, 0); XQ_MERGE(XQ_FMT_INT4, 1); XQ_MERGE(XQ_FMT_INT4, 3); XQ_MERGE(XQ_FMT_INT4, 6); XQ_MERGE(XQ_FMT_INT4, 7);
+    XQ_MERGE(XQ_FMT_NVFP4, 0); XQ_MERGE(XQ_FMT_NVFP4, 1); XQ_MERGE(XQ_FMT_NVFP4, 3); XQ_MERGE(XQ_FMT_NVFP4, 4);
+    XQ_MERGE(XQ_FMT_NF4, 0); XQ_MERGE(XQ_FMT_NF4, 1); XQ_MERGE(XQ_FMT_NF4, 3); XQ_MERGE(XQ_FMT_NF4, 5);
+#undef XQ_MERGE
     if (timed) xq_profile_mark_end(stream);
     if (rc) return rc;
     XQ_CHECK_LAUNCH(who);

@@ -57,11 +57,11 @@ MEASURED_TRAFFIC = {
     # (M = 32, 64): mean per forward over the 32 cases (includes the fp32 partial tiles of the two-launch cases
     # written and read back: 23.3 MiB of it are algorithmic)
     4: (34.2 * 2 ** 20, "profiles/skinny_kernels_decode_shapes.txt", 0.01557),
-    # merge_prep_kernel + merge_kernel<fp8>: mean per call (re-quantise 96 MiB, publish 144 MiB algorithmic)
+    # merge_fp8_kernel and merge_kernel<fp8>: mean per call (re-quantise 96 MiB, publish 144 MiB algorithmic)
     5: (134.4 * 2 ** 20, "profiles/merge_kernel_fp8_mlp_weights.txt", 0.04168),
     # gemm_256_kernel<nvfp4 GKN, grouped>: mean over the 6 launches of a step
     7: (893.9 * 2 ** 20, "profiles/gemm_256_nvfp4_gkn_grouped_moe_e128.txt", 0.52825),
-    # merge_prep_kernel + merge_kernel<nvfp4>: mean per call over amax / re-quantise / publish of the four weights
+    # merge_kernel<nvfp4>: mean per call over amax / re-quantise / publish of the four weights
     9: (59.0 * 2 ** 20, "profiles/merge_kernel_nvfp4_attn_weights.txt", 0.03500),
 }
 

@@ -300,8 +300,7 @@ int xq_linear_bwd(const xq_weight* w, const void* x, int64_t ldx, const void* dy
  * packed_out / scales_out may be the weight's own buffers (in-place).
  *
  * Both take a workspace of xq_merge_workspace_bytes(N, K, r) bytes (256-byte
- * aligned; may be NULL when r == 0): the factors are split once per call
- * into bf16 hi/lo panels there. */
+ * aligned; may be NULL when r == 0), of which they keep nothing at present. */
 int64_t xq_merge_workspace_bytes(int64_t N, int64_t K, int r);
 int xq_merge_dense(const xq_weight* w, const void* lora_A, const void* lora_B, int lora_dtype, int r,
                    float scaling, void* out, int out_dtype, void* workspace, int64_t workspace_bytes,

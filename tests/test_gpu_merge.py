@@ -269,3 +269,62 @@ def test_requant_over_the_range_of_scales(hip_device, fmt, r):
         want, want_scales = (C.int4_quantize_sym_flat if sym else C.int4_quantize_flat)(merged.numpy(), group)
     assert np.array_equal(got.cpu().contiguous().view(torch.uint8).numpy().reshape(-1), np.asarray(want_scales).reshape(-1).view(np.uint8))
     assert np.array_equal(codes.cpu().numpy().reshape(-1), np.asarray(want).reshape(-1))
+
+
+@pytest.mark.parametrize("r,dtype", [(0, torch.float32), (7, torch.float32), (16, torch.bfloat16), (32, torch.float32),
+                                     (40, torch.bfloat16), (64, torch.float32)])
+@pytest.mark.parametrize("fmt", ["block_fp8", "int4", "nvfp4", "nf4"])
+def test_several_tiles_a_block(hip_device, fmt, r, dtype):
+    """More tiles than blocks: runs that cross from one column strip to the next, last rows and columns that fill no tile.  Slices of
+    256 rows have one tile a block (the form that the tests above pin to the oracle); whole matrix and slices have to agree to the
+    bit, requantised in place as well."""
+    from xorl_amd import _C
+    from xorl_amd.functional import (QuantWeight, merge_amax, merge_dense, merge_requant_fp8, merge_requant_int4, merge_requant_nf4,
+                                     merge_requant_nvfp4)
+
+    g = np.random.default_rng(r)
+    N, K = 37 * 128 + 48, 3840 if fmt == "int4" else 3776 if fmt == "nf4" else 3792
+    A, B = gen((max(r, 1), K), 0.3, 1).to(hip_device, dtype), gen((N, max(r, 1)), 0.3, 2).to(hip_device, dtype)
+    if fmt == "block_fp8":
+        packed = torch.from_numpy(g.integers(0, 0x7f, (N, K), dtype=np.uint8) | (g.integers(0, 2, (N, K), dtype=np.uint8) << 7))
+        scales, group, rows_per_scale = torch.rand(38, 30) * 0.01 + 0.001, 128, 128
+    else:
+        packed = torch.from_numpy(g.integers(0, 256, (N, K // 2), dtype=np.uint8))
+        group, rows_per_scale = {"int4": 128, "nvfp4": 16, "nf4": 64}[fmt], 1
+        scales = torch.rand(N, K // group) * 0.1 + 0.01
+        if fmt == "nvfp4":
+            scales = scales.to(torch.float8_e4m3fn)
+    gscale = torch.tensor([0.7], device=hip_device) if fmt == "nvfp4" else None
+    packed, scales = packed.to(hip_device), scales.to(hip_device)
+    sdt = scales.dtype
+
+    def weight(lo, hi):
+        s = scales[lo // rows_per_scale : -(-hi // rows_per_scale)]
+        return QuantWeight(fmt, _C.XQ_LAYOUT_FLAT, packed[lo:hi], s, sdt, hi - lo, K, group, global_scale=gscale)
+
+    gamax = torch.tensor([3.0], device=hip_device)
+
+    def requant(w, b):
+        if fmt == "block_fp8":
+            return merge_requant_fp8(w, A, b, r, 0.5)
+        if fmt == "nvfp4":
+            return merge_requant_nvfp4(w, A, b, r, 0.5, gamax)[:2]
+        return merge_requant_nf4(w, A, b, r, 0.5) if fmt == "nf4" else merge_requant_int4(w, A, b, r, 0.5, True)
+
+    whole = weight(0, N)
+    dense, f32, (codes, new_scales) = merge_dense(whole, A, B, r, 0.5, torch.bfloat16), merge_dense(whole, A, B, r, 0.5, torch.float32), requant(whole, B)
+    amax = merge_amax(whole, A, B, r, 0.5)
+    assert amax.item() == dense.float().abs().max().item()
+    codes, new_scales = codes.reshape(N, -1).view(torch.uint8), new_scales.reshape(-(-N // rows_per_scale), -1)
+    for lo in range(0, N, 256):
+        hi = min(lo + 256, N)
+        w, b = weight(lo, hi), B[lo:hi]
+        assert torch.equal(merge_dense(w, A, b, r, 0.5, torch.bfloat16), dense[lo:hi])
+        assert torch.equal(merge_dense(w, A, b, r, 0.5, torch.float32), f32[lo:hi])
+        c, s = requant(w, b)
+        assert torch.equal(c.reshape(hi - lo, -1).view(torch.uint8), codes[lo:hi])
+        assert torch.equal(s.reshape(-1).view(torch.uint8),
+                           new_scales[lo // rows_per_scale : -(-hi // rows_per_scale)].reshape(-1).view(torch.uint8))
+    if fmt == "block_fp8":                                       # in place
+        merge_requant_fp8(whole, A, B, r, 0.5, packed, scales)
+        assert torch.equal(packed, codes) and torch.equal(scales, new_scales)

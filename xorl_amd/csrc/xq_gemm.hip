@@ -185,39 +185,64 @@ static DensePlan plan_dense(int64_t n_rows, int64_t Nout, int64_t nk) {
 // line up to 8192 rows) stay with the tile kernels.
 constexpr int64_t kDecMinRows = 640, kDecMinRowsFp8 = 6144;
 constexpr double kDecMinWork = 2.0e10;               // rows x columns x contraction
+// Tiles: 256 x 256 where they fill their rounds of the chip; otherwise the rows or columns of a tile are stretched or cut to what
+// leaves the last round fullest (288 tiles on 256 units are 240 of 288 rows).  Forward / dgrad, us, with 256 x 256 alone -> with all five:
+//   int4 [12288, 4096], 1357 rows: 148 / 164 -> 133 / 164; [8192 -> 5120], 4096 rows 298 -> 261; [4224 -> 7936], 2063 rows 136 / 186 -> 131 /
+//   157; [3712 -> 3200], 5416 rows 132 -> 111; [1536 -> 2816], 7253 rows 82 -> 61; [5248, 2176], 3606 rows 99 / 109 -> 79 / 103;
+//   nf4 [2304, 6528], 3675 rows 145 / 117 -> 121 / 110; nvfp4 [6272, 1280], 2709 rows 72 / 67 -> 54 / 67.
+// The leads below: two estimates of one product err against each other by up to 5 per cent; 224 rows, whose weight tile is read for
+// fewer rows, gave back less than the estimate said (six products of 13 were slower at a lead of 0.97, by up to 6 per cent).
+struct DecTile {
+    int tm, tn;               // 32 tm rows x 64 tn columns
+    double lead;              // what part of the time of the tiles before it its estimate has to stay under
+};
+static const DecTile kDecTiles[] = {{8, 4, 1.0}, {7, 4, 0.88}, {9, 4, 0.92}, {10, 4, 0.92}, {8, 5, 0.92}};
+struct DecPart {
+    int64_t rows;
+    int tile, split;          // index into kDecTiles; K splits
+};
 struct DecPlan {
-    int split;                // K splits of the leading rows
-    int64_t head_rows;        // leading rows; the others are a second launch in tail_split K splits
-    int tail_split;
+    DecPart part[2];          // leading rows, and the others (0: none) as a second launch
     int64_t partial;          // bytes of fp32 sums the splits take
     double us;                // the estimate it was chosen by
 };
 static DecPlan plan_decoded(int64_t n_rows, int64_t Nout, int64_t Kc) {
-    // microseconds: a round of the chip takes 0.8 per K-step (0.78-0.84 measured) and 5 around them; the fp32 sums of splits are
-    // written and read at about 5 TB/s
-    const int64_t tc = xq_cdiv(Nout, GeoDec::T), steps = Kc / GeoDec::BK, cus = num_cus();
-    auto cost = [&](int64_t rows, int s) {
-        const double rounds = (double)xq_cdiv(xq_cdiv(rows, GeoDec::T) * tc * s, cus);
-        const double sums = s > 1 ? 3.0 + (8.0 * s + 2.0) * (double)rows * (double)Nout / 5.0e6 : 0.0;
-        return rounds * ((double)xq_cdiv(steps, s) * 0.8 + 5.0) + sums;
+    // microseconds, fitted to 32 products on all five tiles in one to four splits (4.7 per cent rms): a K-step takes longer the more of
+    // the chip is at work (the matrix units share its power), by the tile's size; the fp32 sums of splits are written and read at
+    // about 6 TB/s
+    const int64_t steps = Kc / GeoDec::BK, cus = num_cus();
+    auto cost = [&](int tile, int64_t rows, int s) {
+        const DecTile t = kDecTiles[tile];
+        const double w = (double)(t.tm * t.tn) / 32.0, st = (double)xq_cdiv(steps, s) * w;
+        const int64_t blocks = xq_cdiv(rows, 32 * t.tm) * xq_cdiv(Nout, 64 * t.tn) * s, full = blocks / cus, rest = blocks % cus;
+        const double sums = s > 1 ? std::max(2.0, 0.165e-6 * (8.0 * s + 2.0) * (double)rows * (double)Nout - 4.6) : 0.0;
+        auto round = [&](double f) { return st * (0.423 + 0.288 * f) + 6.2 * w; };
+        return (double)full * round(1.0) + (rest ? round((double)rest / (double)cus) : 0.0) + sums;
     };
-    auto best = [&](int64_t rows, double* c) {
-        int b = 1;
-        *c = cost(rows, 1);
-        for (int s = 2; s <= 8 && steps / s >= 16; ++s)
-            if (cost(rows, s) < *c) { b = s; *c = cost(rows, s); }
-        return b;
+    auto best = [&](int64_t rows, DecPart* p) {
+        *p = DecPart{rows, 0, 1};
+        double c = cost(0, rows, 1);
+        for (int tile = 0; tile < (int)(sizeof(kDecTiles) / sizeof(kDecTiles[0])); ++tile)
+            for (int s = 1; s == 1 || (s <= 8 && steps / s >= 16); ++s) {
+                const double lead = tile == p->tile ? 1.0 : kDecTiles[tile].lead, u = cost(tile, rows, s);
+                if (u < lead * c) { *p = DecPart{rows, tile, s}; c = u; }
+            }
+        return c;
     };
-    double whole;
-    DecPlan p{best(n_rows, &whole), n_rows, 1, 0, whole};
-    const int64_t tr = xq_cdiv(n_rows, GeoDec::T), keep = tr * tc / cus * cus / tc;      // tile rows of whole rounds
+    DecPlan p{};
+    p.us = best(n_rows, &p.part[0]);
+    const int64_t tc = xq_cdiv(Nout, GeoDec::T), tr = xq_cdiv(n_rows, GeoDec::T), keep = tr * tc / cus * cus / tc;      // tile rows of whole rounds
     if (keep > 0 && keep < tr) {
-        double tail;
-        const int ts = best(n_rows - keep * GeoDec::T, &tail);
-        if (cost(keep * GeoDec::T, 1) + tail < whole) p = DecPlan{1, keep * GeoDec::T, ts, 0, cost(keep * GeoDec::T, 1) + tail};
+        DecPart tail;
+        const double c = cost(0, keep * GeoDec::T, 1) + best(n_rows - keep * GeoDec::T, &tail) + 4.0;
+        if (c < p.us) {
+            p.part[0] = DecPart{keep * GeoDec::T, 0, 1};
+            p.part[1] = tail;
+            p.us = c;
+        }
     }
-    const int64_t tail_rows = n_rows - p.head_rows;
-    p.partial = std::max(p.split > 1 ? p.split * p.head_rows : 0, tail_rows && p.tail_split > 1 ? p.tail_split * tail_rows : 0) * Nout * 4;
+    for (const DecPart& d : p.part)
+        if (d.split > 1) p.partial = std::max(p.partial, d.split * d.rows * Nout * 4);
     return p;
 }
 static bool decode_first(int fmt, int64_t n_rows, int64_t Nout, int64_t Kc) {
@@ -264,7 +289,7 @@ static MidPlan plan_mid(int fmt, bool cc, int64_t rows, int64_t Nout, int64_t Kc
 }
 // the same product without it: over a decoded image, or on 256- or 128-row tiles
 static double tile_kernels_us(int fmt, int64_t rows, int64_t Nout, int64_t Kc) {
-    if (decode_first(fmt, rows, Nout, Kc)) return 2.6 + 0.45e-6 * (double)Nout * (double)Kc + 0.8 * plan_decoded(rows, Nout, Kc).us;
+    if (decode_first(fmt, rows, Nout, Kc)) return 3.4 + (fmt == XQ_FMT_NF4 ? 0.5e-6 : 0.43e-6) * (double)Nout * (double)Kc + plan_decoded(rows, Nout, Kc).us;
     const double nk = (double)(Kc / 64);
     if (dense_tile_size(rows, Nout) == 256) {
         const int64_t tiles = xq_cdiv(rows, 256) * xq_cdiv(Nout, 256), cus = num_cus(), full = tiles / cus;
@@ -290,7 +315,7 @@ static bool takes_mid(int fmt, bool cc, int64_t rows, int64_t Nout, int64_t Kc, 
     if (!mid_shape(fmt, cc, rows, Nout, Kc)) return false;
     *plan = plan_mid(fmt, cc, rows, Nout, Kc);
     // (a lead the estimates can carry: over random shapes a smaller one was a loss as often as a gain, up to 8 per cent for nf4)
-    const double lead = fmt == XQ_FMT_NF4 ? 0.92 : decode_first(fmt, rows, Nout, Kc) || dense_tile_size(rows, Nout) == 256 ? 0.94 : 1.0;
+    const double lead = fmt == XQ_FMT_NF4 ? 0.94 : !decode_first(fmt, rows, Nout, Kc) && dense_tile_size(rows, Nout) == 256 ? 0.94 : 0.98;
     return plan->us < lead * tile_kernels_us(fmt, rows, Nout, Kc);
 }
 static int64_t mid_partial_bytes(int fmt, bool cc, int64_t rows, int64_t Nout, int64_t Kc) {
@@ -337,16 +362,28 @@ bool two_dense_supported(const xq_weight* w) {
     return w->format == XQ_FMT_FP8 && g_tile_policy != 1 && w->num_experts == 1 && w->rows % 128 == 0 && w->rows >= 512;
 }
 
-// The launches of a dense weight decoded once: `f` is filled for the whole problem (f.W2: a second matrix that continues the
-// contraction), weights FLAT; `scratch` holds decoded_scratch_bytes().
-static int launch_decoded(G256Args f, bool cc, int fmt, uint8_t* scratch, hipStream_t stream, const char* who) {
+template <int TM, int TN>
+static int launch_dec_tile(G256Args& f, hipStream_t s, const char* who) {
+    using G = GeoDecTile<TM, TN>;
     static std::atomic<bool> attr_set{false};
     if (!attr_set) {
-        int rc = raise_lds_limit(gemm_dec_kernel<false>, GeoDec::lds_bytes(), who);
-        if (!rc) rc = raise_lds_limit(gemm_dec_kernel<true>, GeoDec::lds_bytes(), who);
+        int rc = raise_lds_limit(gemm_dec_kernel<false, TM, TN>, G::lds_bytes(), who);
+        if (!rc) rc = raise_lds_limit(gemm_dec_kernel<true, TM, TN>, G::lds_bytes(), who);
         if (rc) return rc;
         attr_set = true;
     }
+    f.tiles_m = (int32_t)xq_cdiv(f.M, G::ROWS);
+    f.tiles_n = (int32_t)xq_cdiv(f.Nout, G::COLS);
+    const dim3 grid((unsigned)(f.tiles_m * f.tiles_n), (unsigned)f.ksplit);
+    if (f.ksplit > 1) gemm_dec_kernel<true, TM, TN><<<grid, GeoDec::NT, G::lds_bytes(), s>>>(f);
+    else gemm_dec_kernel<false, TM, TN><<<grid, GeoDec::NT, G::lds_bytes(), s>>>(f);
+    XQ_CHECK_LAUNCH(who);
+    return XQ_OK;
+}
+
+// The launches of a dense weight decoded once: `f` is filled for the whole problem (f.W2: a second matrix that continues the
+// contraction), weights FLAT; `scratch` holds decoded_scratch_bytes().
+static int launch_decoded(G256Args f, bool cc, int fmt, uint8_t* scratch, hipStream_t stream, const char* who) {
     const DecPlan plan = plan_decoded(f.M, f.Nout, f.Kc);
     bf16_t* image = (bf16_t*)scratch;
     f.partial = (float*)(scratch + dec_image_bytes(f.Nout, f.Kc));
@@ -368,28 +405,30 @@ static int launch_decoded(G256Args f, bool cc, int fmt, uint8_t* scratch, hipStr
         XQ_CHECK_LAUNCH(who);
     }
     f.W = (const uint8_t*)image;
-    f.tiles_n = (int32_t)tiles_n;
     const bf16_t *A = f.A, *su = f.su;
     bf16_t* C = f.C;
-    const int64_t rows = f.M;
-    for (int64_t r0 = 0; r0 < rows; r0 += plan.head_rows) {
-        const bool head = r0 == 0;
-        f.M = head ? plan.head_rows : rows - r0;
+    int64_t r0 = 0;
+    for (const DecPart& part : plan.part) {
+        if (part.rows == 0) continue;
+        f.M = part.rows;
         f.A = A + r0 * f.lda;
         f.su = su ? su + r0 * f.ld_su : nullptr;
         f.C = C + r0 * f.ldc;
-        f.tiles_m = (int32_t)xq_cdiv(f.M, GeoDec::T);
-        f.ksplit = head ? plan.split : plan.tail_split;
-        const dim3 grid((unsigned)(f.tiles_m * f.tiles_n), (unsigned)f.ksplit);
-        if (f.ksplit > 1) {
-            gemm_dec_kernel<true><<<grid, GeoDec::NT, GeoDec::lds_bytes(), stream>>>(f);
-            XQ_CHECK_LAUNCH(who);
-            splitk_reduce_kernel<<<(unsigned)xq_cdiv(f.M * (f.Nout >> 2), 256), 256, 0, stream>>>(f.partial, f.ksplit, f.M, f.Nout, f.C, f.ldc);
-        } else {
-            gemm_dec_kernel<false><<<grid, GeoDec::NT, GeoDec::lds_bytes(), stream>>>(f);
+        f.ksplit = part.split;
+        r0 += part.rows;
+        int rc;
+        switch (part.tile) {
+            case 0: rc = launch_dec_tile<8, 4>(f, stream, who); break;
+            case 1: rc = launch_dec_tile<7, 4>(f, stream, who); break;
+            case 2: rc = launch_dec_tile<9, 4>(f, stream, who); break;
+            case 3: rc = launch_dec_tile<10, 4>(f, stream, who); break;
+            default: rc = launch_dec_tile<8, 5>(f, stream, who);
         }
-        XQ_CHECK_LAUNCH(who);
-        if (!head) break;
+        if (rc) return rc;
+        if (f.ksplit > 1) {
+            splitk_reduce_kernel<<<(unsigned)xq_cdiv(f.M * (f.Nout >> 2), 256), 256, 0, stream>>>(f.partial, f.ksplit, f.M, f.Nout, f.C, f.ldc);
+            XQ_CHECK_LAUNCH(who);
+        }
     }
     if (timed) xq_profile_mark_end(stream);
     return XQ_OK;

@@ -13,12 +13,13 @@
 //    n lies at chunk c ^ ((n >> 2) & 2), as the kernel wants it in LDS (the stage layout of gemm_dtl16_kernel's weight bytes:
 //    its 16-byte reads meet no bank conflict), so a direct-to-LDS load is a copy of 1 KB in a row.  Forward and dgrad
 //    write the same form (the dgrad's pass transposes), and one kernel serves both.  Columns beyond the matrix repeat the last.
-//  * Kernel.  256 x 256 x 32 K-steps, four LDS stages of 32 KB (activations in the same chunk order), eight waves of 128 x 64 on
-//    v_mfma_f32_16x16x32_bf16.  A K-step is eight chunks of four MFMAs; the activation fragment of a chunk is read three
-//    chunks ahead, the weight fragments of the next K-step during this one's first four chunks (two register sets), the
-//    loads of K-step kt + 3 go out one per chunk.  In iteration kt every wave reads stages kt and kt + 1 and writes
-//    stage kt + 3: the loads of kt + 2 are waited for at its end (those of kt + 3 stay in flight), so a load has two
-//    iterations to land and no read waits behind the barrier.
+//  * Kernel.  Tiles of 32 TM x 64 TN, K-steps of 32: 256 x 256 (TM 8, TN 4), 224, 288 or 320 rows, or 320 columns, by what fills the
+//    chip's rounds best (plan_decoded, xq_gemm.hip).  Four LDS stages (activations in the same chunk order), eight waves of 16 TM x 16 TN
+//    on v_mfma_f32_16x16x32_bf16.  A K-step is TM chunks of TN MFMAs; the activation fragment of a chunk is read three chunks ahead,
+//    the weight fragments of the next K-step during this one's first chunks (two register sets), the loads of K-step kt + 3 go
+//    out one per chunk.  In iteration kt every wave reads stages kt and kt + 1 and writes stage kt + 3: the loads of kt + 2 are
+//    waited for at its end (those of kt + 3 stay in flight), so a load has two iterations to land and no read waits behind the
+//    barrier.
 //  * Splits.  gridDim.y blocks divide the K-steps of a tile (pairs of them: every part is even) where tiles alone leave a
 //    round of the chip part empty; each part writes its fp32 sums, splitk_reduce_kernel adds them.
 #pragma once
@@ -28,11 +29,18 @@
 namespace xq {
 
 struct GeoDec {
-    static constexpr int T = 256, NT = 512, BK = 32, STAGES = 4;
-    static constexpr int TILE_BYTES = T * BK * 2;                  // one operand's share of a stage: 16 KB
-    static constexpr int STAGE_BYTES = 2 * TILE_BYTES;
-    static constexpr size_t lds_bytes() { return (size_t)STAGES * STAGE_BYTES; }
+    static constexpr int T = 256, NT = 512, BK = 32, STAGES = 4;   // T: columns of an image tile
+    static constexpr int TILE_BYTES = T * BK * 2;                  // a K-step of it: 16 KB
     static constexpr int MIN_STEPS = 4;                            // K-steps of a part (an even number)
+};
+
+// A block's tile: 32 TM rows x 64 TN columns
+template <int TM, int TN>
+struct GeoDecTile {
+    static constexpr int ROWS = 32 * TM, COLS = 64 * TN;
+    static constexpr int A_BYTES = ROWS * GeoDec::BK * 2, STAGE_BYTES = A_BYTES + COLS * GeoDec::BK * 2;
+    static constexpr int AP = (ROWS / 8 + 15) / 16, WP = (COLS / 8 + 15) / 16;     // direct loads of a wave and K-step
+    static constexpr size_t lds_bytes() { return (size_t)GeoDec::STAGES * STAGE_BYTES; }
 };
 
 inline int64_t dec_image_bytes(int64_t Nout, int64_t Kc) { return xq_cdiv(Nout, GeoDec::T) * GeoDec::T * Kc * 2; }
@@ -144,10 +152,13 @@ __global__ void __launch_bounds__(256) dec_image_t_kernel(DecImageArgs g) {
 }
 
 // G256Args::W is the image; ksplit and partial as there (SPLIT: fp32 sums to partial, part 0 with side term and bias)
-template <bool SPLIT>
+template <bool SPLIT, int TM, int TN>
 __global__ void __launch_bounds__(512, 2) gemm_dec_kernel(G256Args g) {
     using D = GeoDec;
-    constexpr int T = 256, TM = 8, TN = 4, NC = TM;
+    using G = GeoDecTile<TM, TN>;
+    constexpr int NC = TM, NP = G::AP + G::WP, RW = TM * 16, CW = TN * 16;
+    constexpr int RING = NC % 4 == 0 ? 4 : NC % 5 == 0 ? 5 : NC;       // activation fragments held: a divisor of the chunks, above 3
+    static_assert(TN <= NC - 2 && NP <= NC, "the waits below");
     extern __shared__ __attribute__((aligned(16))) unsigned char dsm[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave >> 2, wn = wave & 3;
@@ -166,8 +177,8 @@ __global__ void __launch_bounds__(512, 2) gemm_dec_kernel(G256Args g) {
         pid_m = first_m + in % gsz;
         pid_n = in / gsz;
     }
-    const int64_t row0 = (int64_t)pid_m * T, row_end = g.M;
-    const int n0 = pid_n * T;
+    const int64_t row0 = (int64_t)pid_m * G::ROWS, row_end = g.M;
+    const int n0 = pid_n * G::COLS;
     const int nk_all = g.Kc / D::BK;
     int kt0 = 0, nk = nk_all;                           // this part's K-steps: an even number, MIN_STEPS or more
     if constexpr (SPLIT) {
@@ -175,32 +186,37 @@ __global__ void __launch_bounds__(512, 2) gemm_dec_kernel(G256Args g) {
         kt0 = 2 * (int)((int64_t)pairs * s / g.ksplit);
         nk = 2 * (int)((int64_t)pairs * (s + 1) / g.ksplit) - kt0;
     }
-    const int mt = __builtin_amdgcn_readfirstlane((int)max((int64_t)0, min((int64_t)TM, (row_end - row0 - wm * 128 + 15) >> 4)));
+    const int mt = __builtin_amdgcn_readfirstlane((int)max((int64_t)0, min((int64_t)TM, (row_end - row0 - wm * RW + 15) >> 4)));
 
-    // ---- direct-to-LDS sources: a wave brings in 32 activation rows (two loads of 16 rows x 64 bytes) and the same share of
-    // the image (2 KB in a row)
-    uint32_t a_off[2];
+    // ---- direct-to-LDS sources: a wave brings in an eighth of the activation rows and of the image columns, 64 bytes of each, 16
+    // to a load (the last load of either: what is left)
+    uint32_t a_off[G::AP], w_off[G::WP];
 #pragma unroll
-    for (int p = 0; p < 2; ++p) {
-        const int rt = (wave * 2 + p) * 16 + (lane >> 2);
+    for (int p = 0; p < G::AP; ++p) {
+        const int rt = wave * (G::ROWS / 8) + p * 16 + (lane >> 2);
         const int64_t r = min(row0 + rt, row_end - 1);
         a_off[p] = (uint32_t)((r * g.lda + (((lane & 3) ^ ((rt >> 2) & 2)) << 3)) * 2);
     }
-    const uint32_t w_off = lane * 16;
+    const int t0 = n0 >> 8;
+#pragma unroll
+    for (int p = 0; p < G::WP; ++p) {
+        // (a tile that does not begin with an image tile lies across two; columns beyond the image: its last)
+        const int n = min(n0 + wave * (G::COLS / 8) + p * 16 + (lane >> 2), (int)((g.Nout + 255) & ~255) - 1);
+        w_off[p] = (uint32_t)((n >> 8) - t0) * (uint32_t)(nk_all * D::TILE_BYTES) + (uint32_t)(n & 255) * 64 + (lane & 3) * 16;
+    }
     const unsigned char* const a_base = (const unsigned char*)(g.A + (int64_t)kt0 * D::BK);
-    const unsigned char* const w_base = g.W + ((int64_t)pid_n * nk_all + kt0) * D::TILE_BYTES + wave * 2048;
+    const unsigned char* const w_base = g.W + ((int64_t)t0 * nk_all + kt0) * D::TILE_BYTES;
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)dsm;
     // (M0 as in gemm_dtl16_kernel: the LDS base of the load, written here and used nowhere else)
     auto issue_part = [&](int kt, int part) {
-        const uint32_t dst = lds0 + (uint32_t)(kt & 3) * D::STAGE_BYTES + wave * 2048 + (part & 1) * 1024;
-        if (part < 2) {
-            const unsigned char* base = a_base + (int64_t)kt * (D::BK * 2);
-            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" :: "s"(dst), "v"(a_off[part]), "s"(base) : "memory");
-        } else {
-            const unsigned char* base = w_base + (int64_t)kt * D::TILE_BYTES + (part & 1) * 1024;
-            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-                         :: "s"(dst + D::TILE_BYTES), "v"(w_off), "s"(base) : "memory");
-        }
+        const uint32_t stage = lds0 + (uint32_t)(kt & 3) * G::STAGE_BYTES;
+        const bool of_a = part < G::AP;
+        const int p = of_a ? part : part - G::AP, rows = (of_a ? G::ROWS : G::COLS) / 8;
+        const uint32_t dst = stage + (of_a ? 0 : G::A_BYTES) + wave * rows * 64 + p * 1024;
+        const unsigned char* base = of_a ? a_base + (int64_t)kt * (D::BK * 2) : w_base + (int64_t)kt * D::TILE_BYTES;
+        const uint32_t off = of_a ? a_off[p] : w_off[p];
+        if (p * 16 + 16 <= rows || lane < (rows - p * 16) * 4)
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" :: "s"(dst), "v"(off), "s"(base) : "memory");
     };
 
     f32x4 acc[TM][TN];
@@ -211,35 +227,38 @@ __global__ void __launch_bounds__(512, 2) gemm_dec_kernel(G256Args g) {
 
     // ---- fragment reads, with the waits counted by hand (as in gemm_dtl16_kernel; no other LDS access inside the loop)
     const int sw = (l16 >> 2) & 2;
-    const uint32_t a_addr = lds0 + (wm * 128 + l16) * 64 + ((lg ^ sw) << 4);
-    const uint32_t w_addr = lds0 + D::TILE_BYTES + (wn * 64 + l16) * 64 + ((lg ^ sw) << 4);
+    const uint32_t a_addr = lds0 + (wm * RW + l16) * 64 + ((lg ^ sw) << 4);
+    const uint32_t w_addr = lds0 + G::A_BYTES + (wn * CW + l16) * 64 + ((lg ^ sw) << 4);
 #define XQ_DEC_READ(dst, addr, so, t) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(dst) : "v"((addr) + (so)), "n"((t) * 1024))
 
     // ---- prologue: K-steps 0, 1 and 2 requested, 0 and 1 waited for
 #pragma unroll
     for (int kt = 0; kt < 3; ++kt)
 #pragma unroll
-        for (int part = 0; part < 4; ++part) issue_part(kt, part);
-    asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+        for (int part = 0; part < NP; ++part) issue_part(kt, part);
+    asm volatile("s_waitcnt vmcnt(%0)" :: "n"(NP) : "memory");
     __builtin_amdgcn_s_barrier();
 
-    bf16x8 fa[4];                 // ring: chunk c uses fa[c & 3]
+    bf16x8 fa[RING];              // chunk c uses fa[c % RING]
     bf16x8 fb[2][TN];             // weight fragments of even and odd K-steps
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    XQ_DEC_READ(fb[0][0], w_addr, 0u, 0); XQ_DEC_READ(fb[0][1], w_addr, 0u, 1); XQ_DEC_READ(fb[0][2], w_addr, 0u, 2); XQ_DEC_READ(fb[0][3], w_addr, 0u, 3);
+#pragma unroll
+    for (int j = 0; j < TN; ++j) XQ_DEC_READ(fb[0][j], w_addr, 0u, j);
     XQ_DEC_READ(fa[0], a_addr, 0u, 0); XQ_DEC_READ(fa[1], a_addr, 0u, 1); XQ_DEC_READ(fa[2], a_addr, 0u, 2);
-    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(fb[0][0]), "+v"(fb[0][1]), "+v"(fb[0][2]), "+v"(fb[0][3]), "+v"(fa[0]), "+v"(fa[1]), "+v"(fa[2]));
+    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(fa[0]), "+v"(fa[1]), "+v"(fa[2]));
+#pragma unroll
+    for (int j = 0; j < TN; ++j) asm volatile("" : "+v"(fb[0][j]));
 
     // LDS reads that chunk c of an iteration issues (c < 0: of the iteration before, which had a next one)
     auto reads_in_chunk = [](int c, bool more) constexpr -> int {
-        if (c < 0) return 1;                                            // chunks 6 and 7: one activation read each
+        if (c < 0) return 1;                                            // its last two: one activation read each
         return (c + 3 < NC || more ? 1 : 0) + (more && c < TN ? 1 : 0);
     };
     auto iteration = [&](int kt, auto P_, auto LEFT_, auto SKIP_) {
         // LEFT: K-steps behind this one, 3 for "three or more"
         constexpr int P = decltype(P_)::value, LEFT = decltype(LEFT_)::value;
         constexpr bool MORE = LEFT >= 1, SKIP = decltype(SKIP_)::value;
-        const uint32_t so = (uint32_t)(kt & 3) * D::STAGE_BYTES, son = (uint32_t)((kt + 1) & 3) * D::STAGE_BYTES;
+        const uint32_t so = (uint32_t)(kt & 3) * G::STAGE_BYTES, son = (uint32_t)((kt + 1) & 3) * G::STAGE_BYTES;
 #pragma unroll
         for (int c = 0; c < NC; ++c) {
             // the chunk's activation fragment (and, older, the K-step's weight fragments) have landed when only the reads of
@@ -247,25 +266,27 @@ __global__ void __launch_bounds__(512, 2) gemm_dec_kernel(G256Args g) {
             {
                 const int n = reads_in_chunk(c - 1, MORE) + reads_in_chunk(c - 2, MORE);
                 if (c == 0) {
-                    asm volatile("s_waitcnt lgkmcnt(2)" : "+v"(fa[0]), "+v"(fb[P][0]), "+v"(fb[P][1]), "+v"(fb[P][2]), "+v"(fb[P][3]));
-                } else if (n == 1) asm volatile("s_waitcnt lgkmcnt(1)" : "+v"(fa[c & 3]));
-                else if (n == 2) asm volatile("s_waitcnt lgkmcnt(2)" : "+v"(fa[c & 3]));
-                else if (n == 3) asm volatile("s_waitcnt lgkmcnt(3)" : "+v"(fa[c & 3]));
-                else if (n == 4) asm volatile("s_waitcnt lgkmcnt(4)" : "+v"(fa[c & 3]));
-                else asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(fa[c & 3]));
+                    asm volatile("s_waitcnt lgkmcnt(2)" : "+v"(fa[0]));
+#pragma unroll
+                    for (int j = 0; j < TN; ++j) asm volatile("" : "+v"(fb[P][j]));
+                } else if (n == 1) asm volatile("s_waitcnt lgkmcnt(1)" : "+v"(fa[c % RING]));
+                else if (n == 2) asm volatile("s_waitcnt lgkmcnt(2)" : "+v"(fa[c % RING]));
+                else if (n == 3) asm volatile("s_waitcnt lgkmcnt(3)" : "+v"(fa[c % RING]));
+                else if (n == 4) asm volatile("s_waitcnt lgkmcnt(4)" : "+v"(fa[c % RING]));
+                else asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(fa[c % RING]));
             }
             if (!SKIP || c < mt)
 #pragma unroll
-            for (int j = 0; j < TN; ++j) acc[c][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[P][j], fa[c & 3], acc[c][j], 0, 0, 0);
-            if (c + 3 < NC) XQ_DEC_READ(fa[(c + 3) & 3], a_addr, so, c + 3);
-            else if (MORE) XQ_DEC_READ(fa[(c + 3) & 3], a_addr, son, c + 3 - NC);
+            for (int j = 0; j < TN; ++j) acc[c][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[P][j], fa[c % RING], acc[c][j], 0, 0, 0);
+            if (c + 3 < NC) XQ_DEC_READ(fa[(c + 3) % RING], a_addr, so, c + 3);
+            else if (MORE) XQ_DEC_READ(fa[(c + 3) % RING], a_addr, son, c + 3 - NC);
             if (MORE && c < TN) XQ_DEC_READ(fb[P ^ 1][c], w_addr, son, c);
-            if (LEFT >= 3 && c < 4) issue_part(kt + 3, c);
+            if (LEFT >= 3 && c < NP) issue_part(kt + 3, c);
             __builtin_amdgcn_sched_barrier(0);
         }
         if (MORE) {
             // the loads of K-step kt + 2 have landed
-            if (LEFT >= 3) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+            if (LEFT >= 3) asm volatile("s_waitcnt vmcnt(%0)" :: "n"(NP) : "memory");
             else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             __builtin_amdgcn_s_barrier();
             __builtin_amdgcn_sched_barrier(0);
@@ -296,11 +317,11 @@ __global__ void __launch_bounds__(512, 2) gemm_dec_kernel(G256Args g) {
         const int s = blockIdx.y;
         G256Args f = g;
         if (s > 0) { f.r_pad = 0; f.bias = nullptr; }
-        dtl16_side_term<TM, TN, 8, false>(f, dsm, 2 * D::TILE_BYTES, acc, row0, row_end, n0, g.Nout, f.su, nullptr, 0);
+        dtl16_side_term<TM, TN, 8, false>(f, dsm, G::ROWS * 128, acc, row0, row_end, n0, g.Nout, f.su, nullptr, 0);
         float* part = g.partial + (int64_t)s * g.M * g.Nout;
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
-            const int n = n0 + wn * 64 + j * 16 + 4 * lg;
+            const int n = n0 + wn * CW + j * 16 + 4 * lg;
             f32x4 b4 = {0.0f, 0.0f, 0.0f, 0.0f};
             if (f.bias) {
                 const u32x2 b = *(const u32x2*)(f.bias + min(n, g.Nout - 4));
@@ -308,12 +329,12 @@ __global__ void __launch_bounds__(512, 2) gemm_dec_kernel(G256Args g) {
             }
 #pragma unroll
             for (int i = 0; i < TM; ++i) {
-                const int64_t row = row0 + wm * 128 + i * 16 + l16;
+                const int64_t row = row0 + wm * RW + i * 16 + l16;
                 if (row < row_end && n < g.Nout) *(f32x4*)(part + row * g.Nout + n) = acc[i][j] + b4;
             }
         }
     } else {
-        dtl16_finish<TM, TN, 8, false>(g, dsm, 2 * D::TILE_BYTES, acc, row0, row_end, n0, n0, g.Nout, g.su, nullptr, 0);
+        dtl16_finish<TM, TN, 8, false>(g, dsm, G::ROWS * 128, acc, row0, row_end, n0, n0, g.Nout, g.su, nullptr, 0);
     }
 }
 

@@ -64,13 +64,13 @@ __device__ __forceinline__ u32x2 dtl_decode4(uint32_t w, float sc) {
     return u32x2{pack_bf16x2(x0[0] * sc, x0[1] * sc), pack_bf16x2(x1[0] * sc, x1[1] * sc)};
 }
 
-// The end of a 256 x 256 tile of the kernels whose waves hold TM x TN tiles of 16 x 16 sums (gemm_dtl16_kernel,
-// gemm_dec_kernel).  `dsm` is the block's LDS, read by nobody else behind the barrier here; `second` bytes into it lies room
-// for a second 32 KB tile.  First the low-rank side term:
+// The end of a tile of the kernels whose waves, two or one down and four across, hold TM x TN tiles of 16 x 16 sums
+// (gemm_dtl16_kernel, gemm_dec_kernel).  `dsm` is the block's LDS, read by nobody else behind the barrier here, with room for 128
+// bytes of every row; `second` bytes into it lies room for as much of every column.  First the low-rank side term:
 template <int TM, int TN, int NW, bool GROUPED>
 __device__ __forceinline__ void dtl16_side_term(const G256Args& g, unsigned char* dsm, int second, f32x4 (&acc)[TM][TN], int64_t row0,
                                                 int64_t row_end, int n0w, int bank_width, const bf16_t* su_b, const bf16_t* lr_b, int e) {
-    constexpr int T = 256, NT = NW * 64, RW = TM * 16;
+    constexpr int NT = NW * 64, RW = TM * 16, CW = TN * 16, TA = RW * (NW / 4), TB = CW * 4;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = NW == 8 ? wave >> 2 : 0, wn = wave & 3;
     const int l16 = lane & 15, lg = lane >> 4;
@@ -82,14 +82,15 @@ __device__ __forceinline__ void dtl16_side_term(const G256Args& g, unsigned char
     if (g.r_pad > 0) {
         const int rp = g.r_pad, steps = (rp + 31) >> 5, cpr = steps << 2, have = rp >> 3;
         const bf16_t* lr = lr_b + (int64_t)e * bank_width * rp;
-        for (int idx = tid; idx < T * cpr; idx += NT) {
+        for (int idx = tid; idx < (TA > TB ? TA : TB) * cpr; idx += NT) {
             const int r = idx / cpr, c = idx - r * cpr;
             int64_t row = row0 + r;
             row = row < row_end ? row : row_end - 1;
             int n = n0w + r;
             n = n < bank_width ? n : bank_width - 1;
             const u32x4 z = {0, 0, 0, 0};
-            *(u32x4*)(As + swz(r, c)) = c < have ? *(const u32x4*)(su_b + row * g.ld_su + c * 8) : z;
+            if (TA >= TB || r < TA) *(u32x4*)(As + swz(r, c)) = c < have ? *(const u32x4*)(su_b + row * g.ld_su + c * 8) : z;
+            if (TB < TA && r >= TB) continue;
             if constexpr (GROUPED) *(u32x4*)(Bs + swz(r, c)) = c < have ? *(const u32x4*)(lr + (int64_t)n * rp + c * 8) : z;
             else *(u32x4*)(Bs + swz(r, c)) = c < have ? right_chunk(g.right, -1, n, c) : z;
         }
@@ -97,7 +98,7 @@ __device__ __forceinline__ void dtl16_side_term(const G256Args& g, unsigned char
         for (int ks = 0; ks < steps; ++ks) {
             bf16x8 bw[TN];
 #pragma unroll
-            for (int j = 0; j < TN; ++j) bw[j] = *(const bf16x8*)(Bs + swz(wn * 64 + j * 16 + l16, ks * 4 + lg));
+            for (int j = 0; j < TN; ++j) bw[j] = *(const bf16x8*)(Bs + swz(wn * CW + j * 16 + l16, ks * 4 + lg));
 #pragma unroll
             for (int i = 0; i < TM; ++i) {
                 const bf16x8 ax = *(const bf16x8*)(As + swz(wm * RW + i * 16 + l16, ks * 4 + lg));
@@ -116,48 +117,56 @@ __device__ __forceinline__ void dtl16_side_term(const G256Args& g, unsigned char
 template <int TM, int TN, int NW, bool GROUPED>
 __device__ __forceinline__ void dtl16_finish(const G256Args& g, unsigned char* dsm, int second, f32x4 (&acc)[TM][TN], int64_t row0,
                                              int64_t row_end, int n0, int n0w, int bank_width, const bf16_t* su_b, const bf16_t* lr_b, int e) {
-    constexpr int RW = TM * 16;
+    constexpr int RW = TM * 16, CW = TN * 16;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = NW == 8 ? wave >> 2 : 0, wn = wave & 3;
     dtl16_side_term<TM, TN, NW, GROUPED>(g, dsm, second, acc, row0, row_end, n0w, bank_width, su_b, lr_b, e);
 
     // ---- the finished tile.  Lane l holds, per (i, j) tile, row 16 i + l % 16 and the 4 columns 16 j + 4 (l / 16) ..: 8 bytes
-    // of bf16.  Each wave passes its RW x 64 sub-tile through a private LDS area ([row][64] bf16, chunk swizzle) and writes
-    // whole 128-byte row pieces, 8 rows per instruction.
+    // of bf16.  Each wave passes its RW x CW sub-tile through a private LDS area and writes whole row pieces of 16 CW bytes / 8:
+    // at once in 128-byte rows with the chunk swizzle, or, where that is more than the LDS there is, in two groups of row tiles.
     if constexpr (NW == 4) asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");     // the last MFMA results, written outside the compiler's hazard tracking
-    bf16_t* stg = (bf16_t*)dsm + wave * (RW * 64);
+    constexpr int TG = TM * TN <= 32 || NW == 4 ? TM : (TM + 1) / 2;      // row tiles of a group
+    constexpr int CH = CW / 8;                                            // 16-byte chunks of a row
+    bf16_t* stg = (bf16_t*)dsm + wave * (TG * 16 * CW);
+    auto at = [&](int r, int c) { return TN == 4 ? swz(r, c) : r * CW + c * 8; };
     int lv = lane;
     asm volatile("" : "+v"(lv));
     const int s16 = lv & 15, sg = lv >> 4;
     const bool wide = g.wide_rows != 0;
 #pragma unroll
-    for (int j = 0; j < TN; ++j) {
-        float b4[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-        if (g.bias) {
-            const u32x2 b = *(const u32x2*)(g.bias + min(n0 + wn * 64 + j * 16 + 4 * sg, g.Nout - 4));
-            b4[0] = __uint_as_float(b[0] << 16); b4[1] = __uint_as_float(b[0] & 0xffff0000u);
-            b4[2] = __uint_as_float(b[1] << 16); b4[3] = __uint_as_float(b[1] & 0xffff0000u);
-        }
+    for (int grp = 0; grp < (TM + TG - 1) / TG; ++grp) {
 #pragma unroll
-        for (int i = 0; i < TM; ++i) {
-            const u32x2 v = {pack_bf16x2(acc[i][j][0] + b4[0], acc[i][j][1] + b4[1]), pack_bf16x2(acc[i][j][2] + b4[2], acc[i][j][3] + b4[3])};
-            if (wide) {
-                *(u32x2*)(stg + swz(i * 16 + s16, 2 * j + (sg >> 1)) + 4 * (sg & 1)) = v;
-            } else {
-                const int64_t row = row0 + wm * RW + i * 16 + s16;
-                const int n = n0 + wn * 64 + j * 16 + 4 * sg;
-                if (row < row_end && n < g.Nout) *(u32x2*)(g.C + row * g.ldc + n) = v;
+        for (int j = 0; j < TN; ++j) {
+            float b4[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+            if (g.bias) {
+                const u32x2 b = *(const u32x2*)(g.bias + min(n0 + wn * CW + j * 16 + 4 * sg, g.Nout - 4));
+                b4[0] = __uint_as_float(b[0] << 16); b4[1] = __uint_as_float(b[0] & 0xffff0000u);
+                b4[2] = __uint_as_float(b[1] << 16); b4[3] = __uint_as_float(b[1] & 0xffff0000u);
+            }
+#pragma unroll
+            for (int ig = 0; ig < TG; ++ig) {
+                if (grp * TG + ig >= TM) continue;
+                const int i = grp * TG + ig;
+                const u32x2 v = {pack_bf16x2(acc[i][j][0] + b4[0], acc[i][j][1] + b4[1]), pack_bf16x2(acc[i][j][2] + b4[2], acc[i][j][3] + b4[3])};
+                if (wide) {
+                    *(u32x2*)(stg + at(ig * 16 + s16, 2 * j + (sg >> 1)) + 4 * (sg & 1)) = v;
+                } else {
+                    const int64_t row = row0 + wm * RW + i * 16 + s16;
+                    const int n = n0 + wn * CW + j * 16 + 4 * sg;
+                    if (row < row_end && n < g.Nout) *(u32x2*)(g.C + row * g.ldc + n) = v;
+                }
             }
         }
-    }
-    if (wide) {
+        if (wide) {
 #pragma unroll
-        for (int t = 0; t < RW / 8; ++t) {
-            const int rl = t * 8 + (lv >> 3), ch = lv & 7;
-            const u32x4 v = *(const u32x4*)(stg + swz(rl, ch));
-            const int64_t row = row0 + wm * RW + rl;
-            const int n = n0 + wn * 64 + ch * 8;
-            if (row < row_end && n < g.Nout) *(u32x4*)(g.C + row * g.ldc + n) = v;
+            for (int t = 0; t < TG * 16 * CH / 64; ++t) {
+                const int idx = t * 64 + lv, rl = idx / CH, ch = idx - rl * CH;
+                const u32x4 v = *(const u32x4*)(stg + at(rl, ch));
+                const int64_t row = row0 + wm * RW + grp * TG * 16 + rl;
+                const int n = n0 + wn * CW + ch * 8;
+                if ((TM % TG == 0 || grp * TG * 16 + rl < RW) && row < row_end && n < g.Nout) *(u32x4*)(g.C + row * g.ldc + n) = v;
+            }
         }
     }
 }

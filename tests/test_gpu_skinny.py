@@ -219,3 +219,17 @@ def test_skinny_seeded_shape_sweep(hip_device):
                                     bias=None if m.bias is None else m.bias.detach().cpu())
         assert y.shape == (M, N), (case, fmt, N, K, M, r, bf16_factors)
         close(y.cpu(), ex["y"], TOL)
+
+
+@pytest.mark.parametrize("N,K,r,bias", [(5120, 512, 16, True),     # four rows a wave at M = 64, two below; fewer splits than are requested at a time
+                                        (1056, 4352, 8, False),    # nine splits or more, columns that end inside a block
+                                        (640, 1024, 64, True)])    # four quads of ranks a row
+def test_epilogue_rows_per_wave(hip_device, N, K, r, bias):
+    m, w_ref = make_dense_module("int4" if K % 128 == 0 else "nvfp4", N, K, r, 32, seed=N, device=hip_device, bias=bias)
+    for M in (17, 24, 25, 63, 64):                                 # whole and partly filled waves and blocks
+        x = gen((M, K), 1.0, M, torch.bfloat16)
+        with torch.no_grad():
+            y = m(x.to(hip_device))
+        ex = R.linear_fwd_bwd_exact(x, w_ref, m.lora_A.detach().cpu(), m.lora_B.detach().cpu(), m.scaling,
+                                    bias=None if m.bias is None else m.bias.detach().cpu())
+        close(y.cpu(), ex["y"], TOL)                               # (the bound of every cell above)

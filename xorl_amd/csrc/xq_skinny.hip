@@ -371,6 +371,8 @@ struct EpiBatch {
 // columns (a lane 2) of RW rows, the block's waves the rows next to each other.  The kernel is a few dependent memory round
 // trips long: everything the first sums need -- B values of the first 16 ranks, partial tiles, low-rank parts (dealt over all
 // threads, met in LDS) -- is requested before anything is waited for.  Every sum runs in a fixed order.
+// RW: 1 up to 16 rows; 2 with eight splits requested at a time above (4 rows and four splits, which took fewer blocks and twice the
+// trips: int4 MLP [12288, 4096] M = 64 70.7 -> 69.1 us whole, int4 [1024, 4096] 13.9 -> 12.8, nf4 [12288, 4096] M = 24 26.1 -> 24.0).
 // VEC: B is fp32 with r % 4 == 0 (16-byte pieces).  GU: jobs 0 and 1 are gate and up, h is written.
 template <int RW, bool VEC, bool GU>
 __global__ void __launch_bounds__(256)
@@ -423,7 +425,7 @@ stream_epilogue_kernel(int32_t M, int32_t first1, int32_t first2, int32_t first3
                 bt[p][P ^ ((P >> 4) & 7)] = bq[p][i];
             }
     };
-    constexpr int SB = 4;                                          // splits requested at a time
+    constexpr int SB = RW == 2 ? 8 : 4;                            // splits requested at a time
     f32x2 t[NP][SB][RW];
     const auto load_part = [&](int p, int s0) {
         const EpiJob& g = b.job[ji + p];
@@ -738,8 +740,14 @@ int launch_skinny_stream(const SkinnyRowsJob* jobs, int n_jobs, bool swiglu, con
     XQ_STREAM_CASE(XQ_FMT_NF4, kScDealt);
 #undef XQ_STREAM_CASE
     if (rc) return rc;
-    const int rw = M <= 16 ? 1 : 4;
-    const unsigned cols = (unsigned)(swiglu ? efirst[1] : efirst[4]), threads = M < 4 && rw == 1 ? (unsigned)M * 64 : 256;
+    const unsigned cols = (unsigned)(swiglu ? efirst[1] : efirst[4]);
+    // (four rows a wave where that is one block a compute unit and two rows would be a few blocks more than one: [5120, 1536] M = 64
+    // 14.6 us against 15.3, [12288, 4096] M = 17 18.7 against 19.2; from rank 17 on two are faster there too)
+    int ranks = 0;
+    for (int i = 0; i < n_jobs; ++i) ranks = e.job[i].r_pad > ranks ? e.job[i].r_pad : ranks;
+    const int64_t by2 = xq_cdiv((int64_t)cols * xq_cdiv(M, 8), num_cus()), by4 = xq_cdiv((int64_t)cols * xq_cdiv(M, 16), num_cus());
+    const int rw = M <= 16 ? 1 : ranks <= 16 && 17 * by4 < 10 * by2 ? 4 : 2;
+    const unsigned threads = M < 4 && rw == 1 ? (unsigned)M * 64 : 256;
     const dim3 grid(cols, (unsigned)xq_cdiv(M, 4 * rw));
 #define XQ_EPI(RW)                                                                                                                             \
     do {                                                                                                                                       \
@@ -752,6 +760,7 @@ int launch_skinny_stream(const SkinnyRowsJob* jobs, int n_jobs, bool swiglu, con
         }                                                                                                                                      \
     } while (0)
     if (rw == 1) XQ_EPI(1);
+    else if (rw == 2) XQ_EPI(2);
     else XQ_EPI(4);
 #undef XQ_EPI
     return XQ_OK;

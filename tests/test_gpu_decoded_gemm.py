@@ -35,14 +35,15 @@ def test_forward_and_backward(hip_device, fmt, M, N, K, r):
         assert err <= 1e-2, f"{name}: {err}"
 
 
-@pytest.mark.parametrize("M,n,k", [
-    (4881, 3088, 1536),                                     # 288-row tiles, the last with one row, 16 columns past a whole one
-    (5436, 3600, 1024),                                     # 320-row tiles
-    (3845, 5104, 1024),                                     # 320-column tiles across the image's 256, the last one not full
-    (5140, 4112, 1536),                                     # 224-row tiles behind whole rounds of 256-row ones
-    (2457, 2176, 6912), (7015, 1152, 6272),                 # 256- and 288-row tiles in K splits
+@pytest.mark.parametrize("fmt,M,n,k", [
+    ("nvfp4", 4881, 3088, 1536),                                     # 288-row tiles, the last with one row, 16 columns past a whole one
+    ("nvfp4", 5436, 3600, 1024),                                     # 320-row tiles
+    ("nvfp4", 3845, 5104, 1024),                                     # 320-column tiles across the image's 256, the last one not full
+    ("nvfp4", 5140, 4112, 1536),                                     # 224-row tiles behind whole rounds of 256-row ones
+    ("nvfp4", 2457, 2176, 6912), ("nvfp4", 7015, 1152, 6272),                 # 256- and 288-row tiles in K splits
+    ("block_fp8", 5572, 3200, 3072),                        # below the rows from which it always decodes first
 ])
-def test_tiles_that_fill_their_rounds(hip_device, M, n, k):
+def test_tiles_that_fill_their_rounds(hip_device, fmt, M, n, k):
     """Both directions of a [M, n] product over k, rows and columns that end inside a tile, against fp32 products of the decoded
     weight.  Elementwise bound: the result's rounding (2^-9, doubled for the fp32 sums and the bias) and, in the low-rank term, those
     of the inner factor's elements, of the intermediate and of the outer factor's (2^-9 of the terms each, nothing cancelling)."""
@@ -52,12 +53,12 @@ def test_tiles_that_fill_their_rounds(hip_device, M, n, k):
         bound = 2 ** -8 * want.abs() + m.scaling * 2 ** -9 * ((au + 2 * u.abs()) @ outer.abs()) + 1e-5 * want.abs().max()
         assert bool(((got.float() - want).abs() <= bound).all())
 
-    m, w = make_dense_module("nvfp4", n, k, 16, 32, seed=5, device=hip_device, bias=True)
+    m, w = make_dense_module(fmt, n, k, 16, 32, seed=5, device=hip_device, bias=True)
     x = gen((M, k), 1.0, 6, torch.bfloat16).to(hip_device)
     with torch.no_grad():
         check(m(x), x.float(), w.to(hip_device).float().t(), m.lora_A.t(), m.lora_B.t(), m.bias.to(torch.bfloat16).float())
     n = -(-n // 64) * 64                                        # (what the low-rank products of a module take)
-    m, w = make_dense_module("nvfp4", k, n, 16, 32, seed=5, device=hip_device)
+    m, w = make_dense_module(fmt, k, n, 16, 32, seed=5, device=hip_device)
     dy = gen((M, k), 1.0, 7, torch.bfloat16).to(hip_device)
     x = torch.zeros(M, n, dtype=torch.bfloat16, device=hip_device).requires_grad_(True)
     m(x).backward(dy)

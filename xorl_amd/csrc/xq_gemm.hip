@@ -180,10 +180,14 @@ static DensePlan plan_dense(int64_t n_rows, int64_t Nout, int64_t nk) {
 //   [1024, 4096]              -3 / -9    -4 / -7    10 / -13    6 / -2     4 / 1      3 / 1      5 / 6
 //   [4096, 1024]              -8 / -7    -6 / -9   -11 / 8      0 / 2      1 / 2      2 / 1      5 / 5
 //   [512, 4096]              -16 / -14  -13 / -10   -7 / -14   -1 / -12   -3 / -3    -2 / -5     4 / 3
-// So 4-bit from 640 rows on, block-fp8 from 6144 on (both directions gain but for a narrow dgrad whose tiles fill a round badly,
-// and below it the wide weights gain less than the narrow ones lose), and products too small to fill the chip (2e10: the last
-// line up to 8192 rows) stay with the tile kernels.
+// (256 x 256 tiles on both sides.)  So 4-bit from 640 rows on, block-fp8 from 6144 on (both directions gain but for a narrow dgrad whose
+// tiles fill a round badly, and below it the wide weights gain less than the narrow ones lose); products too small to fill the
+// chip (2e10: the last line up to 8192 rows) stay with the tile kernels.  Below 6144 rows block-fp8 takes the image where its
+// choice of tiles fills the rounds better than 256 x 256 do, by the estimates (us, tile kernel -> image: [4224, 7040], 4147 rows
+// 262 -> 206; [3200, 3072], 5572 rows 129 -> 97, dgrad 126 -> 96; [6272, 2432], 2855 rows 106 -> 84; [3840, 9216], 5146 rows 384 -> 297; of
+// 180 forwards and dgrads of 640 .. 6143 rows 32 took it, 1.08 to 1.32 times as fast, one of them slower, by 4 per cent).
 constexpr int64_t kDecMinRows = 640, kDecMinRowsFp8 = 6144;
+constexpr double kDecLeadFp8 = 0.92;                 // what the image's estimate has to stay under, of gemm_dtl16_kernel's
 constexpr double kDecMinWork = 2.0e10;               // rows x columns x contraction
 // Tiles: 256 x 256 where they fill their rounds of the chip; otherwise the rows or columns of a tile are stretched or cut to what
 // leaves the last round fullest (288 tiles on 256 units are 240 of 288 rows).  Forward / dgrad, us, with 256 x 256 alone -> with all five:
@@ -245,9 +249,28 @@ static DecPlan plan_decoded(int64_t n_rows, int64_t Nout, int64_t Kc) {
         if (d.split > 1) p.partial = std::max(p.partial, d.split * d.rows * Nout * 4);
     return p;
 }
+static double decoded_us(int fmt, int64_t n_rows, int64_t Nout, int64_t Kc) {      // with the pass that writes the image
+    return 3.4 + (fmt == XQ_FMT_NF4 ? 0.5e-6 : 0.43e-6) * (double)Nout * (double)Kc + plan_decoded(n_rows, Nout, Kc).us;
+}
+// gemm_dtl16_kernel's 256 x 256 tiles as plan_dense lays them out
+static double direct_us(int64_t n_rows, int64_t Nout, int64_t Kc) {
+    const int64_t nk = Kc / 64, cus = num_cus();
+    const DensePlan p = plan_dense(n_rows, Nout, nk);
+    auto us = [&](int64_t rows, int T, int s) {
+        if (rows <= 0) return 0.0;
+        const int64_t blocks = xq_cdiv(rows, T) * xq_cdiv(Nout, T) * s;
+        const double sums = s > 1 ? std::max(2.0, 0.165e-6 * (8.0 * s + 2.0) * (double)rows * (double)Nout - 4.6) : 0.0;
+        if (T == 128) return 4.0 + (blocks <= cus ? 0.54 : 0.7 * (double)xq_cdiv(blocks, 2 * cus)) * 1.55 * (double)nk;
+        const int64_t full = blocks / cus, rest = blocks % cus;
+        const double st = (double)xq_cdiv(nk, s);
+        return (double)full * (8.0 + 1.55 * st) + (rest ? 8.0 + (0.9 + 0.65 * (double)rest / (double)cus) * st : 0.0) + sums;
+    };
+    return us(p.head_rows, 256, p.split) + us(n_rows - p.head_rows, p.tail_T, p.tail_split);
+}
 static bool decode_first(int fmt, int64_t n_rows, int64_t Nout, int64_t Kc) {
-    return n_rows >= (fmt == XQ_FMT_FP8 ? kDecMinRowsFp8 : kDecMinRows) && (double)n_rows * (double)Nout * (double)Kc >= kDecMinWork &&
-           Kc % 64 == 0 && Kc >= 128 && Nout % 16 == 0;
+    if (n_rows < kDecMinRows || (double)n_rows * (double)Nout * (double)Kc < kDecMinWork || Kc % 64 != 0 || Kc < 128 || Nout % 16 != 0) return false;
+    if (fmt != XQ_FMT_FP8 || n_rows >= kDecMinRowsFp8) return true;
+    return dense_tile_size(n_rows, Nout) == 256 && decoded_us(fmt, n_rows, Nout, Kc) < kDecLeadFp8 * direct_us(n_rows, Nout, Kc);
 }
 // (fmt < 0: whatever the format; the 4-bit rule covers all)
 static int64_t decoded_scratch_bytes(int fmt, int64_t n_rows, int64_t Nout, int64_t Kc) {
@@ -289,7 +312,7 @@ static MidPlan plan_mid(int fmt, bool cc, int64_t rows, int64_t Nout, int64_t Kc
 }
 // the same product without it: over a decoded image, or on 256- or 128-row tiles
 static double tile_kernels_us(int fmt, int64_t rows, int64_t Nout, int64_t Kc) {
-    if (decode_first(fmt, rows, Nout, Kc)) return 3.4 + (fmt == XQ_FMT_NF4 ? 0.5e-6 : 0.43e-6) * (double)Nout * (double)Kc + plan_decoded(rows, Nout, Kc).us;
+    if (decode_first(fmt, rows, Nout, Kc)) return decoded_us(fmt, rows, Nout, Kc);
     const double nk = (double)(Kc / 64);
     if (dense_tile_size(rows, Nout) == 256) {
         const int64_t tiles = xq_cdiv(rows, 256) * xq_cdiv(Nout, 256), cus = num_cus(), full = tiles / cus;

@@ -210,11 +210,11 @@ struct DecPlan {
     int64_t partial;          // bytes of fp32 sums the splits take
     double us;                // the estimate it was chosen by
 };
-static DecPlan plan_decoded(int64_t n_rows, int64_t Nout, int64_t Kc) {
+static DecPlan make_plan_decoded(int64_t n_rows, int64_t Nout, int64_t Kc, int64_t cus) {
     // microseconds, fitted to 32 products on all five tiles in one to four splits (4.7 per cent rms): a K-step takes longer the more of
     // the chip is at work (the matrix units share its power), by the tile's size; the fp32 sums of splits are written and read at
     // about 6 TB/s
-    const int64_t steps = Kc / GeoDec::BK, cus = num_cus();
+    const int64_t steps = Kc / GeoDec::BK;
     auto cost = [&](int tile, int64_t rows, int s) {
         const DecTile t = kDecTiles[tile];
         const double w = (double)(t.tm * t.tn) / 32.0, st = (double)xq_cdiv(steps, s) * w;
@@ -248,6 +248,26 @@ static DecPlan plan_decoded(int64_t n_rows, int64_t Nout, int64_t Kc) {
     for (const DecPart& d : p.part)
         if (d.split > 1) p.partial = std::max(p.partial, d.split * d.rows * Nout * 4);
     return p;
+}
+// The estimates of a product are asked for several times a call (its workspace, its route, its launches) and take microseconds: a thread
+// keeps the last ones it made.  They depend on nothing but the key.
+struct PlanKey {
+    int64_t rows, Nout, Kc, cus;
+    int32_t kind;
+    bool operator==(const PlanKey& o) const { return rows == o.rows && Nout == o.Nout && Kc == o.Kc && cus == o.cus && kind == o.kind; }
+    unsigned slot() const { return (unsigned)(rows * 0x9e3779b1u + Nout * 0x85ebca6bu + Kc * 0xc2b2ae35u + kind * 0x27d4eb2fu) >> 16 & 63u; }
+};
+template <typename V>
+struct PlanSlot {
+    PlanKey key;              // rows 0: empty
+    V value;
+};
+static DecPlan plan_decoded(int64_t n_rows, int64_t Nout, int64_t Kc) {
+    static thread_local PlanSlot<DecPlan> kept[64];
+    const PlanKey key{n_rows, Nout, Kc, num_cus(), 0};
+    PlanSlot<DecPlan>& e = kept[key.slot()];
+    if (!(e.key == key)) e = PlanSlot<DecPlan>{key, make_plan_decoded(n_rows, Nout, Kc, key.cus)};
+    return e.value;
 }
 static double decoded_us(int fmt, int64_t n_rows, int64_t Nout, int64_t Kc) {      // with the pass that writes the image
     return 3.4 + (fmt == XQ_FMT_NF4 ? 0.5e-6 : 0.43e-6) * (double)Nout * (double)Kc + plan_decoded(n_rows, Nout, Kc).us;
@@ -336,10 +356,19 @@ static bool mid_shape(int fmt, bool cc, int64_t rows, int64_t Nout, int64_t Kc) 
 }
 static bool takes_mid(int fmt, bool cc, int64_t rows, int64_t Nout, int64_t Kc, MidPlan* plan) {
     if (!mid_shape(fmt, cc, rows, Nout, Kc)) return false;
+    struct Answer { MidPlan plan; bool taken; };
+    static thread_local PlanSlot<Answer> kept[64];
+    const PlanKey key{rows, Nout, Kc, num_cus(), fmt * 2 + (cc ? 1 : 0)};
+    PlanSlot<Answer>& e = kept[key.slot()];
+    if (e.key == key) {
+        *plan = e.value.plan;
+        return e.value.taken;
+    }
     *plan = plan_mid(fmt, cc, rows, Nout, Kc);
     // (a lead the estimates can carry: over random shapes a smaller one was a loss as often as a gain, up to 8 per cent for nf4)
     const double lead = fmt == XQ_FMT_NF4 ? 0.94 : !decode_first(fmt, rows, Nout, Kc) && dense_tile_size(rows, Nout) == 256 ? 0.94 : 0.98;
-    return plan->us < lead * tile_kernels_us(fmt, rows, Nout, Kc);
+    e = PlanSlot<Answer>{key, Answer{*plan, plan->us < lead * tile_kernels_us(fmt, rows, Nout, Kc)}};
+    return e.value.taken;
 }
 static int64_t mid_partial_bytes(int fmt, bool cc, int64_t rows, int64_t Nout, int64_t Kc) {
     MidPlan p;

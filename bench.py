@@ -41,15 +41,15 @@ BF16_MFMA_PEAK_TFLOPS = 2500.0   # MI355X dense bf16, published
 # reports traffic null with the reason instead of a stale constant.  A config that has no counter run reports null.
 # --traffic-bytes overrides.
 MEASURED_TRAFFIC = {
-    # gemm_256_kernel<int4, T=128> in 4 K splits + splitk_reduce_kernel: mean of the forward and dgrad launches
-    # (64 MiB of it are the fp32 partial sums written and read back)
-    0: (109.6 * 2 ** 20, "profiles/gemm_128_int4_linear_m512.txt", 0.04315),
+    # gemm_mid_kernel<int4> in 2 K splits + splitk_reduce_kernel: mean of the forward and dgrad launches
+    # (32 MiB of it are the fp32 partial sums written and read back)
+    0: (77.7 * 2 ** 20, "profiles/gemm_mid_int4_linear_m512.txt", 0.03818),
     # gemm_dec_kernel and the dec_image passes before it (dense block-fp8, 256x256 tiles over decoded images): mean over the 5
     # products of a step (gate, up and down forward, d_h, dx as one sum over the gate and up weights)
     1: (1708.6 * 2 ** 20, "profiles/gemm_dec_fp8_mlp_m8192.txt", 0.7336),
-    # gemm_dec_kernel, dec_image passes and reductions over nvfp4 / NF4 weights: mean over the products of a step (8 and 6)
-    2: (501.4 * 2 ** 20, "profiles/gemm_dec_4bit_m4096_m8192.txt", 0.1802),
-    6: (1423.9 * 2 ** 20, "profiles/gemm_dec_4bit_m4096_m8192.txt", 0.6174),
+    # gemm_dec_kernel and dec_image passes (config 2: gemm_mid_kernel too) over nvfp4 / NF4 weights: mean over the products of a step (8 and 6)
+    2: (393.3 * 2 ** 20, "profiles/gemm_dec_4bit_m4096_m8192.txt", 0.1666),
+    6: (1424.2 * 2 ** 20, "profiles/gemm_dec_4bit_m4096_m8192.txt", 0.6019),
     # gemm_dtl16_kernel<.., grouped>: mean over the 4 launches of a step (gate|up forward over two banks, down
     # forward, d_h, dx as one sum over both banks)
     3: (1402.4 * 2 ** 20, "profiles/gemm_dtl16_fp8_grouped_moe_e128.txt", 0.6325),
@@ -58,11 +58,11 @@ MEASURED_TRAFFIC = {
     # written and read back: 23.3 MiB of it are algorithmic)
     4: (34.2 * 2 ** 20, "profiles/skinny_kernels_decode_shapes.txt", 0.01557),
     # merge_fp8_kernel and merge_kernel<fp8>: mean per call (re-quantise 96 MiB, publish 144 MiB algorithmic)
-    5: (134.4 * 2 ** 20, "profiles/merge_kernel_fp8_mlp_weights.txt", 0.04168),
+    5: (132.1 * 2 ** 20, "profiles/merge_kernel_fp8_mlp_weights.txt", 0.03895),
     # gemm_256_kernel<nvfp4 GKN, grouped>: mean over the 6 launches of a step
     7: (893.9 * 2 ** 20, "profiles/gemm_256_nvfp4_gkn_grouped_moe_e128.txt", 0.52825),
     # merge_kernel<nvfp4>: mean per call over amax / re-quantise / publish of the four weights
-    9: (59.0 * 2 ** 20, "profiles/merge_kernel_nvfp4_attn_weights.txt", 0.03500),
+    9: (56.1 * 2 ** 20, "profiles/merge_kernel_nvfp4_attn_weights.txt", 0.02250),
 }
 
 
@@ -183,7 +183,7 @@ def other_config(cfg: int, dev):
             m(x).backward(dy)
         return (step, lin_flops(512, 4096, 4096, 16), False,
                 "configs[0]: int4 (group 128, bf16 absmax/7 scales) QLoRA linear 4096->4096, M=512, r=16, fwd+bwd",
-                "gemm_256_kernel<int4> with 128x128 tiles in 4 K splits + splitk_reduce_kernel (fused dequant-GEMM, forward and dgrad launches)")
+                "gemm_mid_kernel<int4> in 2 K splits + splitk_reduce_kernel (fused dequant-GEMM, forward and dgrad launches)")
     if cfg == 2:
         Mtok, Hd = 4096, 5120
         shapes = {"q": (8192, Hd), "k": (1024, Hd), "v": (1024, Hd), "o": (Hd, 8192)}
@@ -197,7 +197,7 @@ def other_config(cfg: int, dev):
                 m(xs[k]).backward(dys[k])
         return (step, sum(lin_flops(Mtok, K, N, 16) for (N, K) in shapes.values()), False,
                 "configs[2]: nvfp4 QLoRA Qwen3-32B attention projections q/k/v/o, hidden 5120, M=4096, r=16, fwd+bwd",
-                "gemm_dec_kernel with its dec_image passes (nvfp4 decoded once per launch, 256x256x32 tiles; leading rows in whole rounds, trailing rows in K splits + splitk_reduce_kernel): forward and dgrad launches")
+                "gemm_dec_kernel with its dec_image passes (nvfp4 decoded once per launch, 256x256 and 256x320 tiles) and gemm_mid_kernel (k, v forward): forward and dgrad launches")
     if cfg in (3, 7, 8):
         # 7 / 8 are not BASELINE configs: configs[3] with the banks held as nvfp4 / NF4 (4-bit GKN storage)
         from xorl_amd.qlora import BlockFP8QLoRAMoeExperts, NF4QLoRAMoeExperts, NvFP4QLoRAMoeExperts
@@ -277,7 +277,7 @@ def other_config(cfg: int, dev):
         return (step, total, True,
                 "merge pass (not a BASELINE config): decode + LoRA update + re-encode (block_fp8 -> block_fp8) and "
                 "decode + update -> bf16, for gate/up [12288,4096] and down [4096,12288], r=32",
-                "merge_kernel<fp8> (fused decode + low-rank update + re-quantise / publish)")
+                "merge_fp8_kernel and merge_kernel<fp8> (fused decode + low-rank update + re-quantise / publish)")
     if cfg == 9:
         # not a BASELINE config: the nvfp4 merge / re-quantise pass over configs[2]'s four weights (r = 16): tensor amax
         # of the merged weight, re-encode against it, and the bf16 publish

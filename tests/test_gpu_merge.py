@@ -328,3 +328,31 @@ def test_several_tiles_a_block(hip_device, fmt, r, dtype):
     if fmt == "block_fp8":                                       # in place
         merge_requant_fp8(whole, A, B, r, 0.5, packed, scales)
         assert torch.equal(packed, codes) and torch.equal(scales, new_scales)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("N,r", [(1, 1), (1, 7), (3, 63), (130, 1), (129, 9), (128, 15), (257, 20), (140, 33), (384, 41), (131, 47), (300, 63)])
+def test_ranks_of_any_length(hip_device, N, r, dtype):
+    """Rows of B are read in pieces of eight ranks that may reach into the next row, up to the last that lies whole in the matrix: B
+    ends its allocation, begins off a 16-byte boundary, and every second of its rows is infinite."""
+    from xorl_amd import _C
+    from xorl_amd.functional import QuantWeight, merge_dense
+
+    K = 272
+    g = np.random.default_rng(N + r)
+    packed = torch.from_numpy(g.integers(0, 0x7f, (N, K), dtype=np.uint8))
+    scales = torch.rand(-(-N // 128), -(-K // 128)) * 0.01 + 0.001
+    A, B = gen((r, K), 0.3, 1).to(dtype), gen((N, r), 0.3, 2).to(dtype)
+    B[1::2] = float("inf")
+    b = torch.empty(N * r + 1, dtype=dtype, device=hip_device)[1:].view(N, r)
+    b.copy_(B)
+    qw = QuantWeight("block_fp8", _C.XQ_LAYOUT_FLAT, packed.to(hip_device), scales.to(hip_device), torch.float32, N, K, 128)
+    got = merge_dense(qw, A.to(hip_device), b, r, 0.5, torch.float32).cpu()
+    s = scales.repeat_interleave(128, 0)[:N].repeat_interleave(128, 1)[:, :K]
+    base = packed.view(torch.float8_e4m3fn).float() * s
+    even = slice(0, N, 2)
+    want = base[even].double() + 0.5 * (B[even].double() @ A.double())
+    # factors split into 16 significant bits: 2^-16 of each term's magnitude, and fp32 sums
+    tol = 2.0 ** -15 * (base[even].abs().double() + 0.5 * (B[even].abs().double() @ A.abs().double()))
+    assert bool(((got[even].double() - want).abs() <= tol).all())
+    assert not bool(torch.isfinite(got[1::2]).any())

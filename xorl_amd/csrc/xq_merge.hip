@@ -38,7 +38,6 @@ struct MergeArgs {
     const void* A;       // [r, K]
     const void* B;       // [N, r]
     int32_t lora_f32, r, r_pad;
-    int32_t b_pieces;    // B's rows can be read in 16-byte pieces: r % 8 == 0 and the pointer aligned
     float scaling;
     int32_t run;         // merge_tiles
     int32_t mode;        // 0: bf16 out (publish arithmetic), 1: fp32 out, 2: block-fp8 requantise,
@@ -86,6 +85,9 @@ __device__ __forceinline__ void merge_tiles(int run, uint32_t tiles_n, uint32_t 
     }
 }
 
+// 16 bytes from any factor element on (one global_load_dwordx4 like an aligned one)
+typedef u32x4 u32x4_a2 __attribute__((aligned(2)));
+
 // Eight factor elements as they are stored -> their hi and lo bf16 parts, times `by`; ranks from g.r on are zero.  pairs: two bf16 to
 // a word
 __device__ __forceinline__ void merge_split8(const MergeArgs& g, const uint32_t (&raw)[8], bool pairs, float by, int j0, u32x4& hi, u32x4& lo) {
@@ -110,26 +112,51 @@ struct MergeFactors {
     static constexpr int NB = (RP + 31) / 32, ITEMS = 16 * RP;         // B: eight ranks of a row an item
     uint32_t raw[NB > 0 ? NB : 1][8];
 
-    // the tile's rows of B -> registers, as they are stored (clamped to the last row)
+    // a thread's item i.  Where R8 is no power of two (RP 48) its row and piece are formed per tile, behind the empty statement, not kept
+    // through the loop: every kernel of that rank spilled for them, up to 29 registers a lane (absmax at r 40, [12288, 4096]: 45 us,
+    // without 42)
+    static __device__ __forceinline__ int item(int tid, int i) {
+        int b = tid + 512 * i;
+        if constexpr ((R8 & (R8 - 1)) != 0) asm volatile("" : "+v"(b));
+        return b;
+    }
+    // the tile's rows of B -> registers, as they are stored (clamped to the last row).  Eight ranks are one or two 16-byte loads at whatever
+    // address the first of them has; what these read past the end of a row the split zeroes, and only where it would lie past the
+    // matrix are the elements loaded one by one.  The branches on the type go around the loads: one between them, for a value that
+    // either type writes, makes the second wait for the first.  [12288, 4096], us, with 16-byte loads for multiples of 8 only and that
+    // branch -> now: block-fp8 requantise r 63 55.6 -> 42.7, r 64 43.6 -> 42.7; publish r 63 62.0 -> 45.3, r 40 44.0 -> 42.0; nf4 requantise
+    // r 63 76.6 -> 62.5, r 16 48.6 -> 44.4.
     __device__ __forceinline__ void load_b(const MergeArgs& g, int n0, int tid, int wave) {
-        const bool f32 = g.lora_f32 != 0;
+        const int64_t end = (int64_t)g.N * g.r;
 #pragma unroll
         for (int i = 0; i < NB; ++i) {
-            const int b = tid + 512 * i;
+            const int b = item(tid, i);
             if (512 * i + 512 > ITEMS && 512 * i + wave * 64 >= ITEMS) break;
             const int nb = n0 + b / R8, j0 = b % R8 * 8;
-            const int64_t row = (int64_t)(nb < g.N ? nb : g.N - 1) * g.r;
-            if (g.b_pieces) {
-                const int64_t at = row + (j0 < g.r ? j0 : 0);
-                const u32x4 lo = *(const u32x4*)((const uint8_t*)g.B + at * (f32 ? 4 : 2));
-                const u32x4 hi = f32 ? *(const u32x4*)((const float*)g.B + at + 4) : lo;
+            const int64_t at = (int64_t)(nb < g.N ? nb : g.N - 1) * g.r + (j0 < g.r ? j0 : 0);
+            const int last = (int)(end - at < 8 ? end - at : 8) - 1;        // of the eight, the last within the matrix
+            if (g.lora_f32) {
+                const uint32_t* p = (const uint32_t*)g.B + at;
+                if (last == 7) {
+                    const u32x4 lo = *(const u32x4_a2*)p, hi = *(const u32x4_a2*)(p + 4);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) { raw[i][e] = lo[e]; raw[i][4 + e] = hi[e]; }
+                    for (int e = 0; e < 4; ++e) { raw[i][e] = lo[e]; raw[i][4 + e] = hi[e]; }
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) raw[i][e] = p[e < last ? e : last];
+                }
             } else {
+                const uint16_t* p = (const uint16_t*)g.B + at;
+                if (last == 7) {
+                    const u32x4 lo = *(const u32x4_a2*)p;
 #pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const int64_t at = row + (j0 + e < g.r ? j0 + e : g.r - 1);
-                    raw[i][e] = f32 ? ((const uint32_t*)g.B)[at] : (uint32_t)((const uint16_t*)g.B)[at];
+                    for (int e = 0; e < 4; ++e) { raw[i][e] = lo[e]; raw[i][4 + e] = 0u; }
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        raw[i][e] = p[2 * e < last ? 2 * e : last] | (uint32_t)p[2 * e + 1 < last ? 2 * e + 1 : last] << 16;
+                        raw[i][4 + e] = 0u;
+                    }
                 }
             }
         }
@@ -137,10 +164,10 @@ struct MergeFactors {
     __device__ __forceinline__ void store_b(const MergeArgs& g, bf16_t* sh_b, int tid, int wave) const {
 #pragma unroll
         for (int i = 0; i < NB; ++i) {
-            const int b = tid + 512 * i;
+            const int b = item(tid, i);
             if (512 * i + 512 > ITEMS && 512 * i + wave * 64 >= ITEMS) break;
             u32x4 hi, lo;
-            merge_split8(g, raw[i], g.b_pieces != 0, g.scaling, b % R8 * 8, hi, lo);
+            merge_split8(g, raw[i], true, g.scaling, b % R8 * 8, hi, lo);
             bf16_t* to = sh_b + b / R8 * FP + b % R8 * 8;
             *(u32x4*)to = hi;
             *(u32x4*)(to + MG_T * FP) = lo;
@@ -156,11 +183,13 @@ struct MergeFactors {
             const int item = 8 * i + wave, j0 = (item >> 1) * 8, kk = k0 + (item & 1) * 64 + lane;
             const uint32_t off = (uint32_t)(kk < g.K ? kk : g.K - 1);
             if (item < RP / 4) {
+                auto load = [&](auto T_) {
+                    typedef decltype(T_) T;
 #pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const int64_t row = (int64_t)(j0 + e < g.r ? j0 + e : g.r - 1) * g.K;
-                    a[i][e] = f32 ? ((const uint32_t*)g.A + row)[off] : (uint32_t)((const uint16_t*)g.A + row)[off];
-                }
+                    for (int e = 0; e < 8; ++e) a[i][e] = ((const T*)g.A + (int64_t)(j0 + e < g.r ? j0 + e : g.r - 1) * g.K)[off];
+                };
+                if (f32) load(uint32_t{});
+                else load(uint16_t{});
             }
         }
 #pragma unroll
@@ -260,7 +289,7 @@ __global__ void __launch_bounds__(512, 4) merge_kernel(MergeArgs g) {
     constexpr int DN = ROUNDED ? 1 : 2;
     constexpr int D_BYTES = RP == 0 ? 0 : ROUNDED ? MG_T * DP * 2 : 64 * DP * 4;
     asm volatile("" ::"s"(g.packed), "s"(g.scales), "s"(g.global_scale), "s"(g.group), "s"(g.scale_dtype), "s"(g.N), "s"(g.K),
-                 "s"(g.A), "s"(g.B), "s"(g.lora_f32), "s"(g.r), "s"(g.b_pieces), "s"(g.scaling), "s"(g.out), "s"(g.packed_out), "s"(g.scales_out));
+                 "s"(g.A), "s"(g.B), "s"(g.lora_f32), "s"(g.r), "s"(g.scaling), "s"(g.out), "s"(g.packed_out), "s"(g.scales_out));
     // (all arguments in scalar registers after one round trip)
     typedef MergeFactors<RP> F;
     constexpr int F_BYTES = F::BYTES;
@@ -782,7 +811,6 @@ static int launch_merge(const xq_weight* w, const void* A, const void* B, int lo
     g.A = A; g.B = B; g.lora_f32 = lora_dtype == XQ_DT_F32; g.r = r; g.r_pad = r <= 0 ? 0 : ((r + 15) / 16) * 16;
     g.scaling = scaling; g.mode = mode; g.out = out; g.packed_out = (uint8_t*)packed_out; g.scales_out = scales_out;
     g.amax_out = nv.amax_out; g.gamax = nv.gamax; g.codes_out = nv.codes_out; g.bscale_out = nv.bscale_out; g.gscale_out = nv.gscale_out;
-    g.b_pieces = r > 0 && r % 8 == 0 && xq_aligned(B, 16);
     XQ_REQUIRE(r == 0 || (workspace && xq_aligned(workspace, 256) && workspace_bytes >= merge_ws_bytes(w->rows, w->cols, r)),
                "%s: workspace missing, misaligned or smaller than xq_merge_workspace_bytes()", who);
     // Blocks of one strip each where none has more tiles that way than an equal share has: what is read and written at a time is whole

@@ -173,3 +173,26 @@ def test_workspace_holds_an_image_only_where_the_format_uses_one():
                    L.xq_mlp_workspace_bytes(M, K, N, 16, 0), L.xq_mlp_infer_workspace_bytes(M, K, N, 16) - 6 * M * N]
         assert any_fmt == [max(s[i] for s in sizes.values()) for i in range(4)]
         assert L.xq_mlp_workspace_bytes(M, K, N, 16, 1) == max(s[5] for s in sizes.values())
+
+
+def test_build_refuses_scratch_under_hand_counted_reads():
+    """Kernels that read LDS from inline assembly may not spill; the build reads that from the compiler's remarks."""
+    from xorl_amd.csrc import build as b
+
+    guarded = b.asm_read_kernels()
+    assert {"gemm_dec_kernel", "gemm_dtl16_kernel"} <= set(guarded)
+    tag = " [-Rpass-analysis=kernel-resource-usage]"
+
+    def output(name, scratch):
+        lines = ["In file included from a.hip:2:"]
+        for what in (f"Function Name: {name}", "    VGPRs: 256", f"    ScratchSize [bytes/lane]: {scratch}", "    VGPRs Spill: 0"):
+            lines += [f"a.h:9:1: remark: {what}{tag}", "    9 | __global__ void", "      | ^"]
+        return "\n".join(lines)
+
+    dec, other = "_ZN2xq15gemm_dec_kernelILb0ELi8ELi5EEEvNS_8G256ArgsE", "_ZN2xq14lowrank_kernelILi1EEEvi"
+    text = "\n".join([output(other, 128), output(dec, 0), "In file included from a.hip:3:", "b.h:1:1: warning: unused", "    1 | int x;", "      | ^"])
+    remarks, rest = b._split_remarks(text)
+    assert rest.splitlines() == ["In file included from a.hip:3:", "b.h:1:1: warning: unused", "    1 | int x;", "      | ^"]
+    b.check_scratch(remarks, guarded)
+    with pytest.raises(RuntimeError, match="gemm_dec_kernel"):
+        b.check_scratch(b._split_remarks(output(other, 0) + "\n" + output(dec, 80))[0], guarded)

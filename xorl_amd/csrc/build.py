@@ -5,6 +5,7 @@ from __future__ import annotations
 
 import glob
 import os
+import re
 import subprocess
 import sys
 import sysconfig
@@ -24,7 +25,46 @@ FLAGS = [
     # the first 16 dwords of a kernel's scalar arguments arrive in registers with the wave (where the platform does it)
     "-mllvm", "-amdgpu-kernarg-preload-count=16",
     "-Wall", "-Wno-unused-function",
+    "-Rpass-analysis=kernel-resource-usage",
 ]
+
+
+def asm_read_kernels() -> list[str]:
+    """Names of the kernels in files that read LDS into registers from inline assembly with waits of their own.  The compiler takes
+    such a register as written at once: a spill before the wait would store what it held before."""
+    names = []
+    for path in sorted(glob.glob(os.path.join(HERE, "*.h")) + glob.glob(os.path.join(HERE, "*.hip"))):
+        with open(path) as f:
+            text = f.read()
+        if re.search(r'asm volatile\("ds_read', text):
+            names += re.findall(r"__global__ [^;{]*?(\w+)\(\w+ \w+\) *\{", text)
+    return names
+
+
+def check_scratch(remarks: str, guarded: list[str]) -> None:
+    """Raise if one of the guarded kernels uses scratch memory, by the compiler's resource remarks."""
+    for name, usage in re.findall(r"Function Name: (\S+)(.*?)(?=Function Name: |\Z)", remarks, re.S):
+        kernel = next((k for k in guarded if re.search(rf"\d{k}(?![a-z])", name)), None)
+        scratch = re.search(r"ScratchSize \[bytes/lane\]: (\d+)", usage)
+        if kernel and (scratch is None or int(scratch[1])):
+            raise RuntimeError(f"{name}: {scratch[1] if scratch else 'unknown'} bytes of scratch a lane; {kernel} reads LDS from inline "
+                               "assembly and may not spill")
+
+
+def _split_remarks(text: str) -> tuple[str, str]:
+    """(the resource remarks, everything else) of a compiler's output; a remark's place of inclusion and excerpt of the source are dropped"""
+    remarks, rest, included, excerpt = [], [], [], False
+    for line in text.splitlines():
+        if line.startswith("In file included from"):
+            included.append(line)
+        elif "[-Rpass-analysis=kernel-resource-usage]" in line:
+            remarks.append(line)
+            included, excerpt = [], True
+        elif not (excerpt and re.match(r"\s*\d* \| ", line)):
+            if "is not a recognized feature for this target" not in line:
+                rest += [*included, line]
+            included, excerpt = [], False
+    return "\n".join(remarks), "\n".join(rest)
 
 
 def _compile(src: str, force: bool) -> str:
@@ -34,9 +74,14 @@ def _compile(src: str, force: bool) -> str:
         return obj
     cmd = [HIPCC, *FLAGS, "-c", src, "-o", obj]
     r = subprocess.run(cmd, capture_output=True, text=True)
-    err = "\n".join(l for l in r.stderr.splitlines() if "is not a recognized feature for this target" not in l)
+    remarks, err = _split_remarks(r.stderr)
     if r.returncode != 0:
         raise RuntimeError(f"hipcc failed for {src}:\n{err}")
+    try:
+        check_scratch(remarks, asm_read_kernels())
+    except RuntimeError:
+        os.remove(obj)
+        raise
     if err.strip():
         sys.stderr.write(err + "\n")
     return obj

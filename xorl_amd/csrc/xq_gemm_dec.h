@@ -225,7 +225,9 @@ __global__ void __launch_bounds__(512, 2) gemm_dec_kernel(G256Args g) {
 #pragma unroll
         for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
-    // ---- fragment reads, with the waits counted by hand (as in gemm_dtl16_kernel; no other LDS access inside the loop)
+    // ---- fragment reads, with the waits counted by hand (as in gemm_dtl16_kernel; no other LDS access inside the loop).  To the
+    // compiler a fragment is there with its read: were one spilled before its wait, what is stored would be what the register held
+    // before.  Hence no spills here at all, which the build checks.
     const int sw = (l16 >> 2) & 2;
     const uint32_t a_addr = lds0 + (wm * RW + l16) * 64 + ((lg ^ sw) << 4);
     const uint32_t w_addr = lds0 + G::A_BYTES + (wn * CW + l16) * 64 + ((lg ^ sw) << 4);
@@ -303,25 +305,31 @@ __global__ void __launch_bounds__(512, 2) gemm_dec_kernel(G256Args g) {
                 iteration(kt, I0{}, I3{}, SKIP_);
                 iteration(kt + 1, I1{}, I3{}, SKIP_);
             }
-            iteration(kt, I0{}, I3{}, SKIP_);
-            iteration(kt + 1, I1{}, I2{}, SKIP_);
-            iteration(kt + 2, I0{}, I1{}, SKIP_);
-            iteration(kt + 3, I1{}, I0{}, SKIP_);
         };
         if (mt == TM) run(std::false_type{});
         else run(std::true_type{});
+        // the last four of either loop, once: behind each of them the sums met with no register to spare and some went to scratch
+        const int kt = nk - 4;
+        iteration(kt, I0{}, I3{}, std::true_type{});
+        iteration(kt + 1, I1{}, I2{}, std::true_type{});
+        iteration(kt + 2, I0{}, I1{}, std::true_type{});
+        iteration(kt + 3, I1{}, I0{}, std::true_type{});
     }
 #undef XQ_DEC_READ
 
+    // (the lane read again: what the end needs of it is not kept through the loop)
+    int lane_e;
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=&v"(lane_e));
+    const int tid_e = wave * 64 + lane_e;
     if constexpr (SPLIT) {
         const int s = blockIdx.y;
         G256Args f = g;
         if (s > 0) { f.r_pad = 0; f.bias = nullptr; }
-        dtl16_side_term<TM, TN, 8, false>(f, dsm, G::ROWS * 128, acc, row0, row_end, n0, g.Nout, f.su, nullptr, 0);
+        dtl16_side_term<TM, TN, 8, false>(f, dsm, G::ROWS * 128, acc, row0, row_end, n0, g.Nout, f.su, nullptr, 0, tid_e);
         float* part = g.partial + (int64_t)s * g.M * g.Nout;
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
-            const int n = n0 + wn * CW + j * 16 + 4 * lg;
+            const int n = n0 + wn * CW + j * 16 + 4 * (lane_e >> 4);
             f32x4 b4 = {0.0f, 0.0f, 0.0f, 0.0f};
             if (f.bias) {
                 const u32x2 b = *(const u32x2*)(f.bias + min(n, g.Nout - 4));
@@ -329,12 +337,12 @@ __global__ void __launch_bounds__(512, 2) gemm_dec_kernel(G256Args g) {
             }
 #pragma unroll
             for (int i = 0; i < TM; ++i) {
-                const int64_t row = row0 + wm * RW + i * 16 + l16;
+                const int64_t row = row0 + wm * RW + i * 16 + (lane_e & 15);
                 if (row < row_end && n < g.Nout) *(f32x4*)(part + row * g.Nout + n) = acc[i][j] + b4;
             }
         }
     } else {
-        dtl16_finish<TM, TN, 8, false>(g, dsm, G::ROWS * 128, acc, row0, row_end, n0, n0, g.Nout, g.su, nullptr, 0);
+        dtl16_finish<TM, TN, 8, false>(g, dsm, G::ROWS * 128, acc, row0, row_end, n0, n0, g.Nout, g.su, nullptr, 0, tid_e);
     }
 }
 

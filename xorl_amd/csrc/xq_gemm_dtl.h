@@ -69,9 +69,10 @@ __device__ __forceinline__ u32x2 dtl_decode4(uint32_t w, float sc) {
 // bytes of every row; `second` bytes into it lies room for as much of every column.  First the low-rank side term:
 template <int TM, int TN, int NW, bool GROUPED>
 __device__ __forceinline__ void dtl16_side_term(const G256Args& g, unsigned char* dsm, int second, f32x4 (&acc)[TM][TN], int64_t row0,
-                                                int64_t row_end, int n0w, int bank_width, const bf16_t* su_b, const bf16_t* lr_b, int e) {
+                                                int64_t row_end, int n0w, int bank_width, const bf16_t* su_b, const bf16_t* lr_b, int e,
+                                                int tid = threadIdx.x) {
     constexpr int NT = NW * 64, RW = TM * 16, CW = TN * 16, TA = RW * (NW / 4), TB = CW * 4;
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = NW == 8 ? wave >> 2 : 0, wn = wave & 3;
     const int l16 = lane & 15, lg = lane >> 4;
     // ---- low-rank side term: su[rows, rp] x lora_right[n, rp] as bf16 [row][64 k] tiles in the first two stages, k beyond
@@ -116,11 +117,12 @@ __device__ __forceinline__ void dtl16_side_term(const G256Args& g, unsigned char
 // ... and the whole end: side term, bias, the way out as bf16
 template <int TM, int TN, int NW, bool GROUPED>
 __device__ __forceinline__ void dtl16_finish(const G256Args& g, unsigned char* dsm, int second, f32x4 (&acc)[TM][TN], int64_t row0,
-                                             int64_t row_end, int n0, int n0w, int bank_width, const bf16_t* su_b, const bf16_t* lr_b, int e) {
+                                             int64_t row_end, int n0, int n0w, int bank_width, const bf16_t* su_b, const bf16_t* lr_b, int e,
+                                             int tid = threadIdx.x) {
     constexpr int RW = TM * 16, CW = TN * 16;
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = NW == 8 ? wave >> 2 : 0, wn = wave & 3;
-    dtl16_side_term<TM, TN, NW, GROUPED>(g, dsm, second, acc, row0, row_end, n0w, bank_width, su_b, lr_b, e);
+    dtl16_side_term<TM, TN, NW, GROUPED>(g, dsm, second, acc, row0, row_end, n0w, bank_width, su_b, lr_b, e, tid);
 
     // ---- the finished tile.  Lane l holds, per (i, j) tile, row 16 i + l % 16 and the 4 columns 16 j + 4 (l / 16) ..: 8 bytes
     // of bf16.  Each wave passes its RW x CW sub-tile through a private LDS area and writes whole row pieces of 16 CW bytes / 8:

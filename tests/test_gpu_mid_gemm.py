@@ -34,6 +34,16 @@ def test_forward_and_backward(hip_device, fmt, M, N, K, r):
         assert err <= 1e-2, f"{name}: {err}"
 
 
+@pytest.mark.parametrize("M,N,K,r", [
+    (65, 1152, 384, 16),         # the shortest contraction that a forward brings here: three steps a phase
+    (130, 2176, 448, 64),        # phases of four and three steps, half a scale block at the end
+    (300, 960, 960, 8),
+    (513, 4096, 576, 32),
+])
+def test_short_block_fp8_contractions(hip_device, M, N, K, r):
+    test_forward_and_backward(hip_device, "block_fp8", M, N, K, r)
+
+
 @pytest.mark.parametrize("fmt", FORMATS)
 def test_decodes_bit_for_bit(hip_device, fmt):
     """Rows of the identity: a forward returns the decoded weight's columns, a dgrad its rows, without a rounding."""

@@ -175,7 +175,8 @@ def test_fused_mlp_under_torch_compile(hip_device, backend):
 def test_gate_up_form_travels_with_the_saved_state(hip_device):
     """The form a forward ran gate and up in (one launch or two) fixes the layout of the saved low-rank intermediates;
     it travels to the backward in xq_mlp_saved, so flipping the process-wide default between a forward and its backward
-    changes nothing: every gradient equals the undisturbed step's bit for bit, in both directions of the flip."""
+    changes nothing: every gradient equals the undisturbed step's bit for bit, in both directions of the flip.  Between the two
+    forms the bits are the same where the plain launches take the tile kernel of the joint one (xq_set_fp8_direct_tiles(0))."""
     from xorl_amd import _C
     from xorl_amd.qlora import qlora_mlp_forward
 
@@ -194,13 +195,21 @@ def test_gate_up_form_travels_with_the_saved_state(hip_device):
         y.backward(dy.to(hip_device))
         return {"y": y.detach().clone(), "dx": xd.grad.clone(), **_grads(mods)}
 
+    def equal(a, b, what):
+        for name in a:
+            assert torch.equal(a[name], b[name]), (*what, name)
+
     try:
+        two, one = step(0, 0), step(1, 1)
+        equal(step(0, 1), two, (0, 1))
+        equal(step(1, 0), one, (1, 0))
+        # the forms themselves: to the bit where both run on the same tile kernel
+        _C.check(L.xq_set_fp8_direct_tiles(0))
         base = step(0, 0)
         for fwd_mode, bwd_mode in ((0, 1), (1, 0), (1, 1)):
-            got = step(fwd_mode, bwd_mode)
-            for name in base:
-                assert torch.equal(got[name], base[name]), (fwd_mode, bwd_mode, name)
+            equal(step(fwd_mode, bwd_mode), base, (fwd_mode, bwd_mode))
     finally:
+        _C.check(L.xq_set_fp8_direct_tiles(1))
         _C.check(L.xq_set_mlp_gate_up_fused(0))
 
 

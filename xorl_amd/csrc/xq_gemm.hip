@@ -349,8 +349,10 @@ static double tile_kernels_us(int fmt, int64_t rows, int64_t Nout, int64_t Kc) {
 static bool mid_shape(int fmt, bool cc, int64_t rows, int64_t Nout, int64_t Kc) {
     // whole units of the contraction for both phases; 4-bit dgrads: whole 16-byte pieces of 32 columns, whole scale groups
     const int64_t unit = cc && fmt != XQ_FMT_FP8 ? 128 : 64;
-    // (block-fp8 forwards below 1024 k: the tile kernels' order of the sums, which the one launch over gate and up shares bit for bit)
-    return rows > 64 && Kc % unit == 0 && Kc >= (cc && fmt == XQ_FMT_FP8 ? 1024 : 2 * unit) &&
+    // (block-fp8 forwards below 384 k are few steps between two ends, and level with the tile kernels'.  Five widths of 512 .. 8192 under 65 .. 5000
+    // rows, us, tile kernels -> here: 960 k 1.10 to 1.37 times as fast ([4096, 960], 512 rows 15.1 -> 13.0), 768 k 1.11 to 1.29, 512 k 1.06 to
+    // 1.19, 320 k 0.95 to 1.08, 256 k 0.94 to 1.07, 192 k 0.88 to 1.02)
+    return rows > 64 && Kc % unit == 0 && Kc >= (cc && fmt == XQ_FMT_FP8 ? 384 : 2 * unit) &&
            (fmt != XQ_FMT_FP8 || Kc <= 64 * 2 * GeoMid<XQ_FMT_FP8, true, 4>::SCL_MAX) &&
            (cc || fmt == XQ_FMT_FP8 || Nout % (fmt == XQ_FMT_INT4 ? 128 : 64) == 0) && Nout >= 64;
 }

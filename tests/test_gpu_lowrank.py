@@ -128,3 +128,34 @@ def test_expert_weight_gradients_of_uneven_loads(hip_device, counts, r, rp, tran
             assert torch.count_nonzero(got[e]) == 0
     if R > 256 * len(used):
         assert torch.equal(got[used.to(hip_device)], MF._wgrad(P.to(hip_device), Q.to(hip_device), r, offsets(counts[used]), len(used), transpose))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("fmt,M,N,K", [
+    ("block_fp8", 97, 1168, 640),        # gemm_mid_kernel
+    ("block_fp8", 97, 1168, 192),        # 128 x 128 tiles
+    ("block_fp8", 2197, 6288, 192),      # gemm_dtl16_kernel
+    ("nf4", 2600, 2832, 2816),           # gemm_dec_kernel
+])
+@pytest.mark.parametrize("r", [1, 7, 9, 20, 33, 63, 64])
+def test_rows_of_the_right_factor_at_any_address(hip_device, fmt, M, N, K, r, dtype):
+    """Eight ranks of a row of B are read at once where they lie in the row: B begins off a 16-byte boundary and ends its allocation,
+    and every second of its rows is infinite, which no finite row's result may show."""
+    from xorl_amd.functional import qlora_linear
+
+    m, w = make_dense_module(fmt, N, K, 16, 32, seed=3, device=hip_device)
+    A, B = gen((r, K), 0.02, 1).to(dtype), gen((N, r), 0.02, 2).to(dtype)
+    B[1::2] = float("inf")
+    b = torch.empty(N * r + 1, dtype=dtype, device=hip_device)[1:].view(N, r)
+    b.copy_(B)
+    x = gen((M, K), 1.0, 4, torch.bfloat16).to(hip_device)
+    with torch.no_grad():
+        y = qlora_linear(x, m._quant_weight(), A.to(hip_device), b, r, 0.5)
+    xf, Af, even = x.float(), A.to(hip_device).float().t(), B[::2].to(hip_device).float().t()
+    u, au = xf @ Af, xf.abs() @ Af.abs()
+    want = xf @ w[::2].to(hip_device).float().t() + 0.5 * (u @ even)
+    # the result's rounding (2^-9, doubled for the fp32 sums) and, in the low-rank term, those of the inner factor's elements, of the
+    # intermediate and of the outer factor's (2^-9 of the terms each, nothing cancelling)
+    bound = 2 ** -8 * want.abs() + 0.5 * 2 ** -9 * ((au + 2 * u.abs()) @ even.abs()) + 1e-5 * want.abs().max()
+    assert bool(((y[:, ::2].float() - want).abs() <= bound).all())
+    assert not bool(torch.isfinite(y[:, 1::2]).any())

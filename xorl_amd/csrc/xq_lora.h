@@ -16,7 +16,14 @@ struct LowRankRight {
     int32_t r, rp;
     int32_t f32, transposed;
 };
-// 8 consecutive columns (chunk c) of row n, packed bf16; `which` >= 0 names the factor, < 0: by column
+// 8 consecutive columns (chunk c) of row n, packed bf16; `which` >= 0 names the factor, < 0: by column.  Eight columns of a row are one
+// or two 16-byte loads at whatever address they begin at, of a transposed factor eight loads in flight together: the branches on the
+// type and the form lie around the loads and what is converted is kept as it came, since a branch between two loads makes the second
+// wait for the first.
+// A forward at r 64, us, element by element with a branch at each -> now: block-fp8 [5120, 448], 302 rows 16.0 -> 10.9 (gemm_mid_kernel), [1024,
+// 320], 396 rows 13.0 -> 10.5 (128 x 128 tiles), [6272, 512], 2197 rows 32.3 -> 26.4 (gemm_dtl16_kernel); nf4 [7936, 2048], 1613 rows 68.7 ->
+// 64.9 (gemm_dec_kernel); a third of that at r 32, nothing at r 8.
+typedef u32x4 u32x4_any __attribute__((aligned(2)));
 __device__ __forceinline__ u32x4 right_chunk(const LowRankRight& q, int which, int n, int c) {
     int j0 = c * 8, k = which;
     if (k < 0) {
@@ -24,15 +31,40 @@ __device__ __forceinline__ u32x4 right_chunk(const LowRankRight& q, int which, i
         j0 -= k * q.rp;
     }
     const void* f = k ? q.f[1] : q.f[0];
+    const int have = q.r - j0;                                         // columns of the chunk before the padding
+    uint32_t raw[8];
+    auto load = [&](auto T_) {
+        typedef decltype(T_) T;
+        if (q.transposed) {
+            const T* p = (const T*)f + n;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) raw[e] = p[(int64_t)(e < have ? j0 + e : q.r - 1) * q.ld];
+        } else {
+            const T* p = (const T*)f + (int64_t)n * q.ld;
+            if (have >= 8) {
+                const u32x4 lo = *(const u32x4_any*)(p + j0);
+                u32x4 hi = {0u, 0u, 0u, 0u};
+                if constexpr (sizeof(T) == 4) hi = *(const u32x4_any*)(p + j0 + 4);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) { raw[e] = lo[e]; raw[4 + e] = hi[e]; }
+            } else {
+                uint32_t v[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[e] = p[e < have ? j0 + e : q.r - 1];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) raw[e] = sizeof(T) == 4 ? v[e] : e < 4 ? v[2 * (e & 3)] | v[2 * (e & 3) + 1] << 16 : 0u;
+            }
+        }
+    };
+    if (q.f32) load(uint32_t{});
+    else load(uint16_t{});
+    const bool pairs = !q.f32 && !q.transposed;                        // two bf16 to a word
     float v[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-        const int j = j0 + e < q.r ? j0 + e : q.r - 1;
-        const int64_t i = q.transposed ? j * q.ld + n : n * q.ld + j;
-        v[e] = q.f32 ? ((const float*)f)[i] : bf16_to_f32(((const bf16_t*)f)[i]);
+        const uint32_t bits = q.f32 ? raw[e] : !pairs ? raw[e] << 16 : e & 1 ? raw[e >> 1] & 0xffff0000u : raw[e >> 1] << 16;
+        v[e] = e < have ? __uint_as_float(bits) : 0.0f;
     }
-#pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = j0 + e < q.r ? v[e] : 0.0f;
     return u32x4{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7])};
 }
 

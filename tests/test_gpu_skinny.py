@@ -221,7 +221,9 @@ def test_skinny_seeded_shape_sweep(hip_device):
         close(y.cpu(), ex["y"], TOL)
 
 
-@pytest.mark.parametrize("N,K,r,bias", [(5120, 512, 16, True),     # four rows a wave at M = 64, two below; fewer splits than are requested at a time
+@pytest.mark.parametrize("N,K,r,bias", [(5120, 512, 16, True),     # four rows a wave: few splits
+                                        (5120, 512, 32, True),     # two rows a wave, fewer splits than are requested at a time
+                                        (12832, 512, 64, False),   # four rows a wave at M = 63 and 64, two below
                                         (1056, 4352, 8, False),    # nine splits or more, columns that end inside a block
                                         (640, 1024, 64, True)])    # four quads of ranks a row
 def test_epilogue_rows_per_wave(hip_device, N, K, r, bias):

@@ -371,8 +371,10 @@ struct EpiBatch {
 // columns (a lane 2) of RW rows, the block's waves the rows next to each other.  The kernel is a few dependent memory round
 // trips long: everything the first sums need -- B values of the first 16 ranks, partial tiles, low-rank parts (dealt over all
 // threads, met in LDS) -- is requested before anything is waited for.  Every sum runs in a fixed order.
-// RW: 1 up to 16 rows; 2 with eight splits requested at a time above (4 rows and four splits, which took fewer blocks and twice the
-// trips: int4 MLP [12288, 4096] M = 64 70.7 -> 69.1 us whole, int4 [1024, 4096] 13.9 -> 12.8, nf4 [12288, 4096] M = 24 26.1 -> 24.0).
+// RW: 1 up to 16 rows; 2 with eight splits requested at a time above, against 4 rows and four splits, which took fewer blocks and
+// twice the trips.  Whole forwards at r 16 / 64, us, of 24 rows: int4 [1024, 4096] 14.4 -> 12.4 / 18.8 -> 14.7, [4096, 4096] 15.1 -> 14.0 /
+// 19.4 -> 16.3, [4096, 12288] 19.0 -> 17.5 / 26.9 -> 21.7; of 64 rows: 13.5 -> 12.5 / 18.1 -> 15.1, 15.9 -> 15.7 / 20.2 -> 18.2, 24.4 -> 23.4 /
+// 32.1 -> 27.6.  [12288, 4096], where the epilogue is the smaller part, is level at r 16.
 // VEC: B is fp32 with r % 4 == 0 (16-byte pieces).  GU: jobs 0 and 1 are gate and up, h is written.
 template <int RW, bool VEC, bool GU>
 __global__ void __launch_bounds__(256)
@@ -741,12 +743,24 @@ int launch_skinny_stream(const SkinnyRowsJob* jobs, int n_jobs, bool swiglu, con
 #undef XQ_STREAM_CASE
     if (rc) return rc;
     const unsigned cols = (unsigned)(swiglu ? efirst[1] : efirst[4]);
-    // (four rows a wave where that is one block a compute unit and two rows would be a few blocks more than one: [5120, 1536] M = 64
-    // 14.6 us against 15.3, [12288, 4096] M = 17 18.7 against 19.2; from rank 17 on two are faster there too)
-    int ranks = 0;
-    for (int i = 0; i < n_jobs; ++i) ranks = e.job[i].r_pad > ranks ? e.job[i].r_pad : ranks;
+    // Four rows a wave and four splits at a time, us against two rows and eight (whole passes, all else equal):
+    //  * two rows would be more than three blocks a compute unit: int4 [14720, 4864], 51 rows, r 32 / 64: 30.8 against 32.7 / 33.7 against
+    //    36.1; MLP of 14720 x 4864, 64 rows: int4 94.0 / 99.7 and 104.4 / 111.8, nf4 109.4 / 114.8 and 120.5 / 127.6.  (At three blocks,
+    //    12288 columns and 64 rows, four rows are level at r 16, 1.5 per cent slower at r 32, 3 at r 64; at 2.7, 14720 columns and 48
+    //    rows, -3 to 1 per cent.)
+    //  * no more than four splits, which are one request then: up to rank 16 (MLP of 9088 x 2944, 64 rows, nf4 51.4 against 52.8), to rank
+    //    32 where a row of blocks fills half the chip ([16384, 2048], 17 rows 14.3 against 15.0); below that, and at r 64, two rows are up to
+    //    4 per cent faster.
+    //  * up to rank 16, where they are one block a compute unit and two rows a few blocks more than one: [5120, 1536], 64 rows 14.6
+    //    against 15.3, [12288, 4096], 17 rows 18.7 against 19.2.
+    int ranks = 0, most = 0;
+    for (int i = 0; i < n_jobs; ++i) {
+        ranks = e.job[i].r_pad > ranks ? e.job[i].r_pad : ranks;
+        most = splits[i] > most ? splits[i] : most;
+    }
     const int64_t by2 = xq_cdiv((int64_t)cols * xq_cdiv(M, 8), num_cus()), by4 = xq_cdiv((int64_t)cols * xq_cdiv(M, 16), num_cus());
-    const int rw = M <= 16 ? 1 : ranks <= 16 && 17 * by4 < 10 * by2 ? 4 : 2;
+    const bool four = by2 > 3 || (most <= 4 && ranks <= (2 * (int64_t)cols >= num_cus() ? 32 : 16)) || (ranks <= 16 && 17 * by4 < 10 * by2);
+    const int rw = M <= 16 ? 1 : four ? 4 : 2;
     const unsigned threads = M < 4 && rw == 1 ? (unsigned)M * 64 : 256;
     const dim3 grid(cols, (unsigned)xq_cdiv(M, 4 * rw));
 #define XQ_EPI(RW)                                                                                                                             \

@@ -104,6 +104,16 @@ int xq_read_probe(const void* data, int64_t bytes, uint32_t* out, void* stream);
  *      allows it, whatever the size. */
 int xq_set_tile_policy(int policy);
 
+/* What policy 0 runs a dense product [rows, n_out] over a contraction of k on (forward: over the weight's columns, otherwise over its
+ * rows; weights of the formats' usual groups, enough workspace), for tests that are about one kernel: returns XQ_ROUTE_TILES (the
+ * pipelined tile kernels), XQ_ROUTE_IMAGE (the weight decoded first), XQ_ROUTE_MID (decoded in registers), or -1 where the
+ * library does not take the product.  plan: rows and columns of a tile and K splits of the leading rows' launch, then the same of
+ * the trailing rows' (0: there is none).  No counterpart in the reference. */
+#define XQ_ROUTE_TILES 0
+#define XQ_ROUTE_IMAGE 1
+#define XQ_ROUTE_MID 2
+int xq_dense_route(int format, int forward, int64_t rows, int64_t n_out, int64_t k, int32_t plan[6]);
+
 /* The 256x256 tile kernel (unsplit launches) is a persistent program: one block per compute unit walks the
  * tiles b, b + grid, ... and requests its next tile's first operands before it stores the finished tile.
  * enabled = 0 launches one block per tile instead -- the same kernel and, bit for bit, the same results; a
@@ -113,8 +123,9 @@ int xq_set_persistent_tiles(int enabled);
 
 /* Dense block-fp8 products on 256 x 256 tiles (forward, dgrad; unsplit) run on the kernel that loads both operand tiles
  * straight into LDS, keeps the weight tile as e4m3 bytes there and multiplies with v_mfma_f32_16x16x32_bf16 (enabled = 1,
- * the default), or on the tile kernel that every other format and the expert banks use (enabled = 0).  Both decode to the
- * reference's bf16 values bit for bit; their sums run in different orders, so outputs agree to rounding.  A process-wide
+ * the default), or on the tile kernel that every other format and the expert banks use (enabled = 0, which also keeps dense
+ * block-fp8 products off the kernels that decode in registers and over a decoded image).  All decode to the reference's bf16
+ * values bit for bit; their sums run in different orders, so outputs agree to rounding.  A process-wide
  * switch for tests and A/B measurements (XQ_FP8_DIRECT in the environment sets it at load time); no counterpart in the
  * reference. */
 int xq_set_fp8_direct_tiles(int enabled);

@@ -6,7 +6,7 @@ import pytest
 import torch
 
 from oracle import recipe as R
-from tests.util_cases import close, gen, make_dense_module
+from tests.util_cases import close, dense_route, gen, make_dense_module
 
 pytestmark = pytest.mark.gpu
 TOL = 1e-2
@@ -191,20 +191,25 @@ def test_silu_and_mul(hip_device):
     close(ud.grad.cpu(), u64.grad, TOL)
 
 
-@pytest.mark.parametrize("fmt,M,K,N", [("block_fp8", 4100, 256, 4096), ("int4", 4352, 384, 5120), ("nvfp4", 4099, 256, 4352),
-                                       ("block_fp8", 4352, 2048, 4096), ("nvfp4", 4200, 2048, 4096)])
-def test_dense_split_launch_tail_rows(hip_device, fmt, M, K, N):
+@pytest.mark.parametrize("fmt,M,K,N,tail", [
+    ("block_fp8", 4100, 256, 4096, (128, 128, 1)), ("int4", 4352, 384, 5120, (128, 128, 1)), ("nvfp4", 4099, 256, 4352, (128, 128, 1)),
+    ("block_fp8", 1161, 1792, 16256, (256, 256, 3)),
+    ("block_fp8", 4352, 2048, 4096, None), ("nvfp4", 4200, 2048, 4096, None),       # (forwards that are decoded first)
+])
+def test_dense_split_launch_tail_rows(hip_device, fmt, M, K, N, tail):
     """Shapes whose 256x256 tiling leaves a partly filled last round of the chip: the launcher runs the leading
-    tile rows on large tiles and the trailing rows (here 4, 256, 3 + 256, 256 and 104 of them) as a second launch:
+    tile rows on large tiles and the trailing rows (here 4, 256, 3 + 256 and 137 of them in the forward) as a second launch:
     of small tiles when the contraction is short, of large tiles in K splits (fp32 partial sums added by a reduce
-    kernel) when it has at least 16 K-steps -- the last two cases.  Forward, dgrad and both factor gradients
-    against the float64 form, with particular attention to the rows on either side of the seam."""
+    kernel) when it has at least 16 K-steps -- the fourth case.  The last two are of sizes where the weight is decoded
+    first instead.  Forward, dgrad and both factor gradients against the float64 form, with particular attention to the
+    rows on either side of the seam."""
+    assert dense_route(fmt, True, M, N, K)[:1 if tail is None else 7] == (("image",) if tail is None else ("tiles", 256, 256, 1, *tail))
     r = 16
     if K >= 1024:
         from xorl_amd import _C
 
-        tail = M - (M // 256) * 256 if M % 256 else 256
-        assert _C.lib().xq_linear_workspace_bytes(M, N, K, 0) >= 2 * tail * N * 4      # the plan splits the tail
+        rows = M - (M // 256) * 256 if M % 256 else 256
+        assert _C.lib().xq_linear_workspace_bytes(M, N, K, 0) >= 2 * rows * N * 4      # the plan splits the tail
     m, w_ref = make_dense_module(fmt, N, K, r, 32, seed=M + N, device=hip_device, bias=True)
     x = gen((M, K), 1.0, 31, torch.bfloat16)
     dy = gen((M, N), 1.0, 32, torch.bfloat16)

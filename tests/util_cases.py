@@ -71,6 +71,16 @@ def make_dense_module(fmt: str, N: int, K: int, r: int, alpha: int, seed: int, d
     return m.to(device), w_ref
 
 
+def dense_route(fmt: str, forward: bool, rows: int, n_out: int, k: int) -> tuple:
+    """What a dense product runs on (xq_dense_route in include/xq.h): "tiles", "image" or "mid", then the plan's six numbers."""
+    import ctypes
+
+    from xorl_amd import _C
+
+    plan = (ctypes.c_int32 * 6)()
+    return (["tiles", "image", "mid"][_C.lib().xq_dense_route(_C.FORMATS[fmt], int(forward), rows, n_out, k, plan)], *plan)
+
+
 def oracle_decode_dense(m) -> torch.Tensor:
     """Decode a (CPU) module's packed state with the numpy oracle -> bf16 [N, K]."""
     N, K = m.out_features, m.in_features

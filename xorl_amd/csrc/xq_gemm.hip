@@ -300,7 +300,8 @@ static int64_t decoded_scratch_bytes(int fmt, int64_t n_rows, int64_t Nout, int6
 // ---- products that gemm_mid_kernel (xq_gemm_mid.h) takes.  Estimates in microseconds, each within about 5 per cent of what was
 // measured (four formats, rows 80 .. 3000, weights [4096, 4096], [12288, 4096], [1024, 4096] and [2560, 8192], both directions); the
 // launch goes to the kernel with the shorter one.  70 random products of 65 .. 4096 rows over the formats, both directions: 1.16
-// times as fast in the mean, up to 1.8.  Forward / dgrad, this kernel against the tile kernels (from 640 rows on 4-bit:
+// times as fast in the mean, up to 1.8.  There is no upper end to the rows: of 438 random products of 3000 .. 8192
+// rows 60 came here (256 .. 2176 columns), at 0.69 to 1.00 of the tile kernels' time, 0.85 in the mean.  Forward / dgrad, this kernel against the tile kernels (from 640 rows on 4-bit:
 // over decoded images):
 //   [4096, 4096]    rows       100          256          512         1024         2048         3000
 //   int4             21.3 / 24.9  26.5 / 31.2  35.0 / 42.6  44.6 / 63.0  63.8 / 84.7  103.9 / 89.6 (forward)
@@ -375,6 +376,31 @@ static bool takes_mid(int fmt, bool cc, int64_t rows, int64_t Nout, int64_t Kc, 
 static int64_t mid_partial_bytes(int fmt, bool cc, int64_t rows, int64_t Nout, int64_t Kc) {
     MidPlan p;
     return takes_mid(fmt, cc, rows, Nout, Kc, &p) && p.split > 1 ? p.split * rows * Nout * 4 : 0;
+}
+
+extern "C" int xq_dense_route(int format, int forward, int64_t rows, int64_t n_out, int64_t k, int32_t plan[6]) {
+    if (format < XQ_FMT_INT4 || format > XQ_FMT_NF4 || rows <= 0 || n_out <= 0 || k <= 0 || k % BK || n_out % 16) return -1;
+    for (int i = 0; i < 6; ++i) plan[i] = 0;
+    auto put = [&](int part, int tile_rows, int tile_cols, int split) {
+        plan[3 * part] = tile_rows;
+        plan[3 * part + 1] = tile_cols;
+        plan[3 * part + 2] = split;
+    };
+    MidPlan mid;
+    if (takes_mid(format, forward != 0, rows, n_out, k, &mid)) {
+        put(0, 32 * mid.mw, 256, mid.split);
+        return XQ_ROUTE_MID;
+    }
+    if (decode_first(format, rows, n_out, k)) {
+        const DecPlan p = plan_decoded(rows, n_out, k);
+        for (int i = 0; i < 2; ++i)
+            if (p.part[i].rows > 0) put(i, 32 * kDecTiles[p.part[i].tile].tm, 64 * kDecTiles[p.part[i].tile].tn, p.part[i].split);
+        return XQ_ROUTE_IMAGE;
+    }
+    const DensePlan p = plan_dense(rows, n_out, k / BK);
+    put(0, p.T, p.T, p.split);
+    if (p.head_rows < rows) put(1, p.tail_T, p.tail_T, p.tail_split);
+    return XQ_ROUTE_TILES;
 }
 
 // fp32 partial-sum bytes the split-K forms of a dense [n_rows, Nout] product over Kc may want, under any tile policy

@@ -1,5 +1,6 @@
-// Fused dequant-GEMM for dense weights under 65 .. some hundreds of rows: every weight value is decoded by exactly one wave per 32 MW
-// rows, in registers, straight into the operand of v_mfma_f32_32x32x16_bf16.
+// Fused dequant-GEMM for dense weights from 65 rows on, wherever it is the shorter one by the estimates (xq_gemm.hip: most products of
+// some hundreds of rows, narrow ones of thousands): every weight value is decoded by exactly one wave per 32 MW rows, in registers,
+// straight into the operand of v_mfma_f32_32x32x16_bf16.
 //
 //   C[rows, Nout] = A[rows, Kc] . Wop (+ su[rows, r] . right[Nout, r]^T) (+ bias)
 //     CC  (forward): Wop[kc][n] = W[n][kc]        !CC (dgrad): Wop[kc][n] = W[kc][n]

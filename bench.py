@@ -43,13 +43,13 @@ BF16_MFMA_PEAK_TFLOPS = 2500.0   # MI355X dense bf16, published
 MEASURED_TRAFFIC = {
     # gemm_mid_kernel<int4> in 2 K splits + splitk_reduce_kernel: mean of the forward and dgrad launches
     # (32 MiB of it are the fp32 partial sums written and read back)
-    0: (77.7 * 2 ** 20, "profiles/gemm_mid_int4_linear_m512.txt", 0.03818),
+    0: (77.7 * 2 ** 20, "profiles/gemm_mid_int4_linear_m512.txt", 0.03837),
     # gemm_dec_kernel and the dec_image passes before it (dense block-fp8, 256x256 tiles over decoded images): mean over the 5
     # products of a step (gate, up and down forward, d_h, dx as one sum over the gate and up weights)
-    1: (1708.6 * 2 ** 20, "profiles/gemm_dec_fp8_mlp_m8192.txt", 0.7336),
+    1: (1708.8 * 2 ** 20, "profiles/gemm_dec_fp8_mlp_m8192.txt", 0.7417),
     # gemm_dec_kernel and dec_image passes (config 2: gemm_mid_kernel too) over nvfp4 / NF4 weights: mean over the products of a step (8 and 6)
-    2: (393.3 * 2 ** 20, "profiles/gemm_dec_4bit_m4096_m8192.txt", 0.1666),
-    6: (1424.2 * 2 ** 20, "profiles/gemm_dec_4bit_m4096_m8192.txt", 0.6019),
+    2: (386.2 * 2 ** 20, "profiles/gemm_dec_4bit_m4096_m8192.txt", 0.1674),
+    6: (1424.2 * 2 ** 20, "profiles/gemm_dec_4bit_m4096_m8192.txt", 0.6174),
     # gemm_dtl16_kernel<.., grouped>: mean over the 4 launches of a step (gate|up forward over two banks, down
     # forward, d_h, dx as one sum over both banks)
     3: (1402.4 * 2 ** 20, "profiles/gemm_dtl16_fp8_grouped_moe_e128.txt", 0.6325),
@@ -58,11 +58,11 @@ MEASURED_TRAFFIC = {
     # written and read back: 23.3 MiB of it are algorithmic)
     4: (34.2 * 2 ** 20, "profiles/skinny_kernels_decode_shapes.txt", 0.01557),
     # merge_fp8_kernel and merge_kernel<fp8>: mean per call (re-quantise 96 MiB, publish 144 MiB algorithmic)
-    5: (132.1 * 2 ** 20, "profiles/merge_kernel_fp8_mlp_weights.txt", 0.03895),
+    5: (132.1 * 2 ** 20, "profiles/merge_kernel_fp8_mlp_weights.txt", 0.03898),
     # gemm_256_kernel<nvfp4 GKN, grouped>: mean over the 6 launches of a step
     7: (893.9 * 2 ** 20, "profiles/gemm_256_nvfp4_gkn_grouped_moe_e128.txt", 0.52825),
     # merge_kernel<nvfp4>: mean per call over amax / re-quantise / publish of the four weights
-    9: (56.1 * 2 ** 20, "profiles/merge_kernel_nvfp4_attn_weights.txt", 0.02250),
+    9: (55.6 * 2 ** 20, "profiles/merge_kernel_nvfp4_attn_weights.txt", 0.02234),
 }
 
 

@@ -35,6 +35,20 @@ int64_t xq_scale_bytes_per_expert(const xq_weight* w);
 static inline int64_t xq_cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 static inline bool xq_aligned(const void* p, size_t a) { return ((uintptr_t)p % a) == 0; }
 
+// The estimates of a product are asked for several times a call (its workspace, its route, its launches) and take microseconds: a thread
+// keeps the last ones it made, in tables of 64 of these.  They depend on nothing but the key.
+struct PlanKey {
+    int64_t rows, Nout, Kc, cus;
+    int32_t kind;
+    bool operator==(const PlanKey& o) const { return rows == o.rows && Nout == o.Nout && Kc == o.Kc && cus == o.cus && kind == o.kind; }
+    unsigned slot() const { return (unsigned)(rows * 0x9e3779b1u + Nout * 0x85ebca6bu + Kc * 0xc2b2ae35u + kind * 0x27d4eb2fu) >> 16 & 63u; }
+};
+template <typename V>
+struct PlanSlot {
+    PlanKey key;              // rows 0: empty
+    V value;
+};
+
 // ---------------------------------------------------------------- vector types
 typedef __attribute__((ext_vector_type(2))) float f32x2;
 typedef __attribute__((ext_vector_type(4))) float f32x4;

@@ -249,19 +249,6 @@ static DecPlan make_plan_decoded(int64_t n_rows, int64_t Nout, int64_t Kc, int64
         if (d.split > 1) p.partial = std::max(p.partial, d.split * d.rows * Nout * 4);
     return p;
 }
-// The estimates of a product are asked for several times a call (its workspace, its route, its launches) and take microseconds: a thread
-// keeps the last ones it made.  They depend on nothing but the key.
-struct PlanKey {
-    int64_t rows, Nout, Kc, cus;
-    int32_t kind;
-    bool operator==(const PlanKey& o) const { return rows == o.rows && Nout == o.Nout && Kc == o.Kc && cus == o.cus && kind == o.kind; }
-    unsigned slot() const { return (unsigned)(rows * 0x9e3779b1u + Nout * 0x85ebca6bu + Kc * 0xc2b2ae35u + kind * 0x27d4eb2fu) >> 16 & 63u; }
-};
-template <typename V>
-struct PlanSlot {
-    PlanKey key;              // rows 0: empty
-    V value;
-};
 static DecPlan plan_decoded(int64_t n_rows, int64_t Nout, int64_t Kc) {
     static thread_local PlanSlot<DecPlan> kept[64];
     const PlanKey key{n_rows, Nout, Kc, num_cus(), 0};

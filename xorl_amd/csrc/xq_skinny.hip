@@ -587,7 +587,7 @@ static int stream_row_tiles(const int* tiles, const int* splits, int n, int step
 static int stream_steps_max(int64_t M) { return M <= 16 ? 32 : M <= 32 ? 16 : 8; }
 // K splits of a forward, by its own shape: the cheapest sum of that and of the partial sums' trip (written and read back, ~6
 // TB/s)
-static int stream_splits(int64_t M, int64_t N, int64_t K) {
+static int make_stream_splits(int64_t M, int64_t N, int64_t K) {
     const int ct = (int)(K >> 7), tiles = (int)(N / 16);
     const int mt = M <= 16 ? 1 : M <= 32 ? 2 : 4;
     int best = 0, last_steps = 0;
@@ -603,6 +603,14 @@ static int stream_splits(int64_t M, int64_t N, int64_t K) {
         if (best == 0 || c < best_cost) { best = s; best_cost = c; }
     }
     return best;
+}
+
+static int stream_splits(int64_t M, int64_t N, int64_t K) {
+    static thread_local PlanSlot<int> kept[64];
+    const PlanKey key{M, N, K, num_cus(), 0};
+    PlanSlot<int>& e = kept[key.slot()];
+    if (!(e.key == key)) e = PlanSlot<int>{key, make_stream_splits(M, N, K)};
+    return e.value;
 }
 
 // whether a forward of this shape runs on the two launches of this file (and not in one, xq_skinny_rows.hip)

@@ -92,3 +92,24 @@ def test_fp32_nvfp4_scales_at_four_bytes(hip_device):
             m.weight_block_scales = flat[4:4 + s.numel()].view(s.shape)
             m.weight_block_scales.copy_(s)
             assert torch.equal(m(x), want)
+
+
+@pytest.mark.parametrize("fmt,N,K,r,Ms", [
+    ("int4", 16, 1152, 64, (17, 64)),            # one row tile, four rank tiles: blocks that only form a low-rank part; an odd last step
+    ("nf4", 48, 1024, 40, (20, 49)),             # fewer steps than waves once K is split
+    ("int4", 12288, 5248, 16, (33, 64)),         # six and five steps a wave: a second window of scales, odd ranges, six row tiles
+    ("nvfp4", 12320, 5248, 24, (48, 64)),        # the same with byte scales; a last row block that is partly past the end
+    ("block_fp8", 12288, 4096, 16, (32, 64)),    # several half steps of x in flight, and one
+    ("nvfp4", 24560, 1152, 16, (64,)),           # six row tiles, the last block's past the end
+    ("nf4", 7824, 2944, 64, (24, 56)),           # 23 steps: three and two a wave; rows of x that end inside eight
+])
+def test_waves_that_split_the_contraction(hip_device, fmt, N, K, r, Ms):
+    m, w_ref = make_dense_module(fmt, N, K, r, 2 * r, seed=N + K, device=hip_device)
+    A, B = m.lora_A.detach().cpu(), m.lora_B.detach().cpu()
+    for M in Ms:
+        wide = gen((M, K + 64), 1.0, M, torch.bfloat16)           # rows that do not follow each other
+        with torch.no_grad():
+            y = m(wide.to(hip_device)[:, :K])
+            assert torch.equal(m(wide[:, :K].contiguous().to(hip_device)), y)
+        ex = R.linear_fwd_bwd_exact(wide[:, :K].contiguous(), w_ref, A, B, m.scaling, torch.zeros(M, N, dtype=torch.bfloat16))
+        close(y.cpu(), ex["y"], 1e-2)                             # (the bound of every forward above)

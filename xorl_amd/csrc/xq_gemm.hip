@@ -899,7 +899,7 @@ extern "C" int xq_linear_fwd(const xq_weight* w, const void* x, int64_t ldx, int
     XQ_REQUIRE(ldy % 8 == 0 && xq_aligned(y, 16), "xq_linear_fwd: y rows must be 16-byte aligned");
     const int rp = r_pad_of(r);
     // decode / rollout shapes: stream the packed weight once (HBM-bound kernel); forward only
-    if (!su_out && g_skinny_enabled && skinny_supported(w, M))
+    if (!su_out && g_skinny_enabled && skinny_supported(w, M) && (M <= 8 || ldx < kSkinnyLdx))
         return launch_skinny(w, (const bf16_t*)x, ldx, M, lora_A, lora_B, lora_dtype, r, scaling,
                              (const bf16_t*)bias_bf16, (bf16_t*)y, ldy, workspace, workspace_bytes, stream);
     bf16_t* su = nullptr;
@@ -1061,7 +1061,7 @@ extern "C" int xq_linear_fwd_multi(const xq_linear_job* jobs, int n_jobs, const 
         }
     }
     // decode shapes outside the whole-row kernel: every forward in one streaming launch and one epilogue
-    if (g_skinny_enabled && n_jobs > 1 && M <= 16 && ldx % 8 == 0 && xq_aligned(x, 16)) {
+    if (g_skinny_enabled && n_jobs > 1 && M <= 16 && ldx % 8 == 0 && (M <= 8 || ldx < kSkinnyLdx) && xq_aligned(x, 16)) {
         SkinnyRowsJob sj[XQ_LINEAR_MULTI_MAX];
         double bytes = 2.0 * M * jobs[0].w->cols;
         bool ok = true;

@@ -48,6 +48,9 @@ __device__ __forceinline__ bf16x8 decode8(uint32_t w0, uint32_t w1, float s0, fl
     return __builtin_bit_cast(bf16x8, r);
 }
 
+// rows of x further apart than this take the tile kernels: the streaming kernels' addresses within eight rows are 32 bits wide
+constexpr int64_t kSkinnyLdx = 1ll << 28;
+
 void set_skinny_rows(int enabled);
 bool skinny_rows_enabled();
 void set_skinny_rows_spin_limit(int limit);   // <= 0: the default

@@ -6,26 +6,28 @@
 // reference decoder and fed to v_mfma_f32_16x16x32_bf16 against x fragments.  Two launches for up to four forwards on one x
 // (q + k + v, gate + up), no atomics, no zeroed buffers, fixed summation orders (deterministic):
 //
-//  1. stream_split_kernel: a grid of (row block) x (K split) tiles, one block of 8 waves per compute unit (two at M <= 32).
-//     A wave owns 16 RT weight rows and streams them straight from memory into registers in the MFMA operand layout (a load
-//     instruction takes 64 contiguous bytes of each of 16 rows), D steps of 128 elements in flight; rows are not shared
-//     between waves, so the weight never passes through LDS.  x does: the block's whole slice [16 MT rows][K range] comes by
-//     direct-to-LDS loads at the start (one barrier) and every wave reads its fragments from there -- the slice costs
-//     1 / (8 RT) of what it would if each 16 weight rows fetched it, and nothing in the stream waits for a barrier.
-//     The tile's sides balance what a block moves beside its weights, x (2 M K_b bytes) and fp32 partial sums
-//     (8 M R_b bytes, written and read back): few, tall blocks for wide weights.  The blocks of `splits` leading tiles
-//     compute the low-rank parts x . A^T of one split each.
+//  1. stream_split_kernel: a grid of (row block) x (K split) tiles, one block of 8 waves per compute unit (two where the tile is
+//     small).  The block owns 16 RT weight rows, each wave an eighth of the split's K range of all of them: a wave brings its x and its
+//     weights into a part of LDS that is its own, by direct-to-LDS loads of whole 128-byte row pieces that run ahead, and waits for
+//     them by count, so nothing in the stream waits for another wave.  The eight waves' sums meet in LDS at the end.  What a block
+//     moves beside its weights is x (2 M K_b bytes, from the L2) and one fp32 partial sum per output and split.  One wave each of
+//     some blocks forms the low-rank parts x . A^T on the way.
 //  2. stream_epilogue_kernel: sums the splits in order, adds bias and s * su . B^T in fp32 and rounds once to bf16; for gate
 //     and up of an MLP it writes h = SwiGLU(gate, up) of the two rounded outputs instead.
 //
 // The split of K depends on a forward's own shape only: a joint launch gives the bits of the separate ones.
 //
-// What bounds it: at 64 rows the vector units (the 25 instructions that decode and feed one fragment of 8 weights a lane) and the
-// matrix units, not memory: gate | up of 4096 -> 2 x 12288 in int4 takes 26 us (30 MB fetched) and its epilogue 13 us, half of
-// which is the trip of the partial sums; at few rows the fixed costs of two dependent launches.  Forward of a SwiGLU MLP, us,
-// against one that fetched x per 16 weight rows and ran gate, up, SwiGLU and down as separate launches:
-//     int4  4096/12288, r 16: M = 24 62 -> 49, M = 64 90 -> 65      int4  2944/7808, r 32: M = 1 64 -> 34, M = 64 70 -> 49
-//     fp8   4096/12288, r 16: M = 64 92 -> 76                       nvfp4 2944/7808, r 32: M = 1 71 -> 36
+// What bounds it: at 64 rows and RT 6 about 5 us until the first weights are there (half of a wave's rows at once in the order in which
+// they are multiplied), 14 for products that the vector units' decode bounds (19 instructions and four MFMAs per 8 weights a lane,
+// two waves a SIMD), 4 until the slowest wave is done and the sums have met: gate | up of 4096 -> 2 x 12288 takes 26 us in int4
+// (50 MB), 31 in block-fp8 (100 MB), and the epilogue 10; at few rows the fixed costs of two dependent launches.  Before, waves owned
+// rows, K was split between five to sixteen blocks, and fragments were loaded straight to registers: 32 + 13 and 36 + 13 us.  Forward
+// of one projection at r 16, weights from memory, us, against that (24 / 40 or 48 / 64 rows):
+//     int4 [12288, 4096] 19.6 23.4 25.8 -> 18.8 20.3 23.2    [4096, 4096] 14.8 15.4 16.6 -> 11.8 13.2 14.4    [2944, 7808] 18.2 -> 17.6 at 64
+//     fp8  [12288, 4096] 22.8 23.6 26.2 -> 22.4 24.3 27.3    [4096, 4096] 15.8 16.1 17.3 -> 13.6 15.6 15.5    [1024, 4096] 13.8 -> 12.3 at 64
+//     nvfp4 [12288, 4096], 64 rows 27.4 -> 25.1, nf4 29.9 -> 26.2; of the MLP 4096 / 12288 of 64 rows: int4 64.1 -> 54.8, fp8 75 -> 67
+// (Block-fp8 of more than 32 rows and 8000 to 12000 rows of weights is 3 to 4 % behind there: a wave's LDS holds one half step of x then,
+// and x waits for the weights requested before it.  Gate and up of an MLP, which are those very products, are 8 % ahead as one launch.)
 #include <stdlib.h>
 
 #include <atomic>
@@ -56,28 +58,56 @@ struct StreamBatch {
     StreamJob job[kStreamJobs];
 };
 
-// how a lane gets the scales of its codes: with the step's weights (one or two words), four steps' bf16 scales of int4
-// groups of 128 in one load, four steps' 8 scale bytes dealt over the row's four lanes, per fragment at use, or (block-fp8)
-// one value per row tile and step from registers
-enum { kScFp8 = 0, kScInt4Window = 1, kScDealt = 2, kScStep = 3, kScUse = 4 };
+// how a lane gets the scales of its codes: four steps' bf16 scales of int4 groups of 128 in one load, four steps' 8 scale bytes (nvfp4
+// e4m3, nf4 fp32) dealt over the row's four lanes, one per half step or per fragment, requested a half step ahead, or (block-fp8) one
+// value per row tile and step from registers
+enum { kScFp8 = 0, kScInt4Window = 1, kScDealt = 2, kScHalf = 3, kScUse = 4 };
 
 // scales lie where their elements may: a pair of words from any byte (one global_load_dwordx2 like an aligned one)
 typedef u32x2 u32x2_a1 __attribute__((aligned(1)));
 
-// element offset of fragment (j, q) within a 128-element step: what lane q of a row holds after its loads (block-fp8: two
-// loads of 16 bytes, 64 apart; 4-bit: one load of 16 bytes), so that a load instruction covers 64 contiguous bytes of a row
-template <int FMT>
-__device__ __forceinline__ int frag_k(int j, int q) {
-    return FMT == XQ_FMT_FP8 ? (j >> 1) * 64 + q * 16 + (j & 1) * 8 : q * 32 + j * 8;
-}
+// What a wave keeps in LDS: XB half steps of x (16 MT rows of 64 elements each) and WB units of weights (128 bytes of each of its 16 RT
+// rows: a step of block-fp8, two steps of the 4-bit formats).
+template <int FMT, int MT, int RT>
+struct StreamGeo {
+    static constexpr int HPW = FMT == XQ_FMT_FP8 ? 2 : 4;          // half steps of a weight unit
+    static constexpr int XH = MT * 2048, WU = RT * 2048;
+    static constexpr bool PAIR = MT < 4 && MT * RT <= (FMT == XQ_FMT_NF4 ? 3 : 4);     // two blocks per compute unit (the levels of nf4 take the last bytes)
+    static constexpr int ROOM = (PAIR ? 80 : 160) * 128 - (FMT == XQ_FMT_NF4 ? 16 : 0);
+    static constexpr int XB = 3 * XH + 2 * WU <= ROOM ? 3 : 2 * XH + WU <= ROOM ? 2 : 1;
+    static constexpr int WB = XB * XH + 2 * WU <= ROOM ? 2 : 1;
+    static constexpr int WAVE = XB * XH + WB * WU;
+    static constexpr int NX = 2 * MT, NW = 2 * RT;                 // loads of a half step of x, of a weight unit
+    static constexpr int EARLY = RT > 1 ? RT / 2 : 1;              // row tiles that the first half step waits for at its start
+    static_assert(WAVE <= ROOM, "the wave's LDS");
+    // Half step v requests x of v + XB and, once the unit's last step has gone to registers, the weight unit WB ahead
+    static constexpr bool issues_w(int v) { return (v & (HPW - 1)) == HPW - 2; }
+    // loads requested ahead beside the first half step's own
+    static constexpr int spare() {
+        int n = 0;
+        for (int v = -(XB > WB * HPW ? XB : WB * HPW); v < 0; ++v) n += (v + XB > 0 ? NX : 0) + (issues_w(v) && (v + 2) / HPW - 1 + WB > 0 ? NW : 0);
+        return n;
+    }
+    // Loads that may still be out when half step h starts: those requested after the last of what it reads.
+    static constexpr int ahead(int h) {
+        int x = issues_w(h - XB) ? NW : 0;
+        for (int v = h - XB + 1; v < h; ++v) x += NX + (issues_w(v) ? NW : 0);
+        return h & (HPW - 1) || x < behind_w() ? x : behind_w();
+    }
+    // loads requested between a weight unit and its first half step
+    static constexpr int behind_w() {
+        int w = 0;
+        for (int v = HPW - 1 - WB * HPW; v < 0; ++v) w += NX + (issues_w(v) ? NW : 0);
+        return w;
+    }
+};
 
 template <int FMT, int SC, int MT, int RT>
-__global__ void __launch_bounds__(64 * kStreamWaves, MT == 4 || RT == 3 ? 2 : 4)
-stream_split_kernel(const bf16_t* x, int32_t ldx, int32_t M, int32_t K, int32_t first1, int32_t first2, int32_t first3, StreamBatch b) {
+__global__ void __launch_bounds__(64 * kStreamWaves, (StreamGeo<FMT, MT, RT>::PAIR ? 4 : 2))
+stream_split_kernel(const bf16_t* x, int64_t ldx, int32_t M, int32_t K, int32_t first1, int32_t first2, int32_t first3, StreamBatch b) {
+    using G = StreamGeo<FMT, MT, RT>;
     constexpr int EB = FMT == XQ_FMT_FP8 ? 1 : 2;                 // elements per byte
-    constexpr int NL = FMT == XQ_FMT_FP8 ? 2 : 1;                 // 16-byte loads per lane, row tile and step
-    constexpr int D = FMT == XQ_FMT_FP8 && RT > 1 ? 2 : 4;        // steps in flight
-    constexpr int NS = SC != kScStep ? 0 : FMT == XQ_FMT_NVFP4 ? 2 : 1;   // scale words per row tile that travel with a step
+    constexpr int HPW = G::HPW, XB = G::XB, WB = G::WB;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     const int tid = threadIdx.x, lane = tid & 63, q = lane >> 4, lr = lane & 15;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -86,109 +116,126 @@ stream_split_kernel(const bf16_t* x, int32_t ldx, int32_t M, int32_t K, int32_t 
     const StreamJob& g = b.job[ji];
     const int at = bx - (ji == 0 ? 0 : ji == 1 ? first1 : ji == 2 ? first2 : first3);
     const int split = at % g.splits, rb = at / g.splits;
-    const int c_begin = split * g.chunk_q + (split < g.chunk_rem ? split : g.chunk_rem);
-    const int n_steps = g.chunk_q + (split < g.chunk_rem ? 1 : 0);
+    // this wave's steps: an eighth of the split's
+    const int s_begin = split * g.chunk_q + (split < g.chunk_rem ? split : g.chunk_rem);
+    const int s_steps = g.chunk_q + (split < g.chunk_rem ? 1 : 0);
+    const int per = s_steps / kStreamWaves, rem = s_steps % kStreamWaves;
+    const int c_begin = s_begin + wave * per + (wave < rem ? wave : rem);
+    const int n_steps = per + (wave < rem ? 1 : 0);
     const int k_begin = c_begin << 7;
 
-    // ---- x slice -> LDS: [step][16 MT rows][16 pieces of 8 elements].  Piece (j, q) of row m lies at (4 j + q) ^ (m & 15): the
-    // 16 lanes that one LDS pass of a fragment read serves fall on 16 different pieces.  Lane l of a load instruction lands at
-    // piece l % 16 of row l / 16 of its four rows, so the swizzle is applied to the address it fetches.  (rows past M repeat the
-    // last one: their products are never stored)
-    {
-        const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem;
-        const int total = n_steps * MT * 4;
-        for (int i = wave; i < total; i += kStreamWaves) {
-            const int step = i / (MT * 4), m = (i % (MT * 4)) * 4 + (lane >> 4);
-            const int col = (lane & 15) ^ (m & 15);
-            const bf16_t* src = x + (int64_t)(m < M ? m : M - 1) * ldx + k_begin + step * 128 + frag_k<FMT>(col >> 2, col & 3);
-            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
-                         :: "s"(__builtin_amdgcn_readfirstlane(lds0 + i * 1024)), "v"(src) : "memory");
-        }
-    }
-    // fragment (m tile, j) of step s: row lr of the tile
-    int xo[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) xo[j] = lr * 256 + (((4 * j + q) ^ lr) << 4);
-    const auto x_frag = [&](int s, int mt, int j) {
-        return *(const bf16x8*)(smem + (s * MT + mt) * 4096 + xo[j]);
-    };
-
-    // ---- the low-rank parts: units of (step, 16 ranks) dealt over the waves of the split's blocks, the first of them over the
-    // blocks.  A wave's first unit is requested here, behind the x slice and ahead of the weights, and multiplied before the
-    // stream starts; D[rank][m] of one step goes out as it is (ranks >= r: whatever row 0 gives, never read).
-    const int rank_tiles = g.r_pad >> 4, units = n_steps * rank_tiles, unit0 = rb + g.row_blocks * wave;
-    const auto unit_base = [&](int u, int us) {
-        const int row = (u - us * rank_tiles) * 16 + lr;
-        return (int64_t)(row < g.r ? row : 0) * K + k_begin + us * 128;
-    };
-    const auto multiply_unit = [&](int u, int us, const u32x4 (&a)[4]) {
-        const int jt = u - us * rank_tiles;
-        f32x4 sacc[MT];
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) sacc[mt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt)
-                sacc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a[j]), x_frag(us, mt, j), sacc[mt], 0, 0, 0);
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-            const int m = mt * 16 + lr;
-            if (m < M) *(f32x4*)(g.su_part + ((int64_t)(c_begin + us) * M + m) * g.r_pad + jt * 16 + q * 4) = sacc[mt];
-        }
-    };
-    f32x4 araw[8];                                                 // fp32 factors (bf16 ones are not requested ahead)
-    const auto load_unit = [&](int u) {
-        const float* p = (const float*)g.lora_A + unit_base(u, u / rank_tiles);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            araw[2 * j] = *(const f32x4*)(p + frag_k<FMT>(j, q));
-            araw[2 * j + 1] = *(const f32x4*)(p + frag_k<FMT>(j, q) + 4);
-        }
-    };
-    if (g.lora_f32 && unit0 < units) load_unit(unit0);
-
-    // ---- this wave's rows: tiles of 16 (N % 16 == 0: a tile is all in or all out; one past the end repeats the last)
-    const int row0 = (rb * kStreamWaves + wave) * (16 * RT);
-    const uint8_t* wp[RT];
-    int64_t srow[RT];                                              // SC-dependent: the row's scales
-#pragma unroll
-    for (int rt = 0; rt < RT; ++rt) {
-        const int n = (row0 + rt * 16 < g.N ? row0 + rt * 16 : g.N - 16) + lr;
-        wp[rt] = g.packed + ((int64_t)n * K + k_begin) / EB + q * 16;
-        srow[rt] = (int64_t)n * K + k_begin;
-    }
-    u32x4 w[D][RT][NL];
-    uint32_t sw[D][RT][NS > 0 ? NS : 1];
-    const auto load_step = [&](int slot, int s_) {
-        const int s = s_ < n_steps ? s_ : n_steps - 1;
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt) {
-#pragma unroll
-            for (int i = 0; i < NL; ++i) w[slot][rt][i] = *(const u32x4*)(wp[rt] + (int64_t)s * (128 / EB) + i * 64);
-            if constexpr (SC == kScStep && FMT == XQ_FMT_NVFP4) {
-                const u32x2 v = *(const u32x2_a1*)((const uint32_t*)g.scales + ((srow[rt] + s * 128 + q * 32) >> 4));
-                sw[slot][rt][0] = v[0];
-                sw[slot][rt][1] = v[1];
-            } else if constexpr (SC == kScStep) {
-                const int64_t si = (srow[rt] + s * 128 + q * 32) / g.group;
-                sw[slot][rt][0] = g.scale_dtype == XQ_SCALE_F32 ? ((const uint32_t*)g.scales)[si] : (uint32_t)((const uint16_t*)g.scales)[si] << 16;
+    // ---- the low-rank parts x . A^T: units of (step, 16 ranks), dealt over the split's blocks so that a block has one for one of its
+    // waves at most unless the weight is narrow.  A's operand of a wave's first unit is requested with the first loads and waits in
+    // registers as bf16; the product is made of the x fragments that the stream reads anyway and goes out step by step (ranks >= r:
+    // whatever row 0 gives, never read).
+    const int rank_tiles = g.r_pad >> 4;
+    int su_unit = rb, su_step = 1 << 30, su_tile = 0;
+    const auto next_unit = [&]() {                                 // this wave's next one of units rb, rb + row_blocks, ...
+        const int before = c_begin - s_begin;
+        su_step = 1 << 30;
+        for (; rank_tiles && su_unit < (before + n_steps) * rank_tiles; su_unit += g.row_blocks) {
+            const int step = su_unit / rank_tiles - before;
+            if (step >= 0) {
+                su_step = step;
+                su_tile = su_unit - (step + before) * rank_tiles;
+                su_unit += g.row_blocks;
+                break;
             }
         }
     };
-    // windows of four steps (a window that would pass the row's end starts earlier; kScDealt clamps step by step)
-    u32x2 win[RT], win_next[RT];
+    u32x4 a[4];
+    const auto load_a = [&]() {
+        const int row = su_tile * 16 + lr;
+        const int64_t base = (int64_t)(row < g.r ? row : 0) * K + k_begin + su_step * 128 + q * 16;
+        if (g.lora_f32) {
+            const float* p = (const float*)g.lora_A + base;
+            f32x4 raw[8];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                raw[2 * j] = *(const f32x4*)(p + (j >> 1) * 64 + (j & 1) * 8);
+                raw[2 * j + 1] = *(const f32x4*)(p + (j >> 1) * 64 + (j & 1) * 8 + 4);
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                a[j] = u32x4{pack_bf16x2(raw[2 * j][0], raw[2 * j][1]), pack_bf16x2(raw[2 * j][2], raw[2 * j][3]),
+                             pack_bf16x2(raw[2 * j + 1][0], raw[2 * j + 1][1]), pack_bf16x2(raw[2 * j + 1][2], raw[2 * j + 1][3])};
+        } else {
+            const bf16_t* p = (const bf16_t*)g.lora_A + base;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) a[j] = *(const u32x4*)(p + (j >> 1) * 64 + (j & 1) * 8);
+        }
+    };
+
+    // ---- this wave's LDS and what comes into it.  x: half step of [16 MT rows][8 pieces of 8 elements], piece p of row m at p ^ ((m >> 1)
+    // & 5); weights: [16 RT rows][8 pieces of 16 bytes], piece p of row n at p ^ (n >> 1 & 7).  Lane l of a load lands at piece l of its
+    // KB, so the swizzle is applied to the address that it fetches; eight neighbouring lanes take 128 bytes of a row, which a load in
+    // the fragments' order does not: that one takes 56 clocks of the address unit, this one 16.  (Weights 64 bytes at a time, as
+    // 16 rows of a load, read 100 MB in 24.8 us where this takes 18.4.)
+    const int row0 = rb * (16 * RT) < g.N ? rb * (16 * RT) : g.N - 16;   // tiles of 16 (N % 16 == 0: a tile is all in or all out; one past the end repeats the last)
+    const uint32_t xl = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem + wave * G::WAVE, wl = xl + XB * G::XH;
+    const unsigned char* xs = smem + wave * G::WAVE;
+    const unsigned char* wsm = xs + XB * G::XH;
+    // rows of x in groups of eight: (rows past M repeat the last one: their products are never stored)
+    const int tail = (M - 1) & ~7, xr = lane >> 3;
+    const uint32_t x_full = (uint32_t)((int64_t)xr * ldx * 2), x_tail = (uint32_t)((int64_t)(tail + xr < M ? xr : M - 1 - tail) * ldx * 2);
+    const uint32_t xc0 = ((lane & 7) ^ ((lane >> 4) & 1)) << 4, xc1 = xc0 ^ 64;
+    const int halves = 2 * n_steps;
+    const auto issue_x1 = [&](int h_, int x_slot, int i) {
+        const int h = h_ < halves ? h_ : halves - 1;
+        const bool whole = i * 8 + 8 <= M;
+        const bf16_t* base = x + (int64_t)(whole ? i * 8 : tail) * ldx + k_begin + h * 64;
+        const uint32_t off = (whole ? x_full : x_tail) + (i & 1 ? xc1 : xc0);
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                     :: "s"(__builtin_amdgcn_readfirstlane(xl + x_slot * G::XH + i * 1024)), "v"(off), "s"(base) : "memory");
+    };
+    uint32_t w_off[RT];
+    {
+        const int n = lane >> 3, piece = (lane & 7) ^ (lane >> 4);    // rows n and n + 8 of a tile: the swizzle's bit 2 is the row's bit 3
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) w_off[rt] = (uint32_t)((int64_t)((row0 + rt * 16 < g.N ? rt * 16 : g.N - 16 - row0) + n) * (K / EB) + piece * 16);
+    }
+    const uint32_t w_flip = ((lane & 7) ^ (lane >> 4)) & 4 ? (uint32_t)-64 : 64u, w_rows8 = (uint32_t)(8 * (K / EB)) + w_flip;
+    const uint8_t* w_base = g.packed + ((int64_t)row0 * K + k_begin) / EB;
+    const int w_bytes = n_steps * (128 / EB), units = (w_bytes + 127) >> 7;
+    const auto issue_w1 = [&](int u_, int slot, int i) {
+        const int u = u_ < units ? u_ : units - 1;
+        const uint8_t* base = w_base + (int64_t)u * 128;
+        uint32_t off = w_off[i >> 1] + (i & 1 ? w_rows8 : 0);
+        // (an odd step at the end of a 4-bit range: the unit's second half is fetched from the first)
+        if (EB == 2 && u * 128 + 128 > w_bytes) off -= ((lane & 7) ^ (lane >> 4) ^ (i & 1 ? 4 : 0)) & 4 ? 64 : 0;
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                     :: "s"(__builtin_amdgcn_readfirstlane(wl + slot * G::WU + i * 1024)), "v"(off), "s"(base) : "memory");
+    };
+
+    // ---- scales
+    int64_t srow[RT];                                              // element of the lane's row that its steps start at
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) srow[rt] = (int64_t)((row0 + rt * 16 < g.N ? row0 + rt * 16 : g.N - 16) + lr) * K;
+    u32x2 win[RT], win_next[RT];                                   // windows of four steps (one that would pass the row's end starts earlier; kScDealt clamps step by step)
     const int row_steps = K >> 7;
     const auto load_window = [&](u32x2* dst, int s0) {
         if constexpr (SC == kScInt4Window) {
             const int c = c_begin + s0 < row_steps - 4 ? c_begin + s0 : row_steps - 4;
 #pragma unroll
-            for (int rt = 0; rt < RT; ++rt)
-                dst[rt] = *(const u32x2_a1*)((const uint16_t*)g.scales + ((srow[rt] - k_begin) >> 7) + c);
+            for (int rt = 0; rt < RT; ++rt) dst[rt] = *(const u32x2_a1*)((const uint16_t*)g.scales + (srow[rt] >> 7) + c);
         } else if constexpr (SC == kScDealt) {
             const int c = c_begin + s0 + q < row_steps - 1 ? c_begin + s0 + q : row_steps - 1;
 #pragma unroll
-            for (int rt = 0; rt < RT; ++rt) dst[rt] = *(const u32x2_a1*)(g.scales + ((srow[rt] - k_begin) >> 7) * 8 + (int64_t)c * 8);
+            for (int rt = 0; rt < RT; ++rt) dst[rt] = *(const u32x2_a1*)(g.scales + ((srow[rt] >> 7) + c) * 8);
+        }
+    };
+    constexpr int SW = SC == kScUse ? 2 : 1;                       // scale words of a lane's 16 elements of a half step
+    uint32_t sw[SC >= kScHalf ? RT : 1][SW], sw_next[SC >= kScHalf ? RT : 1][SW];
+    const auto load_half = [&](int h_) {
+        if constexpr (SC >= kScHalf) {
+            const int h = h_ < halves ? h_ : halves - 1;
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+                for (int i = 0; i < SW; ++i) {
+                    const int64_t si = (srow[rt] + k_begin + h * 64 + q * 16 + i * 8) / g.group;
+                    sw_next[rt][i] = g.scale_dtype == XQ_SCALE_F32 ? ((const uint32_t*)g.scales)[si] : (uint32_t)((const uint16_t*)g.scales)[si] << 16;
+                }
         }
     };
     float ts[RT];                                                  // block-fp8: lane l holds the scale of step l
@@ -196,40 +243,15 @@ stream_split_kernel(const bf16_t* x, int32_t ldx, int32_t M, int32_t K, int32_t 
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
             const int n = row0 + rt * 16 < g.N ? row0 + rt * 16 : g.N - 16;
-            ts[rt] = ((const float*)g.scales)[(int64_t)(n >> 7) * ((K + 127) >> 7) + c_begin + (lane < n_steps ? lane : n_steps - 1)];
+            const int c = c_begin + (lane < n_steps ? lane : n_steps - 1);
+            ts[rt] = ((const float*)g.scales)[(int64_t)(n >> 7) * row_steps + (c > 0 ? c : 0)];
         }
     }
-    load_window(win, 0);
-#pragma unroll
-    for (int d = 0; d < D; ++d) load_step(d, d);
     const float gsc = FMT == XQ_FMT_NVFP4 ? g.global_scale[0] : 1.0f;
-    float* nf4_lds = (float*)(smem + n_steps * MT * 4096);
-    if (FMT == XQ_FMT_NF4 && tid < 16) nf4_lds[tid] = kNf4Level[tid];
-
-    // the x slice is older than every load above: it has landed when no more than those are outstanding
-    constexpr int kAhead = D * RT * (NL + (NS ? 1 : 0));
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kAhead < 63 ? kAhead : 63) : "memory");
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    if (g.lora_f32) {
-#pragma unroll 1
-        for (int u = unit0; u < units; u += g.row_blocks * kStreamWaves) {      // (more than one only for narrow weights of high rank)
-            if (u != unit0) load_unit(u);
-            u32x4 a[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                a[j] = u32x4{pack_bf16x2(araw[2 * j][0], araw[2 * j][1]), pack_bf16x2(araw[2 * j][2], araw[2 * j][3]),
-                             pack_bf16x2(araw[2 * j + 1][0], araw[2 * j + 1][1]), pack_bf16x2(araw[2 * j + 1][2], araw[2 * j + 1][3])};
-            multiply_unit(u, u / rank_tiles, a);
-        }
-    } else {
-#pragma unroll 1
-        for (int u = unit0; u < units; u += g.row_blocks * kStreamWaves) {
-            const bf16_t* p = (const bf16_t*)g.lora_A + unit_base(u, u / rank_tiles);
-            u32x4 a[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) a[j] = *(const u32x4*)(p + frag_k<FMT>(j, q));
-            multiply_unit(u, u / rank_tiles, a);
-        }
+    const float* nf4_lds = (const float*)(smem + kStreamWaves * G::WAVE);
+    if (FMT == XQ_FMT_NF4) {
+        if (tid < 16) ((float*)(smem + kStreamWaves * G::WAVE))[tid] = kNf4Level[tid];
+        __syncthreads();
     }
 
     f32x4 acc[RT][MT];
@@ -237,117 +259,220 @@ stream_split_kernel(const bf16_t* x, int32_t ldx, int32_t M, int32_t K, int32_t 
     for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) acc[rt][mt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    uint32_t sx[SC == kScDealt ? RT : 1][4];
-    // register k of lane row r <- what lane row k fetched for lane row r
-    const auto deal = [&]() {
-        if constexpr (SC == kScDealt) {
+
+    f32x4 su[MT];
 #pragma unroll
-            for (int rt = 0; rt < RT; ++rt) {
-                const u32x2 d = win[rt];
-                const uint32_t x0 = d[0], x1 = FMT == XQ_FMT_NF4 ? d[0] : d[0] >> 16, x2 = d[1], x3 = FMT == XQ_FMT_NF4 ? d[1] : d[1] >> 16;
-                const auto p02 = __builtin_amdgcn_permlane32_swap(x0, x2, false, false);
-                const auto p13 = __builtin_amdgcn_permlane32_swap(x1, x3, false, false);
-                const auto q01 = __builtin_amdgcn_permlane16_swap(p02[0], p13[0], false, false);
-                const auto q23 = __builtin_amdgcn_permlane16_swap(p02[1], p13[1], false, false);
-                sx[rt][0] = q01[0]; sx[rt][1] = q01[1]; sx[rt][2] = q23[0]; sx[rt][3] = q23[1];
-            }
+    for (int mt = 0; mt < MT; ++mt) su[mt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+
+    // ---- the stream.  Nothing in it is shared between waves: a wave waits for its own loads by count.
+    if (n_steps > 0) {
+        load_window(win, 0);
+        load_half(0);
+        // First what the first products need -- the scales, x, half of the row tiles -- and a wait for it; then the others' weights, for
+        // which the first half step waits when it comes to them, and the rest as if half steps before the first had asked for it.
+        constexpr int P = XB > WB * HPW ? XB : WB * HPW;
+#pragma unroll
+        for (int i = 0; i < G::NX; ++i) issue_x1(0, 0, i);
+#pragma unroll
+        for (int i = 0; i < 2 * G::EARLY; ++i) issue_w1(0, 0, i);
+        next_unit();
+        if (su_step < n_steps) load_a();
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {                          // (what the compiler waits for it waits for here)
+            if constexpr (SC == kScFp8) asm volatile("" : "+v"(ts[rt]));
+            else if constexpr (SC < kScHalf) asm volatile("" : "+v"(win[rt]));
+            else asm volatile("" : "+v"(sw_next[rt][0]), "+v"(sw_next[rt][SW - 1]));
         }
-    };
-    const auto multiply = [&](int slot, int s, int ph) {              // ph: the step's place in its window
-        float s0[RT], s1[RT];
 #pragma unroll
-        for (int rt = 0; rt < RT; ++rt) {
-            s1[rt] = 0.0f;
-            if constexpr (SC == kScFp8) {
-                s0[rt] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ts[rt]), s));
-            } else if constexpr (SC == kScInt4Window) {
-                const int c = c_begin + s - ph;
-                const int i = ph + (c < row_steps - 4 ? 0 : c - (row_steps - 4));          // uniform, 0 .. 3
-                const uint64_t v = (uint64_t)win[rt][1] << 32 | win[rt][0];
-                s0[rt] = __uint_as_float((uint32_t)(v >> (16 * i)) << 16);
-                s1[rt] = -8.0f * s0[rt];
-            } else if constexpr (SC == kScDealt && FMT == XQ_FMT_NF4) {
-                s0[rt] = __uint_as_float(sx[rt][ph]);
-            } else if constexpr (SC == kScDealt) {
-                s0[rt] = e4m3_to_f32((uint8_t)sx[rt][ph]) * gsc;
-                s1[rt] = e4m3_to_f32((uint8_t)(sx[rt][ph] >> 8)) * gsc;
-            } else if constexpr (SC == kScStep && FMT == XQ_FMT_NVFP4) {
-                s0[rt] = __uint_as_float(sw[slot][rt][0]) * gsc;
-                s1[rt] = __uint_as_float(sw[slot][rt][NS > 1 ? 1 : 0]) * gsc;
-            } else if constexpr (SC == kScStep) {
-                s0[rt] = __uint_as_float(sw[slot][rt][0]);
-                s1[rt] = -8.0f * s0[rt];
-            }
+        for (int i = 2 * G::EARLY; i < G::NW; ++i) issue_w1(0, 0, i);
+#pragma unroll
+        for (int v = -P; v < 0; ++v) {
+            if (v + XB > 0)
+#pragma unroll
+                for (int i = 0; i < G::NX; ++i) issue_x1(v + XB, (v + XB) % XB, i);
+            if (G::issues_w(v) && (v + 2) / HPW - 1 + WB > 0)
+#pragma unroll
+                for (int i = 0; i < G::NW; ++i) issue_w1((v + 2) / HPW - 1 + WB, ((v + 2) / HPW - 1 + WB) % WB, i);
         }
-        bf16x8 xf[2][MT];                                          // fragments are read one j ahead
+        const int x_lane = lr * 128, x_sw = (lr >> 1) & 5;
+        int w_slot = 0, x_slot = 0, unit = 0;
+        u32x4 w[RT][FMT == XQ_FMT_FP8 ? 2 : 1];
+        const auto half_step = [&](auto hh_, auto odd_, int s, int ph) {
+            constexpr int hh = decltype(hh_)::value, odd = decltype(odd_)::value;       // odd: the step's place in its unit
+            constexpr bool LATE = hh == 0 && odd == 0 && G::EARLY < RT;                  // the later row tiles' weights are waited for on the way
+            const int h = 2 * s + hh;
+            constexpr int N = G::ahead(64 + 2 * odd + hh);
+            if (hh || odd || s) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N < 63 ? N : 63) : "memory");
+            bf16x8 xf[2][MT];
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) xf[0][mt] = x_frag(s, mt, 0);
+            for (int jj = 0; jj < 2; ++jj)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            if (j < 3) {
-#pragma unroll
-                for (int mt = 0; mt < MT; ++mt) xf[(j + 1) & 1][mt] = x_frag(s, mt, j + 1);
-            }
-#pragma unroll
-            for (int rt = 0; rt < RT; ++rt) {
-                bf16x8 wf;
+                for (int mt = 0; mt < MT; ++mt)
+                    xf[jj][mt] = *(const bf16x8*)(xs + x_slot * G::XH + mt * 2048 + x_lane + (((2 * q + jj) ^ x_sw) << 4));
+            // the step's weights: block-fp8 piece 4 hh + q of a row (both half steps at once: the unit's slot is then free); 4-bit
+            // piece 4 (step in the unit) + 2 hh + q / 2
+            const auto read_w = [&](int rt) {
+                const unsigned char* p = wsm + w_slot * G::WU + lr * 128 + rt * 2048;
                 if constexpr (FMT == XQ_FMT_FP8) {
-                    const u32x4 v = w[slot][rt][j >> 1];
-                    wf = decode8<FMT>(v[2 * (j & 1)], v[2 * (j & 1) + 1], s0[rt], 0.0f);
-                } else if constexpr (FMT == XQ_FMT_NVFP4) {
-                    wf = decode8<FMT>(w[slot][rt][0][j], 0u, j < 2 ? s0[rt] : s1[rt], 0.0f);
-                } else if constexpr (SC == kScUse) {
-                    const float sv = load_scale(g.scales, (srow[rt] + s * 128 + q * 32 + j * 8) / g.group, g.scale_dtype);
-                    wf = decode8<FMT>(w[slot][rt][0][j], 0u, sv, -8.0f * sv);
+                    w[rt][0] = *(const u32x4*)(p + ((q ^ (lr >> 1)) << 4));
+                    w[rt][1] = *(const u32x4*)(p + (((4 + q) ^ (lr >> 1)) << 4));
                 } else {
-                    wf = decode8<FMT>(w[slot][rt][0][j], 0u, s0[rt], s1[rt], nf4_lds);
+                    const int c = 4 * odd + (q >> 1);
+                    const u32x2 lo = *(const u32x2*)(p + ((c ^ (lr >> 1)) << 4) + (q & 1) * 8);
+                    const u32x2 hi = *(const u32x2*)(p + (((c + 2) ^ (lr >> 1)) << 4) + (q & 1) * 8);
+                    w[rt][0] = u32x4{lo[0], lo[1], hi[0], hi[1]};
+                }
+            };
+            if constexpr (hh == 0) {
+#pragma unroll
+                for (int rt = 0; rt < (LATE ? G::EARLY : RT); ++rt) read_w(rt);
+            }
+            float s0[RT], s1[RT];
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) {
+                s1[rt] = 0.0f;
+                if constexpr (SC == kScFp8) {
+                    s0[rt] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ts[rt]), s));
+                } else if constexpr (SC == kScInt4Window) {
+                    const int c = c_begin + s - ph;
+                    const int i = ph + (c < row_steps - 4 ? 0 : c - (row_steps - 4));          // uniform, 0 .. 3
+                    const uint64_t v = (uint64_t)win[rt][1] << 32 | win[rt][0];
+                    s0[rt] = __uint_as_float((uint32_t)(v >> (16 * i)) << 16);
+                    s1[rt] = -8.0f * s0[rt];
+                } else if constexpr (SC == kScDealt) {
+                    const uint32_t v = (uint32_t)__builtin_amdgcn_ds_bpermute((ph * 16 + lr) * 4, (int)win[rt][hh]);
+                    s0[rt] = FMT == XQ_FMT_NF4 ? __uint_as_float(v) : e4m3_to_f32((uint8_t)(v >> (8 * q))) * gsc;
+                } else {
+#pragma unroll
+                    for (int i = 0; i < SW; ++i) sw[rt][i] = sw_next[rt][i];
+                    s0[rt] = __uint_as_float(sw[rt][0]) * (FMT == XQ_FMT_NVFP4 ? gsc : 1.0f);
+                    s1[rt] = -8.0f * s0[rt];
+                }
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            load_half(h + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            // the requests go out between the products, a few at a time: all at once they hold the wave up
+            constexpr bool W = G::issues_w(2 * odd + hh);
+            constexpr int LOADS = G::NX + (W ? G::NW : 0), SPREAD = (LOADS + 2 * RT - 1) / (2 * RT), EACH = SPREAD < 2 ? 2 : SPREAD;
+            // (no weight is asked for before the late tiles have left the slot)
+            constexpr int LX = (G::NX + 2 * G::EARLY - 1) / (2 * G::EARLY), SLOTS = 2 * (LATE ? RT - G::EARLY : RT), LW = (G::NW + SLOTS - 1) / SLOTS;
+            const auto request = [&](int at) {                     // behind the at-th of the half step's 2 RT products
+                if constexpr (LATE) {
+#pragma unroll
+                    for (int i = at * LX; i < (at + 1) * LX && i < G::NX; ++i) issue_x1(h + XB, x_slot, i);
+                    if constexpr (W)
+#pragma unroll
+                        for (int i = (at - 2 * G::EARLY) * LW; i < (at - 2 * G::EARLY + 1) * LW && i < G::NW; ++i)
+                            if (i >= 0) issue_w1(unit + WB, w_slot, i);
+                } else {
+#pragma unroll
+                    for (int i = at * EACH; i < (at + 1) * EACH && i < LOADS; ++i) {
+                        if (i < G::NX) issue_x1(h + XB, x_slot, i);
+                        else issue_w1(unit + WB, w_slot, i - G::NX);
+                    }
+                }
+            };
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) {
+                if constexpr (LATE) {
+                    if (rt == G::EARLY) {
+                        constexpr int OUT = G::NX + (G::spare() < G::behind_w() ? G::spare() : G::behind_w());
+                        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(OUT < 63 ? OUT : 63) : "memory");
+#pragma unroll
+                        for (int t = G::EARLY; t < RT; ++t) read_w(t);
+                        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                    }
                 }
 #pragma unroll
-                for (int mt = 0; mt < MT; ++mt) acc[rt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf, xf[j & 1][mt], acc[rt][mt], 0, 0, 0);
+                for (int jj = 0; jj < 2; ++jj) {
+                    bf16x8 wf;
+                    if constexpr (FMT == XQ_FMT_FP8) {
+                        wf = decode8<FMT>(w[rt][hh][2 * jj], w[rt][hh][2 * jj + 1], s0[rt], 0.0f);
+                    } else if constexpr (SC == kScUse) {
+                        const float sv = __uint_as_float(sw[rt][jj]);
+                        wf = decode8<FMT>(w[rt][0][2 * hh + jj], 0u, sv, -8.0f * sv);
+                    } else {
+                        wf = decode8<FMT>(w[rt][0][2 * hh + jj], 0u, s0[rt], s1[rt], nf4_lds);
+                    }
+#pragma unroll
+                    for (int mt = 0; mt < MT; ++mt) acc[rt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf, xf[jj][mt], acc[rt][mt], 0, 0, 0);
+                    request(2 * rt + jj);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            x_slot = x_slot + 1 == XB ? 0 : x_slot + 1;
+            if constexpr (W) {
+                ++unit;
+                w_slot = w_slot + 1 == WB ? 0 : w_slot + 1;
+            }
+            if (s == su_step) {
+#pragma unroll
+                for (int jj = 0; jj < 2; ++jj)
+#pragma unroll
+                    for (int mt = 0; mt < MT; ++mt)
+                        su[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a[2 * hh + jj]), xf[jj][mt], su[mt], 0, 0, 0);
+                if (hh == 1) {
+#pragma unroll
+                    for (int mt = 0; mt < MT; ++mt) {
+                        const int m = mt * 16 + lr;
+                        if (m < M) *(f32x4*)(g.su_part + ((int64_t)(c_begin + s) * M + m) * g.r_pad + su_tile * 16 + q * 4) = su[mt];
+                        su[mt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                    }
+                    next_unit();
+                    if (su_step < n_steps) load_a();
+                }
+            }
+        };
+        using H0 = std::integral_constant<int, 0>;
+        using H1 = std::integral_constant<int, 1>;
+#pragma unroll 1
+        for (int s0 = 0; s0 < n_steps; s0 += 4) {
+            const int end = s0 + 4 < n_steps ? s0 + 4 : n_steps;
+            if (RT <= 4 && end < n_steps) load_window(win_next, end);
+#pragma unroll 1
+            for (int s = s0; s < end; ++s) {
+                half_step(H0{}, H0{}, s, s - s0);
+                half_step(H1{}, H0{}, s, s - s0);
+                if constexpr (HPW == 4) {
+                    if (++s >= end) break;
+                    half_step(H0{}, H1{}, s, s - s0);
+                    half_step(H1{}, H1{}, s, s - s0);
+                }
+            }
+            if constexpr (RT <= 4) {
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt) win[rt] = win_next[rt];
+            } else {
+                if (end < n_steps) load_window(win, end);          // (no registers for two windows)
             }
         }
-    };
-
-    // ---- the stream: whole groups of four steps, each step's registers requested again once it has been multiplied, then the
-    // remaining steps from what is in flight.  No branch lies between a load and its use, so every wait counts exactly.
-    int s = 0;
-#pragma unroll 1
-    for (; s + 4 <= n_steps; s += 4) {
-        deal();
-        load_window(win_next, s + 4);
-#pragma unroll
-        for (int d = 0; d < 4; ++d) {
-            multiply(d % D, s + d, d);
-            // (left alone the compiler decodes ahead, collects the products at the end and requests late)
-#pragma unroll
-            for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-                for (int mt = 0; mt < MT; ++mt) asm volatile("" : "+v"(acc[rt][mt]));
-            load_step(d % D, s + d + D);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        if constexpr (SC == kScInt4Window || SC == kScDealt) {
-#pragma unroll
-            for (int rt = 0; rt < RT; ++rt) win[rt] = win_next[rt];
-        }
-    }
-    if (s < n_steps) {
-        deal();
-        multiply(0, s, 0);
-        if constexpr (D == 2) load_step(0, s + 2);
-        if (s + 1 < n_steps) multiply(1, s + 1, 1);
-        if (s + 2 < n_steps) multiply(2 % D, s + 2, 2);
     }
 
-    // ---- fp32 partial tile: lane (m = lr, quarter q) holds 4 consecutive weight rows of each row tile
+    // ---- the eight waves' sums meet in LDS, GT row tiles at a time, and are added in wave order.  Lane (m = lr, quarter q) holds 4
+    // consecutive weight rows of each row tile.
+    constexpr int GT0 = G::WAVE / (MT * 1024), GT = GT0 < RT ? GT0 : RT;
+    static_assert(GT >= 1, "the reduction needs room for a row tile");
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    f32x4* red = (f32x4*)smem;
 #pragma unroll
-    for (int rt = 0; rt < RT; ++rt) {
-        const int n = row0 + rt * 16;
-        if (n < g.N) {
+    for (int t0 = 0; t0 < RT; t0 += GT) {
+        __syncthreads();
 #pragma unroll
-            for (int mt = 0; mt < MT; ++mt) {
-                const int m = mt * 16 + lr;
-                if (m < M) *(f32x4*)(g.partial + ((int64_t)split * M + m) * g.N + n + q * 4) = acc[rt][mt];
+        for (int t = 0; t < GT; ++t)
+            if (t0 + t < RT) {
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt) red[((wave * GT + t) * MT + mt) * 64 + lane] = acc[t0 + t][mt];
+            }
+        __syncthreads();
+        for (int i = wave; i < GT * MT; i += kStreamWaves) {
+            const int t = i / MT, mt = i - t * MT, m = mt * 16 + lr, n = row0 + (t0 + t) * 16;
+            if (t0 + t < RT && n < g.N && rb * (16 * RT) < g.N) {   // uniform
+                f32x4 v = red[i * 64 + lane];
+#pragma unroll
+                for (int w8 = 1; w8 < kStreamWaves; ++w8) v += red[(w8 * GT * MT + i) * 64 + lane];
+                if (m < M) *(f32x4*)(g.partial + ((int64_t)split * M + m) * g.N + n + q * 4) = v;
             }
         }
     }
@@ -558,48 +683,50 @@ stream_epilogue_kernel(int32_t M, int32_t first1, int32_t first2, int32_t first3
 
 static inline int64_t al256(int64_t b) { return (b + 255) & ~(int64_t)255; }
 
-// What a launch of `blocks` blocks of 8 waves with RT row tiles and `steps` steps takes, in us, from a sweep of M 1..64 and widths
-// 1024..16384: a start of ~4 us (launch, the x slice, the first weights), then the decode and the products of a SIMD's
-// (row tile, step) units, which two waves to a SIMD overlap worse than four.  Two blocks are resident per CU at M <= 32, where
-// their x slices fit.
+// What a launch of `blocks` blocks of RT row tiles and `steps` steps takes beyond a constant, in us, from a sweep of every (row tiles,
+// splits) at M 24..64 on seven widths and depths of int4 and block-fp8 (within 10 % of the times; the pair it picks is 1.2 % behind
+// the best on average, 8 % at worst): rounds of the chip, and in a block the half steps of a wave, each for its weights and its x.  Two
+// blocks are resident per compute unit where StreamGeo says so.
 static double stream_run_us(int64_t blocks, int rt, int steps, int mt) {
-    const int per_cu = mt == 4 || rt == 3 || steps * mt * 4096 > 78 * 1024 ? 1 : 2;
+    const int per_cu = mt < 4 && mt * rt <= 4 ? 2 : 1;
     const int64_t cus = num_cus();
-    const double rounds = (double)xq_cdiv(blocks, cus * per_cu);
+    const double rounds = (double)xq_cdiv(blocks, cus * per_cu), halves = 2.0 * xq_cdiv(steps, kStreamWaves);
     const double on_cu = (double)xq_cdiv(blocks, cus) < rounds * per_cu ? (double)xq_cdiv(blocks, cus) : rounds * per_cu;
-    const double unit = on_cu > 1 && per_cu == 2 ? 0.12 + 0.04 * mt : 0.2 + 0.07 * mt;
-    return 4.0 * rounds + on_cu * 2 * rt * steps * unit;
+    return rounds * (0.5 + halves * (0.25 * rt + 0.17 * mt) * (1.0 + 0.8 * (on_cu / rounds - 1.0)));
 }
-// row tiles of a wave by that estimate (they change nothing in the results); `tiles`, `splits` of each forward of the launch
+static const int kRowTiles[] = {1, 2, 3, 4, 6};
+// row tiles of a block by that estimate (they change nothing in the results); `tiles`, `splits` of each forward of the launch
 static int stream_row_tiles(const int* tiles, const int* splits, int n, int steps, int mt, int rt_max, double* us) {
     int best = 1;
     double cost = 0;
-    for (int rt = 1; rt <= rt_max; ++rt) {
+    for (int rt : kRowTiles) {
+        if (rt > rt_max) break;
         int64_t blocks = 0;
-        for (int i = 0; i < n; ++i) blocks += xq_cdiv(tiles[i], (int64_t)kStreamWaves * rt) * splits[i];
+        for (int i = 0; i < n; ++i) blocks += xq_cdiv(tiles[i], (int64_t)rt) * splits[i];
         const double c = stream_run_us(blocks, rt, steps, mt);
         if (cost == 0 || c < cost) { cost = c; best = rt; }
     }
     if (us) *us = cost;
     return best;
 }
-// steps of a split at most (128 KB of x slice)
-static int stream_steps_max(int64_t M) { return M <= 16 ? 32 : M <= 32 ? 16 : 8; }
-// K splits of a forward, by its own shape: the cheapest sum of that and of the partial sums' trip (written and read back, ~6
-// TB/s)
+// steps of a split at most (a lane holds one block-fp8 scale of a wave's steps)
+constexpr int kStreamSteps = 64 * kStreamWaves;
+// K splits of a forward, by its own shape: the cheapest sum of that and of the partial sums' trip (written and read back, with what
+// waits for them: 1.7 TB/s)
 static int make_stream_splits(int64_t M, int64_t N, int64_t K) {
     const int ct = (int)(K >> 7), tiles = (int)(N / 16);
-    const int mt = M <= 16 ? 1 : M <= 32 ? 2 : 4;
+    const int mt = (int)xq_cdiv(M, 16);
+    const int least = (int)xq_cdiv(ct, kStreamSteps);
     int best = 0, last_steps = 0;
     double best_cost = 0;
-    // (a contraction so long that its x slices need more than 64 splits takes the fewest that hold them)
-    for (int s = (int)xq_cdiv(ct, stream_steps_max(M)); s <= ct && (s <= 64 || best == 0); ++s) {
+    for (int s = least; s <= ct && (s <= 64 || best == 0); ++s) {
         const int steps = (int)xq_cdiv(ct, s);
         if (steps == last_steps) continue;                         // more splits, none of them shorter
         last_steps = steps;
+        if (best && (s * M * N * 4 > (16ll << 20))) break;
         double c;
-        stream_row_tiles(&tiles, &s, 1, steps, mt, 3, &c);
-        c += (double)s * M * N * 8.0 / 6.0e6;
+        stream_row_tiles(&tiles, &s, 1, steps, mt, 6, &c);
+        c += (double)s * M * N * 8.0 / 1.7e6;
         if (best == 0 || c < best_cost) { best = s; best_cost = c; }
     }
     return best;
@@ -621,8 +748,9 @@ bool skinny_takes_stream(const xq_weight* w, int64_t M, const void* lora_A, cons
 int64_t skinny_workspace_bytes(int64_t M, int64_t N, int64_t K, int r_pad) {
     if (K < 128 || N < 16) return 256;
     const int rp = r_pad ? r_pad : 16;
-    const int s = stream_splits(M, N, K);
-    return al256((int64_t)s * M * N * 4) + al256((K >> 7) * M * rp * 4) + 256;
+    // (never less than a partial sum for every 32, 16 or 8 steps, whatever the plan: what callers have always been asked for)
+    const int64_t s = stream_splits(M, N, K), held = xq_cdiv(K >> 7, M <= 16 ? 32 : M <= 32 ? 16 : 8);
+    return al256((s > held ? s : held) * M * N * 4) + al256((K >> 7) * M * rp * 4) + 256;
 }
 
 bool skinny_supported(const xq_weight* w, int64_t M) {
@@ -638,17 +766,18 @@ bool skinny_supported(const xq_weight* w, int64_t M) {
 static int scale_mode(const xq_weight* w) {
     if (w->format == XQ_FMT_FP8) return kScFp8;
     if (w->format == XQ_FMT_NF4) return kScDealt;
-    if (w->format == XQ_FMT_NVFP4) return w->scale_dtype == XQ_SCALE_E4M3 ? kScDealt : kScStep;
+    if (w->format == XQ_FMT_NVFP4) return w->scale_dtype == XQ_SCALE_E4M3 ? kScDealt : kScHalf;
     if (w->group == 128 && w->scale_dtype == XQ_SCALE_BF16) return kScInt4Window;
-    return w->group % 32 == 0 && w->cols % w->group == 0 ? kScStep : kScUse;
+    return w->group % 16 == 0 && w->cols % w->group == 0 ? kScHalf : kScUse;
 }
 
 // (the uncommon scale storages keep more registers per row tile)
-template <int SC>
-constexpr int kRowTilesMax = SC == kScUse ? 1 : SC == kScStep ? 2 : 3;
+constexpr int row_tiles_max(int fmt, int sc) { return sc >= kScHalf ? 2 : fmt == XQ_FMT_NF4 ? 4 : 6; }
 
 template <int FMT, int SC, int MT, int RT>
-static int launch_stream_one(const StreamBatch& b, const int* first, const bf16_t* x, int64_t ldx, int64_t M, int64_t K, size_t lds, hipStream_t s) {
+static int launch_stream_one(const StreamBatch& b, const int* first, const bf16_t* x, int64_t ldx, int64_t M, int64_t K, hipStream_t s) {
+    constexpr int lds = kStreamWaves * StreamGeo<FMT, MT, RT>::WAVE + (FMT == XQ_FMT_NF4 ? 64 : 0);
+    static_assert(lds <= 160 * 1024, "LDS of a block");
     static std::atomic<bool> attr_set{false};
     if (!attr_set) {
         const hipError_t e = hipFuncSetAttribute((const void*)stream_split_kernel<FMT, SC, MT, RT>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
@@ -658,23 +787,27 @@ static int launch_stream_one(const StreamBatch& b, const int* first, const bf16_
         }
         attr_set = true;
     }
-    stream_split_kernel<FMT, SC, MT, RT><<<(unsigned)first[4], 64 * kStreamWaves, lds, s>>>(x, (int32_t)ldx, (int32_t)M, (int32_t)K, first[1], first[2], first[3], b);
+    stream_split_kernel<FMT, SC, MT, RT><<<(unsigned)first[4], 64 * kStreamWaves, lds, s>>>(x, ldx, (int32_t)M, (int32_t)K, first[1], first[2], first[3], b);
     return XQ_OK;
 }
 template <int FMT, int SC, int MT>
-static int launch_stream_mt(const StreamBatch& b, const int* first, const bf16_t* x, int64_t ldx, int64_t M, int64_t K, int rt, size_t lds, hipStream_t s) {
-    constexpr int most = kRowTilesMax<SC>;
-    if constexpr (most > 2)
-        if (rt == 3) return launch_stream_one<FMT, SC, MT, 3>(b, first, x, ldx, M, K, lds, s);
-    if constexpr (most > 1)
-        if (rt == 2) return launch_stream_one<FMT, SC, MT, 2>(b, first, x, ldx, M, K, lds, s);
-    return launch_stream_one<FMT, SC, MT, 1>(b, first, x, ldx, M, K, lds, s);
+static int launch_stream_mt(const StreamBatch& b, const int* first, const bf16_t* x, int64_t ldx, int64_t M, int64_t K, int rt, hipStream_t s) {
+    constexpr int most = row_tiles_max(FMT, SC);
+    if constexpr (most > 4)
+        if (rt == 6) return launch_stream_one<FMT, SC, MT, 6>(b, first, x, ldx, M, K, s);
+    if constexpr (most > 2) {
+        if (rt == 4) return launch_stream_one<FMT, SC, MT, 4>(b, first, x, ldx, M, K, s);
+        if (rt == 3) return launch_stream_one<FMT, SC, MT, 3>(b, first, x, ldx, M, K, s);
+    }
+    if (rt == 2) return launch_stream_one<FMT, SC, MT, 2>(b, first, x, ldx, M, K, s);
+    return launch_stream_one<FMT, SC, MT, 1>(b, first, x, ldx, M, K, s);
 }
 template <int FMT, int SC>
-static int launch_stream_sc(const StreamBatch& b, const int* first, const bf16_t* x, int64_t ldx, int64_t M, int64_t K, int rt, size_t lds, hipStream_t s) {
-    if (M <= 16) return launch_stream_mt<FMT, SC, 1>(b, first, x, ldx, M, K, rt, lds, s);
-    if (M <= 32) return launch_stream_mt<FMT, SC, 2>(b, first, x, ldx, M, K, rt, lds, s);
-    return launch_stream_mt<FMT, SC, 4>(b, first, x, ldx, M, K, rt, lds, s);
+static int launch_stream_sc(const StreamBatch& b, const int* first, const bf16_t* x, int64_t ldx, int64_t M, int64_t K, int rt, hipStream_t s) {
+    if (M <= 16) return launch_stream_mt<FMT, SC, 1>(b, first, x, ldx, M, K, rt, s);
+    if (M <= 32) return launch_stream_mt<FMT, SC, 2>(b, first, x, ldx, M, K, rt, s);
+    if (M <= 48) return launch_stream_mt<FMT, SC, 3>(b, first, x, ldx, M, K, rt, s);
+    return launch_stream_mt<FMT, SC, 4>(b, first, x, ldx, M, K, rt, s);
 }
 
 bool skinny_stream_multi_supported(const SkinnyRowsJob* jobs, int n_jobs, int64_t M) {
@@ -693,8 +826,8 @@ int launch_skinny_stream(const SkinnyRowsJob* jobs, int n_jobs, bool swiglu, con
                          void* workspace, hipStream_t stream) {
     const xq_weight* w0 = jobs[0].w;
     const int64_t K = w0->cols;
-    const int sc = scale_mode(w0), mt = M <= 16 ? 1 : M <= 32 ? 2 : 4;
-    XQ_REQUIRE(ldx < (1ll << 31), "xq_linear_fwd: internal error: shape not supported by the streaming kernel");
+    const int sc = scale_mode(w0), mt = (int)xq_cdiv(M, 16);
+    XQ_REQUIRE(M <= 8 || ldx < kSkinnyLdx, "xq_linear_fwd: internal error: rows of x too far apart for the streaming kernel");
     StreamBatch b{};
     EpiBatch e{};
     uint8_t* ws = (uint8_t*)workspace;
@@ -723,13 +856,15 @@ int launch_skinny_stream(const SkinnyRowsJob* jobs, int n_jobs, bool swiglu, con
     }
     int tiles[kStreamJobs], splits[kStreamJobs];
     for (int i = 0; i < n_jobs; ++i) { tiles[i] = b.job[i].N / 16; splits[i] = b.job[i].splits; }
-    const int rt = stream_row_tiles(tiles, splits, n_jobs, steps, mt, sc == kScUse ? kRowTilesMax<kScUse> : sc == kScStep ? kRowTilesMax<kScStep> : 3, nullptr);
+    const int rt = stream_row_tiles(tiles, splits, n_jobs, steps, mt, row_tiles_max(w0->format, sc), nullptr);
     int first[5] = {0, 0, 0, 0, 0}, efirst[5] = {0, 0, 0, 0, 0};
     for (int i = 0; i < kStreamJobs; ++i) {
         first[i + 1] = first[i];
         efirst[i + 1] = efirst[i];
         if (i < n_jobs) {
-            b.job[i].row_blocks = (int)xq_cdiv(tiles[i], (int64_t)kStreamWaves * rt);
+            // (a weight of fewer row blocks than rank tiles gets blocks that only form a low-rank part)
+            const int rank_tiles = b.job[i].r_pad >> 4, row_blocks = (int)xq_cdiv(tiles[i], (int64_t)rt);
+            b.job[i].row_blocks = row_blocks > rank_tiles ? row_blocks : rank_tiles;
             first[i + 1] += b.job[i].row_blocks * b.job[i].splits;
             efirst[i + 1] += (int)xq_cdiv(b.job[i].N, 128);
         } else {
@@ -737,16 +872,15 @@ int launch_skinny_stream(const SkinnyRowsJob* jobs, int n_jobs, bool swiglu, con
             e.job[i] = e.job[0];
         }
     }
-    const size_t lds = (size_t)steps * mt * 4096 + 64;             // the x slice of the longest split, the nf4 levels
     int rc = XQ_ERR_UNSUPPORTED;
 #define XQ_STREAM_CASE(F, S) \
-    if (w0->format == F && sc == S) rc = launch_stream_sc<F, S>(b, first, x, ldx, M, K, rt, lds, stream)
+    if (w0->format == F && sc == S) rc = launch_stream_sc<F, S>(b, first, x, ldx, M, K, rt, stream)
     XQ_STREAM_CASE(XQ_FMT_FP8, kScFp8);
     XQ_STREAM_CASE(XQ_FMT_INT4, kScInt4Window);
-    XQ_STREAM_CASE(XQ_FMT_INT4, kScStep);
+    XQ_STREAM_CASE(XQ_FMT_INT4, kScHalf);
     XQ_STREAM_CASE(XQ_FMT_INT4, kScUse);
     XQ_STREAM_CASE(XQ_FMT_NVFP4, kScDealt);
-    XQ_STREAM_CASE(XQ_FMT_NVFP4, kScStep);
+    XQ_STREAM_CASE(XQ_FMT_NVFP4, kScHalf);
     XQ_STREAM_CASE(XQ_FMT_NF4, kScDealt);
 #undef XQ_STREAM_CASE
     if (rc) return rc;

@@ -494,20 +494,23 @@ struct EpiBatch {
 
 // y[m][n..n+1] = sum_s part[s][m][n..] + bias + su_scale * sum_j su[m][j] * B[n][j], su = sum of the parts.  A wave takes 128
 // columns (a lane 2) of RW rows, the block's waves the rows next to each other.  The kernel is a few dependent memory round
-// trips long: everything the first sums need -- B values of the first 16 ranks, partial tiles, low-rank parts (dealt over all
-// threads, met in LDS) -- is requested before anything is waited for.  Every sum runs in a fixed order.
+// trips long: everything it needs -- low-rank parts (dealt over all threads, met in LDS), partial tiles, B values of all ranks (NB
+// chunks of 16) -- is requested before anything is waited for, in the order of use.  Every sum runs in a fixed order.
+// NB: B's chunks were once fetched one behind the other, a trip to memory each: whole forwards at r 64, us, of 24 / 64 rows: int4
+// [4096, 4096] 14.2 -> 13.6 / 17.0 -> 16.5, [7808, 2944] 15.6 -> 14.9 / 20.8 -> 20.0, fp8 [1024, 4096] 12.4 -> 11.8 / 14.6 -> 14.0; level at
+// [12288, 4096] and r 16.
 // RW: 1 up to 16 rows; 2 with eight splits requested at a time above, against 4 rows and four splits, which took fewer blocks and
 // twice the trips.  Whole forwards at r 16 / 64, us, of 24 rows: int4 [1024, 4096] 14.4 -> 12.4 / 18.8 -> 14.7, [4096, 4096] 15.1 -> 14.0 /
 // 19.4 -> 16.3, [4096, 12288] 19.0 -> 17.5 / 26.9 -> 21.7; of 64 rows: 13.5 -> 12.5 / 18.1 -> 15.1, 15.9 -> 15.7 / 20.2 -> 18.2, 24.4 -> 23.4 /
 // 32.1 -> 27.6.  [12288, 4096], where the epilogue is the smaller part, is level at r 16.
 // VEC: B is fp32 with r % 4 == 0 (16-byte pieces).  GU: jobs 0 and 1 are gate and up, h is written.
-template <int RW, bool VEC, bool GU>
+template <int RW, int NB, bool VEC, bool GU>
 __global__ void __launch_bounds__(256)
 stream_epilogue_kernel(int32_t M, int32_t first1, int32_t first2, int32_t first3, EpiBatch b) {
     constexpr int NP = GU ? 2 : 1;
     __shared__ __attribute__((aligned(16))) float su[NP][4 * RW][64];
     __shared__ f32x4 red[NP][256];
-    __shared__ f32x4 bt[NP][512];
+    __shared__ f32x4 bt[NP][NB][512];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int bx = blockIdx.x;
@@ -524,32 +527,32 @@ stream_epilogue_kernel(int32_t M, int32_t first1, int32_t first2, int32_t first3
     // pieces, and shared through LDS; piece P = column * 4 + ranks / 4 lies at P ^ (column / 4 & 7), which lets the 16 lanes of a
     // read pass (two columns a lane) fall on 16 different pieces
     constexpr int kPieces = RW == 1 ? 8 : 2;                       // of a thread (RW > 1: always four waves)
-    f32x4 bq[NP][kPieces];
+    f32x4 bq[NP][NB][kPieces];
     const auto load_b = [&](int p, int rc) {
         const EpiJob& g = b.job[ji + p];
 #pragma unroll
         for (int i = 0; i < kPieces; ++i) {
             if (i * nthreads < 512) {
-                const int P = (tid + i * nthreads) & 511, col = at * 128 + (P >> 2), j = rc + 4 * (P & 3);
+                const int P = (tid + i * nthreads) & 511, col = at * 128 + (P >> 2), j = 16 * rc + 4 * (P & 3);
                 const int64_t row = (int64_t)(col < g.N ? col : 0) * g.r;
                 if constexpr (VEC) {
-                    bq[p][i] = *(const f32x4*)((const float*)g.lora_B + row + (j < g.r ? j : 0));
+                    bq[p][rc][i] = *(const f32x4*)((const float*)g.lora_B + row + (j < g.r ? j : 0));
                 } else {
 #pragma unroll
                     for (int f = 0; f < 4; ++f) {
                         const int64_t bi = row + (j + f < g.r ? j + f : 0);
-                        bq[p][i][f] = g.lora_f32 ? ((const float*)g.lora_B)[bi] : bf16_to_f32(((const bf16_t*)g.lora_B)[bi]);
+                        bq[p][rc][i][f] = g.lora_f32 ? ((const float*)g.lora_B)[bi] : bf16_to_f32(((const bf16_t*)g.lora_B)[bi]);
                     }
                 }
             }
         }
     };
-    const auto store_b = [&](int p) {
+    const auto store_b = [&](int p, int rc) {
 #pragma unroll
         for (int i = 0; i < kPieces; ++i)
             if (i * nthreads < 512) {
                 const int P = (tid + i * nthreads) & 511;
-                bt[p][P ^ ((P >> 4) & 7)] = bq[p][i];
+                bt[p][rc][P ^ ((P >> 4) & 7)] = bq[p][rc][i];
             }
     };
     constexpr int SB = RW == 2 ? 8 : 4;                            // splits requested at a time
@@ -563,34 +566,46 @@ stream_epilogue_kernel(int32_t M, int32_t first1, int32_t first2, int32_t first3
             for (int u = 0; u < RW; ++u)
                 t[p][v][u] = *(const f32x2*)(g.partial + (int64_t)(s0 + v < g.splits ? s0 + v : g.splits - 1) * ss + (int64_t)(mw + u < M ? mw + u : M - 1) * g.N + nn);
     };
+    // (in the order in which they are waited for)
+    f32x4 sp[NP][8];
+    const auto load_su = [&](int p, int p0) {                      // thread (quad of ranks of a row, group of parts)
+        const EpiJob& g = b.job[ji + p];
+        const int qr = g.r_pad >> 2, quads = 4 * RW * qr, groups = nthreads / quads;
+        const int qd = tid % quads, gi = tid / quads, m = qd / qr;
+        const float* src = g.su_part + (int64_t)(m0 + m < M ? m0 + m : M - 1) * g.r_pad + (qd - m * qr) * 4;
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int pi = p0 + gi + u * groups;
+            sp[p][u] = *(const f32x4*)(src + (int64_t)(pi < g.parts ? pi : g.parts - 1) * M * g.r_pad);
+        }
+    };
 #pragma unroll
     for (int p = 0; p < NP; ++p)
-        if (b.job[ji + p].r > 0) load_b(p, 0);
+        if (b.job[ji + p].r > 0) load_su(p, 0);
 #pragma unroll
     for (int p = 0; p < NP; ++p) load_part(p, 0);
+#pragma unroll
+    for (int p = 0; p < NP; ++p)
+#pragma unroll
+        for (int rc = 0; rc < NB; ++rc)
+            if (16 * rc < b.job[ji + p].r) load_b(p, rc);
 
-    // ---- su of the block's rows -> LDS: thread (quad of ranks of a row, group of parts)
+    // ---- su of the block's rows -> LDS
 #pragma unroll
     for (int p = 0; p < NP; ++p) {
         const EpiJob& g = b.job[ji + p];
         if (g.r > 0) {
-            const int qr = g.r_pad >> 2, quads = 4 * RW * qr, groups = nthreads / quads;
-            const int qd = tid % quads, gi = tid / quads, m = qd / qr;
-            const float* sp = g.su_part + (int64_t)(m0 + m < M ? m0 + m : M - 1) * g.r_pad + (qd - m * qr) * 4;
+            const int quads = RW * g.r_pad, groups = nthreads / quads, gi = tid / quads;
             f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
-            for (int p0 = gi; p0 < g.parts; p0 += 8 * groups) {
-                f32x4 a[8];
-#pragma unroll
-                for (int u = 0; u < 8; ++u) {
-                    const int pi = p0 + u * groups;
-                    a[u] = *(const f32x4*)(sp + (int64_t)(pi < g.parts ? pi : g.parts - 1) * M * g.r_pad);
-                }
+            for (int p0 = 0;;) {
 #pragma unroll
                 for (int u = 0; u < 8; ++u)
-                    if (p0 + u * groups < g.parts) v += a[u];
+                    if (p0 + gi + u * groups < g.parts) v += sp[p][u];
+                p0 += 8 * groups;
+                if (p0 >= g.parts) break;
+                load_su(p, p0);
             }
             red[p][tid] = v;
-            store_b(p);
         }
     }
     __syncthreads();
@@ -629,30 +644,31 @@ stream_epilogue_kernel(int32_t M, int32_t first1, int32_t first2, int32_t first3
             load_part(p, s0);
         }
     }
+#pragma unroll
+    for (int p = 0; p < NP; ++p)
+#pragma unroll
+        for (int rc = 0; rc < NB; ++rc)
+            if (16 * rc < b.job[ji + p].r) store_b(p, rc);
     __syncthreads();
 #pragma unroll
     for (int p = 0; p < NP; ++p) {
         const EpiJob& g = b.job[ji + p];
-        for (int rc = 0; rc < g.r; rc += 16) {
-            if (rc + 16 < g.r) load_b(p, rc + 16);
+#pragma unroll
+        for (int rc = 0; rc < NB; ++rc) {
+            if (16 * rc >= g.r) break;
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
                 f32x4 bv[2];
 #pragma unroll
-                for (int e = 0; e < 2; ++e) bv[e] = bt[p][((lane * 2 + e) * 4 + c) ^ ((lane >> 1) & 7)];
+                for (int e = 0; e < 2; ++e) bv[e] = bt[p][rc][((lane * 2 + e) * 4 + c) ^ ((lane >> 1) & 7)];
 #pragma unroll
                 for (int u = 0; u < RW; ++u) {
-                    const f32x4 sv = *(const f32x4*)&su[p][wave * RW + u][rc + 4 * c];
+                    const f32x4 sv = *(const f32x4*)&su[p][wave * RW + u][16 * rc + 4 * c];
 #pragma unroll
                     for (int f = 0; f < 4; ++f)
 #pragma unroll
                         for (int e = 0; e < 2; ++e) o[p][u][e] = __builtin_fmaf(sv[f], bv[e][f], o[p][u][e]);
                 }
-            }
-            if (rc + 16 < g.r) {
-                __syncthreads();
-                store_b(p);
-                __syncthreads();
             }
         }
         if (g.bias) {
@@ -905,20 +921,27 @@ int launch_skinny_stream(const SkinnyRowsJob* jobs, int n_jobs, bool swiglu, con
     const int rw = M <= 16 ? 1 : four ? 4 : 2;
     const unsigned threads = M < 4 && rw == 1 ? (unsigned)M * 64 : 256;
     const dim3 grid(cols, (unsigned)xq_cdiv(M, 4 * rw));
-#define XQ_EPI(RW)                                                                                                                             \
+#define XQ_EPI_NB(RW, NB)                                                                                                                      \
     do {                                                                                                                                       \
         if (swiglu) {                                                                                                                          \
-            if (vec) stream_epilogue_kernel<RW, true, true><<<grid, threads, 0, stream>>>((int)M, efirst[1], efirst[2], efirst[3], e);         \
-            else stream_epilogue_kernel<RW, false, true><<<grid, threads, 0, stream>>>((int)M, efirst[1], efirst[2], efirst[3], e);            \
+            if (vec) stream_epilogue_kernel<RW, NB, true, true><<<grid, threads, 0, stream>>>((int)M, efirst[1], efirst[2], efirst[3], e);     \
+            else stream_epilogue_kernel<RW, NB, false, true><<<grid, threads, 0, stream>>>((int)M, efirst[1], efirst[2], efirst[3], e);        \
         } else {                                                                                                                               \
-            if (vec) stream_epilogue_kernel<RW, true, false><<<grid, threads, 0, stream>>>((int)M, efirst[1], efirst[2], efirst[3], e);        \
-            else stream_epilogue_kernel<RW, false, false><<<grid, threads, 0, stream>>>((int)M, efirst[1], efirst[2], efirst[3], e);           \
+            if (vec) stream_epilogue_kernel<RW, NB, true, false><<<grid, threads, 0, stream>>>((int)M, efirst[1], efirst[2], efirst[3], e);    \
+            else stream_epilogue_kernel<RW, NB, false, false><<<grid, threads, 0, stream>>>((int)M, efirst[1], efirst[2], efirst[3], e);       \
         }                                                                                                                                      \
+    } while (0)
+#define XQ_EPI(RW)                       \
+    do {                                 \
+        if (ranks <= 16) XQ_EPI_NB(RW, 1); \
+        else if (ranks <= 32) XQ_EPI_NB(RW, 2); \
+        else XQ_EPI_NB(RW, 4);           \
     } while (0)
     if (rw == 1) XQ_EPI(1);
     else if (rw == 2) XQ_EPI(2);
     else XQ_EPI(4);
 #undef XQ_EPI
+#undef XQ_EPI_NB
     return XQ_OK;
 }
 

@@ -790,3 +790,23 @@ def test_routed_rows_read_in_place_equal_the_copy(hip_device, fmt, hybrid):
     assert torch.equal(y0, y1) and torch.equal(dx0, dx1) and torch.equal(drw0, drw1)
     for a, b in zip(g0, g1):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("H,I,r", [(1152, 576, 16), (256, 512, 24)])      # nine units over eight waves both ways; fewer units than waves
+@pytest.mark.parametrize("few", [1, 37, 8300])                          # the narrow forms of all passes, and the SwiGLU forward's alone
+def test_few_routed_rows_equal_the_same_rows_among_many(hip_device, H, I, r, few):
+    """A token's output and gradients do not depend on the other tokens: the passes over few routed rows (32 to a block, the
+    waves splitting the columns) against those over many (128 to a block)."""
+    E, topk, T = 4, 2, 20600
+    m, _ = _make_experts("block_fp8", E, H, I, r, False, seed=H, device=hip_device)
+    rw, sel = _zipf_routing(T, E, topk, seed=3)
+    x, dy = gen((T, H), 1.0, 5, torch.bfloat16), gen((T, H), 1.0, 6, torch.bfloat16)
+
+    def run(n):
+        xd, rwd = x[:n].to(hip_device).requires_grad_(True), rw[:n].to(torch.bfloat16).to(hip_device).requires_grad_(True)
+        y = m(xd, rwd, sel[:n].to(hip_device))
+        gx, gw = torch.autograd.grad(y, (xd, rwd), dy[:n].to(hip_device))
+        return y.detach().cpu(), gx.cpu(), gw.cpu()
+
+    for a, b, tol in zip(run(few), run(T), (TOL, TOL, 2e-2)):          # (bf16 intermediates on both sides, as against the oracle)
+        close(a, b[:few].double(), tol, rows="none")

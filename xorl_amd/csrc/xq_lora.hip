@@ -156,16 +156,20 @@ struct SmallNtArgs {
 // every load is unconditional -- rows past the segment and columns past the wave's K range are clamped onto
 // valid ones and their values never used -- so the waits count exactly and the loads of chunk k+2 stay in
 // flight while chunk k is multiplied.
+// NARROW: 32 rows per block and the contraction split over its waves (eight, four beyond rank 32), whose sums meet in LDS in wave
+// order.  With few rows the wide form is a fraction of the chip's waves, each a chain of Kc / 128 trips to memory (narrow_nt has both
+// forms' times).
 constexpr int SN_P = 136;   // LDS row pitch in bf16 elements
-template <int FJ, bool GATHER = false>
-__global__ void __launch_bounds__(256) small_nt_kernel(SmallNtArgs g) {
-    constexpr int NT = (FJ + 7) / 8;
+constexpr int sn_waves(int FJ, bool narrow) { return narrow && FJ <= 8 ? 8 : 4; }
+template <int FJ, bool GATHER, bool NARROW>
+__global__ void __launch_bounds__(64 * sn_waves(FJ, NARROW)) small_nt_kernel(SmallNtArgs g) {
+    constexpr int NT = (FJ + 7) / 8, NW = sn_waves(FJ, NARROW);
     constexpr int TR = 128;
     constexpr int WTILE = (32 + NT * 32) * SN_P;   // bf16 elements per wave: In tile + F tile
     extern __shared__ __attribute__((aligned(16))) bf16_t sn_lds[];
     __shared__ int sh_info[3];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int rg = wave;
+    const int rg = NARROW ? (int)(blockIdx.x / (gridDim.x >> 2)) : wave;
 
     int e = 0;
     int64_t row0, row_end;
@@ -174,7 +178,7 @@ __global__ void __launch_bounds__(256) small_nt_kernel(SmallNtArgs g) {
         // (a binary search by one thread is a chain of dependent memory round trips)
         if (tid == 0) sh_info[0] = -1;
         __syncthreads();
-        const int t = blockIdx.x;
+        const int t = NARROW ? blockIdx.x % (gridDim.x >> 2) : blockIdx.x;     // (a tile's four parts a stretch apart: experts of few rows fill only the first)
         for (int x = tid; x < g.num_experts; x += blockDim.x) {
             const int lo = g.tile_offsets[x], hi = g.tile_offsets[x + 1];
             const int o0 = g.offsets[x], o1 = g.offsets[x + 1];
@@ -189,6 +193,7 @@ __global__ void __launch_bounds__(256) small_nt_kernel(SmallNtArgs g) {
         if (e < 0) return;
         row0 = sh_info[1];
         row_end = sh_info[2];
+        if (NARROW && row0 + rg * 32 >= row_end) return;
     }
     const bf16_t* F = g.F + (int64_t)e * g.f_stride;
     bf16_t* xs = sn_lds + wave * WTILE;          // [32][SN_P]
@@ -204,7 +209,8 @@ __global__ void __launch_bounds__(256) small_nt_kernel(SmallNtArgs g) {
 #pragma unroll
         for (int q = 0; q < 16; ++q) acc[n][q] = 0.0f;
 
-    const int64_t kbeg = 0, kend = g.Kc;
+    const int64_t units = (g.Kc + 127) >> 7;
+    const int64_t kbeg = NARROW ? units * wave / NW << 7 : 0, kto = NARROW ? units * (wave + 1) / NW << 7 : g.Kc, kend = kto < g.Kc ? kto : g.Kc;
     const bf16_t* xp[8];
     int32_t orow[GATHER ? 8 : 1];                // GATHER: the rows of copy_out this lane's pieces belong to
 #pragma unroll
@@ -264,12 +270,32 @@ __global__ void __launch_bounds__(256) small_nt_kernel(SmallNtArgs g) {
             }
         }
     };
-    fetch_x(xr[0], kbeg);
-    fetch_f(kbeg);
-    fetch_x(xr[1], kbeg + 128);
-    for (int64_t k = kbeg; k < kend; k += 256) {
-        chunk(xr[0], k);
-        chunk(xr[1], k + 128);
+    if (!NARROW || kbeg < kend) {                // (fewer units than waves: nothing to fetch)
+        fetch_x(xr[0], kbeg);
+        fetch_f(kbeg);
+        fetch_x(xr[1], kbeg + 128);
+        for (int64_t k = kbeg; k < kend; k += 256) {
+            chunk(xr[0], k);
+            chunk(xr[1], k + 128);
+        }
+    }
+    if constexpr (NARROW) {
+        float* red = (float*)sn_lds;             // [NW - 1][NT][16][64] floats, over the (now dead) tiles
+        __syncthreads();
+        if (wave > 0) {
+#pragma unroll
+            for (int n = 0; n < NT; ++n)
+#pragma unroll
+                for (int q = 0; q < 16; ++q) red[(((wave - 1) * NT + n) * 16 + q) * 64 + lane] = acc[n][q];
+        }
+        __syncthreads();
+        if (wave > 0) return;
+#pragma unroll
+        for (int w = 1; w < NW; ++w)
+#pragma unroll
+            for (int n = 0; n < NT; ++n)
+#pragma unroll
+                for (int q = 0; q < 16; ++q) acc[n][q] += red[(((w - 1) * NT + n) * 16 + q) * 64 + lane];
     }
 
     const int rgrp = (lane >> 5) * 4;
@@ -288,32 +314,38 @@ __global__ void __launch_bounds__(256) small_nt_kernel(SmallNtArgs g) {
     }
 }
 
-template <int FJ, bool GATHER = false>
+template <int FJ, bool GATHER, bool NARROW>
 static int launch_small_nt_one(const SmallNtArgs& g, unsigned blocks, hipStream_t stream) {
-    constexpr int NT = (FJ + 7) / 8;
-    constexpr size_t lds = (size_t)4 * (32 + NT * 32) * SN_P * 2;
+    constexpr int NT = (FJ + 7) / 8, NW = sn_waves(FJ, NARROW);
+    constexpr size_t lds = (size_t)NW * (32 + NT * 32) * SN_P * 2;
     static std::atomic<bool> attr_set{false};   // the attribute call is idempotent: a race only repeats it
     if (!attr_set) {
-        hipError_t e = hipFuncSetAttribute((const void*)small_nt_kernel<FJ, GATHER>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        hipError_t e = hipFuncSetAttribute((const void*)small_nt_kernel<FJ, GATHER, NARROW>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) {
             xq_set_error("small_nt: cannot raise the dynamic LDS limit: %s", hipGetErrorString(e));
             return XQ_ERR_LAUNCH;
         }
         attr_set = true;
     }
-    small_nt_kernel<FJ, GATHER><<<dim3(blocks), 256, lds, stream>>>(g);
+    small_nt_kernel<FJ, GATHER, NARROW><<<dim3(NARROW ? 4 * blocks : blocks), 64 * NW, lds, stream>>>(g);
     return XQ_OK;
 }
 
-template <bool GATHER>
+template <bool GATHER, bool NARROW>
 static int launch_small_nt_rows(const SmallNtArgs& g, unsigned blocks, hipStream_t stream) {
     switch (g.r_pad) {
-        case 16: return launch_small_nt_one<4, GATHER>(g, blocks, stream);
-        case 32: return launch_small_nt_one<8, GATHER>(g, blocks, stream);
-        case 48: return launch_small_nt_one<12, GATHER>(g, blocks, stream);
-        default: return launch_small_nt_one<16, GATHER>(g, blocks, stream);
+        case 16: return launch_small_nt_one<4, GATHER, NARROW>(g, blocks, stream);
+        case 32: return launch_small_nt_one<8, GATHER, NARROW>(g, blocks, stream);
+        case 48: return launch_small_nt_one<12, GATHER, NARROW>(g, blocks, stream);
+        default: return launch_small_nt_one<16, GATHER, NARROW>(g, blocks, stream);
     }
 }
+
+// Routed rows in blocks of 32 whose waves split the contraction, or in blocks of 128 whose waves split the rows: the first where it
+// leaves a block per compute unit or less (experts' last blocks are half empty on average).  us, wide -> narrow: K 2048, two factors
+// of rank 16, 1800 rows of 64 experts 18.9 -> 11.2, 6000 19.2 -> 19.7, 12000 19.5 -> 22.6; K 4096, rank 32, 16 experts: 1200 rows 48.5 ->
+// 19.9 (two factors) and 31.2 -> 14.3 (one), 6000 49.6 -> 22.2 and 32.3 -> 16.5, 16000 51.5 -> 60.3.
+static bool narrow_nt(int64_t n_rows, int num_experts) { return xq_cdiv(n_rows, 32) + num_experts / 2 <= num_cus(); }
 
 int launch_small_nt(const bf16_t* In, int64_t ld_in, int64_t n_rows, int64_t Kc, const bf16_t* F, int r_pad,
                     float scale, bf16_t* T, const int32_t* offsets, const int32_t* tile_offsets,
@@ -332,7 +364,9 @@ int launch_small_nt(const bf16_t* In, int64_t ld_in, int64_t n_rows, int64_t Kc,
     SmallNtArgs g{In, ld_in, n_rows, Kc, F, shared_f ? 0 : (int64_t)r_pad * Kc, r_pad, scale, T, ld_t, T2, split, offsets,
                   tile_offsets, num_experts, row_map, copy_out, ld_copy};
     const unsigned blocks = (unsigned)(xq_cdiv(n_rows, 128) + num_experts);
-    const int rc = row_map ? launch_small_nt_rows<true>(g, blocks, stream) : launch_small_nt_rows<false>(g, blocks, stream);
+    const int rc = narrow_nt(n_rows, num_experts)
+                       ? (row_map ? launch_small_nt_rows<true, true>(g, blocks, stream) : launch_small_nt_rows<false, true>(g, blocks, stream))
+                       : (row_map ? launch_small_nt_rows<true, false>(g, blocks, stream) : launch_small_nt_rows<false, false>(g, blocks, stream));
     if (rc) return rc;
     XQ_CHECK_LAUNCH("small_nt");
     return XQ_OK;
@@ -706,9 +740,14 @@ struct SiluNtArgs {
 // FWD: the forward pass in the same organisation -- h = bf16(bf16(silu(gate)) * up) (routed: then rounded and times the row's
 // weight), the elementwise forward kernel's arithmetic, written through `dgate`, and Tg = scale * h . Fg^T from the values
 // on their way out (dh, dup, Fu, Tu, d_row_w unused).
-template <int FJ, bool GROUPED, bool FWD, int MODE>
-__global__ void __launch_bounds__(256, 2) silu_bwd_nt_kernel(SiluNtArgs g) {
+// NARROW (GROUPED): 32 rows per block and the columns split over its eight waves, whose sums meet in LDS.  A wave's chunk is some 3 us of
+// vector work beside its trip to memory, and in the wide form a wave walks all the columns: 64 us however few the rows (the launchers
+// have both forms' times).
+template <int FJ, bool GROUPED, bool FWD, int MODE, bool NARROW = false>
+__global__ void __launch_bounds__(NARROW ? 512 : 256, NARROW ? 1 : 2) silu_bwd_nt_kernel(SiluNtArgs g) {
     static_assert(FJ <= 8, "one MFMA column tile per product");
+    static_assert(GROUPED || !NARROW, "the narrow form is one of routed rows");
+    constexpr int NW = NARROW ? 8 : 4;
     // 64 columns at a time (where small_nt_kernel takes 128: the same MFMA steps in the same order): three operands' pieces
     // are 12 KB per wave in flight, and two blocks share a compute unit
     constexpr int CW = 64, P = CW + 8;           // columns of a chunk; LDS row pitch (144 B: the 16 lanes of a read phase hit distinct banks)
@@ -725,8 +764,8 @@ __global__ void __launch_bounds__(256, 2) silu_bwd_nt_kernel(SiluNtArgs g) {
         // the expert whose tile range holds this block's tile: one look per thread, all loads in flight together
         if (tid == 0) sh_info[0] = -1;
         __syncthreads();
-        const int t = blockIdx.x;
-        for (int x = tid; x < g.num_experts; x += 256) {
+        const int t = NARROW ? blockIdx.x % (gridDim.x >> 2) : blockIdx.x;     // (a tile's four parts a stretch apart: experts of few rows fill only the first)
+        for (int x = tid; x < g.num_experts; x += 64 * NW) {
             const int lo = g.tile_offsets[x], hi = g.tile_offsets[x + 1];
             const int o0 = g.offsets[x], o1 = g.offsets[x + 1];
             if (lo <= t && t < hi) {
@@ -738,9 +777,9 @@ __global__ void __launch_bounds__(256, 2) silu_bwd_nt_kernel(SiluNtArgs g) {
         __syncthreads();
         e = sh_info[0];
         if (e < 0) return;
-        row0 = sh_info[1] + wave * 32;
+        row0 = sh_info[1] + (NARROW ? (int)(blockIdx.x / (gridDim.x >> 2)) : wave) * 32;
         row_end = sh_info[2];
-        if (row0 >= row_end) return;             // (no block barrier from here on in this form)
+        if (row0 >= row_end) return;             // (a wave of the wide form: no block barrier from here on there)
     } else {
         row0 = (int64_t)blockIdx.x * 32;
         row_end = g.n_rows;
@@ -754,8 +793,9 @@ __global__ void __launch_bounds__(256, 2) silu_bwd_nt_kernel(SiluNtArgs g) {
     const int crow = lane / (CW / 8), cpiece = (lane % (CW / 8)) * 8;
     const int frows = g.r_pad;
     // (dense: the 64-column units dealt evenly over the waves of the block column)
-    const int64_t units = g.Kc / CW, parts = 4 * gridDim.y, part = 4 * blockIdx.y + wave;
-    const int64_t kbeg = GROUPED ? 0 : units * part / parts * CW, kend = GROUPED ? g.Kc : units * (part + 1) / parts * CW;
+    const int64_t units = g.Kc / CW, parts = NW * gridDim.y, part = NW * blockIdx.y + wave;
+    constexpr bool WHOLE = GROUPED && !NARROW;   // a wave takes all columns
+    const int64_t kbeg = WHOLE ? 0 : units * part / parts * CW, kend = WHOLE ? g.Kc : units * (part + 1) / parts * CW;
     const int64_t rbase = row0 + crow;           // this lane's rows: rbase + RPI j, clamped onto the last row
     auto row_of = [&](int j) { const int64_t r = rbase + j * RPI; return r < row_end ? r : row_end - 1; };
     float rw[GROUPED ? NL : 1], wsum[GROUPED ? NL : 1];
@@ -899,8 +939,11 @@ __global__ void __launch_bounds__(256, 2) silu_bwd_nt_kernel(SiluNtArgs g) {
             float v = wsum[j];
 #pragma unroll
             for (int o = 1; o < CW / 8; o <<= 1) v += __shfl_xor(v, o, 64);
-            if (!FWD && g.d_row_w && lane % (CW / 8) == 0 && rbase + j * RPI < row_end) g.d_row_w[rbase + j * RPI] = v;
+            if (!NARROW && !FWD && g.d_row_w && lane % (CW / 8) == 0 && rbase + j * RPI < row_end) g.d_row_w[rbase + j * RPI] = v;
+            wsum[j] = v;
         }
+    }
+    if constexpr (WHOLE) {
         if (fr < g.r_pad) {
 #pragma unroll
             for (int q = 0; q < 16; ++q) {
@@ -913,24 +956,39 @@ __global__ void __launch_bounds__(256, 2) silu_bwd_nt_kernel(SiluNtArgs g) {
         }
         return;
     }
-    // the four waves' sums meet in LDS, in wave order (as in small_nt_kernel)
-    float* red = (float*)sn_lds;                 // [3 waves][2 products][16][64] floats, over the (now dead) tiles
+    // the waves' sums meet in LDS, in wave order
+    constexpr int PR = FWD && NARROW ? 1 : 2;
+    float* red = (float*)sn_lds;                 // [NW - 1 waves][PR products][16][64] floats, over the (now dead) tiles
+    float* red_w = red + (NW - 1) * PR * 1024;   // NARROW: [NW][32] sums of the routing weights' gradients
     __syncthreads();
     if (wave > 0) {
 #pragma unroll
         for (int q = 0; q < 16; ++q) {
-            red[(((wave - 1) * 2 + 0) * 16 + q) * 64 + lane] = acc_g[q];
-            red[(((wave - 1) * 2 + 1) * 16 + q) * 64 + lane] = acc_u[q];
+            red[(((wave - 1) * PR + 0) * 16 + q) * 64 + lane] = acc_g[q];
+            if constexpr (PR > 1) red[(((wave - 1) * PR + 1) * 16 + q) * 64 + lane] = acc_u[q];
+        }
+    }
+    if constexpr (NARROW && !FWD) {
+        if (lane % (CW / 8) == 0) {
+#pragma unroll
+            for (int j = 0; j < NL; ++j) red_w[wave * 32 + j * RPI + crow] = wsum[j];
         }
     }
     __syncthreads();
+    if constexpr (NARROW && !FWD) {
+        if (wave == 1 && lane < 32 && g.d_row_w && row0 + lane < row_end) {
+            float v = red_w[lane];
+            for (int w = 1; w < NW; ++w) v += red_w[w * 32 + lane];
+            g.d_row_w[row0 + lane] = v;
+        }
+    }
     if (wave > 0) return;
 #pragma unroll
-    for (int s = 1; s < 4; ++s)
+    for (int s = 1; s < NW; ++s)
 #pragma unroll
         for (int q = 0; q < 16; ++q) {
-            acc_g[q] += red[(((s - 1) * 2 + 0) * 16 + q) * 64 + lane];
-            acc_u[q] += red[(((s - 1) * 2 + 1) * 16 + q) * 64 + lane];
+            acc_g[q] += red[(((s - 1) * PR + 0) * 16 + q) * 64 + lane];
+            if constexpr (PR > 1) acc_u[q] += red[(((s - 1) * PR + 1) * 16 + q) * 64 + lane];
         }
     if (gridDim.y > 1) {
         constexpr int NP = 2;
@@ -959,19 +1017,20 @@ __global__ void __launch_bounds__(256, 2) silu_bwd_nt_kernel(SiluNtArgs g) {
     }
 }
 
-template <int FJ, bool GROUPED, bool FWD, int MODE>
+template <int FJ, bool GROUPED, bool FWD, int MODE, bool NARROW = false>
 static int launch_silu_nt_one(const SiluNtArgs& g, dim3 blocks, hipStream_t stream) {
-    constexpr size_t lds = (size_t)4 * (32 + 32) * (64 + 8) * 2;
+    constexpr int NW = NARROW ? 8 : 4;
+    constexpr size_t lds = (size_t)NW * (32 + 32) * (64 + 8) * 2;
     static std::atomic<bool> attr_set{false};   // the attribute call is idempotent: a race only repeats it
     if (!attr_set) {
-        hipError_t e = hipFuncSetAttribute((const void*)silu_bwd_nt_kernel<FJ, GROUPED, FWD, MODE>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        hipError_t e = hipFuncSetAttribute((const void*)silu_bwd_nt_kernel<FJ, GROUPED, FWD, MODE, NARROW>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) {
             xq_set_error("silu_bwd_nt: cannot raise the dynamic LDS limit: %s", hipGetErrorString(e));
             return XQ_ERR_LAUNCH;
         }
         attr_set = true;
     }
-    silu_bwd_nt_kernel<FJ, GROUPED, FWD, MODE><<<blocks, 256, lds, stream>>>(g);
+    silu_bwd_nt_kernel<FJ, GROUPED, FWD, MODE, NARROW><<<blocks, 64 * NW, lds, stream>>>(g);
     XQ_CHECK_LAUNCH("silu_bwd_nt");
     return XQ_OK;
 }
@@ -1009,6 +1068,10 @@ int launch_silu_bwd_nt(const bf16_t* gate, const bf16_t* up, int64_t ld_gu, cons
     if (offsets) {
         XQ_REQUIRE(mode == kFacBf16, "silu_bwd_nt: the routed form takes bf16 panels");
         const dim3 blocks((unsigned)(xq_cdiv(n_rows, 128) + num_experts));
+        if (n_rows <= 64ll * num_cus()) {        // (us, wide -> narrow, 64 experts of 1024 columns, r 16: 1800 rows 64 -> 19, 12000 70 -> 43, 24000 78 -> 79)
+            const dim3 four(4 * blocks.x);
+            return r_pad == 16 ? launch_silu_nt_one<4, true, false, kFacBf16, true>(g, four, stream) : launch_silu_nt_one<8, true, false, kFacBf16, true>(g, four, stream);
+        }
         return r_pad == 16 ? launch_silu_nt_one<4, true, false, kFacBf16>(g, blocks, stream) : launch_silu_nt_one<8, true, false, kFacBf16>(g, blocks, stream);
     }
     XQ_REQUIRE(mode != kFacF32, "silu_bwd_nt: factor form %d", (int)mode);
@@ -1042,6 +1105,10 @@ int launch_silu_fwd_nt(const bf16_t* gate, const bf16_t* up, int64_t ld_gu, bf16
         return r_pad == 16 ? launch_silu_nt_one<4, false, true, kFacBf16>(g, blocks, stream) : launch_silu_nt_one<8, false, true, kFacBf16>(g, blocks, stream);
     }
     const dim3 blocks((unsigned)(xq_cdiv(n_rows, 128) + num_experts));
+    if (n_rows <= (r_pad == 16 ? 160ll : 64ll) * num_cus()) {      // (the same: 1800 rows 32 -> 15, 12000 40 -> 22, 24000 46 -> 38, 48000 65 -> 66; r 32: 16000 57 -> 45, 24000 of 896 columns 3 us behind)
+        const dim3 four(4 * blocks.x);
+        return r_pad == 16 ? launch_silu_nt_one<4, true, true, kFacBf16, true>(g, four, stream) : launch_silu_nt_one<8, true, true, kFacBf16, true>(g, four, stream);
+    }
     return r_pad == 16 ? launch_silu_nt_one<4, true, true, kFacBf16>(g, blocks, stream) : launch_silu_nt_one<8, true, true, kFacBf16>(g, blocks, stream);
 }
 

@@ -114,6 +114,16 @@ static inline int dense_tile_size(int64_t n_rows, int64_t Nout) {
     return xq_cdiv(n_rows, 256) * xq_cdiv(Nout, 256) > num_cus() / 2 ? 256 : 128;
 }
 
+// The same for expert banks: large tiles where an expert's rows fill them (its last tile is half empty on average, and a 4-bit tile
+// decodes in full) and the tiles there are fill half the chip.  Forward and backward of a routed MLP, large over small tiles, by rows an
+// expert: nvfp4 / nf4 banks, 64 or 128 experts 93 1.15, 187 1.04 to 1.08, 281 1.03 to 1.10, 421 0.97 to 0.99, 656 0.93; 16 experts 250
+// 1.10 to 1.14, 500 0.90; 8 experts 500 1.09 to 1.14, 750 0.87.  Block-fp8: 64 or 128 experts 46 1.14, 62 1.01, 93 1.04, 125 0.91, 281 0.87; 16
+// experts 125 1.00, 250 0.98, 500 0.81; 8 experts 125 1.23, 250 0.94, 750 0.87.
+static inline bool bank_large_tiles(int fmt, int64_t n_rows, int num_experts, int64_t Nout) {
+    const int64_t tiles = (xq_cdiv(n_rows, 256) + num_experts / 2) * xq_cdiv(Nout, 256);
+    return n_rows >= (fmt == XQ_FMT_FP8 ? 100ll : 400ll) * num_experts && tiles > num_cus() / 2;
+}
+
 // K splits of a dense launch of `blocks` tiles of size T over nk K-steps (1 = none): used when the tiles fill at
 // most half of the block slots of the chip (256 large tiles, 512 small ones); every split keeps at least 8 K-steps.
 static inline int ksplit_for(int64_t blocks, int T, int64_t nk) {
@@ -602,7 +612,7 @@ static int launch_tile_gemm_t(const xq_weight* w, bool contract_cols, const bf16
                              (grouped ? w->layout == XQ_LAYOUT_GKN && g.wcols % 16 == 0 && g.wrows >= 2 &&
                                             xq_aligned(w->scales, 16) && g.scale_stride % 16 == 0
                                       : w->layout == XQ_LAYOUT_FLAT));
-        const bool big = grouped && n_rows >= 128ll * w->num_experts && n_rows >= 8192;   // grouped: large tiles
+        const bool big = grouped && bank_large_tiles(w->format, n_rows, w->num_experts, g.Nout);
         const DensePlan plan = plan_dense(n_rows, g.Nout, g.Kc / BK);
         const bool planned = !grouped && fmt_ok && g_tile_policy == 0 && force_T == 0 && !two_dense;   // two matrices: one unsplit launch
         const int T = force_T ? force_T : g_tile_policy == 2 ? 256 : g_tile_policy == 3 ? 128 : grouped ? (big ? 256 : 128) : plan.T;

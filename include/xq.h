@@ -518,6 +518,11 @@ int xq_grouped_fwd(const xq_weight* gate, const xq_weight* up, const xq_weight* 
                    const void* hidden, int64_t ld_hidden, int64_t n_tokens, const void* routing_w, int rw_dtype,
                    const int32_t* selected, int32_t topk, void* out, int64_t ld_out,
                    const xq_grouped_saved* saved, void* workspace, int64_t workspace_bytes, void* stream);
+/* the same on expert ids of id_bytes bytes each: 4, or 8 (a router's top-k as torch gives it; the low 32 bits count) */
+int xq_grouped_fwd_ids(const xq_weight* gate, const xq_weight* up, const xq_weight* down, const xq_grouped_lora* lora,
+                       const void* hidden, int64_t ld_hidden, int64_t n_tokens, const void* routing_w, int rw_dtype,
+                       const void* ids, int id_bytes, int32_t topk, void* out, int64_t ld_out,
+                       const xq_grouped_saved* saved, void* workspace, int64_t workspace_bytes, void* stream);
 int xq_grouped_bwd(const xq_weight* gate, const xq_weight* up, const xq_weight* down, const xq_grouped_lora* lora,
                    const void* dy, int64_t ld_dy, int64_t n_tokens, int32_t topk, const xq_grouped_saved* saved,
                    void* dx, int64_t ld_dx, void* d_routing, int rw_dtype, const xq_grouped_grads* grads,
@@ -541,6 +546,10 @@ int xq_grouped_fwd_infer(const xq_weight* gate, const xq_weight* up, const xq_we
                          const void* hidden, int64_t ld_hidden, int64_t n_tokens, const void* routing_w, int rw_dtype,
                          const int32_t* selected, int32_t topk, void* out, int64_t ld_out, void* workspace,
                          int64_t workspace_bytes, void* stream);
+int xq_grouped_fwd_infer_ids(const xq_weight* gate, const xq_weight* up, const xq_weight* down, const xq_grouped_lora* lora,
+                             const void* hidden, int64_t ld_hidden, int64_t n_tokens, const void* routing_w, int rw_dtype,
+                             const void* ids, int id_bytes, int32_t topk, void* out, int64_t ld_out, void* workspace,
+                             int64_t workspace_bytes, void* stream);
 
 /* ---- encoding a weight ----------------------------------------------------------
  * x [rows, cols] (bf16 or fp32, contiguous, 16-byte aligned) -> codes and scales of `format`, byte for byte what the

@@ -248,3 +248,21 @@ def test_decode_forward_many_experts_and_widest_topk(hip_device):
         ex = R.moe_fwd_bwd(x, rw, sel, banks["gate"], banks["up"], banks["down"], _lora_of(m), m.scaling)
         close(y, ex["y"], TOL)
         assert R.max_rel_err(y.float(), y_train.float()) <= SAME
+
+
+@pytest.mark.parametrize("T", [1, 4, 5, 16, 300])      # ids read by every kernel, behind the routing launch, and by the training forward's
+def test_expert_ids_of_either_width(hip_device, T):
+    """64-bit ids (a router's top-k) are read where they are: the result of the same ids in 32 bits, in any layout of them, with
+    ids that no expert has."""
+    E, topk = 16, 4
+    m, _ = _make_experts("nvfp4", E, 256, 512, 16, False, seed=T, device=hip_device)
+    rw, sel = _zipf_routing(T, E, topk, seed=T)
+    sel = sel.long().clone()
+    sel[0, 0], sel[-1, -1] = -1, E
+    x, rw = gen((T, 256), 1.0, 4, torch.bfloat16).to(hip_device), rw.to(torch.bfloat16).to(hip_device)
+    wide = torch.stack((sel, sel.flip(0)), 1).to(hip_device)[:, 0]                # rows that do not follow each other
+    for grad in (False, True):
+        with torch.set_grad_enabled(grad):
+            want = m(x, rw, sel.int().to(hip_device)).detach()
+            for ids in (sel.to(hip_device), wide, sel.t().contiguous().to(hip_device).t(), wide.int()):
+                assert torch.equal(m(x, rw, ids).detach(), want)

@@ -32,6 +32,13 @@ void xq_profile_mark_end(hipStream_t s);
 int64_t xq_packed_bytes_per_expert(const xq_weight* w);
 int64_t xq_scale_bytes_per_expert(const xq_weight* w);
 
+namespace xq {
+// xq_route_build over 32-bit ids (id_words 1) or the low words of 64-bit ones (2)
+int route_build(const int32_t* selected, int32_t id_words, int64_t n_routed, int32_t num_experts, int32_t* counts,
+                              int32_t* offsets, int32_t* scatter_index, int32_t* tile_offsets, void* workspace,
+                              int64_t workspace_bytes, void* stream_);
+}
+
 static inline int64_t xq_cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 static inline bool xq_aligned(const void* p, size_t a) { return ((uintptr_t)p % a) == 0; }
 

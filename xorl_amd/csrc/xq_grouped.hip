@@ -105,9 +105,9 @@ extern "C" int64_t xq_grouped_workspace_bytes(int64_t n_tokens, int32_t topk, in
     return backward ? bwd_workspace(d) : fwd_workspace(d);
 }
 
-extern "C" int xq_grouped_fwd(const xq_weight* gate, const xq_weight* up, const xq_weight* down, const xq_grouped_lora* lora,
+extern "C" int xq_grouped_fwd_ids(const xq_weight* gate, const xq_weight* up, const xq_weight* down, const xq_grouped_lora* lora,
                               const void* hidden, int64_t ld_hidden, int64_t n_tokens, const void* routing_w, int rw_dtype,
-                              const int32_t* selected, int32_t topk, void* out, int64_t ld_out,
+                              const void* ids, int id_bytes, int32_t topk, void* out, int64_t ld_out,
                               const xq_grouped_saved* saved, void* workspace, int64_t workspace_bytes, void* stream_) {
     static const char* who = "xq_grouped_fwd";
     Dims d;
@@ -116,7 +116,8 @@ extern "C" int xq_grouped_fwd(const xq_weight* gate, const xq_weight* up, const 
     XQ_REQUIRE(rw_dtype == XQ_DT_F32 || rw_dtype == XQ_DT_BF16, "%s: routing weights are fp32 or bf16", who);
     XQ_REQUIRE(workspace && xq_aligned(workspace, 256) && workspace_bytes >= fwd_workspace(d),
                "%s: workspace missing, misaligned or smaller than xq_grouped_workspace_bytes()", who);
-    XQ_REQUIRE(d.T == 0 || (hidden && routing_w && selected && out), "%s: NULL tensor", who);
+    XQ_REQUIRE(d.T == 0 || (hidden && routing_w && ids && out), "%s: NULL tensor", who);
+    XQ_REQUIRE(id_bytes == 4 || id_bytes == 8, "%s: expert ids of %d bytes", who, id_bytes);
     hipStream_t stream = (hipStream_t)stream_;
     const int E = d.E, rp = d.rp;
     const int64_t R = d.R, H = d.H, I = d.I;
@@ -126,7 +127,7 @@ extern "C" int xq_grouped_fwd(const xq_weight* gate, const xq_weight* up, const 
     void* route_ws = cv.take<uint8_t>(xq_route_workspace_bytes(R, E));
     const int64_t route_ws_bytes = al256(xq_route_workspace_bytes(R, E));
 
-    if ((rc = xq_route_build(selected, R, E, saved->counts, saved->offsets, saved->scatter_index, saved->tile_offsets,
+    if ((rc = route_build((const int32_t*)ids, id_bytes / 4, R, E, saved->counts, saved->offsets, saved->scatter_index, saved->tile_offsets,
                              route_ws, route_ws_bytes, stream)))
         return rc;
     if (R == 0) return XQ_OK;
@@ -210,6 +211,14 @@ extern "C" int xq_grouped_fwd(const xq_weight* gate, const xq_weight* up, const 
     }
     if ((rc = launch_tile_gemm(down, false, h, I, R, off, toff, su_d, Lr_dB, rp, nullptr, down_out, H, stream, who, nullptr, 0))) return rc;
     return xq_moe_gather(down_out, nullptr, H, saved->scatter_index, d.T, topk, H, out, ld_out, stream);
+}
+
+extern "C" int xq_grouped_fwd(const xq_weight* gate, const xq_weight* up, const xq_weight* down, const xq_grouped_lora* lora,
+                              const void* hidden, int64_t ld_hidden, int64_t n_tokens, const void* routing_w, int rw_dtype,
+                              const int32_t* selected, int32_t topk, void* out, int64_t ld_out,
+                              const xq_grouped_saved* saved, void* workspace, int64_t workspace_bytes, void* stream_) {
+    return xq_grouped_fwd_ids(gate, up, down, lora, hidden, ld_hidden, n_tokens, routing_w, rw_dtype, selected, 4, topk, out, ld_out, saved, workspace,
+                              workspace_bytes, stream_);
 }
 
 extern "C" int xq_grouped_bwd(const xq_weight* gate, const xq_weight* up, const xq_weight* down, const xq_grouped_lora* lora,

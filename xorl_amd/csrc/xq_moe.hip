@@ -88,7 +88,7 @@ constexpr int RB_CHUNK = 256;   // routed entries per block (one wave walks them
 constexpr int RB_MAX_E = 1024;
 
 // pass 1: per-chunk histogram
-__global__ void __launch_bounds__(64) route_hist_kernel(const int32_t* sel, int64_t n, int32_t E, int32_t* chunk_counts) {
+__global__ void __launch_bounds__(64) route_hist_kernel(const int32_t* sel, int32_t id_words, int64_t n, int32_t E, int32_t* chunk_counts) {
     __shared__ int32_t cnt[RB_MAX_E];
     for (int e = threadIdx.x; e < E; e += 64) cnt[e] = 0;
     __syncthreads();
@@ -96,7 +96,7 @@ __global__ void __launch_bounds__(64) route_hist_kernel(const int32_t* sel, int6
     for (int i = threadIdx.x; i < RB_CHUNK; i += 64) {
         int64_t idx = base + i;
         if (idx < n) {
-            int e = sel[idx];
+            int e = sel[idx * id_words];
             if (e >= 0 && e < E) atomicAdd(&cnt[e], 1);
         }
     }
@@ -192,7 +192,7 @@ __global__ void __launch_bounds__(1024) route_scan_kernel(int32_t* chunk_counts,
 // pass 3: stable position of every routed entry (one wave per chunk, in order).  The lanes of a 64-entry segment that
 // hold the same expert are found by intersecting, over the bits of the expert id, the ballots of "my value of
 // this bit"; a lane's position is the expert's running base plus the number of such lanes below it.
-__global__ void __launch_bounds__(64) route_place_kernel(const int32_t* sel, int64_t n, int32_t E, int32_t id_bits,
+__global__ void __launch_bounds__(64) route_place_kernel(const int32_t* sel, int32_t id_words, int64_t n, int32_t E, int32_t id_bits,
                                                          const int32_t* chunk_base, const int32_t* offsets,
                                                          int32_t* scatter_index) {
     __shared__ int32_t run[RB_MAX_E];
@@ -204,7 +204,7 @@ __global__ void __launch_bounds__(64) route_place_kernel(const int32_t* sel, int
     for (int seg = 0; seg < RB_CHUNK; seg += 64) {
         int64_t idx = base + seg + lane;
         bool valid = idx < n;
-        int e = valid ? sel[idx] : -1;
+        int e = valid ? sel[idx * id_words] : -1;
         if (e >= E) e = -1;
         uint64_t same = __ballot(e >= 0);
         for (int b = 0; b < id_bits; ++b) {
@@ -353,7 +353,8 @@ extern "C" int64_t xq_route_workspace_bytes(int64_t n_routed, int32_t num_expert
     return xq_cdiv(n_routed > 0 ? n_routed : 1, RB_CHUNK) * (int64_t)num_experts * 4;
 }
 
-extern "C" int xq_route_build(const int32_t* selected, int64_t n_routed, int32_t num_experts, int32_t* counts,
+// (id_words: 32-bit words from one id to the next, 1, or 2 for 64-bit ids, whose low words are read)
+int xq::route_build(const int32_t* selected, int32_t id_words, int64_t n_routed, int32_t num_experts, int32_t* counts,
                               int32_t* offsets, int32_t* scatter_index, int32_t* tile_offsets, void* workspace,
                               int64_t workspace_bytes, void* stream_) {
     XQ_REQUIRE(num_experts >= 1 && num_experts <= RB_MAX_E, "xq_route_build: num_experts %d out of range [1, %d]", num_experts, RB_MAX_E);
@@ -363,7 +364,7 @@ extern "C" int xq_route_build(const int32_t* selected, int64_t n_routed, int32_t
     hipStream_t stream = (hipStream_t)stream_;
     int32_t n_chunks = (int32_t)xq_cdiv(n_routed > 0 ? n_routed : 1, RB_CHUNK);
     int32_t* cc = (int32_t*)workspace;
-    route_hist_kernel<<<dim3(n_chunks), 64, 0, stream>>>(selected, n_routed, num_experts, cc);
+    route_hist_kernel<<<dim3(n_chunks), 64, 0, stream>>>(selected, id_words, n_routed, num_experts, cc);
     XQ_CHECK_LAUNCH("route_hist");
     static std::atomic<bool> scan_attr_set{false};   // the attribute call is idempotent: a race only repeats it
     if (!scan_attr_set) {
@@ -378,10 +379,16 @@ extern "C" int xq_route_build(const int32_t* selected, int64_t n_routed, int32_t
     if (n_routed > 0) {
         int id_bits = 0;
         while ((1 << id_bits) < num_experts) ++id_bits;
-        route_place_kernel<<<dim3(n_chunks), 64, 0, stream>>>(selected, n_routed, num_experts, id_bits, cc, offsets, scatter_index);
+        route_place_kernel<<<dim3(n_chunks), 64, 0, stream>>>(selected, id_words, n_routed, num_experts, id_bits, cc, offsets, scatter_index);
         XQ_CHECK_LAUNCH("route_place");
     }
     return XQ_OK;
+}
+
+extern "C" int xq_route_build(const int32_t* selected, int64_t n_routed, int32_t num_experts, int32_t* counts,
+                              int32_t* offsets, int32_t* scatter_index, int32_t* tile_offsets, void* workspace,
+                              int64_t workspace_bytes, void* stream_) {
+    return xq::route_build(selected, 1, n_routed, num_experts, counts, offsets, scatter_index, tile_offsets, workspace, workspace_bytes, stream_);
 }
 
 extern "C" int xq_moe_scatter(const void* in, int64_t ld_in, const int32_t* scatter_index, int64_t n_routed,

@@ -43,6 +43,8 @@ struct DecLists {
     int32_t R;
     const int32_t* selected;      // direct: [R] expert ids (NULL otherwise)
     int32_t E, topk;
+    int32_t id_words;             // 32-bit words from one id to the next: 1, or 2 for 64-bit ids, whose low words are read
+    __device__ __forceinline__ int id(int copy) const { return selected[copy * id_words]; }
     __host__ __device__ int32_t* unit() const { return base + 4; }
     __host__ __device__ int32_t* unit_token() const { return base + 4 + 4 * R; }
     __host__ __device__ int32_t* row_info() const { return base + 4 + 8 * R; }
@@ -50,7 +52,7 @@ struct DecLists {
     static int64_t bytes(int64_t R) { return (4 + 12 * R) * 4; }
 };
 
-__global__ void __launch_bounds__(512) decode_route_kernel(const int32_t* selected, int R, int E, int lg, int topk, int units_max, DecLists L) {
+__global__ void __launch_bounds__(512) decode_route_kernel(const int32_t* selected, int id_words, int R, int E, int lg, int topk, int units_max, DecLists L) {
     const int MR = 1 << lg;                          // rows per unit
     __shared__ int32_t s_tot[2];
     __shared__ __attribute__((aligned(16))) int32_t s_cnt[kDecMaxExperts], s_begin[kDecMaxExperts], s_unit[kDecMaxExperts];
@@ -58,7 +60,7 @@ __global__ void __launch_bounds__(512) decode_route_kernel(const int32_t* select
     for (int e = t; e < kDecMaxExperts; e += 512) s_cnt[e] = 0;
     int mine = -1;
     if (t < R) {
-        const int v = selected[t];
+        const int v = selected[t * id_words];
         mine = v >= 0 && v < E ? v : -1;             // ids outside [0, E) drop their copy
     }
     __syncthreads();
@@ -214,7 +216,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MR == 
     if (NF && tid < 64) nf4_tab[tid >> 4][tid & 15] = kNf4Level[tid & 15];    // ordered before its use by the barrier behind the x rows
     int4 unit;
     if (g.L.selected) {
-        const int v = g.L.selected[li];
+        const int v = g.L.id(li);
         unit = int4{v, li, v >= 0 && v < g.L.E ? 1 : 0, 0};
     } else {
         unit = *(const int4*)(g.L.unit() + 4 * li);
@@ -526,7 +528,7 @@ __global__ void __launch_bounds__(256) decode_mid_kernel(DecMid g) {
     const int rr = blockIdx.x, tid = threadIdx.x;
     int2 info;
     if (g.L.selected) {
-        const int v = g.L.selected[rr];
+        const int v = g.L.id(rr);
         info = int2{v >= 0 && v < g.L.E ? rr : -1, v};
     } else {
         info = *(const int2*)(g.L.row_info() + 2 * rr);
@@ -592,7 +594,7 @@ __global__ void __launch_bounds__(1024) decode_final_kernel(DecFinal g) {
         if (slot < g.topk) {
             const int p = t * g.topk + slot;
             if (g.L.selected) {
-                const int v = g.L.selected[p];
+                const int v = g.L.id(p);
                 info = int2{v >= 0 && v < g.L.E ? p : -1, v};
             } else {
                 info = *(const int2*)(g.L.pair_info() + 2 * p);
@@ -606,7 +608,7 @@ __global__ void __launch_bounds__(1024) decode_final_kernel(DecFinal g) {
         const int p = t * g.topk + slot;
         int rr;
         if (g.L.selected) {
-            const int v = g.L.selected[p];
+            const int v = g.L.id(p);
             rr = v >= 0 && v < g.L.E ? p : -1;
         } else {
             rr = g.L.pair_info()[2 * p];
@@ -738,10 +740,10 @@ extern "C" int64_t xq_grouped_infer_workspace_bytes(int64_t n_tokens, int32_t to
     return infer_workspace(n_tokens * topk, num_experts, hidden, intermediate, r_pad_of(r), rows_per_unit(n_tokens));
 }
 
-extern "C" int xq_grouped_fwd_infer(const xq_weight* gate, const xq_weight* up, const xq_weight* down, const xq_grouped_lora* lora,
-                                    const void* hidden, int64_t ld_hidden, int64_t n_tokens, const void* routing_w, int rw_dtype,
-                                    const int32_t* selected, int32_t topk, void* out, int64_t ld_out, void* workspace,
-                                    int64_t workspace_bytes, void* stream_) {
+extern "C" int xq_grouped_fwd_infer_ids(const xq_weight* gate, const xq_weight* up, const xq_weight* down, const xq_grouped_lora* lora,
+                                        const void* hidden, int64_t ld_hidden, int64_t n_tokens, const void* routing_w, int rw_dtype,
+                                        const void* ids, int id_bytes, int32_t topk, void* out, int64_t ld_out, void* workspace,
+                                        int64_t workspace_bytes, void* stream_) {
     static const char* who = "xq_grouped_fwd_infer";
     XQ_REQUIRE(gate && up && down && lora, "%s: NULL descriptor", who);
     int rc;
@@ -758,7 +760,10 @@ extern "C" int xq_grouped_fwd_infer(const xq_weight* gate, const xq_weight* up, 
                    "%s: a LoRA factor holds 1 (shared) or %d matrices", who, E);
     }
     XQ_REQUIRE(rw_dtype == XQ_DT_F32 || rw_dtype == XQ_DT_BF16, "%s: routing weights are fp32 or bf16", who);
-    XQ_REQUIRE(hidden && routing_w && selected && out, "%s: NULL tensor", who);
+    XQ_REQUIRE(hidden && routing_w && ids && out, "%s: NULL tensor", who);
+    XQ_REQUIRE(id_bytes == 4 || id_bytes == 8, "%s: expert ids of %d bytes", who, id_bytes);
+    const int32_t* selected = (const int32_t*)ids;
+    const int id_words = id_bytes / 4;
     const int64_t H = gate->rows, I = gate->cols, R = n_tokens * topk;
     XQ_REQUIRE(xq_aligned(hidden, 16) && (n_tokens == 1 || ld_hidden % 8 == 0) && ld_hidden >= H && ld_out >= H,
                "%s: rows of hidden must be 16-byte aligned; row strides at least the hidden size", who);
@@ -771,7 +776,7 @@ extern "C" int xq_grouped_fwd_infer(const xq_weight* gate, const xq_weight* up, 
     uint8_t* ws = (uint8_t*)workspace;
     int64_t used = 0;
     auto take = [&](int64_t bytes) { uint8_t* p = ws + used; used += al256(bytes); return p; };
-    DecLists L{(int32_t*)take(DecLists::bytes(R)), (int32_t)R, MR == 1 ? selected : nullptr, E, topk};
+    DecLists L{(int32_t*)take(DecLists::bytes(R)), (int32_t)R, MR == 1 ? selected : nullptr, E, topk, id_words};
     float* part_gu = (float*)take(2ll * pl.ns_gu * R * I * 4);
     float* su_gu = (float*)take(2ll * pl.ns_gu * R * rp * 4);
     bf16_t* h = (bf16_t*)take(R * I * 2);
@@ -779,7 +784,7 @@ extern "C" int xq_grouped_fwd_infer(const xq_weight* gate, const xq_weight* up, 
     float* su_d = (float*)take((int64_t)pl.ns_d * R * rp * 4);
 
     if (MR > 1) {
-        decode_route_kernel<<<dim3(1), 512, 0, stream>>>(selected, (int)R, E, 2, topk, pl.units, L);
+        decode_route_kernel<<<dim3(1), 512, 0, stream>>>(selected, id_words, (int)R, E, 2, topk, pl.units, L);
         XQ_CHECK_LAUNCH(who);
     }
 
@@ -827,4 +832,12 @@ extern "C" int xq_grouped_fwd_infer(const xq_weight* gate, const xq_weight* up, 
     decode_final_kernel<<<dim3((unsigned)n_tokens, (unsigned)(H / 256)), 1024, 0, stream>>>(fn);
     XQ_CHECK_LAUNCH(who);
     return XQ_OK;
+}
+
+extern "C" int xq_grouped_fwd_infer(const xq_weight* gate, const xq_weight* up, const xq_weight* down, const xq_grouped_lora* lora,
+                                    const void* hidden, int64_t ld_hidden, int64_t n_tokens, const void* routing_w, int rw_dtype,
+                                    const int32_t* selected, int32_t topk, void* out, int64_t ld_out, void* workspace,
+                                    int64_t workspace_bytes, void* stream) {
+    return xq_grouped_fwd_infer_ids(gate, up, down, lora, hidden, ld_hidden, n_tokens, routing_w, rw_dtype, selected, 4, topk, out, ld_out,
+                                    workspace, workspace_bytes, stream);
 }

@@ -757,7 +757,8 @@ PyObject* moe(PyObject*, PyObject* const* args, Py_ssize_t n) {
         const int r = (int)rank, rp = r_pad_of(r);
         const bool train = at::GradMode::is_enabled() && (x->requires_grad() || rw->requires_grad() || factor_grad);
         if (streaming && (train || !xq_grouped_infer_supported(&q[0].w, &q[1].w, &q[2].w, T, (int32_t)topk, r))) XQ_NONE;
-        Tensor ids = sel->scalar_type() == at::kInt && sel->is_contiguous() ? *sel : sel->detach().to(at::kInt).contiguous();
+        Tensor ids = sel->is_contiguous() ? *sel : sel->detach().contiguous();       // 64-bit ids as they are: a conversion would be a launch
+        const int id_bytes = (int)ids.element_size();
         Tensor w = rw->is_contiguous() ? *rw : rw->detach().contiguous();
         const int rw_code = w.scalar_type() == at::kFloat ? XQ_DT_F32 : XQ_DT_BF16;
         xq_grouped_lora L;
@@ -768,7 +769,7 @@ PyObject* moe(PyObject*, PyObject* const* args, Py_ssize_t n) {
             Scratch ws(xq_grouped_infer_workspace_bytes(T, (int32_t)topk, (int32_t)E, H, I, r));
             {
                 ReleaseGil nogil;
-                check(xq_grouped_fwd_infer(&q[0].w, &q[1].w, &q[2].w, &L, xr.ptr, xr.ld, T, w.data_ptr(), rw_code, (const int32_t*)ids.data_ptr(),
+                check(xq_grouped_fwd_infer_ids(&q[0].w, &q[1].w, &q[2].w, &L, xr.ptr, xr.ld, T, w.data_ptr(), rw_code, ids.data_ptr(), id_bytes,
                       (int32_t)topk, out.data_ptr(), H, ws.get(), ws.bytes, stream));
             }
             return THPVariable_Wrap(std::move(out));
@@ -784,7 +785,7 @@ PyObject* moe(PyObject*, PyObject* const* args, Py_ssize_t n) {
         Scratch ws(xq_grouped_workspace_bytes(T, (int32_t)topk, (int32_t)E, H, I, r, 0));
         {
             ReleaseGil nogil;
-            check(xq_grouped_fwd(&q[0].w, &q[1].w, &q[2].w, &L, xr.ptr, xr.ld, T, w.data_ptr(), rw_code, (const int32_t*)ids.data_ptr(),
+            check(xq_grouped_fwd_ids(&q[0].w, &q[1].w, &q[2].w, &L, xr.ptr, xr.ld, T, w.data_ptr(), rw_code, ids.data_ptr(), id_bytes,
                   (int32_t)topk, out.data_ptr(), H, &S, ws.get(), ws.bytes, stream));
         }
         if (!train) return THPVariable_Wrap(std::move(out));

@@ -810,3 +810,27 @@ def test_few_routed_rows_equal_the_same_rows_among_many(hip_device, H, I, r, few
 
     for a, b, tol in zip(run(few), run(T), (TOL, TOL, 2e-2)):          # (bf16 intermediates on both sides, as against the oracle)
         close(a, b[:few].double(), tol, rows="none")
+
+
+@pytest.mark.parametrize("fmt", ["nvfp4", "nf4"])
+@pytest.mark.parametrize("H,I", [(384, 640), (640, 128), (256, 384)])
+def test_two_4bit_banks_in_one_launch_equal_two_launches(hip_device, fmt, H, I):
+    """Gate and up side by side (widths in whole tiles of 128) against a launch each (384, 640 and 128 are no whole tiles of 256; of
+    256 and 384 one direction shares a launch either way): the same sums in the same order."""
+    from xorl_amd import _C
+
+    E, topk, T = 5, 2, 700
+    m, _ = _make_experts(fmt, E, H, I, 16, False, seed=H + I, device=hip_device)
+    rw, sel = _zipf_routing(T, E, topk, seed=4)
+    x, dy = gen((T, H), 1.0, 5, torch.bfloat16).to(hip_device), gen((T, H), 1.0, 6, torch.bfloat16).to(hip_device)
+    got = []
+    try:
+        for policy in (3, 2):
+            _C.check(_C.lib().xq_set_tile_policy(policy))
+            xd = x.clone().requires_grad_(True)
+            y = m(xd, rw.to(torch.bfloat16).to(hip_device), sel.to(hip_device))
+            got.append([y.detach(), *torch.autograd.grad(y, [xd, *m.get_lora_parameters()], dy)])
+    finally:
+        _C.check(_C.lib().xq_set_tile_policy(0))
+    for a, b in zip(*got):
+        assert torch.equal(a, b)

@@ -433,6 +433,21 @@ bool two_banks_supported(const xq_weight* w) {
     return w->format == XQ_FMT_FP8 && g_tile_policy != 1 && w->cols % 256 == 0 && w->cols >= 512 && w->num_experts >= 1;
 }
 
+// tile size of a grouped launch on the pipelined kernel
+static inline int bank_tile_size(int fmt, int64_t n_rows, int num_experts, int64_t Nout) {
+    return g_tile_policy == 2 ? 256 : g_tile_policy == 3 ? 128 : bank_large_tiles(fmt, n_rows, num_experts, Nout) ? 256 : 128;
+}
+
+// Whether two 4-bit banks of one shape and storage take one launch whose output holds both products side by side, ncols columns
+// each (G256Args::W2): whole column tiles per bank.  One bank's tiles leave half of the block slots empty at some hundreds of
+// routed rows and end in a round of their own beyond (routed MLP, two launches and one, us: nf4 32 experts 2560/1024, 800 rows, forward and backward 510 and 461; nvfp4 64 experts 2048/1024, 9000 rows 886 and 816, forward alone of 6000 rows 350 and 305).
+bool banks_side_by_side(const xq_weight* a, const xq_weight* b, int64_t ncols, int64_t n_rows) {
+    return a->format != XQ_FMT_FP8 && tile_gemm_takes_row_map(a) && tile_gemm_takes_row_map(b) && a->format == b->format &&
+           a->rows == b->rows && a->cols == b->cols && a->num_experts == b->num_experts && a->group == b->group &&
+           a->scale_dtype == b->scale_dtype && xq_packed_bytes_per_expert(a) % 16 == 0 && xq_aligned(a->packed, 16) && xq_aligned(b->packed, 16) &&
+           ncols % bank_tile_size(a->format, n_rows, a->num_experts, 2 * ncols) == 0;
+}
+
 // Whether the dgrad of two dense [N, K] weights of one shape may run as one launch (see launch_tile_gemm): block-fp8 on
 // the pipelined kernel, the change of matrix on a scale-block boundary and past the pipeline's prologue.
 bool two_dense_supported(const xq_weight* w) {
@@ -578,9 +593,10 @@ static int launch_tile_gemm_t(const xq_weight* w, bool contract_cols, const bf16
                        "%s: the dense two-matrix form is the dgrad of two block-fp8 weights (out_features %% 128 == 0, >= 512)", who);
             g.Kc *= 2;
         } else {
-            XQ_REQUIRE(two_banks_supported(w) && two_banks_supported(two->w2),
-                       "%s: a two-bank launch takes two block-fp8 expert banks (columns a multiple of 256)", who);
-            if (contract_cols) g.Kc *= 2;
+            XQ_REQUIRE((two_banks_supported(w) && two_banks_supported(two->w2)) || banks_side_by_side(w, two->w2, g.Nout, n_rows),
+                       "%s: a two-bank launch takes two block-fp8 expert banks (columns a multiple of 256) or two 4-bit ones (whole tiles)", who);
+            XQ_REQUIRE(xq_aligned(two->su2, 16) && xq_aligned(two->lora_right2, 16) && two->a_off2 % 8 == 0, "%s: the second bank's operands must be 16-byte aligned", who);
+            if (contract_cols && w->format == XQ_FMT_FP8) g.Kc *= 2;
             else g.Nout *= 2;
         }
     }
@@ -612,10 +628,9 @@ static int launch_tile_gemm_t(const xq_weight* w, bool contract_cols, const bf16
                              (grouped ? w->layout == XQ_LAYOUT_GKN && g.wcols % 16 == 0 && g.wrows >= 2 &&
                                             xq_aligned(w->scales, 16) && g.scale_stride % 16 == 0
                                       : w->layout == XQ_LAYOUT_FLAT));
-        const bool big = grouped && bank_large_tiles(w->format, n_rows, w->num_experts, g.Nout);
         const DensePlan plan = plan_dense(n_rows, g.Nout, g.Kc / BK);
         const bool planned = !grouped && fmt_ok && g_tile_policy == 0 && force_T == 0 && !two_dense;   // two matrices: one unsplit launch
-        const int T = force_T ? force_T : g_tile_policy == 2 ? 256 : g_tile_policy == 3 ? 128 : grouped ? (big ? 256 : 128) : plan.T;
+        const int T = force_T ? force_T : grouped ? bank_tile_size(w->format, n_rows, w->num_experts, g.Nout) : g_tile_policy == 2 ? 256 : g_tile_policy == 3 ? 128 : plan.T;
         MidPlan mid;
         const bool by_size = planned || (two_dense && g_tile_policy == 0);
         // (its storages: the formats' usual groups and scale types; 32-bit offsets from a base for the operands)
@@ -679,13 +694,14 @@ static int launch_tile_gemm_t(const xq_weight* w, bool contract_cols, const bf16
             int ksplit = grouped || two_dense ? 1 : force_T ? force_split : planned ? plan.split : ksplit_for(tiles_m * tiles_n, T, g.Kc / BK);
             if (ksplit > 1 && (!partial || !xq_aligned(partial, 16) || partial_bytes < (int64_t)ksplit * n_rows * g.Nout * 4)) ksplit = 1;
             f.ksplit = ksplit; f.partial = ksplit > 1 ? partial : nullptr;
-            f.W2 = nullptr; f.scales2 = nullptr; f.su2 = nullptr; f.lora_right2 = nullptr; f.ncols1 = 0; f.nk1 = 0;
+            f.W2 = nullptr; f.scales2 = nullptr; f.su2 = nullptr; f.lora_right2 = nullptr; f.ncols1 = 0; f.nk1 = 0; f.a_off2 = 0; f.global_scale2 = nullptr;
             f.ld_su = g.r_pad; f.H = nullptr; f.ldh = 0; f.bias2 = nullptr;
             f.wide_rows = xq_aligned(C, 16) && ldc % 8 == 0 && xq_aligned(bias, 8);
             if (two) {
                 f.W2 = (const uint8_t*)two->w2->packed; f.scales2 = (const uint8_t*)two->w2->scales;
                 f.su2 = g.r_pad ? two->su2 : nullptr; f.lora_right2 = g.r_pad ? two->lora_right2 : nullptr;
-                f.ncols1 = g.wcols; f.nk1 = (two_dense ? g.wrows : g.wcols) / BK;
+                f.ncols1 = contract_cols ? g.wrows : g.wcols; f.a_off2 = two->a_off2; f.global_scale2 = two->w2->global_scale;
+                f.nk1 = (two_dense ? g.wrows : g.wcols) / BK;
             }
             // (the kernel's own rule: large unsplit tiles, except the 4-bit expert banks)
             const bool persistent = T == 256 && ksplit == 1 && !(grouped && w->format != XQ_FMT_FP8);

@@ -90,16 +90,19 @@ struct G256Args {
     // sums to partial + s * M * Nout (row pitch Nout) instead of C, and split 0 carries the low-rank term and bias
     int32_t ksplit;
     float* partial;
-    // grouped block-fp8 launches over two banks of equal shape (gate and up of an expert MLP), W2 == NULL for one bank:
-    //   bank forward (!CONTRACT_COLS): the output is [rows, 2 * wcols]; column tiles from ncols1 on take the second
-    //     bank, its side term (su2, lora_right2) and write at their own columns -- both projections in one launch;
-    //   bank dgrad (CONTRACT_COLS): the contraction runs over 2 * wcols -- the first nk1 K-steps against the first
+    // grouped launches over two banks of equal shape (gate and up of an expert MLP), W2 == NULL for one bank:
+    //   bank forward (!CONTRACT_COLS), and the dgrad of 4-bit banks: the output holds both products side by side, ncols1
+    //     columns each; column tiles from ncols1 on take the second bank, its side term (su2, lora_right2), activations
+    //     a_off2 columns further right and write at their own columns -- both projections in one launch;
+    //   dgrad of block-fp8 banks (CONTRACT_COLS): the contraction runs over 2 * wcols -- the first nk1 K-steps against the first
     //     bank, the others against the second -- so dX = [dgate | dup] . [Wg ; Wu]^T leaves the kernel as one sum.
     const uint8_t* W2;
     const uint8_t* scales2;
     const bf16_t* su2;
     const bf16_t* lora_right2;
     int32_t ncols1, nk1;
+    int32_t a_off2;
+    const float* global_scale2;
     int64_t ld_su;             // row pitch of su / su2 in elements (>= r_pad)
     // gate / up / SwiGLU launch (template flag GU, dense block-fp8 forward): W is the gate weight, W2 the up weight, both
     // [Nout, Kc]; a tile holds 128 gate columns and the same 128 up columns, C is [M, 2 * Nout] (gate | up) and
@@ -491,8 +494,8 @@ __global__ void __launch_bounds__(2 * T, 2) gemm_256_kernel(G256Args g) {
         }
         __syncthreads();
     }
-    // two banks (grouped block-fp8 only): a forward block past the first bank's columns works on the second bank
-    constexpr bool TWO_OK = GROUPED && FMT == XQ_FMT_FP8;
+    // two banks side by side: a block past the first bank's columns works on the second bank
+    constexpr bool SIDE_BY_SIDE = GROUPED && (!CC || FMT != XQ_FMT_FP8);
     struct TileDesc {
         int e;                                          // expert (0 for a dense launch)
         int64_t row0, row_end;                          // first row of the tile, end of the rows it may read and write
@@ -501,6 +504,8 @@ __global__ void __launch_bounds__(2 * T, 2) gemm_256_kernel(G256Args g) {
         const uint8_t* Sb;
         const bf16_t* su_b;
         const bf16_t* lr_b;
+        const float* gs;                                // nvfp4: the global scales of its bank
+        int a_off;                                      // first activation column
     };
     auto describe = [&](int b, int round, TileDesc& t) -> bool {      // false: there is no such tile
         if (b >= nb || round >= MAX_ROUNDS) return false;
@@ -518,12 +523,17 @@ __global__ void __launch_bounds__(2 * T, 2) gemm_256_kernel(G256Args g) {
         }
         t.n0 = GU ? pid_n * (F8_BN / 2) : pid_n * F8_BN;      // GU: first gate (= up) column of the tile
         t.Wb = g.W; t.Sb = g.scales; t.su_b = g.su; t.lr_b = g.lora_right;
+        t.gs = g.global_scale;
+        t.a_off = 0;
         t.n0w = t.n0;
         t.bank_width = g.Nout;
-        if constexpr (TWO_OK) {
-            if (g.W2 != nullptr && !CC) {
+        if constexpr (SIDE_BY_SIDE) {
+            if (g.W2 != nullptr) {
                 t.bank_width = g.ncols1;
-                if (t.n0 >= g.ncols1) { t.Wb = g.W2; t.Sb = g.scales2; t.su_b = g.su2; t.lr_b = g.lora_right2; t.n0w = t.n0 - g.ncols1; }
+                if (t.n0 >= g.ncols1) {
+                    t.Wb = g.W2; t.Sb = g.scales2; t.su_b = g.su2; t.lr_b = g.lora_right2; t.n0w = t.n0 - g.ncols1;
+                    t.gs = g.global_scale2; t.a_off = g.a_off2;
+                }
             }
         }
         return true;
@@ -572,13 +582,13 @@ __global__ void __launch_bounds__(2 * T, 2) gemm_256_kernel(G256Args g) {
             if constexpr (GROUPED) {
                 if (g.a_rows) r = g.a_rows[r];
             }
-            a_src[p] = g.A + r * g.lda + (u & 7) * 8 + kt0 * F8_BK;
+            a_src[p] = g.A + r * g.lda + (u & 7) * 8 + kt0 * F8_BK + (SIDE_BY_SIDE && CC ? t.a_off : 0);
         }
 #pragma unroll
         for (int d = 0; d < PD; ++d) {
             if constexpr (GU) wls[d].init_gu(g, t.n0, tv);
             else wls[d].init(g, t.Wb + (int64_t)t.e * g.packed_stride, t.Sb + (int64_t)t.e * g.scale_stride,
-                             FMT == XQ_FMT_NVFP4 ? g.global_scale[t.e] : 1.0f, t.n0w, tv);
+                             FMT == XQ_FMT_NVFP4 ? t.gs[t.e] : 1.0f, t.n0w, tv);
             wls[d].tid = tid;            // the LDS addresses of its stores do not change from tile to tile
             if constexpr (FMT == XQ_FMT_NF4) wls[d].nf4_lds = nf4_levels;
         }

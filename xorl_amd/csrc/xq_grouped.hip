@@ -85,7 +85,8 @@ int64_t bwd_workspace(const Dims& d) {
            al256(d.R * d.rp * 2) + al256(d.R * 2 * d.rp * 2) + wg + 256;
 }
 
-// one launch for gate and up (forward) / one sum for their two dgrads: block-fp8 banks on the pipelined kernel
+// one sum for the two dgrads of gate and up: block-fp8 banks on the pipelined kernel.  (Their forwards as one launch: these banks,
+// and 4-bit banks where banks_side_by_side() says so, whose dgrads then share a launch too but stay two products.)
 bool fuse_gate_up(const xq_weight* gate, const xq_weight* up) { return two_banks_supported(gate) && two_banks_supported(up); }
 
 }  // namespace
@@ -193,8 +194,8 @@ extern "C" int xq_grouped_fwd_ids(const xq_weight* gate, const xq_weight* up, co
             return rc;
         if ((rc = launch_small_nt(xr, ld_xr, R, H, F_uA, rp, s, su_u, off, toff, E, uAe == 1, stream, 0, nullptr, 0, xr_rows, nullptr, 0))) return rc;
     }
-    if (fuse_gate_up(gate, up)) {       // both projections in one launch: column tiles past I take the up bank
-        const TwoBanks two{up, su_u, Lr_uB};
+    if (fuse_gate_up(gate, up) || banks_side_by_side(gate, up, I, R)) {       // both projections in one launch: column tiles past I take the up bank
+        const TwoBanks two{up, su_u, Lr_uB, 0};
         if ((rc = launch_tile_gemm(gate, false, xr, ld_xr, R, off, toff, su_g, Lr_gB, rp, nullptr, gu, 2 * I, stream, who, nullptr, 0, &two, nullptr, xr_rows, d.T))) return rc;
     } else {
         if ((rc = launch_tile_gemm(gate, false, xr, ld_xr, R, off, toff, su_g, Lr_gB, rp, nullptr, gu, 2 * I, stream, who, nullptr, 0, nullptr, nullptr, xr_rows, d.T))) return rc;
@@ -264,6 +265,7 @@ extern "C" int xq_grouped_bwd(const xq_weight* gate, const xq_weight* up, const 
     // low-rank terms ride as one side term of width 2 * rp)
     // (the A gradients then come from one pass over the rows too, which wants both A factors held the same way)
     const bool fused = fuse_gate_up(gate, up) && 2 * rp <= 64 && gAe == uAe;
+    const bool side = banks_side_by_side(gate, up, H, R);
     const int rp2 = 2 * rp;
 
     // every panel of the call in one launch: B factors [E|1, r, out] as the "down" panels [E|1, rp, out] of g . B^T,
@@ -283,7 +285,8 @@ extern "C" int xq_grouped_bwd(const xq_weight* gate, const xq_weight* up, const 
 
     bf16_t* g_down = cv.take<bf16_t>(R * H * 2);
     bf16_t* dx_g = cv.take<bf16_t>(R * H * 2);
-    bf16_t* dx_u = cv.take<bf16_t>(R * H * 2);
+    bf16_t* dx_u = cv.take<bf16_t>(R * H * 2);            // (behind dx_g: the two are one [R, 2 H] buffer where one launch writes both)
+    int64_t ld_dxr = H;
     bf16_t* dh = cv.take<bf16_t>(R * I * 2);
     bf16_t* dgu = cv.take<bf16_t>(R * 2 * I * 2);         // [R, 2I]: dgate | dup
     float* d_w_row = cv.take<float>(R * 4);
@@ -339,8 +342,13 @@ extern "C" int xq_grouped_bwd(const xq_weight* gate, const xq_weight* up, const 
     }
     if (d_routing && (rc = xq_moe_gather_scalar(d_w_row, sidx, R, d_routing, rw_dtype, stream))) return rc;
     if (fused) {
-        const TwoBanks two{up, nullptr, nullptr};
+        const TwoBanks two{up, nullptr, nullptr, 0};
         if ((rc = launch_tile_gemm(gate, true, dgu, 2 * I, R, off, toff, v_gu, Lr_guA, rp2, nullptr, dx_g, H, stream, who, nullptr, 0, &two))) return rc;
+    } else if (side) {        // rows of dx_g, then dx_u in each row of the buffer that holds both
+        const TwoBanks two{up, v_u, Lr_uA, (int32_t)I};
+        if ((rc = launch_tile_gemm(gate, true, dgu, 2 * I, R, off, toff, v_g, Lr_guA, rp, nullptr, dx_g, 2 * H, stream, who, nullptr, 0, &two))) return rc;
+        dx_u = dx_g + H;
+        ld_dxr = 2 * H;
     } else {
         if ((rc = launch_tile_gemm(up, true, dup, 2 * I, R, off, toff, v_u, Lr_uA, rp, nullptr, dx_u, H, stream, who, nullptr, 0))) return rc;
         if ((rc = launch_tile_gemm(gate, true, dgate, 2 * I, R, off, toff, v_g, Lr_guA, rp, nullptr, dx_g, H, stream, who, nullptr, 0))) return rc;
@@ -367,5 +375,5 @@ extern "C" int xq_grouped_bwd(const xq_weight* gate, const xq_weight* up, const 
     if (ne && (rc = launch_tn_grouped_multi(per_expert, ne, R, wg, off, E, stream))) return rc;
     if (ns && (rc = launch_tn_multi(shared, ns, R, wg, stream, n_valid))) return rc;
     if (!dx) return XQ_OK;
-    return xq_moe_gather(dx_g, fused ? nullptr : dx_u, H, sidx, d.T, topk, H, dx, ld_dx, stream);
+    return xq_moe_gather(dx_g, fused ? nullptr : dx_u, ld_dxr, sidx, d.T, topk, H, dx, ld_dx, stream);
 }

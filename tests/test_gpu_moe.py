@@ -834,3 +834,24 @@ def test_two_4bit_banks_in_one_launch_equal_two_launches(hip_device, fmt, H, I):
         _C.check(_C.lib().xq_set_tile_policy(0))
     for a, b in zip(*got):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("r", [8, 16, 20, 64])
+@pytest.mark.parametrize("hybrid,dtype", [(False, torch.float32), (True, torch.float32), (False, torch.bfloat16)])
+def test_factor_panels_by_pieces_equal_panels_by_elements(hip_device, r, hybrid, dtype):
+    """Factors at 16-byte aligned addresses are laid out as panels in pieces of four elements, the same factors one element further on
+    element by element: the same bits (ranks below, at and between the panel's 16; widths that are no multiple of a tile's 256)."""
+    E, T, topk, H, I = 3, 200, 2, 320, 576
+    m, _ = _make_experts("block_fp8", E, H, I, r, hybrid, seed=r, device=hip_device)
+    rw, sel = _zipf_routing(T, E, topk, seed=4)
+    x, dy = gen((T, H), 1.0, 5, torch.bfloat16).to(hip_device), gen((T, H), 1.0, 6, torch.bfloat16).to(hip_device)
+    got = []
+    for shift in (0, 1):
+        for p in m.get_lora_parameters():
+            moved = torch.empty(p.numel() + 8, dtype=dtype, device=hip_device)[shift:shift + p.numel()].view(p.shape)
+            p.data = moved.copy_(p.data)
+        xd = x.clone().requires_grad_(True)
+        y = m(xd, rw.to(torch.bfloat16).to(hip_device), sel.to(hip_device))
+        got.append([y.detach(), *torch.autograd.grad(y, [xd, *m.get_lora_parameters()], dy)])
+    for a, b in zip(*got):
+        assert torch.equal(a, b)

@@ -107,6 +107,85 @@ __global__ void __launch_bounds__(256) panel_prep_kernel(PanelJobs j) {
     }
 }
 
+// The same where four elements of a source row and of a destination row are one aligned piece (panel_vec): 16-byte loads of fp32
+// factors, 8-byte stores, and no LDS where nothing is transposed.  By single elements the kernel is bound by address arithmetic and
+// 2-byte stores, at half the rate of a copy.  Panels of 128 experts (hidden 2048, intermediate 768, r 16; 69 MB read, 35 written): 33 us by elements, 23 here;
+// 64 experts with factors shared by all on one side 15 and 8.
+template <bool F32>
+__global__ void __launch_bounds__(256) panel_prep_vec_kernel(PanelJobs j) {
+    __shared__ float tile[PP_L][PP_S + 1];
+    const int k = blockIdx.y, tid = threadIdx.x;
+    const int R_in = (int)j.R_in[k], C_in = (int)j.C_in[k], C_out = (int)j.C_out[k], R_out = (int)j.R_out[k];
+    const bool tr = j.transpose[k] != 0, wide = C_out >= R_out;
+    const int TRW = wide ? PP_S : PP_L, TCW = wide ? PP_L : PP_S;
+    const uint32_t tiles_c = (uint32_t)(C_out + TCW - 1) / TCW, per = (uint32_t)(R_out + TRW - 1) / TRW * tiles_c;
+    const uint32_t total = per * (uint32_t)j.n_out[k];
+    const bool load_long_first = wide != tr;
+    for (uint32_t t = blockIdx.x; t < total; t += gridDim.x) {
+        const uint32_t e = t / per, rem = t - e * per;
+        const int i0 = (int)(rem / tiles_c) * TRW, c0 = (int)(rem % tiles_c) * TCW;
+        const int64_t base = j.n_src[k] == 1 ? 0 : (int64_t)e * R_in * C_in;
+        bf16_t* out = j.out[k] + e * j.e_stride[k];
+        u32x4 val[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {            // (unconditional: a piece past the source is clamped onto it and dropped)
+            const int idx = u * 256 + tid;
+            const int l = load_long_first ? idx % 64 * 4 : idx / 4, sh = load_long_first ? idx / 64 : idx % 4 * 4;
+            const int i = i0 + (wide ? sh : l), c = c0 + (wide ? l : sh);
+            const int si = tr ? c : i, sj = tr ? i : c;
+            const int64_t src = base + (int64_t)min(si, R_in - 1) * C_in + min(sj, C_in - 4);
+            if (F32) {
+                val[u] = *(const u32x4*)((const float*)j.in[k] + src);
+            } else {
+                const u32x2 h = *(const u32x2*)((const bf16_t*)j.in[k] + src);
+                val[u] = u32x4{h[0] << 16, h[0] & 0xffff0000u, h[1] << 16, h[1] & 0xffff0000u};
+            }
+            const uint32_t keep = si < R_in && sj < C_in ? 0xffffffffu : 0u;
+            val[u] = u32x4{val[u][0] & keep, val[u][1] & keep, val[u][2] & keep, val[u][3] & keep};
+        }
+        auto put = [&](int l, int sh, float v0, float v1, float v2, float v3) {
+            const int i = i0 + (wide ? sh : l), c = c0 + (wide ? l : sh);
+            if (i < R_out && c < C_out) *(u32x2*)(out + (int64_t)i * j.pitch[k] + c) = u32x2{pack_bf16x2(v0, v1), pack_bf16x2(v2, v3)};
+        };
+        if (!tr) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int idx = u * 256 + tid;
+                put(wide ? idx % 64 * 4 : idx / 4, wide ? idx / 64 : idx % 4 * 4, __uint_as_float(val[u][0]), __uint_as_float(val[u][1]),
+                    __uint_as_float(val[u][2]), __uint_as_float(val[u][3]));
+            }
+            continue;
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int idx = u * 256 + tid;
+            const int l = load_long_first ? idx % 64 * 4 : idx / 4, sh = load_long_first ? idx / 64 : idx % 4 * 4;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) tile[load_long_first ? l + q : l][load_long_first ? sh : sh + q] = __uint_as_float(val[u][q]);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int idx = u * 256 + tid;
+            const int l = wide ? idx % 64 * 4 : idx / 4, sh = wide ? idx / 64 : idx % 4 * 4;
+            if (wide) put(l, sh, tile[l][sh], tile[l + 1][sh], tile[l + 2][sh], tile[l + 3][sh]);
+            else put(l, sh, tile[l][sh], tile[l][sh + 1], tile[l][sh + 2], tile[l][sh + 3]);
+        }
+        __syncthreads();
+    }
+}
+
+static bool panel_vec(const PanelJobs& j) {
+    for (int k = 0; k < j.n; ++k) {
+        const int64_t tiles = xq_cdiv(j.R_out[k], PP_S) * xq_cdiv(j.C_out[k], PP_S) * j.n_out[k];
+        if (j.C_in[k] % 4 || j.C_out[k] % 4 || j.pitch[k] % 4 || j.e_stride[k] % 4 || j.R_in[k] < 1 || j.C_in[k] < 4 || tiles >= (1ll << 31) ||
+            j.R_in[k] >= (1ll << 30) || j.C_in[k] >= (1ll << 30) || j.R_out[k] >= (1ll << 30) || j.C_out[k] >= (1ll << 30) ||
+            !xq_aligned(j.in[k], j.in_f32 ? 16 : 8) || !xq_aligned(j.out[k], 8))
+            return false;
+    }
+    return true;
+}
+
 int launch_panel_prep(const PanelJobs& j, hipStream_t stream) {
     int64_t most = 0;
     for (int k = 0; k < j.n; ++k) {
@@ -116,6 +195,12 @@ int launch_panel_prep(const PanelJobs& j, hipStream_t stream) {
     }
     if (j.n == 0 || most == 0) return XQ_OK;
     if (most > 16384) most = 16384;
+    if (panel_vec(j)) {
+        if (j.in_f32) panel_prep_vec_kernel<true><<<dim3((unsigned)most, (unsigned)j.n), 256, 0, stream>>>(j);
+        else panel_prep_vec_kernel<false><<<dim3((unsigned)most, (unsigned)j.n), 256, 0, stream>>>(j);
+        XQ_CHECK_LAUNCH("panel_prep");
+        return XQ_OK;
+    }
     if (j.in_f32) panel_prep_kernel<true><<<dim3((unsigned)most, (unsigned)j.n), 256, 0, stream>>>(j);
     else panel_prep_kernel<false><<<dim3((unsigned)most, (unsigned)j.n), 256, 0, stream>>>(j);
     XQ_CHECK_LAUNCH("panel_prep");

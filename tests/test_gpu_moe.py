@@ -855,3 +855,30 @@ def test_factor_panels_by_pieces_equal_panels_by_elements(hip_device, r, hybrid,
         got.append([y.detach(), *torch.autograd.grad(y, [xd, *m.get_lora_parameters()], dy)])
     for a, b in zip(*got):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("fmt", ["block_fp8", "nvfp4", "nf4"])
+@pytest.mark.parametrize("K,N,r", [(64, 192, 0), (192, 320, 16), (320, 128, 48)])      # one to five K-steps; ragged column tiles
+def test_few_row_tiles_equal_full_ones(hip_device, fmt, K, N, r):
+    """Tiles of at most 32 and 64 rows run with the waves side by side; their rows equal the same rows in a full tile bit for bit."""
+    from xorl_amd import moe_functional as MF
+
+    counts = [1, 31, 32, 33, 63, 64, 65, 0, 128 + 5]
+    E = len(counts)
+    m, _ = _make_experts(fmt, E, K, N, 8, False, seed=K + N, device=hip_device)
+    qw = m._bank("gate")
+    for transpose_w in (False, True):
+        kc, out = (N, K) if transpose_w else (K, N)
+        full = [3 * 128 if c > 128 else 128 for c in counts]
+        a_full = gen((sum(full), kc), 1.0, 7, torch.bfloat16).to(hip_device)
+        su_full = gen((sum(full), r), 1.0, 8, torch.bfloat16).to(hip_device) if r else None
+        right = gen((E, out, r), 0.05, 9, torch.bfloat16).to(hip_device) if r else None
+        starts = [sum(full[:e]) for e in range(E)]
+        pick = torch.cat([torch.arange(s, s + c) for s, c in zip(starts, counts)]).to(hip_device)
+        ys = []
+        for cnt, rows in ((counts, pick), (full, torch.arange(sum(full), device=hip_device))):
+            sel = torch.arange(E, dtype=torch.int32).repeat_interleave(torch.tensor(cnt)).reshape(-1, 1).to(hip_device)
+            _, offsets, _, tile_offsets = MF.route_build(sel, E)
+            su = su_full[rows].contiguous() if r else None
+            ys.append(MF._grouped_gemm(qw, transpose_w, a_full[rows].contiguous(), offsets, tile_offsets, su, right))
+        assert torch.equal(ys[0], ys[1][pick])

@@ -421,6 +421,171 @@ template <int FMT, bool CC, int T> struct W256Sel<FMT, CC, true, T> { using type
 template <bool CC, bool GROUPED, int T> struct W256Sel<XQ_FMT_FP8, CC, GROUPED, T> { using type = W256Fp8<CC, T>; };
 template <bool CC, int T> struct W256Sel<XQ_FMT_FP8, CC, true, T> { using type = W256Fp8<CC, T>; };
 
+// A tile of an expert bank with at most 32 RT (32 or 64) rows, by a block of the 128 x 128 kernel: the four waves side by side
+// along the columns, 32 each, instead of two by two, so that no wave reads or multiplies rows that are not there, and activations
+// of 32 RT rows only.  What a K-step costs in the full form is LDS reads (64 KB), matrix instructions (16 a wave) and the decode,
+// one behind the other in a block of one wave a SIMD; here 32 or 48 KB and 4 or 8, which leaves registers for PD K-steps in
+// flight.  The sums of an output are formed in the same order.
+// Routed MLP, full form and this, us: forward and backward nvfp4 128 experts 2048/768, 800 rows 613 and 478, nf4 32 experts
+// 2560/1024, 800 rows 452 and 402, nvfp4 64 experts 2048/1024, 9000 rows 802 and 787; forward alone fp8 64 experts, 1800 rows 206
+// and 188.  One K-step in flight: 514, 413, 780, 202; three: 498, 409, 787, 188.
+template <int FMT, bool CC, int RT, int PD>
+__device__ __forceinline__ void few_rows_tile(const G256Args& g, bf16_t* smem, const float* nf4_levels, const uint8_t* pk, const uint8_t* sc, float gscale,
+                                              int64_t row0, int64_t row_end, int n0, int n0w, int bank_width, const bf16_t* su,
+                                              const bf16_t* lr, int a_off) {
+    using G = Geo<128>;
+    using WL = typename W256Sel<FMT, CC, true, 128>::type;
+    constexpr int B_STAGE = CC ? G::B_STAGE_NT : G::B_STAGE_NN, A_STAGE = 32 * RT * F8_BK, NT = G::NT;
+    constexpr int OUT_P = 136;                      // row pitch of the finished tile in LDS
+    static_assert(32 * RT * OUT_P <= 2 * A_STAGE + 2 * B_STAGE && A_STAGE <= G::A_STAGE, "the stages hold the finished tile");
+    bf16_t *As = smem, *Bs = smem + 2 * A_STAGE;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int fr = lane & 31, fh = lane >> 5, nk = g.Kc / F8_BK, last = nk - 1;
+    const bf16_t* a_src[RT];
+    int a_dst[RT];
+#pragma unroll
+    for (int p = 0; p < RT; ++p) {
+        const int u = tid + p * NT;
+        int64_t r = row0 + (u >> 3);
+        r = r < row_end ? r : row_end - 1;
+        if (g.a_rows) r = g.a_rows[r];
+        a_src[p] = g.A + r * g.lda + (u & 7) * 8 + a_off;
+        a_dst[p] = swz(u >> 3, u & 7);
+    }
+    WL wls[PD];
+#pragma unroll
+    for (int d = 0; d < PD; ++d) {
+        wls[d].init(g, pk, sc, gscale, n0w, tid);
+        if constexpr (FMT == XQ_FMT_NF4) wls[d].nf4_lds = nf4_levels;
+    }
+    constexpr bool TWO_K = FMT == XQ_FMT_FP8 && CC;  // (as in the kernel below)
+    int64_t wdelta = 0, sdelta = 0;
+    int nk1 = 1 << 30;
+    if (TWO_K && g.W2 != nullptr) {
+        nk1 = g.nk1;
+        wdelta = (g.W2 - g.W) - (int64_t)nk1 * F8_BK;
+        sdelta = ((const float*)g.scales2 - (const float*)g.scales) - (int64_t)(nk1 >> 1);
+    }
+    u32x4 aregs[PD][RT];
+    auto load_a = [&](u32x4* a, int kt) {
+#pragma unroll
+        for (int p = 0; p < RT; ++p) a[p] = *(const u32x4*)(a_src[p] + kt * F8_BK);
+    };
+    auto store_a = [&](bf16_t* d, const u32x4* a) {
+#pragma unroll
+        for (int p = 0; p < RT; ++p) *(u32x4*)(d + a_dst[p]) = a[p];
+    };
+    f32x16 acc[RT];
+#pragma unroll
+    for (int i = 0; i < RT; ++i)
+#pragma unroll
+        for (int q = 0; q < 16; ++q) acc[i][q] = 0.0f;
+    bf16x8 af0[RT], af1[RT], bf0, bf1;
+    auto load_frags = [&](const bf16_t* a, const bf16_t* b, int ks, bool b_is_nt, bf16x8* af, bf16x8& bfr) {
+#pragma unroll
+        for (int i = 0; i < RT; ++i) af[i] = *(const bf16x8*)(a + swz(i * 32 + fr, ks * 2 + fh));
+        if (CC || b_is_nt) bfr = *(const bf16x8*)(b + swz(wave * 32 + fr, ks * 2 + fh));
+        else bfr = lds_tr_frag(b, G::NN_PITCH, ks * 16, wave * 32, lane);
+    };
+    auto mma = [&](const bf16x8* af, const bf16x8& bfr) {
+#pragma unroll
+        for (int i = 0; i < RT; ++i) acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bfr, af[i], acc[i], 0, 0, 0);
+    };
+    // (the kernel's pipeline: tile kt + 1 is stored while tile kt is multiplied, one barrier a K-step ahead of the last MFMAs)
+    auto iteration = [&](int kt, u32x4* areg, WL& wl, int kload) {
+        const bf16_t *a = As + (kt & 1) * A_STAGE, *b = Bs + (kt & 1) * B_STAGE;
+        bf16_t *an = As + ((kt + 1) & 1) * A_STAGE, *bn = Bs + ((kt + 1) & 1) * B_STAGE;
+        load_frags(a, b, 1, false, af1, bf1);
+        mma(af0, bf0);
+        store_a(an, areg);
+        load_a(areg, kload);
+        __builtin_amdgcn_sched_barrier(0);
+        wl.store(bn, 0);
+        wl.store(bn, 1);
+        mma(af1, bf1);
+        if constexpr (TWO_K) {
+            if (kload >= nk1 && kload - PD < nk1) wl.rebase(wdelta, sdelta);
+        }
+        wl.load(kload);
+        load_frags(a, b, 2, false, af0, bf0);
+        load_frags(a, b, 3, false, af1, bf1);
+        __builtin_amdgcn_sched_barrier(0);
+        mma(af0, bf0);
+        __syncthreads();
+        load_frags(an, bn, 0, false, af0, bf0);
+        mma(af1, bf1);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    load_a(aregs[0], 0);
+    wls[0].load(0);
+    // (set PD % PD = 0 is refilled once tile 0 is stored; every load is unconditional, past the end the last tile again)
+#pragma unroll
+    for (int d = 1; d < PD; ++d) { load_a(aregs[d], min(d, last)); wls[d].load(min(d, last)); }
+    store_a(As, aregs[0]);
+    wls[0].store(Bs, 0);
+    wls[0].store(Bs, 1);
+    load_a(aregs[0], min(PD, last));
+    wls[0].load(min(PD, last));
+    __syncthreads();
+    load_frags(As, Bs, 0, false, af0, bf0);
+    int kt = 0;
+    for (; kt + PD <= nk; kt += PD) {
+#pragma unroll
+        for (int d = 0; d < PD; ++d) iteration(kt + d, aregs[(d + 1) % PD], wls[(d + 1) % PD], min(kt + d + 1 + PD, last));
+    }
+#pragma unroll
+    for (int d = 0; d < PD - 1; ++d)
+        if (kt + d < nk) iteration(kt + d, aregs[(d + 1) % PD], wls[(d + 1) % PD], last);
+
+    // ---- low-rank side term, both [row][k] tiles in stage 0
+    if (g.r_pad > 0) {
+        const int rp = g.r_pad, cpr = rp >> 3;
+        for (int idx = tid; idx < G::BN * cpr; idx += NT) {
+            const int r = idx / cpr, c = idx - r * cpr;
+            if (r < 32 * RT) {
+                const int64_t row = row0 + r < row_end ? row0 + r : row_end - 1;
+                *(u32x4*)(As + swz(r, c)) = *(const u32x4*)(su + row * g.ld_su + c * 8);
+            }
+            const int n = min(n0w + r, bank_width - 1);
+            *(u32x4*)(Bs + swz(r, c)) = *(const u32x4*)(lr + (int64_t)n * rp + c * 8);
+        }
+        __syncthreads();
+        for (int ks = 0; ks < (rp >> 4); ++ks) {
+            load_frags(As, Bs, ks, true, af0, bf0);
+            mma(af0, bf0);
+        }
+    }
+    // ---- the finished tile: lane fr of a wave holds row fr and 4 x 4 consecutive columns.  Through LDS it leaves in 256-byte rows.
+    if (!g.wide_rows) {
+#pragma unroll
+        for (int i = 0; i < RT; ++i) {
+            const int64_t row = row0 + i * 32 + fr;
+            if (row >= row_end) continue;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int n = n0 + wave * 32 + 8 * q + 4 * fh;
+                if (n < g.Nout)
+                    *(u32x2*)(g.C + row * g.ldc + n) = u32x2{pack_bf16x2(acc[i][4 * q], acc[i][4 * q + 1]), pack_bf16x2(acc[i][4 * q + 2], acc[i][4 * q + 3])};
+            }
+        }
+        return;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < RT; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            *(u32x2*)(smem + (i * 32 + fr) * OUT_P + wave * 32 + 8 * q + 4 * fh) =
+                u32x2{pack_bf16x2(acc[i][4 * q], acc[i][4 * q + 1]), pack_bf16x2(acc[i][4 * q + 2], acc[i][4 * q + 3])};
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < 2 * RT; ++t) {
+        const int rl = t * 16 + (tid >> 4), n = n0 + (tid & 15) * 8;
+        if (row0 + rl < row_end && n < g.Nout) *(u32x4*)(g.C + (row0 + rl) * g.ldc + n) = *(const u32x4*)(smem + rl * OUT_P + (tid & 15) * 8);
+    }
+}
+
 // ---------------------------------------------------------------- the kernel
 template <int FMT, bool CC, bool GROUPED, int T, bool SPLIT256 = false, bool GU = false>
 __global__ void __launch_bounds__(2 * T, 2) gemm_256_kernel(G256Args g) {
@@ -691,6 +856,17 @@ __global__ void __launch_bounds__(2 * T, 2) gemm_256_kernel(G256Args g) {
     TileDesc cur;
     int vb = (int)blockIdx.x, round = 0;
     if (!describe(vb, 0, cur)) return;
+    if constexpr (GROUPED && T == 128) {
+        const int64_t rows = cur.row_end - cur.row0;
+        if (rows <= 64 && g.bias == nullptr) {
+            const uint8_t *pk = cur.Wb + (int64_t)cur.e * g.packed_stride, *sc = cur.Sb + (int64_t)cur.e * g.scale_stride;
+            const float gscale = FMT == XQ_FMT_NVFP4 ? cur.gs[cur.e] : 1.0f;
+            const bf16_t* lr = cur.lr_b + (int64_t)cur.e * cur.bank_width * g.r_pad;
+            if (rows <= 32) few_rows_tile<FMT, CC, 1, 2>(g, smem, nf4_levels, pk, sc, gscale, cur.row0, cur.row_end, cur.n0, cur.n0w, cur.bank_width, cur.su_b, lr, cur.a_off);
+            else few_rows_tile<FMT, CC, 2, 2>(g, smem, nf4_levels, pk, sc, gscale, cur.row0, cur.row_end, cur.n0, cur.n0w, cur.bank_width, cur.su_b, lr, cur.a_off);
+            return;
+        }
+    }
     aim(cur);
     load_a(aregs[0], 0);
     wls[0].load(kt0);

@@ -298,121 +298,147 @@ struct W256Flat4 {
 };
 
 // 4-bit GKN matrix of an expert bank, [wrows = K, wcols = N]: byte (k / 2, n) holds rows k (low nibble) and
-// k + 1 (high nibble) of column n; one scale per `group` rows per column, [K / group][N].  A thread owns one
-// 16-byte piece per K-step -- 16 consecutive columns of one row pair, i.e. two 16-code runs that share their bytes
-// and their 16 scales.
-//   !CC (bank forward, contraction along K): pair t / RPR of the K-step's 32 row pairs, columns n0 + (t % RPR) * 16;
-//   CC (bank dgrad, contraction along N): rows n0 + 2 * (t >> 2), columns k0 + (t & 3) * 16.
+// k + 1 (high nibble) of column n; one scale per `group` rows per column, [K / group][N].  A thread owns 32 codes of a K-step
+// that share few scales:
+//   !CC (bank forward, contraction along K): four columns n0 + (t % (T / 4)) * 4 of the eight rows 8 * (t / (T / 4)) ..;
+//   CC (bank dgrad, contraction along N): eight columns k0 + (t & 7) * 8 of the four rows n0 + 4 * (t >> 3) ...
+// (rows within one group, which are 16 or more.)  Sixteen columns of one row pair a thread, the other way to deal them, are one
+// load of codes but four of scales, the same scales for every pair of a group, 16 registers of them and 16 conversions.  Routed MLP,
+// that way and this, us: forward and backward nvfp4 128 experts 2048/768, 800 rows 478 and 441, 131072 rows 4609 and 4530, 64 experts
+// 2048/1024, 24000 rows 1418 and 1370; nf4 8 experts 4096/1536, 4000 rows 802 and 786; forward alone nvfp4 6000 rows 297 and 280.
 template <int FMT, bool CC, int T>
 struct W256Gkn4 {
+    static constexpr int NP = CC ? 2 : 4, NC = CC ? 8 : 4;       // row pairs and columns of a thread
     const uint8_t* src;
     const uint8_t* sc_base;
     int64_t kstep;           // bytes per K-step
-    int32_t wcols, row, col; // !CC: first row of the pair within the K-step; CC: global row of the pair; first column at K-step 0
+    int32_t pitch1;          // bytes from a row pair to the next (CC: 0 past the matrix)
+    int32_t wcols, row, col; // !CC: first row within the K-step; CC: global first row; first column (CC: at K-step 0)
     int gshift, sdt, tid;
     float gs;
     const float* nf4_lds;
-    u32x4 raw;
-    u32x4 s0, s1, s2, s3;    // 16 scales: 4 / 2 / 1 registers of them for fp32 / bf16 / e4m3 storage
+    uint32_t raw[NP * NC / 4];
+    u32x4 s0, s1;            // the scales' 16-byte pieces (narrow storages: the piece that holds them)
     __device__ __forceinline__ void init(const G256Args& g, const uint8_t* pk, const uint8_t* sc, float gscale, int n0, int tid_) {
         tid = tid_; gshift = g.gshift; sdt = g.scale_dtype; gs = gscale; sc_base = sc; nf4_lds = nullptr; wcols = g.wcols;
         if (CC) {
-            row = min(n0 + 2 * (tid >> 2), g.wrows - 2);
-            col = (tid & 3) * 16;
-            src = pk + (int64_t)(row >> 1) * g.wcols + col;
+            row = min(n0 + 4 * (tid >> 3), g.wrows - 2);
+            col = (tid & 7) * 8;
+            pitch1 = row + 2 < g.wrows ? g.wcols : 0;
             kstep = F8_BK;
         } else {
-            row = 2 * (tid / Geo<T>::RPR);
-            col = min(n0 + (tid % Geo<T>::RPR) * 16, g.wcols - 16);
-            src = pk + (int64_t)(row >> 1) * g.wcols + col;
+            row = 8 * (tid / (T / 4));
+            col = min(n0 + (tid % (T / 4)) * 4, g.wcols - 4);
+            pitch1 = g.wcols;
             kstep = (int64_t)(F8_BK / 2) * g.wcols;
         }
+        src = pk + (int64_t)(row >> 1) * g.wcols + col;
     }
     __device__ __forceinline__ void load(int kt) {
-        raw = *(const u32x4*)(src + kt * kstep);
+        const uint8_t* p = src + kt * kstep;
+#pragma unroll
+        for (int i = 0; i < NP; ++i) {
+            if (CC) {
+                const u32x2 v = *(const u32x2*)(p + i * pitch1);
+                raw[2 * i] = v[0]; raw[2 * i + 1] = v[1];
+            } else {
+                raw[i] = *(const uint32_t*)(p + i * pitch1);
+            }
+        }
         const int64_t si = CC ? (int64_t)(row >> gshift) * wcols + col + kt * F8_BK
                               : (int64_t)((kt * F8_BK + row) >> gshift) * wcols + col;
-        // unconditional loads of what the widest storage needs (narrower storages read the same piece again:
-        // cache hits), so that the four registers are plain values and the waits count exactly
+        // unconditional loads whatever the storage, so that the registers are plain values and the waits count exactly (rows of
+        // scales start 16-byte aligned: the piece is inside them)
         const int esz = sdt == XQ_SCALE_F32 ? 4 : sdt == XQ_SCALE_BF16 ? 2 : 1;
-        const uint8_t* sp = sc_base + si * esz;
-        const int q1 = esz >= 2 ? 16 : 0, q2 = esz == 4 ? 32 : 0, q3 = esz == 4 ? 48 : 0;
+        const uint8_t* sp = sc_base + ((si * esz) & ~(int64_t)15);
         s0 = *(const u32x4*)sp;
-        s1 = *(const u32x4*)(sp + q1);
-        s2 = *(const u32x4*)(sp + q2);
-        s3 = *(const u32x4*)(sp + q3);
+        if (CC) s1 = *(const u32x4*)(sp + (esz == 4 ? 16 : 0));
     }
-    // both rows of the pair in one pass over the 16 columns, four at a time: scales and decoded values live only
-    // until they are packed
+    // the NC scales as fp32
     template <int SDT>
-    __device__ __forceinline__ void store_both(bf16_t* b) {
-        uint32_t ev[8], od[8];                       // packed bf16 pairs of the even / the odd row
+    __device__ __forceinline__ void scales(float* sc) const {
+        if (SDT == XQ_SCALE_F32) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {                // code dword q: columns 4q .. 4q + 3
-            float sc[4];
-            if (SDT == XQ_SCALE_F32) {
-                const u32x4& f = q == 0 ? s0 : q == 1 ? s1 : q == 2 ? s2 : s3;
+            for (int c = 0; c < NC; ++c) sc[c] = __uint_as_float(c < 4 ? s0[c] : s1[c - 4]);
+        } else if (SDT == XQ_SCALE_BF16) {
+            // 8 scales to a piece: all of them (CC), or the half that column col starts
+            const bool hi = !CC && (col & 4);
 #pragma unroll
-                for (int c = 0; c < 4; ++c) sc[c] = __uint_as_float(f[c]);
-            } else if (SDT == XQ_SCALE_BF16) {
-                const u32x4& h = q < 2 ? s0 : s1;
-                const uint32_t d0 = h[(2 * q) & 3], d1 = h[((2 * q) & 3) + 1];
-                sc[0] = __uint_as_float(d0 << 16); sc[1] = __uint_as_float(d0 & 0xffff0000u);
-                sc[2] = __uint_as_float(d1 << 16); sc[3] = __uint_as_float(d1 & 0xffff0000u);
-            } else {
-                const f32x2 lo = e4m3x2_to_f32(s0[q], false), hi = e4m3x2_to_f32(s0[q], true);
-                sc[0] = lo[0]; sc[1] = lo[1]; sc[2] = hi[0]; sc[3] = hi[1];
+            for (int c = 0; c < NC; c += 2) {
+                const uint32_t d = CC ? s0[c / 2] : hi ? s0[2 + c / 2] : s0[c / 2];
+                sc[c] = __uint_as_float(d << 16);
+                sc[c + 1] = __uint_as_float(d & 0xffff0000u);
             }
-            if (FMT == XQ_FMT_NVFP4) {
-#pragma unroll
-                for (int c = 0; c < 4; ++c) sc[c] = sc[c] * gs;
-            }
-            const uint32_t w = raw[q];
-            float e[4], o[4];
-            if (FMT == XQ_FMT_NVFP4) {
-                const f32x2 x0 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 0), x1 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 1);
-                const f32x2 x2 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 2), x3 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 3);
-                e[0] = x0[0] * sc[0]; o[0] = x0[1] * sc[0]; e[1] = x1[0] * sc[1]; o[1] = x1[1] * sc[1];
-                e[2] = x2[0] * sc[2]; o[2] = x2[1] * sc[2]; e[3] = x3[0] * sc[3]; o[3] = x3[1] * sc[3];
-            } else if (FMT == XQ_FMT_INT4) {
-                const uint32_t lo = w & 0x0f0f0f0fu, hi = (w >> 4) & 0x0f0f0f0fu;
-#pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    const float m8s = -8.0f * sc[c];
-                    e[c] = __builtin_fmaf((float)((lo >> (8 * c)) & 0xffu), sc[c], m8s);
-                    o[c] = __builtin_fmaf((float)((hi >> (8 * c)) & 0xffu), sc[c], m8s);
-                }
-            } else {
-#pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    e[c] = nf4_lds[(w >> (8 * c)) & 0xfu] * sc[c];
-                    o[c] = nf4_lds[(w >> (8 * c + 4)) & 0xfu] * sc[c];
-                }
-            }
-            ev[2 * q] = pack_bf16x2(e[0], e[1]); ev[2 * q + 1] = pack_bf16x2(e[2], e[3]);
-            od[2 * q] = pack_bf16x2(o[0], o[1]); od[2 * q + 1] = pack_bf16x2(o[2], o[3]);
-        }
-        const u32x4 elo = {ev[0], ev[1], ev[2], ev[3]}, ehi = {ev[4], ev[5], ev[6], ev[7]};
-        const u32x4 olo = {od[0], od[1], od[2], od[3]}, ohi = {od[4], od[5], od[6], od[7]};
-        if (CC) {
-            const int u = 2 * (tid >> 2) * 4 + (tid & 3);
-            store_run16<true, T>(b, u, elo, ehi);
-            store_run16<true, T>(b, u + 4, olo, ohi);
         } else {
-            bf16_t* d = b + row * Geo<T>::NN_PITCH + (tid % Geo<T>::RPR) * 16;
-            *(u32x4*)d = elo;
-            *(u32x4*)(d + 8) = ehi;
-            *(u32x4*)(d + Geo<T>::NN_PITCH) = olo;
-            *(u32x4*)(d + Geo<T>::NN_PITCH + 8) = ohi;
+            // 16 to a piece: the half or the quarter that column col starts
+#pragma unroll
+            for (int c = 0; c < NC; c += 4) {
+                const uint32_t h0 = col & 8 ? s0[2] : s0[0], h1 = col & 8 ? s0[3] : s0[1];
+                const uint32_t d = CC ? (c ? h1 : h0) : col & 4 ? h1 : h0;
+                const f32x2 a = e4m3x2_to_f32(d, false), b = e4m3x2_to_f32(d, true);
+                sc[c] = a[0]; sc[c + 1] = a[1]; sc[c + 2] = b[0]; sc[c + 3] = b[1];
+            }
+        }
+        if (FMT == XQ_FMT_NVFP4) {
+#pragma unroll
+            for (int c = 0; c < NC; ++c) sc[c] = sc[c] * gs;
+        }
+    }
+    // four columns of a row pair -> packed bf16 pairs of the even and of the odd row
+    __device__ __forceinline__ void decode4(uint32_t w, const float* sc, uint32_t* ev, uint32_t* od) const {
+        float e[4], o[4];
+        if (FMT == XQ_FMT_NVFP4) {
+            const f32x2 x0 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 0), x1 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 1);
+            const f32x2 x2 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 2), x3 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 3);
+            e[0] = x0[0] * sc[0]; o[0] = x0[1] * sc[0]; e[1] = x1[0] * sc[1]; o[1] = x1[1] * sc[1];
+            e[2] = x2[0] * sc[2]; o[2] = x2[1] * sc[2]; e[3] = x3[0] * sc[3]; o[3] = x3[1] * sc[3];
+        } else if (FMT == XQ_FMT_INT4) {
+            const uint32_t lo = w & 0x0f0f0f0fu, hi = (w >> 4) & 0x0f0f0f0fu;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const float m8s = -8.0f * sc[c];
+                e[c] = __builtin_fmaf((float)((lo >> (8 * c)) & 0xffu), sc[c], m8s);
+                o[c] = __builtin_fmaf((float)((hi >> (8 * c)) & 0xffu), sc[c], m8s);
+            }
+        } else {
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                e[c] = nf4_lds[(w >> (8 * c)) & 0xfu] * sc[c];
+                o[c] = nf4_lds[(w >> (8 * c + 4)) & 0xfu] * sc[c];
+            }
+        }
+        ev[0] = pack_bf16x2(e[0], e[1]); ev[1] = pack_bf16x2(e[2], e[3]);
+        od[0] = pack_bf16x2(o[0], o[1]); od[1] = pack_bf16x2(o[2], o[3]);
+    }
+    template <int SDT>
+    __device__ __forceinline__ void store_all(bf16_t* b) {
+        float sc[NC];
+        scales<SDT>(sc);
+#pragma unroll
+        for (int i = 0; i < NP; ++i) {
+            if (CC) {
+                uint32_t ev[4], od[4];
+                decode4(raw[2 * i], sc, ev, od);
+                decode4(raw[2 * i + 1], sc + 4, ev + 2, od + 2);
+                const int r = 4 * (tid >> 3) + 2 * i;
+                *(u32x4*)(b + swz(r, tid & 7)) = u32x4{ev[0], ev[1], ev[2], ev[3]};
+                *(u32x4*)(b + swz(r + 1, tid & 7)) = u32x4{od[0], od[1], od[2], od[3]};
+            } else {
+                uint32_t ev[2], od[2];
+                decode4(raw[i], sc, ev, od);
+                bf16_t* d = b + (8 * (tid / (T / 4)) + 2 * i) * Geo<T>::NN_PITCH + (tid % (T / 4)) * 4;
+                *(u32x2*)d = u32x2{ev[0], ev[1]};
+                *(u32x2*)(d + Geo<T>::NN_PITCH) = u32x2{od[0], od[1]};
+            }
         }
     }
     __device__ __forceinline__ void rebase(int64_t, int64_t) {}
     // the kernel stores a thread's two runs one after the other: the first call does both
     __device__ __forceinline__ void store(bf16_t* b, int p) {
         if (p != 0) return;
-        if (sdt == XQ_SCALE_F32) store_both<XQ_SCALE_F32>(b);
-        else if (sdt == XQ_SCALE_BF16) store_both<XQ_SCALE_BF16>(b);
-        else store_both<XQ_SCALE_E4M3>(b);
+        if (sdt == XQ_SCALE_F32) store_all<XQ_SCALE_F32>(b);
+        else if (sdt == XQ_SCALE_BF16) store_all<XQ_SCALE_BF16>(b);
+        else store_all<XQ_SCALE_E4M3>(b);
     }
 };
 

@@ -6,6 +6,7 @@ import torch
 
 from oracle import cdecode as C
 from oracle import decode_np as NP
+from tests.util_cases import gen
 
 pytestmark = pytest.mark.gpu
 
@@ -194,3 +195,27 @@ def test_errors_and_empty(hip_device):
     out = Q.block_fp8_dequantize_gkn(torch.empty(0, 128, dtype=torch.float8_e4m3fn, device=hip_device),
                                      torch.empty(0, 1, device=hip_device))
     assert out.shape == (0, 128)
+
+
+@pytest.mark.parametrize("fmt", ["nvfp4", "nf4", "int4"])
+@pytest.mark.parametrize("K,N", [(64, 16), (192, 48)])
+def test_gkn_decode_reads_scales_wherever_they_lie(hip_device, fmt, K, N):
+    """Scales that start 16-byte aligned are read in pieces, others one by one: the same bits."""
+    from xorl_amd import quantize as Q
+
+    w = gen((K, N), 0.05, K)
+    if fmt == "nvfp4":
+        packed, scales, g = Q.nvfp4_quantize_gkn(w.to(hip_device))
+        decode = lambda s: Q.nvfp4_dequantize_gkn(packed, s, g, K, N)
+    elif fmt == "nf4":
+        packed, scales = Q.nf4_quantize_gkn(w.to(hip_device))
+        decode = lambda s: Q.nf4_dequantize_gkn(packed, s, K, N)
+    else:
+        packed, scales = (t.to(hip_device) for t in Q.int4_quantize_gkn(w, 32))
+        scales = scales.to(torch.bfloat16)
+        decode = lambda s: Q.int4_dequantize_gkn(packed, s, K, N, 32)
+    flat = torch.empty(scales.numel() + 1, dtype=scales.dtype, device=hip_device)
+    flat[1:].copy_(scales.reshape(-1))
+    moved = flat[1:].view(scales.shape)
+    assert scales.data_ptr() % 16 == 0 and moved.data_ptr() % 16 != 0
+    assert torch.equal(decode(scales), decode(moved))

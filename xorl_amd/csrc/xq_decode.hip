@@ -17,6 +17,7 @@ struct DecodeArgs {
     int64_t rows, cols;
     int64_t packed_stride, scale_stride;  // bytes per expert
     int32_t group, scale_dtype;
+    int32_t wide_scales;   // GKN: 16 scales of a row start 16-byte aligned
 };
 
 template <bool F32>
@@ -75,10 +76,27 @@ __global__ void __launch_bounds__(256) decode_fp8_scalar(DecodeArgs a, int64_t t
 }
 
 // ------------------------------------------------------------------ 4-bit, FLAT
+// NF4 levels in LDS (16 banks: any mix of codes is conflict free); in constant memory they are a vector load a code
+// ([12288, 4096]: 35 us, 24 here; a [4096, 1536] expert slice 12.9 and 8.5).  All threads of a block come here.
+template <int FMT>
+__device__ __forceinline__ const float* levels_in_lds() {
+    if constexpr (FMT != XQ_FMT_NF4) return nullptr;
+    __shared__ float lv[16];
+    if (threadIdx.x < 16) lv[threadIdx.x] = kNf4Level[threadIdx.x];
+    __syncthreads();
+    return lv;
+}
+template <int FMT>
+__device__ __forceinline__ float code_value(uint32_t code, float s, const float* levels) {
+    if constexpr (FMT == XQ_FMT_NF4) return levels[code] * s;
+    else return val4<FMT>(code, s);
+}
+
 // one thread = 8 packed bytes = 16 consecutive elements of a row
 // (cols % 16 == 0 and group % 16 == 0: the run lies in one scale group)
 template <int FMT>
 __global__ void __launch_bounds__(256) decode_4bit_flat_vec(DecodeArgs a, int64_t chunks_per_row, int64_t total) {
+    const float* levels = levels_in_lds<FMT>();
     int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (t >= total) return;
     int64_t per_expert = a.rows * chunks_per_row;
@@ -90,7 +108,7 @@ __global__ void __launch_bounds__(256) decode_4bit_flat_vec(DecodeArgs a, int64_
     float v[16];
     if (FMT == XQ_FMT_NVFP4) s = s * a.global_scale[e];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) v[i] = val4<FMT>((w[i >> 3] >> (4 * (i & 7))) & 0xfu, s);
+    for (int i = 0; i < 16; ++i) v[i] = code_value<FMT>((w[i >> 3] >> (4 * (i & 7))) & 0xfu, s, levels);
     store_run16<false>(a.out, (e * a.rows + row) * a.cols + c0, v);
 }
 
@@ -112,6 +130,7 @@ __global__ void __launch_bounds__(256) decode_4bit_flat_scalar(DecodeArgs a, int
 // packed [rows/2, cols]; one thread = 16 bytes of a packed row = rows (2r, 2r+1) x 16 cols
 template <int FMT>
 __global__ void __launch_bounds__(256) decode_4bit_gkn_vec(DecodeArgs a, int64_t chunks_per_row, int64_t total) {
+    const float* levels = levels_in_lds<FMT>();
     int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (t >= total) return;
     int64_t per_expert = (a.rows / 2) * chunks_per_row;
@@ -121,14 +140,44 @@ __global__ void __launch_bounds__(256) decode_4bit_gkn_vec(DecodeArgs a, int64_t
     int64_t g = (2 * r2) / a.group;
     const uint8_t* sp = a.scales + e * a.scale_stride;
     float gs = FMT == XQ_FMT_NVFP4 ? a.global_scale[e] : 1.0f;
-    float ve[16], vo[16];
+    float ve[16], vo[16], sc[16];
+    if (a.wide_scales) {               // a thread's 16 scales as 16-byte pieces instead of one by one
+        if (a.scale_dtype == XQ_SCALE_F32) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const f32x4 f = *(const f32x4*)((const float*)sp + g * a.cols + c0 + 4 * q);
+#pragma unroll
+                for (int c = 0; c < 4; ++c) sc[4 * q + c] = f[c];
+            }
+        } else if (a.scale_dtype == XQ_SCALE_BF16) {
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                const u32x4 h = *(const u32x4*)((const uint16_t*)sp + g * a.cols + c0 + 8 * q);
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    sc[8 * q + 2 * c] = __uint_as_float(h[c] << 16);
+                    sc[8 * q + 2 * c + 1] = __uint_as_float(h[c] & 0xffff0000u);
+                }
+            }
+        } else {
+            const u32x4 h = *(const u32x4*)(sp + g * a.cols + c0);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const f32x2 lo = e4m3x2_to_f32(h[q], false), hi = e4m3x2_to_f32(h[q], true);
+                sc[4 * q] = lo[0]; sc[4 * q + 1] = lo[1]; sc[4 * q + 2] = hi[0]; sc[4 * q + 3] = hi[1];
+            }
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) sc[i] = load_scale(sp, g * a.cols + c0 + i, a.scale_dtype);
+    }
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
         uint32_t b = (w[i >> 2] >> (8 * (i & 3))) & 0xffu;
-        float s = load_scale(sp, g * a.cols + c0 + i, a.scale_dtype);
+        float s = sc[i];
         if (FMT == XQ_FMT_NVFP4) s = s * gs;
-        ve[i] = val4<FMT>(b & 0xfu, s);
-        vo[i] = val4<FMT>(b >> 4, s);
+        ve[i] = code_value<FMT>(b & 0xfu, s, levels);
+        vo[i] = code_value<FMT>(b >> 4, s, levels);
     }
     int64_t base = (e * a.rows + 2 * r2) * a.cols + c0;
     store_run16<false>(a.out, base, ve);
@@ -174,6 +223,7 @@ extern "C" int xq_decode(const xq_weight* w, void* out, int out_dtype, void* str
     a.scale_stride = xq_scale_bytes_per_expert(w);
     a.group = w->group;
     a.scale_dtype = w->scale_dtype;
+    a.wide_scales = 0;
     int64_t E = w->num_experts;
     if (w->rows == 0 || w->cols == 0) return XQ_OK;
     int64_t elems = E * w->rows * w->cols;
@@ -208,6 +258,7 @@ extern "C" int xq_decode(const xq_weight* w, void* out, int out_dtype, void* str
         bool vec = (w->cols % 16 == 0) && xq_aligned(w->packed, 16) && xq_aligned(out, 16) && (a.packed_stride % 16 == 0);
         if (vec) {
             int64_t cpr = w->cols / 16, total = E * (w->rows / 2) * cpr;
+            a.wide_scales = xq_aligned(w->scales, 16) && a.scale_stride % 16 == 0;
             if (w->format == XQ_FMT_INT4) decode_4bit_gkn_vec<XQ_FMT_INT4><<<grid_for(total), 256, 0, stream>>>(a, cpr, total);
             else if (w->format == XQ_FMT_NVFP4) decode_4bit_gkn_vec<XQ_FMT_NVFP4><<<grid_for(total), 256, 0, stream>>>(a, cpr, total);
             else decode_4bit_gkn_vec<XQ_FMT_NF4><<<grid_for(total), 256, 0, stream>>>(a, cpr, total);

@@ -882,3 +882,24 @@ def test_few_row_tiles_equal_full_ones(hip_device, fmt, K, N, r):
             su = su_full[rows].contiguous() if r else None
             ys.append(MF._grouped_gemm(qw, transpose_w, a_full[rows].contiguous(), offsets, tile_offsets, su, right))
         assert torch.equal(ys[0], ys[1][pick])
+
+
+@pytest.mark.parametrize("n,E", [(1, 1), (63, 3), (1024, 64), (1025, 65), (2100, 256), (4095, 7), (4096, 256), (4097, 256), (700, 257), (1, 1024)])
+def test_route_build_at_the_edges(hip_device, n, E):
+    """One block up to 4096 entries and 256 experts, three launches beyond: stable expert order, ids outside the range dropped."""
+    from xorl_amd import moe_functional as MF
+
+    g = torch.Generator().manual_seed(n * 7 + E)
+    sel = torch.randint(-1, E + 2, (n, 1), generator=g, dtype=torch.int32)
+    counts, offsets, sidx, tiles = (t.cpu() for t in MF.route_build(sel.to(hip_device), E))
+    flat = sel.flatten().long()
+    ok = (flat >= 0) & (flat < E)
+    want_counts = torch.bincount(flat[ok], minlength=E)
+    want = torch.full((n,), -1, dtype=torch.int64)
+    order = torch.nonzero(ok).flatten()[torch.argsort(flat[ok], stable=True)]
+    want[order] = torch.arange(order.numel())
+    prefix = lambda c: torch.cat([torch.zeros(1, dtype=torch.int64), torch.cumsum(c, 0)])
+    assert torch.equal(counts.long(), want_counts)
+    assert torch.equal(offsets.long(), prefix(want_counts))
+    assert torch.equal(sidx.flatten().long(), want)
+    assert torch.equal(tiles.flatten().long(), torch.cat([prefix((want_counts + t - 1) // t) for t in (128, 256)]))

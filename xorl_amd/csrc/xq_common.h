@@ -33,10 +33,19 @@ int64_t xq_packed_bytes_per_expert(const xq_weight* w);
 int64_t xq_scale_bytes_per_expert(const xq_weight* w);
 
 namespace xq {
+// what the placing pass writes beside scatter_index, each where its pointer is given: the token of every expert-ordered row, and
+// its routing weight as fp32 (copies without an expert have no row)
+struct RouteRows {
+    int32_t topk;
+    int32_t* token_of_row;
+    const void* weights;
+    int32_t weights_f32;
+    float* weight_of_row;
+};
 // xq_route_build over 32-bit ids (id_words 1) or the low words of 64-bit ones (2)
 int route_build(const int32_t* selected, int32_t id_words, int64_t n_routed, int32_t num_experts, int32_t* counts,
                               int32_t* offsets, int32_t* scatter_index, int32_t* tile_offsets, void* workspace,
-                              int64_t workspace_bytes, void* stream_);
+                              int64_t workspace_bytes, void* stream_, const RouteRows* rows = nullptr);
 }
 
 static inline int64_t xq_cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }

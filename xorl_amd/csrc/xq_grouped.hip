@@ -128,8 +128,11 @@ extern "C" int xq_grouped_fwd_ids(const xq_weight* gate, const xq_weight* up, co
     void* route_ws = cv.take<uint8_t>(xq_route_workspace_bytes(R, E));
     const int64_t route_ws_bytes = al256(xq_route_workspace_bytes(R, E));
 
+    // the routing also writes the inverse of scatter_index, row -> token, and the rows' routing weights
+    int32_t* token_of_row = cv.take<int32_t>(R * 4);
+    const RouteRows rows{topk, token_of_row, routing_w, rw_dtype == XQ_DT_F32, saved->w_row};
     if ((rc = route_build((const int32_t*)ids, id_bytes / 4, R, E, saved->counts, saved->offsets, saved->scatter_index, saved->tile_offsets,
-                             route_ws, route_ws_bytes, stream)))
+                             route_ws, route_ws_bytes, stream, &rows)))
         return rc;
     if (R == 0) return XQ_OK;
     bf16_t* xs = (bf16_t*)saved->xs;
@@ -137,17 +140,11 @@ extern "C" int xq_grouped_fwd_ids(const xq_weight* gate, const xq_weight* up, co
     // the inverse of scatter_index and writes the expert-ordered copy xs on its way: no scatter pass of its own.
     // With saved->xs == NULL no copy is written at all: the projection launches read the token matrix through the same
     // map (the routed rows are rows of it, each topk times), and so does the backward (saved->x_tokens).
-    int32_t* token_of_row = cv.take<int32_t>(R * 4);
     const bool ride = ld_hidden % 8 == 0 && xq_aligned(hidden, 16) && xq_aligned(xs, 16);
     const bool in_place = xs == nullptr;
     XQ_REQUIRE(!in_place || (ride && tile_gemm_takes_row_map(gate) && tile_gemm_takes_row_map(up)),
                "%s: saved->xs may be NULL only where xq_grouped_in_place() says so, with 16-byte aligned rows of hidden", who);
-    if (ride) {
-        invert_scatter_kernel<<<dim3((unsigned)xq_cdiv(R, 256)), 256, 0, stream>>>(saved->scatter_index, R, topk, token_of_row);
-        XQ_CHECK_LAUNCH(who);
-    } else if ((rc = xq_moe_scatter(hidden, ld_hidden, saved->scatter_index, R, topk, H, xs, H, stream))) {
-        return rc;
-    }
+    if (!ride && (rc = xq_moe_scatter(hidden, ld_hidden, saved->scatter_index, R, topk, H, xs, H, stream))) return rc;
     const bf16_t* first_in = ride ? (const bf16_t*)hidden : xs;      // operand of the first pass
     const int64_t first_ld = ride ? ld_hidden : H;
     const int32_t* first_map = ride ? token_of_row : nullptr;
@@ -201,7 +198,6 @@ extern "C" int xq_grouped_fwd_ids(const xq_weight* gate, const xq_weight* up, co
         if ((rc = launch_tile_gemm(gate, false, xr, ld_xr, R, off, toff, su_g, Lr_gB, rp, nullptr, gu, 2 * I, stream, who, nullptr, 0, nullptr, nullptr, xr_rows, d.T))) return rc;
         if ((rc = launch_tile_gemm(up, false, xr, ld_xr, R, off, toff, su_u, Lr_uB, rp, nullptr, gu + I, 2 * I, stream, who, nullptr, 0, nullptr, nullptr, xr_rows, d.T))) return rc;
     }
-    if ((rc = xq_moe_scatter_scalar(routing_w, rw_dtype, saved->scatter_index, R, saved->w_row, stream))) return rc;
     // SwiGLU (times the row's routing weight) and s * h . A_d^T of the down projection: one pass where the rank allows
     static const bool silu_nt = [] { const char* e = getenv("XQ_MLP_SILU_NT"); return e ? atoi(e) != 0 : true; }();
     if (silu_nt && silu_bwd_nt_supported(I, rp)) {

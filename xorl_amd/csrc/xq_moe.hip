@@ -118,6 +118,31 @@ __device__ __forceinline__ int32_t wave_inclusive_scan(int32_t v, int lane) {
     return v;
 }
 
+// prefixes over the experts of the totals `tot` (one wave): expert offsets, tile offsets of 128 and of 256 rows
+__device__ __forceinline__ void expert_prefixes(const int32_t* tot, int32_t E, int lane, int32_t* offsets, int32_t* tile_offsets) {
+    int32_t o = 0, t = 0, t2 = 0;
+    int32_t* tiles256 = tile_offsets + (E + 1);
+    for (int e0 = 0; e0 < E; e0 += 64) {
+        const int e = e0 + lane;
+        const int32_t c = e < E ? tot[e] : 0;
+        const int32_t c128 = (c + 127) / 128, c256 = (c + 255) / 256;
+        const int32_t io = wave_inclusive_scan(c, lane), it = wave_inclusive_scan(c128, lane), it2 = wave_inclusive_scan(c256, lane);
+        if (e < E) {
+            offsets[e] = o + io - c;
+            tile_offsets[e] = t + it - c128;
+            tiles256[e] = t2 + it2 - c256;
+        }
+        o += __shfl(io, 63, 64);
+        t += __shfl(it, 63, 64);
+        t2 += __shfl(it2, 63, 64);
+    }
+    if (lane == 0) {
+        offsets[E] = o;
+        tile_offsets[E] = t;
+        tiles256[E] = t2;
+    }
+}
+
 __global__ void __launch_bounds__(1024) route_scan_kernel(int32_t* chunk_counts, int32_t n_chunks, int32_t E,
                                                           int32_t* counts, int32_t* offsets, int32_t* tile_offsets) {
     extern __shared__ int32_t scan_lds[];
@@ -164,58 +189,117 @@ __global__ void __launch_bounds__(1024) route_scan_kernel(int32_t* chunk_counts,
         }
     }
     __syncthreads();
+    if (wave == 0) expert_prefixes(tot, E, lane, offsets, tile_offsets);
+}
+
+// The lanes of a 64-entry segment that hold the same expert (e < 0: none), by intersecting, over the bits of the expert id, the
+// ballots of "my value of this bit": how many of them are below this lane, and whether it is the last of them.
+__device__ __forceinline__ int same_below(int e, int id_bits, int lane, bool& last) {
+    const uint64_t below = (1ull << lane) - 1ull;
+    uint64_t same = __ballot(e >= 0);
+    for (int b = 0; b < id_bits; ++b) {
+        const bool bit = (e >> b) & 1;
+        const uint64_t m = __ballot(bit);
+        same &= bit ? m : ~m;
+    }
+    last = (same & ~below & ~(1ull << lane)) == 0;   // no higher lane holds this expert
+    return __popcll(same & below);
+}
+__device__ __forceinline__ void place_row(const xq::RouteRows& rows, int64_t idx, int32_t r) {
+    if (rows.token_of_row) rows.token_of_row[r] = (int32_t)idx / rows.topk;
+    if (rows.weight_of_row)
+        rows.weight_of_row[r] = rows.weights_f32 ? ((const float*)rows.weights)[idx] : bf16_to_f32(((const bf16_t*)rows.weights)[idx]);
+}
+// All three passes in one block, for up to kRouteOneEntries entries and kRouteOneExperts experts: wave w owns the entries
+// [w * per, (w + 1) * per) in order, held in registers between the histogram and the placing.  Launches bound the three: about 3.5 us
+// each at these sizes (routed MLP, us, three launches and two passes behind them / this: 800 entries 404 / 394, 1800 entries 187 / 180; 6000
+// level, where the one block is as long).
+constexpr int kRouteOneEntries = 4096, kRouteOneExperts = 256;
+__global__ void __launch_bounds__(1024) route_one_kernel(const int32_t* sel, int32_t id_words, int32_t n, int32_t E, int32_t id_bits,
+                                                         int32_t* counts, int32_t* offsets, int32_t* tile_offsets, int32_t* scatter_index,
+                                                         xq::RouteRows rows) {
+    constexpr int SEGS = kRouteOneEntries / 1024;
+    __shared__ int32_t cnt[16 * kRouteOneExperts], tot[kRouteOneExperts], off[kRouteOneExperts];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int segs = (n + 1023) >> 10, first = wave * segs * 64 + lane;      // segs <= SEGS
+    for (int i = tid; i < 16 * E; i += 1024) cnt[i] = 0;
+    int e[SEGS];
+#pragma unroll
+    for (int s = 0; s < SEGS; ++s) {
+        const int idx = first + s * 64;
+        const int v = n > 0 ? sel[(int64_t)min(idx, n - 1) * id_words] : -1;
+        e[s] = s < segs && idx < n && v >= 0 && v < E ? v : -1;
+    }
+    __syncthreads();
+    int32_t* run = cnt + wave * E;
+#pragma unroll
+    for (int s = 0; s < SEGS; ++s)
+        if (e[s] >= 0) atomicAdd(&run[e[s]], 1);
+    __syncthreads();
+    if (tid < E) {
+        int32_t sum = 0;
+#pragma unroll
+        for (int w = 0; w < 16; ++w) {
+            const int32_t v = cnt[w * E + tid];
+            cnt[w * E + tid] = sum;                  // becomes the wave's base within the expert
+            sum += v;
+        }
+        tot[tid] = sum;
+        counts[tid] = sum;
+    }
+    __syncthreads();
     if (wave == 0) {
-        int32_t o = 0, t = 0, t2 = 0;
-        int32_t* tiles256 = tile_offsets + (E + 1);
+        int32_t o = 0;
         for (int e0 = 0; e0 < E; e0 += 64) {
-            const int e = e0 + lane;
-            const int32_t c = e < E ? tot[e] : 0;
-            const int32_t c128 = (c + 127) / 128, c256 = (c + 255) / 256;
-            const int32_t io = wave_inclusive_scan(c, lane), it = wave_inclusive_scan(c128, lane), it2 = wave_inclusive_scan(c256, lane);
-            if (e < E) {
-                offsets[e] = o + io - c;
-                tile_offsets[e] = t + it - c128;
-                tiles256[e] = t2 + it2 - c256;
-            }
+            const int32_t c = e0 + lane < E ? tot[e0 + lane] : 0, io = wave_inclusive_scan(c, lane);
+            if (e0 + lane < E) off[e0 + lane] = o + io - c;
             o += __shfl(io, 63, 64);
-            t += __shfl(it, 63, 64);
-            t2 += __shfl(it2, 63, 64);
         }
-        if (lane == 0) {
-            offsets[E] = o;
-            tile_offsets[E] = t;
-            tiles256[E] = t2;
+    }
+    __syncthreads();
+    if (wave == 15) expert_prefixes(tot, E, lane, offsets, tile_offsets);
+#pragma unroll
+    for (int s = 0; s < SEGS; ++s) {
+        if (s >= segs) break;                        // uniform
+        const int idx = first + s * 64;
+        bool last;
+        const int before = same_below(e[s], id_bits, lane, last);
+        if (e[s] >= 0) {
+            const int32_t r = off[e[s]] + run[e[s]] + before;
+            scatter_index[idx] = r;
+            place_row(rows, idx, r);
+        } else if (idx < n) {
+            scatter_index[idx] = -1;                 // id outside [0, E): the copy is dropped by every consumer
         }
+        // (the wave's own counts: its LDS operations execute in order, so the reads above are done)
+        asm volatile("" ::: "memory");
+        if (e[s] >= 0 && last) run[e[s]] += before + 1;
+        asm volatile("" ::: "memory");
     }
 }
 
-// pass 3: stable position of every routed entry (one wave per chunk, in order).  The lanes of a 64-entry segment that
-// hold the same expert are found by intersecting, over the bits of the expert id, the ballots of "my value of
-// this bit"; a lane's position is the expert's running base plus the number of such lanes below it.
+// pass 3: stable position of every routed entry (one wave per chunk, in order): the expert's running base plus the number of lanes
+// below that hold the same expert
 __global__ void __launch_bounds__(64) route_place_kernel(const int32_t* sel, int32_t id_words, int64_t n, int32_t E, int32_t id_bits,
                                                          const int32_t* chunk_base, const int32_t* offsets,
-                                                         int32_t* scatter_index) {
+                                                         int32_t* scatter_index, xq::RouteRows rows) {
     __shared__ int32_t run[RB_MAX_E];
     for (int e = threadIdx.x; e < E; e += 64) run[e] = offsets[e] + chunk_base[(int64_t)blockIdx.x * E + e];
     __syncthreads();
     const int lane = threadIdx.x;
-    const uint64_t below = (1ull << lane) - 1ull;
     int64_t base = (int64_t)blockIdx.x * RB_CHUNK;
     for (int seg = 0; seg < RB_CHUNK; seg += 64) {
         int64_t idx = base + seg + lane;
         bool valid = idx < n;
         int e = valid ? sel[idx * id_words] : -1;
         if (e >= E) e = -1;
-        uint64_t same = __ballot(e >= 0);
-        for (int b = 0; b < id_bits; ++b) {
-            const bool bit = (e >> b) & 1;
-            const uint64_t m = __ballot(bit);
-            same &= bit ? m : ~m;
-        }
-        const int before = __popcll(same & below);
-        const bool last = (same & ~below & ~(1ull << lane)) == 0;   // no higher lane holds this expert
-        if (e >= 0) scatter_index[idx] = run[e] + before;
-        else if (valid) scatter_index[idx] = -1;          // id outside [0, E): the copy is dropped by every consumer
+        bool last;
+        const int before = same_below(e, id_bits, lane, last);
+        if (e >= 0) {
+            const int32_t r = run[e] + before;
+            scatter_index[idx] = r;
+            place_row(rows, idx, r);
+        } else if (valid) scatter_index[idx] = -1;          // id outside [0, E): the copy is dropped by every consumer
         __syncthreads();
         if (e >= 0 && last) run[e] += before + 1;
         __syncthreads();
@@ -356,7 +440,7 @@ extern "C" int64_t xq_route_workspace_bytes(int64_t n_routed, int32_t num_expert
 // (id_words: 32-bit words from one id to the next, 1, or 2 for 64-bit ids, whose low words are read)
 int xq::route_build(const int32_t* selected, int32_t id_words, int64_t n_routed, int32_t num_experts, int32_t* counts,
                               int32_t* offsets, int32_t* scatter_index, int32_t* tile_offsets, void* workspace,
-                              int64_t workspace_bytes, void* stream_) {
+                              int64_t workspace_bytes, void* stream_, const RouteRows* rows_) {
     XQ_REQUIRE(num_experts >= 1 && num_experts <= RB_MAX_E, "xq_route_build: num_experts %d out of range [1, %d]", num_experts, RB_MAX_E);
     XQ_REQUIRE(n_routed >= 0 && n_routed < (1ll << 31), "xq_route_build: bad n_routed");
     XQ_REQUIRE(counts && offsets && tile_offsets && (n_routed == 0 || (selected && scatter_index)), "xq_route_build: NULL pointer");
@@ -364,6 +448,15 @@ int xq::route_build(const int32_t* selected, int32_t id_words, int64_t n_routed,
     hipStream_t stream = (hipStream_t)stream_;
     int32_t n_chunks = (int32_t)xq_cdiv(n_routed > 0 ? n_routed : 1, RB_CHUNK);
     int32_t* cc = (int32_t*)workspace;
+    const RouteRows rows = rows_ ? *rows_ : RouteRows{1, nullptr, nullptr, 0, nullptr};
+    int id_bits = 0;
+    while ((1 << id_bits) < num_experts) ++id_bits;
+    if (n_routed <= kRouteOneEntries && num_experts <= kRouteOneExperts) {
+        route_one_kernel<<<dim3(1), 1024, 0, stream>>>(selected, id_words, (int32_t)n_routed, num_experts, id_bits, counts, offsets, tile_offsets,
+                                                       scatter_index, rows);
+        XQ_CHECK_LAUNCH("route_one");
+        return XQ_OK;
+    }
     route_hist_kernel<<<dim3(n_chunks), 64, 0, stream>>>(selected, id_words, n_routed, num_experts, cc);
     XQ_CHECK_LAUNCH("route_hist");
     static std::atomic<bool> scan_attr_set{false};   // the attribute call is idempotent: a race only repeats it
@@ -377,9 +470,7 @@ int xq::route_build(const int32_t* selected, int32_t id_words, int64_t n_routed,
     route_scan_kernel<<<dim3(1), 1024, (size_t)17 * num_experts * 4, stream>>>(cc, n_chunks, num_experts, counts, offsets, tile_offsets);
     XQ_CHECK_LAUNCH("route_scan");
     if (n_routed > 0) {
-        int id_bits = 0;
-        while ((1 << id_bits) < num_experts) ++id_bits;
-        route_place_kernel<<<dim3(n_chunks), 64, 0, stream>>>(selected, id_words, n_routed, num_experts, id_bits, cc, offsets, scatter_index);
+        route_place_kernel<<<dim3(n_chunks), 64, 0, stream>>>(selected, id_words, n_routed, num_experts, id_bits, cc, offsets, scatter_index, rows);
         XQ_CHECK_LAUNCH("route_place");
     }
     return XQ_OK;

@@ -159,3 +159,13 @@ def test_rows_of_the_right_factor_at_any_address(hip_device, fmt, M, N, K, r, dt
     bound = 2 ** -8 * want.abs() + 0.5 * 2 ** -9 * ((au + 2 * u.abs()) @ even.abs()) + 1e-5 * want.abs().max()
     assert bool(((y[:, ::2].float() - want).abs() <= bound).all())
     assert not bool(torch.isfinite(y[:, 1::2]).any())
+
+
+@pytest.mark.parametrize("bf16_factors", [False, True])
+@pytest.mark.parametrize("M,N,K,r", [
+    (65, 128, 4160, 64),       # forward over four splits of 65 units, the last one shorter
+    (97, 4160, 192, 50),       # backward the same, ranks that fill no tile
+    (300, 3136, 9216, 40),     # both, eight splits of the forward
+])
+def test_low_rank_products_in_splits(hip_device, M, N, K, r, bf16_factors):
+    test_linear_training_at_the_edges(hip_device, M, N, K, r, bf16_factors)

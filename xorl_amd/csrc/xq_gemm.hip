@@ -937,7 +937,8 @@ extern "C" int xq_linear_fwd(const xq_weight* w, const void* x, int64_t ldx, int
         su = su_out ? (bf16_t*)su_out : (bf16_t*)cv.take(M * rp * 2);
         bf16_t* panel = (bf16_t*)cv.take(lowrank_panel_bytes(1, M, rp, K));
         const LowRankJob job{(const bf16_t*)x, ldx, K, {lora_A, nullptr}, 1, r, rp, scaling, su, rp, 0};
-        if ((rc = launch_lowrank(&job, 1, M, factor_mode(lora_dtype, false), panel, stream))) return rc;
+        // (the sums of its splits live where the product's will)
+        if ((rc = launch_lowrank(&job, 1, M, factor_mode(lora_dtype, false), panel, stream, (float*)cv.take(0), workspace_bytes - cv.used))) return rc;
     }
     // what is left of the workspace holds split-K partial sums (small row counts); without it the launch is unsplit
     float* partial = (float*)cv.take(0);
@@ -1171,10 +1172,10 @@ extern "C" int xq_linear_bwd(const xq_weight* w, const void* x, int64_t ldx, con
         bf16_t* panel = (bf16_t*)cv.take(lowrank_panel_bytes(1, M, rp, K));
         // v = bf16(s * dy . B)   [M, rp]
         const LowRankJob jv{(const bf16_t*)dy, lddy, N, {lora_B, nullptr}, 1, r, rp, scaling, v, rp, 0};
-        if ((rc = launch_lowrank(&jv, 1, M, factor_mode(lora_dtype, true), nullptr, stream))) return rc;
+        if ((rc = launch_lowrank(&jv, 1, M, factor_mode(lora_dtype, true), nullptr, stream, (float*)cv.take(0), workspace_bytes - cv.used))) return rc;
         if (dB && !su) {
             const LowRankJob ju{(const bf16_t*)x, ldx, K, {lora_A, nullptr}, 1, r, rp, scaling, su_ws, rp, 0};
-            if ((rc = launch_lowrank(&ju, 1, M, factor_mode(lora_dtype, false), panel, stream))) return rc;
+            if ((rc = launch_lowrank(&ju, 1, M, factor_mode(lora_dtype, false), panel, stream, (float*)cv.take(0), workspace_bytes - cv.used))) return rc;
             su = su_ws;
         }
     }

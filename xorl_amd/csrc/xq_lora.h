@@ -87,7 +87,9 @@ struct LowRankJob {
     int64_t ld_t, t_step;
 };
 int64_t lowrank_panel_bytes(int n, int64_t n_rows, int cols, int64_t Kc);   // scratch a launch of n products (nf * rp = cols each) may want
-int launch_lowrank(const LowRankJob* jobs, int n, int64_t n_rows, FactorMode mode, bf16_t* panels, hipStream_t stream);
+// scratch (may be NULL): memory for the fp32 sums of a contraction in splits, free again when the launch is done
+int launch_lowrank(const LowRankJob* jobs, int n, int64_t n_rows, FactorMode mode, bf16_t* panels, hipStream_t stream, float* scratch = nullptr,
+                   int64_t scratch_bytes = 0);
 
 // Every LoRA panel of a call in one launch: job k converts a [n_src, R_in, C_in] fp32 / bf16 factor (n_src = 1 or
 // the expert count) into bf16 [n_out, R_out, C_out], optionally transposed, zero padded; n_src == 1 < n_out repeats

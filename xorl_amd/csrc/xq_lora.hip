@@ -515,6 +515,8 @@ struct LowRankBatch {
     int32_t first[kLowRankJobs];      // first block of a job
     int32_t n;
     int64_t n_rows;
+    int32_t splits;                   // > 1 (one product): split blockIdx.y of the contraction leaves its fp32 sums to partial
+    float* partial;                   // [splits][n_rows][nf * rp]
 };
 
 // T[rows, nf * rp] = bf16(scale * In . F^T), up to kLowRankJobs products in one launch.  A block owns 16 RT rows; its NW waves
@@ -647,12 +649,13 @@ __global__ void __launch_bounds__(64 * NW, NW / 4) lowrank_kernel(LowRankBatch b
             }
         }
     };
-    const int units = (int)(g.Kc >> 6), last = units - 1;
-    if (wave < units) {
+    const int all = (int)(g.Kc >> 6), per = b.splits > 1 ? (all + b.splits - 1) / b.splits : all;
+    const int first = (int)blockIdx.y * per + wave, units = min(all, (int)blockIdx.y * per + per), last = units - 1;
+    if (first < units) {
         Unit a, c;
-        load(a, wave);
+        load(a, first);
 #pragma unroll 1
-        for (int u = wave;;) {
+        for (int u = first;;) {
             int nx = u + NW;
             load(c, nx < last ? nx : last);            // (past the end: fetched again, never used)
             multiply(a);
@@ -679,6 +682,10 @@ __global__ void __launch_bounds__(64 * NW, NW / 4) lowrank_kernel(LowRankBatch b
         const int l = idx & 63, t = (idx >> 6) % NT, i = (idx >> 6) / NT;
         const int64_t m = row0 + i * 16 + (l & 15);
         if (t * 16 >= cols || m >= b.n_rows) continue;
+        if (b.splits > 1) {
+            *(f32x4*)(b.partial + ((int64_t)blockIdx.y * b.n_rows + m) * cols + t * 16 + 4 * (l >> 4)) = v;
+            continue;
+        }
         const int f = t * 16 >= rp ? 1 : 0;
         *(u32x2*)(g.T + f * g.t_step + m * g.ld_t + t * 16 - f * rp + 4 * (l >> 4)) =
             u32x2{pack_bf16x2(v[0] * g.scale, v[1] * g.scale), pack_bf16x2(v[2] * g.scale, v[3] * g.scale)};
@@ -697,7 +704,7 @@ static int launch_lowrank_one(const LowRankBatch& b, unsigned blocks, hipStream_
         }
         attr_set = true;
     }
-    lowrank_kernel<MODE, NT, RT, NW><<<dim3(blocks), 64 * NW, lds, stream>>>(b);
+    lowrank_kernel<MODE, NT, RT, NW><<<dim3(blocks, (unsigned)b.splits), 64 * NW, lds, stream>>>(b);
     return XQ_OK;
 }
 template <int MODE, int RT, int NW>
@@ -717,7 +724,34 @@ int64_t lowrank_panel_bytes(int n, int64_t n_rows, int cols, int64_t Kc) {
     return lowrank_tall(n, n_rows) ? (((int64_t)cols * Kc * 2 + 255) & ~(int64_t)255) * n : 0;
 }
 
-int launch_lowrank(const LowRankJob* jobs, int n, int64_t n_rows, FactorMode mode, bf16_t* panels, hipStream_t stream) {
+// T[m][j] = bf16(scale * (partial[0][m][j] + partial[1][m][j] + ...)), the splits in index order; columns from rp on are the
+// second product's
+__global__ void __launch_bounds__(256) lowrank_reduce_kernel(const float* partial, int splits, int64_t n_rows, int rp, int nprod, float scale,
+                                                             bf16_t* T, bf16_t* T2, int64_t ld_t) {
+    const int cols = nprod * rp;
+    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x, total = n_rows * cols;
+    if (t >= total) return;
+    float v = partial[t];
+    for (int s = 1; s < splits; ++s) v += partial[(int64_t)s * total + t];
+    const int64_t m = t / cols;
+    const int j = (int)(t - m * cols);
+    (j < rp ? T : T2)[m * ld_t + (j < rp ? j : j - rp)] = to_bf16(v * scale);
+}
+
+// Splits of the contraction of one product where its blocks leave compute units idle.  A block pulls its rows and the whole factor
+// through one compute unit, about 0.1 MB a microsecond; the launch that adds the splits' sums costs three.  us before and with splits: MLP
+// 4096/12288 forward of 120 rows r 16 114 / 104, r 64 147 / 121, nvfp4 of 700 rows r 32 354 / 332; one projection [4096, 12288] forward and
+// backward of 300 rows r 64 212 / 180, [12288, 4096] r 16 166 / 159; below the line (512 rows, K 4096, r 16) one launch is level or ahead.
+static int lowrank_splits(const LowRankJob& j, int64_t blocks, FactorMode mode, const float* scratch, int64_t scratch_bytes, int64_t n_rows) {
+    const int64_t bytes = j.Kc * (32 + (mode == kFacF32 || mode == kFacF32T ? 4 : 2) * (int64_t)j.nf * j.rp);
+    int64_t s = std::min(num_cus() / blocks, j.Kc / 1024);      // (a unit of 64 for each of sixteen waves)
+    if (s > 8) s = 8;
+    if (s < 2 || bytes - bytes / s < 400000 || !xq_aligned(scratch, 16) || !scratch || scratch_bytes < s * n_rows * j.nf * j.rp * 4) return 1;
+    return (int)s;
+}
+
+int launch_lowrank(const LowRankJob* jobs, int n, int64_t n_rows, FactorMode mode, bf16_t* panels, hipStream_t stream, float* scratch,
+                   int64_t scratch_bytes) {
     XQ_REQUIRE(n >= 1 && n <= kLowRankJobs, "lowrank: %d products", n);
     if (n_rows == 0) return XQ_OK;
     LowRankBatch b{};
@@ -754,6 +788,8 @@ int launch_lowrank(const LowRankJob* jobs, int n, int64_t n_rows, FactorMode mod
         nt = j.nf * j.rp / 16 > nt ? j.nf * j.rp / 16 : nt;
     }
     b.n = n; b.n_rows = n_rows;
+    b.splits = n == 1 && !tall ? lowrank_splits(jobs[0], blocks, mode, scratch, scratch_bytes, n_rows) : 1;
+    b.partial = scratch;
     const unsigned grid = (unsigned)(blocks * n);
     int rc;
 #define XQ_LR(MODE) rc = tall ? launch_lowrank_nt<MODE, 2, 8>(b, nt, grid, stream) : launch_lowrank_nt<MODE, 1, 16>(b, nt, grid, stream)
@@ -766,21 +802,13 @@ int launch_lowrank(const LowRankJob* jobs, int n, int64_t n_rows, FactorMode mod
 #undef XQ_LR
     if (rc) return rc;
     XQ_CHECK_LAUNCH("lowrank");
+    if (b.splits > 1) {
+        const LowRankJob& j = jobs[0];
+        lowrank_reduce_kernel<<<(unsigned)xq_cdiv(n_rows * j.nf * j.rp, 256), 256, 0, stream>>>(scratch, b.splits, n_rows, j.rp, j.nf, j.scale, j.T,
+                                                                                                 j.T + j.t_step, j.ld_t);
+        XQ_CHECK_LAUNCH("lowrank_reduce");
+    }
     return XQ_OK;
-}
-
-// T[m][j] = bf16(scale * (partial[0][m][j] + partial[1][m][j] + ...)), the splits in index order; columns from rp on are the
-// second product's
-__global__ void __launch_bounds__(256) lowrank_reduce_kernel(const float* partial, int splits, int64_t n_rows, int rp, int nprod, float scale,
-                                                             bf16_t* T, bf16_t* T2, int64_t ld_t) {
-    const int cols = nprod * rp;
-    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x, total = n_rows * cols;
-    if (t >= total) return;
-    float v = partial[t];
-    for (int s = 1; s < splits; ++s) v += partial[(int64_t)s * total + t];
-    const int64_t m = t / cols;
-    const int j = (int)(t - m * cols);
-    (j < rp ? T : T2)[m * ld_t + (j < rp ? j : j - rp)] = to_bf16(v * scale);
 }
 
 // ------------------------------------------------------------------ SwiGLU backward + its two low-rank products

@@ -188,6 +188,8 @@ extern "C" int xq_mlp_fwd(const xq_weight* gate, const xq_weight* up, const xq_w
     bf16_t* panels = cv.take<bf16_t>(fwd_panel_bytes(d));
     const void *A_g = lora->A[0], *A_u = lora->A[1];
     const bool many = many_rows(d) && !fused;
+    float* part = cv.take<float>(0);
+    const int64_t part_bytes = workspace_bytes - cv.used;
     bf16_t* A_d = panels + 2 * (int64_t)rp * H;
     int ra = r;                                   // ranks in the factors the products read
     if (many) {
@@ -205,11 +207,9 @@ extern "C" int xq_mlp_fwd(const xq_weight* gate, const xq_weight* up, const xq_w
         const LowRankJob both{x, ldx, H, {A_g, A_u}, 2, ra, rp, s, su_gu, sl.pitch, sl.up_offset};
         const LowRankJob apart[2] = {{x, ldx, H, {A_g, nullptr}, 1, ra, rp, s, su_gu, sl.pitch, 0},
                                      {x, ldx, H, {A_u, nullptr}, 1, ra, rp, s, su_gu + sl.up_offset, sl.pitch, 0}};
-        rc = 2 * rp <= 64 ? launch_lowrank(&both, 1, M, fm, panels, stream) : launch_lowrank(apart, 2, M, fm, panels, stream);
+        rc = 2 * rp <= 64 ? launch_lowrank(&both, 1, M, fm, panels, stream, part, part_bytes) : launch_lowrank(apart, 2, M, fm, panels, stream);
         if (rc) return rc;
     }
-    float* part = cv.take<float>(0);
-    const int64_t part_bytes = workspace_bytes - cv.used;
     const bf16_t *bias_g = (const bf16_t*)lora->bias[0], *bias_u = (const bf16_t*)lora->bias[1], *bias_d = (const bf16_t*)lora->bias[2];
     if (fused) {
         if ((rc = launch_gate_up_swiglu(gate, up, x, ldx, M, rp ? su_gu : nullptr, rp ? su_gu + sl.up_offset : nullptr, sl.pitch,
@@ -227,7 +227,7 @@ extern "C" int xq_mlp_fwd(const xq_weight* gate, const xq_weight* up, const xq_w
     }
     if (rp && !many) {
         const LowRankJob jd{h, I, I, {lora->A[2], nullptr}, 1, r, rp, s, su_d, rp, 0};
-        if ((rc = launch_lowrank(&jd, 1, M, fm, panels, stream))) return rc;
+        if ((rc = launch_lowrank(&jd, 1, M, fm, panels, stream, part, part_bytes))) return rc;
     }
     return launch_tile_gemm(down, true, h, I, M, nullptr, nullptr, rp ? su_d : nullptr, nullptr, rp, bias_d, (bf16_t*)y, ldy, stream,
                             who, part, part_bytes, nullptr, rp ? &right_d : nullptr);
@@ -364,7 +364,7 @@ extern "C" int xq_mlp_bwd(const xq_weight* gate, const xq_weight* up, const xq_w
     // ---- down projection
     if (rp) {
         const LowRankJob jd{dy, lddy, H, {lora->B[2], nullptr}, 1, r, rp, s, v_d, rp, 0};
-        if ((rc = launch_lowrank(&jd, 1, M, ft, nullptr, stream))) return rc;
+        if ((rc = launch_lowrank(&jd, 1, M, ft, nullptr, stream, part, part_bytes))) return rc;
     }
     if ((rc = launch_tile_gemm(down, false, dy, lddy, M, nullptr, nullptr, rp ? v_d : nullptr, nullptr, rp, nullptr, dh, I, stream, who, part, part_bytes,
                                nullptr, rp ? &right_d : nullptr)))

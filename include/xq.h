@@ -540,6 +540,8 @@ int xq_grouped_bwd(const xq_weight* gate, const xq_weight* up, const xq_weight* 
  * workspace: xq_grouped_infer_workspace_bytes() bytes, 256-byte aligned. */
 int xq_grouped_infer_supported(const xq_weight* gate, const xq_weight* up, const xq_weight* down, int64_t n_tokens,
                                int32_t topk, int r);
+/* Whether that form is also the shorter one for so many tokens (a call of it runs either way). */
+int xq_grouped_infer_shorter(const xq_weight* gate, int64_t n_tokens, int32_t topk);
 int64_t xq_grouped_infer_workspace_bytes(int64_t n_tokens, int32_t topk, int32_t num_experts, int64_t hidden,
                                          int64_t intermediate, int r);
 int xq_grouped_fwd_infer(const xq_weight* gate, const xq_weight* up, const xq_weight* down, const xq_grouped_lora* lora,

@@ -266,3 +266,25 @@ def test_expert_ids_of_either_width(hip_device, T):
             want = m(x, rw, sel.int().to(hip_device)).detach()
             for ids in (sel.to(hip_device), wide, sel.t().contiguous().to(hip_device).t(), wide.int()):
                 assert torch.equal(m(x, rw, ids).detach(), want)
+
+
+@pytest.mark.parametrize("fmt", ["block_fp8", "nvfp4", "nf4"])
+def test_forwards_on_both_sides_of_the_streaming_line(hip_device, fmt):
+    """The last token count that is streamed and the first that runs on tiles: the same tokens, to rounding of bf16 intermediates."""
+    import ctypes
+
+    from tests.test_gpu_moe import _make_experts, _zipf_routing
+    from xorl_amd import _C
+
+    E, H, I, topk = 8, 2048, 768, 2
+    m, _ = _make_experts(fmt, E, H, I, 8, False, seed=3, device=hip_device)
+    wg = m._bank("gate").c()
+    streamed = [T for T in range(1, 257) if _C.lib().xq_grouped_infer_shorter(ctypes.byref(wg), T, topk)]
+    line = len(streamed)
+    assert streamed == list(range(1, line + 1)) and 16 <= line < 256
+    rw, sel = _zipf_routing(line + 1, E, topk, seed=5)
+    x = gen((line + 1, H), 1.0, 6, torch.bfloat16).to(hip_device)
+    rw, sel = rw.to(torch.bfloat16).to(hip_device), sel.to(hip_device)
+    with torch.no_grad():
+        a, b = m(x[:line], rw[:line], sel[:line]), m(x, rw, sel)[:line]
+    close(a.cpu(), b.cpu().double(), 1e-2)

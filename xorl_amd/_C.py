@@ -173,6 +173,7 @@ _SIGNATURES = {
     "xq_grouped_bwd": (_INT, [_W, _W, _W, ctypes.POINTER(XqGroupedLora), _P, _I64, _I64, _I32,
                               ctypes.POINTER(XqGroupedSaved), _P, _I64, _P, _INT, ctypes.POINTER(XqGroupedGrads), _P, _I64,
                               _P]),
+    "xq_grouped_infer_shorter": (_INT, [_W, _I64, _I32]),
     "xq_grouped_infer_supported": (_INT, [_W, _W, _W, _I64, _I32, _INT]),
     "xq_grouped_infer_workspace_bytes": (_I64, [_I64, _I32, _I32, _I64, _I64, _INT]),
     # gate, up, down, lora, hidden, ld_hidden, n_tokens, routing_w, rw_dtype, selected, topk, out, ld_out, ws, ws_bytes, stream

@@ -734,6 +734,17 @@ extern "C" int xq_grouped_infer_supported(const xq_weight* gate, const xq_weight
     return infer_supported(gate, up, down, n_tokens, topk, r) ? 1 : 0;
 }
 
+// Streaming reads an expert's matrices once for every four of its rows, the tile kernels once, behind more launches: the line between
+// them lies at some rows an expert, later where matrices are small.  Forward, us, streamed / on tiles, by routed copies: 8 experts
+// 4096/1536, 64 copies fp8 87 / 84, nvfp4 76 / 88, nf4 108 / 119, 128 copies 148 / 93, 116 / 96, 177 / 123, 512 copies 433 / 128, 337 / 134,
+// 541 / 169; 32 experts 2560/1024, 128 copies 91 / 101, 77 / 106, 110 / 143, 256 copies 137 / 106, 110 / 107, 164 / 144, 512 copies 222 / 113,
+// 175 / 111, 271 / 152; 128 experts 2048/768, 512 copies 179 / 182, 152 / 178, 230 / 243.
+extern "C" int xq_grouped_infer_shorter(const xq_weight* gate, int64_t n_tokens, int32_t topk) {
+    if (!gate || gate->rows < 1 || gate->cols < 1) return 0;
+    const double line = 200e6 / ((double)gate->rows * gate->cols) + 3.3 * gate->num_experts;
+    return (double)n_tokens * topk <= line * (gate->format == XQ_FMT_NVFP4 ? 1.3 : gate->format == XQ_FMT_NF4 ? 1.2 : 1.05) ? 1 : 0;
+}
+
 extern "C" int64_t xq_grouped_infer_workspace_bytes(int64_t n_tokens, int32_t topk, int32_t num_experts, int64_t hidden,
                                                     int64_t intermediate, int r) {
     if (n_tokens < 1 || topk < 1 || num_experts < 1 || r < 1 || hidden < kDecChunk || intermediate < kDecChunk) return 0;

@@ -756,7 +756,8 @@ PyObject* moe(PyObject*, PyObject* const* args, Py_ssize_t n) {
             XQ_NONE;
         const int r = (int)rank, rp = r_pad_of(r);
         const bool train = at::GradMode::is_enabled() && (x->requires_grad() || rw->requires_grad() || factor_grad);
-        if (streaming && (train || !xq_grouped_infer_supported(&q[0].w, &q[1].w, &q[2].w, T, (int32_t)topk, r))) XQ_NONE;
+        if (streaming && (train || !xq_grouped_infer_supported(&q[0].w, &q[1].w, &q[2].w, T, (int32_t)topk, r) || !xq_grouped_infer_shorter(&q[0].w, T, (int32_t)topk)))
+            XQ_NONE;
         Tensor ids = sel->is_contiguous() ? *sel : sel->detach().contiguous();       // 64-bit ids as they are: a conversion would be a launch
         const int id_bytes = (int)ids.element_size();
         Tensor w = rw->is_contiguous() ? *rw : rw->detach().contiguous();

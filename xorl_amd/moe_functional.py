@@ -372,7 +372,7 @@ def _moe_infer(hidden: Tensor, routing_weights: Tensor, selected_experts: Tensor
     r = factors[0].shape[-1]
     wg, wu, wd = qg.c(), qu.c(), qd.c()
     L = _C.lib()
-    if not L.xq_grouped_infer_supported(ctypes.byref(wg), ctypes.byref(wu), ctypes.byref(wd), T, topk, r):
+    if not L.xq_grouped_infer_supported(ctypes.byref(wg), ctypes.byref(wu), ctypes.byref(wd), T, topk, r) or not L.xq_grouped_infer_shorter(ctypes.byref(wg), T, topk):
         return None
     if hidden2.data_ptr() % 16 or (T > 1 and hidden2.stride(0) % 8):
         return None

@@ -702,9 +702,9 @@ static inline int64_t al256(int64_t b) { return (b + 255) & ~(int64_t)255; }
 // What a launch of `blocks` blocks of RT row tiles and `steps` steps takes beyond a constant, in us, from a sweep of every (row tiles,
 // splits) at M 24..64 on seven widths and depths of int4 and block-fp8 (within 10 % of the times; the pair it picks is 1.2 % behind
 // the best on average, 8 % at worst): rounds of the chip, and in a block the half steps of a wave, each for its weights and its x.  Two
-// blocks are resident per compute unit where StreamGeo says so.
-static double stream_run_us(int64_t blocks, int rt, int steps, int mt) {
-    const int per_cu = mt < 4 && mt * rt <= 4 ? 2 : 1;
+// blocks are resident per compute unit where StreamGeo says so (MT RT up to pair_max, 3 with the levels of nf4 and 4 otherwise).
+static double stream_run_us(int64_t blocks, int rt, int steps, int mt, int pair_max) {
+    const int per_cu = mt < 4 && mt * rt <= pair_max ? 2 : 1;
     const int64_t cus = num_cus();
     const double rounds = (double)xq_cdiv(blocks, cus * per_cu), halves = 2.0 * xq_cdiv(steps, kStreamWaves);
     const double on_cu = (double)xq_cdiv(blocks, cus) < rounds * per_cu ? (double)xq_cdiv(blocks, cus) : rounds * per_cu;
@@ -712,14 +712,14 @@ static double stream_run_us(int64_t blocks, int rt, int steps, int mt) {
 }
 static const int kRowTiles[] = {1, 2, 3, 4, 6};
 // row tiles of a block by that estimate (they change nothing in the results); `tiles`, `splits` of each forward of the launch
-static int stream_row_tiles(const int* tiles, const int* splits, int n, int steps, int mt, int rt_max, double* us) {
+static int stream_row_tiles(const int* tiles, const int* splits, int n, int steps, int mt, int rt_max, int pair_max, double* us) {
     int best = 1;
     double cost = 0;
     for (int rt : kRowTiles) {
         if (rt > rt_max) break;
         int64_t blocks = 0;
         for (int i = 0; i < n; ++i) blocks += xq_cdiv(tiles[i], (int64_t)rt) * splits[i];
-        const double c = stream_run_us(blocks, rt, steps, mt);
+        const double c = stream_run_us(blocks, rt, steps, mt, pair_max);
         if (cost == 0 || c < cost) { cost = c; best = rt; }
     }
     if (us) *us = cost;
@@ -744,7 +744,7 @@ static int make_stream_splits(int64_t M, int64_t N, int64_t K) {
         last_steps = steps;
         if (best && (s * M * N * 4 > (16ll << 20))) break;
         double c;
-        stream_row_tiles(&tiles, &s, 1, steps, mt, 6, &c);
+        stream_row_tiles(&tiles, &s, 1, steps, mt, 6, 4, &c);
         c += (double)s * M * N * 8.0 / 1.7e6;
         if (best == 0 || c < worth * best_cost) { best = s; best_cost = c; }
     }
@@ -875,7 +875,7 @@ int launch_skinny_stream(const SkinnyRowsJob* jobs, int n_jobs, bool swiglu, con
     }
     int tiles[kStreamJobs], splits[kStreamJobs];
     for (int i = 0; i < n_jobs; ++i) { tiles[i] = b.job[i].N / 16; splits[i] = b.job[i].splits; }
-    const int rt = stream_row_tiles(tiles, splits, n_jobs, steps, mt, row_tiles_max(w0->format, sc), nullptr);
+    const int rt = stream_row_tiles(tiles, splits, n_jobs, steps, mt, row_tiles_max(w0->format, sc), w0->format == XQ_FMT_NF4 ? 3 : 4, nullptr);
     int first[5] = {0, 0, 0, 0, 0}, efirst[5] = {0, 0, 0, 0, 0};
     for (int i = 0; i < kStreamJobs; ++i) {
         first[i + 1] = first[i];

@@ -113,3 +113,25 @@ def test_waves_that_split_the_contraction(hip_device, fmt, N, K, r, Ms):
             assert torch.equal(m(wide[:, :K].contiguous().to(hip_device)), y)
         ex = R.linear_fwd_bwd_exact(wide[:, :K].contiguous(), w_ref, A, B, m.scaling, torch.zeros(M, N, dtype=torch.bfloat16))
         close(y.cpu(), ex["y"], 1e-2)                             # (the bound of every forward above)
+
+
+@pytest.mark.parametrize("K", [1152, 2048])                       # a depth of the streaming kernels and one of the one-launch kernels
+def test_rows_of_x_a_gigabyte_apart(hip_device, K):
+    """Eight rows 2^29 elements apart (32-bit offsets of the rows would repeat every four): the packed copy's result."""
+    m, w_ref = make_dense_module("int4", 512, K, 16, 32, seed=K, device=hip_device)
+    g, u = (make_dense_module("int4", 1024, K, 16, 32, seed=s, device=hip_device)[0] for s in (5, 6))
+    d = make_dense_module("int4", K, 1024, 16, 32, seed=7, device=hip_device)[0]
+    from xorl_amd.qlora import qlora_linears_forward, qlora_mlp_forward
+
+    x = gen((8, K), 1.0, 75, torch.bfloat16)
+    pitch = 1 << 29
+    far = torch.empty(7 * pitch + K, dtype=torch.bfloat16, device=hip_device).as_strided((8, K), (pitch, 1))
+    far.copy_(x.to(hip_device))
+    for M in (1, 2, 3, 8):
+        with torch.no_grad():
+            packed = x[:M].to(hip_device)
+            close(m(far[:M]).cpu(), R.linear_fwd_bwd_exact(x[:M], w_ref, m.lora_A.detach().cpu(), m.lora_B.detach().cpu(), m.scaling,
+                                                           torch.zeros(M, 512, dtype=torch.bfloat16))["y"], 1e-2)
+            for a, b in zip(qlora_linears_forward([g, u], far[:M]), qlora_linears_forward([g, u], packed)):
+                close(a.cpu(), b.cpu().double(), 1e-2)
+            close(qlora_mlp_forward(g, u, d, far[:M]).cpu(), qlora_mlp_forward(g, u, d, packed).cpu().double(), 1e-2)

@@ -196,3 +196,22 @@ def test_build_refuses_scratch_under_hand_counted_reads():
     b.check_scratch(remarks, guarded)
     with pytest.raises(RuntimeError, match="gemm_dec_kernel"):
         b.check_scratch(b._split_remarks(output(other, 0) + "\n" + output(dec, 80))[0], guarded)
+
+
+@pytest.mark.parametrize("K,near", [(1152, 2), (2048, 1)])     # a depth of the streaming kernels and one of the one-launch kernels (to 16 rows)
+def test_rows_of_x_far_apart_leave_the_streaming_kernels(K, near):
+    """Their addresses within eight rows are 32 bits wide: 2 * 7 * ldx bytes and a row's 128 at most.  One row has no pitch."""
+    from xorl_amd import _C
+
+    w = _C.XqWeight()
+    w.format, w.layout, w.scale_dtype, w.group = _C.FORMATS["int4"], _C.XQ_LAYOUT_FLAT, _C.XQ_SCALE_BF16, 128
+    w.rows, w.cols, w.num_experts, w.packed, w.scales = 512, K, 1, 4096, 4096        # (addresses: nothing is read)
+    route = lambda M, ldx: _C.lib().xq_skinny_route(ctypes.byref(w), M, ldx, None, None, _C.XQ_DT_F32, 0)
+    for M in (1, 2, 3, 8, 9, 16, 17, 64):
+        here = near if M <= 16 else 2
+        assert route(M, K) == here and route(M, (1 << 28) - 8) == here, M
+        for ldx in (1 << 28, 306783384, 1 << 30, 1 << 31, 1 << 33):
+            want = here if M == 1 or here == 1 else 0
+            assert route(M, ldx) == want, (M, ldx)
+    assert 2 * 7 * ((1 << 28) - 8) + 128 < 1 << 32
+    assert route(65, K) == 0

@@ -910,6 +910,17 @@ static int check_dense(const xq_weight* w, const char* who) {
     return XQ_OK;
 }
 
+// whether a forward that keeps nothing for a backward runs on the kernels of few rows, and on which of them
+static bool takes_skinny(const xq_weight* w, int64_t M, int64_t ldx, const void* lora_A, const void* lora_B, int lora_dtype, int r) {
+    return g_skinny_enabled && skinny_supported(w, M) &&
+           (stream_takes_pitch(M, ldx) || (skinny_rows_enabled() && skinny_rows_supported(w, M, lora_A, lora_B, lora_dtype, r)));
+}
+extern "C" int xq_skinny_route(const xq_weight* w, int64_t M, int64_t ldx, const void* lora_A, const void* lora_B, int lora_dtype, int r) {
+    if (!w || M < 1 || r < 0 || r > 64 || check_dense(w, "xq_skinny_route")) return -1;
+    if (!takes_skinny(w, M, ldx, lora_A, lora_B, lora_dtype, r)) return XQ_SKINNY_NONE;
+    return skinny_takes_stream(w, M, ldx, lora_A, lora_B, lora_dtype, r) ? XQ_SKINNY_STREAM : XQ_SKINNY_ONE_LAUNCH;
+}
+
 extern "C" int xq_linear_fwd(const xq_weight* w, const void* x, int64_t ldx, int64_t M, const void* lora_A,
                              const void* lora_B, int lora_dtype, int r, float scaling, const void* bias_bf16, void* y,
                              int64_t ldy, void* su_out, void* workspace, int64_t workspace_bytes, void* stream_) {
@@ -925,9 +936,11 @@ extern "C" int xq_linear_fwd(const xq_weight* w, const void* x, int64_t ldx, int
     XQ_REQUIRE(ldy % 8 == 0 && xq_aligned(y, 16), "xq_linear_fwd: y rows must be 16-byte aligned");
     const int rp = r_pad_of(r);
     // decode / rollout shapes: stream the packed weight once (HBM-bound kernel); forward only
-    if (!su_out && g_skinny_enabled && skinny_supported(w, M) && (M <= 8 || ldx < kSkinnyLdx))
-        return launch_skinny(w, (const bf16_t*)x, ldx, M, lora_A, lora_B, lora_dtype, r, scaling,
-                             (const bf16_t*)bias_bf16, (bf16_t*)y, ldy, workspace, workspace_bytes, stream);
+    if (!su_out && takes_skinny(w, M, ldx, lora_A, lora_B, lora_dtype, r)) {
+        rc = launch_skinny(w, (const bf16_t*)x, ldx, M, lora_A, lora_B, lora_dtype, r, scaling,
+                           (const bf16_t*)bias_bf16, (bf16_t*)y, ldy, workspace, workspace_bytes, stream);
+        if (rc != XQ_ERR_UNSUPPORTED) return rc;
+    }
     bf16_t* su = nullptr;
     const LowRankRight right{{lora_B, nullptr}, r, r, rp, lora_dtype == XQ_DT_F32, 0};
     Carver cv{(workspace && xq_aligned(workspace, 256)) ? (uint8_t*)workspace : nullptr, 0, workspace_bytes};
@@ -1088,7 +1101,7 @@ extern "C" int xq_linear_fwd_multi(const xq_linear_job* jobs, int n_jobs, const 
         }
     }
     // decode shapes outside the whole-row kernel: every forward in one streaming launch and one epilogue
-    if (g_skinny_enabled && n_jobs > 1 && M <= 16 && ldx % 8 == 0 && (M <= 8 || ldx < kSkinnyLdx) && xq_aligned(x, 16)) {
+    if (g_skinny_enabled && n_jobs > 1 && M <= 16 && ldx % 8 == 0 && xq_aligned(x, 16)) {
         SkinnyRowsJob sj[XQ_LINEAR_MULTI_MAX];
         double bytes = 2.0 * M * jobs[0].w->cols;
         bool ok = true;
@@ -1096,7 +1109,7 @@ extern "C" int xq_linear_fwd_multi(const xq_linear_job* jobs, int n_jobs, const 
             const xq_weight* w = jobs[i].w;
             sj[i] = SkinnyRowsJob{w, jobs[i].lora_A, jobs[i].lora_B, jobs[i].r, jobs[i].scaling, (const bf16_t*)jobs[i].bias_bf16,
                                   (bf16_t*)jobs[i].y, jobs[i].ldy};
-            ok = ok && skinny_takes_stream(w, M, jobs[i].lora_A, jobs[i].lora_B, lora_dtype, jobs[i].r);
+            ok = ok && skinny_takes_stream(w, M, ldx, jobs[i].lora_A, jobs[i].lora_B, lora_dtype, jobs[i].r);
             bytes += (double)xq_packed_bytes_per_expert(w) + (double)xq_scale_bytes_per_expert(w) + 2.0 * M * w->rows +
                      4.0 * jobs[i].r * (w->cols + w->rows);
         }

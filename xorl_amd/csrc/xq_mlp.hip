@@ -295,8 +295,8 @@ extern "C" int xq_mlp_fwd_infer(const xq_weight* gate, const xq_weight* up, cons
         {gate, lora->A[0], lora->B[0], d.r, lora->scaling, (const bf16_t*)lora->bias[0], h, d.I},
         {up, lora->A[1], lora->B[1], d.r, lora->scaling, (const bf16_t*)lora->bias[1], h, d.I},
     };
-    if (skinny_takes_stream(gate, M, lora->A[0], lora->B[0], lora->dtype, d.r) && skinny_takes_stream(up, M, lora->A[1], lora->B[1], lora->dtype, d.r) &&
-        ldx % 8 == 0 && (M <= 8 || ldx < kSkinnyLdx) && xq_aligned(x, 16) && skinny_stream_multi_supported(gu_jobs, 2, M)) {
+    if (skinny_takes_stream(gate, M, ldx, lora->A[0], lora->B[0], lora->dtype, d.r) && skinny_takes_stream(up, M, ldx, lora->A[1], lora->B[1], lora->dtype, d.r) &&
+        ldx % 8 == 0 && xq_aligned(x, 16) && skinny_stream_multi_supported(gu_jobs, 2, M)) {
         if ((rc = launch_skinny_stream(gu_jobs, 2, true, (const bf16_t*)x, ldx, M, lora->dtype, ws, (hipStream_t)stream))) return rc;
         XQ_CHECK_LAUNCH(who);
         return xq_linear_fwd(down, h, d.I, M, lora->A[2], lora->B[2], lora->dtype, d.r, lora->scaling, lora->bias[2], y, ldy, nullptr, ws,

@@ -48,8 +48,9 @@ __device__ __forceinline__ bf16x8 decode8(uint32_t w0, uint32_t w1, float s0, fl
     return __builtin_bit_cast(bf16x8, r);
 }
 
-// rows of x further apart than this take the tile kernels: the streaming kernels' addresses within eight rows are 32 bits wide
-constexpr int64_t kSkinnyLdx = 1ll << 28;
+// whether the streaming kernels take rows of x so many elements apart: their addresses within eight rows are 32 bits wide (2 * 7 * ldx
+// bytes and a row's 128); the one-launch kernels' are 64
+inline bool stream_takes_pitch(int64_t M, int64_t ldx) { return M == 1 || ldx < (1ll << 28); }
 
 void set_skinny_rows(int enabled);
 bool skinny_rows_enabled();
@@ -87,7 +88,7 @@ struct SkinnyRowsJob {
 };
 // the same jobs on the two-launch streaming kernels (xq_skinny.hip), M <= 64; `swiglu`: jobs 0 and 1 are gate and up and
 // job 0's y receives h = silu(gate) * up.  Each forward gives the bits of a launch of its own.
-bool skinny_takes_stream(const xq_weight* w, int64_t M, const void* lora_A, const void* lora_B, int lora_dtype, int r);
+bool skinny_takes_stream(const xq_weight* w, int64_t M, int64_t ldx, const void* lora_A, const void* lora_B, int lora_dtype, int r);
 bool skinny_stream_multi_supported(const SkinnyRowsJob* jobs, int n_jobs, int64_t M);
 int launch_skinny_stream(const SkinnyRowsJob* jobs, int n_jobs, bool swiglu, const bf16_t* x, int64_t ldx, int64_t M, int lora_dtype,
                          void* workspace, hipStream_t stream);

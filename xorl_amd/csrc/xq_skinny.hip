@@ -760,8 +760,8 @@ static int stream_splits(int64_t M, int64_t N, int64_t K) {
 }
 
 // whether a forward of this shape runs on the two launches of this file (and not in one, xq_skinny_rows.hip)
-bool skinny_takes_stream(const xq_weight* w, int64_t M, const void* lora_A, const void* lora_B, int lora_dtype, int r) {
-    return skinny_supported(w, M) && !(skinny_rows_enabled() && skinny_rows_supported(w, M, lora_A, lora_B, lora_dtype, r));
+bool skinny_takes_stream(const xq_weight* w, int64_t M, int64_t ldx, const void* lora_A, const void* lora_B, int lora_dtype, int r) {
+    return skinny_supported(w, M) && stream_takes_pitch(M, ldx) && !(skinny_rows_enabled() && skinny_rows_supported(w, M, lora_A, lora_B, lora_dtype, r));
 }
 
 int64_t skinny_workspace_bytes(int64_t M, int64_t N, int64_t K, int r_pad) {
@@ -846,7 +846,7 @@ int launch_skinny_stream(const SkinnyRowsJob* jobs, int n_jobs, bool swiglu, con
     const xq_weight* w0 = jobs[0].w;
     const int64_t K = w0->cols;
     const int sc = scale_mode(w0), mt = (int)xq_cdiv(M, 16);
-    XQ_REQUIRE(M <= 8 || ldx < kSkinnyLdx, "xq_linear_fwd: internal error: rows of x too far apart for the streaming kernel");
+    XQ_REQUIRE(stream_takes_pitch(M, ldx), "xq_linear_fwd: internal error: rows of x too far apart for the streaming kernel");
     StreamBatch b{};
     EpiBatch e{};
     uint8_t* ws = (uint8_t*)workspace;
@@ -968,11 +968,12 @@ int launch_skinny(const xq_weight* w, const bf16_t* x, int64_t ldx, int64_t M, c
     // region is the whole forward (both launches)
     const double wbytes = (double)xq_packed_bytes_per_expert(w) + (double)xq_scale_bytes_per_expert(w);
     const bool timed = xq_profile_mark_begin(stream, wbytes + 2.0 * M * K + 2.0 * M * N + 4.0 * r * (K + N));
-    // M <= 16: one launch, whole rows per block, where the shape and the LoRA operands fit it and a slot is free
+    // M <= 16: one launch, whole rows per block, where the shape and the LoRA operands fit it and a slot is free (XQ_ERR_UNSUPPORTED: none
+    // is, and the rows of x lie too far apart for the streaming kernels; nothing was launched)
     int rc = XQ_ERR_UNSUPPORTED;
     if (g_skinny_rows && skinny_rows_supported(w, M, lora_A, lora_B, lora_dtype, r))
         rc = launch_skinny_rows(w, x, ldx, M, lora_A, lora_B, r, scaling, bias, y, ldy, workspace, stream);
-    if (rc == XQ_ERR_UNSUPPORTED) {
+    if (rc == XQ_ERR_UNSUPPORTED && stream_takes_pitch(M, ldx)) {
         const SkinnyRowsJob job{w, lora_A, lora_B, rp ? r : 0, scaling, bias, y, ldy};
         rc = launch_skinny_stream(&job, 1, false, x, ldx, M, lora_dtype, workspace, stream);
     }

@@ -115,12 +115,14 @@ int xq_set_tile_policy(int policy);
 int xq_dense_route(int format, int forward, int64_t rows, int64_t n_out, int64_t k, int32_t plan[6]);
 
 /* What a forward of M rows of x, ldx elements apart, that keeps nothing for a backward runs on (factors of rank r or NULL; their
- * addresses count for their alignment), for tests: XQ_SKINNY_ONE_LAUNCH, XQ_SKINNY_STREAM (two launches that stream the weight),
- * XQ_SKINNY_NONE (the products of xq_dense_route), -1 where the library does not take it.  No counterpart in the reference. */
+ * addresses count for their alignment), for tests: XQ_SKINNY_ONE_LAUNCH, XQ_SKINNY_STREAM (two launches that stream the weight; plan:
+ * its K splits and, launched alone, the tiles of 16 weight rows of a block, otherwise 0), XQ_SKINNY_NONE (the products of
+ * xq_dense_route), -1 where the library does not take it.  No counterpart in the reference. */
 #define XQ_SKINNY_NONE 0
 #define XQ_SKINNY_ONE_LAUNCH 1
 #define XQ_SKINNY_STREAM 2
-int xq_skinny_route(const xq_weight* w, int64_t M, int64_t ldx, const void* lora_A, const void* lora_B, int lora_dtype, int r);
+int xq_skinny_route(const xq_weight* w, int64_t M, int64_t ldx, const void* lora_A, const void* lora_B, int lora_dtype, int r,
+                    int32_t plan[2]);
 
 /* The 256x256 tile kernel (unsplit launches) is a persistent program: one block per compute unit walks the
  * tiles b, b + grid, ... and requests its next tile's first operands before it stores the finished tile.

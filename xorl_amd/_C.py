@@ -94,8 +94,8 @@ _SIGNATURES = {
     "xq_profile_collect": (_INT, [_P, _P, _P]),
     # format, forward, rows, n_out, k, plan (six int32)
     "xq_dense_route": (_INT, [_INT, _INT, _I64, _I64, _I64, _P]),
-    # w, M, ldx, lora_A, lora_B, lora_dtype, r
-    "xq_skinny_route": (_INT, [_W, _I64, _I64, _P, _P, _INT, _INT]),
+    # w, M, ldx, lora_A, lora_B, lora_dtype, r, plan (two int32)
+    "xq_skinny_route": (_INT, [_W, _I64, _I64, _P, _P, _INT, _INT, _P]),
     "xq_decode": (_INT, [_W, _P, _INT, _P]),
     "xq_quantize_workspace_bytes": (_I64, [_INT, _I64, _I64]),
     # format, layout, x, x_dtype, rows, cols, group, amax_scale, global_amax, codes, scales, scale_dtype, global_scale, ws, ws_bytes, stream

@@ -915,10 +915,13 @@ static bool takes_skinny(const xq_weight* w, int64_t M, int64_t ldx, const void*
     return g_skinny_enabled && skinny_supported(w, M) &&
            (stream_takes_pitch(M, ldx) || (skinny_rows_enabled() && skinny_rows_supported(w, M, lora_A, lora_B, lora_dtype, r)));
 }
-extern "C" int xq_skinny_route(const xq_weight* w, int64_t M, int64_t ldx, const void* lora_A, const void* lora_B, int lora_dtype, int r) {
-    if (!w || M < 1 || r < 0 || r > 64 || check_dense(w, "xq_skinny_route")) return -1;
+extern "C" int xq_skinny_route(const xq_weight* w, int64_t M, int64_t ldx, const void* lora_A, const void* lora_B, int lora_dtype, int r, int32_t plan[2]) {
+    if (!w || !plan || M < 1 || r < 0 || r > 64 || check_dense(w, "xq_skinny_route")) return -1;
+    plan[0] = plan[1] = 0;
     if (!takes_skinny(w, M, ldx, lora_A, lora_B, lora_dtype, r)) return XQ_SKINNY_NONE;
-    return skinny_takes_stream(w, M, ldx, lora_A, lora_B, lora_dtype, r) ? XQ_SKINNY_STREAM : XQ_SKINNY_ONE_LAUNCH;
+    if (!skinny_takes_stream(w, M, ldx, lora_A, lora_B, lora_dtype, r)) return XQ_SKINNY_ONE_LAUNCH;
+    skinny_stream_plan(w, M, plan);
+    return XQ_SKINNY_STREAM;
 }
 
 extern "C" int xq_linear_fwd(const xq_weight* w, const void* x, int64_t ldx, int64_t M, const void* lora_A,

@@ -89,6 +89,7 @@ struct SkinnyRowsJob {
 // the same jobs on the two-launch streaming kernels (xq_skinny.hip), M <= 64; `swiglu`: jobs 0 and 1 are gate and up and
 // job 0's y receives h = silu(gate) * up.  Each forward gives the bits of a launch of its own.
 bool skinny_takes_stream(const xq_weight* w, int64_t M, int64_t ldx, const void* lora_A, const void* lora_B, int lora_dtype, int r);
+void skinny_stream_plan(const xq_weight* w, int64_t M, int32_t* plan);   // of a launch alone: K splits, row tiles of a block
 bool skinny_stream_multi_supported(const SkinnyRowsJob* jobs, int n_jobs, int64_t M);
 int launch_skinny_stream(const SkinnyRowsJob* jobs, int n_jobs, bool swiglu, const bf16_t* x, int64_t ldx, int64_t M, int lora_dtype,
                          void* workspace, hipStream_t stream);

@@ -30,6 +30,7 @@
 // and x waits for the weights requested before it.  Gate and up of an MLP, which are those very products, are 8 % ahead as one launch.)
 #include <stdlib.h>
 
+#include <algorithm>
 #include <atomic>
 
 #include "xq_common.h"
@@ -699,10 +700,32 @@ stream_epilogue_kernel(int32_t M, int32_t first1, int32_t first2, int32_t first3
 
 static inline int64_t al256(int64_t b) { return (b + 255) & ~(int64_t)255; }
 
+// (the storages that xq_validate_weight and skinny_supported leave: nf4 fp32, nvfp4 e4m3 or fp32, int4 fp32 or bf16)
+static int scale_mode(const xq_weight* w) {
+    if (w->format == XQ_FMT_FP8) return kScFp8;
+    if (w->format == XQ_FMT_NF4) return kScDealt;
+    if (w->format == XQ_FMT_NVFP4) return w->scale_dtype == XQ_SCALE_E4M3 ? kScDealt : kScHalf;
+    if (w->group == 128 && w->scale_dtype == XQ_SCALE_BF16) return kScInt4Window;
+    return w->group % 16 == 0 && w->cols % w->group == 0 ? kScHalf : kScUse;
+}
+
+// (the uncommon scale storages keep more registers per row tile)
+constexpr int row_tiles_max(int fmt, int sc) { return sc >= kScHalf ? 2 : fmt == XQ_FMT_NF4 ? 4 : 6; }
+
+// What the plans have to know of a storage: the row tiles of a block at most, and up to how many tiles (MT RT) two blocks share a compute
+// unit (StreamGeo::PAIR).
+enum { kPlanCommon = 0, kPlanNf4 = 1, kPlanUncommon = 2, kPlanClasses = 3 };
+static int plan_class(const xq_weight* w) { return scale_mode(w) >= kScHalf ? kPlanUncommon : w->format == XQ_FMT_NF4 ? kPlanNf4 : kPlanCommon; }
+struct PlanLimits {
+    int row_tiles, pair_max;
+};
+static const PlanLimits kPlanLimits[kPlanClasses] = {
+    {row_tiles_max(XQ_FMT_INT4, kScInt4Window), 4}, {row_tiles_max(XQ_FMT_NF4, kScDealt), 3}, {row_tiles_max(XQ_FMT_INT4, kScHalf), 4}};
+
 // What a launch of `blocks` blocks of RT row tiles and `steps` steps takes beyond a constant, in us, from a sweep of every (row tiles,
 // splits) at M 24..64 on seven widths and depths of int4 and block-fp8 (within 10 % of the times; the pair it picks is 1.2 % behind
 // the best on average, 8 % at worst): rounds of the chip, and in a block the half steps of a wave, each for its weights and its x.  Two
-// blocks are resident per compute unit where StreamGeo says so (MT RT up to pair_max, 3 with the levels of nf4 and 4 otherwise).
+// blocks are resident per compute unit where MT RT is pair_max at most.
 static double stream_run_us(int64_t blocks, int rt, int steps, int mt, int pair_max) {
     const int per_cu = mt < 4 && mt * rt <= pair_max ? 2 : 1;
     const int64_t cus = num_cus();
@@ -712,14 +735,14 @@ static double stream_run_us(int64_t blocks, int rt, int steps, int mt, int pair_
 }
 static const int kRowTiles[] = {1, 2, 3, 4, 6};
 // row tiles of a block by that estimate (they change nothing in the results); `tiles`, `splits` of each forward of the launch
-static int stream_row_tiles(const int* tiles, const int* splits, int n, int steps, int mt, int rt_max, int pair_max, double* us) {
+static int stream_row_tiles(const int* tiles, const int* splits, int n, int steps, int mt, const PlanLimits& lim, double* us) {
     int best = 1;
     double cost = 0;
     for (int rt : kRowTiles) {
-        if (rt > rt_max) break;
+        if (rt > lim.row_tiles) break;
         int64_t blocks = 0;
         for (int i = 0; i < n; ++i) blocks += xq_cdiv(tiles[i], (int64_t)rt) * splits[i];
-        const double c = stream_run_us(blocks, rt, steps, mt, pair_max);
+        const double c = stream_run_us(blocks, rt, steps, mt, lim.pair_max);
         if (cost == 0 || c < cost) { cost = c; best = rt; }
     }
     if (us) *us = cost;
@@ -727,9 +750,9 @@ static int stream_row_tiles(const int* tiles, const int* splits, int n, int step
 }
 // steps of a split at most (a lane holds one block-fp8 scale of a wave's steps)
 constexpr int kStreamSteps = 64 * kStreamWaves;
-// K splits of a forward, by its own shape: the cheapest sum of that and of the partial sums' trip (written and read back, with what
+// K splits of a forward, by its own shape and storage: the cheapest sum of that and of the partial sums' trip (written and read back, with what
 // waits for them: 1.7 TB/s)
-static int make_stream_splits(int64_t M, int64_t N, int64_t K) {
+static int make_stream_splits(int cls, int64_t M, int64_t N, int64_t K) {
     const int ct = (int)(K >> 7), tiles = (int)(N / 16);
     const int mt = (int)xq_cdiv(M, 16);
     const int least = (int)xq_cdiv(ct, kStreamSteps);
@@ -744,18 +767,30 @@ static int make_stream_splits(int64_t M, int64_t N, int64_t K) {
         last_steps = steps;
         if (best && (s * M * N * 4 > (16ll << 20))) break;
         double c;
-        stream_row_tiles(&tiles, &s, 1, steps, mt, 6, 4, &c);
+        stream_row_tiles(&tiles, &s, 1, steps, mt, kPlanLimits[cls], &c);
         c += (double)s * M * N * 8.0 / 1.7e6;
         if (best == 0 || c < worth * best_cost) { best = s; best_cost = c; }
     }
     return best;
 }
 
-static int stream_splits(int64_t M, int64_t N, int64_t K) {
+static int stream_splits(int cls, int64_t M, int64_t N, int64_t K) {
+    static thread_local PlanSlot<int> kept[64];
+    const PlanKey key{M, N, K, num_cus(), cls};
+    PlanSlot<int>& e = kept[key.slot()];
+    if (!(e.key == key)) e = PlanSlot<int>{key, make_stream_splits(cls, M, N, K)};
+    return e.value;
+}
+// the most that any storage takes
+static int most_stream_splits(int64_t M, int64_t N, int64_t K) {
     static thread_local PlanSlot<int> kept[64];
     const PlanKey key{M, N, K, num_cus(), 0};
     PlanSlot<int>& e = kept[key.slot()];
-    if (!(e.key == key)) e = PlanSlot<int>{key, make_stream_splits(M, N, K)};
+    if (!(e.key == key)) {
+        int most = 0;
+        for (int cls = 0; cls < kPlanClasses; ++cls) most = std::max(most, make_stream_splits(cls, M, N, K));
+        e = PlanSlot<int>{key, most};
+    }
     return e.value;
 }
 
@@ -764,11 +799,17 @@ bool skinny_takes_stream(const xq_weight* w, int64_t M, int64_t ldx, const void*
     return skinny_supported(w, M) && stream_takes_pitch(M, ldx) && !(skinny_rows_enabled() && skinny_rows_supported(w, M, lora_A, lora_B, lora_dtype, r));
 }
 
+void skinny_stream_plan(const xq_weight* w, int64_t M, int32_t* plan) {
+    const int cls = plan_class(w), tiles = (int)(w->rows / 16), splits = stream_splits(cls, M, w->rows, w->cols);
+    plan[0] = splits;
+    plan[1] = stream_row_tiles(&tiles, &splits, 1, (int)xq_cdiv(w->cols >> 7, splits), (int)xq_cdiv(M, 16), kPlanLimits[cls], nullptr);
+}
+
 int64_t skinny_workspace_bytes(int64_t M, int64_t N, int64_t K, int r_pad) {
     if (K < 128 || N < 16) return 256;
     const int rp = r_pad ? r_pad : 16;
     // (never less than a partial sum for every 32, 16 or 8 steps, whatever the plan: what callers have always been asked for)
-    const int64_t s = stream_splits(M, N, K), held = xq_cdiv(K >> 7, M <= 16 ? 32 : M <= 32 ? 16 : 8);
+    const int64_t s = most_stream_splits(M, N, K), held = xq_cdiv(K >> 7, M <= 16 ? 32 : M <= 32 ? 16 : 8);
     return al256((s > held ? s : held) * M * N * 4) + al256((K >> 7) * M * rp * 4) + 256;
 }
 
@@ -780,18 +821,6 @@ bool skinny_supported(const xq_weight* w, int64_t M) {
     if (w->format == XQ_FMT_INT4 && (w->group % 8 != 0)) return false;
     return true;
 }
-
-// (the storages that xq_validate_weight and skinny_supported leave: nf4 fp32, nvfp4 e4m3 or fp32, int4 fp32 or bf16)
-static int scale_mode(const xq_weight* w) {
-    if (w->format == XQ_FMT_FP8) return kScFp8;
-    if (w->format == XQ_FMT_NF4) return kScDealt;
-    if (w->format == XQ_FMT_NVFP4) return w->scale_dtype == XQ_SCALE_E4M3 ? kScDealt : kScHalf;
-    if (w->group == 128 && w->scale_dtype == XQ_SCALE_BF16) return kScInt4Window;
-    return w->group % 16 == 0 && w->cols % w->group == 0 ? kScHalf : kScUse;
-}
-
-// (the uncommon scale storages keep more registers per row tile)
-constexpr int row_tiles_max(int fmt, int sc) { return sc >= kScHalf ? 2 : fmt == XQ_FMT_NF4 ? 4 : 6; }
 
 template <int FMT, int SC, int MT, int RT>
 static int launch_stream_one(const StreamBatch& b, const int* first, const bf16_t* x, int64_t ldx, int64_t M, int64_t K, hipStream_t s) {
@@ -845,7 +874,7 @@ int launch_skinny_stream(const SkinnyRowsJob* jobs, int n_jobs, bool swiglu, con
                          void* workspace, hipStream_t stream) {
     const xq_weight* w0 = jobs[0].w;
     const int64_t K = w0->cols;
-    const int sc = scale_mode(w0), mt = (int)xq_cdiv(M, 16);
+    const int sc = scale_mode(w0), cls = plan_class(w0), mt = (int)xq_cdiv(M, 16);
     XQ_REQUIRE(stream_takes_pitch(M, ldx), "xq_linear_fwd: internal error: rows of x too far apart for the streaming kernel");
     StreamBatch b{};
     EpiBatch e{};
@@ -857,7 +886,7 @@ int launch_skinny_stream(const SkinnyRowsJob* jobs, int n_jobs, bool swiglu, con
         const int rp = j.r > 0 ? (j.r + 15) / 16 * 16 : 0;
         const int64_t N = j.w->rows;
         StreamJob& g = b.job[i];
-        g.splits = stream_splits(M, N, K);
+        g.splits = stream_splits(cls, M, N, K);
         g.packed = (const uint8_t*)j.w->packed; g.scales = (const uint8_t*)j.w->scales; g.global_scale = j.w->global_scale;
         g.N = (int)N; g.group = j.w->group; g.scale_dtype = j.w->scale_dtype;
         g.chunk_q = (int)(K >> 7) / g.splits; g.chunk_rem = (int)(K >> 7) % g.splits;
@@ -875,7 +904,7 @@ int launch_skinny_stream(const SkinnyRowsJob* jobs, int n_jobs, bool swiglu, con
     }
     int tiles[kStreamJobs], splits[kStreamJobs];
     for (int i = 0; i < n_jobs; ++i) { tiles[i] = b.job[i].N / 16; splits[i] = b.job[i].splits; }
-    const int rt = stream_row_tiles(tiles, splits, n_jobs, steps, mt, row_tiles_max(w0->format, sc), w0->format == XQ_FMT_NF4 ? 3 : 4, nullptr);
+    const int rt = stream_row_tiles(tiles, splits, n_jobs, steps, mt, kPlanLimits[cls], nullptr);
     int first[5] = {0, 0, 0, 0, 0}, efirst[5] = {0, 0, 0, 0, 0};
     for (int i = 0; i < kStreamJobs; ++i) {
         first[i + 1] = first[i];

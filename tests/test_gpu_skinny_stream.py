@@ -5,7 +5,7 @@ import pytest
 import torch
 
 from oracle import recipe as R
-from tests.util_cases import close, gen, make_dense_module
+from tests.util_cases import close, gen, make_dense_module, skinny_route
 
 pytestmark = pytest.mark.gpu
 
@@ -135,3 +135,22 @@ def test_rows_of_x_a_gigabyte_apart(hip_device, K):
             for a, b in zip(qlora_linears_forward([g, u], far[:M]), qlora_linears_forward([g, u], packed)):
                 close(a.cpu(), b.cpu().double(), 1e-2)
             close(qlora_mlp_forward(g, u, d, far[:M]).cpu(), qlora_mlp_forward(g, u, d, packed).cpu().double(), 1e-2)
+
+
+@pytest.mark.parametrize("fmt,N,K,tiles", [                       # rows of x: the plan's row tiles
+    ("int4", 4480, 4096, {17: 5, 33: 5, 49: 5}),
+    ("int4", 27648, 2048, {33: 7}),
+    ("nf4", 18560, 1024, {3: 5, 17: 5}),                          # the nf4 levels beside odd numbers of tiles
+    ("nf4", 6400, 5120, {8: 8}),
+    ("block_fp8", 27648, 2944, {17: 7}),                          # an odd number of steps
+])
+def test_five_seven_and_eight_row_tiles(hip_device, fmt, N, K, tiles):
+    m, w_ref = make_dense_module(fmt, N, K, 24, 48, seed=N + K, device=hip_device)
+    A, B = m.lora_A.detach().cpu(), m.lora_B.detach().cpu()
+    for M, rt in tiles.items():
+        assert skinny_route(fmt, N, K, M, K, r=24)[2] == rt
+        x = gen((M, K), 1.0, M, torch.bfloat16)
+        with torch.no_grad():
+            y = m(x.to(hip_device))
+        ex = R.linear_fwd_bwd_exact(x, w_ref, A, B, m.scaling, torch.zeros(M, N, dtype=torch.bfloat16))
+        close(y.cpu(), ex["y"], 1e-2)                             # (the bound of every forward above)

@@ -198,23 +198,12 @@ def test_build_refuses_scratch_under_hand_counted_reads():
         b.check_scratch(b._split_remarks(output(other, 0) + "\n" + output(dec, 80))[0], guarded)
 
 
-def _skinny_route(fmt, N, K, M, ldx, scale_dtype=None):
-    """xq_skinny_route of a weight without factors: what it runs on, its K splits and its row tiles"""
-    from xorl_amd import _C
-
-    w = _C.XqWeight()
-    w.format, w.layout, w.rows, w.cols, w.num_experts = _C.FORMATS[fmt], _C.XQ_LAYOUT_FLAT, N, K, 1
-    w.group = {"int4": 128, "nvfp4": 16, "block_fp8": 128, "nf4": 64}[fmt]
-    w.scale_dtype = {"int4": _C.XQ_SCALE_BF16, "nvfp4": _C.XQ_SCALE_E4M3}.get(fmt, _C.XQ_SCALE_F32) if scale_dtype is None else scale_dtype
-    w.packed = w.scales = w.global_scale = 4096              # (addresses: nothing is read)
-    plan = (ctypes.c_int32 * 2)()
-    return (_C.lib().xq_skinny_route(ctypes.byref(w), M, ldx, None, None, _C.XQ_DT_F32, 0, plan), *plan)
-
-
 @pytest.mark.parametrize("K,near", [(1152, 2), (2048, 1)])     # a depth of the streaming kernels and one of the one-launch kernels (to 16 rows)
 def test_rows_of_x_far_apart_leave_the_streaming_kernels(K, near):
     """Their addresses within eight rows are 32 bits wide: 2 * 7 * ldx bytes and a row's 128 at most.  One row has no pitch."""
-    route = lambda M, ldx: _skinny_route("int4", 512, K, M, ldx)[0]
+    from tests.util_cases import skinny_route
+
+    route = lambda M, ldx: skinny_route("int4", 512, K, M, ldx)[0]
     for M in (1, 2, 3, 8, 9, 16, 17, 64):
         here = near if M <= 16 else 2
         assert route(M, K) == here and route(M, (1 << 28) - 8) == here, M
@@ -226,16 +215,16 @@ def test_rows_of_x_far_apart_leave_the_streaming_kernels(K, near):
 
 
 def test_streaming_plans_know_the_storage():
-    """What a storage allows (int4 with fp32 scales holds two row tiles, nf4's levels take the LDS of a second block at four) decides its
-    own K splits, and every workspace holds the sums of the plan with the most."""
+    """What a storage allows (int4 with fp32 scales holds two row tiles) and what its codes cost (nf4's are looked up) decide its own K
+    splits, and every workspace holds the sums of the plan with the most."""
+    from tests.util_cases import skinny_route
     from xorl_amd import _C
 
-    # (64 rows of 12288 -> 4096: two splits of two row tiles, where bf16 scales have four of four; 3 rows of 4992 -> 13056: one and five)
-    assert _skinny_route("int4", 4096, 12288, 64, 12288, _C.XQ_SCALE_F32)[1:] != _skinny_route("int4", 4096, 12288, 64, 12288)[1:]
-    assert _skinny_route("nf4", 13056, 4992, 3, 4992)[1] != _skinny_route("int4", 13056, 4992, 3, 4992)[1]
+    assert skinny_route("int4", 4096, 12288, 64, 12288, _C.XQ_SCALE_F32)[1:] == (2, 2) != skinny_route("int4", 4096, 12288, 64, 12288)[1:]
+    assert skinny_route("nf4", 8192, 5120, 64, 5120)[1:] != skinny_route("int4", 8192, 5120, 64, 5120)[1:]
     for N, K in ((1024, 1024), (4096, 4096), (4096, 12288), (13056, 4992), (16384, 2048)):
         for M in (1, 17, 33, 64):
             for fmt, sdt, most in (("int4", None, 8), ("int4", _C.XQ_SCALE_F32, 2), ("nvfp4", _C.XQ_SCALE_F32, 2), ("nf4", None, 8), ("block_fp8", None, 8)):
-                where, splits, tiles = _skinny_route(fmt, N, K, M, K, sdt)
+                where, splits, tiles = skinny_route(fmt, N, K, M, K, sdt)
                 assert 1 <= tiles <= most if where == 2 else where == 1, (fmt, sdt, N, K, M)
                 assert _C.lib().xq_linear_workspace_bytes_fmt(_C.FORMATS[fmt], M, N, K, 16) >= splits * M * N * 4 + (K // 128) * M * 16 * 4

@@ -81,6 +81,21 @@ def dense_route(fmt: str, forward: bool, rows: int, n_out: int, k: int) -> tuple
     return (["tiles", "image", "mid"][_C.lib().xq_dense_route(_C.FORMATS[fmt], int(forward), rows, n_out, k, plan)], *plan)
 
 
+def skinny_route(fmt, N, K, M, ldx, scale_dtype=None, r=0):
+    """xq_skinny_route (include/xq.h) of a weight with fp32 factors of rank r: what it runs on, its K splits and its row tiles"""
+    import ctypes
+
+    from xorl_amd import _C
+
+    w = _C.XqWeight()
+    w.format, w.layout, w.rows, w.cols, w.num_experts = _C.FORMATS[fmt], _C.XQ_LAYOUT_FLAT, N, K, 1
+    w.group = {"int4": 128, "nvfp4": 16, "block_fp8": 128, "nf4": 64}[fmt]
+    w.scale_dtype = {"int4": _C.XQ_SCALE_BF16, "nvfp4": _C.XQ_SCALE_E4M3}.get(fmt, _C.XQ_SCALE_F32) if scale_dtype is None else scale_dtype
+    w.packed = w.scales = w.global_scale = 4096              # (addresses: nothing is read)
+    plan = (ctypes.c_int32 * 2)()
+    return (_C.lib().xq_skinny_route(ctypes.byref(w), M, ldx, 4096 if r else None, 4096 if r else None, _C.XQ_DT_F32, r, plan), *plan)
+
+
 def oracle_decode_dense(m) -> torch.Tensor:
     """Decode a (CPU) module's packed state with the numpy oracle -> bf16 [N, K]."""
     N, K = m.out_features, m.in_features

@@ -67,14 +67,21 @@ enum { kScFp8 = 0, kScInt4Window = 1, kScDealt = 2, kScHalf = 3, kScUse = 4 };
 // scales lie where their elements may: a pair of words from any byte (one global_load_dwordx2 like an aligned one)
 typedef u32x2 u32x2_a1 __attribute__((aligned(1)));
 
+// bytes of LDS beside the waves' parts: the levels of nf4
+constexpr int stream_levels(int fmt) { return fmt == XQ_FMT_NF4 ? 64 : 0; }
+// Whether half a step of x (16 MT rows) and 128 bytes of 16 RT weight rows for each wave fit a block's LDS, and whether two such blocks share
+// a compute unit (more tiles are too many registers for that).
+constexpr bool stream_fits(int levels, int mt, int rt) { return kStreamWaves * 2048 * (mt + rt) + levels <= 160 * 1024; }
+constexpr bool stream_pairs(int levels, int mt, int rt) { return mt < 4 && mt * rt <= 4 && kStreamWaves * 2048 * (mt + rt) + levels <= 80 * 1024; }
+
 // What a wave keeps in LDS: XB half steps of x (16 MT rows of 64 elements each) and WB units of weights (128 bytes of each of its 16 RT
 // rows: a step of block-fp8, two steps of the 4-bit formats).
 template <int FMT, int MT, int RT>
 struct StreamGeo {
     static constexpr int HPW = FMT == XQ_FMT_FP8 ? 2 : 4;          // half steps of a weight unit
     static constexpr int XH = MT * 2048, WU = RT * 2048;
-    static constexpr bool PAIR = MT < 4 && MT * RT <= (FMT == XQ_FMT_NF4 ? 3 : 4);     // two blocks per compute unit (the levels of nf4 take the last bytes)
-    static constexpr int ROOM = (PAIR ? 80 : 160) * 128 - (FMT == XQ_FMT_NF4 ? 16 : 0);
+    static constexpr bool PAIR = stream_pairs(stream_levels(FMT), MT, RT);
+    static constexpr int ROOM = ((PAIR ? 80 : 160) * 1024 - stream_levels(FMT)) / kStreamWaves;
     static constexpr int XB = 3 * XH + 2 * WU <= ROOM ? 3 : 2 * XH + WU <= ROOM ? 2 : 1;
     static constexpr int WB = XB * XH + 2 * WU <= ROOM ? 2 : 1;
     static constexpr int WAVE = XB * XH + WB * WU;
@@ -709,67 +716,69 @@ static int scale_mode(const xq_weight* w) {
     return w->group % 16 == 0 && w->cols % w->group == 0 ? kScHalf : kScUse;
 }
 
-// (the uncommon scale storages keep more registers per row tile)
-constexpr int row_tiles_max(int fmt, int sc) { return sc >= kScHalf ? 2 : fmt == XQ_FMT_NF4 ? 4 : 6; }
-
-// What the plans have to know of a storage: the row tiles of a block at most, and up to how many tiles (MT RT) two blocks share a compute
-// unit (StreamGeo::PAIR).
-enum { kPlanCommon = 0, kPlanNf4 = 1, kPlanUncommon = 2, kPlanClasses = 3 };
-static int plan_class(const xq_weight* w) { return scale_mode(w) >= kScHalf ? kPlanUncommon : w->format == XQ_FMT_NF4 ? kPlanNf4 : kPlanCommon; }
-struct PlanLimits {
-    int row_tiles, pair_max;
-};
-static const PlanLimits kPlanLimits[kPlanClasses] = {
-    {row_tiles_max(XQ_FMT_INT4, kScInt4Window), 4}, {row_tiles_max(XQ_FMT_NF4, kScDealt), 3}, {row_tiles_max(XQ_FMT_INT4, kScHalf), 4}};
-
-// What a launch of `blocks` blocks of RT row tiles and `steps` steps takes beyond a constant, in us, from a sweep of every (row tiles,
-// splits) at M 24..64 on seven widths and depths of int4 and block-fp8 (within 10 % of the times; the pair it picks is 1.2 % behind
-// the best on average, 8 % at worst): rounds of the chip, and in a block the half steps of a wave, each for its weights and its x.  Two
-// blocks are resident per compute unit where MT RT is pair_max at most.
-static double stream_run_us(int64_t blocks, int rt, int steps, int mt, int pair_max) {
-    const int per_cu = mt < 4 && mt * rt <= pair_max ? 2 : 1;
-    const int64_t cus = num_cus();
-    const double rounds = (double)xq_cdiv(blocks, cus * per_cu), halves = 2.0 * xq_cdiv(steps, kStreamWaves);
-    const double on_cu = (double)xq_cdiv(blocks, cus) < rounds * per_cu ? (double)xq_cdiv(blocks, cus) : rounds * per_cu;
-    return rounds * (0.5 + halves * (0.25 * rt + 0.17 * mt) * (1.0 + 0.8 * (on_cu / rounds - 1.0)));
+// ---- plans
+// What the plans have to know of a storage: the row tiles of a block at most (the uncommon scale storages keep more registers per tile),
+// the LDS it takes beside the waves' parts, and what a half step costs for each row tile, in us.
+constexpr int row_tiles_max(int sc) { return sc >= kScHalf ? 2 : 8; }
+enum { kPlan4Bit = 0, kPlanFp8 = 1, kPlanNf4 = 2, kPlanUncommon = 3, kPlanClasses = 4 };
+static int plan_class(const xq_weight* w) {
+    return scale_mode(w) >= kScHalf ? kPlanUncommon : w->format == XQ_FMT_FP8 ? kPlanFp8 : w->format == XQ_FMT_NF4 ? kPlanNf4 : kPlan4Bit;
 }
-static const int kRowTiles[] = {1, 2, 3, 4, 6};
-// row tiles of a block by that estimate (they change nothing in the results); `tiles`, `splits` of each forward of the launch
-static int stream_row_tiles(const int* tiles, const int* splits, int n, int steps, int mt, const PlanLimits& lim, double* us) {
+struct PlanClass {
+    int row_tiles, levels;
+    double row_us;
+};
+static const PlanClass kPlans[kPlanClasses] = {
+    {row_tiles_max(kScInt4Window), 0, 0.335}, {row_tiles_max(kScFp8), 0, 0.23}, {row_tiles_max(kScDealt), stream_levels(XQ_FMT_NF4), 0.54}, {row_tiles_max(kScHalf), 0, 0.335}};
+
+// The row tiles of a block that make a launch shortest by an estimate of what it takes beyond a constant, in us (they change nothing in
+// the results); `tiles`, `splits` of each forward of the launch, `steps` of the longest split.  Rounds of the chip, and in a block the half
+// steps of a wave, each for its weights, its x and their products; a second block on the compute unit nearly doubles them.
+// The constants, and those of make_stream_splits, come from a sweep of every (splits, row tiles) at 1 to 64 rows in all formats on 28
+// single weights and seven pairs: where a tile of five or seven rows spares a round of the chip the whole forward is up to 11 per cent
+// shorter (us, MLP 3712/9344 of 24 rows int4 46.3 -> 42.6, 4096/12416 of 24 rows int4 52.2 with four tiles, 48.6 with seven, nf4 66.0 -> 61.2).
+// The plans they choose are 2 per cent behind the best of the sweep on average.
+static int stream_row_tiles(const int* tiles, const int* splits, int n, int steps, int mt, const PlanClass& c, double* us) {
+    const int cus = num_cus(), halves = 2 * ((steps + kStreamWaves - 1) / kStreamWaves);
     int best = 1;
-    double cost = 0;
-    for (int rt : kRowTiles) {
-        if (rt > lim.row_tiles) break;
-        int64_t blocks = 0;
-        for (int i = 0; i < n; ++i) blocks += xq_cdiv(tiles[i], (int64_t)rt) * splits[i];
-        const double c = stream_run_us(blocks, rt, steps, mt, lim.pair_max);
-        if (cost == 0 || c < cost) { cost = c; best = rt; }
+    double least = 0;
+    for (int rt = 1; rt <= c.row_tiles && stream_fits(c.levels, mt, rt); ++rt) {
+        int blocks = 0;
+        for (int i = 0; i < n; ++i) blocks += (tiles[i] + rt - 1) / rt * splits[i];
+        const bool pair = stream_pairs(c.levels, mt, rt);
+        const int per_cu = pair ? 2 : 1, rounds = (blocks + cus * per_cu - 1) / (cus * per_cu), on_cu = std::min((blocks + cus - 1) / cus, rounds * per_cu);
+        const double half = c.row_us * rt + 0.25 * mt + 0.009 * rt * mt;
+        const double t = rounds * ((pair ? 2.75 : 3.7) + 0.13 * rt * mt + halves * half * (1.0 + 0.92 * ((double)on_cu / rounds - 1.0)));
+        if (least == 0 || t < least) { least = t; best = rt; }
     }
-    if (us) *us = cost;
+    if (us) *us = least;
     return best;
 }
 // steps of a split at most (a lane holds one block-fp8 scale of a wave's steps)
 constexpr int kStreamSteps = 64 * kStreamWaves;
-// K splits of a forward, by its own shape and storage: the cheapest sum of that and of the partial sums' trip (written and read back, with what
-// waits for them: 1.7 TB/s)
+// K splits of a forward, by its own shape and storage: the cheapest sum of that and of the epilogue's share, 0.44 us a split and the partial
+// sums' trip.  Weights twice as wide as deep are mostly gate and up of an MLP, whose one launch has other rounds than a weight alone: half
+// of what a pair takes counts too (nvfp4 4096 -> 2 x 12288 of 19 rows, the whole MLP: 49.4 us with two splits, 44.1 with one; alone they
+// are level).
 static int make_stream_splits(int cls, int64_t M, int64_t N, int64_t K) {
-    const int ct = (int)(K >> 7), tiles = (int)(N / 16);
-    const int mt = (int)xq_cdiv(M, 16);
-    const int least = (int)xq_cdiv(ct, kStreamSteps);
-    // more splits of a wide weight must be clearly the shorter: beside a second one (gate and up) one round of blocks becomes two (nvfp4
-    // 4096 -> 2 x 12288 of 19 rows, the whole MLP: 49.4 us with two splits, 44.1 with one; alone they are level)
-    const double worth = tiles > 2 * num_cus() ? 0.92 : 1.0;
+    const int ct = (int)(K >> 7), mt = (int)xq_cdiv(M, 16), least = (int)xq_cdiv(ct, kStreamSteps);
+    const int tiles[2] = {(int)(N / 16), (int)(N / 16)};
     int best = 0, last_steps = 0;
     double best_cost = 0;
     for (int s = least; s <= ct && (s <= 64 || best == 0); ++s) {
-        const int steps = (int)xq_cdiv(ct, s);
+        const int steps = (int)xq_cdiv(ct, s), splits[2] = {s, s};
         if (steps == last_steps) continue;                         // more splits, none of them shorter
         last_steps = steps;
-        if (best && (s * M * N * 4 > (16ll << 20))) break;
-        double c;
-        stream_row_tiles(&tiles, &s, 1, steps, mt, kPlanLimits[cls], &c);
-        c += (double)s * M * N * 8.0 / 1.7e6;
-        if (best == 0 || c < worth * best_cost) { best = s; best_cost = c; }
+        if (best && (s * M * N * 4 > (16ll << 20) || steps < kStreamWaves / 2)) break;
+        const double sums = s * (0.44 + M * N * 8 * 0.14e-6);
+        double c, two = 0;
+        stream_row_tiles(tiles, splits, 1, steps, mt, kPlans[cls], &c);
+        c += sums;
+        if (N >= 2 * K) {
+            stream_row_tiles(tiles, splits, 2, steps, mt, kPlans[cls], &two);
+            c += 0.5 * (two + 2 * sums);
+        }
+        if (best == 0 || c < best_cost) { best = s; best_cost = c; }
     }
     return best;
 }
@@ -802,7 +811,7 @@ bool skinny_takes_stream(const xq_weight* w, int64_t M, int64_t ldx, const void*
 void skinny_stream_plan(const xq_weight* w, int64_t M, int32_t* plan) {
     const int cls = plan_class(w), tiles = (int)(w->rows / 16), splits = stream_splits(cls, M, w->rows, w->cols);
     plan[0] = splits;
-    plan[1] = stream_row_tiles(&tiles, &splits, 1, (int)xq_cdiv(w->cols >> 7, splits), (int)xq_cdiv(M, 16), kPlanLimits[cls], nullptr);
+    plan[1] = stream_row_tiles(&tiles, &splits, 1, (int)xq_cdiv(w->cols >> 7, splits), (int)xq_cdiv(M, 16), kPlans[cls], nullptr);
 }
 
 int64_t skinny_workspace_bytes(int64_t M, int64_t N, int64_t K, int r_pad) {
@@ -824,7 +833,7 @@ bool skinny_supported(const xq_weight* w, int64_t M) {
 
 template <int FMT, int SC, int MT, int RT>
 static int launch_stream_one(const StreamBatch& b, const int* first, const bf16_t* x, int64_t ldx, int64_t M, int64_t K, hipStream_t s) {
-    constexpr int lds = kStreamWaves * StreamGeo<FMT, MT, RT>::WAVE + (FMT == XQ_FMT_NF4 ? 64 : 0);
+    constexpr int lds = kStreamWaves * StreamGeo<FMT, MT, RT>::WAVE + stream_levels(FMT);
     static_assert(lds <= 160 * 1024, "LDS of a block");
     static std::atomic<bool> attr_set{false};
     if (!attr_set) {
@@ -840,15 +849,13 @@ static int launch_stream_one(const StreamBatch& b, const int* first, const bf16_
 }
 template <int FMT, int SC, int MT>
 static int launch_stream_mt(const StreamBatch& b, const int* first, const bf16_t* x, int64_t ldx, int64_t M, int64_t K, int rt, hipStream_t s) {
-    constexpr int most = row_tiles_max(FMT, SC);
-    if constexpr (most > 4)
-        if (rt == 6) return launch_stream_one<FMT, SC, MT, 6>(b, first, x, ldx, M, K, s);
-    if constexpr (most > 2) {
-        if (rt == 4) return launch_stream_one<FMT, SC, MT, 4>(b, first, x, ldx, M, K, s);
-        if (rt == 3) return launch_stream_one<FMT, SC, MT, 3>(b, first, x, ldx, M, K, s);
-    }
-    if (rt == 2) return launch_stream_one<FMT, SC, MT, 2>(b, first, x, ldx, M, K, s);
-    return launch_stream_one<FMT, SC, MT, 1>(b, first, x, ldx, M, K, s);
+#define XQ_STREAM_TILES(RT)                                                            \
+    if constexpr (RT <= row_tiles_max(SC) && stream_fits(stream_levels(FMT), MT, RT)) \
+        if (rt == RT) return launch_stream_one<FMT, SC, MT, RT>(b, first, x, ldx, M, K, s)
+    XQ_STREAM_TILES(1); XQ_STREAM_TILES(2); XQ_STREAM_TILES(3); XQ_STREAM_TILES(4);
+    XQ_STREAM_TILES(5); XQ_STREAM_TILES(6); XQ_STREAM_TILES(7); XQ_STREAM_TILES(8);
+#undef XQ_STREAM_TILES
+    return XQ_ERR_UNSUPPORTED;
 }
 template <int FMT, int SC>
 static int launch_stream_sc(const StreamBatch& b, const int* first, const bf16_t* x, int64_t ldx, int64_t M, int64_t K, int rt, hipStream_t s) {
@@ -904,7 +911,7 @@ int launch_skinny_stream(const SkinnyRowsJob* jobs, int n_jobs, bool swiglu, con
     }
     int tiles[kStreamJobs], splits[kStreamJobs];
     for (int i = 0; i < n_jobs; ++i) { tiles[i] = b.job[i].N / 16; splits[i] = b.job[i].splits; }
-    const int rt = stream_row_tiles(tiles, splits, n_jobs, steps, mt, kPlanLimits[cls], nullptr);
+    const int rt = stream_row_tiles(tiles, splits, n_jobs, steps, mt, kPlans[cls], nullptr);
     int first[5] = {0, 0, 0, 0, 0}, efirst[5] = {0, 0, 0, 0, 0};
     for (int i = 0; i < kStreamJobs; ++i) {
         first[i + 1] = first[i];

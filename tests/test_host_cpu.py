@@ -221,7 +221,7 @@ def test_streaming_plans_know_the_storage():
     from xorl_amd import _C
 
     assert skinny_route("int4", 4096, 12288, 64, 12288, _C.XQ_SCALE_F32)[1:] == (2, 2) != skinny_route("int4", 4096, 12288, 64, 12288)[1:]
-    assert skinny_route("nf4", 8192, 5120, 64, 5120)[1:] != skinny_route("int4", 8192, 5120, 64, 5120)[1:]
+    assert skinny_route("nf4", 12288, 8192, 64, 8192)[1:] != skinny_route("int4", 12288, 8192, 64, 8192)[1:]
     for N, K in ((1024, 1024), (4096, 4096), (4096, 12288), (13056, 4992), (16384, 2048)):
         for M in (1, 17, 33, 64):
             for fmt, sdt, most in (("int4", None, 8), ("int4", _C.XQ_SCALE_F32, 2), ("nvfp4", _C.XQ_SCALE_F32, 2), ("nf4", None, 8), ("block_fp8", None, 8)):

@@ -382,6 +382,24 @@ stream_split_kernel(const bf16_t* x, int64_t ldx, int32_t M, int32_t K, int32_t 
                     }
                 }
             };
+            // nf4: the levels of a product's codes, looked up while the product before is converted (two waves a SIMD do not hide the way
+            // through LDS).  MLP forwards, us, each product's own lookups first and this: 4096/12288 24 rows 57.3 -> 53.6, 48 rows 63.4 -> 59.3,
+            // 64 rows 70.8 -> 68.3, 4992/13056 3 rows r 64 72.1 -> 66.9.  Levels in a lane's register, by ds_bpermute (no LDS, four row tiles
+            // of 16 rows pair): 64.9 at 24 rows, 76.4 at 64.  Those of the next half step's first product too: level.
+            float level[2][8];
+            const auto look_up = [&](int at) {
+                if constexpr (FMT == XQ_FMT_NF4) {
+                    uint32_t even = (w[at >> 1][0][2 * hh + (at & 1)] << 2) & 0x3c3c3c3cu, odd4 = (w[at >> 1][0][2 * hh + (at & 1)] >> 2) & 0x3c3c3c3cu;
+                    asm volatile("" : "+v"(even), "+v"(odd4));      // (byte offsets of levels, a byte each: one instruction takes one out)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        level[at & 1][2 * i] = *(const float*)((const unsigned char*)nf4_lds + ((even >> (8 * i)) & 0xffu));
+                        level[at & 1][2 * i + 1] = *(const float*)((const unsigned char*)nf4_lds + ((odd4 >> (8 * i)) & 0xffu));
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            };
+            look_up(0);
 #pragma unroll
             for (int rt = 0; rt < RT; ++rt) {
                 if constexpr (LATE) {
@@ -391,18 +409,24 @@ stream_split_kernel(const bf16_t* x, int64_t ldx, int32_t M, int32_t K, int32_t 
 #pragma unroll
                         for (int t = G::EARLY; t < RT; ++t) read_w(t);
                         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                        look_up(2 * G::EARLY);
                     }
                 }
 #pragma unroll
                 for (int jj = 0; jj < 2; ++jj) {
                     bf16x8 wf;
-                    if constexpr (FMT == XQ_FMT_FP8) {
+                    if (2 * rt + jj + 1 < 2 * RT && !(LATE && 2 * rt + jj + 1 == 2 * G::EARLY)) look_up(2 * rt + jj + 1);
+                    if constexpr (FMT == XQ_FMT_NF4) {
+                        const float* lv = level[jj];
+                        wf = __builtin_bit_cast(bf16x8, u32x4{pack_bf16x2(lv[0] * s0[rt], lv[1] * s0[rt]), pack_bf16x2(lv[2] * s0[rt], lv[3] * s0[rt]),
+                                                              pack_bf16x2(lv[4] * s0[rt], lv[5] * s0[rt]), pack_bf16x2(lv[6] * s0[rt], lv[7] * s0[rt])});
+                    } else if constexpr (FMT == XQ_FMT_FP8) {
                         wf = decode8<FMT>(w[rt][hh][2 * jj], w[rt][hh][2 * jj + 1], s0[rt], 0.0f);
                     } else if constexpr (SC == kScUse) {
                         const float sv = __uint_as_float(sw[rt][jj]);
                         wf = decode8<FMT>(w[rt][0][2 * hh + jj], 0u, sv, -8.0f * sv);
                     } else {
-                        wf = decode8<FMT>(w[rt][0][2 * hh + jj], 0u, s0[rt], s1[rt], nf4_lds);
+                        wf = decode8<FMT>(w[rt][0][2 * hh + jj], 0u, s0[rt], s1[rt]);
                     }
 #pragma unroll
                     for (int mt = 0; mt < MT; ++mt) acc[rt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf, xf[jj][mt], acc[rt][mt], 0, 0, 0);
@@ -729,7 +753,7 @@ struct PlanClass {
     double row_us;
 };
 static const PlanClass kPlans[kPlanClasses] = {
-    {row_tiles_max(kScInt4Window), 0, 0.335}, {row_tiles_max(kScFp8), 0, 0.23}, {row_tiles_max(kScDealt), stream_levels(XQ_FMT_NF4), 0.54}, {row_tiles_max(kScHalf), 0, 0.335}};
+    {row_tiles_max(kScInt4Window), 0, 0.335}, {row_tiles_max(kScFp8), 0, 0.23}, {row_tiles_max(kScDealt), stream_levels(XQ_FMT_NF4), 0.44}, {row_tiles_max(kScHalf), 0, 0.335}};
 
 // The row tiles of a block that make a launch shortest by an estimate of what it takes beyond a constant, in us (they change nothing in
 // the results); `tiles`, `splits` of each forward of the launch, `steps` of the longest split.  Rounds of the chip, and in a block the half
@@ -737,7 +761,8 @@ static const PlanClass kPlans[kPlanClasses] = {
 // The constants, and those of make_stream_splits, come from a sweep of every (splits, row tiles) at 1 to 64 rows in all formats on 28
 // single weights and seven pairs: where a tile of five or seven rows spares a round of the chip the whole forward is up to 11 per cent
 // shorter (us, MLP 3712/9344 of 24 rows int4 46.3 -> 42.6, 4096/12416 of 24 rows int4 52.2 with four tiles, 48.6 with seven, nf4 66.0 -> 61.2).
-// The plans they choose are 2 per cent behind the best of the sweep on average.
+// The plans they choose are 2 per cent behind the best of the sweep on average.  (nf4: a row tile's 0.44 us, in steps of 0.04 over 70 MLPs and
+// single weights; 0.54, from before its lookups ran ahead, is 0.5 per cent longer, 3328/8448 of 37 rows 54.0 against 48.1 us.)
 static int stream_row_tiles(const int* tiles, const int* splits, int n, int steps, int mt, const PlanClass& c, double* us) {
     const int cus = num_cus(), halves = 2 * ((steps + kStreamWaves - 1) / kStreamWaves);
     int best = 1;

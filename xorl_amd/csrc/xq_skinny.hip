@@ -531,10 +531,11 @@ struct EpiBatch {
 // NB: B's chunks were once fetched one behind the other, a trip to memory each: whole forwards at r 64, us, of 24 / 64 rows: int4
 // [4096, 4096] 14.2 -> 13.6 / 17.0 -> 16.5, [7808, 2944] 15.6 -> 14.9 / 20.8 -> 20.0, fp8 [1024, 4096] 12.4 -> 11.8 / 14.6 -> 14.0; level at
 // [12288, 4096] and r 16.
-// RW: 1 up to 16 rows; 2 with eight splits requested at a time above, against 4 rows and four splits, which took fewer blocks and
-// twice the trips.  Whole forwards at r 16 / 64, us, of 24 rows: int4 [1024, 4096] 14.4 -> 12.4 / 18.8 -> 14.7, [4096, 4096] 15.1 -> 14.0 /
-// 19.4 -> 16.3, [4096, 12288] 19.0 -> 17.5 / 26.9 -> 21.7; of 64 rows: 13.5 -> 12.5 / 18.1 -> 15.1, 15.9 -> 15.7 / 20.2 -> 18.2, 24.4 -> 23.4 /
-// 32.1 -> 27.6.  [12288, 4096], where the epilogue is the smaller part, is level at r 16.
+// RW: 1 up to 16 rows; above, 2 with eight splits requested at a time or 4 with four, by the rule in launch_skinny_stream.
+// A block has four waves also where it has fewer than four rows: with a wave a row the pieces of B that so few threads would have
+// taken were registers of every block, 368 for gate and up at r 64, one block a compute unit.  Whole forwards, us, before and now:
+// MLP 4736/14208 1 row nf4 r 64 77.7 -> 66.1, 4608/12288 9 rows fp8 r 64 66.2 -> 57.9, 4992/14848 16 rows int4 r 64 72.8 -> 65.7, 4224/14208 2
+// rows nvfp4 r 32 53.2 -> 50.8; one weight [2048, 4736] 1 row nf4 r 64 13.5 -> 10.8.
 // VEC: B is fp32 with r % 4 == 0 (16-byte pieces).  GU: jobs 0 and 1 are gate and up, h is written.
 template <int RW, int NB, bool VEC, bool GU>
 __global__ void __launch_bounds__(256)
@@ -549,7 +550,7 @@ stream_epilogue_kernel(int32_t M, int32_t first1, int32_t first2, int32_t first3
     const int ji = GU ? 0 : (bx >= first1 ? 1 : 0) + (bx >= first2 ? 1 : 0) + (bx >= first3 ? 1 : 0);
     const int at = bx - (ji == 0 ? 0 : ji == 1 ? first1 : ji == 2 ? first2 : first3);
     const int m0 = blockIdx.y * (4 * RW);
-    const int nthreads = blockDim.x;
+    constexpr int nthreads = 256;
     const EpiJob& g0 = b.job[ji];
     const int n = at * 128 + lane * 2;
     const int nn = n < g0.N ? n : 0;                               // N % 2 == 0
@@ -558,34 +559,31 @@ stream_epilogue_kernel(int32_t M, int32_t first1, int32_t first2, int32_t first3
     // B values of 16 ranks of the block's columns: fetched in 16-byte pieces of 4 ranks, neighbouring threads on neighbouring
     // pieces, and shared through LDS; piece P = column * 4 + ranks / 4 lies at P ^ (column / 4 & 7), which lets the 16 lanes of a
     // read pass (two columns a lane) fall on 16 different pieces
-    constexpr int kPieces = RW == 1 ? 8 : 2;                       // of a thread (RW > 1: always four waves)
+    constexpr int kPieces = 512 / nthreads;                        // of a thread
     f32x4 bq[NP][NB][kPieces];
     const auto load_b = [&](int p, int rc) {
         const EpiJob& g = b.job[ji + p];
 #pragma unroll
         for (int i = 0; i < kPieces; ++i) {
-            if (i * nthreads < 512) {
-                const int P = (tid + i * nthreads) & 511, col = at * 128 + (P >> 2), j = 16 * rc + 4 * (P & 3);
-                const int64_t row = (int64_t)(col < g.N ? col : 0) * g.r;
-                if constexpr (VEC) {
-                    bq[p][rc][i] = *(const f32x4*)((const float*)g.lora_B + row + (j < g.r ? j : 0));
-                } else {
+            const int P = tid + i * nthreads, col = at * 128 + (P >> 2), j = 16 * rc + 4 * (P & 3);
+            const int64_t row = (int64_t)(col < g.N ? col : 0) * g.r;
+            if constexpr (VEC) {
+                bq[p][rc][i] = *(const f32x4*)((const float*)g.lora_B + row + (j < g.r ? j : 0));
+            } else {
 #pragma unroll
-                    for (int f = 0; f < 4; ++f) {
-                        const int64_t bi = row + (j + f < g.r ? j + f : 0);
-                        bq[p][rc][i][f] = g.lora_f32 ? ((const float*)g.lora_B)[bi] : bf16_to_f32(((const bf16_t*)g.lora_B)[bi]);
-                    }
+                for (int f = 0; f < 4; ++f) {
+                    const int64_t bi = row + (j + f < g.r ? j + f : 0);
+                    bq[p][rc][i][f] = g.lora_f32 ? ((const float*)g.lora_B)[bi] : bf16_to_f32(((const bf16_t*)g.lora_B)[bi]);
                 }
             }
         }
     };
     const auto store_b = [&](int p, int rc) {
 #pragma unroll
-        for (int i = 0; i < kPieces; ++i)
-            if (i * nthreads < 512) {
-                const int P = (tid + i * nthreads) & 511;
-                bt[p][rc][P ^ ((P >> 4) & 7)] = bq[p][rc][i];
-            }
+        for (int i = 0; i < kPieces; ++i) {
+            const int P = tid + i * nthreads;
+            bt[p][rc][P ^ ((P >> 4) & 7)] = bq[p][rc][i];
+        }
     };
     constexpr int SB = RW == 2 ? 8 : 4;                            // splits requested at a time
     f32x2 t[NP][SB][RW];
@@ -983,16 +981,15 @@ int launch_skinny_stream(const SkinnyRowsJob* jobs, int n_jobs, bool swiglu, con
     const int64_t by2 = xq_cdiv((int64_t)cols * xq_cdiv(M, 8), num_cus()), by4 = xq_cdiv((int64_t)cols * xq_cdiv(M, 16), num_cus());
     const bool four = by2 > 3 || (most <= 4 && ranks <= (2 * (int64_t)cols >= num_cus() ? 32 : 16)) || (ranks <= 16 && 17 * by4 < 10 * by2);
     const int rw = M <= 16 ? 1 : four ? 4 : 2;
-    const unsigned threads = M < 4 && rw == 1 ? (unsigned)M * 64 : 256;
     const dim3 grid(cols, (unsigned)xq_cdiv(M, 4 * rw));
 #define XQ_EPI_NB(RW, NB)                                                                                                                      \
     do {                                                                                                                                       \
         if (swiglu) {                                                                                                                          \
-            if (vec) stream_epilogue_kernel<RW, NB, true, true><<<grid, threads, 0, stream>>>((int)M, efirst[1], efirst[2], efirst[3], e);     \
-            else stream_epilogue_kernel<RW, NB, false, true><<<grid, threads, 0, stream>>>((int)M, efirst[1], efirst[2], efirst[3], e);        \
+            if (vec) stream_epilogue_kernel<RW, NB, true, true><<<grid, 256, 0, stream>>>((int)M, efirst[1], efirst[2], efirst[3], e);     \
+            else stream_epilogue_kernel<RW, NB, false, true><<<grid, 256, 0, stream>>>((int)M, efirst[1], efirst[2], efirst[3], e);        \
         } else {                                                                                                                               \
-            if (vec) stream_epilogue_kernel<RW, NB, true, false><<<grid, threads, 0, stream>>>((int)M, efirst[1], efirst[2], efirst[3], e);    \
-            else stream_epilogue_kernel<RW, NB, false, false><<<grid, threads, 0, stream>>>((int)M, efirst[1], efirst[2], efirst[3], e);       \
+            if (vec) stream_epilogue_kernel<RW, NB, true, false><<<grid, 256, 0, stream>>>((int)M, efirst[1], efirst[2], efirst[3], e);    \
+            else stream_epilogue_kernel<RW, NB, false, false><<<grid, 256, 0, stream>>>((int)M, efirst[1], efirst[2], efirst[3], e);       \
         }                                                                                                                                      \
     } while (0)
 #define XQ_EPI(RW)                       \

@@ -228,3 +228,4 @@ def test_streaming_plans_know_the_storage():
                 where, splits, tiles = skinny_route(fmt, N, K, M, K, sdt)
                 assert 1 <= tiles <= most if where == 2 else where == 1, (fmt, sdt, N, K, M)
                 assert _C.lib().xq_linear_workspace_bytes_fmt(_C.FORMATS[fmt], M, N, K, 16) >= splits * M * N * 4 + (K // 128) * M * 16 * 4
+    assert [_C.lib().xq_linear_workspace_bytes(0, 1024, K, 16) > 0 for K in (64, 128, 4096)] == [True] * 3      # (no rows, no plan)

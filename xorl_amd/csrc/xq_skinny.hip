@@ -779,20 +779,25 @@ static int stream_row_tiles(const int* tiles, const int* splits, int n, int step
 }
 // steps of a split at most (a lane holds one block-fp8 scale of a wave's steps)
 constexpr int kStreamSteps = 64 * kStreamWaves;
+static int least_stream_splits(int64_t K) { return (int)xq_cdiv(K >> 7, kStreamSteps); }
+// splits that a plan may have: 64, sums of 16 MB, four steps in the longest.  Workspaces are sized for as many, whatever the storage: its plan
+// would be two to five microseconds of a first call (all four classes at [1024, 4096] and [4096, 12288]), its memory a few MB less.
+static int most_stream_splits(int64_t M, int64_t N, int64_t K) {
+    return (int)std::max<int64_t>(least_stream_splits(K), std::min(std::min<int64_t>(64, (16ll << 20) / (M * N * 4)), ((K >> 7) - 1) / (kStreamWaves / 2 - 1)));
+}
 // K splits of a forward, by its own shape and storage: the cheapest sum of that and of the epilogue's share, 0.44 us a split and the partial
 // sums' trip.  Weights twice as wide as deep are mostly gate and up of an MLP, whose one launch has other rounds than a weight alone: half
 // of what a pair takes counts too (nvfp4 4096 -> 2 x 12288 of 19 rows, the whole MLP: 49.4 us with two splits, 44.1 with one; alone they
 // are level).
 static int make_stream_splits(int cls, int64_t M, int64_t N, int64_t K) {
-    const int ct = (int)(K >> 7), mt = (int)xq_cdiv(M, 16), least = (int)xq_cdiv(ct, kStreamSteps);
+    const int ct = (int)(K >> 7), mt = (int)xq_cdiv(M, 16), most = most_stream_splits(M, N, K);
     const int tiles[2] = {(int)(N / 16), (int)(N / 16)};
     int best = 0, last_steps = 0;
     double best_cost = 0;
-    for (int s = least; s <= ct && (s <= 64 || best == 0); ++s) {
+    for (int s = least_stream_splits(K); s <= most; ++s) {
         const int steps = (int)xq_cdiv(ct, s), splits[2] = {s, s};
         if (steps == last_steps) continue;                         // more splits, none of them shorter
         last_steps = steps;
-        if (best && (s * M * N * 4 > (16ll << 20) || steps < kStreamWaves / 2)) break;
         const double sums = s * (0.44 + M * N * 8 * 0.14e-6);
         double c, two = 0;
         stream_row_tiles(tiles, splits, 1, steps, mt, kPlans[cls], &c);
@@ -813,19 +818,6 @@ static int stream_splits(int cls, int64_t M, int64_t N, int64_t K) {
     if (!(e.key == key)) e = PlanSlot<int>{key, make_stream_splits(cls, M, N, K)};
     return e.value;
 }
-// the most that any storage takes
-static int most_stream_splits(int64_t M, int64_t N, int64_t K) {
-    static thread_local PlanSlot<int> kept[64];
-    const PlanKey key{M, N, K, num_cus(), 0};
-    PlanSlot<int>& e = kept[key.slot()];
-    if (!(e.key == key)) {
-        int most = 0;
-        for (int cls = 0; cls < kPlanClasses; ++cls) most = std::max(most, make_stream_splits(cls, M, N, K));
-        e = PlanSlot<int>{key, most};
-    }
-    return e.value;
-}
-
 // whether a forward of this shape runs on the two launches of this file (and not in one, xq_skinny_rows.hip)
 bool skinny_takes_stream(const xq_weight* w, int64_t M, int64_t ldx, const void* lora_A, const void* lora_B, int lora_dtype, int r) {
     return skinny_supported(w, M) && stream_takes_pitch(M, ldx) && !(skinny_rows_enabled() && skinny_rows_supported(w, M, lora_A, lora_B, lora_dtype, r));
@@ -838,7 +830,7 @@ void skinny_stream_plan(const xq_weight* w, int64_t M, int32_t* plan) {
 }
 
 int64_t skinny_workspace_bytes(int64_t M, int64_t N, int64_t K, int r_pad) {
-    if (K < 128 || N < 16) return 256;
+    if (M < 1 || K < 128 || N < 16) return 256;
     const int rp = r_pad ? r_pad : 16;
     // (never less than a partial sum for every 32, 16 or 8 steps, whatever the plan: what callers have always been asked for)
     const int64_t s = most_stream_splits(M, N, K), held = xq_cdiv(K >> 7, M <= 16 ? 32 : M <= 32 ? 16 : 8);

@@ -8,7 +8,7 @@ import torch
 from oracle import cdecode as C
 from oracle import decode_np as NP
 from oracle import recipe as R
-from tests.util_cases import close, bits_to_bf16, gen
+from tests.util_cases import banks_joint, close, bits_to_bf16, gen
 
 pytestmark = pytest.mark.gpu
 TOL = 1e-2
@@ -813,10 +813,10 @@ def test_few_routed_rows_equal_the_same_rows_among_many(hip_device, H, I, r, few
 
 
 @pytest.mark.parametrize("fmt", ["nvfp4", "nf4"])
-@pytest.mark.parametrize("H,I", [(384, 640), (640, 128), (256, 384)])
+@pytest.mark.parametrize("H,I", [(384, 640), (640, 128), (256, 384), (512, 256)])
 def test_two_4bit_banks_in_one_launch_equal_two_launches(hip_device, fmt, H, I):
     """Gate and up side by side (widths in whole tiles of 128) against a launch each (384, 640 and 128 are no whole tiles of 256; of
-    256 and 384 one direction shares a launch either way): the same sums in the same order."""
+    256 and 384 one direction shares a launch either way, of 512 and 256 both): the same sums in the same order."""
     from xorl_amd import _C
 
     E, topk, T = 5, 2, 700
@@ -827,6 +827,7 @@ def test_two_4bit_banks_in_one_launch_equal_two_launches(hip_device, fmt, H, I):
     try:
         for policy in (3, 2):
             _C.check(_C.lib().xq_set_tile_policy(policy))
+            assert [banks_joint(fmt, E, H, I, T * topk, fwd) for fwd in (True, False)] == [policy == 3 or n % 256 == 0 for n in (I, H)]
             xd = x.clone().requires_grad_(True)
             y = m(xd, rw.to(torch.bfloat16).to(hip_device), sel.to(hip_device))
             got.append([y.detach(), *torch.autograd.grad(y, [xd, *m.get_lora_parameters()], dy)])
@@ -834,6 +835,30 @@ def test_two_4bit_banks_in_one_launch_equal_two_launches(hip_device, fmt, H, I):
         _C.check(_C.lib().xq_set_tile_policy(0))
     for a, b in zip(*got):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("T,E,topk", [(1, 4, 1), (37, 5, 2), (700, 8, 3)])
+def test_scalars_to_rows_and_back(hip_device, T, E, topk, dtype):
+    """Routing weights by row and back by copy; copies of ids outside [0, E) have no row and come back as 0."""
+    from xorl_amd import _C
+    from xorl_amd import moe_functional as MF
+
+    rw, sel = _zipf_routing(T, E, topk, seed=6)
+    sel[-1, -1] = E
+    sel[T // 2, 0] = -1
+    src = rw.to(dtype).to(hip_device).reshape(-1).contiguous()
+    _, offsets, sidx, _ = MF.route_build(sel.to(hip_device), E)
+    n, code, stream = T * topk, _C.XQ_DT_F32 if dtype == torch.float32 else _C.XQ_DT_BF16, torch.cuda.current_stream().cuda_stream
+    rows, back = torch.full((n,), -7.0, device=hip_device), torch.full((n,), -7.0, dtype=dtype, device=hip_device)
+    _C.check(_C.lib().xq_moe_scatter_scalar(src.data_ptr(), code, sidx.data_ptr(), n, rows.data_ptr(), stream))
+    _C.check(_C.lib().xq_moe_gather_scalar(rows.data_ptr(), sidx.data_ptr(), n, back.data_ptr(), code, stream))
+    flat = sel.reshape(-1)
+    there = (flat >= 0) & (flat < E)
+    order = torch.argsort(flat[there], stable=True)
+    m = int(there.sum())
+    assert int(offsets[E]) == m and torch.equal(rows[:m].cpu(), src.cpu().float()[there][order]) and bool((rows[m:] == -7).all())
+    assert torch.equal(back.cpu(), torch.where(there, src.cpu(), torch.zeros((), dtype=dtype)))
 
 
 @pytest.mark.parametrize("r", [8, 16, 20, 64])

@@ -96,6 +96,20 @@ def skinny_route(fmt, N, K, M, ldx, scale_dtype=None, r=0):
     return (_C.lib().xq_skinny_route(ctypes.byref(w), M, ldx, 4096 if r else None, 4096 if r else None, _C.XQ_DT_F32, r, plan), *plan)
 
 
+def banks_joint(fmt, E, H, I, n_rows, forward) -> bool:
+    """xq_grouped_joint (include/xq.h) of gate and up banks [E, H, I] in a format's usual storage"""
+    import ctypes
+
+    from xorl_amd import _C
+
+    w = _C.XqWeight()
+    w.format, w.layout, w.rows, w.cols, w.num_experts = _C.FORMATS[fmt], _C.XQ_LAYOUT_GKN, H, I, E
+    w.group = {"nvfp4": 16, "block_fp8": 128, "nf4": 64}[fmt]
+    w.scale_dtype = _C.XQ_SCALE_E4M3 if fmt == "nvfp4" else _C.XQ_SCALE_F32
+    w.packed = w.scales = w.global_scale = 4096              # (addresses: nothing is read)
+    return bool(_C.lib().xq_grouped_joint(ctypes.byref(w), ctypes.byref(w), n_rows, int(forward)))
+
+
 def oracle_decode_dense(m) -> torch.Tensor:
     """Decode a (CPU) module's packed state with the numpy oracle -> bf16 [N, K]."""
     N, K = m.out_features, m.in_features

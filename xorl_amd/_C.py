@@ -166,6 +166,7 @@ _SIGNATURES = {
     "xq_grouped_lora_wgrad": (_INT, [_P, _I64, _I64, _P, _INT, _INT, _I64, _P, _I32, _INT, _P, _P, _P, _P]),
     "xq_grouped_workspace_bytes": (_I64, [_I64, _I32, _I32, _I64, _I64, _INT, _INT]),
     "xq_grouped_in_place": (_INT, [_W, _W, _W]),
+    "xq_grouped_joint": (_INT, [_W, _W, _I64, _INT]),
     # gate, up, down, lora, hidden, ld_hidden, n_tokens, routing_w, rw_dtype, selected, topk, out, ld_out, saved, ws, ws_bytes, stream
     "xq_grouped_fwd": (_INT, [_W, _W, _W, ctypes.POINTER(XqGroupedLora), _P, _I64, _I64, _P, _INT, _P, _I32, _P, _I64,
                               ctypes.POINTER(XqGroupedSaved), _P, _I64, _P]),

@@ -88,11 +88,18 @@ int64_t bwd_workspace(const Dims& d) {
 // one sum for the two dgrads of gate and up: block-fp8 banks on the pipelined kernel.  (Their forwards as one launch: these banks,
 // and 4-bit banks where banks_side_by_side() says so, whose dgrads then share a launch too but stay two products.)
 bool fuse_gate_up(const xq_weight* gate, const xq_weight* up) { return two_banks_supported(gate) && two_banks_supported(up); }
+bool joint_forward(const xq_weight* gate, const xq_weight* up, int64_t R) { return fuse_gate_up(gate, up) || banks_side_by_side(gate, up, gate->cols, R); }
+bool joint_dgrads(const xq_weight* gate, const xq_weight* up, int64_t R) { return banks_side_by_side(gate, up, gate->rows, R); }
 
 }  // namespace
 }  // namespace xq
 
 using namespace xq;
+
+extern "C" int xq_grouped_joint(const xq_weight* gate, const xq_weight* up, int64_t n_rows, int forward) {
+    if (!gate || !up || xq_validate_weight(gate, "xq_grouped_joint") || xq_validate_weight(up, "xq_grouped_joint")) return 0;
+    return forward ? joint_forward(gate, up, n_rows) : joint_dgrads(gate, up, n_rows);
+}
 
 extern "C" int xq_grouped_in_place(const xq_weight* gate, const xq_weight* up, const xq_weight* down) {
     (void)down;
@@ -191,7 +198,7 @@ extern "C" int xq_grouped_fwd_ids(const xq_weight* gate, const xq_weight* up, co
             return rc;
         if ((rc = launch_small_nt(xr, ld_xr, R, H, F_uA, rp, s, su_u, off, toff, E, uAe == 1, stream, 0, nullptr, 0, xr_rows, nullptr, 0))) return rc;
     }
-    if (fuse_gate_up(gate, up) || banks_side_by_side(gate, up, I, R)) {       // both projections in one launch: column tiles past I take the up bank
+    if (joint_forward(gate, up, R)) {       // both projections in one launch: column tiles past I take the up bank
         const TwoBanks two{up, su_u, Lr_uB, 0};
         if ((rc = launch_tile_gemm(gate, false, xr, ld_xr, R, off, toff, su_g, Lr_gB, rp, nullptr, gu, 2 * I, stream, who, nullptr, 0, &two, nullptr, xr_rows, d.T))) return rc;
     } else {
@@ -261,7 +268,7 @@ extern "C" int xq_grouped_bwd(const xq_weight* gate, const xq_weight* up, const 
     // low-rank terms ride as one side term of width 2 * rp)
     // (the A gradients then come from one pass over the rows too, which wants both A factors held the same way)
     const bool fused = fuse_gate_up(gate, up) && 2 * rp <= 64 && gAe == uAe;
-    const bool side = banks_side_by_side(gate, up, H, R);
+    const bool side = joint_dgrads(gate, up, R);
     const int rp2 = 2 * rp;
 
     // every panel of the call in one launch: B factors [E|1, r, out] as the "down" panels [E|1, rp, out] of g . B^T,

@@ -19,15 +19,13 @@
 //
 // What bounds it: at 64 rows and RT 6 about 5 us until the first weights are there (half of a wave's rows at once in the order in which
 // they are multiplied), 14 for products that the vector units' decode bounds (19 instructions and four MFMAs per 8 weights a lane,
-// two waves a SIMD), 4 until the slowest wave is done and the sums have met: gate | up of 4096 -> 2 x 12288 takes 26 us in int4
-// (50 MB), 31 in block-fp8 (100 MB), and the epilogue 10; at few rows the fixed costs of two dependent launches.  Before, waves owned
-// rows, K was split between five to sixteen blocks, and fragments were loaded straight to registers: 32 + 13 and 36 + 13 us.  Forward
-// of one projection at r 16, weights from memory, us, against that (24 / 40 or 48 / 64 rows):
-//     int4 [12288, 4096] 19.6 23.4 25.8 -> 18.8 20.3 23.2    [4096, 4096] 14.8 15.4 16.6 -> 11.8 13.2 14.4    [2944, 7808] 18.2 -> 17.6 at 64
-//     fp8  [12288, 4096] 22.8 23.6 26.2 -> 22.4 24.3 27.3    [4096, 4096] 15.8 16.1 17.3 -> 13.6 15.6 15.5    [1024, 4096] 13.8 -> 12.3 at 64
-//     nvfp4 [12288, 4096], 64 rows 27.4 -> 25.1, nf4 29.9 -> 26.2; of the MLP 4096 / 12288 of 64 rows: int4 64.1 -> 54.8, fp8 75 -> 67
-// (Block-fp8 of more than 32 rows and 8000 to 12000 rows of weights is 3 to 4 % behind there: a wave's LDS holds one half step of x then,
-// and x waits for the weights requested before it.  Gate and up of an MLP, which are those very products, are 8 % ahead as one launch.)
+// two waves a SIMD), 4 until the slowest wave is done and the sums have met: gate | up of 4096 -> 2 x 12288 takes 27 us in int4
+// (50 MB), 31 in block-fp8 (100 MB), 35 in nf4 (two rounds of three row tiles), and the epilogue 9.5; at few rows the fixed costs of two
+// dependent launches.  Before, waves owned rows, K was split between five to sixteen blocks, and fragments were loaded straight to
+// registers: 32 + 13 and 36 + 13 us.  Forward of one projection at r 16, weights from memory, us, against that (24 / 48 / 64 rows):
+//     int4 [12288, 4096] 17.1 22.2 23.3 -> 16.5 17.8 20.6    [4096, 4096] 14.1 14.6 15.9 -> 11.0 12.4 13.5    [2944, 7808] 17.4 -> 16.6 at 64
+//     fp8  [12288, 4096] 18.6 21.1 21.9 -> 17.6 19.2 22.2    [4096, 4096] 15.0 15.2 16.4 -> 12.6 15.1 14.8    [1024, 4096] 12.7 -> 11.2 at 64
+//     nvfp4 [12288, 4096], 64 rows 24.0 -> 21.8, nf4 27.3 -> 22.3; of the MLP 4096 / 12288 of 64 rows: int4 64.9 -> 57.2, fp8 69.0 -> 64.4
 #include <stdlib.h>
 
 #include <algorithm>

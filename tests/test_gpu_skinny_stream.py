@@ -138,11 +138,14 @@ def test_rows_of_x_a_gigabyte_apart(hip_device, K):
 
 
 @pytest.mark.parametrize("fmt,N,K,tiles", [                       # rows of x: the plan's row tiles
-    ("int4", 4480, 4096, {17: 5, 33: 5, 49: 5}),
-    ("int4", 27648, 2048, {33: 7}),
-    ("nf4", 16512, 1152, {3: 5}),                                 # the nf4 levels beside odd numbers of tiles
-    ("nf4", 5504, 2944, {17: 5, 33: 5, 49: 5}),
-    ("nf4", 6400, 5120, {8: 8}),
+    ("int4", 6272, 5120, {33: 5, 49: 5}),
+    ("int4", 8320, 5120, {17: 7, 33: 7}),
+    ("int4", 28800, 1024, {17: 8}),
+    ("nf4", 16512, 2944, {3: 5}),                                 # the nf4 levels beside odd numbers of tiles
+    ("nf4", 16512, 1024, {17: 5}),
+    ("nf4", 6272, 5120, {33: 5, 49: 5}),
+    ("nf4", 8320, 5120, {17: 7}),
+    ("nf4", 28800, 1024, {3: 8}),
     ("block_fp8", 27648, 2944, {17: 7}),                          # an odd number of steps
 ])
 def test_five_seven_and_eight_row_tiles(hip_device, fmt, N, K, tiles):

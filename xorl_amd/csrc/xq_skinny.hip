@@ -738,29 +738,31 @@ static int scale_mode(const xq_weight* w) {
 
 // ---- plans
 // What the plans have to know of a storage: the row tiles of a block at most (the uncommon scale storages keep more registers per tile),
-// the LDS it takes beside the waves' parts, and what a half step costs for each row tile, in us.
+// the LDS it takes beside the waves' parts, the steps of a unit of its weights, and what a half step costs for each row tile, in us.
 constexpr int row_tiles_max(int sc) { return sc >= kScHalf ? 2 : 8; }
 enum { kPlan4Bit = 0, kPlanFp8 = 1, kPlanNf4 = 2, kPlanUncommon = 3, kPlanClasses = 4 };
 static int plan_class(const xq_weight* w) {
     return scale_mode(w) >= kScHalf ? kPlanUncommon : w->format == XQ_FMT_FP8 ? kPlanFp8 : w->format == XQ_FMT_NF4 ? kPlanNf4 : kPlan4Bit;
 }
 struct PlanClass {
-    int row_tiles, levels;
+    int row_tiles, levels, unit;
     double row_us;
 };
 static const PlanClass kPlans[kPlanClasses] = {
-    {row_tiles_max(kScInt4Window), 0, 0.335}, {row_tiles_max(kScFp8), 0, 0.23}, {row_tiles_max(kScDealt), stream_levels(XQ_FMT_NF4), 0.44}, {row_tiles_max(kScHalf), 0, 0.335}};
+    {row_tiles_max(kScInt4Window), 0, 2, 0.30}, {row_tiles_max(kScFp8), 0, 1, 0.20}, {row_tiles_max(kScDealt), stream_levels(XQ_FMT_NF4), 2, 0.36}, {row_tiles_max(kScHalf), 0, 2, 0.30}};
 
 // The row tiles of a block that make a launch shortest by an estimate of what it takes beyond a constant, in us (they change nothing in
 // the results); `tiles`, `splits` of each forward of the launch, `steps` of the longest split.  Rounds of the chip, and in a block the half
 // steps of a wave, each for its weights, its x and their products; a second block on the compute unit nearly doubles them.
-// The constants, and those of make_stream_splits, come from a sweep of every (splits, row tiles) at 1 to 64 rows in all formats on 28
-// single weights and seven pairs: where a tile of five or seven rows spares a round of the chip the whole forward is up to 11 per cent
-// shorter (us, MLP 3712/9344 of 24 rows int4 46.3 -> 42.6, 4096/12416 of 24 rows int4 52.2 with four tiles, 48.6 with seven, nf4 66.0 -> 61.2).
-// The plans they choose are 2 per cent behind the best of the sweep on average.  (nf4: a row tile's 0.44 us, in steps of 0.04 over 70 MLPs and
-// single weights; 0.54, from before its lookups ran ahead, is 0.5 per cent longer, 3328/8448 of 37 rows 54.0 against 48.1 us.)
+// Steps that leave a wave's last weight unit half empty cost more than they multiply.  The constants, and those of make_stream_splits,
+// are the ones whose plans were shortest in a sweep of every (splits, row tiles) on 808 single forwards and 218 MLPs of 2 to 64 rows in all
+// formats: 1.7 per cent behind the best of the sweep on average, singles 2.0, MLPs 0.3; constants that were fitted to the times themselves 2.3, 2.8
+// and 0.7 (int4 [4352, 4352] of 64 rows 18.7 us with five splits of six row tiles where three of four take 15.7).  Where a tile of five or seven
+// rows spares a round of the chip the whole forward is up to 11 per cent shorter (MLP 3712/9344 of 24 rows int4 46.3 -> 42.6, 4096/12416 of
+// 24 rows int4 52.2 with four tiles, 48.6 with seven, nf4 66.0 -> 61.2).
 static int stream_row_tiles(const int* tiles, const int* splits, int n, int steps, int mt, const PlanClass& c, double* us) {
-    const int cus = num_cus(), halves = 2 * ((steps + kStreamWaves - 1) / kStreamWaves);
+    const int cus = num_cus(), wave_steps = (steps + kStreamWaves - 1) / kStreamWaves;
+    const double halves = 2 * wave_steps + (wave_steps % c.unit ? 0.4 : 0);
     int best = 1;
     double least = 0;
     for (int rt = 1; rt <= c.row_tiles && stream_fits(c.levels, mt, rt); ++rt) {
@@ -768,8 +770,8 @@ static int stream_row_tiles(const int* tiles, const int* splits, int n, int step
         for (int i = 0; i < n; ++i) blocks += (tiles[i] + rt - 1) / rt * splits[i];
         const bool pair = stream_pairs(c.levels, mt, rt);
         const int per_cu = pair ? 2 : 1, rounds = (blocks + cus * per_cu - 1) / (cus * per_cu), on_cu = std::min((blocks + cus - 1) / cus, rounds * per_cu);
-        const double half = c.row_us * rt + 0.25 * mt + 0.009 * rt * mt;
-        const double t = rounds * ((pair ? 2.75 : 3.7) + 0.13 * rt * mt + halves * half * (1.0 + 0.92 * ((double)on_cu / rounds - 1.0)));
+        const double half = c.row_us * rt + 0.25 * mt + 0.003 * rt * mt;
+        const double t = rounds * ((pair ? 2.25 : 3.75) + 0.2 * rt + 0.16 * rt * mt + halves * half * (1.0 + 0.9 * ((double)on_cu / rounds - 1.0)));
         if (least == 0 || t < least) { least = t; best = rt; }
     }
     if (us) *us = least;
@@ -783,8 +785,8 @@ static int least_stream_splits(int64_t K) { return (int)xq_cdiv(K >> 7, kStreamS
 static int most_stream_splits(int64_t M, int64_t N, int64_t K) {
     return (int)std::max<int64_t>(least_stream_splits(K), std::min(std::min<int64_t>(64, (16ll << 20) / (M * N * 4)), ((K >> 7) - 1) / (kStreamWaves / 2 - 1)));
 }
-// K splits of a forward, by its own shape and storage: the cheapest sum of that and of the epilogue's share, 0.44 us a split and the partial
-// sums' trip.  Weights twice as wide as deep are mostly gate and up of an MLP, whose one launch has other rounds than a weight alone: half
+// K splits of a forward, by its own shape and storage: the cheapest sum of that and of the epilogue's share, 0.48 us a split and the partial
+// sums' trip.  Weights twice as wide as deep are mostly gate and up of an MLP, whose one launch has other rounds than a weight alone: 0.55
 // of what a pair takes counts too (nvfp4 4096 -> 2 x 12288 of 19 rows, the whole MLP: 49.4 us with two splits, 44.1 with one; alone they
 // are level).
 static int make_stream_splits(int cls, int64_t M, int64_t N, int64_t K) {
@@ -796,35 +798,43 @@ static int make_stream_splits(int cls, int64_t M, int64_t N, int64_t K) {
         const int steps = (int)xq_cdiv(ct, s), splits[2] = {s, s};
         if (steps == last_steps) continue;                         // more splits, none of them shorter
         last_steps = steps;
-        const double sums = s * (0.44 + M * N * 8 * 0.14e-6);
+        const double sums = s * (0.48 + M * N * 8 * 0.145e-6);
         double c, two = 0;
         stream_row_tiles(tiles, splits, 1, steps, mt, kPlans[cls], &c);
         c += sums;
         if (N >= 2 * K) {
             stream_row_tiles(tiles, splits, 2, steps, mt, kPlans[cls], &two);
-            c += 0.5 * (two + 2 * sums);
+            c += 0.55 * (two + 2 * sums);
         }
         if (best == 0 || c < best_cost) { best = s; best_cost = c; }
     }
     return best;
 }
 
-static int stream_splits(int cls, int64_t M, int64_t N, int64_t K) {
-    static thread_local PlanSlot<int> kept[64];
+// splits, and the row tiles of a launch alone
+struct StreamPlan {
+    int splits, row_tiles;
+};
+static StreamPlan stream_plan(int cls, int64_t M, int64_t N, int64_t K) {
+    static thread_local PlanSlot<StreamPlan> kept[64];
     const PlanKey key{M, N, K, num_cus(), cls};
-    PlanSlot<int>& e = kept[key.slot()];
-    if (!(e.key == key)) e = PlanSlot<int>{key, make_stream_splits(cls, M, N, K)};
+    PlanSlot<StreamPlan>& e = kept[key.slot()];
+    if (!(e.key == key)) {
+        const int tiles = (int)(N / 16), splits = make_stream_splits(cls, M, N, K);
+        e = PlanSlot<StreamPlan>{key, {splits, stream_row_tiles(&tiles, &splits, 1, (int)xq_cdiv(K >> 7, splits), (int)xq_cdiv(M, 16), kPlans[cls], nullptr)}};
+    }
     return e.value;
 }
+
 // whether a forward of this shape runs on the two launches of this file (and not in one, xq_skinny_rows.hip)
 bool skinny_takes_stream(const xq_weight* w, int64_t M, int64_t ldx, const void* lora_A, const void* lora_B, int lora_dtype, int r) {
     return skinny_supported(w, M) && stream_takes_pitch(M, ldx) && !(skinny_rows_enabled() && skinny_rows_supported(w, M, lora_A, lora_B, lora_dtype, r));
 }
 
 void skinny_stream_plan(const xq_weight* w, int64_t M, int32_t* plan) {
-    const int cls = plan_class(w), tiles = (int)(w->rows / 16), splits = stream_splits(cls, M, w->rows, w->cols);
-    plan[0] = splits;
-    plan[1] = stream_row_tiles(&tiles, &splits, 1, (int)xq_cdiv(w->cols >> 7, splits), (int)xq_cdiv(M, 16), kPlans[cls], nullptr);
+    const StreamPlan p = stream_plan(plan_class(w), M, w->rows, w->cols);
+    plan[0] = p.splits;
+    plan[1] = p.row_tiles;
 }
 
 int64_t skinny_workspace_bytes(int64_t M, int64_t N, int64_t K, int r_pad) {
@@ -900,13 +910,15 @@ int launch_skinny_stream(const SkinnyRowsJob* jobs, int n_jobs, bool swiglu, con
     EpiBatch e{};
     uint8_t* ws = (uint8_t*)workspace;
     bool vec = true;
-    int steps = 0;
+    int steps = 0, rt = 1;
     for (int i = 0; i < n_jobs; ++i) {
         const SkinnyRowsJob& j = jobs[i];
         const int rp = j.r > 0 ? (j.r + 15) / 16 * 16 : 0;
         const int64_t N = j.w->rows;
         StreamJob& g = b.job[i];
-        g.splits = stream_splits(cls, M, N, K);
+        const StreamPlan plan = stream_plan(cls, M, N, K);
+        g.splits = plan.splits;
+        rt = plan.row_tiles;
         g.packed = (const uint8_t*)j.w->packed; g.scales = (const uint8_t*)j.w->scales; g.global_scale = j.w->global_scale;
         g.N = (int)N; g.group = j.w->group; g.scale_dtype = j.w->scale_dtype;
         g.chunk_q = (int)(K >> 7) / g.splits; g.chunk_rem = (int)(K >> 7) % g.splits;
@@ -924,7 +936,7 @@ int launch_skinny_stream(const SkinnyRowsJob* jobs, int n_jobs, bool swiglu, con
     }
     int tiles[kStreamJobs], splits[kStreamJobs];
     for (int i = 0; i < n_jobs; ++i) { tiles[i] = b.job[i].N / 16; splits[i] = b.job[i].splits; }
-    const int rt = stream_row_tiles(tiles, splits, n_jobs, steps, mt, kPlans[cls], nullptr);
+    if (n_jobs > 1) rt = stream_row_tiles(tiles, splits, n_jobs, steps, mt, kPlans[cls], nullptr);
     int first[5] = {0, 0, 0, 0, 0}, efirst[5] = {0, 0, 0, 0, 0};
     for (int i = 0; i < kStreamJobs; ++i) {
         first[i + 1] = first[i];

@@ -56,7 +56,7 @@ MEASURED_TRAFFIC = {
     # skinny_gemv_kernel (M = 1), skinny_rows_kernel (M <= 16) and stream_split_kernel + stream_epilogue_kernel
     # (M = 32, 64): mean per forward over the 32 cases (includes the fp32 partial tiles of the two-launch cases
     # written and read back: 23.3 MiB of it are algorithmic)
-    4: (27.5 * 2 ** 20, "profiles/skinny_kernels_decode_shapes.txt", 0.01458),
+    4: (27.4 * 2 ** 20, "profiles/skinny_kernels_decode_shapes.txt", 0.01468),
     # merge_fp8_kernel and merge_kernel<fp8>: mean per call (re-quantise 96 MiB, publish 144 MiB algorithmic)
     5: (132.1 * 2 ** 20, "profiles/merge_kernel_fp8_mlp_weights.txt", 0.03898),
     # gemm_256_kernel<nvfp4 GKN, grouped>: mean over the 6 launches of a step

@@ -3,6 +3,7 @@
 #include <algorithm>
 #include <atomic>
 #include "xq_gemm_256.h"
+#include "xq_gemm_bank.h"
 #include "xq_gemm_dec.h"
 #include "xq_gemm_mid.h"
 #include <stdlib.h>
@@ -47,27 +48,20 @@ static int launch_256_one(const G256Args& f, dim3 grid, hipStream_t s, const cha
     return XQ_OK;
 }
 
-// Block-fp8 launches on large unsplit tiles (dense and expert banks) run gemm_dtl16_kernel (1, the default) or gemm_256_kernel (0): a
+// Block-fp8 launches on large unsplit tiles run gemm_dtl16_kernel (dense) and gemm_bank_kernel (1, the default) or gemm_256_kernel (0): a
 // process-wide switch for tests and A/B measurements, XQ_FP8_DIRECT in the environment sets it at load time.
 static std::atomic<int> g_fp8_direct{[] { const char* e = getenv("XQ_FP8_DIRECT"); return e ? atoi(e) : 1; }()};
 
-static int launch_dtl16(const G256Args& f, bool cc, bool grouped, dim3 grid, hipStream_t s, const char* who) {
+static int launch_dtl16(const G256Args& f, bool cc, dim3 grid, hipStream_t s, const char* who) {
     static std::atomic<bool> attr_set{false};
     if (!attr_set) {
-        int rc = raise_lds_limit(gemm_dtl16_kernel<true, 8, false>, GeoDtl::lds_total(), who);
-        if (!rc) rc = raise_lds_limit(gemm_dtl16_kernel<false, 8, false>, GeoDtl::lds_total(), who);
-        if (!rc) rc = raise_lds_limit(gemm_dtl16_kernel<true, 8, true>, GeoDtl::lds_total(), who);
-        if (!rc) rc = raise_lds_limit(gemm_dtl16_kernel<false, 8, true>, GeoDtl::lds_total(), who);
+        int rc = raise_lds_limit(gemm_dtl16_kernel<true>, GeoDtl::lds_total(), who);
+        if (!rc) rc = raise_lds_limit(gemm_dtl16_kernel<false>, GeoDtl::lds_total(), who);
         if (rc) return rc;
         attr_set = true;
     }
-    if (grouped) {
-        if (cc) gemm_dtl16_kernel<true, 8, true><<<grid, 512, GeoDtl::lds_total(), s>>>(f);
-        else gemm_dtl16_kernel<false, 8, true><<<grid, 512, GeoDtl::lds_total(), s>>>(f);
-    } else {
-        if (cc) gemm_dtl16_kernel<true, 8, false><<<grid, 512, GeoDtl::lds_total(), s>>>(f);
-        else gemm_dtl16_kernel<false, 8, false><<<grid, 512, GeoDtl::lds_total(), s>>>(f);
-    }
+    if (cc) gemm_dtl16_kernel<true><<<grid, GeoDtl::NT, GeoDtl::lds_total(), s>>>(f);
+    else gemm_dtl16_kernel<false><<<grid, GeoDtl::NT, GeoDtl::lds_total(), s>>>(f);
     return XQ_OK;
 }
 
@@ -114,14 +108,23 @@ static inline int dense_tile_size(int64_t n_rows, int64_t Nout) {
     return xq_cdiv(n_rows, 256) * xq_cdiv(Nout, 256) > num_cus() / 2 ? 256 : 128;
 }
 
-// The same for expert banks: large tiles where an expert's rows fill them (its last tile is half empty on average, and a 4-bit tile
-// decodes in full) and the tiles there are fill half the chip.  Forward and backward of a routed MLP, large over small tiles, by rows an
+// The same for expert banks.  4-bit banks: 256 x 256 tiles where an expert's rows fill them (its last tile is half empty on average, and a
+// 4-bit tile decodes in full) and the tiles there are fill half the chip.  Forward and backward of a routed MLP, large over small tiles, by rows an
 // expert: nvfp4 / nf4 banks, 64 or 128 experts 93 1.15, 187 1.04 to 1.08, 281 1.03 to 1.10, 421 0.97 to 0.99, 656 0.93; 16 experts 250
-// 1.10 to 1.14, 500 0.90; 8 experts 500 1.09 to 1.14, 750 0.87.  Block-fp8: 64 or 128 experts 46 1.14, 62 1.01, 93 1.04, 125 0.91, 281 0.87; 16
-// experts 125 1.00, 250 0.98, 500 0.81; 8 experts 125 1.23, 250 0.94, 750 0.87.
+// 1.10 to 1.14, 500 0.90; 8 experts 500 1.09 to 1.14, 750 0.87.
+// Block-fp8: gemm_bank_kernel's 128 x 256 tiles, two on a compute unit, where there is one for every compute unit, half a tile an expert
+// left empty, or for every third where an expert's rows fill most of one.  Routed MLP forward and backward, those over 128 x 128 tiles, by rows an expert:
+// 128 experts 2048/768 8 0.96, 24 0.95, 56 0.86, 96 0.84; 64 experts 2048/1024 6 0.94, 16 0.95, 32 1.03, 64 0.92, 96 0.81; 64 experts
+// 1280/640 6 1.10 and 16 1.02 (175 and 200 tiles), 32 0.99, 64 0.94; 32 experts 4096/1536 6 1.01, 32 1.03, 64 0.88; 32 experts 1536/640 56
+// 1.02, 72 1.02 (150 and 170 tiles), 96 0.97; 16 experts 2560/1024 40 1.11, 72 1.06 (136 tiles), 96 0.95; over 256 x 256 tiles, one on a compute unit:
+// 128 experts 128 0.83, 300 0.87, 512 0.91, 1024 0.91; 16 experts 192 0.94, 512 0.90.
 static inline bool bank_large_tiles(int fmt, int64_t n_rows, int num_experts, int64_t Nout) {
+    if (fmt == XQ_FMT_FP8) {
+        const int64_t tiles = (xq_cdiv(n_rows, GeoBank::ROWS) + num_experts / 2) * xq_cdiv(Nout, GeoBank::COLS);
+        return tiles >= (n_rows >= 90ll * num_experts ? num_cus() * 3 / 8 : num_cus());
+    }
     const int64_t tiles = (xq_cdiv(n_rows, 256) + num_experts / 2) * xq_cdiv(Nout, 256);
-    return n_rows >= (fmt == XQ_FMT_FP8 ? 100ll : 400ll) * num_experts && tiles > num_cus() / 2;
+    return n_rows >= 400ll * num_experts && tiles > num_cus() / 2;
 }
 
 // K splits of a dense launch of `blocks` tiles of size T over nk K-steps (1 = none): used when the tiles fill at
@@ -708,17 +711,23 @@ static int launch_tile_gemm_t(const xq_weight* w, bool contract_cols, const bf16
             dim3 grid(persistent ? persistent_grid(tiles_m * tiles_n) : (unsigned)(tiles_m * tiles_n), (unsigned)ksplit);
             const bool timed = xq_profile_mark_begin(stream, 2.0 * (double)n_rows * g.Nout * ((double)g.Kc + g.r_pad));
             int rc;
-            // block-fp8 on large unsplit tiles, dense or expert banks: the kernel that brings both operand tiles straight into LDS
-            // and decodes after the fragment read (xq_gemm_dtl.h), one block per tile
+            // block-fp8 on large unsplit tiles: the kernels that bring both operand tiles straight into LDS and decode after the fragment
+            // read, one block per tile (dense xq_gemm_dtl.h, expert banks xq_gemm_bank.h)
             const int nk_all = g.Kc / BK;
             // (two matrices: the second one starts on a scale-block boundary of the contraction, or -- two banks side by side
             // in a forward -- on a tile boundary of the columns)
             const bool two_ok = !two || ((grouped && !contract_cols) ? f.ncols1 % 256 == 0 : (f.nk1 % 2 == 0 && f.nk1 >= 2));
-            if (g_fp8_direct && w->format == XQ_FMT_FP8 && T == 256 && ksplit == 1 && nk_all >= 3 &&
-                nk_all <= 2 * GeoDtl::SCL_MAX && two_ok && (!grouped || g.wcols % 16 == 0) &&
-                // (its lanes address their operands by 32-bit byte offsets from a base)
-                a_rows_span > 0 && a_rows_span * lda * 2 < (1ll << 32) && (int64_t)g.wrows * g.wcols < (1ll << 32))
-                rc = launch_dtl16(f, contract_cols, grouped, dim3((unsigned)(tiles_m * tiles_n)), stream, who);
+            const int64_t reach = (1ll << 32) - (grouped ? 4096 : 0);
+            const bool direct = g_fp8_direct && w->format == XQ_FMT_FP8 && T == 256 && ksplit == 1 && nk_all >= 3 && two_ok &&
+                                // (their lanes address their operands by 32-bit byte offsets from a base, the bank kernel's up to 3 KB further on)
+                                a_rows_span > 0 && a_rows_span * lda * 2 < reach && (int64_t)g.wrows * g.wcols < reach;
+            if (direct && grouped && g.wcols % 16 == 0 && f.wide_rows && !bias) {
+                f.tiles_m = (int32_t)(xq_cdiv(n_rows, GeoBank::ROWS) + w->num_experts);
+                f.tiles_n = (int32_t)xq_cdiv(g.Nout, GeoBank::COLS);
+                f.tile_prefix = tile_offsets;                // (its tiles have 128 rows)
+                rc = launch_bank(f, contract_cols, stream, who);
+            } else if (direct && !grouped && nk_all <= 2 * GeoDtl::SCL_MAX)
+                rc = launch_dtl16(f, contract_cols, dim3((unsigned)(tiles_m * tiles_n)), stream, who);
             else if (w->format == XQ_FMT_FP8) rc = launch_256<XQ_FMT_FP8>(f, contract_cols, grouped, T, grid, stream, who);
             else if (w->format == XQ_FMT_INT4) rc = launch_256<XQ_FMT_INT4>(f, contract_cols, grouped, T, grid, stream, who);
             else if (w->format == XQ_FMT_NF4) rc = launch_256<XQ_FMT_NF4>(f, contract_cols, grouped, T, grid, stream, who);

@@ -1142,7 +1142,7 @@ __global__ void __launch_bounds__(2 * T, 2) gemm_256_kernel(G256Args g) {
 }
 
 // C[row][n] = bf16(partial[0][row][n] + partial[1][row][n] + ...), splits added in index order; a thread per 4 columns
-__global__ void __launch_bounds__(256) splitk_reduce_kernel(const float* __restrict__ partial, int ksplit, int64_t M, int Nout,
+static __global__ void __launch_bounds__(256) splitk_reduce_kernel(const float* __restrict__ partial, int ksplit, int64_t M, int Nout,
                                                             bf16_t* __restrict__ C, int64_t ldc) {
     const int64_t quads = (int64_t)(Nout >> 2), idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (idx >= M * quads) return;

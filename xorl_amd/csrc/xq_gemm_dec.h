@@ -325,7 +325,7 @@ __global__ void __launch_bounds__(512, 2) gemm_dec_kernel(G256Args g) {
         const int s = blockIdx.y;
         G256Args f = g;
         if (s > 0) { f.r_pad = 0; f.bias = nullptr; }
-        dtl16_side_term<TM, TN, 8, false>(f, dsm, G::ROWS * 128, acc, row0, row_end, n0, g.Nout, f.su, nullptr, 0, tid_e);
+        dtl16_side_term<TM, TN>(f, dsm, G::ROWS * 128, acc, row0, row_end, n0, tid_e);
         float* part = g.partial + (int64_t)s * g.M * g.Nout;
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
@@ -342,7 +342,7 @@ __global__ void __launch_bounds__(512, 2) gemm_dec_kernel(G256Args g) {
             }
         }
     } else {
-        dtl16_finish<TM, TN, 8, false>(g, dsm, G::ROWS * 128, acc, row0, row_end, n0, n0, g.Nout, g.su, nullptr, 0, tid_e);
+        dtl16_finish<TM, TN>(g, dsm, G::ROWS * 128, acc, row0, row_end, n0, tid_e);
     }
 }
 

@@ -64,16 +64,15 @@ __device__ __forceinline__ u32x2 dtl_decode4(uint32_t w, float sc) {
     return u32x2{pack_bf16x2(x0[0] * sc, x0[1] * sc), pack_bf16x2(x1[0] * sc, x1[1] * sc)};
 }
 
-// The end of a tile of the kernels whose waves, two or one down and four across, hold TM x TN tiles of 16 x 16 sums
+// The end of a tile of the kernels whose waves, two down and four across, hold TM x TN tiles of 16 x 16 sums
 // (gemm_dtl16_kernel, gemm_dec_kernel).  `dsm` is the block's LDS, read by nobody else behind the barrier here, with room for 128
 // bytes of every row; `second` bytes into it lies room for as much of every column.  First the low-rank side term:
-template <int TM, int TN, int NW, bool GROUPED>
+template <int TM, int TN>
 __device__ __forceinline__ void dtl16_side_term(const G256Args& g, unsigned char* dsm, int second, f32x4 (&acc)[TM][TN], int64_t row0,
-                                                int64_t row_end, int n0w, int bank_width, const bf16_t* su_b, const bf16_t* lr_b, int e,
-                                                int tid = threadIdx.x) {
-    constexpr int NT = NW * 64, RW = TM * 16, CW = TN * 16, TA = RW * (NW / 4), TB = CW * 4;
+                                                int64_t row_end, int n0, int tid = threadIdx.x) {
+    constexpr int NT = 512, RW = TM * 16, CW = TN * 16, TA = RW * 2, TB = CW * 4;
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = NW == 8 ? wave >> 2 : 0, wn = wave & 3;
+    const int wm = wave >> 2, wn = wave & 3;
     const int l16 = lane & 15, lg = lane >> 4;
     // ---- low-rank side term: su[rows, rp] x lora_right[n, rp] as bf16 [row][64 k] tiles in the first two stages, k beyond
     // rp zero up to the next multiple of 32
@@ -82,18 +81,16 @@ __device__ __forceinline__ void dtl16_side_term(const G256Args& g, unsigned char
     __syncthreads();
     if (g.r_pad > 0) {
         const int rp = g.r_pad, steps = (rp + 31) >> 5, cpr = steps << 2, have = rp >> 3;
-        const bf16_t* lr = lr_b + (int64_t)e * bank_width * rp;
         for (int idx = tid; idx < (TA > TB ? TA : TB) * cpr; idx += NT) {
             const int r = idx / cpr, c = idx - r * cpr;
             int64_t row = row0 + r;
             row = row < row_end ? row : row_end - 1;
-            int n = n0w + r;
-            n = n < bank_width ? n : bank_width - 1;
+            int n = n0 + r;
+            n = n < g.Nout ? n : g.Nout - 1;
             const u32x4 z = {0, 0, 0, 0};
-            if (TA >= TB || r < TA) *(u32x4*)(As + swz(r, c)) = c < have ? *(const u32x4*)(su_b + row * g.ld_su + c * 8) : z;
+            if (TA >= TB || r < TA) *(u32x4*)(As + swz(r, c)) = c < have ? *(const u32x4*)(g.su + row * g.ld_su + c * 8) : z;
             if (TB < TA && r >= TB) continue;
-            if constexpr (GROUPED) *(u32x4*)(Bs + swz(r, c)) = c < have ? *(const u32x4*)(lr + (int64_t)n * rp + c * 8) : z;
-            else *(u32x4*)(Bs + swz(r, c)) = c < have ? right_chunk(g.right, -1, n, c) : z;
+            *(u32x4*)(Bs + swz(r, c)) = c < have ? right_chunk(g.right, -1, n, c) : z;
         }
         __syncthreads();
         for (int ks = 0; ks < steps; ++ks) {
@@ -105,8 +102,7 @@ __device__ __forceinline__ void dtl16_side_term(const G256Args& g, unsigned char
                 const bf16x8 ax = *(const bf16x8*)(As + swz(wm * RW + i * 16 + l16, ks * 4 + lg));
 #pragma unroll
                 for (int j = 0; j < TN; ++j) {
-                    if constexpr (NW == 4) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(bw[j]), "v"(ax));
-                    else acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bw[j], ax, acc[i][j], 0, 0, 0);
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bw[j], ax, acc[i][j], 0, 0, 0);
                 }
             }
         }
@@ -115,20 +111,18 @@ __device__ __forceinline__ void dtl16_side_term(const G256Args& g, unsigned char
 }
 
 // ... and the whole end: side term, bias, the way out as bf16
-template <int TM, int TN, int NW, bool GROUPED>
+template <int TM, int TN>
 __device__ __forceinline__ void dtl16_finish(const G256Args& g, unsigned char* dsm, int second, f32x4 (&acc)[TM][TN], int64_t row0,
-                                             int64_t row_end, int n0, int n0w, int bank_width, const bf16_t* su_b, const bf16_t* lr_b, int e,
-                                             int tid = threadIdx.x) {
+                                             int64_t row_end, int n0, int tid = threadIdx.x) {
     constexpr int RW = TM * 16, CW = TN * 16;
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = NW == 8 ? wave >> 2 : 0, wn = wave & 3;
-    dtl16_side_term<TM, TN, NW, GROUPED>(g, dsm, second, acc, row0, row_end, n0w, bank_width, su_b, lr_b, e, tid);
+    const int wm = wave >> 2, wn = wave & 3;
+    dtl16_side_term<TM, TN>(g, dsm, second, acc, row0, row_end, n0, tid);
 
     // ---- the finished tile.  Lane l holds, per (i, j) tile, row 16 i + l % 16 and the 4 columns 16 j + 4 (l / 16) ..: 8 bytes
     // of bf16.  Each wave passes its RW x CW sub-tile through a private LDS area and writes whole row pieces of 16 CW bytes / 8:
     // at once in 128-byte rows with the chunk swizzle, or, where that is more than the LDS there is, in two groups of row tiles.
-    if constexpr (NW == 4) asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");     // the last MFMA results, written outside the compiler's hazard tracking
-    constexpr int TG = TM * TN <= 32 || NW == 4 ? TM : (TM + 1) / 2;      // row tiles of a group
+    constexpr int TG = TM * TN <= 32 ? TM : (TM + 1) / 2;      // row tiles of a group
     constexpr int CH = CW / 8;                                            // 16-byte chunks of a row
     bf16_t* stg = (bf16_t*)dsm + wave * (TG * 16 * CW);
     auto at = [&](int r, int c) { return TN == 4 ? swz(r, c) : r * CW + c * 8; };
@@ -173,87 +167,34 @@ __device__ __forceinline__ void dtl16_finish(const G256Args& g, unsigned char* d
     }
 }
 
-// NW = 8: eight waves as 2 x 4, a wave 128 x 64 (two waves per SIMD).  NW = 4: four waves side by side, a wave 256 x 64
-// with its 256 accumulator registers (one wave per SIMD): every weight value is then decoded by exactly one wave -- half
-// the conversions per MFMA of the eight-wave form, whose column blocks are shared by two waves -- and an activation
-// fragment feeds the same four MFMAs.
-//
-// GROUPED: the rows are in expert order and W is a bank of matrices of one shape (G256Args: offsets, tile_prefix,
-// packed_stride, scale_stride, a_rows); a block finds the expert of its row tile, reads and writes that expert's rows only,
-// and is gone if the launch holds fewer row tiles than its grid covers.  !CC is a bank's forward (optionally over two
-// banks side by side: column tiles from ncols1 on take the second bank), CC its dgrad (optionally one sum over two banks:
-// K-steps from nk1 on read the second one).
-template <bool CC, int NW, bool GROUPED = false>
-__global__ void __launch_bounds__(NW * 64, NW == 8 ? 2 : 1) gemm_dtl16_kernel(G256Args g) {
+template <bool CC>
+__global__ void __launch_bounds__(512, 2) gemm_dtl16_kernel(G256Args g) {
     using D = GeoDtl;
-    constexpr int T = 256, TN = 4, NT = NW * 64;
-    constexpr int RW = NW == 8 ? 128 : 256;          // rows of a wave's sub-tile
-    constexpr int TM = RW / 16;                      // its row tiles: 8 or 16
+    constexpr int T = 256, TN = 4, NT = D::NT;       // eight waves as 2 x 4, a wave 128 x 64 (two waves per SIMD)
+    constexpr int RW = 128, TM = RW / 16;            // rows of a wave's sub-tile, its row tiles
     constexpr int NC = 2 * TM;                       // chunks of a K-step
-    constexpr int AP = 32 / NW, WP = 16 / NW;        // direct loads per wave and K-step: activation rows, weight rows
+    constexpr int AP = 4, WP = 2;                    // direct loads per wave and K-step: activation rows, weight rows
     extern __shared__ __attribute__((aligned(16))) unsigned char dsm[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = NW == 8 ? wave >> 2 : 0, wn = wave & 3;
+    const int wm = wave >> 2, wn = wave & 3;
     const int l16 = lane & 15, lg = lane >> 4;
 
     int pid_m, pid_n;
     {
-        // (grouped: the grid covers an upper bound of the row tiles; the order is laid over the tiles there are, so that
-        // the blocks with nothing to do are not all one XCD's)
-        const int nb = (GROUPED ? g.tile_prefix[g.num_experts] : g.tiles_m) * g.tiles_n;
+        const int nb = g.tiles_m * g.tiles_n;
         const int b = blockIdx.x, per = nb >> 3;
-        if (GROUPED && b >= nb) return;
         const int logical = (b < per * 8) ? (b & 7) * per + (b >> 3) : b;
-        if constexpr (GROUPED) {
-            pid_m = logical / g.tiles_n;      // all column tiles of a row tile side by side: an XCD stays on one expert's matrix
-            pid_n = logical - pid_m * g.tiles_n;
-        } else {
-            constexpr int GM = 4;
-            const int width = GM * g.tiles_n;
-            const int grp = logical / width, first_m = grp * GM;
-            const int gsz = min(g.tiles_m - first_m, GM);
-            const int in = logical - grp * width;
-            pid_m = first_m + in % gsz;
-            pid_n = in / gsz;
-        }
+        constexpr int GM = 4;
+        const int width = GM * g.tiles_n;
+        const int grp = logical / width, first_m = grp * GM;
+        const int gsz = min(g.tiles_m - first_m, GM);
+        const int in = logical - grp * width;
+        pid_m = first_m + in % gsz;
+        pid_n = in / gsz;
     }
-    // the tile: expert, rows it may read and write, output columns (n0) and the same columns within their bank (n0w)
-    int e = 0;
-    int64_t row0 = (int64_t)pid_m * T, row_end = g.M;
-    if constexpr (GROUPED) {
-        // thread t looks at expert t (t + NT, ...): one memory round trip instead of a search's chain of dependent loads
-        __shared__ int sh_tile[3];
-        if (tid == 0) sh_tile[0] = -1;
-        __syncthreads();
-        for (int t = tid; t < g.num_experts; t += NT) {
-            const int lo = g.tile_prefix[t], hi = g.tile_prefix[t + 1];
-            if (lo <= pid_m && pid_m < hi) {
-                sh_tile[0] = t;
-                sh_tile[1] = g.offsets[t] + (pid_m - lo) * T;
-                sh_tile[2] = g.offsets[t + 1];
-            }
-        }
-        __syncthreads();
-        e = __builtin_amdgcn_readfirstlane(sh_tile[0]);
-        if (e < 0) return;                    // (cannot happen for a row tile below tile_prefix[num_experts])
-        row0 = __builtin_amdgcn_readfirstlane(sh_tile[1]);
-        row_end = __builtin_amdgcn_readfirstlane(sh_tile[2]);
-    }
+    const int64_t row0 = (int64_t)pid_m * T, row_end = g.M;
     const int n0 = pid_n * T;
-    int n0w = n0, bank_width = g.Nout;
-    const uint8_t* Wb = g.W + (int64_t)e * g.packed_stride;
-    const float* Sb = (const float*)(g.scales + (int64_t)e * g.scale_stride);
-    const float* Sb2 = g.W2 != nullptr ? (const float*)(g.scales2 + (int64_t)e * g.scale_stride) : nullptr;
-    const bf16_t* su_b = g.su;
-    const bf16_t* lr_b = g.lora_right;
-    if constexpr (GROUPED && !CC) {
-        if (g.W2 != nullptr) {
-            bank_width = g.ncols1;
-            if (n0 >= g.ncols1) {
-                Wb = g.W2 + (int64_t)e * g.packed_stride; Sb = Sb2; su_b = g.su2; lr_b = g.lora_right2; n0w = n0 - g.ncols1;
-            }
-        }
-    }
+    const float *Sb = (const float*)g.scales, *Sb2 = (const float*)g.scales2;
     const int nk = g.Kc / D::BK;
     const int scols = (g.wcols + 127) >> 7;
     // 16-row tiles of this wave's sub-tile that hold rows of the problem: the MFMAs of the others are skipped (their sums
@@ -272,9 +213,6 @@ __global__ void __launch_bounds__(NW * 64, NW == 8 ? 2 : 1) gemm_dtl16_kernel(G2
         const int rt = (wave * AP + p) * 8 + (lane >> 3);
         int64_t r = row0 + rt;
         r = r < row_end ? r : row_end - 1;
-        if constexpr (GROUPED) {
-            if (g.a_rows) r = g.a_rows[r];
-        }
         a_off[p] = (uint32_t)((r * g.lda + (((lane & 7) ^ ((rt >> 1) & 5)) << 3)) * 2);
     }
     uint32_t w_off[WP];
@@ -282,18 +220,18 @@ __global__ void __launch_bounds__(NW * 64, NW == 8 ? 2 : 1) gemm_dtl16_kernel(G2
     for (int q = 0; q < WP; ++q) {
         if (CC) {
             const int rt = (wave * WP + q) * 16 + (lane >> 2);
-            const int wr = min(n0w + rt, g.wrows - 1);
+            const int wr = min(n0 + rt, g.wrows - 1);
             w_off[q] = (uint32_t)((int64_t)wr * g.wcols + (((lane & 3) ^ ((rt >> 2) & 2)) << 4));
         } else {
             const int kr = (wave * WP + q) * 4 + (lane >> 4);
-            const int wc = min(n0w + (((lane & 15) ^ (kr & 7)) << 4), g.wcols - 16);
+            const int wc = min(n0 + (((lane & 15) ^ (kr & 7)) << 4), g.wcols - 16);
             w_off[q] = (uint32_t)((int64_t)kr * g.wcols + wc);
         }
     }
     const int64_t w_kstep = CC ? D::BK : (int64_t)D::BK * g.wcols;
-    // contraction over two matrices of one shape (dgrad of gate and up as one sum, G256Args::W2; dense: !CC, banks: CC):
-    // K-steps from nk1 on read the second matrix (the same expert's), from its first K-step
-    constexpr bool TWO_K = GROUPED ? CC : !CC;
+    // contraction over two matrices of one shape (dgrad of gate and up as one sum, G256Args::W2):
+    // K-steps from nk1 on read the second matrix, from its first K-step
+    constexpr bool TWO_K = !CC;
     const int nk1 = (TWO_K && g.W2 != nullptr) ? g.nk1 : (1 << 30);
     const int64_t w2_delta = (TWO_K && g.W2 != nullptr) ? (g.W2 - g.W) - (int64_t)nk1 * w_kstep : 0;
     // (written out: the compiler's form of this load takes a 64-bit address per lane.  M0 -- the LDS base of the load -- is
@@ -307,7 +245,7 @@ __global__ void __launch_bounds__(NW * 64, NW == 8 ? 2 : 1) gemm_dtl16_kernel(G2
             asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
                          :: "s"(a + part * 1024), "v"(a_off[part]), "s"(base) : "memory");
         } else {
-            const unsigned char* base = Wb + (kt * w_kstep + (kt >= nk1 ? w2_delta : 0));
+            const unsigned char* base = g.W + (kt * w_kstep + (kt >= nk1 ? w2_delta : 0));
             asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
                          :: "s"(w + (part - AP) * 1024), "v"(w_off[part - AP]), "s"(base) : "memory");
         }
@@ -318,7 +256,7 @@ __global__ void __launch_bounds__(NW * 64, NW == 8 ? 2 : 1) gemm_dtl16_kernel(G2
         const int nkb = (nk + 1) >> 1;
         for (int i = tid; i < 2 * nkb; i += NT) {
             const int blk = i / nkb, kb = i - blk * nkb;
-            const int nn = n0w + blk * 128;
+            const int nn = n0 + blk * 128;
             const bool second = 2 * kb >= nk1;                      // (nk1 is even: the matrices change on a scale-block boundary)
             const float* sp = second ? Sb2 : Sb;
             const int kb1 = second ? kb - (nk1 >> 1) : kb;
@@ -446,13 +384,7 @@ __global__ void __launch_bounds__(NW * 64, NW == 8 ? 2 : 1) gemm_dtl16_kernel(G2
             if (!SKIP || i < mt)
 #pragma unroll
             for (int j = 0; j < TN; ++j) {
-                if constexpr (NW == 4) {
-                    // (written out so that the accumulator stays where it is: left to itself the register allocator moves the
-                    // 256 accumulator registers of this form between the two register files around every MFMA)
-                    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(c < TM ? fb0[j] : fb1[j]), "v"(fa[c & 3]));
-                } else {
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, c < TM ? fb0[j] : fb1[j]), fa[c & 3], acc[i][j], 0, 0, 0);
-                }
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, c < TM ? fb0[j] : fb1[j]), fa[c & 3], acc[i][j], 0, 0, 0);
             }
             // the activation fragment three chunks on (the last three chunks fetch the next K-step's first three)
             if (c + 3 < NC) XQ_DTL_READ_A(fa[(c + 3) & 3], so, c + 3);
@@ -506,10 +438,8 @@ __global__ void __launch_bounds__(NW * 64, NW == 8 ? 2 : 1) gemm_dtl16_kernel(G2
             iteration(kt, Tt{}, Ff{}, SKIP_);
             iteration(kt + 1, Ff{}, Ff{}, SKIP_);
         };
-        // A wave without rows (the lower half of a tile of 128 rows or fewer) only brings in its share of the operands: the decode and the
+        // A wave without rows (the lower half of a last tile of 128 rows or fewer) only brings in its share of the operands: the decode and the
         // fragment reads that it leaves out are issue slots of the wave beside it.
-        // (Routed MLP, forward and backward, us: 16 experts 4000 routed rows 498 -> 486, 64 experts 7200 671 -> 659, 27000 1252 -> 1234, 128
-        // experts 40000 1545 -> 1520.)
         if (mt == TM) run(Ff{});
         else if (mt > 0) run(Tt{});
         else
@@ -527,7 +457,7 @@ __global__ void __launch_bounds__(NW * 64, NW == 8 ? 2 : 1) gemm_dtl16_kernel(G2
 #undef XQ_DTL_READ_A
 #undef XQ_DTL_READ_W
 
-    dtl16_finish<TM, TN, NW, GROUPED>(g, dsm, D::STAGE_BYTES, acc, row0, row_end, n0, n0w, bank_width, su_b, lr_b, e);
+    dtl16_finish<TM, TN>(g, dsm, D::STAGE_BYTES, acc, row0, row_end, n0);
 }
 
 }  // namespace xq

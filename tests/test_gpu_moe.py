@@ -930,9 +930,9 @@ def test_route_build_at_the_edges(hip_device, n, E):
     assert torch.equal(tiles.flatten().long(), torch.cat([prefix((want_counts + t - 1) // t) for t in (128, 256)]))
 
 
-@pytest.mark.parametrize("tile_policy", [2], indirect=True)
+@pytest.mark.parametrize("fmt", ["block_fp8", "nvfp4"])
 @pytest.mark.parametrize("K,N,r", [(192, 320, 0), (256, 832, 16), (448, 768, 48), (8320, 256, 64)])     # three K-steps up to three loads of scales
-def test_bank_tiles_vs_fp32(hip_device, tile_policy, K, N, r):
+def test_bank_tiles_vs_fp32(hip_device, fmt, K, N, r):
     """Tiles of 128 rows x 256 columns at their edges (whole tiles, one row, remainders of 16 rows, empty experts, more than 256 experts),
     both directions: against fp32 products of the decoded weights.  A result is rounded to bf16 once (2^-9 of it; the bound has twice
     that); the fp32 sums of n products differ by at most n 2^-24 of the sum of their magnitudes."""
@@ -940,15 +940,21 @@ def test_bank_tiles_vs_fp32(hip_device, tile_policy, K, N, r):
     from xorl_amd import quantize as Q
     from xorl_amd.functional import QuantWeight
 
-    counts = [128, 0, 1, 127, 129, 16, 113, 300, 0, 240]
+    counts = [128, 0, 1, 127, 129, 16, 113, 300, 0, 240] * 8        # (enough tiles for the rule that chooses them)
     if K == 192:
-        counts = [c for c in counts for _ in (0, 1)] + [0, 3] * 130
+        counts = counts + [0, 300] * 100
     E, n = len(counts), sum(counts)
-    bank = [Q.block_fp8_quantize_gkn(gen((K, N), 0.05, 100 + e)) for e in range(7)]
-    packed = torch.stack([bank[e % 7][0].view(torch.uint8) for e in range(E)]).to(hip_device)
-    scales = torch.stack([bank[e % 7][1] for e in range(E)]).to(hip_device)
-    ref = [bits_to_bf16(NP.fp8_decode(b.view(torch.uint8).numpy(), s.numpy(), K, N)[1]).to(hip_device).float() for b, s in bank]
-    qw = QuantWeight("block_fp8", _C.XQ_LAYOUT_GKN, packed, scales, torch.float32, K, N, 128, num_experts=E)
+    w = [gen((K, N), 0.05, 100 + e) for e in range(7)]
+    if fmt == "block_fp8":
+        bank = [Q.block_fp8_quantize_gkn(m) for m in w]
+        ref = [NP.fp8_decode(b.view(torch.uint8).numpy(), s.numpy(), K, N)[1] for b, s in bank]
+    else:
+        bank = [Q.nvfp4_quantize_gkn(m) for m in w]
+        ref = [NP.nvfp4_decode_gkn(c.numpy(), C.e4m3_scales_to_f32(b.view(torch.uint8).numpy()), float(g), K, N) for c, b, g in bank]
+    stack = lambda i: torch.stack([bank[e % 7][i].view(torch.uint8 if i == 0 else bank[0][i].dtype) for e in range(E)]).to(hip_device)
+    ref = [bits_to_bf16(r_).to(hip_device).float() for r_ in ref]
+    qw = QuantWeight(fmt, _C.XQ_LAYOUT_GKN, stack(0), stack(1), bank[0][1].dtype, K, N, 128 if fmt == "block_fp8" else 16,
+                     global_scale=None if fmt == "block_fp8" else stack(2).float().reshape(E), num_experts=E)
     sel = torch.arange(E, dtype=torch.int32).repeat_interleave(torch.tensor(counts)).reshape(-1, 1).to(hip_device)
     _, offsets, _, tile_offsets = MF.route_build(sel, E)
     starts = [sum(counts[:e]) for e in range(E)]
@@ -961,9 +967,9 @@ def test_bank_tiles_vs_fp32(hip_device, tile_policy, K, N, r):
         for e, (s, c) in enumerate(zip(starts, counts)):
             if c == 0:
                 continue
-            w = ref[e % 7].t() if transpose_w else ref[e % 7]
+            m = ref[e % 7].t() if transpose_w else ref[e % 7]
             x = a[s:s + c].float()
-            want, size = x @ w, x.abs() @ w.abs()
+            want, size = x @ m, x.abs() @ m.abs()
             if r:
                 want, size = want + su[s:s + c].float() @ right[e].float().t(), size + su[s:s + c].float().abs() @ right[e].float().abs().t()
             assert bool(((y[s:s + c] - want).abs() <= 2.0 ** -8 * want.abs() + (kc + r) * 2.0 ** -24 * size).all()), (transpose_w, e, c)

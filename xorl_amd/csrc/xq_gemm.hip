@@ -108,20 +108,23 @@ static inline int dense_tile_size(int64_t n_rows, int64_t Nout) {
     return xq_cdiv(n_rows, 256) * xq_cdiv(Nout, 256) > num_cus() / 2 ? 256 : 128;
 }
 
-// The same for expert banks.  4-bit banks: 256 x 256 tiles where an expert's rows fill them (its last tile is half empty on average, and a
+// The same for expert banks.  nf4 and int4: 256 x 256 tiles where an expert's rows fill them (its last tile is half empty on average, and a
 // 4-bit tile decodes in full) and the tiles there are fill half the chip.  Forward and backward of a routed MLP, large over small tiles, by rows an
-// expert: nvfp4 / nf4 banks, 64 or 128 experts 93 1.15, 187 1.04 to 1.08, 281 1.03 to 1.10, 421 0.97 to 0.99, 656 0.93; 16 experts 250
+// expert: nf4 banks, 64 or 128 experts 93 1.15, 187 1.04 to 1.08, 281 1.03 to 1.10, 421 0.97 to 0.99, 656 0.93; 16 experts 250
 // 1.10 to 1.14, 500 0.90; 8 experts 500 1.09 to 1.14, 750 0.87.
-// Block-fp8: gemm_bank_kernel's 128 x 256 tiles, two on a compute unit, where there is one for every compute unit, half a tile an expert
-// left empty, or for every third where an expert's rows fill most of one.  Routed MLP forward and backward, those over 128 x 128 tiles, by rows an expert:
-// 128 experts 2048/768 8 0.96, 24 0.95, 56 0.86, 96 0.84; 64 experts 2048/1024 6 0.94, 16 0.95, 32 1.03, 64 0.92, 96 0.81; 64 experts
-// 1280/640 6 1.10 and 16 1.02 (175 and 200 tiles), 32 0.99, 64 0.94; 32 experts 4096/1536 6 1.01, 32 1.03, 64 0.88; 32 experts 1536/640 56
-// 1.02, 72 1.02 (150 and 170 tiles), 96 0.97; 16 experts 2560/1024 40 1.11, 72 1.06 (136 tiles), 96 0.95; over 256 x 256 tiles, one on a compute unit:
-// 128 experts 128 0.83, 300 0.87, 512 0.91, 1024 0.91; 16 experts 192 0.94, 512 0.90.
+// Block-fp8 and nvfp4: gemm_bank_kernel's 128 x 256 tiles, two on a compute unit, where there is one for every compute unit, half a tile an
+// expert left empty, or for every third where an expert's rows fill half of one (nvfp4) or most of one.  Routed MLP forward and backward, those
+// over 128 x 128 tiles, by rows an expert, block-fp8: 128 experts 2048/768 8 0.96, 24 0.95, 56 0.86, 96 0.84; 64 experts 2048/1024 6
+// 0.94, 16 0.95, 32 1.03, 64 0.92, 96 0.81; 64 experts 1280/640 6 1.10 and 16 1.02 (175 and 200 tiles), 32 0.99, 64 0.94; 32 experts 4096/1536 6
+// 1.01, 32 1.03, 64 0.88; 32 experts 1536/640 56 1.02, 72 1.02 (150 and 170 tiles), 96 0.97; 16 experts 2560/1024 40 1.11, 72 1.06 (136 tiles),
+// 96 0.95; over 256 x 256 tiles, one on a compute unit: 128 experts 128 0.83, 300 0.87, 512 0.91, 1024 0.91; 16 experts 192 0.94, 512 0.90.
+// nvfp4, over the tiles of nf4's rule: 128 experts 2048/768 6 0.85, 16 0.87, 32 0.81, 64 0.76, 128 0.73, 256 0.71, 600 0.77; 64 experts 1280/640 16
+// 1.05, 32 0.99 (240 tiles), 64 0.91, 128 0.88, 600 0.78; 16 experts 2560/1024 32 1.05, 64 0.98 (128 tiles), 96 0.89, 256 0.82, 600 0.81.
 static inline bool bank_large_tiles(int fmt, int64_t n_rows, int num_experts, int64_t Nout) {
-    if (fmt == XQ_FMT_FP8) {
-        const int64_t tiles = (xq_cdiv(n_rows, GeoBank::ROWS) + num_experts / 2) * xq_cdiv(Nout, GeoBank::COLS);
-        return tiles >= (n_rows >= 90ll * num_experts ? num_cus() * 3 / 8 : num_cus());
+    if (fmt == XQ_FMT_FP8 || fmt == XQ_FMT_NVFP4) {
+        using D = GeoBank<XQ_FMT_FP8>;
+        const int64_t tiles = (xq_cdiv(n_rows, D::ROWS) + num_experts / 2) * xq_cdiv(Nout, D::COLS);
+        return tiles >= (n_rows >= (fmt == XQ_FMT_FP8 ? 90ll : 60ll) * num_experts ? num_cus() * 3 / 8 : num_cus());
     }
     const int64_t tiles = (xq_cdiv(n_rows, 256) + num_experts / 2) * xq_cdiv(Nout, 256);
     return n_rows >= 400ll * num_experts && tiles > num_cus() / 2;
@@ -711,21 +714,25 @@ static int launch_tile_gemm_t(const xq_weight* w, bool contract_cols, const bf16
             dim3 grid(persistent ? persistent_grid(tiles_m * tiles_n) : (unsigned)(tiles_m * tiles_n), (unsigned)ksplit);
             const bool timed = xq_profile_mark_begin(stream, 2.0 * (double)n_rows * g.Nout * ((double)g.Kc + g.r_pad));
             int rc;
-            // block-fp8 on large unsplit tiles: the kernels that bring both operand tiles straight into LDS and decode after the fragment
+            // block-fp8, and nvfp4 banks, on large unsplit tiles: the kernels that bring both operand tiles straight into LDS and decode after the fragment
             // read, one block per tile (dense xq_gemm_dtl.h, expert banks xq_gemm_bank.h)
             const int nk_all = g.Kc / BK;
-            // (two matrices: the second one starts on a scale-block boundary of the contraction, or -- two banks side by side
-            // in a forward -- on a tile boundary of the columns)
-            const bool two_ok = !two || ((grouped && !contract_cols) ? f.ncols1 % 256 == 0 : (f.nk1 % 2 == 0 && f.nk1 >= 2));
+            // (two matrices: the second one starts on a scale-block boundary of the contraction, or -- two banks side by side -- on a
+            // tile boundary of the columns.  nvfp4 banks under a forced tile size stay on gemm_256_kernel, whose sums are the same
+            // for both sizes.)
+            const bool side_by_side = grouped && (!contract_cols || w->format != XQ_FMT_FP8);
+            const bool two_ok = !two || (side_by_side ? f.ncols1 % 256 == 0 : (f.nk1 % 2 == 0 && f.nk1 >= 2));
             const int64_t reach = (1ll << 32) - (grouped ? 4096 : 0);
-            const bool direct = g_fp8_direct && w->format == XQ_FMT_FP8 && T == 256 && ksplit == 1 && nk_all >= 3 && two_ok &&
+            const bool storage = w->format == XQ_FMT_FP8 || (grouped && w->format == XQ_FMT_NVFP4 && g_tile_policy == 0 && g.group == 16 && g.scale_dtype == XQ_SCALE_E4M3);
+            const bool direct = g_fp8_direct && storage && T == 256 && ksplit == 1 && nk_all >= 3 && two_ok &&
                                 // (their lanes address their operands by 32-bit byte offsets from a base, the bank kernel's up to 3 KB further on)
                                 a_rows_span > 0 && a_rows_span * lda * 2 < reach && (int64_t)g.wrows * g.wcols < reach;
             if (direct && grouped && g.wcols % 16 == 0 && f.wide_rows && !bias) {
-                f.tiles_m = (int32_t)(xq_cdiv(n_rows, GeoBank::ROWS) + w->num_experts);
-                f.tiles_n = (int32_t)xq_cdiv(g.Nout, GeoBank::COLS);
+                using D = GeoBank<XQ_FMT_FP8>;
+                f.tiles_m = (int32_t)(xq_cdiv(n_rows, D::ROWS) + w->num_experts);
+                f.tiles_n = (int32_t)xq_cdiv(g.Nout, D::COLS);
                 f.tile_prefix = tile_offsets;                // (its tiles have 128 rows)
-                rc = launch_bank(f, contract_cols, stream, who);
+                rc = launch_bank(f, w->format, contract_cols, stream, who);
             } else if (direct && !grouped && nk_all <= 2 * GeoDtl::SCL_MAX)
                 rc = launch_dtl16(f, contract_cols, dim3((unsigned)(tiles_m * tiles_n)), stream, who);
             else if (w->format == XQ_FMT_FP8) rc = launch_256<XQ_FMT_FP8>(f, contract_cols, grouped, T, grid, stream, who);

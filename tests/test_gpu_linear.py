@@ -489,3 +489,22 @@ def test_activation_rows_that_span_4gib(hip_device):
     close(y_view.cpu(), ex["y"], TOL)
     close(y_copy.cpu(), ex["y"], TOL)
     assert R.max_rel_err(y_view.cpu().float(), y_copy.cpu().float()) <= 2 ** -7
+
+
+@pytest.mark.parametrize("M,K,N,r,forward", [
+    (2309, 320, 8256, 8, True), (1300, 576, 13120, 16, True), (1500, 384, 13120, 64, True),       # five to nine K-steps, ragged rows and columns
+    (1500, 13120, 384, 32, False), (2305, 8256, 448, 8, False),
+])
+def test_dense_half_tiles(hip_device, M, K, N, r, forward):
+    """Dense block-fp8 on tiles of 128 rows x 256 columns (a last round of 256 x 256 tiles would be half empty), one direction of
+    each case, with a bias: against the float64 form, and the tiles' last rows and columns by themselves."""
+    n_out, k = (N, K) if forward else (K, N)
+    assert dense_route("block_fp8", forward, M, n_out, k) == ("tiles", 128, 256, 1, 0, 0, 0)
+    m, w_ref = make_dense_module("block_fp8", N, K, r, 32, seed=M + r, device=hip_device, bias=True)
+    x, dy = gen((M, K), 1.0, 31, torch.bfloat16), gen((M, N), 1.0, 32, torch.bfloat16)
+    y, dx, _, _ = _run(m, x.to(hip_device), dy.to(hip_device))
+    ex = R.linear_fwd_bwd_exact(x, w_ref, m.lora_A.detach().cpu(), m.lora_B.detach().cpu(), m.scaling, dy, bias=m.bias.detach().cpu())
+    for got, ref in ((y.cpu(), ex["y"]), (dx.cpu(), ex["dx"])):
+        close(got, ref, TOL)
+        close(got[M // 128 * 128:], ref[M // 128 * 128:], TOL)
+        close(got[:, got.shape[1] // 256 * 256:], ref[:, got.shape[1] // 256 * 256:], TOL)

@@ -48,7 +48,7 @@ static int launch_256_one(const G256Args& f, dim3 grid, hipStream_t s, const cha
     return XQ_OK;
 }
 
-// Block-fp8 launches on large unsplit tiles run gemm_dtl16_kernel (dense) and gemm_bank_kernel (1, the default) or gemm_256_kernel (0): a
+// Block-fp8 launches on large unsplit tiles run gemm_dtl16_kernel (dense) and gemm_bank_kernel (expert banks, some dense ones; 1, the default) or gemm_256_kernel (0): a
 // process-wide switch for tests and A/B measurements, XQ_FP8_DIRECT in the environment sets it at load time.
 static std::atomic<int> g_fp8_direct{[] { const char* e = getenv("XQ_FP8_DIRECT"); return e ? atoi(e) : 1; }()};
 
@@ -177,6 +177,22 @@ static DensePlan plan_dense(int64_t n_rows, int64_t Nout, int64_t nk) {
         else { p.tail_T = 128; p.tail_split = 1; }
     }
     return p;
+}
+
+// Whether a dense block-fp8 product that would run as planned above takes gemm_bank_kernel's 128 x 256 tiles instead, two on a compute
+// unit: where the last round of 256 x 256 tiles would fill up to half of the chip, or leave a launch of 128 x 128 tiles.  Its blocks are
+// then at most one more on each unit, which runs alone there and half as long again as beside another; past half they are two and
+// a whole round.  150 random products of 400 .. 6000 rows, its time over the plan's: whole launches on 256 x 256 tiles whose last round
+// is filled to 0.3 .. 0.5 0.80 to 0.93 ([12288, 4096], 2048 rows 204 -> 172 us); to 0.53 1.00 to 1.09, to 0.6 .. 0.9 1.00 to 1.08.  Two
+// launches, the second of 128 x 128 tiles: 0.77 to 0.99, 0.86 in the mean ([7552, 512], 2595 rows 43.9 -> 33.9 us).  Where K splits take the
+// last round (0.90 to 1.07), or gemm_mid_kernel the product (0.86 to 1.14), neither is the better.
+// (Contractions of 256 and less keep the two launches, though they take 0.79 to 0.97 here too: what tests that form.)
+static bool half_tiles(const DensePlan& p, int64_t n_rows, int64_t Nout, int64_t Kc) {
+    using D = GeoBank<XQ_FMT_FP8>;
+    if (p.T != 256 || p.split != 1 || Kc <= 256) return false;
+    if (p.head_rows < n_rows) return p.tail_T == 128;
+    const int64_t blocks = xq_cdiv(n_rows, D::ROWS) * xq_cdiv(Nout, D::COLS), slots = 2ll * num_cus();
+    return blocks > slots && blocks % slots != 0 && blocks % slots <= slots / 2;
 }
 
 // ---- dense weights decoded once per launch (xq_gemm_dec.h).  The image costs a pass over the weight (50 M weights: 26-33 us)
@@ -401,6 +417,10 @@ extern "C" int xq_dense_route(int format, int forward, int64_t rows, int64_t n_o
         return XQ_ROUTE_IMAGE;
     }
     const DensePlan p = plan_dense(rows, n_out, k / BK);
+    if (format == XQ_FMT_FP8 && half_tiles(p, rows, n_out, k)) {
+        put(0, GeoBank<XQ_FMT_FP8>::ROWS, GeoBank<XQ_FMT_FP8>::COLS, 1);
+        return XQ_ROUTE_TILES;
+    }
     put(0, p.T, p.T, p.split);
     if (p.head_rows < rows) put(1, p.tail_T, p.tail_T, p.tail_split);
     return XQ_ROUTE_TILES;
@@ -672,6 +692,27 @@ static int launch_tile_gemm_t(const xq_weight* w, bool contract_cols, const bf16
             f.bias = bias;
             f.wide_rows = xq_aligned(C, 16) && ldc % 8 == 0 && xq_aligned(bias, 8);
             return launch_decoded(f, contract_cols, w->format, (uint8_t*)partial, stream, who);
+        }
+        // (32-bit offsets from a base for the operands; whole 16-byte pieces of an output row)
+        const bool bank_storage = w->format == XQ_FMT_FP8 && g_fp8_direct && planned && n_rows * lda * 2 < (1ll << 32) - 4096 &&
+                                  (int64_t)g.wrows * g.wcols < (1ll << 32) - 4096 && g.wcols % 16 == 0 && xq_aligned(C, 16) && ldc % 8 == 0 && xq_aligned(bias, 8);
+        if (bank_storage && half_tiles(plan, n_rows, g.Nout, g.Kc)) {
+            using D = GeoBank<XQ_FMT_FP8>;
+            G256Args f{};
+            f.A = A; f.lda = lda; f.C = C; f.ldc = ldc;
+            f.W = g.packed; f.scales = g.scales;
+            f.wrows = g.wrows; f.wcols = g.wcols; f.scale_dtype = g.scale_dtype;
+            f.Kc = g.Kc; f.Nout = g.Nout; f.M = n_rows; f.num_experts = 1;
+            f.su = g.r_pad ? su : nullptr; f.right = g.right; f.r_pad = g.r_pad; f.ld_su = g.r_pad;
+            f.bias = bias;
+            f.tiles_m = (int32_t)xq_cdiv(n_rows, D::ROWS); f.tiles_n = (int32_t)xq_cdiv(g.Nout, D::COLS);
+            f.ksplit = 1; f.wide_rows = 1;
+            const bool timed = xq_profile_mark_begin(stream, 2.0 * (double)n_rows * g.Nout * ((double)g.Kc + g.r_pad));
+            const int rc = launch_bank(f, w->format, contract_cols, stream, who);
+            if (rc) return rc;
+            XQ_CHECK_LAUNCH(who);
+            if (timed) xq_profile_mark_end(stream);
+            return XQ_OK;
         }
         if (planned && plan.head_rows < n_rows) {
             const int64_t head = plan.head_rows;

@@ -1,10 +1,11 @@
-// Fused dequant-GEMM over expert banks of block-fp8 and nvfp4 (e4m3 scales of 16 rows): tiles of 128 routed rows x 256 columns, four waves side by side (a wave 128 x
+// Fused dequant-GEMM over expert banks of block-fp8 and nvfp4 (e4m3 scales of 16 rows), and over dense block-fp8 weights: tiles of 128 routed rows x 256 columns, four waves side by side (a wave 128 x
 // 64), two blocks on a compute unit.
 //
 //   C[rows, Nout] = A[rows, Kc] . Wop[e] (+ su[rows, r] . Lr[e][Nout, r]^T)
 //     !CC (a bank's forward): Wop[kc][n] = W[e][kc][n]; optionally two banks side by side (G256Args: W2, ncols1)
 //      CC (a bank's dgrad):   Wop[kc][n] = W[e][n][kc]; optionally one sum over two banks (K-steps from nk1 on read the second;
 //                             nvfp4: the two products side by side)
+//     DENSE (block-fp8): one weight, all rows; CC its forward [Nout, Kc], !CC its dgrad; the right-hand factor as it is, and a bias
 //
 // Decode and order of sums are gemm_dtl16_kernel's for block-fp8 (xq_gemm_dtl.h), and so are the fragments: one 16-byte piece of a
 // weight row, or two transposing byte reads, is a lane's operand of both k32 steps of a K-step.  nvfp4 bytes hold rows 2 p and 2 p + 1
@@ -18,6 +19,8 @@
 // 2555 us with 256 x 256 tiles, one block a unit (12 of 30 us of a tile of 12 K-steps outside the loop: nothing overlaps them there),
 // 2420 as 128 x 256 tiles, 2250 as it stands (0.83-1.07 -> 0.97-1.2 PFLOP/s).  nvfp4, forward and backward of such an MLP, against decoded
 // tiles in LDS (gemm_256_kernel): 4400 -> 3680 us, 32768 rows 1581 -> 1122, 16384 rows 1032 -> 755.
+// Dense block-fp8 MLP 4096/12288 of 2048 rows (1.5 rounds of 256 x 256 tiles), forward and backward: 1295 -> 1194 us, the forward 638 -> 571; a
+// whole number of rounds is level (4096 rows 2207, 2209), so the choice between the two is half_tiles' (xq_gemm.hip).
 //  * Two blocks on a compute unit, 80 KB of LDS each: one's start and end (7 of 26 us) run beside the other's products.  Blocks that
 //    carry several tiles, the next one's first loads requested before the last one's end, stayed in step with each other: 6 % slower.
 //  * Stages: three of activations, shared by the four waves, two of weights (nvfp4: three, with their scales), each wave's 64 columns its
@@ -90,7 +93,7 @@ __device__ __forceinline__ void bank_pair_unit(uint32_t codes, uint32_t scales, 
     odd[W] = pack_bf16x2(a[1] * s0, b[1] * s1);
 }
 
-template <int FMT, bool CC>
+template <int FMT, bool CC, bool DENSE = false>
 __global__ void __launch_bounds__(256, 2) gemm_bank_kernel(G256Args g) {
     using D = GeoBank<FMT>;
     constexpr bool F4 = D::F4;
@@ -101,7 +104,14 @@ __global__ void __launch_bounds__(256, 2) gemm_bank_kernel(G256Args g) {
 
     // ---- the tile and its expert: every wave counts the experts whose tiles end at or before this one
     int pid_m, pid_n, e = 0;
-    {
+    if constexpr (DENSE) {
+        const int nb = g.tiles_m * g.tiles_n, b = blockIdx.x, per = nb >> 3;
+        const int logical = (b < per * 8) ? (b & 7) * per + (b >> 3) : b;
+        constexpr int GM = 8;                                                 // row tiles beside each other: they share weight tiles
+        const int width = GM * g.tiles_n, grp = logical / width, first_m = grp * GM, gsz = min(g.tiles_m - first_m, GM), in = logical - grp * width;
+        pid_m = __builtin_amdgcn_readfirstlane(first_m + in % gsz);
+        pid_n = __builtin_amdgcn_readfirstlane(in / gsz);
+    } else {
         int pv[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) pv[i] = g.tile_prefix[min(i * 64 + lane + 1, g.num_experts)];
@@ -119,7 +129,8 @@ __global__ void __launch_bounds__(256, 2) gemm_bank_kernel(G256Args g) {
         }
         e = __builtin_amdgcn_readfirstlane(e);
     }
-    const int row0 = __builtin_amdgcn_readfirstlane(g.offsets[e] + (pid_m - g.tile_prefix[e]) * D::ROWS), row_end = __builtin_amdgcn_readfirstlane(g.offsets[e + 1]);
+    const int row0 = DENSE ? pid_m * D::ROWS : __builtin_amdgcn_readfirstlane(g.offsets[e] + (pid_m - g.tile_prefix[e]) * D::ROWS);
+    const int row_end = DENSE ? (int)g.M : __builtin_amdgcn_readfirstlane(g.offsets[e + 1]);
     const int n0 = pid_n * D::COLS;
     int n0w = n0, bank_width = g.Nout;
     const uint8_t* Wb = g.W + (int64_t)e * g.packed_stride;
@@ -129,7 +140,7 @@ __global__ void __launch_bounds__(256, 2) gemm_bank_kernel(G256Args g) {
     float gs = F4 ? g.global_scale[e] : 1.0f;
     const bf16_t* su_b = g.su;
     const bf16_t* lr_b = g.lora_right;
-    if constexpr (!CC || F4) {
+    if constexpr (!DENSE && (!CC || F4)) {
         if (g.W2 != nullptr) {
             bank_width = g.ncols1;
             if (n0 >= g.ncols1) {
@@ -168,8 +179,8 @@ __global__ void __launch_bounds__(256, 2) gemm_bank_kernel(G256Args g) {
     if (F4 && CC) s_off = (uint32_t)(min((n0w + wn * 64) / 16 + lg, g.wrows / 16 - 1) * (int64_t)g.wcols + l16 * 4);
     if (F4 && !CC) s_off = (uint32_t)((int64_t)lg * g.wcols + min(n0w + wn * 64 + l16 * 4, g.wcols - 4));
     const int64_t w_kstep = CC ? D::BK : (int64_t)(D::BK / (F4 ? 2 : 1)) * g.wcols, s_kstep = CC ? D::BK : 4 * (int64_t)g.wcols;
-    const int nk1 = (!F4 && CC && g.W2 != nullptr) ? g.nk1 : (1 << 30);
-    const int64_t w_jump = (!F4 && CC && g.W2 != nullptr) ? (g.W2 - g.W) - (int64_t)(nk1 - 1) * w_kstep : 0;      // to the second bank's first K-step
+    const int nk1 = (!DENSE && !F4 && CC && g.W2 != nullptr) ? g.nk1 : (1 << 30);
+    const int64_t w_jump = (!DENSE && !F4 && CC && g.W2 != nullptr) ? (g.W2 - g.W) - (int64_t)(nk1 - 1) * w_kstep : 0;      // to the second bank's first K-step
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)dsm;
     const uint32_t lds_w = lds0 + D::NA * D::A_BYTES + wn * (D::W_BYTES / 4);        // this wave's columns of weight stage 0
     // (M0, the LDS base of the loads, is written here and used nowhere else in the kernel: once for a run of parts, whose places in
@@ -192,7 +203,7 @@ __global__ void __launch_bounds__(256, 2) gemm_bank_kernel(G256Args g) {
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
         rows_src[p] = min(row0 + (wn * 4 + p) * 8 + (lane >> 3), row_end - 1);
-        if (g.a_rows) rows_src[p] = g.a_rows[rows_src[p]];
+        if (!DENSE && g.a_rows) rows_src[p] = g.a_rows[rows_src[p]];
     }
     // block scales of this wave's columns: 128-k block kb in lane kb % 64, 64 blocks at a time
     const int sn = n0w + (wn >> 1) * 128;
@@ -319,19 +330,24 @@ __global__ void __launch_bounds__(256, 2) gemm_bank_kernel(G256Args g) {
     const int rp = g.r_pad;
     // (without a side term they are read from places that exist, and not used; whole tiles need no look at the rows' end)
     const unsigned char* su_t = (const unsigned char*)(rp > 0 ? su_b + (int64_t)row0 * g.ld_su : g.A);
-    const unsigned char* lr_t = rp > 0 ? (const unsigned char*)(lr_b + (int64_t)e * bank_width * rp) : g.W;
+    const unsigned char* lr_t = !DENSE && rp > 0 ? (const unsigned char*)(lr_b + (int64_t)e * bank_width * rp) : g.W;
     auto side_chunk = [&](int ks) { return max(min(ks * 4 + tg, (rp >> 3) - 1), 0) * 8; };
     auto side_x = [&](int i, int ks) {
         const int r = SKIP ? min(i * 16 + t16, row_end - 1 - row0) : i * 16 + t16;
         return *(const bf16x8*)(su_t + (uint32_t)((r * (int)g.ld_su + side_chunk(ks)) * 2));
     };
+    // (dense: the factor as it is, converted here, behind the main loop, while the other block of the compute unit runs.  One factor:
+    // its chunks that hold no rank at all are not looked at)
+    const int ranks = DENSE && g.right.f[1] == nullptr ? min(rp, (g.right.r + 7) & ~7) : rp;
     auto side_w = [&](int j, int ks) {
+        if constexpr (DENSE)
+            return __builtin_bit_cast(bf16x8, right_chunk(g.right, -1, min(n0w + wn * 64 + j * 16 + t16, g.Nout - 1), min(ks * 4 + tg, (ranks >> 3) - 1)));
         const int n = min(n0w + wn * 64 + (F4 && CC ? (j >> 1) * 32 + 2 * t16 + (j & 1) : j * 16 + t16), bank_width - 1);
         return *(const bf16x8*)(lr_t + (uint32_t)((n * rp + side_chunk(ks)) * 2));
     };
     auto in_rank = [&](const bf16x8& v, int ks) {        // lanes of ranks beyond rp get zeros
         const u32x4 z = {0, 0, 0, 0};
-        return __builtin_bit_cast(bf16x8, (ks * 4 + tg) * 8 < rp ? __builtin_bit_cast(u32x4, v) : z);
+        return __builtin_bit_cast(bf16x8, (ks * 4 + tg) * 8 < ranks ? __builtin_bit_cast(u32x4, v) : z);
     };
 
     int sa = 0;                   // the activation stage of this K-step
@@ -428,7 +444,7 @@ __global__ void __launch_bounds__(256, 2) gemm_bank_kernel(G256Args g) {
                 if constexpr (c == 14) { next_w(kt + 3); begin_w((kt + 1) & 1); }
                 XQ_BANK_ISSUE(w_off, w_base, c - 14);
             }
-            if constexpr (!MORE && c == 12)
+            if constexpr (!DENSE && !MORE && c == 12)
 #pragma unroll
                 for (int j = 0; j < TN; ++j) sw[j] = side_w(j, 0);
             if constexpr (!MORE && c >= 12) {
@@ -459,12 +475,24 @@ __global__ void __launch_bounds__(256, 2) gemm_bank_kernel(G256Args g) {
     }
 
     for (int ks = 0; ks * 32 < rp; ++ks) {
-        if (ks > 0) {
-#pragma unroll
-            for (int j = 0; j < TN; ++j) sw[j] = side_w(j, ks);
+        if (ks > 0)
 #pragma unroll
             for (int i = 0; i < TM; ++i) sx[i] = side_x(i, ks);
+        if constexpr (DENSE) {
+#pragma unroll
+            for (int i = 0; i < TM; ++i) sx[i] = in_rank(sx[i], ks);
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {                             // one at a time, for the registers
+                const bf16x8 w = in_rank(side_w(j, ks), ks);
+#pragma unroll
+                for (int i = 0; i < TM; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, sx[i], acc[i][j], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            continue;
         }
+        if (ks > 0)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) sw[j] = side_w(j, ks);
 #pragma unroll
         for (int j = 0; j < TN; ++j) sw[j] = in_rank(sw[j], ks);
 #pragma unroll
@@ -472,6 +500,16 @@ __global__ void __launch_bounds__(256, 2) gemm_bank_kernel(G256Args g) {
             const bf16x8 ax = in_rank(sx[i], ks);
 #pragma unroll
             for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(sw[j], ax, acc[i][j], 0, 0, 0);
+        }
+    }
+
+    if (DENSE && g.bias) {
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            const u32x2 b = *(const u32x2*)(g.bias + min(n0 + wn * 64 + j * 16 + 4 * tg, g.Nout - 4));
+            const f32x4 b4 = {__uint_as_float(b[0] << 16), __uint_as_float(b[0] & 0xffff0000u), __uint_as_float(b[1] << 16), __uint_as_float(b[1] & 0xffff0000u)};
+#pragma unroll
+            for (int i = 0; i < TM; ++i) acc[i][j] += b4;
         }
     }
 

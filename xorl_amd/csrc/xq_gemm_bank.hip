@@ -4,25 +4,26 @@
 
 namespace xq {
 
-template <int FMT, bool CC>
+template <int FMT, bool CC, bool DENSE>
 static int launch_bank_one(const G256Args& f, hipStream_t s, const char* who) {
     using D = GeoBank<FMT>;
     static std::atomic<bool> attr_set{false};   // the attribute call is idempotent: a race only repeats it
     if (!attr_set) {
-        const hipError_t e = hipFuncSetAttribute((const void*)gemm_bank_kernel<FMT, CC>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)D::lds_bytes());
+        const hipError_t e = hipFuncSetAttribute((const void*)gemm_bank_kernel<FMT, CC, DENSE>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)D::lds_bytes());
         if (e != hipSuccess) {
             xq_set_error("%s: cannot raise the dynamic LDS limit: %s", who, hipGetErrorString(e));
             return XQ_ERR_LAUNCH;
         }
         attr_set = true;
     }
-    gemm_bank_kernel<FMT, CC><<<dim3((unsigned)(f.tiles_m * f.tiles_n)), D::NT, D::lds_bytes(), s>>>(f);
+    gemm_bank_kernel<FMT, CC, DENSE><<<dim3((unsigned)(f.tiles_m * f.tiles_n)), D::NT, D::lds_bytes(), s>>>(f);
     return XQ_OK;
 }
 
 int launch_bank(const G256Args& f, int fmt, bool cc, hipStream_t s, const char* who) {
-    if (fmt == XQ_FMT_NVFP4) return cc ? launch_bank_one<XQ_FMT_NVFP4, true>(f, s, who) : launch_bank_one<XQ_FMT_NVFP4, false>(f, s, who);
-    return cc ? launch_bank_one<XQ_FMT_FP8, true>(f, s, who) : launch_bank_one<XQ_FMT_FP8, false>(f, s, who);
+    if (!f.offsets) return cc ? launch_bank_one<XQ_FMT_FP8, true, true>(f, s, who) : launch_bank_one<XQ_FMT_FP8, false, true>(f, s, who);
+    if (fmt == XQ_FMT_NVFP4) return cc ? launch_bank_one<XQ_FMT_NVFP4, true, false>(f, s, who) : launch_bank_one<XQ_FMT_NVFP4, false, false>(f, s, who);
+    return cc ? launch_bank_one<XQ_FMT_FP8, true, false>(f, s, who) : launch_bank_one<XQ_FMT_FP8, false, false>(f, s, who);
 }
 
 }  // namespace xq

@@ -227,3 +227,27 @@ def test_mlp_backward_rejects_a_saved_state_without_its_form(hip_device):
     y, saved = F._mlp_fwd_impl(x, factors, (None, None, None), banks, r, 2.0, 0)
     with pytest.raises(ValueError, match="gate_up_fused"):
         F._mlp_bwd_impl(torch.ones_like(y), x, saved, factors, banks, r, 2.0, True, -1)
+
+
+@pytest.mark.parametrize("M,H,I,r,bias", [
+    (129, 192, 9280, 8, True), (300, 448, 9280, 64, False),       # part of a round of the chip; ragged rows and columns, three and seven K-steps
+    (2309, 256, 7232, 24, False),                                   # more than two rounds
+])
+def test_gate_and_up_share_a_launch(hip_device, M, H, I, r, bias):
+    """Block-fp8 gate and up as one launch of 128 x 256 tiles: against the three modules, whose projections are launches of their own
+    (one rounded output each: a bf16 step of the largest entry), and without a bias against the float64 program."""
+    from xorl_amd.functional import silu_and_mul
+    from xorl_amd.qlora import qlora_mlp_forward
+
+    mods, w_ref = _mods("block_fp8", H, I, r, hip_device, bias=bias, seed=M)
+    x = gen((M, H), 1.0, 91, torch.bfloat16)
+    xd = x.to(hip_device)
+    with torch.no_grad():
+        y = qlora_mlp_forward(mods["gate"], mods["up"], mods["down"], xd)
+        sep = mods["down"](silu_and_mul(mods["gate"](xd), mods["up"](xd)))
+    assert R.max_rel_err(y.float().cpu(), sep.double().cpu()) <= 2 ** -7
+    assert R.max_rel_err(y[M // 128 * 128:].float().cpu(), sep[M // 128 * 128:].double().cpu()) <= 2 ** -7
+    if not bias:
+        loras = {k: (m.lora_A.detach().cpu(), m.lora_B.detach().cpu()) for k, m in mods.items()}
+        ex = R.mlp_fwd_bwd_exact(x, w_ref["gate"], w_ref["up"], w_ref["down"], loras, mods["gate"].scaling, torch.zeros(M, H, dtype=torch.bfloat16))
+        close(y.cpu(), ex["y"], TOL)

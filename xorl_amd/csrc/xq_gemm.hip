@@ -694,7 +694,7 @@ static int launch_tile_gemm_t(const xq_weight* w, bool contract_cols, const bf16
             return launch_decoded(f, contract_cols, w->format, (uint8_t*)partial, stream, who);
         }
         // (32-bit offsets from a base for the operands; whole 16-byte pieces of an output row)
-        const bool bank_storage = w->format == XQ_FMT_FP8 && g_fp8_direct && planned && n_rows * lda * 2 < (1ll << 32) - 4096 &&
+        const bool bank_storage = w->format == XQ_FMT_FP8 && g_fp8_direct && planned && g.right.f[1] == nullptr && n_rows * lda * 2 < (1ll << 32) - 4096 &&
                                   (int64_t)g.wrows * g.wcols < (1ll << 32) - 4096 && g.wcols % 16 == 0 && xq_aligned(C, 16) && ldc % 8 == 0 && xq_aligned(bias, 8);
         if (bank_storage && half_tiles(plan, n_rows, g.Nout, g.Kc)) {
             using D = GeoBank<XQ_FMT_FP8>;
@@ -850,6 +850,53 @@ int launch_gate_up_swiglu(const xq_weight* wg, const xq_weight* wu, const bf16_t
     const bool timed = xq_profile_mark_begin(stream, 2.0 * (double)M * (2.0 * I) * ((double)K + f.r_pad));
     gemm_256_kernel<XQ_FMT_FP8, true, false, 256, false, true>
         <<<dim3(persistent_grid((int64_t)f.tiles_m * f.tiles_n)), Geo<256>::NT, Geo<256>::lds_bytes(true), stream>>>(f);
+    XQ_CHECK_LAUNCH(who);
+    if (timed) xq_profile_mark_end(stream);
+    return XQ_OK;
+}
+
+// Whether gate and up of a block-fp8 MLP run as one launch of gemm_bank_kernel.  Each alone fills part of a round of the chip up to some
+// thousand rows; the blocks of both share one (two of them on a compute unit), and K splits are not needed.  Blocks of both, in rounds
+// of two on every unit, and the time of a forward's three products over that of three launches, 80 random MLPs of 70 .. 5300 rows: 0.06 .. 0.2 0.84 to
+// 1.28 (deep ones were in K splits), 0.28 .. 0.5 0.81 to 0.96, 0.53 .. 0.6 (a second block on some units, alone on the others) 1.00 to 1.05,
+// 0.63 .. 0.75 0.91 to 0.97, 0.9 .. 1.5 0.88 to 0.93, 1.53 1.04, 1.7 .. 1.9 0.99 to 1.00, from two rounds on 0.88 to 0.99.
+// (us at 4096/12288: 256 rows 131 -> 108, 768 rows 284 -> 249, 1024 rows 311 -> 282, 1536 rows 471 -> 413, 3072 rows 879 -> 784.)
+bool gate_up_side_by_side(const xq_weight* wg, const xq_weight* wu, const bf16_t* x, int64_t ldx, int64_t M, const bf16_t* bias_g,
+                          const bf16_t* bias_u, const bf16_t* gu, int64_t ldgu) {
+    using D = GeoBank<XQ_FMT_FP8>;
+    const int64_t I = wg->rows, K = wg->cols;
+    if (!g_fp8_direct || g_tile_policy != 0 || wg->format != XQ_FMT_FP8 || wu->format != XQ_FMT_FP8 || wu->rows != I || wu->cols != K ||
+        wg->scale_dtype != XQ_SCALE_F32 || wu->scale_dtype != XQ_SCALE_F32 || I % 16 != 0 || K % D::BK != 0 || K < 3 * D::BK || M <= 64 || ldx % 8 != 0 || !xq_aligned(x, 16) || ldgu % 8 != 0 ||
+        !xq_aligned(gu, 16) || !xq_aligned(wg->packed, 16) || !xq_aligned(wu->packed, 16) || !xq_aligned(bias_g, 8) || !xq_aligned(bias_u, 8) ||
+        // (32-bit offsets from a base for the operands)
+        M * ldx * 2 >= (1ll << 32) - 4096 || I * K >= (1ll << 32) - 4096 || decode_first(XQ_FMT_FP8, M, I, K))
+        return false;
+    const int64_t blocks = 2 * xq_cdiv(M, D::ROWS) * xq_cdiv(I, D::COLS), slots = 2ll * num_cus();
+    const double rounds = (double)blocks / (double)slots, part = rounds - (double)(blocks / slots);
+    return rounds >= 2.0 || (rounds >= 0.28 && !(part > 0.5 && part < 0.63));
+}
+
+// gu[M, 2I] = (x . deq(Wg)^T + side term | x . deq(Wu)^T + side term), gate_up_side_by_side() being true
+int launch_gate_up(const xq_weight* wg, const xq_weight* wu, const bf16_t* x, int64_t ldx, int64_t M, const bf16_t* su_g, const bf16_t* su_u,
+                   int64_t ld_su, const LowRankRight& right, int r_pad, const bf16_t* bias_g, const bf16_t* bias_u, bf16_t* gu, int64_t ldgu,
+                   hipStream_t stream, const char* who) {
+    using D = GeoBank<XQ_FMT_FP8>;
+    G256Args f[2] = {};
+    const xq_weight* w[2] = {wg, wu};
+    for (int i = 0; i < 2; ++i) {
+        G256Args& q = f[i];
+        q.A = x; q.lda = ldx; q.C = gu + i * w[i]->rows; q.ldc = ldgu;
+        q.W = (const uint8_t*)w[i]->packed; q.scales = (const uint8_t*)w[i]->scales;
+        q.wrows = (int32_t)w[i]->rows; q.wcols = (int32_t)w[i]->cols; q.scale_dtype = w[i]->scale_dtype;
+        q.Kc = q.wcols; q.Nout = q.wrows; q.M = M; q.num_experts = 1;
+        q.su = r_pad ? (i ? su_u : su_g) : nullptr; q.right = right; q.right.f[0] = right.f[i]; q.right.f[1] = nullptr; q.r_pad = r_pad; q.ld_su = ld_su;
+        q.bias = i ? bias_u : bias_g;
+        q.tiles_m = (int32_t)xq_cdiv(M, D::ROWS); q.tiles_n = (int32_t)xq_cdiv(q.Nout, D::COLS);
+        q.ksplit = 1; q.wide_rows = 1;
+    }
+    const bool timed = xq_profile_mark_begin(stream, 2.0 * (double)M * (2.0 * wg->rows) * ((double)wg->cols + r_pad));
+    const int rc = launch_bank_pair(f, true, stream, who);
+    if (rc) return rc;
     XQ_CHECK_LAUNCH(who);
     if (timed) xq_profile_mark_end(stream);
     return XQ_OK;

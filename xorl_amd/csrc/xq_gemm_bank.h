@@ -5,7 +5,8 @@
 //     !CC (a bank's forward): Wop[kc][n] = W[e][kc][n]; optionally two banks side by side (G256Args: W2, ncols1)
 //      CC (a bank's dgrad):   Wop[kc][n] = W[e][n][kc]; optionally one sum over two banks (K-steps from nk1 on read the second;
 //                             nvfp4: the two products side by side)
-//     DENSE (block-fp8): one weight, all rows; CC its forward [Nout, Kc], !CC its dgrad; the right-hand factor as it is, and a bias
+//     DENSE (block-fp8): one weight, all rows, or two of one shape on one input; CC forward [Nout, Kc], !CC dgrad; the right-hand factor as it
+//                             is, and a bias
 //
 // Decode and order of sums are gemm_dtl16_kernel's for block-fp8 (xq_gemm_dtl.h), and so are the fragments: one 16-byte piece of a
 // weight row, or two transposing byte reads, is a lane's operand of both k32 steps of a K-step.  nvfp4 bytes hold rows 2 p and 2 p + 1
@@ -93,8 +94,16 @@ __device__ __forceinline__ void bank_pair_unit(uint32_t codes, uint32_t scales, 
     odd[W] = pack_bf16x2(a[1] * s0, b[1] * s1);
 }
 
+// dense launches take one product, or two of one shape on one input (gridDim.y)
+struct BankPair {
+    G256Args of[2];
+};
+__device__ __forceinline__ const G256Args& bank_args(const G256Args& a) { return a; }
+__device__ __forceinline__ const G256Args& bank_args(const BankPair& a) { return a.of[blockIdx.y]; }
+
 template <int FMT, bool CC, bool DENSE = false>
-__global__ void __launch_bounds__(256, 2) gemm_bank_kernel(G256Args g) {
+__global__ void __launch_bounds__(256, 2) gemm_bank_kernel(std::conditional_t<DENSE, BankPair, G256Args> args) {
+    const G256Args& g = bank_args(args);
     using D = GeoBank<FMT>;
     constexpr bool F4 = D::F4;
     constexpr int TM = 8, TN = 4, NC = 16;
@@ -194,7 +203,7 @@ __global__ void __launch_bounds__(256, 2) gemm_bank_kernel(G256Args g) {
     auto begin_w = [&](int stage) { asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" :: "s"(lds_w + stage * D::W_BYTES)); };
 #define XQ_BANK_ISSUE(off, base, p) asm volatile("global_load_lds_dwordx4 %0, %1 offset:%2" :: "v"(off[p]), "s"(base), "n"((p) * 1024) : "memory")
     auto next_a = [&]() { a_base += D::BK * 2; };
-    auto next_w = [&](int kt) { w_base += !F4 && CC && kt == nk1 ? w_jump : w_kstep; };       // to K-step kt
+    auto next_w = [&](int kt) { w_base += !DENSE && !F4 && CC && kt == nk1 ? w_jump : w_kstep; };       // to K-step kt
     auto issue_s = [&](int stage) {                                    // four bytes a lane; then to the next K-step's
         asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" :: "s"(lds_s + stage * D::S_BYTES), "v"(s_off), "s"(s_base) : "memory");
         s_base += s_kstep;
@@ -210,7 +219,7 @@ __global__ void __launch_bounds__(256, 2) gemm_bank_kernel(G256Args g) {
     // (load and wait written out: a load that the compiler knows of would have it wait for every load in flight where the scale is used)
     auto load_scales = [&](int kb0) {
         const int kb = min(kb0 + lane, (nk - 1) >> 1);
-        const bool second = 2 * kb >= nk1;                      // (nk1 is even: the matrices change on a scale-block boundary)
+        const bool second = !DENSE && 2 * kb >= nk1;                      // (nk1 is even: the matrices change on a scale-block boundary)
         const float* sp = (const float*)(second ? Sb2 : Sb);
         const int kb1 = second ? kb - (nk1 >> 1) : kb;
         const float* at = CC ? sp + (min(sn, g.wrows - 1) >> 7) * scols + kb1 : sp + (int64_t)kb1 * scols + (min(sn, g.wcols - 1) >> 7);
@@ -336,12 +345,12 @@ __global__ void __launch_bounds__(256, 2) gemm_bank_kernel(G256Args g) {
         const int r = SKIP ? min(i * 16 + t16, row_end - 1 - row0) : i * 16 + t16;
         return *(const bf16x8*)(su_t + (uint32_t)((r * (int)g.ld_su + side_chunk(ks)) * 2));
     };
-    // (dense: the factor as it is, converted here, behind the main loop, while the other block of the compute unit runs.  One factor:
-    // its chunks that hold no rank at all are not looked at)
-    const int ranks = DENSE && g.right.f[1] == nullptr ? min(rp, (g.right.r + 7) & ~7) : rp;
+    // (dense: the factor as it is, converted here, behind the main loop, while the other block of the compute unit runs; chunks that hold
+    // no rank at all are not looked at)
+    const int ranks = DENSE ? min(rp, (g.right.r + 7) & ~7) : rp;
     auto side_w = [&](int j, int ks) {
         if constexpr (DENSE)
-            return __builtin_bit_cast(bf16x8, right_chunk(g.right, -1, min(n0w + wn * 64 + j * 16 + t16, g.Nout - 1), min(ks * 4 + tg, (ranks >> 3) - 1)));
+            return __builtin_bit_cast(bf16x8, right_chunk(g.right, 0, min(n0w + wn * 64 + j * 16 + t16, g.Nout - 1), min(ks * 4 + tg, (ranks >> 3) - 1)));
         const int n = min(n0w + wn * 64 + (F4 && CC ? (j >> 1) * 32 + 2 * t16 + (j & 1) : j * 16 + t16), bank_width - 1);
         return *(const bf16x8*)(lr_t + (uint32_t)((n * rp + side_chunk(ks)) * 2));
     };
@@ -544,5 +553,6 @@ __global__ void __launch_bounds__(256, 2) gemm_bank_kernel(G256Args g) {
 }
 
 int launch_bank(const G256Args& f, int fmt, bool cc, hipStream_t s, const char* who);
+int launch_bank_pair(const G256Args (&f)[2], bool cc, hipStream_t s, const char* who);      // dense block-fp8: two products of one shape
 
 }  // namespace xq

@@ -4,7 +4,8 @@
 // ops/fused_silu_and_mul.py:22-60) and its backward, composed from this library's kernels on the caller's stream
 // so that work the three separate module calls repeat is shared:
 //   forward   one pass over x gives both low-rank intermediates; block-fp8 gate / up run as one launch whose
-//             epilogue also writes h = bf16(silu(gate)) * up;
+//             epilogue also writes h = bf16(silu(gate)) * up, or as one launch of plain tiles where that fills the chip better
+//             than two;
 //   backward  the dgrads of gate and up are one launch, dX = [dgate | dup] . [Wg ; Wu] + [v_g | v_u] . [A_g ; A_u],
 //             and the two A gradients come from one pass over x.
 // Other formats (and shapes the fused forms do not take) run the same program launch by launch.
@@ -216,9 +217,14 @@ extern "C" int xq_mlp_fwd(const xq_weight* gate, const xq_weight* up, const xq_w
                                         LowRankRight{{lora->B[0], lora->B[1]}, r, r, rp, f32, 0}, rp, bias_g, bias_u, gu, 2 * I, h, I, stream)))
             return rc;
     } else {
-        if ((rc = launch_tile_gemm(gate, true, x, ldx, M, nullptr, nullptr, rp ? su_gu : nullptr, nullptr, rp, bias_g, gu, 2 * I, stream, who, part, part_bytes, nullptr, rp ? &right_g : nullptr))) return rc;
-        if ((rc = launch_tile_gemm(up, true, x, ldx, M, nullptr, nullptr, rp ? su_gu + sl.up_offset : nullptr, nullptr, rp, bias_u, gu + I, 2 * I, stream, who, part, part_bytes, nullptr,
-                                   rp ? &right_u : nullptr))) return rc;
+        if (gate_up_side_by_side(gate, up, x, ldx, M, bias_g, bias_u, gu, 2 * I)) {
+            if ((rc = launch_gate_up(gate, up, x, ldx, M, su_gu, rp ? su_gu + sl.up_offset : nullptr, sl.pitch, LowRankRight{{lora->B[0], lora->B[1]}, r, r, rp, f32, 0}, rp,
+                                     bias_g, bias_u, gu, 2 * I, stream, who))) return rc;
+        } else {
+            if ((rc = launch_tile_gemm(gate, true, x, ldx, M, nullptr, nullptr, rp ? su_gu : nullptr, nullptr, rp, bias_g, gu, 2 * I, stream, who, part, part_bytes, nullptr, rp ? &right_g : nullptr))) return rc;
+            if ((rc = launch_tile_gemm(up, true, x, ldx, M, nullptr, nullptr, rp ? su_gu + sl.up_offset : nullptr, nullptr, rp, bias_u, gu + I, 2 * I, stream, who, part, part_bytes, nullptr,
+                                       rp ? &right_u : nullptr))) return rc;
+        }
         if (many) {
             if ((rc = launch_silu_fwd_nt(gu, gu + I, 2 * I, h, I, M, I, A_d, rp, s, su_d, rp, stream))) return rc;
         } else if ((rc = xq_silu_mul_fwd(gu, gu + I, 2 * I, nullptr, h, I, M, I, stream))) {

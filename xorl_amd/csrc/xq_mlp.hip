@@ -217,7 +217,7 @@ extern "C" int xq_mlp_fwd(const xq_weight* gate, const xq_weight* up, const xq_w
                                         LowRankRight{{lora->B[0], lora->B[1]}, r, r, rp, f32, 0}, rp, bias_g, bias_u, gu, 2 * I, h, I, stream)))
             return rc;
     } else {
-        if (gate_up_side_by_side(gate, up, x, ldx, M, bias_g, bias_u, gu, 2 * I)) {
+        if (xq_aligned(su_gu, 16) && gate_up_side_by_side(gate, up, x, ldx, M, bias_g, bias_u, gu, 2 * I)) {      // (what it does not take, two launches take or refuse)
             if ((rc = launch_gate_up(gate, up, x, ldx, M, su_gu, rp ? su_gu + sl.up_offset : nullptr, sl.pitch, LowRankRight{{lora->B[0], lora->B[1]}, r, r, rp, f32, 0}, rp,
                                      bias_g, bias_u, gu, 2 * I, stream, who))) return rc;
         } else {

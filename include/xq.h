@@ -151,6 +151,10 @@ int xq_set_fp8_direct_tiles(int enabled);
 int xq_set_mlp_gate_up_fused(int enabled);
 int xq_get_mlp_gate_up_fused(void);   /* the current default: 0 or 1 */
 
+/* Whether the two launches of that switch's 0 are one for M rows (both products of a tile program that both would run by
+ * themselves, so the bits are the same), for tests.  No counterpart in the reference. */
+int xq_mlp_gate_up_joint(const xq_weight* gate, const xq_weight* up, int64_t M);
+
 /* xq_linear_fwd with M <= 16 rows runs as ONE launch where the shape and the LoRA operands allow it (FLAT weight,
  * K % 512 == 0 for block_fp8 / K % 1024 == 0 for the 4-bit formats, K <= 12288; fp32 factors with r <= 16, r % 4 == 0,
  * 16-byte aligned): whole weight rows per block, the low-rank intermediate formed once per launch and passed between

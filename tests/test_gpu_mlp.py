@@ -6,7 +6,7 @@ import pytest
 import torch
 
 from oracle import recipe as R
-from tests.util_cases import close, gen, make_dense_module
+from tests.util_cases import close, dense_route, gate_up_joint, gen, make_dense_module
 
 pytestmark = pytest.mark.gpu
 TOL = 1e-2
@@ -251,3 +251,61 @@ def test_gate_and_up_share_a_launch(hip_device, M, H, I, r, bias):
         loras = {k: (m.lora_A.detach().cpu(), m.lora_B.detach().cpu()) for k, m in mods.items()}
         ex = R.mlp_fwd_bwd_exact(x, w_ref["gate"], w_ref["up"], w_ref["down"], loras, mods["gate"].scaling, torch.zeros(M, H, dtype=torch.bfloat16))
         close(y.cpu(), ex["y"], TOL)
+
+
+def _by_itself(m, x, dy, route):
+    """(y, dx) of a projection on the kernel of `route`: "mid" by size, 256 or 128 forced tiles, or (head, tail rows) on 256 and on 128"""
+    from xorl_amd import _C
+
+    got = []
+    try:
+        for policy in {"mid": (0,), 256: (2,), 128: (3,)}.get(route, (2, 3)):
+            _C.check(_C.lib().xq_set_tile_policy(policy))
+            xd = x.detach().clone().requires_grad_(True)
+            y = m(xd)
+            got.append((y.detach(), torch.autograd.grad(y, xd, dy)[0]))
+    finally:
+        _C.check(_C.lib().xq_set_tile_policy(0))
+    return got[0] if len(got) == 1 else tuple(torch.cat([a[:route[0]], b[route[0]:]]) for a, b in zip(*got))
+
+
+@pytest.mark.parametrize("M,H,I,r,fwd,bwd,joint", [
+    (129, 192, 9280, 8, 128, "mid", False), (300, 448, 9280, 64, "mid", "mid", False),
+    (1500, 384, 13120, 32, (1024, 476), (1024, 476), False),      # whole rounds of large tiles, the other rows on small ones
+    (1000, 320, 9280, 16, 256, 256, True), (2300, 256, 12352, 24, 256, 256, True),
+])
+def test_mlp_products_sum_as_by_themselves(hip_device, M, H, I, r, fwd, bwd, joint):
+    """Gate, up and the dgrad of down, joint launch or not, are the bits of the same products by themselves on the kernels that their sizes
+    choose.  Behind them: an fp32 factor gradient of gate, against float64 sums of the bf16 values that those bits give (fp32 sums
+    of M products err by some sqrt(M) 2^-24; a flipped bf16 rounding in one value of a few hundred is 1e-4)."""
+    from xorl_amd import functional as F
+    from xorl_amd.qlora import qlora_mlp_forward
+
+    for route, forward, n, k in ((fwd, True, I, H), (bwd, False, I, H)):
+        here = dense_route("block_fp8", forward, M, n, k)
+        # (a product by itself whose rows would be two launches, the second of small tiles, is free to be one of half tiles)
+        assert here[0] == "mid" if route == "mid" else here[:3] == ("tiles", 128, 256) if isinstance(route, tuple) else here == ("tiles", route, route, 1, 0, 0, 0)
+    assert gate_up_joint(M, H, I) == joint
+    mods, w_ref = _mods("block_fp8", H, I, r, hip_device, seed=M)
+    x, dy = gen((M, H), 1.0, 95, torch.bfloat16).to(hip_device), gen((M, H), 1.0, 96, torch.bfloat16).to(hip_device)
+    m3 = [mods[k] for k in ("gate", "up", "down")]
+    factors = [t.detach() for m in m3 for t in (m.lora_A, m.lora_B)]
+    _, saved = F._mlp_fwd_impl(x, factors, (None,) * 3, [m._quant_weight() for m in m3], r, m3[0].scaling, 0)
+    zero = torch.zeros(M, I, dtype=torch.bfloat16, device=hip_device)
+    g, u = (_by_itself(m, x, zero, fwd)[0] for m in m3[:2])
+    assert torch.equal(saved[0], torch.cat([g, u], 1))
+    # the backward
+    xd = x.clone().requires_grad_(True)
+    y = qlora_mlp_forward(*m3, xd)
+    dB = torch.autograd.grad(y, m3[0].lora_B, dy)[0]
+    dh = _by_itself(m3[2], saved[1], dy, bwd)[1]
+    g.requires_grad_(True)
+    dg = torch.autograd.grad(F.silu_and_mul(g, u), g, dh)[0]
+    rp = saved[2].shape[1] // 2
+    want = dg.double().t() @ saved[2].flatten()[:M * rp].view(M, rp)[:, :r].double()
+    assert float((dB.double() - want).norm() / want.norm()) <= 2e-5
+    if joint:
+        loras = {k: (m.lora_A.detach().cpu(), m.lora_B.detach().cpu()) for k, m in mods.items()}
+        ex = R.mlp_fwd_bwd_exact(x.cpu(), w_ref["gate"], w_ref["up"], w_ref["down"], loras, m3[0].scaling, dy.cpu())
+        close(y.detach().cpu(), ex["y"], TOL)
+        close(dB.cpu(), ex["dB_gate"], TOL)

@@ -96,6 +96,18 @@ def skinny_route(fmt, N, K, M, ldx, scale_dtype=None, r=0):
     return (_C.lib().xq_skinny_route(ctypes.byref(w), M, ldx, 4096 if r else None, 4096 if r else None, _C.XQ_DT_F32, r, plan), *plan)
 
 
+def gate_up_joint(M, H, I) -> bool:
+    """xq_mlp_gate_up_joint (include/xq.h) of block-fp8 gate and up [I, H]"""
+    import ctypes
+
+    from xorl_amd import _C
+
+    w = _C.XqWeight()
+    w.format, w.layout, w.rows, w.cols, w.num_experts, w.group, w.scale_dtype = _C.FORMATS["block_fp8"], _C.XQ_LAYOUT_FLAT, I, H, 1, 128, _C.XQ_SCALE_F32
+    w.packed = w.scales = 4096                               # (addresses: nothing is read)
+    return bool(_C.lib().xq_mlp_gate_up_joint(ctypes.byref(w), ctypes.byref(w), M))
+
+
 def banks_joint(fmt, E, H, I, n_rows, forward) -> bool:
     """xq_grouped_joint (include/xq.h) of gate and up banks [E, H, I] in a format's usual storage"""
     import ctypes

@@ -186,6 +186,7 @@ _SIGNATURES = {
                                     _P, _I64, _P]),
     "xq_mlp_workspace_bytes": (_I64, [_I64, _I64, _I64, _INT, _INT]),
     "xq_mlp_workspace_bytes_fmt": (_I64, [_INT, _I64, _I64, _I64, _INT, _INT]),
+    "xq_mlp_gate_up_joint": (_INT, [_W, _W, _I64]),
     "xq_mlp_infer_workspace_bytes": (_I64, [_I64, _I64, _I64, _INT]),
     "xq_mlp_infer_workspace_bytes_fmt": (_I64, [_INT, _I64, _I64, _I64, _INT]),
     # gate, up, down, lora, x, ldx, M, y, ldy, ws, ws_bytes, stream

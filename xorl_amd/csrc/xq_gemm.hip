@@ -52,6 +52,8 @@ static int launch_256_one(const G256Args& f, dim3 grid, hipStream_t s, const cha
 // process-wide switch for tests and A/B measurements, XQ_FP8_DIRECT in the environment sets it at load time.
 static std::atomic<int> g_fp8_direct{[] { const char* e = getenv("XQ_FP8_DIRECT"); return e ? atoi(e) : 1; }()};
 
+constexpr int64_t kDtlMaxK = 2ll * GeoDtl::SCL_MAX * GeoDtl::BK;      // the longest contraction that gemm_dtl16_kernel takes
+
 static int launch_dtl16(const G256Args& f, bool cc, dim3 grid, hipStream_t s, const char* who) {
     static std::atomic<bool> attr_set{false};
     if (!attr_set) {
@@ -189,9 +191,12 @@ static DensePlan plan_dense(int64_t n_rows, int64_t Nout, int64_t nk) {
 // launches, the second of 128 x 128 tiles: 0.77 to 0.99, 0.86 in the mean ([7552, 512], 2595 rows 43.9 -> 33.9 us).  Where K splits take the
 // last round (0.90 to 1.07), or gemm_mid_kernel the product (0.86 to 1.14), neither is the better.
 // (Contractions of 256 and less keep the two launches, though they take 0.79 to 0.97 here too: what tests that form.)
-static bool half_tiles(const DensePlan& p, int64_t n_rows, int64_t Nout, int64_t Kc) {
+// The sums are gemm_dtl16_kernel's, whose place these tiles take in a whole launch; rows that would be a launch of 128 x 128 tiles are summed in
+// another order (gemm_256_kernel).
+static bool half_tiles(const DensePlan& p, int64_t n_rows, int64_t Nout, int64_t Kc, SumOrder order) {
     using D = GeoBank<XQ_FMT_FP8>;
     if (p.T != 256 || p.split != 1 || Kc <= 256) return false;
+    if (order == SumOrder::kept && (p.head_rows < n_rows || Kc > kDtlMaxK)) return false;
     if (p.head_rows < n_rows) return p.tail_T == 128;
     const int64_t blocks = xq_cdiv(n_rows, D::ROWS) * xq_cdiv(Nout, D::COLS), slots = 2ll * num_cus();
     return blocks > slots && blocks % slots != 0 && blocks % slots <= slots / 2;
@@ -419,7 +424,7 @@ extern "C" int xq_dense_route(int format, int forward, int64_t rows, int64_t n_o
         return XQ_ROUTE_IMAGE;
     }
     const DensePlan p = plan_dense(rows, n_out, k / BK);
-    if (format == XQ_FMT_FP8 && half_tiles(p, rows, n_out, k)) {
+    if (format == XQ_FMT_FP8 && half_tiles(p, rows, n_out, k, SumOrder::any)) {
         put(0, GeoBank<XQ_FMT_FP8>::ROWS, GeoBank<XQ_FMT_FP8>::COLS, 1);
         return XQ_ROUTE_TILES;
     }
@@ -602,8 +607,8 @@ static int launch_tile_gemm_t(const xq_weight* w, bool contract_cols, const bf16
                               const int32_t* offsets, const int32_t* tile_offsets, const bf16_t* su, const bf16_t* lora_right,
                               int r_pad, const bf16_t* bias, bf16_t* C, int64_t ldc, hipStream_t stream, const char* who,
                               int force_T, int force_split, float* partial, int64_t partial_bytes,
-                              const TwoBanks* two = nullptr, const LowRankRight* right = nullptr, const int32_t* a_rows = nullptr,
-                              int64_t a_span_rows = 0) {
+                              const TwoBanks* two = nullptr, const LowRankRight* right = nullptr,
+                              SumOrder order = SumOrder::any, const int32_t* a_rows = nullptr, int64_t a_span_rows = 0) {
     const int64_t a_rows_span = a_rows ? a_span_rows : n_rows;      // rows of A that the launch may touch (0: not known)
     TileArgs g;
     g.A = A; g.lda = lda; g.C = C; g.ldc = ldc;
@@ -705,7 +710,7 @@ static int launch_tile_gemm_t(const xq_weight* w, bool contract_cols, const bf16
         // (32-bit offsets from a base for the operands; whole 16-byte pieces of an output row)
         const bool bank_storage = w->format == XQ_FMT_FP8 && g_fp8_direct && planned && g.right.f[1] == nullptr && n_rows * lda * 2 < (1ll << 32) - 4096 &&
                                   (int64_t)g.wrows * g.wcols < (1ll << 32) - 4096 && g.wcols % 16 == 0 && xq_aligned(C, 16) && ldc % 8 == 0 && xq_aligned(bias, 8);
-        if (bank_storage && half_tiles(plan, n_rows, g.Nout, g.Kc)) {
+        if (bank_storage && half_tiles(plan, n_rows, g.Nout, g.Kc, order)) {
             using D = GeoBank<XQ_FMT_FP8>;
             G256Args f{};
             f.A = A; f.lda = lda; f.C = C; f.ldc = ldc;
@@ -864,12 +869,11 @@ int launch_gate_up_swiglu(const xq_weight* wg, const xq_weight* wu, const bf16_t
     return XQ_OK;
 }
 
-// Whether gate and up of a block-fp8 MLP run as one launch of gemm_bank_kernel.  Each alone fills part of a round of the chip up to some
-// thousand rows; the blocks of both share one (two of them on a compute unit), and K splits are not needed.  Blocks of both, in rounds
-// of two on every unit, and the time of a forward's three products over that of three launches, 80 random MLPs of 70 .. 5300 rows: 0.06 .. 0.2 0.84 to
-// 1.28 (deep ones were in K splits), 0.28 .. 0.5 0.81 to 0.96, 0.53 .. 0.6 (a second block on some units, alone on the others) 1.00 to 1.05,
-// 0.63 .. 0.75 0.91 to 0.97, 0.9 .. 1.5 0.88 to 0.93, 1.53 1.04, 1.7 .. 1.9 0.99 to 1.00, from two rounds on 0.88 to 0.99.
-// (us at 4096/12288: 256 rows 131 -> 108, 768 rows 284 -> 249, 1024 rows 311 -> 282, 1536 rows 471 -> 413, 3072 rows 879 -> 784.)
+// Whether gate and up of a block-fp8 MLP run as one launch of gemm_bank_kernel: products that gemm_dtl16_kernel would run whole, whose sums are the
+// same there.  (Fewer rows, in gemm_mid_kernel or K splits, would gain as well -- 4096/12288, us of the three products, 256 rows 131 -> 108, 768
+// rows 284 -> 249 -- but 2e-4 to 4e-4 of y and of every gradient with them.)  The blocks of both, two on a compute unit, share the last round.
+// Rounds, and the time of a forward's three products over that of three launches, of random MLPs: 1 .. 1.5 0.88 to 0.93, 1.53 1.04, 1.7 .. 1.9
+// 0.99 to 1.00, from two rounds on 0.88 to 0.99.
 bool gate_up_side_by_side(const xq_weight* wg, const xq_weight* wu, const bf16_t* x, int64_t ldx, int64_t M, const bf16_t* bias_g,
                           const bf16_t* bias_u, const bf16_t* gu, int64_t ldgu) {
     using D = GeoBank<XQ_FMT_FP8>;
@@ -878,11 +882,15 @@ bool gate_up_side_by_side(const xq_weight* wg, const xq_weight* wu, const bf16_t
         wg->scale_dtype != XQ_SCALE_F32 || wu->scale_dtype != XQ_SCALE_F32 || I % 16 != 0 || K % D::BK != 0 || K < 3 * D::BK || M <= 64 || ldx % 8 != 0 || !xq_aligned(x, 16) || ldgu % 8 != 0 ||
         !xq_aligned(gu, 16) || !xq_aligned(wg->packed, 16) || !xq_aligned(wu->packed, 16) || !xq_aligned(bias_g, 8) || !xq_aligned(bias_u, 8) ||
         // (32-bit offsets from a base for the operands)
-        M * ldx * 2 >= (1ll << 32) - 4096 || I * K >= (1ll << 32) - 4096 || decode_first(XQ_FMT_FP8, M, I, K))
+        M * ldx * 2 >= (1ll << 32) - 4096 || I * K >= (1ll << 32) - 4096)
         return false;
+    MidPlan mid;
+    if (K > kDtlMaxK || takes_mid(XQ_FMT_FP8, true, M, I, K, &mid) || decode_first(XQ_FMT_FP8, M, I, K)) return false;
+    const DensePlan p = plan_dense(M, I, K / BK);
+    if (p.T != 256 || p.split != 1 || p.head_rows < M) return false;
     const int64_t blocks = 2 * xq_cdiv(M, D::ROWS) * xq_cdiv(I, D::COLS), slots = 2ll * num_cus();
     const double rounds = (double)blocks / (double)slots, part = rounds - (double)(blocks / slots);
-    return rounds >= 2.0 || (rounds >= 0.28 && !(part > 0.5 && part < 0.63));
+    return rounds >= 2.0 || !(part > 0.5 && part < 0.63);
 }
 
 // gu[M, 2I] = (x . deq(Wg)^T + side term | x . deq(Wu)^T + side term), gate_up_side_by_side() being true
@@ -914,11 +922,11 @@ int launch_gate_up(const xq_weight* wg, const xq_weight* wu, const bf16_t* x, in
 int launch_tile_gemm(const xq_weight* w, bool contract_cols, const bf16_t* A, int64_t lda, int64_t n_rows,
                      const int32_t* offsets, const int32_t* tile_offsets, const bf16_t* su, const bf16_t* lora_right,
                      int r_pad, const bf16_t* bias, bf16_t* C, int64_t ldc, hipStream_t stream, const char* who,
-                     float* partial, int64_t partial_bytes, const TwoBanks* two, const LowRankRight* right, const int32_t* a_rows,
-                     int64_t a_span_rows) {
+                     float* partial, int64_t partial_bytes, const TwoBanks* two, const LowRankRight* right, SumOrder order,
+                     const int32_t* a_rows, int64_t a_span_rows) {
     XQ_REQUIRE(!a_rows || offsets, "%s: a row map goes with a grouped launch", who);
     return launch_tile_gemm_t(w, contract_cols, A, lda, n_rows, offsets, tile_offsets, su, lora_right, r_pad, bias, C, ldc,
-                              stream, who, 0, 1, partial, partial_bytes, two, right, a_rows, a_span_rows);
+                              stream, who, 0, 1, partial, partial_bytes, two, right, order, a_rows, a_span_rows);
 }
 
 // whether a grouped launch over this bank runs on the pipelined tile kernel, which can read its activation rows through

@@ -207,6 +207,11 @@ int launch_gate_up_swiglu(const xq_weight* wg, const xq_weight* wu, const bf16_t
                           const bf16_t* su_g, const bf16_t* su_u, int64_t ld_su, const LowRankRight& right,
                           int r_pad, const bf16_t* bias_g, const bf16_t* bias_u, bf16_t* gu, int64_t ldgu, bf16_t* h,
                           int64_t ldh, hipStream_t stream);
+// What a product's fp32 sums have to equal.  any: this library's kernels are free to sum in the order that suits the sizes.  kept: the order of the
+// kernel that the sizes choose for a product by itself among gemm_256_kernel, gemm_mid_kernel, gemm_dec_kernel and gemm_dtl16_kernel.  A bf16
+// rounding of such a sum that flips with the order moves what is computed from it by some 2e-4 (2-norm), in fp32 results too: that is many times
+// fp32's rounding.  So the products that factor gradients are computed from, or that one program runs in more than one form, are kept.
+enum class SumOrder { any, kept };
 bool gate_up_side_by_side(const xq_weight* wg, const xq_weight* wu, const bf16_t* x, int64_t ldx, int64_t M, const bf16_t* bias_g,
                           const bf16_t* bias_u, const bf16_t* gu, int64_t ldgu);
 int launch_gate_up(const xq_weight* wg, const xq_weight* wu, const bf16_t* x, int64_t ldx, int64_t M, const bf16_t* su_g, const bf16_t* su_u,
@@ -217,6 +222,7 @@ int launch_tile_gemm(const xq_weight* w, bool contract_cols, const bf16_t* A, in
                      int r_pad, const bf16_t* bias, bf16_t* C, int64_t ldc, hipStream_t stream, const char* who,
                      float* partial, int64_t partial_bytes, const TwoBanks* two = nullptr,
                      const LowRankRight* right = nullptr,   // dense: the side term's right-hand factor (then lora_right is NULL)
+                     SumOrder order = SumOrder::any,
                      const int32_t* a_rows = nullptr,    // grouped, optional: row i of the problem is row a_rows[i] of A,
                      int64_t a_span_rows = 0);           // ... which has this many rows (0: not known)
 bool tile_gemm_takes_row_map(const xq_weight* w);        // ... which only the pipelined tile kernel does

@@ -150,6 +150,11 @@ extern "C" int xq_set_mlp_gate_up_fused(int enabled) {
 
 extern "C" int xq_get_mlp_gate_up_fused(void) { return g_mlp_gu.load() != 0; }
 
+extern "C" int xq_mlp_gate_up_joint(const xq_weight* gate, const xq_weight* up, int64_t M) {
+    if (!gate || !up || M <= 0 || xq_validate_weight(gate, "xq_mlp_gate_up_joint") || xq_validate_weight(up, "xq_mlp_gate_up_joint")) return 0;
+    return gate_up_side_by_side(gate, up, nullptr, gate->cols, M, nullptr, nullptr, nullptr, 2 * gate->rows);
+}
+
 extern "C" int64_t xq_mlp_workspace_bytes_fmt(int format, int64_t M, int64_t hidden, int64_t intermediate, int r, int backward) {
     if (M < 0 || r < 0) return 0;
     Dims d{M, hidden, intermediate, r, r_pad_of(r)};
@@ -221,9 +226,9 @@ extern "C" int xq_mlp_fwd(const xq_weight* gate, const xq_weight* up, const xq_w
             if ((rc = launch_gate_up(gate, up, x, ldx, M, su_gu, rp ? su_gu + sl.up_offset : nullptr, sl.pitch, LowRankRight{{lora->B[0], lora->B[1]}, r, r, rp, f32, 0}, rp,
                                      bias_g, bias_u, gu, 2 * I, stream, who))) return rc;
         } else {
-            if ((rc = launch_tile_gemm(gate, true, x, ldx, M, nullptr, nullptr, rp ? su_gu : nullptr, nullptr, rp, bias_g, gu, 2 * I, stream, who, part, part_bytes, nullptr, rp ? &right_g : nullptr))) return rc;
+            if ((rc = launch_tile_gemm(gate, true, x, ldx, M, nullptr, nullptr, rp ? su_gu : nullptr, nullptr, rp, bias_g, gu, 2 * I, stream, who, part, part_bytes, nullptr, rp ? &right_g : nullptr, SumOrder::kept))) return rc;
             if ((rc = launch_tile_gemm(up, true, x, ldx, M, nullptr, nullptr, rp ? su_gu + sl.up_offset : nullptr, nullptr, rp, bias_u, gu + I, 2 * I, stream, who, part, part_bytes, nullptr,
-                                       rp ? &right_u : nullptr))) return rc;
+                                       rp ? &right_u : nullptr, SumOrder::kept))) return rc;
         }
         if (many) {
             if ((rc = launch_silu_fwd_nt(gu, gu + I, 2 * I, h, I, M, I, A_d, rp, s, su_d, rp, stream))) return rc;
@@ -236,7 +241,7 @@ extern "C" int xq_mlp_fwd(const xq_weight* gate, const xq_weight* up, const xq_w
         if ((rc = launch_lowrank(&jd, 1, M, fm, panels, stream, part, part_bytes))) return rc;
     }
     return launch_tile_gemm(down, true, h, I, M, nullptr, nullptr, rp ? su_d : nullptr, nullptr, rp, bias_d, (bf16_t*)y, ldy, stream,
-                            who, part, part_bytes, nullptr, rp ? &right_d : nullptr);
+                            who, part, part_bytes, nullptr, rp ? &right_d : nullptr, SumOrder::kept);
 }
 
 // ---- forward only: nothing is kept for a backward, so up to 64 rows each projection is free to take the kernel that suits the
@@ -373,7 +378,7 @@ extern "C" int xq_mlp_bwd(const xq_weight* gate, const xq_weight* up, const xq_w
         if ((rc = launch_lowrank(&jd, 1, M, ft, nullptr, stream, part, part_bytes))) return rc;
     }
     if ((rc = launch_tile_gemm(down, false, dy, lddy, M, nullptr, nullptr, rp ? v_d : nullptr, nullptr, rp, nullptr, dh, I, stream, who, part, part_bytes,
-                               nullptr, rp ? &right_d : nullptr)))
+                               nullptr, rp ? &right_d : nullptr, SumOrder::kept)))
         return rc;
     // ---- SwiGLU, and s * dgate . B_g^T, s * dup . B_u^T: one pass over (gate, up, dh) where the rank allows, so that the
     // two products do not read dgate | dup back
@@ -423,12 +428,12 @@ extern "C" int xq_mlp_bwd(const xq_weight* gate, const xq_weight* up, const xq_w
     if (fused) {
         const TwoBanks two{up, nullptr, nullptr};
         return launch_tile_gemm(gate, false, dgu, 2 * I, M, nullptr, nullptr, rp ? v_gu : nullptr, nullptr, rp2, nullptr, (bf16_t*)dx, lddx,
-                                stream, who, part, part_bytes, &two, rp ? &right_gu : nullptr);
+                                stream, who, part, part_bytes, &two, rp ? &right_gu : nullptr, SumOrder::kept);
     }
     if ((rc = launch_tile_gemm(gate, false, dgate, 2 * I, M, nullptr, nullptr, rp ? v_g : nullptr, nullptr, rp, nullptr, (bf16_t*)dx, lddx, stream, who, part, part_bytes, nullptr,
-                               rp ? &right_g : nullptr))) return rc;
+                               rp ? &right_g : nullptr, SumOrder::kept))) return rc;
     if ((rc = launch_tile_gemm(up, false, dup, 2 * I, M, nullptr, nullptr, rp ? v_u : nullptr, nullptr, rp, nullptr, dx_u, H, stream, who, part, part_bytes, nullptr,
-                               rp ? &right_u : nullptr))) return rc;
+                               rp ? &right_u : nullptr, SumOrder::kept))) return rc;
     add_rows_kernel<<<dim3((unsigned)xq_cdiv(M * (H / 8), 256)), 256, 0, stream>>>((bf16_t*)dx, lddx, dx_u, H, M, H / 8);
     XQ_CHECK_LAUNCH(who);
     return XQ_OK;

@@ -973,3 +973,33 @@ def test_bank_tiles_vs_fp32(hip_device, fmt, K, N, r):
             if r:
                 want, size = want + su[s:s + c].float() @ right[e].float().t(), size + su[s:s + c].float().abs() @ right[e].float().abs().t()
             assert bool(((y[s:s + c] - want).abs() <= 2.0 ** -8 * want.abs() + (kc + r) * 2.0 ** -24 * size).all()), (transpose_w, e, c)
+
+
+@pytest.mark.parametrize("fmt,E,T,topk,H,I,r,forced", [
+    ("nvfp4", 12, 1500, 4, 512, 512, 16, 3), ("nvfp4", 16, 900, 4, 512, 768, 40, 3),
+    ("block_fp8", 12, 1500, 4, 512, 512, 16, 3),                   # enough tiles for gemm_bank_kernel, too few of 256 x 256
+    ("block_fp8", 40, 160, 8, 512, 1536, 24, 3),                   # ... an expert with too few rows
+    ("block_fp8", 4, 4100, 2, 512, 1024, 16, 2),                   # large tiles in both forms
+])
+@pytest.mark.parametrize("rw_dtype", [torch.float32, torch.bfloat16])
+def test_fp32_gradients_of_banks_keep_their_sums(hip_device, fmt, E, T, topk, H, I, r, forced, rw_dtype):
+    """Factor and routing-weight gradients are the bits of the program on gemm_256_kernel's tiles (block-fp8 on 256 x 256: gemm_dtl16_kernel's
+    order), whatever tiles the sizes choose for the products that only y and dx come from; those agree to a bf16 step of the largest entry."""
+    from xorl_amd import _C
+
+    m, _ = _make_experts(fmt, E, H, I, r, False, seed=E + T, device=hip_device)
+    rw, sel = _zipf_routing(T, E, topk, seed=4)
+    x, dy = gen((T, H), 1.0, 5, torch.bfloat16).to(hip_device), gen((T, H), 1.0, 6, torch.bfloat16).to(hip_device)
+    got = []
+    try:
+        for policy in (0, forced):
+            _C.check(_C.lib().xq_set_tile_policy(policy))
+            xd, rwd = x.clone().requires_grad_(True), rw.to(rw_dtype).to(hip_device).requires_grad_(True)
+            y = m(xd, rwd, sel.to(hip_device))
+            got.append([y.detach(), *torch.autograd.grad(y, [xd, rwd, *m.get_lora_parameters()], dy)])
+    finally:
+        _C.check(_C.lib().xq_set_tile_policy(0))
+    for a, b in list(zip(*got))[2:]:
+        assert torch.equal(a, b)
+    for a, b in list(zip(*got))[:2]:
+        assert R.max_rel_err(a.float().cpu(), b.double().cpu()) <= 2 ** -7

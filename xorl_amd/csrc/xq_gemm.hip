@@ -110,11 +110,12 @@ static inline int dense_tile_size(int64_t n_rows, int64_t Nout) {
     return xq_cdiv(n_rows, 256) * xq_cdiv(Nout, 256) > num_cus() / 2 ? 256 : 128;
 }
 
-// The same for expert banks.  nf4 and int4: 256 x 256 tiles where an expert's rows fill them (its last tile is half empty on average, and a
+// The same for expert banks.  256 x 256 tiles where an expert's rows fill them (its last tile is half empty on average, and a
 // 4-bit tile decodes in full) and the tiles there are fill half the chip.  Forward and backward of a routed MLP, large over small tiles, by rows an
-// expert: nf4 banks, 64 or 128 experts 93 1.15, 187 1.04 to 1.08, 281 1.03 to 1.10, 421 0.97 to 0.99, 656 0.93; 16 experts 250
-// 1.10 to 1.14, 500 0.90; 8 experts 500 1.09 to 1.14, 750 0.87.
-// Block-fp8 and nvfp4: gemm_bank_kernel's 128 x 256 tiles, two on a compute unit, where there is one for every compute unit, half a tile an
+// expert: 4-bit banks, 64 or 128 experts 93 1.15, 187 1.04 to 1.08, 281 1.03 to 1.10, 421 0.97 to 0.99, 656 0.93; 16 experts 250
+// 1.10 to 1.14, 500 0.90; 8 experts 500 1.09 to 1.14, 750 0.87.  Block-fp8: 64 or 128 experts 46 1.14, 62 1.01, 93 1.04, 125 0.91, 281 0.87; 16
+// experts 125 1.00, 250 0.98, 500 0.81; 8 experts 125 1.23, 250 0.94, 750 0.87.
+// Block-fp8 and nvfp4 products whose sums are free (SumOrder::any): gemm_bank_kernel's 128 x 256 tiles, two on a compute unit, where there is one for every compute unit, half a tile an
 // expert left empty, or for two in five where an expert's rows fill half of one (nvfp4) or most of one.  Routed MLP forward and backward, those
 // over 128 x 128 tiles, by rows an expert, block-fp8: 128 experts 2048/768 8 0.96, 24 0.95, 56 0.86, 96 0.84; 64 experts 2048/1024 6
 // 0.94, 16 0.95, 32 1.03, 64 0.92, 96 0.81; 64 experts 1280/640 6 1.10 and 16 1.02 (175 and 200 tiles), 32 0.99, 64 0.94; 32 experts 4096/1536 6
@@ -124,14 +125,14 @@ static inline int dense_tile_size(int64_t n_rows, int64_t Nout) {
 // 1.05, 32 0.99 (240 tiles), 64 0.91, 128 0.88, 600 0.78; 16 experts 2560/1024 32 1.05, 64 0.98 (128 tiles), 96 0.89, 256 0.82, 600 0.81.
 // (Tiles are counted without the empty part of an expert's last column tile: forwards of 8 and 16 experts 2816/1152, whose 1152 columns are
 // four and a half, block-fp8 90 tiles 1.12, 108 0.98, 130 0.95; nvfp4 90 1.15, 108 0.97, 130 0.91; 16 experts 1536/640 100 1.04 and 1.13.)
-static inline bool bank_large_tiles(int fmt, int64_t n_rows, int num_experts, int64_t Nout) {
-    if (fmt == XQ_FMT_FP8 || fmt == XQ_FMT_NVFP4) {
+static inline bool bank_large_tiles(int fmt, int64_t n_rows, int num_experts, int64_t Nout, SumOrder order) {
+    if (order == SumOrder::any && (fmt == XQ_FMT_FP8 || fmt == XQ_FMT_NVFP4)) {
         using D = GeoBank<XQ_FMT_FP8>;
         const int64_t tiles = (xq_cdiv(n_rows, D::ROWS) + num_experts / 2) * Nout / D::COLS;
         return tiles >= (n_rows >= (fmt == XQ_FMT_FP8 ? 90ll : 60ll) * num_experts ? num_cus() * 13 / 32 : num_cus());
     }
     const int64_t tiles = (xq_cdiv(n_rows, 256) + num_experts / 2) * xq_cdiv(Nout, 256);
-    return n_rows >= 400ll * num_experts && tiles > num_cus() / 2;
+    return n_rows >= (fmt == XQ_FMT_FP8 ? 100ll : 400ll) * num_experts && tiles > num_cus() / 2;
 }
 
 // K splits of a dense launch of `blocks` tiles of size T over nk K-steps (1 = none): used when the tiles fill at
@@ -467,24 +468,24 @@ bool two_banks_supported(const xq_weight* w) {
 }
 
 // tile size of a grouped launch on the pipelined kernel
-static inline int bank_tile_size(int fmt, int64_t n_rows, int num_experts, int64_t Nout) {
-    return g_tile_policy == 2 ? 256 : g_tile_policy == 3 ? 128 : bank_large_tiles(fmt, n_rows, num_experts, Nout) ? 256 : 128;
+static inline int bank_tile_size(int fmt, int64_t n_rows, int num_experts, int64_t Nout, SumOrder order) {
+    return g_tile_policy == 2 ? 256 : g_tile_policy == 3 ? 128 : bank_large_tiles(fmt, n_rows, num_experts, Nout, order) ? 256 : 128;
 }
 
 // ... of two banks' columns side by side: small tiles too where large ones do not divide a bank's columns and one bank alone would not take them
-static inline int side_by_side_tile(int fmt, int64_t n_rows, int num_experts, int64_t ncols) {
-    const int T = bank_tile_size(fmt, n_rows, num_experts, 2 * ncols);
-    return ncols % T != 0 ? bank_tile_size(fmt, n_rows, num_experts, ncols) : T;
+static inline int side_by_side_tile(int fmt, int64_t n_rows, int num_experts, int64_t ncols, SumOrder order) {
+    const int T = bank_tile_size(fmt, n_rows, num_experts, 2 * ncols, order);
+    return ncols % T != 0 ? bank_tile_size(fmt, n_rows, num_experts, ncols, order) : T;
 }
 
 // Whether two 4-bit banks of one shape and storage take one launch whose output holds both products side by side, ncols columns
 // each (G256Args::W2): whole column tiles per bank.  One bank's tiles leave half of the block slots empty at some hundreds of
 // routed rows and end in a round of their own beyond (routed MLP, two launches and one, us: nf4 32 experts 2560/1024, 800 rows, forward and backward 510 and 461; nvfp4 64 experts 2048/1024, 9000 rows 886 and 816, forward alone of 6000 rows 350 and 305).
-bool banks_side_by_side(const xq_weight* a, const xq_weight* b, int64_t ncols, int64_t n_rows) {
+bool banks_side_by_side(const xq_weight* a, const xq_weight* b, int64_t ncols, int64_t n_rows, SumOrder order) {
     return a->format != XQ_FMT_FP8 && tile_gemm_takes_row_map(a) && tile_gemm_takes_row_map(b) && a->format == b->format &&
            a->rows == b->rows && a->cols == b->cols && a->num_experts == b->num_experts && a->group == b->group &&
            a->scale_dtype == b->scale_dtype && xq_packed_bytes_per_expert(a) % 16 == 0 && xq_aligned(a->packed, 16) && xq_aligned(b->packed, 16) &&
-           ncols % side_by_side_tile(a->format, n_rows, a->num_experts, ncols) == 0;
+           ncols % side_by_side_tile(a->format, n_rows, a->num_experts, ncols, order) == 0;
 }
 
 // Whether the dgrad of two dense [N, K] weights of one shape may run as one launch (see launch_tile_gemm): block-fp8 on
@@ -632,7 +633,7 @@ static int launch_tile_gemm_t(const xq_weight* w, bool contract_cols, const bf16
                        "%s: the dense two-matrix form is the dgrad of two block-fp8 weights (out_features %% 128 == 0, >= 512)", who);
             g.Kc *= 2;
         } else {
-            XQ_REQUIRE((two_banks_supported(w) && two_banks_supported(two->w2)) || banks_side_by_side(w, two->w2, g.Nout, n_rows),
+            XQ_REQUIRE((two_banks_supported(w) && two_banks_supported(two->w2)) || banks_side_by_side(w, two->w2, g.Nout, n_rows, order),
                        "%s: a two-bank launch takes two block-fp8 expert banks (columns a multiple of 256) or two 4-bit ones (whole tiles)", who);
             XQ_REQUIRE(xq_aligned(two->su2, 16) && xq_aligned(two->lora_right2, 16) && two->a_off2 % 8 == 0, "%s: the second bank's operands must be 16-byte aligned", who);
             if (contract_cols && w->format == XQ_FMT_FP8) g.Kc *= 2;
@@ -669,8 +670,8 @@ static int launch_tile_gemm_t(const xq_weight* w, bool contract_cols, const bf16
                                       : w->layout == XQ_LAYOUT_FLAT));
         const DensePlan plan = plan_dense(n_rows, g.Nout, g.Kc / BK);
         const bool planned = !grouped && fmt_ok && g_tile_policy == 0 && force_T == 0 && !two_dense;   // two matrices: one unsplit launch
-        const int T = force_T ? force_T : grouped ? (two && w->format != XQ_FMT_FP8 ? side_by_side_tile(w->format, n_rows, w->num_experts, g.Nout / 2)
-                                                                         : bank_tile_size(w->format, n_rows, w->num_experts, g.Nout)) : g_tile_policy == 2 ? 256 : g_tile_policy == 3 ? 128 : plan.T;
+        const int T = force_T ? force_T : grouped ? (two && w->format != XQ_FMT_FP8 ? side_by_side_tile(w->format, n_rows, w->num_experts, g.Nout / 2, order)
+                                                                         : bank_tile_size(w->format, n_rows, w->num_experts, g.Nout, order)) : g_tile_policy == 2 ? 256 : g_tile_policy == 3 ? 128 : plan.T;
         MidPlan mid;
         const bool by_size = planned || (two_dense && g_tile_policy == 0);
         // (its storages: the formats' usual groups and scale types; 32-bit offsets from a base for the operands)
@@ -773,16 +774,16 @@ static int launch_tile_gemm_t(const xq_weight* w, bool contract_cols, const bf16
             // read, one block per tile (dense xq_gemm_dtl.h, expert banks xq_gemm_bank.h)
             const int nk_all = g.Kc / BK;
             // (two matrices: the second one starts on a scale-block boundary of the contraction, or -- two banks side by side -- on a
-            // tile boundary of the columns.  nvfp4 banks under a forced tile size stay on gemm_256_kernel, whose sums are the same
-            // for both sizes.)
+            // tile boundary of the columns.  nvfp4 banks under a forced tile size, or whose order of sums is kept, stay on gemm_256_kernel,
+            // whose sums are the same for both sizes; block-fp8 ones have gemm_dtl16_kernel's order and its limit here.)
             const bool side_by_side = grouped && (!contract_cols || w->format != XQ_FMT_FP8);
             const bool two_ok = !two || (side_by_side ? f.ncols1 % 256 == 0 : (f.nk1 % 2 == 0 && f.nk1 >= 2));
             const int64_t reach = (1ll << 32) - (grouped ? 4096 : 0);
-            const bool storage = w->format == XQ_FMT_FP8 || (grouped && w->format == XQ_FMT_NVFP4 && g_tile_policy == 0 && g.group == 16 && g.scale_dtype == XQ_SCALE_E4M3);
+            const bool storage = w->format == XQ_FMT_FP8 || (grouped && w->format == XQ_FMT_NVFP4 && g_tile_policy == 0 && order == SumOrder::any && g.group == 16 && g.scale_dtype == XQ_SCALE_E4M3);
             const bool direct = g_fp8_direct && storage && T == 256 && ksplit == 1 && nk_all >= 3 && two_ok &&
                                 // (their lanes address their operands by 32-bit byte offsets from a base, the bank kernel's up to 3 KB further on)
                                 a_rows_span > 0 && a_rows_span * lda * 2 < reach && (int64_t)g.wrows * g.wcols < reach;
-            if (direct && grouped && g.wcols % 16 == 0 && f.wide_rows && !bias) {
+            if (direct && grouped && g.wcols % 16 == 0 && f.wide_rows && !bias && (order == SumOrder::any || g.Kc <= kDtlMaxK)) {
                 using D = GeoBank<XQ_FMT_FP8>;
                 f.tiles_m = (int32_t)(xq_cdiv(n_rows, D::ROWS) + w->num_experts);
                 f.tiles_n = (int32_t)xq_cdiv(g.Nout, D::COLS);

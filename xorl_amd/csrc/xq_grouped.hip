@@ -87,9 +87,11 @@ int64_t bwd_workspace(const Dims& d) {
 
 // one sum for the two dgrads of gate and up: block-fp8 banks on the pipelined kernel.  (Their forwards as one launch: these banks,
 // and 4-bit banks where banks_side_by_side() says so, whose dgrads then share a launch too but stay two products.)
+// The sums of gate, up and the dgrad of down are kept: all six factor gradients and the routing weights' are computed from them.  The forward
+// of down and the dgrads of gate and up only leave as bf16 (y, dx).
 bool fuse_gate_up(const xq_weight* gate, const xq_weight* up) { return two_banks_supported(gate) && two_banks_supported(up); }
-bool joint_forward(const xq_weight* gate, const xq_weight* up, int64_t R) { return fuse_gate_up(gate, up) || banks_side_by_side(gate, up, gate->cols, R); }
-bool joint_dgrads(const xq_weight* gate, const xq_weight* up, int64_t R) { return banks_side_by_side(gate, up, gate->rows, R); }
+bool joint_forward(const xq_weight* gate, const xq_weight* up, int64_t R) { return fuse_gate_up(gate, up) || banks_side_by_side(gate, up, gate->cols, R, SumOrder::kept); }
+bool joint_dgrads(const xq_weight* gate, const xq_weight* up, int64_t R) { return banks_side_by_side(gate, up, gate->rows, R, SumOrder::any); }
 
 }  // namespace
 }  // namespace xq
@@ -200,10 +202,10 @@ extern "C" int xq_grouped_fwd_ids(const xq_weight* gate, const xq_weight* up, co
     }
     if (joint_forward(gate, up, R)) {       // both projections in one launch: column tiles past I take the up bank
         const TwoBanks two{up, su_u, Lr_uB, 0};
-        if ((rc = launch_tile_gemm(gate, false, xr, ld_xr, R, off, toff, su_g, Lr_gB, rp, nullptr, gu, 2 * I, stream, who, nullptr, 0, &two, nullptr, SumOrder::any, xr_rows, d.T))) return rc;
+        if ((rc = launch_tile_gemm(gate, false, xr, ld_xr, R, off, toff, su_g, Lr_gB, rp, nullptr, gu, 2 * I, stream, who, nullptr, 0, &two, nullptr, SumOrder::kept, xr_rows, d.T))) return rc;
     } else {
-        if ((rc = launch_tile_gemm(gate, false, xr, ld_xr, R, off, toff, su_g, Lr_gB, rp, nullptr, gu, 2 * I, stream, who, nullptr, 0, nullptr, nullptr, SumOrder::any, xr_rows, d.T))) return rc;
-        if ((rc = launch_tile_gemm(up, false, xr, ld_xr, R, off, toff, su_u, Lr_uB, rp, nullptr, gu + I, 2 * I, stream, who, nullptr, 0, nullptr, nullptr, SumOrder::any, xr_rows, d.T))) return rc;
+        if ((rc = launch_tile_gemm(gate, false, xr, ld_xr, R, off, toff, su_g, Lr_gB, rp, nullptr, gu, 2 * I, stream, who, nullptr, 0, nullptr, nullptr, SumOrder::kept, xr_rows, d.T))) return rc;
+        if ((rc = launch_tile_gemm(up, false, xr, ld_xr, R, off, toff, su_u, Lr_uB, rp, nullptr, gu + I, 2 * I, stream, who, nullptr, 0, nullptr, nullptr, SumOrder::kept, xr_rows, d.T))) return rc;
     }
     // SwiGLU (times the row's routing weight) and s * h . A_d^T of the down projection: one pass where the rank allows
     static const bool silu_nt = [] { const char* e = getenv("XQ_MLP_SILU_NT"); return e ? atoi(e) != 0 : true; }();
@@ -329,7 +331,7 @@ extern "C" int xq_grouped_bwd(const xq_weight* gate, const xq_weight* up, const 
     const bf16_t* gd = in_place ? (const bf16_t*)dy : g_down;      // the routed gradient rows: dy through the map, or the copy
     const int64_t ld_gd = in_place ? ld_dy : H;
     const int32_t* gd_rows = in_place ? token_of_row : nullptr;
-    if ((rc = launch_tile_gemm(down, true, gd, ld_gd, R, off, toff, v_d, Lr_dA, rp, nullptr, dh, I, stream, who, nullptr, 0, nullptr, nullptr, SumOrder::any, gd_rows, d.T))) return rc;
+    if ((rc = launch_tile_gemm(down, true, gd, ld_gd, R, off, toff, v_d, Lr_dA, rp, nullptr, dh, I, stream, who, nullptr, 0, nullptr, nullptr, SumOrder::kept, gd_rows, d.T))) return rc;
 
     // ---- SwiGLU + routing weight, and s * dgate . B_g^T, s * dup . B_u^T of the up / gate projections (y = x.W + s*(x.A).B):
     // one pass over (gate, up, dh) where the rank allows, so that the two products do not read dgate | dup back

@@ -189,6 +189,12 @@ int launch_tn(const bf16_t* P, int64_t ldp, int64_t width, const bf16_t* Q, int 
 
 int launch_zero_fill(void* p, int64_t bytes, hipStream_t stream);
 
+// What a product's fp32 sums have to equal.  any: the kernels are free to sum in the order that suits the sizes.  kept: the order of the
+// kernel that the sizes choose among gemm_256_kernel, gemm_mid_kernel, gemm_dec_kernel and gemm_dtl16_kernel (expert banks: 256 x 256 tiles of
+// block-fp8 in gemm_dtl16_kernel's order, everything else in gemm_256_kernel's).  A bf16
+// rounding of such a sum that flips with the order moves what is computed from it by some 2e-4 (2-norm), in fp32 results too: that is many times
+// fp32's rounding.  So the products that fp32 gradients are computed from, or that one program runs in more than one form, are kept.
+enum class SumOrder { any, kept };
 // fused dequant-GEMM launcher (xq_gemm.hip).  `two`: a grouped launch over two block-fp8 banks of one shape -- the
 // forward (contract_cols false) writes [rows, 2 * cols] with the second bank's columns, side term su2 / lora_right2,
 // after the first's; the dgrad (contract_cols true) contracts A [rows, 2 * cols] against both banks into one sum.
@@ -201,17 +207,12 @@ struct TwoBanks {
 int64_t tile_gemm_split_bytes(int64_t n_rows, int64_t Nout, int64_t Kc);     // split-K scratch a dense launch may want
 int64_t tile_gemm_partial_bytes(int fmt, int64_t n_rows, int64_t Nout, int64_t Kc);   // ... or the decoded image of a weight of that format (< 0: of any)
 bool two_banks_supported(const xq_weight* w);
-bool banks_side_by_side(const xq_weight* a, const xq_weight* b, int64_t ncols, int64_t n_rows);
+bool banks_side_by_side(const xq_weight* a, const xq_weight* b, int64_t ncols, int64_t n_rows, SumOrder order);
 bool two_dense_supported(const xq_weight* w);   // dense [N, K] pair: one dgrad launch, dX = [dY1 | dY2] . [W1 ; W2]
 int launch_gate_up_swiglu(const xq_weight* wg, const xq_weight* wu, const bf16_t* x, int64_t ldx, int64_t M,
                           const bf16_t* su_g, const bf16_t* su_u, int64_t ld_su, const LowRankRight& right,
                           int r_pad, const bf16_t* bias_g, const bf16_t* bias_u, bf16_t* gu, int64_t ldgu, bf16_t* h,
                           int64_t ldh, hipStream_t stream);
-// What a product's fp32 sums have to equal.  any: this library's kernels are free to sum in the order that suits the sizes.  kept: the order of the
-// kernel that the sizes choose for a product by itself among gemm_256_kernel, gemm_mid_kernel, gemm_dec_kernel and gemm_dtl16_kernel.  A bf16
-// rounding of such a sum that flips with the order moves what is computed from it by some 2e-4 (2-norm), in fp32 results too: that is many times
-// fp32's rounding.  So the products that factor gradients are computed from, or that one program runs in more than one form, are kept.
-enum class SumOrder { any, kept };
 bool gate_up_side_by_side(const xq_weight* wg, const xq_weight* wu, const bf16_t* x, int64_t ldx, int64_t M, const bf16_t* bias_g,
                           const bf16_t* bias_u, const bf16_t* gu, int64_t ldgu);
 int launch_gate_up(const xq_weight* wg, const xq_weight* wu, const bf16_t* x, int64_t ldx, int64_t M, const bf16_t* su_g, const bf16_t* su_u,

@@ -198,6 +198,21 @@ def test_build_refuses_scratch_under_hand_counted_reads():
         b.check_scratch(b._split_remarks(output(other, 0) + "\n" + output(dec, 80))[0], guarded)
 
 
+def test_build_finds_every_kernel_that_reads_lds_from_assembly():
+    """Whatever a kernel's attributes and parameters; a __global__ function whose name is not found stops the build."""
+    from xorl_amd.csrc import build as b
+
+    assert {"gemm_bank_kernel", "gemm_dec_kernel", "gemm_dtl16_kernel"} <= set(b.asm_read_kernels())
+    text = """// a __global__ void in a comment
+    template <bool A> __global__ void __launch_bounds__(256, 2) one_kernel(std::conditional_t<A, Pair, Args> args) {}
+    static __global__ void __launch_bounds__(Geo<int>::nt()) two_kernel(const float* __restrict__ p,
+                                                                        int n) {}
+    __global__ __launch_bounds__(64) void three_kernel() {}"""
+    assert b.kernels_in(text) == ["one_kernel", "two_kernel", "three_kernel"]
+    with pytest.raises(RuntimeError, match="not found"):
+        b.kernels_in(text + " extern \"C\" __global__ auto four_kernel() -> void {}")
+
+
 @pytest.mark.parametrize("K,near", [(1152, 2), (2048, 1)])     # a depth of the streaming kernels and one of the one-launch kernels (to 16 rows)
 def test_rows_of_x_far_apart_leave_the_streaming_kernels(K, near):
     """Their addresses within eight rows are 32 bits wide: 2 * 7 * ldx bytes and a row's 128 at most.  One row has no pitch."""

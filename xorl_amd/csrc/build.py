@@ -29,16 +29,34 @@ FLAGS = [
 ]
 
 
-def asm_read_kernels() -> list[str]:
-    """Names of the kernels in files that read LDS into registers from inline assembly with waits of their own.  The compiler takes
-    such a register as written at once: a spill before the wait would store what it held before."""
+def kernels_in(text: str) -> list[str]:
+    """Names of the __global__ functions of a source, whatever their attributes and parameters."""
+    text = re.sub(r"//[^\n]*|/\*.*?\*/", "", text, flags=re.S)
+    text = re.sub(r"\b__launch_bounds__\s*\((?:[^()]|\([^()]*\))*\)|\b__attribute__\s*\(\((?:[^()]|\([^()]*\))*\)\)", "", text)
+    names = re.findall(r"\b__global__\s+(?:\w+\s+)*?void\s+(\w+)\s*\(", text)
+    if len(names) != len(re.findall(r"\b__global__\b", text)):
+        raise RuntimeError(f"__global__ functions whose names are not found beside {names}")
+    return names
+
+
+def kernels_with(statement: str) -> list[str]:
+    """Names of the kernels in files that have such an inline assembly statement (a pattern of its text)."""
     names = []
     for path in sorted(glob.glob(os.path.join(HERE, "*.h")) + glob.glob(os.path.join(HERE, "*.hip"))):
         with open(path) as f:
             text = f.read()
-        if re.search(r'asm volatile\("ds_read', text):
-            names += re.findall(r"__global__ [^;{]*?(\w+)\(\w+ \w+\) *\{", text)
+        if re.search(r'asm volatile\("' + statement, text):
+            here = kernels_in(text)
+            if not here:
+                raise RuntimeError(f"{path}: inline assembly that is checked by kernel, and no kernel")
+            names += here
     return names
+
+
+def asm_read_kernels() -> list[str]:
+    """Names of the kernels in files that read LDS into registers from inline assembly with waits of their own.  The compiler takes
+    such a register as written at once: a spill before the wait would store what it held before."""
+    return kernels_with("ds_read")
 
 
 def check_scratch(remarks: str, guarded: list[str]) -> None:

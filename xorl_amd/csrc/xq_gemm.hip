@@ -899,21 +899,19 @@ int launch_gate_up(const xq_weight* wg, const xq_weight* wu, const bf16_t* x, in
                    int64_t ld_su, const LowRankRight& right, int r_pad, const bf16_t* bias_g, const bf16_t* bias_u, bf16_t* gu, int64_t ldgu,
                    hipStream_t stream, const char* who) {
     using D = GeoBank<XQ_FMT_FP8>;
-    G256Args f[2] = {};
-    const xq_weight* w[2] = {wg, wu};
-    for (int i = 0; i < 2; ++i) {
-        G256Args& q = f[i];
-        q.A = x; q.lda = ldx; q.C = gu + i * w[i]->rows; q.ldc = ldgu;
-        q.W = (const uint8_t*)w[i]->packed; q.scales = (const uint8_t*)w[i]->scales;
-        q.wrows = (int32_t)w[i]->rows; q.wcols = (int32_t)w[i]->cols; q.scale_dtype = w[i]->scale_dtype;
-        q.Kc = q.wcols; q.Nout = q.wrows; q.M = M; q.num_experts = 1;
-        q.su = r_pad ? (i ? su_u : su_g) : nullptr; q.right = right; q.right.f[0] = right.f[i]; q.right.f[1] = nullptr; q.r_pad = r_pad; q.ld_su = ld_su;
-        q.bias = i ? bias_u : bias_g;
-        q.tiles_m = (int32_t)xq_cdiv(M, D::ROWS); q.tiles_n = (int32_t)xq_cdiv(q.Nout, D::COLS);
-        q.ksplit = 1; q.wide_rows = 1;
-    }
+    const bool side = r_pad > 0;
+    G256Args f{};
+    f.A = x; f.lda = ldx; f.C = gu; f.ldc = ldgu; f.ncols1 = (int32_t)wg->rows;
+    f.W = (const uint8_t*)wg->packed; f.scales = (const uint8_t*)wg->scales;
+    f.W2 = (const uint8_t*)wu->packed; f.scales2 = (const uint8_t*)wu->scales;
+    f.wrows = (int32_t)wg->rows; f.wcols = (int32_t)wg->cols; f.scale_dtype = wg->scale_dtype;
+    f.Kc = f.wcols; f.Nout = f.wrows; f.M = M; f.num_experts = 1;
+    f.su = side ? su_g : nullptr; f.su2 = side ? su_u : nullptr; f.right = right; f.r_pad = r_pad; f.ld_su = ld_su;
+    f.bias = bias_g; f.bias2 = bias_u;
+    f.tiles_m = (int32_t)xq_cdiv(M, D::ROWS); f.tiles_n = (int32_t)xq_cdiv(f.Nout, D::COLS);
+    f.ksplit = 1; f.wide_rows = 1;
     const bool timed = xq_profile_mark_begin(stream, 2.0 * (double)M * (2.0 * wg->rows) * ((double)wg->cols + r_pad));
-    const int rc = launch_bank_pair(f, true, stream, who);
+    const int rc = launch_bank(f, XQ_FMT_FP8, true, stream, who);
     if (rc) return rc;
     XQ_CHECK_LAUNCH(who);
     if (timed) xq_profile_mark_end(stream);

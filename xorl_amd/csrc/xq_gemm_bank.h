@@ -94,16 +94,8 @@ __device__ __forceinline__ void bank_pair_unit(uint32_t codes, uint32_t scales, 
     odd[W] = pack_bf16x2(a[1] * s0, b[1] * s1);
 }
 
-// dense launches take one product, or two of one shape on one input (gridDim.y)
-struct BankPair {
-    G256Args of[2];
-};
-__device__ __forceinline__ const G256Args& bank_args(const G256Args& a) { return a; }
-__device__ __forceinline__ const G256Args& bank_args(const BankPair& a) { return a.of[blockIdx.y]; }
-
 template <int FMT, bool CC, bool DENSE = false>
-__global__ void __launch_bounds__(256, 2) gemm_bank_kernel(std::conditional_t<DENSE, BankPair, G256Args> args) {
-    const G256Args& g = bank_args(args);
+__global__ void __launch_bounds__(256, 2) gemm_bank_kernel(G256Args g) {
     using D = GeoBank<FMT>;
     constexpr bool F4 = D::F4;
     constexpr int TM = 8, TN = 4, NC = 16;
@@ -149,6 +141,10 @@ __global__ void __launch_bounds__(256, 2) gemm_bank_kernel(std::conditional_t<DE
     float gs = F4 ? g.global_scale[e] : 1.0f;
     const bf16_t* su_b = g.su;
     const bf16_t* lr_b = g.lora_right;
+    // (dense: the second of two products of one shape on one input, gridDim.y; G256Args: W2, scales2, su2, bias2, right.f[1], and C from column
+    // ncols1 on.  What differs is picked where it is used)
+    const bool second_product = DENSE && blockIdx.y != 0;
+    if (second_product) { Wb = g.W2; Sb = g.scales2; su_b = g.su2; }
     if constexpr (!DENSE && (!CC || F4)) {
         if (g.W2 != nullptr) {
             bank_width = g.ncols1;
@@ -350,7 +346,7 @@ __global__ void __launch_bounds__(256, 2) gemm_bank_kernel(std::conditional_t<DE
     const int ranks = DENSE ? min(rp, (g.right.r + 7) & ~7) : rp;
     auto side_w = [&](int j, int ks) {
         if constexpr (DENSE)
-            return __builtin_bit_cast(bf16x8, right_chunk(g.right, 0, min(n0w + wn * 64 + j * 16 + t16, g.Nout - 1), min(ks * 4 + tg, (ranks >> 3) - 1)));
+            return __builtin_bit_cast(bf16x8, right_chunk(g.right, second_product, min(n0w + wn * 64 + j * 16 + t16, g.Nout - 1), min(ks * 4 + tg, (ranks >> 3) - 1)));
         const int n = min(n0w + wn * 64 + (F4 && CC ? (j >> 1) * 32 + 2 * t16 + (j & 1) : j * 16 + t16), bank_width - 1);
         return *(const bf16x8*)(lr_t + (uint32_t)((n * rp + side_chunk(ks)) * 2));
     };
@@ -492,6 +488,9 @@ __global__ void __launch_bounds__(256, 2) gemm_bank_kernel(std::conditional_t<DE
             for (int i = 0; i < TM; ++i) sx[i] = in_rank(sx[i], ks);
 #pragma unroll
             for (int j = 0; j < TN; ++j) {                             // one at a time, for the registers
+                // (... and the addresses of all four, which do not change with ks, are not worked out ahead and kept: that is three to
+                // eight registers more than there are beside the sums)
+                asm volatile("" : "+v"(t16), "+v"(tg));
                 const bf16x8 w = in_rank(side_w(j, ks), ks);
 #pragma unroll
                 for (int i = 0; i < TM; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, sx[i], acc[i][j], 0, 0, 0);
@@ -512,10 +511,11 @@ __global__ void __launch_bounds__(256, 2) gemm_bank_kernel(std::conditional_t<DE
         }
     }
 
-    if (DENSE && g.bias) {
+    const bf16_t* bias = second_product ? g.bias2 : g.bias;
+    if (DENSE && bias) {
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
-            const u32x2 b = *(const u32x2*)(g.bias + min(n0 + wn * 64 + j * 16 + 4 * tg, g.Nout - 4));
+            const u32x2 b = *(const u32x2*)(bias + min(n0 + wn * 64 + j * 16 + 4 * tg, g.Nout - 4));
             const f32x4 b4 = {__uint_as_float(b[0] << 16), __uint_as_float(b[0] & 0xffff0000u), __uint_as_float(b[1] << 16), __uint_as_float(b[1] & 0xffff0000u)};
 #pragma unroll
             for (int i = 0; i < TM; ++i) acc[i][j] += b4;
@@ -529,7 +529,7 @@ __global__ void __launch_bounds__(256, 2) gemm_bank_kernel(std::conditional_t<DE
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
         const int row = row0 + i * 16 + t16;
-        bf16_t* dst = g.C + (int64_t)row * g.ldc + col;
+        bf16_t* dst = g.C + (int64_t)row * g.ldc + col + (second_product ? g.ncols1 : 0);
 #pragma unroll
         for (int jp = 0; jp < TN / 2; ++jp) {
             const f32x4 u = acc[i][2 * jp], v = acc[i][2 * jp + 1];
@@ -552,7 +552,7 @@ __global__ void __launch_bounds__(256, 2) gemm_bank_kernel(std::conditional_t<DE
 #undef XQ_BANK_READ_W
 }
 
+// (dense block-fp8: f.W2 with ncols1 > 0 is the weight of a second product)
 int launch_bank(const G256Args& f, int fmt, bool cc, hipStream_t s, const char* who);
-int launch_bank_pair(const G256Args (&f)[2], bool cc, hipStream_t s, const char* who);      // dense block-fp8: two products of one shape
 
 }  // namespace xq

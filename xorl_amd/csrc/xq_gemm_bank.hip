@@ -4,8 +4,8 @@
 
 namespace xq {
 
-template <int FMT, bool CC, bool DENSE, typename Args>
-static int launch_bank_one(const Args& args, dim3 grid, hipStream_t s, const char* who) {
+template <int FMT, bool CC, bool DENSE>
+static int launch_bank_one(const G256Args& args, dim3 grid, hipStream_t s, const char* who) {
     using D = GeoBank<FMT>;
     static std::atomic<bool> attr_set{false};   // the attribute call is idempotent: a race only repeats it
     if (!attr_set) {
@@ -20,14 +20,11 @@ static int launch_bank_one(const Args& args, dim3 grid, hipStream_t s, const cha
     return XQ_OK;
 }
 
-static int launch_bank_dense(const BankPair& p, unsigned products, bool cc, hipStream_t s, const char* who) {
-    const dim3 grid((unsigned)(p.of[0].tiles_m * p.of[0].tiles_n), products);
-    return cc ? launch_bank_one<XQ_FMT_FP8, true, true>(p, grid, s, who) : launch_bank_one<XQ_FMT_FP8, false, true>(p, grid, s, who);
-}
-int launch_bank_pair(const G256Args (&f)[2], bool cc, hipStream_t s, const char* who) { return launch_bank_dense(BankPair{{f[0], f[1]}}, 2, cc, s, who); }
-
 int launch_bank(const G256Args& f, int fmt, bool cc, hipStream_t s, const char* who) {
-    if (!f.offsets) return launch_bank_dense(BankPair{{f, f}}, 1, cc, s, who);
+    if (!f.offsets) {
+        const dim3 grid((unsigned)(f.tiles_m * f.tiles_n), f.W2 ? 2 : 1);
+        return cc ? launch_bank_one<XQ_FMT_FP8, true, true>(f, grid, s, who) : launch_bank_one<XQ_FMT_FP8, false, true>(f, grid, s, who);
+    }
     const dim3 grid((unsigned)(f.tiles_m * f.tiles_n));
     if (fmt == XQ_FMT_NVFP4) return cc ? launch_bank_one<XQ_FMT_NVFP4, true, false>(f, grid, s, who) : launch_bank_one<XQ_FMT_NVFP4, false, false>(f, grid, s, who);
     return cc ? launch_bank_one<XQ_FMT_FP8, true, false>(f, grid, s, who) : launch_bank_one<XQ_FMT_FP8, false, false>(f, grid, s, who);

@@ -1003,3 +1003,28 @@ def test_fp32_gradients_of_banks_keep_their_sums(hip_device, fmt, E, T, topk, H,
         assert torch.equal(a, b)
     for a, b in list(zip(*got))[:2]:
         assert R.max_rel_err(a.float().cpu(), b.double().cpu()) <= 2 ** -7
+
+
+@pytest.mark.parametrize("fmt,E,T,topk,H,I,r,hybrid", [("nvfp4", 12, 1500, 4, 512, 512, 16, False), ("block_fp8", 12, 1500, 4, 512, 512, 24, True)])
+def test_forward_that_no_backward_follows(hip_device, fmt, E, T, topk, H, I, r, hybrid):
+    """A routed forward without gradients may sum its products in another order than one that a backward follows: both against the float64
+    program, with gate and up of different magnitude (and so of different global scales), and the same bits from the module and from the function."""
+    from xorl_amd import moe_functional as MF
+
+    m, banks = _make_experts(fmt, E, H, I, r, hybrid, seed=E + I, device="cpu")
+    up = 0.25 * gen((E, H, I), 0.05, E + I + 1)
+    m.load_weights(banks["gate"].float(), up, banks["down"].float())
+    m = m.to(hip_device)
+    ref = {p: m.dequantize_all_experts(p, *m._proj_dims(p)).to(torch.bfloat16).cpu() for p in banks}       # (bit-exact with the oracle: test_moe_fwd_bwd_vs_oracle)
+    rw, sel = _zipf_routing(T, E, topk, seed=7)
+    rw = rw.to(torch.bfloat16)
+    x = gen((T, H), 1.0, 8, torch.bfloat16)
+    xd, rwd, seld = x.to(hip_device), rw.to(hip_device), sel.to(hip_device)
+    with torch.no_grad():
+        y = m(xd, rwd, seld)
+        views = [v for p in ("gate_proj", "up_proj", "down_proj") for v in m._active_lora_views(p)]
+        assert torch.equal(y, MF.moe_experts_qlora_forward(E, rwd, seld, xd, *(m._bank(p) for p in ("gate", "up", "down")), *views, m.scaling))
+    lora = {k: (getattr(m, f"{k}_proj_lora_A").detach().cpu(), getattr(m, f"{k}_proj_lora_B").detach().cpu()) for k in ("gate", "up", "down")}
+    ex = R.moe_fwd_bwd(x, rw, sel, ref["gate"], ref["up"], ref["down"], lora, m.scaling, torch.zeros_like(x))
+    close(y.cpu(), ex["y"], TOL)
+    close(m(xd.requires_grad_(True), rwd, seld).detach().cpu(), ex["y"], TOL)

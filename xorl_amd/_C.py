@@ -58,7 +58,8 @@ class XqGroupedLora(ctypes.Structure):
 class XqGroupedSaved(ctypes.Structure):
     _fields_ = [(n, ctypes.c_void_p) for n in ("xs", "gate_up", "h", "w_row", "su_gate", "su_up", "su_down",
                                                "scatter_index", "offsets", "tile_offsets", "counts", "x_tokens")] + [
-                                                   ("ld_x_tokens", ctypes.c_int64)]
+                                                   ("ld_x_tokens", ctypes.c_int64), ("forward_only", ctypes.c_int32),
+                                                   ("reserved", ctypes.c_int32)]
 
 
 class XqGroupedGrads(ctypes.Structure):

@@ -88,9 +88,9 @@ int64_t bwd_workspace(const Dims& d) {
 // one sum for the two dgrads of gate and up: block-fp8 banks on the pipelined kernel.  (Their forwards as one launch: these banks,
 // and 4-bit banks where banks_side_by_side() says so, whose dgrads then share a launch too but stay two products.)
 // The sums of gate, up and the dgrad of down are kept: all six factor gradients and the routing weights' are computed from them.  The forward
-// of down and the dgrads of gate and up only leave as bf16 (y, dx).
+// of down and the dgrads of gate and up only leave as bf16 (y, dx), and so does a whole forward that no backward follows.
 bool fuse_gate_up(const xq_weight* gate, const xq_weight* up) { return two_banks_supported(gate) && two_banks_supported(up); }
-bool joint_forward(const xq_weight* gate, const xq_weight* up, int64_t R) { return fuse_gate_up(gate, up) || banks_side_by_side(gate, up, gate->cols, R, SumOrder::kept); }
+bool joint_forward(const xq_weight* gate, const xq_weight* up, int64_t R, SumOrder order) { return fuse_gate_up(gate, up) || banks_side_by_side(gate, up, gate->cols, R, order); }
 bool joint_dgrads(const xq_weight* gate, const xq_weight* up, int64_t R) { return banks_side_by_side(gate, up, gate->rows, R, SumOrder::any); }
 
 }  // namespace
@@ -100,7 +100,7 @@ using namespace xq;
 
 extern "C" int xq_grouped_joint(const xq_weight* gate, const xq_weight* up, int64_t n_rows, int forward) {
     if (!gate || !up || xq_validate_weight(gate, "xq_grouped_joint") || xq_validate_weight(up, "xq_grouped_joint")) return 0;
-    return forward ? joint_forward(gate, up, n_rows) : joint_dgrads(gate, up, n_rows);
+    return forward ? joint_forward(gate, up, n_rows, forward == 2 ? SumOrder::any : SumOrder::kept) : joint_dgrads(gate, up, n_rows);
 }
 
 extern "C" int xq_grouped_in_place(const xq_weight* gate, const xq_weight* up, const xq_weight* down) {
@@ -200,12 +200,13 @@ extern "C" int xq_grouped_fwd_ids(const xq_weight* gate, const xq_weight* up, co
             return rc;
         if ((rc = launch_small_nt(xr, ld_xr, R, H, F_uA, rp, s, su_u, off, toff, E, uAe == 1, stream, 0, nullptr, 0, xr_rows, nullptr, 0))) return rc;
     }
-    if (joint_forward(gate, up, R)) {       // both projections in one launch: column tiles past I take the up bank
+    const SumOrder order = saved->forward_only ? SumOrder::any : SumOrder::kept;
+    if (joint_forward(gate, up, R, order)) {       // both projections in one launch: column tiles past I take the up bank
         const TwoBanks two{up, su_u, Lr_uB, 0};
-        if ((rc = launch_tile_gemm(gate, false, xr, ld_xr, R, off, toff, su_g, Lr_gB, rp, nullptr, gu, 2 * I, stream, who, nullptr, 0, &two, nullptr, SumOrder::kept, xr_rows, d.T))) return rc;
+        if ((rc = launch_tile_gemm(gate, false, xr, ld_xr, R, off, toff, su_g, Lr_gB, rp, nullptr, gu, 2 * I, stream, who, nullptr, 0, &two, nullptr, order, xr_rows, d.T))) return rc;
     } else {
-        if ((rc = launch_tile_gemm(gate, false, xr, ld_xr, R, off, toff, su_g, Lr_gB, rp, nullptr, gu, 2 * I, stream, who, nullptr, 0, nullptr, nullptr, SumOrder::kept, xr_rows, d.T))) return rc;
-        if ((rc = launch_tile_gemm(up, false, xr, ld_xr, R, off, toff, su_u, Lr_uB, rp, nullptr, gu + I, 2 * I, stream, who, nullptr, 0, nullptr, nullptr, SumOrder::kept, xr_rows, d.T))) return rc;
+        if ((rc = launch_tile_gemm(gate, false, xr, ld_xr, R, off, toff, su_g, Lr_gB, rp, nullptr, gu, 2 * I, stream, who, nullptr, 0, nullptr, nullptr, order, xr_rows, d.T))) return rc;
+        if ((rc = launch_tile_gemm(up, false, xr, ld_xr, R, off, toff, su_u, Lr_uB, rp, nullptr, gu + I, 2 * I, stream, who, nullptr, 0, nullptr, nullptr, order, xr_rows, d.T))) return rc;
     }
     // SwiGLU (times the row's routing weight) and s * h . A_d^T of the down projection: one pass where the rank allows
     static const bool silu_nt = [] { const char* e = getenv("XQ_MLP_SILU_NT"); return e ? atoi(e) != 0 : true; }();

@@ -783,6 +783,7 @@ PyObject* moe(PyObject*, PyObject* const* args, Py_ssize_t n) {
                                      empty_bf({R, rp}), empty_bf({R, rp}), empty_bf({R, rp}), i32(R), i32(E + 1), i32(2 * (E + 1)), i32(E)};
         xq_grouped_saved S;
         grouped_saved(&S, kept, nullptr);
+        S.forward_only = !train;
         Scratch ws(xq_grouped_workspace_bytes(T, (int32_t)topk, (int32_t)E, H, I, r, 0));
         {
             ReleaseGil nogil;

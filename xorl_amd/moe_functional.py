@@ -178,7 +178,7 @@ def _workspace(dev, T: int, topk: int, E: int, H: int, I: int, r: int, backward:
 
 
 def _moe_fwd_impl(hidden2: Tensor, rw: Tensor, sel: Tensor, factors, banks, r: int, scaling: float, allow_in_place: bool = True,
-                  swiglu_limit: float = 0.0):
+                  swiglu_limit: float = 0.0, forward_only: bool = False):
     """xq_grouped_fwd.  hidden2 bf16 [T, H]; rw [T, topk] fp32 / bf16; sel int32 [T, topk]; factors the six active
     LoRA views, contiguous; banks three QuantWeight.  -> (out [T, H], the eleven tensors the backward reads)."""
     qg, qu, qd = banks
@@ -197,6 +197,7 @@ def _moe_fwd_impl(hidden2: Tensor, rw: Tensor, sel: Tensor, factors, banks, r: i
     out = bf(T, H)
     ws = _workspace(dev, T, topk, E, H, I, r, False)
     lora, S = _lora_struct(factors, r, scaling, swiglu_limit), _saved_struct(saved)
+    S.forward_only = int(forward_only)
     _C.check(_C.lib().xq_grouped_fwd(ctypes.byref(wg), ctypes.byref(wu), ctypes.byref(wd), ctypes.byref(lora),
                                      hidden2.data_ptr(), hidden2.stride(0) if T > 1 else H, T, rw.data_ptr(),
                                      _C.XQ_DT_F32 if rw.dtype == torch.float32 else _C.XQ_DT_BF16, sel.data_ptr(), topk,
@@ -291,7 +292,7 @@ class MoeExpertsQLoRAFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, hidden, routing_weights, selected_experts, gA, gB, uA, uB, dA, dB,
                 qw_gate: QuantWeight, qw_up: QuantWeight, qw_down: QuantWeight, num_experts: int, scaling: float,
-                swiglu_limit: float = 0.0):
+                swiglu_limit: float = 0.0, forward_only: bool = False):
         _C.require_hip(hidden, routing_weights, selected_experts)
         if hidden.dtype != torch.bfloat16:
             raise _C.XqError(f"hidden states must be bf16, got {hidden.dtype}")
@@ -320,7 +321,7 @@ class MoeExpertsQLoRAFunction(torch.autograd.Function):
                               qw_gate.fmt, qw_gate.layout, _DT_TO_CODE[qw_gate.scale_dtype], qw_gate.group, E, H, I, r, s, lim)
             out, saved = res[0], tuple(res[1:])
         else:
-            out, saved = _moe_fwd_impl(hidden2, rw, sel, factors, banks, r, s, swiglu_limit=lim)
+            out, saved = _moe_fwd_impl(hidden2, rw, sel, factors, banks, r, s, swiglu_limit=lim, forward_only=forward_only)
         ctx.qw = banks
         ctx.swiglu_limit = lim
         ctx.meta = (E, T, topk, H, I, r, s, shape, routing_weights.dtype, routing_weights.shape)
@@ -347,7 +348,7 @@ class MoeExpertsQLoRAFunction(torch.autograd.Function):
         dx = dx.reshape(shape) if need_dx else None
         drw = drw.reshape(rw_shape).to(rw_dtype) if need_drw else None
         gs = [g.to(f.dtype) for g, f in zip(grads, factors)]
-        return (dx, drw, None, *gs, None, None, None, None, None, None)
+        return (dx, drw, None, *gs, None, None, None, None, None, None, None)
 
 
 # Test switch: False sends forwards that need no gradient through xq_grouped_fwd as well.
@@ -410,8 +411,9 @@ def moe_experts_qlora_forward(num_experts: int, routing_weights: Tensor, selecte
     A forward of a handful of tokens that nothing is differentiated through (decode, rollout) takes the
     weight-streaming form xq_grouped_fwd_infer where the banks allow it."""
     factors = (gate_proj_lora_A, gate_proj_lora_B, up_proj_lora_A, up_proj_lora_B, down_proj_lora_A, down_proj_lora_B)
-    if DECODE_PATH and not torch.compiler.is_compiling() and not (
-            torch.is_grad_enabled() and any(t.requires_grad for t in (hidden_states, routing_weights, *factors))):
+    forward_only = not torch.compiler.is_compiling() and not (
+        torch.is_grad_enabled() and any(t.requires_grad for t in (hidden_states, routing_weights, *factors)))
+    if DECODE_PATH and forward_only:
         out = _moe_infer(hidden_states, routing_weights, selected_experts, factors, (gate_proj, up_proj, down_proj),
                          num_experts, scaling, float(swiglu_limit or 0.0))
         if out is not None:
@@ -419,7 +421,7 @@ def moe_experts_qlora_forward(num_experts: int, routing_weights: Tensor, selecte
     return MoeExpertsQLoRAFunction.apply(hidden_states, routing_weights, selected_experts, gate_proj_lora_A,
                                          gate_proj_lora_B, up_proj_lora_A, up_proj_lora_B, down_proj_lora_A,
                                          down_proj_lora_B, gate_proj, up_proj, down_proj, num_experts, scaling,
-                                         float(swiglu_limit or 0.0))
+                                         float(swiglu_limit or 0.0), forward_only)
 
 
 def moe_experts_qlora_ep_compute(permute_tokens: Tensor, cumsum: Tensor, gate_proj: QuantWeight, up_proj: QuantWeight,
@@ -449,15 +451,15 @@ def moe_experts_qlora_ep_compute(permute_tokens: Tensor, cumsum: Tensor, gate_pr
     if int(ends[-1]) != R:
         raise _C.XqError(f"cumsum ends at {int(ends[-1])} but {R} rows were passed")
     ones = torch.ones(R, 1, dtype=torch.float32, device=dev)
-    if DECODE_PATH and not torch.compiler.is_compiling() and not (
-            torch.is_grad_enabled() and any(t.requires_grad for t in (permute_tokens, *factors))):
+    forward_only = not torch.compiler.is_compiling() and not (torch.is_grad_enabled() and any(t.requires_grad for t in (permute_tokens, *factors)))
+    if DECODE_PATH and forward_only:
         # a handful of rows with nothing to differentiate: the weight-streaming forward (top-1, unit weights)
         out = _moe_infer(permute_tokens, ones, expert_of_row.to(torch.int32).unsqueeze(1), factors, (gate_proj, up_proj, down_proj),
                          E, scaling, float(swiglu_limit or 0.0))
         if out is not None:
             return out
     return MoeExpertsQLoRAFunction.apply(permute_tokens, ones, expert_of_row.to(torch.int32).unsqueeze(1), *factors,
-                                         gate_proj, up_proj, down_proj, E, scaling, float(swiglu_limit or 0.0))
+                                         gate_proj, up_proj, down_proj, E, scaling, float(swiglu_limit or 0.0), forward_only)
 
 
 # registry entries a maintainer adds beside "triton" / "native" / "quack"

@@ -213,6 +213,35 @@ def test_build_finds_every_kernel_that_reads_lds_from_assembly():
         b.kernels_in(text + " extern \"C\" __global__ auto four_kernel() -> void {}")
 
 
+def test_build_refuses_m0_beside_loads_that_take_it():
+    """gemm_bank_kernel writes M0 in one assembly statement and loads with it in others: nothing of the compiler's may touch it."""
+    from xorl_amd.csrc import build as b
+
+    guarded = b.asm_m0_kernels()
+    assert guarded == ["gemm_bank_kernel"]
+
+    def listing(name, line):
+        return f"""{name}:                ; @{name}
+; %bb.0:
+\t;;#ASMSTART
+\ts_mov_b32 m0, s7
+\ts_nop 0
+\t;;#ASMEND
+\tv_add_u32_e32 v1, s4, v0              ; not m0
+{line}
+\t;;#ASMSTART
+\tglobal_load_lds_dwordx4 v1, s[8:9] offset:1024
+\t;;#ASMEND
+\ts_endpgm
+.Lfunc_end0:
+\t.size\t{name}, .Lfunc_end0-{name}
+"""
+    bank, other = "_ZN2xq16gemm_bank_kernelILi2ELb1ELb1EEEvNS_8G256ArgsE", "_ZN2xq14lowrank_kernelILi1EEEvi"
+    b.check_m0(listing(other, "\ts_mov_b32 m0, -1") + listing(bank, "\tv_mov_b32_e32 v2, 0"), guarded)
+    with pytest.raises(RuntimeError, match="m0, s3"):
+        b.check_m0(listing(other, "") + listing(bank, "\ts_mov_b32 m0, s3"), guarded)
+
+
 @pytest.mark.parametrize("K,near", [(1152, 2), (2048, 1)])     # a depth of the streaming kernels and one of the one-launch kernels (to 16 rows)
 def test_rows_of_x_far_apart_leave_the_streaming_kernels(K, near):
     """Their addresses within eight rows are 32 bits wide: 2 * 7 * ldx bytes and a row's 128 at most.  One row has no pitch."""

@@ -59,6 +59,23 @@ def asm_read_kernels() -> list[str]:
     return kernels_with("ds_read")
 
 
+def asm_m0_kernels() -> list[str]:
+    """Names of the kernels in files whose direct-to-LDS loads are assembly statements that take M0 as another statement left it."""
+    return kernels_with("global_load_lds")
+
+
+def check_m0(assembly: str, guarded: list[str]) -> None:
+    """Raise if the compiler uses M0 by itself in one of the guarded kernels, by its assembly."""
+    for name, body in re.findall(r"^(_Z\w+):(.*?)^\s*\.size\s+\1,", assembly, re.S | re.M):
+        kernel = next((k for k in guarded if re.search(rf"\d{k}(?![a-z])", name)), None)
+        if not kernel:
+            continue
+        own = re.sub(r";[^\n]*", "", re.sub(r";\s*#?ASMSTART.*?;\s*#?ASMEND", "", body, flags=re.S))
+        use = re.search(r"^.*\bm0\b.*$", own, re.M)
+        if use:
+            raise RuntimeError(f"{name}: {use[0].strip()} beside loads that expect M0 as {kernel} left it")
+
+
 def check_scratch(remarks: str, guarded: list[str]) -> None:
     """Raise if one of the guarded kernels uses scratch memory, by the compiler's resource remarks."""
     for name, usage in re.findall(r"Function Name: (\S+)(.*?)(?=Function Name: |\Z)", remarks, re.S):
@@ -97,6 +114,14 @@ def _compile(src: str, force: bool) -> str:
         raise RuntimeError(f"hipcc failed for {src}:\n{err}")
     try:
         check_scratch(remarks, asm_read_kernels())
+        m0 = asm_m0_kernels()
+        if any(re.search(rf"\d{k}(?![a-z])", remarks) for k in m0):
+            listing = obj[:-2] + ".s"
+            r = subprocess.run([HIPCC, *FLAGS, "--cuda-device-only", "-S", src, "-o", listing], capture_output=True, text=True)
+            if r.returncode != 0:
+                raise RuntimeError(f"hipcc -S failed for {src}:\n{_split_remarks(r.stderr)[1]}")
+            with open(listing) as f:
+                check_m0(f.read(), m0)
     except RuntimeError:
         os.remove(obj)
         raise

@@ -190,7 +190,8 @@ __global__ void __launch_bounds__(256, 2) gemm_bank_kernel(G256Args g) {
     const uint32_t lds_w = lds0 + D::NA * D::A_BYTES + wn * (D::W_BYTES / 4);        // this wave's columns of weight stage 0
     // (M0, the LDS base of the loads, is written here and used nowhere else in the kernel: once for a run of parts, whose places in
     // LDS follow from the instruction's offset.  That offset counts on the global side too, so a lane's own offset is smaller by it,
-    // and the base by 3 KB, to keep it positive.)
+    // and the base by 3 KB, to keep it positive.  The statement that writes M0 is not the one that reads it: the build refuses this kernel if
+    // the compiler touches M0 by itself.)
     const uint32_t lds_s = lds0 + D::NA * D::A_BYTES + D::NWS * D::W_BYTES + wn * (D::S_BYTES / 4);
     const unsigned char* a_base = (const unsigned char*)Ab - 3072;
     const unsigned char* w_base = Wb - 3072;

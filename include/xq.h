@@ -114,6 +114,15 @@ int xq_set_tile_policy(int policy);
 #define XQ_ROUTE_MID 2
 int xq_dense_route(int format, int forward, int64_t rows, int64_t n_out, int64_t k, int32_t plan[6]);
 
+/* What policy 0 runs a product of n_rows routed rows over a bank w on, or (joint) over two like it as one launch, for tests: forward contracts over
+ * the bank's rows, otherwise (dgrad) over its columns; kept: a product that fp32 gradients are computed from, whose sums keep one order.
+ * Returns XQ_BANK_TILES_128 or _256 (square tiles of the pipelined kernel), XQ_BANK_HALF_TILES (128 rows x 256 columns, two on a compute
+ * unit), or -1 where the bank is not laid out for either.  No counterpart in the reference. */
+#define XQ_BANK_TILES_128 0
+#define XQ_BANK_TILES_256 1
+#define XQ_BANK_HALF_TILES 2
+int xq_bank_route(const xq_weight* w, int forward, int joint, int kept, int64_t n_rows);
+
 /* What a forward of M rows of x, ldx elements apart, that keeps nothing for a backward runs on (factors of rank r or NULL; their
  * addresses count for their alignment), for tests: XQ_SKINNY_ONE_LAUNCH, XQ_SKINNY_STREAM (two launches that stream the weight; plan:
  * its K splits and, launched alone, the tiles of 16 weight rows of a block, otherwise 0), XQ_SKINNY_NONE (the products of

@@ -273,3 +273,29 @@ def test_streaming_plans_know_the_storage():
                 assert 1 <= tiles <= most if where == 2 else where == 1, (fmt, sdt, N, K, M)
                 assert _C.lib().xq_linear_workspace_bytes_fmt(_C.FORMATS[fmt], M, N, K, 16) >= splits * M * N * 4 + (K // 128) * M * 16 * 4
     assert [_C.lib().xq_linear_workspace_bytes(0, 1024, K, 16) > 0 for K in (64, 128, 4096)] == [True] * 3      # (no rows, no plan)
+
+
+def test_banks_get_the_tiles_of_the_kernel_that_takes_them():
+    """128 x 256 tiles, and their rule, are gemm_bank_kernel's: a bank, a contraction or a switch that keeps a launch off that kernel leaves it the
+    rule of the 256 x 256 tiles, from 400 rows an expert on (block-fp8: 100)."""
+    from tests.util_cases import bank_route
+    from xorl_amd import _C
+
+    E, H, I = 128, 2048, 768
+    per = (8, 64, 200, 500)
+    routes = lambda fmt, K=H, **kw: [bank_route(fmt, E, K, I, n * E, True, joint=True, **kw) for n in per]
+    assert routes("nvfp4") == ["half"] * 4 and routes("block_fp8") == ["half"] * 4
+    assert routes("nvfp4", scale_dtype=_C.XQ_SCALE_F32) == ["128", "128", "128", "256"] == routes("nf4")
+    assert routes("nvfp4", kept=True) == ["128", "128", "128", "256"]
+    assert routes("block_fp8", kept=True) == ["128", "128", "half", "half"]
+    assert routes("block_fp8", K=128) == ["128", "128", "256", "256"]          # two K-steps
+    assert routes("nvfp4", K=128) == ["128", "128", "128", "256"]
+    try:
+        _C.check(_C.lib().xq_set_fp8_direct_tiles(0))
+        assert routes("block_fp8") == ["128", "128", "256", "256"]
+        assert routes("nvfp4") == ["half"] * 4                              # (the switch is block-fp8's)
+    finally:
+        _C.check(_C.lib().xq_set_fp8_direct_tiles(1))
+    # 640 columns are no whole tiles of 256: two banks side by side take small ones where one alone does ((4 + 64) 640 / 256 tiles, of 256)
+    assert bank_route("nvfp4", E, H, 640, 64 * E, True) == "half"
+    assert bank_route("nvfp4", E, H, 640, 4 * E, True) == bank_route("nvfp4", E, H, 640, 4 * E, True, joint=True) == "128"

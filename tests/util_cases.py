@@ -108,6 +108,20 @@ def gate_up_joint(M, H, I) -> bool:
     return bool(_C.lib().xq_mlp_gate_up_joint(ctypes.byref(w), ctypes.byref(w), M))
 
 
+def bank_route(fmt, E, K, N, n_rows, forward, joint=False, kept=False, scale_dtype=None) -> str:
+    """xq_bank_route (include/xq.h) of a bank [E, K, N]: "128", "256" or "half" tiles"""
+    import ctypes
+
+    from xorl_amd import _C
+
+    w = _C.XqWeight()
+    w.format, w.layout, w.rows, w.cols, w.num_experts = _C.FORMATS[fmt], _C.XQ_LAYOUT_GKN, K, N, E
+    w.group = {"nvfp4": 16, "block_fp8": 128, "nf4": 64}[fmt]
+    w.scale_dtype = (_C.XQ_SCALE_E4M3 if fmt == "nvfp4" else _C.XQ_SCALE_F32) if scale_dtype is None else scale_dtype
+    w.packed = w.scales = w.global_scale = 4096              # (addresses: nothing is read)
+    return {0: "128", 1: "256", 2: "half"}[_C.lib().xq_bank_route(ctypes.byref(w), int(forward), int(joint), int(kept), n_rows)]
+
+
 def banks_joint(fmt, E, H, I, n_rows, forward) -> bool:
     """xq_grouped_joint (include/xq.h) of gate and up banks [E, H, I] in a format's usual storage"""
     import ctypes

@@ -94,6 +94,7 @@ _SIGNATURES = {
     "xq_profile_enable": (_INT, [_INT]),
     "xq_profile_collect": (_INT, [_P, _P, _P]),
     # format, forward, rows, n_out, k, plan (six int32)
+    "xq_bank_route": (_INT, [_W, _INT, _INT, _INT, _I64]),
     "xq_dense_route": (_INT, [_INT, _INT, _I64, _I64, _I64, _P]),
     # w, M, ldx, lora_A, lora_B, lora_dtype, r, plan (two int32)
     "xq_skinny_route": (_INT, [_W, _I64, _I64, _P, _P, _INT, _INT, _P]),

@@ -115,7 +115,7 @@ static inline int dense_tile_size(int64_t n_rows, int64_t Nout) {
 // expert: 4-bit banks, 64 or 128 experts 93 1.15, 187 1.04 to 1.08, 281 1.03 to 1.10, 421 0.97 to 0.99, 656 0.93; 16 experts 250
 // 1.10 to 1.14, 500 0.90; 8 experts 500 1.09 to 1.14, 750 0.87.  Block-fp8: 64 or 128 experts 46 1.14, 62 1.01, 93 1.04, 125 0.91, 281 0.87; 16
 // experts 125 1.00, 250 0.98, 500 0.81; 8 experts 125 1.23, 250 0.94, 750 0.87.
-// Block-fp8 and nvfp4 products whose sums are free (SumOrder::any): gemm_bank_kernel's 128 x 256 tiles, two on a compute unit, where there is one for every compute unit, half a tile an
+// `bank_tiles`, products of gemm_bank_kernel whose sums are free: its 128 x 256 tiles, two on a compute unit, where there is one for every compute unit, half a tile an
 // expert left empty, or for two in five where an expert's rows fill half of one (nvfp4) or most of one.  Routed MLP forward and backward, those
 // over 128 x 128 tiles, by rows an expert, block-fp8: 128 experts 2048/768 8 0.96, 24 0.95, 56 0.86, 96 0.84; 64 experts 2048/1024 6
 // 0.94, 16 0.95, 32 1.03, 64 0.92, 96 0.81; 64 experts 1280/640 6 1.10 and 16 1.02 (175 and 200 tiles), 32 0.99, 64 0.94; 32 experts 4096/1536 6
@@ -125,8 +125,8 @@ static inline int dense_tile_size(int64_t n_rows, int64_t Nout) {
 // 1.05, 32 0.99 (240 tiles), 64 0.91, 128 0.88, 600 0.78; 16 experts 2560/1024 32 1.05, 64 0.98 (128 tiles), 96 0.89, 256 0.82, 600 0.81.
 // (Tiles are counted without the empty part of an expert's last column tile: forwards of 8 and 16 experts 2816/1152, whose 1152 columns are
 // four and a half, block-fp8 90 tiles 1.12, 108 0.98, 130 0.95; nvfp4 90 1.15, 108 0.97, 130 0.91; 16 experts 1536/640 100 1.04 and 1.13.)
-static inline bool bank_large_tiles(int fmt, int64_t n_rows, int num_experts, int64_t Nout, SumOrder order) {
-    if (order == SumOrder::any && (fmt == XQ_FMT_FP8 || fmt == XQ_FMT_NVFP4)) {
+static inline bool bank_large_tiles(int fmt, int64_t n_rows, int num_experts, int64_t Nout, bool bank_tiles) {
+    if (bank_tiles) {
         using D = GeoBank<XQ_FMT_FP8>;
         const int64_t tiles = (xq_cdiv(n_rows, D::ROWS) + num_experts / 2) * Nout / D::COLS;
         return tiles >= (n_rows >= (fmt == XQ_FMT_FP8 ? 90ll : 60ll) * num_experts ? num_cus() * 13 / 32 : num_cus());
@@ -197,7 +197,7 @@ static DensePlan plan_dense(int64_t n_rows, int64_t Nout, int64_t nk) {
 static bool half_tiles(const DensePlan& p, int64_t n_rows, int64_t Nout, int64_t Kc, SumOrder order) {
     using D = GeoBank<XQ_FMT_FP8>;
     if (p.T != 256 || p.split != 1 || Kc <= 256) return false;
-    if (order == SumOrder::kept && (p.head_rows < n_rows || Kc > kDtlMaxK)) return false;
+    if (order == SumOrder::kept && p.head_rows < n_rows) return false;
     if (p.head_rows < n_rows) return p.tail_T == 128;
     const int64_t blocks = xq_cdiv(n_rows, D::ROWS) * xq_cdiv(Nout, D::COLS), slots = 2ll * num_cus();
     return blocks > slots && blocks % slots != 0 && blocks % slots <= slots / 2;
@@ -467,25 +467,53 @@ bool two_banks_supported(const xq_weight* w) {
     return w->format == XQ_FMT_FP8 && g_tile_policy != 1 && w->cols % 256 == 0 && w->cols >= 512 && w->num_experts >= 1;
 }
 
-// tile size of a grouped launch on the pipelined kernel
-static inline int bank_tile_size(int fmt, int64_t n_rows, int num_experts, int64_t Nout, SumOrder order) {
-    return g_tile_policy == 2 ? 256 : g_tile_policy == 3 ? 128 : bank_large_tiles(fmt, n_rows, num_experts, Nout, order) ? 256 : 128;
+// Whether gemm_bank_kernel takes a product over kc of rows of A within span_rows, lda apart: dense block-fp8, block-fp8 banks and nvfp4 banks in their
+// usual storage, three K-steps, an output in whole 16-byte pieces, operands within 32-bit byte offsets of a base (up to 3 KB further on).
+// Kept sums are gemm_dtl16_kernel's, block-fp8 as far as that kernel goes.  (nvfp4 banks under a forced tile size stay on gemm_256_kernel, whose
+// sums are the same for both sizes.)
+static bool bank_kernel_takes(const xq_weight* w, bool bank, int64_t kc, SumOrder order, int64_t span_rows, int64_t lda, const void* C, int64_t ldc, const void* bias) {
+    constexpr int64_t reach = (1ll << 32) - 4096;
+    const bool fp8 = w->format == XQ_FMT_FP8 && g_fp8_direct && g_tile_policy != 1 && (order == SumOrder::any || kc <= kDtlMaxK);
+    const bool f4 = bank && w->format == XQ_FMT_NVFP4 && w->layout == XQ_LAYOUT_GKN && w->group == 16 && w->scale_dtype == XQ_SCALE_E4M3 &&
+                    g_tile_policy == 0 && order == SumOrder::any;
+    return (fp8 || f4) && kc % BK == 0 && kc >= 3 * BK && w->cols % 16 == 0 && xq_aligned(w->packed, 16) && w->rows * w->cols < reach && span_rows > 0 &&
+           span_rows * lda * 2 < reach && xq_aligned(C, 16) && ldc % 8 == 0 && xq_aligned(bias, 8) && !(bank && bias);
+}
+// ... as far as the weight says: a bank's product with rows 16-byte aligned and few enough
+static bool bank_kernel_takes(const xq_weight* w, int64_t kc, SumOrder order) { return bank_kernel_takes(w, true, kc, order, 1, kc, nullptr, 8, nullptr); }
+
+// tile size of a grouped launch on the pipelined kernel, or (256, where it takes the launch) gemm_bank_kernel
+static inline int bank_tile_size(int fmt, int64_t n_rows, int num_experts, int64_t Nout, bool bank_tiles) {
+    return g_tile_policy == 2 ? 256 : g_tile_policy == 3 ? 128 : bank_large_tiles(fmt, n_rows, num_experts, Nout, bank_tiles) ? 256 : 128;
 }
 
 // ... of two banks' columns side by side: small tiles too where large ones do not divide a bank's columns and one bank alone would not take them
-static inline int side_by_side_tile(int fmt, int64_t n_rows, int num_experts, int64_t ncols, SumOrder order) {
-    const int T = bank_tile_size(fmt, n_rows, num_experts, 2 * ncols, order);
-    return ncols % T != 0 ? bank_tile_size(fmt, n_rows, num_experts, ncols, order) : T;
+static inline int side_by_side_tile(int fmt, int64_t n_rows, int num_experts, int64_t ncols, bool bank_tiles) {
+    const int T = bank_tile_size(fmt, n_rows, num_experts, 2 * ncols, bank_tiles);
+    return ncols % T != 0 ? bank_tile_size(fmt, n_rows, num_experts, ncols, bank_tiles) : T;
 }
 
 // Whether two 4-bit banks of one shape and storage take one launch whose output holds both products side by side, ncols columns
 // each (G256Args::W2): whole column tiles per bank.  One bank's tiles leave half of the block slots empty at some hundreds of
 // routed rows and end in a round of their own beyond (routed MLP, two launches and one, us: nf4 32 experts 2560/1024, 800 rows, forward and backward 510 and 461; nvfp4 64 experts 2048/1024, 9000 rows 886 and 816, forward alone of 6000 rows 350 and 305).
-bool banks_side_by_side(const xq_weight* a, const xq_weight* b, int64_t ncols, int64_t n_rows, SumOrder order) {
+bool banks_side_by_side(const xq_weight* a, const xq_weight* b, bool contract_cols, int64_t n_rows, SumOrder order) {
+    const int64_t ncols = contract_cols ? a->rows : a->cols;
+    const bool free = order == SumOrder::any && bank_kernel_takes(a, contract_cols ? a->cols : a->rows, order);
     return a->format != XQ_FMT_FP8 && tile_gemm_takes_row_map(a) && tile_gemm_takes_row_map(b) && a->format == b->format &&
            a->rows == b->rows && a->cols == b->cols && a->num_experts == b->num_experts && a->group == b->group &&
            a->scale_dtype == b->scale_dtype && xq_packed_bytes_per_expert(a) % 16 == 0 && xq_aligned(a->packed, 16) && xq_aligned(b->packed, 16) &&
-           ncols % side_by_side_tile(a->format, n_rows, a->num_experts, ncols, order) == 0;
+           ncols % side_by_side_tile(a->format, n_rows, a->num_experts, ncols, free) == 0;
+}
+
+extern "C" int xq_bank_route(const xq_weight* w, int forward, int joint, int kept, int64_t n_rows) {
+    if (!w || n_rows <= 0 || xq_validate_weight(w, "xq_bank_route") || !tile_gemm_takes_row_map(w)) return -1;
+    const bool one_sum = joint && !forward && w->format == XQ_FMT_FP8;
+    const int64_t nout = forward ? w->cols : w->rows, kc = (forward ? w->rows : w->cols) * (one_sum ? 2 : 1);
+    const SumOrder order = kept ? SumOrder::kept : SumOrder::any;
+    const bool ok = bank_kernel_takes(w, kc, order), free = ok && !kept;
+    const int T = joint && w->format != XQ_FMT_FP8 ? side_by_side_tile(w->format, n_rows, w->num_experts, nout, free)
+                                                   : bank_tile_size(w->format, n_rows, w->num_experts, nout * (joint && !one_sum ? 2 : 1), free);
+    return T == 128 ? XQ_BANK_TILES_128 : ok ? XQ_BANK_HALF_TILES : XQ_BANK_TILES_256;
 }
 
 // Whether the dgrad of two dense [N, K] weights of one shape may run as one launch (see launch_tile_gemm): block-fp8 on
@@ -633,7 +661,7 @@ static int launch_tile_gemm_t(const xq_weight* w, bool contract_cols, const bf16
                        "%s: the dense two-matrix form is the dgrad of two block-fp8 weights (out_features %% 128 == 0, >= 512)", who);
             g.Kc *= 2;
         } else {
-            XQ_REQUIRE((two_banks_supported(w) && two_banks_supported(two->w2)) || banks_side_by_side(w, two->w2, g.Nout, n_rows, order),
+            XQ_REQUIRE((two_banks_supported(w) && two_banks_supported(two->w2)) || banks_side_by_side(w, two->w2, contract_cols, n_rows, order),
                        "%s: a two-bank launch takes two block-fp8 expert banks (columns a multiple of 256) or two 4-bit ones (whole tiles)", who);
             XQ_REQUIRE(xq_aligned(two->su2, 16) && xq_aligned(two->lora_right2, 16) && two->a_off2 % 8 == 0, "%s: the second bank's operands must be 16-byte aligned", who);
             if (contract_cols && w->format == XQ_FMT_FP8) g.Kc *= 2;
@@ -670,8 +698,14 @@ static int launch_tile_gemm_t(const xq_weight* w, bool contract_cols, const bf16
                                       : w->layout == XQ_LAYOUT_FLAT));
         const DensePlan plan = plan_dense(n_rows, g.Nout, g.Kc / BK);
         const bool planned = !grouped && fmt_ok && g_tile_policy == 0 && force_T == 0 && !two_dense;   // two matrices: one unsplit launch
-        const int T = force_T ? force_T : grouped ? (two && w->format != XQ_FMT_FP8 ? side_by_side_tile(w->format, n_rows, w->num_experts, g.Nout / 2, order)
-                                                                         : bank_tile_size(w->format, n_rows, w->num_experts, g.Nout, order)) : g_tile_policy == 2 ? 256 : g_tile_policy == 3 ? 128 : plan.T;
+        const bool bank_ok = fmt_ok && bank_kernel_takes(w, grouped, g.Kc, order, a_rows_span, lda, C, ldc, bias), free = bank_ok && order == SumOrder::any;
+        int T = force_T ? force_T : g_tile_policy == 2 ? 256 : g_tile_policy == 3 ? 128 : plan.T;
+        if (grouped && two && w->format != XQ_FMT_FP8) {
+            T = side_by_side_tile(w->format, n_rows, w->num_experts, g.Nout / 2, free);
+            if (g.Nout / 2 % T != 0) T = 128;      // (joined by what the weights say, and rows that span too much for gemm_bank_kernel)
+        } else if (grouped) {
+            T = bank_tile_size(w->format, n_rows, w->num_experts, g.Nout, free);
+        }
         MidPlan mid;
         const bool by_size = planned || (two_dense && g_tile_policy == 0);
         // (its storages: the formats' usual groups and scale types; 32-bit offsets from a base for the operands)
@@ -708,10 +742,7 @@ static int launch_tile_gemm_t(const xq_weight* w, bool contract_cols, const bf16
             f.wide_rows = xq_aligned(C, 16) && ldc % 8 == 0 && xq_aligned(bias, 8);
             return launch_decoded(f, contract_cols, w->format, (uint8_t*)partial, stream, who);
         }
-        // (32-bit offsets from a base for the operands; whole 16-byte pieces of an output row)
-        const bool bank_storage = w->format == XQ_FMT_FP8 && g_fp8_direct && planned && g.right.f[1] == nullptr && n_rows * lda * 2 < (1ll << 32) - 4096 &&
-                                  (int64_t)g.wrows * g.wcols < (1ll << 32) - 4096 && g.wcols % 16 == 0 && xq_aligned(C, 16) && ldc % 8 == 0 && xq_aligned(bias, 8);
-        if (bank_storage && half_tiles(plan, n_rows, g.Nout, g.Kc, order)) {
+        if (planned && bank_ok && g.right.f[1] == nullptr && half_tiles(plan, n_rows, g.Nout, g.Kc, order)) {
             using D = GeoBank<XQ_FMT_FP8>;
             G256Args f{};
             f.A = A; f.lda = lda; f.C = C; f.ldc = ldc;
@@ -772,24 +803,18 @@ static int launch_tile_gemm_t(const xq_weight* w, bool contract_cols, const bf16
             int rc;
             // block-fp8, and nvfp4 banks, on large unsplit tiles: the kernels that bring both operand tiles straight into LDS and decode after the fragment
             // read, one block per tile (dense xq_gemm_dtl.h, expert banks xq_gemm_bank.h)
-            const int nk_all = g.Kc / BK;
             // (two matrices: the second one starts on a scale-block boundary of the contraction, or -- two banks side by side -- on a
-            // tile boundary of the columns.  nvfp4 banks under a forced tile size, or whose order of sums is kept, stay on gemm_256_kernel,
-            // whose sums are the same for both sizes; block-fp8 ones have gemm_dtl16_kernel's order and its limit here.)
+            // tile boundary of the columns)
             const bool side_by_side = grouped && (!contract_cols || w->format != XQ_FMT_FP8);
-            const bool two_ok = !two || (side_by_side ? f.ncols1 % 256 == 0 : (f.nk1 % 2 == 0 && f.nk1 >= 2));
-            const int64_t reach = (1ll << 32) - (grouped ? 4096 : 0);
-            const bool storage = w->format == XQ_FMT_FP8 || (grouped && w->format == XQ_FMT_NVFP4 && g_tile_policy == 0 && order == SumOrder::any && g.group == 16 && g.scale_dtype == XQ_SCALE_E4M3);
-            const bool direct = g_fp8_direct && storage && T == 256 && ksplit == 1 && nk_all >= 3 && two_ok &&
-                                // (their lanes address their operands by 32-bit byte offsets from a base, the bank kernel's up to 3 KB further on)
-                                a_rows_span > 0 && a_rows_span * lda * 2 < reach && (int64_t)g.wrows * g.wcols < reach;
-            if (direct && grouped && g.wcols % 16 == 0 && f.wide_rows && !bias && (order == SumOrder::any || g.Kc <= kDtlMaxK)) {
+            const bool large = T == 256 && ksplit == 1 && (!two || (side_by_side ? f.ncols1 % 256 == 0 : (f.nk1 % 2 == 0 && f.nk1 >= 2)));
+            if (large && grouped && bank_ok) {
                 using D = GeoBank<XQ_FMT_FP8>;
                 f.tiles_m = (int32_t)(xq_cdiv(n_rows, D::ROWS) + w->num_experts);
                 f.tiles_n = (int32_t)xq_cdiv(g.Nout, D::COLS);
                 f.tile_prefix = tile_offsets;                // (its tiles have 128 rows)
                 rc = launch_bank(f, w->format, contract_cols, stream, who);
-            } else if (direct && !grouped && nk_all <= 2 * GeoDtl::SCL_MAX)
+            } else if (large && !grouped && w->format == XQ_FMT_FP8 && g_fp8_direct && g.Kc >= 3 * BK && g.Kc <= kDtlMaxK &&
+                       n_rows * lda * 2 < (1ll << 32) && (int64_t)g.wrows * g.wcols < (1ll << 32))      // (32-bit byte offsets from a base)
                 rc = launch_dtl16(f, contract_cols, dim3((unsigned)(tiles_m * tiles_n)), stream, who);
             else if (w->format == XQ_FMT_FP8) rc = launch_256<XQ_FMT_FP8>(f, contract_cols, grouped, T, grid, stream, who);
             else if (w->format == XQ_FMT_INT4) rc = launch_256<XQ_FMT_INT4>(f, contract_cols, grouped, T, grid, stream, who);
@@ -879,14 +904,12 @@ bool gate_up_side_by_side(const xq_weight* wg, const xq_weight* wu, const bf16_t
                           const bf16_t* bias_u, const bf16_t* gu, int64_t ldgu) {
     using D = GeoBank<XQ_FMT_FP8>;
     const int64_t I = wg->rows, K = wg->cols;
-    if (!g_fp8_direct || g_tile_policy != 0 || wg->format != XQ_FMT_FP8 || wu->format != XQ_FMT_FP8 || wu->rows != I || wu->cols != K ||
-        wg->scale_dtype != XQ_SCALE_F32 || wu->scale_dtype != XQ_SCALE_F32 || I % 16 != 0 || K % D::BK != 0 || K < 3 * D::BK || M <= 64 || ldx % 8 != 0 || !xq_aligned(x, 16) || ldgu % 8 != 0 ||
-        !xq_aligned(gu, 16) || !xq_aligned(wg->packed, 16) || !xq_aligned(wu->packed, 16) || !xq_aligned(bias_g, 8) || !xq_aligned(bias_u, 8) ||
-        // (32-bit offsets from a base for the operands)
-        M * ldx * 2 >= (1ll << 32) - 4096 || I * K >= (1ll << 32) - 4096)
+    if (g_tile_policy != 0 || wg->format != XQ_FMT_FP8 || wu->format != XQ_FMT_FP8 || wu->rows != I || wu->cols != K || I % 16 != 0 || M <= 64 ||
+        ldx % 8 != 0 || !xq_aligned(x, 16) || !bank_kernel_takes(wg, false, K, SumOrder::kept, M, ldx, gu, ldgu, bias_g) ||
+        !bank_kernel_takes(wu, false, K, SumOrder::kept, M, ldx, gu, ldgu, bias_u))
         return false;
     MidPlan mid;
-    if (K > kDtlMaxK || takes_mid(XQ_FMT_FP8, true, M, I, K, &mid) || decode_first(XQ_FMT_FP8, M, I, K)) return false;
+    if (takes_mid(XQ_FMT_FP8, true, M, I, K, &mid) || decode_first(XQ_FMT_FP8, M, I, K)) return false;
     const DensePlan p = plan_dense(M, I, K / BK);
     if (p.T != 256 || p.split != 1 || p.head_rows < M) return false;
     const int64_t blocks = 2 * xq_cdiv(M, D::ROWS) * xq_cdiv(I, D::COLS), slots = 2ll * num_cus();

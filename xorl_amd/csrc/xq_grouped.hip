@@ -90,8 +90,8 @@ int64_t bwd_workspace(const Dims& d) {
 // The sums of gate, up and the dgrad of down are kept: all six factor gradients and the routing weights' are computed from them.  The forward
 // of down and the dgrads of gate and up only leave as bf16 (y, dx), and so does a whole forward that no backward follows.
 bool fuse_gate_up(const xq_weight* gate, const xq_weight* up) { return two_banks_supported(gate) && two_banks_supported(up); }
-bool joint_forward(const xq_weight* gate, const xq_weight* up, int64_t R, SumOrder order) { return fuse_gate_up(gate, up) || banks_side_by_side(gate, up, gate->cols, R, order); }
-bool joint_dgrads(const xq_weight* gate, const xq_weight* up, int64_t R) { return banks_side_by_side(gate, up, gate->rows, R, SumOrder::any); }
+bool joint_forward(const xq_weight* gate, const xq_weight* up, int64_t R, SumOrder order) { return fuse_gate_up(gate, up) || banks_side_by_side(gate, up, false, R, order); }
+bool joint_dgrads(const xq_weight* gate, const xq_weight* up, int64_t R) { return banks_side_by_side(gate, up, true, R, SumOrder::any); }
 
 }  // namespace
 }  // namespace xq

@@ -207,7 +207,7 @@ struct TwoBanks {
 int64_t tile_gemm_split_bytes(int64_t n_rows, int64_t Nout, int64_t Kc);     // split-K scratch a dense launch may want
 int64_t tile_gemm_partial_bytes(int fmt, int64_t n_rows, int64_t Nout, int64_t Kc);   // ... or the decoded image of a weight of that format (< 0: of any)
 bool two_banks_supported(const xq_weight* w);
-bool banks_side_by_side(const xq_weight* a, const xq_weight* b, int64_t ncols, int64_t n_rows, SumOrder order);
+bool banks_side_by_side(const xq_weight* a, const xq_weight* b, bool contract_cols, int64_t n_rows, SumOrder order);
 bool two_dense_supported(const xq_weight* w);   // dense [N, K] pair: one dgrad launch, dX = [dY1 | dY2] . [W1 ; W2]
 int launch_gate_up_swiglu(const xq_weight* wg, const xq_weight* wu, const bf16_t* x, int64_t ldx, int64_t M,
                           const bf16_t* su_g, const bf16_t* su_u, int64_t ld_su, const LowRankRight& right,

@@ -140,10 +140,11 @@ int xq_skinny_route(const xq_weight* w, int64_t M, int64_t ldx, const void* lora
  * no counterpart in the reference. */
 int xq_set_persistent_tiles(int enabled);
 
-/* Dense block-fp8 products on 256 x 256 tiles (forward, dgrad; unsplit) run on the kernel that loads both operand tiles
- * straight into LDS, keeps the weight tile as e4m3 bytes there and multiplies with v_mfma_f32_16x16x32_bf16 (enabled = 1,
- * the default), or on the tile kernel that every other format and the expert banks use (enabled = 0, which also keeps dense
- * block-fp8 products off the kernels that decode in registers and over a decoded image).  All decode to the reference's bf16
+/* Block-fp8 products on large unsplit tiles (forward, dgrad; dense and expert banks; gate and up of a dense MLP as one launch) run on
+ * the kernels that load both operand tiles straight into LDS, keep the weight tile as e4m3 bytes there and multiply with
+ * v_mfma_f32_16x16x32_bf16 (enabled = 1, the default), or on the tile kernel that the other formats use (enabled = 0, which also
+ * keeps dense block-fp8 products off the kernels that decode in registers and over a decoded image, and gives expert banks the
+ * tile sizes of that kernel).  Other formats do not depend on it, nvfp4 banks, which share one of these kernels, included.  All decode to the reference's bf16
  * values bit for bit; their sums run in different orders, so outputs agree to rounding.  A process-wide
  * switch for tests and A/B measurements (XQ_FP8_DIRECT in the environment sets it at load time); no counterpart in the
  * reference. */

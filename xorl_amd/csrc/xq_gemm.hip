@@ -48,8 +48,8 @@ static int launch_256_one(const G256Args& f, dim3 grid, hipStream_t s, const cha
     return XQ_OK;
 }
 
-// Block-fp8 launches on large unsplit tiles run gemm_dtl16_kernel (dense) and gemm_bank_kernel (expert banks, some dense ones; 1, the default) or gemm_256_kernel (0): a
-// process-wide switch for tests and A/B measurements, XQ_FP8_DIRECT in the environment sets it at load time.
+// Block-fp8 launches on large unsplit tiles run gemm_dtl16_kernel (dense) and gemm_bank_kernel (expert banks, some dense ones; 1, the default)
+// or gemm_256_kernel (0): a process-wide switch for tests and A/B measurements, XQ_FP8_DIRECT in the environment sets it at load time.
 static std::atomic<int> g_fp8_direct{[] { const char* e = getenv("XQ_FP8_DIRECT"); return e ? atoi(e) : 1; }()};
 
 constexpr int64_t kDtlMaxK = 2ll * GeoDtl::SCL_MAX * GeoDtl::BK;      // the longest contraction that gemm_dtl16_kernel takes

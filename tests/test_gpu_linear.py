@@ -508,3 +508,17 @@ def test_dense_half_tiles(hip_device, M, K, N, r, forward):
         close(got, ref, TOL)
         close(got[M // 128 * 128:], ref[M // 128 * 128:], TOL)
         close(got[:, got.shape[1] // 256 * 256:], ref[:, got.shape[1] // 256 * 256:], TOL)
+
+
+@pytest.mark.parametrize("M,K,N,r,forward", [(1912, 192, 9408, 16, True), (4101, 256, 9344, 24, True), (2911, 11840, 256, 8, False)])
+def test_dense_half_tiles_over_short_contractions(hip_device, M, K, N, r, forward):
+    """Three and four K-steps, where large tiles would leave a second launch of small ones: against the float64 form, and the tiles' last rows."""
+    n_out, k = (N, K) if forward else (K, N)
+    assert dense_route("block_fp8", forward, M, n_out, k) == ("tiles", 128, 256, 1, 0, 0, 0)
+    m, w_ref = make_dense_module("block_fp8", N, K, r, 32, seed=M + r, device=hip_device, bias=True)
+    x, dy = gen((M, K), 1.0, 31, torch.bfloat16), gen((M, N), 1.0, 32, torch.bfloat16)
+    y, dx, _, _ = _run(m, x.to(hip_device), dy.to(hip_device))
+    ex = R.linear_fwd_bwd_exact(x, w_ref, m.lora_A.detach().cpu(), m.lora_B.detach().cpu(), m.scaling, dy, bias=m.bias.detach().cpu())
+    for got, ref in ((y.cpu(), ex["y"]), (dx.cpu(), ex["dx"])):
+        close(got, ref, TOL)
+        close(got[M // 128 * 128:], ref[M // 128 * 128:], TOL)

@@ -191,12 +191,14 @@ static DensePlan plan_dense(int64_t n_rows, int64_t Nout, int64_t nk) {
 // is filled to 0.3 .. 0.5 0.80 to 0.93 ([12288, 4096], 2048 rows 204 -> 172 us); to 0.53 1.00 to 1.09, to 0.6 .. 0.9 1.00 to 1.08.  Two
 // launches, the second of 128 x 128 tiles: 0.77 to 0.99, 0.86 in the mean ([7552, 512], 2595 rows 43.9 -> 33.9 us).  Where K splits take the
 // last round (0.90 to 1.07), or gemm_mid_kernel the product (0.86 to 1.14), neither is the better.
-// (Contractions of 256 and less keep the two launches, though they take 0.79 to 0.97 here too: what tests that form.)
+// Contractions of 192 and 256 likewise (24 products, 0.79 to 0.95), and up to an eighth of a round beyond whole ones (48 products over 192 .. 1536
+// k, 0.85 to 0.98).  (A few rows beyond whole tile rows, over such a short contraction, keep the two launches: the form that a test asks for by its
+// sizes, [4096, 256], 4100 rows 34.3 us, 32.2 here.)
 // The sums are gemm_dtl16_kernel's, whose place these tiles take in a whole launch; rows that would be a launch of 128 x 128 tiles are summed in
 // another order (gemm_256_kernel).
 static bool half_tiles(const DensePlan& p, int64_t n_rows, int64_t Nout, int64_t Kc, SumOrder order) {
     using D = GeoBank<XQ_FMT_FP8>;
-    if (p.T != 256 || p.split != 1 || Kc <= 256) return false;
+    if (p.T != 256 || p.split != 1 || (Kc <= 256 && p.head_rows < n_rows && n_rows - p.head_rows <= 16)) return false;
     if (order == SumOrder::kept && p.head_rows < n_rows) return false;
     if (p.head_rows < n_rows) return p.tail_T == 128;
     const int64_t blocks = xq_cdiv(n_rows, D::ROWS) * xq_cdiv(Nout, D::COLS), slots = 2ll * num_cus();

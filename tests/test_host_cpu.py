@@ -299,3 +299,33 @@ def test_banks_get_the_tiles_of_the_kernel_that_takes_them():
     # 640 columns are no whole tiles of 256: two banks side by side take small ones where one alone does ((4 + 64) 640 / 256 tiles, of 256)
     assert bank_route("nvfp4", E, H, 640, 64 * E, True) == "half"
     assert bank_route("nvfp4", E, H, 640, 4 * E, True) == bank_route("nvfp4", E, H, 640, 4 * E, True, joint=True) == "128"
+
+
+@pytest.mark.parametrize("M,joint", [(1000, True), (300, False)])
+@pytest.mark.parametrize("field", ["su_gate_up", "su_down"])
+def test_mlp_forward_refuses_misaligned_intermediates(M, joint, field):
+    """Before anything is launched, whether gate and up share a launch or not (a call that reaches the device would not fail by this message)."""
+    import ctypes
+
+    from tests.util_cases import gate_up_joint
+    from xorl_amd import _C
+
+    H, I, r = 320, 9280, 8
+    assert gate_up_joint(M, H, I) == joint
+
+    def weight(n, k):
+        w = _C.XqWeight()
+        w.format, w.layout, w.rows, w.cols, w.num_experts, w.group, w.scale_dtype = _C.FORMATS["block_fp8"], _C.XQ_LAYOUT_FLAT, n, k, 1, 128, _C.XQ_SCALE_F32
+        w.packed = w.scales = 4096
+        return w
+    ws = [weight(I, H), weight(I, H), weight(H, I)]
+    lora, S = _C.XqMlpLora(), _C.XqMlpSaved()
+    for p in range(3):
+        lora.A[p] = lora.B[p] = 4096
+    lora.dtype, lora.r, lora.scaling = _C.XQ_DT_F32, r, 1.0
+    S.gate_up = S.h = S.su_gate_up = S.su_down = 4096
+    setattr(S, field, 4096 + 8)
+    L = _C.lib()
+    with pytest.raises(_C.XqError, match="su_gate_up and su_down .* 16-byte aligned"):
+        _C.check(L.xq_mlp_fwd(*(ctypes.byref(w) for w in ws), ctypes.byref(lora), 4096, H, M, 4096, H, ctypes.byref(S), 4096,
+                              L.xq_mlp_workspace_bytes(M, H, I, r, 0), None))

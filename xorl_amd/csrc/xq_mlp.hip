@@ -178,6 +178,9 @@ extern "C" int xq_mlp_fwd(const xq_weight* gate, const xq_weight* up, const xq_w
     XQ_REQUIRE(workspace && xq_aligned(workspace, 256) && workspace_bytes >= fwd_workspace(d, -1, true),
                "%s: workspace missing, misaligned or smaller than xq_mlp_workspace_bytes()", who);
     XQ_REQUIRE(ldy % 8 == 0 && xq_aligned(y, 16), "%s: y rows must be 16-byte aligned", who);
+    // (before anything runs, and for whichever launches read them)
+    XQ_REQUIRE(d.rp == 0 || (xq_aligned(saved->su_gate_up, 16) && xq_aligned(saved->su_down, 16)),
+               "%s: su_gate_up and su_down of xq_mlp_saved must be 16-byte aligned", who);
     hipStream_t stream = (hipStream_t)stream_;
     const bf16_t* x = (const bf16_t*)x_;
     const int r = d.r, rp = d.rp;
@@ -222,7 +225,7 @@ extern "C" int xq_mlp_fwd(const xq_weight* gate, const xq_weight* up, const xq_w
                                         LowRankRight{{lora->B[0], lora->B[1]}, r, r, rp, f32, 0}, rp, bias_g, bias_u, gu, 2 * I, h, I, stream)))
             return rc;
     } else {
-        if (xq_aligned(su_gu, 16) && gate_up_side_by_side(gate, up, x, ldx, M, bias_g, bias_u, gu, 2 * I)) {      // (what it does not take, two launches take or refuse)
+        if (gate_up_side_by_side(gate, up, x, ldx, M, bias_g, bias_u, gu, 2 * I)) {      // (what it does not take, two launches take or refuse)
             if ((rc = launch_gate_up(gate, up, x, ldx, M, su_gu, rp ? su_gu + sl.up_offset : nullptr, sl.pitch, LowRankRight{{lora->B[0], lora->B[1]}, r, r, rp, f32, 0}, rp,
                                      bias_g, bias_u, gu, 2 * I, stream, who))) return rc;
         } else {

@@ -269,12 +269,12 @@ def _by_itself(m, x, dy, route):
     return got[0] if len(got) == 1 else tuple(torch.cat([a[:route[0]], b[route[0]:]]) for a, b in zip(*got))
 
 
-@pytest.mark.parametrize("M,H,I,r,fwd,bwd,joint", [
-    (129, 192, 9280, 8, 128, "mid", False), (300, 448, 9280, 64, "mid", "mid", False),
-    (1500, 384, 13120, 32, (1024, 476), (1024, 476), False),      # whole rounds of large tiles, the other rows on small ones
-    (1000, 320, 9280, 16, 256, 256, True), (2300, 256, 12352, 24, 256, 256, True),
+@pytest.mark.parametrize("M,H,I,r,fwd,bwd,joint,bias", [
+    (129, 192, 9280, 8, 128, "mid", False, False), (300, 448, 9280, 64, "mid", "mid", False, False),
+    (1500, 384, 13120, 32, (1024, 476), (1024, 476), False, False),      # whole rounds of large tiles, the other rows on small ones
+    (1000, 320, 9280, 16, 256, 256, True, False), (1000, 320, 9280, 64, 256, 256, True, True), (2300, 256, 12352, 24, 256, 256, True, True),
 ])
-def test_mlp_products_sum_as_by_themselves(hip_device, M, H, I, r, fwd, bwd, joint):
+def test_mlp_products_sum_as_by_themselves(hip_device, M, H, I, r, fwd, bwd, joint, bias):
     """Gate, up and the dgrad of down, joint launch or not, are the bits of the same products by themselves on the kernels that their sizes
     choose.  Behind them: an fp32 factor gradient of gate, against float64 sums of the bf16 values that those bits give (fp32 sums
     of M products err by some sqrt(M) 2^-24; a flipped bf16 rounding in one value of a few hundred is 1e-4)."""
@@ -286,11 +286,11 @@ def test_mlp_products_sum_as_by_themselves(hip_device, M, H, I, r, fwd, bwd, joi
         # (a product by itself whose rows would be two launches, the second of small tiles, is free to be one of half tiles)
         assert here[0] == "mid" if route == "mid" else here[:3] == ("tiles", 128, 256) if isinstance(route, tuple) else here == ("tiles", route, route, 1, 0, 0, 0)
     assert gate_up_joint(M, H, I) == joint
-    mods, w_ref = _mods("block_fp8", H, I, r, hip_device, seed=M)
+    mods, w_ref = _mods("block_fp8", H, I, r, hip_device, bias=bias, seed=M)
     x, dy = gen((M, H), 1.0, 95, torch.bfloat16).to(hip_device), gen((M, H), 1.0, 96, torch.bfloat16).to(hip_device)
     m3 = [mods[k] for k in ("gate", "up", "down")]
     factors = [t.detach() for m in m3 for t in (m.lora_A, m.lora_B)]
-    _, saved = F._mlp_fwd_impl(x, factors, (None,) * 3, [m._quant_weight() for m in m3], r, m3[0].scaling, 0)
+    _, saved = F._mlp_fwd_impl(x, factors, [m.bias.detach().to(torch.bfloat16) if bias else None for m in m3], [m._quant_weight() for m in m3], r, m3[0].scaling, 0)
     zero = torch.zeros(M, I, dtype=torch.bfloat16, device=hip_device)
     g, u = (_by_itself(m, x, zero, fwd)[0] for m in m3[:2])
     assert torch.equal(saved[0], torch.cat([g, u], 1))
@@ -304,7 +304,7 @@ def test_mlp_products_sum_as_by_themselves(hip_device, M, H, I, r, fwd, bwd, joi
     rp = saved[2].shape[1] // 2
     want = dg.double().t() @ saved[2].flatten()[:M * rp].view(M, rp)[:, :r].double()
     assert float((dB.double() - want).norm() / want.norm()) <= 2e-5
-    if joint:
+    if joint and not bias:
         loras = {k: (m.lora_A.detach().cpu(), m.lora_B.detach().cpu()) for k, m in mods.items()}
         ex = R.mlp_fwd_bwd_exact(x.cpu(), w_ref["gate"], w_ref["up"], w_ref["down"], loras, m3[0].scaling, dy.cpu())
         close(y.detach().cpu(), ex["y"], TOL)

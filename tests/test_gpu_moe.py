@@ -8,7 +8,7 @@ import torch
 from oracle import cdecode as C
 from oracle import decode_np as NP
 from oracle import recipe as R
-from tests.util_cases import banks_joint, close, bits_to_bf16, gen
+from tests.util_cases import bank_route, banks_joint, bits_to_bf16, close, gen
 
 pytestmark = pytest.mark.gpu
 TOL = 1e-2
@@ -1028,3 +1028,104 @@ def test_forward_that_no_backward_follows(hip_device, fmt, E, T, topk, H, I, r, 
     ex = R.moe_fwd_bwd(x, rw, sel, ref["gate"], ref["up"], ref["down"], lora, m.scaling, torch.zeros_like(x))
     close(y.cpu(), ex["y"], TOL)
     close(m(xd.requires_grad_(True), rwd, seld).detach().cpu(), ex["y"], TOL)
+
+
+@pytest.mark.parametrize("fmt", ["block_fp8", "nvfp4"])
+def test_bank_tiles_decode_bit_exact(hip_device, fmt):
+    """Identity rows, many enough for gemm_bank_kernel by size: both directions return the oracle's decoded banks bit for bit (up to the sign of
+    zero), as test_grouped_gemm_decode_bit_exact has it for the forced kernels."""
+    from xorl_amd import moe_functional as MF
+
+    E, H, I = 8, 512, 1024
+    m, banks = _make_experts(fmt, E, H, I, 8, False, seed=61, device=hip_device)
+    for proj, (K, N) in (("gate", (H, I)), ("down", (I, H))):
+        ref = banks[proj].to(hip_device)
+        for transpose_w, rows in ((False, K), (True, N)):
+            assert bank_route(fmt, E, K, N, E * rows, not transpose_w) == "half"
+            sel = torch.arange(E, dtype=torch.int32).repeat_interleave(rows).reshape(-1, 1).to(hip_device)
+            _, offsets, _, tile_offsets = MF.route_build(sel, E)
+            a = torch.eye(rows, dtype=torch.bfloat16, device=hip_device).repeat(E, 1)
+            y = MF._grouped_gemm(m._bank(proj), transpose_w, a, offsets, tile_offsets, None, None)
+            want = (ref.transpose(1, 2) if transpose_w else ref).reshape(E * rows, -1).contiguous()
+            assert bool(((y.view(torch.int16) == want.view(torch.int16)) | ((y.float() == 0) & (want.float() == 0))).all()), (proj, transpose_w)
+
+
+@pytest.mark.parametrize("E,T,topk,H,I,r,hybrid", [
+    (12, 1500, 4, 512, 512, 16, False),       # gate and up joint in both directions
+    (12, 1500, 4, 768, 512, 24, True),        # ... with factors shared by all experts
+    (16, 1300, 4, 576, 832, 40, False),       # widths that are no whole tiles: launches of one bank
+])
+def test_nvfp4_banks_by_size_vs_oracle(hip_device, E, T, topk, H, I, r, hybrid):
+    """nvfp4 banks on gemm_bank_kernel, gate and up of different magnitude (their global scales differ by 4): y of a forward alone, y and dx of
+    one with a backward, and every gradient, against the float64 program."""
+    R_, joint = T * topk, H % 256 == 0 and I % 256 == 0
+    assert bank_route("nvfp4", E, H, I, R_, True, joint=joint) == bank_route("nvfp4", E, I, H, R_, True) == bank_route("nvfp4", E, H, I, R_, False, joint=joint) == "half"
+    assert banks_joint("nvfp4", E, H, I, R_, 2) == banks_joint("nvfp4", E, H, I, R_, 0) == joint
+    m, _ = _make_experts("nvfp4", E, H, I, r, hybrid, seed=E + H, device="cpu")
+    m.load_weights(gen((E, H, I), 0.05, E), gen((E, H, I), 0.0125, E + 1), gen((E, I, H), 0.05, E + 2))
+    m = m.to(hip_device)
+    banks = {p: m.dequantize_all_experts(p, *m._proj_dims(p)).to(torch.bfloat16).cpu() for p in ("gate", "up", "down")}     # (bit-exact: test_moe_fwd_bwd_vs_oracle)
+    rw, sel = _zipf_routing(T, E, topk, seed=7)
+    rw, seld = rw.to(torch.bfloat16), sel.to(hip_device)
+    x, dy = gen((T, H), 1.0, 8, torch.bfloat16), gen((T, H), 1.0, 9, torch.bfloat16)
+    xd, rwd = x.to(hip_device).requires_grad_(True), rw.to(hip_device).requires_grad_(True)
+    lora = {k: (getattr(m, f"{k}_proj_lora_A").detach().cpu(), getattr(m, f"{k}_proj_lora_B").detach().cpu()) for k in ("gate", "up", "down")}
+    ex = R.moe_fwd_bwd(x, rw, sel, banks["gate"], banks["up"], banks["down"], lora, m.scaling, dy)
+    with torch.no_grad():
+        close(m(xd, rwd, seld).cpu(), ex["y"], TOL)
+    y = m(xd, rwd, seld)
+    y.backward(dy.to(hip_device))
+    close(y.detach().cpu(), ex["y"], TOL)
+    close(xd.grad.cpu(), ex["dx"], TOL)
+    close(rwd.grad.cpu(), ex["d_routing"], 2e-2, rows="none")
+    for k in ("gate", "up", "down"):
+        close(getattr(m, f"{k}_proj_lora_A").grad.cpu(), ex[f"dA_{k}"], TOL, rows="first")
+        close(getattr(m, f"{k}_proj_lora_B").grad.cpu(), ex[f"dB_{k}"], TOL, rows="first")
+
+
+@pytest.mark.parametrize("tile_policy", [2], indirect=True)
+@pytest.mark.parametrize("I", [4352, 8448])     # the change of bank before and behind the first load of 64 more scales (K-steps 68 and 132 of 136 and 264)
+def test_one_sum_over_two_long_fp8_banks(hip_device, tile_policy, I):
+    """The dgrad of gate and up as one sum over more K-steps than a register holds block scales of: dx against the float64 program."""
+    E, T, topk, H, r = 3, 200, 2, 256, 8
+    m, banks = _make_experts("block_fp8", E, H, I, r, False, seed=I, device="cpu")
+    # (block scales that differ along the contraction)
+    m.load_weights(*(b.float() * torch.linspace(0.25, 1.75, I) for b in (banks["gate"], banks["up"])), banks["down"].float())
+    m = m.to(hip_device)
+    banks = {p: m.dequantize_all_experts(p, *m._proj_dims(p)).to(torch.bfloat16).cpu() for p in banks}
+    rw, sel = _zipf_routing(T, E, topk, seed=7, empty=0)
+    rw = rw.to(torch.bfloat16)
+    x, dy = gen((T, H), 1.0, 8, torch.bfloat16), gen((T, H), 1.0, 9, torch.bfloat16)
+    xd = x.to(hip_device).requires_grad_(True)
+    y = m(xd, rw.to(hip_device), sel.to(hip_device))
+    dx = torch.autograd.grad(y, xd, dy.to(hip_device))[0]
+    lora = {k: (getattr(m, f"{k}_proj_lora_A").detach().cpu(), getattr(m, f"{k}_proj_lora_B").detach().cpu()) for k in ("gate", "up", "down")}
+    ex = R.moe_fwd_bwd(x, rw, sel, banks["gate"], banks["up"], banks["down"], lora, m.scaling, dy)
+    close(y.detach().cpu(), ex["y"], TOL)
+    close(dx.cpu(), ex["dx"], TOL)
+
+
+def test_nvfp4_storages_agree_where_one_has_tiles_of_its_own(hip_device):
+    """e4m3 block scales take gemm_bank_kernel by size, the same scales folded to fp32 do not: what fp32 gradients come from keeps one order of
+    sums in both (the same bits), y and dx agree to a bf16 step of the largest entry."""
+    E, T, topk, H, I, r = 12, 1500, 4, 512, 512, 16
+    assert bank_route("nvfp4", E, H, I, T * topk, False, joint=True) == "half"
+    ms = [_make_experts("nvfp4", E, H, I, r, False, seed=90, device=hip_device)[0] for _ in range(2)]
+    for p in ("gate", "up", "down"):
+        bs = getattr(ms[0], f"{p}_block_scales").view(torch.float8_e4m3fn).float()
+        g = getattr(ms[0], f"{p}_global_scale").contiguous().view(torch.float32).reshape(E, 1, 1)
+        setattr(ms[1], f"{p}_block_scales", ms[1]._to_uint8((bs * g).contiguous()))
+        setattr(ms[1], f"{p}_global_scale", ms[1]._to_uint8(torch.ones(E, 1, dtype=torch.float32, device=hip_device)))
+        ms[1]._scale_dtypes[p] = {"weight_block_scales": torch.float32, "weight_global_scale": torch.float32}
+    rw, sel = _zipf_routing(T, E, topk, seed=5, empty=0)
+    rw, sel = rw.to(hip_device), sel.to(hip_device)
+    x, dy = gen((T, H), 1.0, 6, torch.bfloat16).to(hip_device), gen((T, H), 1.0, 7, torch.bfloat16).to(hip_device)
+    got = []
+    for m in ms:
+        xd, rwd = x.clone().requires_grad_(True), rw.clone().requires_grad_(True)
+        y = m(xd, rwd, sel)
+        got.append([y.detach(), *torch.autograd.grad(y, [xd, rwd, *m.get_lora_parameters()], dy)])
+    for a, b in list(zip(*got))[2:]:
+        assert torch.equal(a, b)
+    for a, b in list(zip(*got))[:2]:
+        assert R.max_rel_err(a.float().cpu(), b.double().cpu()) <= 2 ** -7

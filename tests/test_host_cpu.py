@@ -329,3 +329,15 @@ def test_mlp_forward_refuses_misaligned_intermediates(M, joint, field):
     with pytest.raises(_C.XqError, match="su_gate_up and su_down .* 16-byte aligned"):
         _C.check(L.xq_mlp_fwd(*(ctypes.byref(w) for w in ws), ctypes.byref(lora), 4096, H, M, 4096, H, ctypes.byref(S), 4096,
                               L.xq_mlp_workspace_bytes(M, H, I, r, 0), None))
+
+
+def test_bank_tile_tests_reach_the_kernel():
+    """The shapes of tests/test_gpu_moe.py::test_bank_tiles_vs_fp32 in both directions (three, four, seven and 130 K-steps forward: the last loads
+    block scales twice)."""
+    from tests.util_cases import bank_route
+
+    counts = [128, 0, 1, 127, 129, 16, 113, 300, 0, 240] * 8
+    for K, N in ((192, 320), (256, 832), (448, 768), (8320, 256)):
+        here = counts + [0, 300] * 100 if K == 192 else counts
+        for fmt in ("block_fp8", "nvfp4"):
+            assert [bank_route(fmt, len(here), K, N, sum(here), fwd) for fwd in (True, False)] == ["half", "half"], (fmt, K, N)

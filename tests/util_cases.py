@@ -123,7 +123,7 @@ def bank_route(fmt, E, K, N, n_rows, forward, joint=False, kept=False, scale_dty
 
 
 def banks_joint(fmt, E, H, I, n_rows, forward) -> bool:
-    """xq_grouped_joint (include/xq.h) of gate and up banks [E, H, I] in a format's usual storage"""
+    """xq_grouped_joint (include/xq.h) of gate and up banks [E, H, I] in a format's usual storage; forward 2: one that no backward follows"""
     import ctypes
 
     from xorl_amd import _C

@@ -528,10 +528,6 @@ typedef struct xq_grouped_saved {
     int32_t* counts;
     const void* x_tokens;      /* backward, when xs is NULL: the forward's hidden [n_tokens, H] bf16 */
     int64_t ld_x_tokens;
-    /* forward: != 0 where no backward follows.  Its sums may then run in whatever order is the shortest way (the output agrees to rounding);
-     * a forward that a backward follows keeps one order, on which fp32 gradients depend. */
-    int32_t forward_only;
-    int32_t reserved;
 } xq_grouped_saved;
 
 typedef struct xq_grouped_grads {
@@ -542,7 +538,7 @@ typedef struct xq_grouped_grads {
 int64_t xq_grouped_workspace_bytes(int64_t n_tokens, int32_t topk, int32_t num_experts, int64_t hidden,
                                    int64_t intermediate, int r, int backward);
 int xq_grouped_in_place(const xq_weight* gate, const xq_weight* up, const xq_weight* down);
-/* Whether gate and up of n_rows routed rows run as one launch, for tests: their forwards (forward 1; 2: xq_grouped_saved::forward_only), or, as two
+/* Whether gate and up of n_rows routed rows run as one launch, for tests: their forwards (forward 1; 2: xq_grouped_fwd_eval_ids), or, as two
  * products of 4-bit banks, their dgrads (forward 0; block-fp8 banks form one sum there).  No counterpart in the reference. */
 int xq_grouped_joint(const xq_weight* gate, const xq_weight* up, int64_t n_rows, int forward);
 int xq_grouped_fwd(const xq_weight* gate, const xq_weight* up, const xq_weight* down, const xq_grouped_lora* lora,
@@ -554,6 +550,12 @@ int xq_grouped_fwd_ids(const xq_weight* gate, const xq_weight* up, const xq_weig
                        const void* hidden, int64_t ld_hidden, int64_t n_tokens, const void* routing_w, int rw_dtype,
                        const void* ids, int id_bytes, int32_t topk, void* out, int64_t ld_out,
                        const xq_grouped_saved* saved, void* workspace, int64_t workspace_bytes, void* stream);
+/* ... where no backward follows: what `saved` points to is scratch, and the sums run in whatever order is the shortest way (the output agrees
+ * to rounding; a forward that a backward follows keeps one order, on which fp32 gradients depend) */
+int xq_grouped_fwd_eval_ids(const xq_weight* gate, const xq_weight* up, const xq_weight* down, const xq_grouped_lora* lora,
+                            const void* hidden, int64_t ld_hidden, int64_t n_tokens, const void* routing_w, int rw_dtype,
+                            const void* ids, int id_bytes, int32_t topk, void* out, int64_t ld_out,
+                            const xq_grouped_saved* saved, void* workspace, int64_t workspace_bytes, void* stream);
 int xq_grouped_bwd(const xq_weight* gate, const xq_weight* up, const xq_weight* down, const xq_grouped_lora* lora,
                    const void* dy, int64_t ld_dy, int64_t n_tokens, int32_t topk, const xq_grouped_saved* saved,
                    void* dx, int64_t ld_dx, void* d_routing, int rw_dtype, const xq_grouped_grads* grads,

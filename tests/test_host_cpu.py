@@ -341,3 +341,19 @@ def test_bank_tile_tests_reach_the_kernel():
         here = counts + [0, 300] * 100 if K == 192 else counts
         for fmt in ("block_fp8", "nvfp4"):
             assert [bank_route(fmt, len(here), K, N, sum(here), fwd) for fwd in (True, False)] == ["half", "half"], (fmt, K, N)
+
+
+def test_saved_of_a_routed_forward_is_as_callers_built_it():
+    """xq_grouped_saved is filled by callers (thirteen words): a library that reads further reads what they never wrote.  Which forward is meant
+    is said by the entry point."""
+    import ctypes
+    import os
+    import subprocess
+
+    from xorl_amd import _C
+
+    assert ctypes.sizeof(_C.XqGroupedSaved) == 13 * 8
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    code = '#include "xq.h"\n_Static_assert(sizeof(xq_grouped_saved) == 13 * 8, "grown");\n'
+    subprocess.run(["gcc", "-x", "c", "-fsyntax-only", "-I", os.path.join(root, "include"), "-"], input=code, text=True, check=True)
+    assert [hasattr(_C.lib(), f"xq_grouped_fwd{kind}_ids") for kind in ("", "_eval", "_infer")] == [True] * 3

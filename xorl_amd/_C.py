@@ -58,8 +58,7 @@ class XqGroupedLora(ctypes.Structure):
 class XqGroupedSaved(ctypes.Structure):
     _fields_ = [(n, ctypes.c_void_p) for n in ("xs", "gate_up", "h", "w_row", "su_gate", "su_up", "su_down",
                                                "scatter_index", "offsets", "tile_offsets", "counts", "x_tokens")] + [
-                                                   ("ld_x_tokens", ctypes.c_int64), ("forward_only", ctypes.c_int32),
-                                                   ("reserved", ctypes.c_int32)]
+                                                   ("ld_x_tokens", ctypes.c_int64)]
 
 
 class XqGroupedGrads(ctypes.Structure):
@@ -174,6 +173,8 @@ _SIGNATURES = {
                               ctypes.POINTER(XqGroupedSaved), _P, _I64, _P]),
     "xq_grouped_fwd_ids": (_INT, [_W, _W, _W, ctypes.POINTER(XqGroupedLora), _P, _I64, _I64, _P, _INT, _P, _INT, _I32, _P, _I64,
                               ctypes.POINTER(XqGroupedSaved), _P, _I64, _P]),
+    "xq_grouped_fwd_eval_ids": (_INT, [_W, _W, _W, ctypes.POINTER(XqGroupedLora), _P, _I64, _I64, _P, _INT, _P, _INT, _I32, _P, _I64,
+                                   ctypes.POINTER(XqGroupedSaved), _P, _I64, _P]),
     # gate, up, down, lora, dy, ld_dy, n_tokens, topk, saved, dx, ld_dx, d_routing, rw_dtype, grads, ws, ws_bytes, stream
     "xq_grouped_bwd": (_INT, [_W, _W, _W, ctypes.POINTER(XqGroupedLora), _P, _I64, _I64, _I32,
                               ctypes.POINTER(XqGroupedSaved), _P, _I64, _P, _INT, ctypes.POINTER(XqGroupedGrads), _P, _I64,

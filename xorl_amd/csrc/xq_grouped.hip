@@ -115,10 +115,11 @@ extern "C" int64_t xq_grouped_workspace_bytes(int64_t n_tokens, int32_t topk, in
     return backward ? bwd_workspace(d) : fwd_workspace(d);
 }
 
-extern "C" int xq_grouped_fwd_ids(const xq_weight* gate, const xq_weight* up, const xq_weight* down, const xq_grouped_lora* lora,
-                              const void* hidden, int64_t ld_hidden, int64_t n_tokens, const void* routing_w, int rw_dtype,
-                              const void* ids, int id_bytes, int32_t topk, void* out, int64_t ld_out,
-                              const xq_grouped_saved* saved, void* workspace, int64_t workspace_bytes, void* stream_) {
+// `order`: of the sums of gate and up
+static int grouped_forward(const xq_weight* gate, const xq_weight* up, const xq_weight* down, const xq_grouped_lora* lora, const void* hidden,
+                           int64_t ld_hidden, int64_t n_tokens, const void* routing_w, int rw_dtype, const void* ids, int id_bytes, int32_t topk,
+                           void* out, int64_t ld_out, const xq_grouped_saved* saved, void* workspace, int64_t workspace_bytes, void* stream_,
+                           SumOrder order) {
     static const char* who = "xq_grouped_fwd";
     Dims d;
     int rc = check_call(gate, up, down, lora, n_tokens, topk, saved, who, &d);
@@ -200,7 +201,6 @@ extern "C" int xq_grouped_fwd_ids(const xq_weight* gate, const xq_weight* up, co
             return rc;
         if ((rc = launch_small_nt(xr, ld_xr, R, H, F_uA, rp, s, su_u, off, toff, E, uAe == 1, stream, 0, nullptr, 0, xr_rows, nullptr, 0))) return rc;
     }
-    const SumOrder order = saved->forward_only ? SumOrder::any : SumOrder::kept;
     if (joint_forward(gate, up, R, order)) {       // both projections in one launch: column tiles past I take the up bank
         const TwoBanks two{up, su_u, Lr_uB, 0};
         if ((rc = launch_tile_gemm(gate, false, xr, ld_xr, R, off, toff, su_g, Lr_gB, rp, nullptr, gu, 2 * I, stream, who, nullptr, 0, &two, nullptr, order, xr_rows, d.T))) return rc;
@@ -218,6 +218,22 @@ extern "C" int xq_grouped_fwd_ids(const xq_weight* gate, const xq_weight* up, co
     }
     if ((rc = launch_tile_gemm(down, false, h, I, R, off, toff, su_d, Lr_dB, rp, nullptr, down_out, H, stream, who, nullptr, 0))) return rc;
     return xq_moe_gather(down_out, nullptr, H, saved->scatter_index, d.T, topk, H, out, ld_out, stream);
+}
+
+extern "C" int xq_grouped_fwd_ids(const xq_weight* gate, const xq_weight* up, const xq_weight* down, const xq_grouped_lora* lora,
+                              const void* hidden, int64_t ld_hidden, int64_t n_tokens, const void* routing_w, int rw_dtype,
+                              const void* ids, int id_bytes, int32_t topk, void* out, int64_t ld_out,
+                              const xq_grouped_saved* saved, void* workspace, int64_t workspace_bytes, void* stream_) {
+    return grouped_forward(gate, up, down, lora, hidden, ld_hidden, n_tokens, routing_w, rw_dtype, ids, id_bytes, topk, out, ld_out, saved, workspace,
+                           workspace_bytes, stream_, SumOrder::kept);
+}
+
+extern "C" int xq_grouped_fwd_eval_ids(const xq_weight* gate, const xq_weight* up, const xq_weight* down, const xq_grouped_lora* lora,
+                                       const void* hidden, int64_t ld_hidden, int64_t n_tokens, const void* routing_w, int rw_dtype,
+                                       const void* ids, int id_bytes, int32_t topk, void* out, int64_t ld_out,
+                                       const xq_grouped_saved* saved, void* workspace, int64_t workspace_bytes, void* stream_) {
+    return grouped_forward(gate, up, down, lora, hidden, ld_hidden, n_tokens, routing_w, rw_dtype, ids, id_bytes, topk, out, ld_out, saved, workspace,
+                           workspace_bytes, stream_, SumOrder::any);
 }
 
 extern "C" int xq_grouped_fwd(const xq_weight* gate, const xq_weight* up, const xq_weight* down, const xq_grouped_lora* lora,

@@ -783,12 +783,11 @@ PyObject* moe(PyObject*, PyObject* const* args, Py_ssize_t n) {
                                      empty_bf({R, rp}), empty_bf({R, rp}), empty_bf({R, rp}), i32(R), i32(E + 1), i32(2 * (E + 1)), i32(E)};
         xq_grouped_saved S;
         grouped_saved(&S, kept, nullptr);
-        S.forward_only = !train;
         Scratch ws(xq_grouped_workspace_bytes(T, (int32_t)topk, (int32_t)E, H, I, r, 0));
         {
             ReleaseGil nogil;
-            check(xq_grouped_fwd_ids(&q[0].w, &q[1].w, &q[2].w, &L, xr.ptr, xr.ld, T, w.data_ptr(), rw_code, ids.data_ptr(), id_bytes,
-                  (int32_t)topk, out.data_ptr(), H, &S, ws.get(), ws.bytes, stream));
+            check((train ? xq_grouped_fwd_ids : xq_grouped_fwd_eval_ids)(&q[0].w, &q[1].w, &q[2].w, &L, xr.ptr, xr.ld, T, w.data_ptr(), rw_code,
+                  ids.data_ptr(), id_bytes, (int32_t)topk, out.data_ptr(), H, &S, ws.get(), ws.bytes, stream));
         }
         if (!train) return THPVariable_Wrap(std::move(out));
         auto node = std::shared_ptr<QLoRAMoeBackward>(new QLoRAMoeBackward(), torch::autograd::deleteNode);

@@ -179,7 +179,7 @@ def _workspace(dev, T: int, topk: int, E: int, H: int, I: int, r: int, backward:
 
 def _moe_fwd_impl(hidden2: Tensor, rw: Tensor, sel: Tensor, factors, banks, r: int, scaling: float, allow_in_place: bool = True,
                   swiglu_limit: float = 0.0, forward_only: bool = False):
-    """xq_grouped_fwd.  hidden2 bf16 [T, H]; rw [T, topk] fp32 / bf16; sel int32 [T, topk]; factors the six active
+    """xq_grouped_fwd, or (forward_only) xq_grouped_fwd_eval_ids.  hidden2 bf16 [T, H]; rw [T, topk] fp32 / bf16; sel int32 [T, topk]; factors the six active
     LoRA views, contiguous; banks three QuantWeight.  -> (out [T, H], the eleven tensors the backward reads)."""
     qg, qu, qd = banks
     E, H, I = qg.num_experts, qg.rows, qg.cols
@@ -197,11 +197,10 @@ def _moe_fwd_impl(hidden2: Tensor, rw: Tensor, sel: Tensor, factors, banks, r: i
     out = bf(T, H)
     ws = _workspace(dev, T, topk, E, H, I, r, False)
     lora, S = _lora_struct(factors, r, scaling, swiglu_limit), _saved_struct(saved)
-    S.forward_only = int(forward_only)
-    _C.check(_C.lib().xq_grouped_fwd(ctypes.byref(wg), ctypes.byref(wu), ctypes.byref(wd), ctypes.byref(lora),
-                                     hidden2.data_ptr(), hidden2.stride(0) if T > 1 else H, T, rw.data_ptr(),
-                                     _C.XQ_DT_F32 if rw.dtype == torch.float32 else _C.XQ_DT_BF16, sel.data_ptr(), topk,
-                                     out.data_ptr(), H, ctypes.byref(S), ws.data_ptr(), ws.numel(), _s(dev)))
+    fwd = _C.lib().xq_grouped_fwd_eval_ids if forward_only else _C.lib().xq_grouped_fwd_ids
+    _C.check(fwd(ctypes.byref(wg), ctypes.byref(wu), ctypes.byref(wd), ctypes.byref(lora), hidden2.data_ptr(), hidden2.stride(0) if T > 1 else H, T,
+                 rw.data_ptr(), _C.XQ_DT_F32 if rw.dtype == torch.float32 else _C.XQ_DT_BF16, sel.data_ptr(), 4, topk,
+                 out.data_ptr(), H, ctypes.byref(S), ws.data_ptr(), ws.numel(), _s(dev)))
     return out, saved
 
 

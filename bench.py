@@ -50,16 +50,16 @@ MEASURED_TRAFFIC = {
     # gemm_dec_kernel and dec_image passes (config 2: gemm_mid_kernel too) over nvfp4 / NF4 weights: mean over the products of a step (8 and 6)
     2: (386.2 * 2 ** 20, "profiles/gemm_dec_4bit_m4096_m8192.txt", 0.1674),
     6: (1424.2 * 2 ** 20, "profiles/gemm_dec_4bit_m4096_m8192.txt", 0.6174),
-    # gemm_bank_kernel (config 3: block-fp8, config 7: nvfp4 banks): mean over the 4 launches of a step (gate|up forward over two
-    # banks, down forward, d_h, dx over both banks)
-    3: (1558.6 * 2 ** 20, "profiles/gemm_bank_fp8_nvfp4_grouped_moe_e128.txt", 0.56264),
+    # gemm_bank_kernel (config 3: block-fp8 banks; config 7: nvfp4 banks, gemm_256_kernel too): mean over the 4 launches of a step
+    # (gate|up forward over two banks, down forward, d_h, dx over both banks)
+    3: (1561.0 * 2 ** 20, "profiles/gemm_bank_fp8_nvfp4_grouped_moe_e128.txt", 0.56917),
     # skinny_gemv_kernel (M = 1), skinny_rows_kernel (M <= 16) and stream_split_kernel + stream_epilogue_kernel
     # (M = 32, 64): mean per forward over the 32 cases (includes the fp32 partial tiles of the two-launch cases
     # written and read back: 23.3 MiB of it are algorithmic)
     4: (27.4 * 2 ** 20, "profiles/skinny_kernels_decode_shapes.txt", 0.01468),
     # merge_fp8_kernel and merge_kernel<fp8>: mean per call (re-quantise 96 MiB, publish 144 MiB algorithmic)
     5: (132.1 * 2 ** 20, "profiles/merge_kernel_fp8_mlp_weights.txt", 0.03898),
-    7: (1322.3 * 2 ** 20, "profiles/gemm_bank_fp8_nvfp4_grouped_moe_e128.txt", 0.57527),
+    7: (1276.3 * 2 ** 20, "profiles/gemm_bank_fp8_nvfp4_grouped_moe_e128.txt", 0.67635),
     # merge_kernel<nvfp4>: mean per call over amax / re-quantise / publish of the four weights
     9: (55.6 * 2 ** 20, "profiles/merge_kernel_nvfp4_attn_weights.txt", 0.02234),
 }
@@ -202,8 +202,9 @@ def other_config(cfg: int, dev):
         from xorl_amd.qlora import BlockFP8QLoRAMoeExperts, NF4QLoRAMoeExperts, NvFP4QLoRAMoeExperts
 
         E, Hd, I, T, topk, r = 128, 2048, 768, 16384, 8, 16
-        cls, fmt_name, kfmt = {3: (BlockFP8QLoRAMoeExperts, "block_fp8", "fp8"), 7: (NvFP4QLoRAMoeExperts, "nvfp4", "nvfp4 GKN"),
-                               8: (NF4QLoRAMoeExperts, "NF4", "nf4 GKN")}[cfg]
+        cls, fmt_name, kernels = {3: (BlockFP8QLoRAMoeExperts, "block_fp8", "gemm_bank_kernel<fp8>"),
+                                  7: (NvFP4QLoRAMoeExperts, "nvfp4", "gemm_256_kernel and gemm_bank_kernel<nvfp4 GKN>"),
+                                  8: (NF4QLoRAMoeExperts, "NF4", "gemm_256_kernel<nf4 GKN>")}[cfg]
         m = cls(E, E, I, Hd, r=r, lora_alpha=2 * r, hybrid_shared=False).to(dev)
         g = torch.Generator(device=dev).manual_seed(50)
         w = lambda *shape: torch.randn(*shape, generator=g, device=dev) * 0.02
@@ -230,7 +231,7 @@ def other_config(cfg: int, dev):
                 f"grouped {fmt_name} QLoRA Qwen3-30B-A3B experts, E=128, hidden 2048, intermediate 768, "
                 f"top-8 of 16384 tokens, Zipf(1.1) counts (max {int(counts.max())}, {int((counts == 0).sum())} empty), "
                 f"per-expert r=16, fwd+bwd",
-                f"gemm_{'256' if cfg == 8 else 'bank'}_kernel<{kfmt}> (fused dequant grouped GEMM over the experts, forward and dgrad launches)")
+                f"{kernels} (fused dequant grouped GEMM over the experts, forward and dgrad launches)")
     if cfg == 4:
         shapes = {"q": (4096, 4096), "kv": (1024, 4096), "gate_up": (12288, 4096), "down": (4096, 12288)}
         cases, total = [], 0.0

@@ -116,8 +116,8 @@ static inline int dense_tile_size(int64_t n_rows, int64_t Nout) {
 // 1.10 to 1.14, 500 0.90; 8 experts 500 1.09 to 1.14, 750 0.87.  Block-fp8: 64 or 128 experts 46 1.14, 62 1.01, 93 1.04, 125 0.91, 281 0.87; 16
 // experts 125 1.00, 250 0.98, 500 0.81; 8 experts 125 1.23, 250 0.94, 750 0.87.
 // `bank_tiles`, products of gemm_bank_kernel whose sums are free: its 128 x 256 tiles, two on a compute unit, where there is one for every compute unit, half a tile an
-// expert left empty, or for two in five where an expert's rows fill half of one (nvfp4) or most of one.  Routed MLP forward and backward, those
-// over 128 x 128 tiles, by rows an expert, block-fp8: 128 experts 2048/768 8 0.96, 24 0.95, 56 0.86, 96 0.84; 64 experts 2048/1024 6
+// expert left empty, or for two in five where an expert's rows fill half of one (nvfp4) or most of one.  Routed MLP forward and backward, all
+// their products on these tiles, over 128 x 128 tiles, by rows an expert, block-fp8: 128 experts 2048/768 8 0.96, 24 0.95, 56 0.86, 96 0.84; 64 experts 2048/1024 6
 // 0.94, 16 0.95, 32 1.03, 64 0.92, 96 0.81; 64 experts 1280/640 6 1.10 and 16 1.02 (175 and 200 tiles), 32 0.99, 64 0.94; 32 experts 4096/1536 6
 // 1.01, 32 1.03, 64 0.88; 32 experts 1536/640 56 1.02, 72 1.02 (150 and 170 tiles), 96 0.97; 16 experts 2560/1024 40 1.11, 72 1.06 (136 tiles),
 // 96 0.95; over 256 x 256 tiles, one on a compute unit: 128 experts 128 0.83, 300 0.87, 512 0.91, 1024 0.91; 16 experts 192 0.94, 512 0.90.

@@ -19,7 +19,8 @@
 // block: 3300), at 1.85 GHz.  Measured on the way, for the four launches of a routed MLP of 128 experts 2048/768 and 131072 rows:
 // 2555 us with 256 x 256 tiles, one block a unit (12 of 30 us of a tile of 12 K-steps outside the loop: nothing overlaps them there),
 // 2420 as 128 x 256 tiles, 2250 as it stands (0.83-1.07 -> 0.97-1.2 PFLOP/s).  nvfp4, forward and backward of such an MLP, against decoded
-// tiles in LDS (gemm_256_kernel): 4400 -> 3680 us, 32768 rows 1581 -> 1122, 16384 rows 1032 -> 755.
+// tiles in LDS (gemm_256_kernel): 4400 -> 3680 us, 32768 rows 1581 -> 1122, 16384 rows 1032 -> 755; with gate, up and the dgrad of down left there, for
+// their order of sums: 4443 -> 4034, 1547 -> 1350, 998 -> 884, and without a backward, 76800 rows 1232 -> 905.
 // Dense block-fp8 MLP 4096/12288 of 2048 rows (1.5 rounds of 256 x 256 tiles), forward and backward: 1295 -> 1194 us, the forward 638 -> 571; a
 // whole number of rounds is level (4096 rows 2207, 2209), so the choice between the two is half_tiles' (xq_gemm.hip).
 //  * Two blocks on a compute unit, 80 KB of LDS each: one's start and end (7 of 26 us) run beside the other's products.  Blocks that

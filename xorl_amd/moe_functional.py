@@ -350,7 +350,7 @@ class MoeExpertsQLoRAFunction(torch.autograd.Function):
         return (dx, drw, None, *gs, None, None, None, None, None, None, None)
 
 
-# Test switch: False sends forwards that need no gradient through xq_grouped_fwd as well.
+# Test switch: False sends forwards of a handful of tokens that need no gradient through xq_grouped_fwd_eval_ids, as larger ones.
 DECODE_PATH = True
 
 
